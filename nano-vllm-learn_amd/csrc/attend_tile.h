@@ -17,6 +17,11 @@ __device__ __forceinline__ u32x2 ds_read_tr16(uint32_t lds_addr) {
     asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(lds_addr), "n"(OFF) : "memory");
     return r;
 }
+// the same read through the compiler's builtin: it places the wait itself and may move other work in between
+__device__ __forceinline__ u32x2 lds_tr16(const void* p) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
+}
 __device__ __forceinline__ uint32_t lds_addr_of(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
 __device__ __forceinline__ float max3f(float x, float y, float z) {
     float r;

@@ -1,6 +1,6 @@
 // Lightning attention: per head a matrix state with a constant decay d,   S = d S + k v^T,   o = S^T q,   q, k, v = silu of the projection's columns.
 //
-// Prompt portions (launch_lightning_chunks): a workgroup owns one (segment, head, 64 value columns) and takes 64 tokens at a time,
+// Prompt portions (launch_lightning_chunks): a workgroup owns one (segment, head, 64 or 128 value columns) and takes 64 tokens at a time,
 //   o_i = d^(i+1) S^T q_i + sum_{j <= i} d^(i-j) (q_i . k_j) v_j          S <- d^n S + sum_j d^(n-1-j) k_j v_j^T
 // on MFMA tiles.  The state stays in fp32 accumulators, laid out so that they are the left operand of S^T q without a shuffle; everything decays touch
 // (weights, state, decayed values) enters the MFMA as bf16 hi + lo halves.  q, k and v go through registers on their way to LDS (silu, one rounding),
@@ -30,12 +30,15 @@ __device__ __forceinline__ void split_hi_lo(const float (&v)[8], bf16x8& hi, bf1
     lo = *reinterpret_cast<const bf16x8*>(&l);
 }
 
+// (a reciprocal, good to one unit of the last place in 32 bits, in place of a division: half the instructions, and the result is rounded to bf16)
+__device__ __forceinline__ float silu_fast(float z) { return z * fast_rcp(1.f + fast_exp2(-kLog2e * z)); }
 __device__ __forceinline__ u32x4 silu8(u32x4 r) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) r[k] = pack_bf16x2(silu_f(bf16_lo(r[k])), silu_f(bf16_hi(r[k])));
+    for (int k = 0; k < 4; ++k) r[k] = pack_bf16x2(silu_fast(bf16_lo(r[k])), silu_fast(bf16_hi(r[k])));
     return r;
 }
 
+// (keys wider than 128: two images of each kind would not fit the LDS)
 template <int DK, bool SUMMARY>
 __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs a) {
     constexpr int KP = DK / 8, KROW = DK * 2, NQ = C * KP / 256, NV = C * (VS / 8) / 256, DT = DK / 16;
@@ -252,6 +255,318 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
     }
 }
 
+// ------------------------------------------------------------------------------------------------ the same walk with two kinds of waves
+// Half of the waves prepare: rows of the next chunk from registers through silu into the images, its weights.  The others consume: 16 value columns each, state
+// and outputs of this chunk.  Two halves a chunk, one barrier behind each:
+//   consume: o(i) = S^T q + weights v                | S(i) behind the chunk
+//   prepare: q, k of chunk i + 1 into its images     | weights of chunk i + 1, its values
+// Images are double (chunk parity), the weights are written in the half in which nobody reads them; rows are asked for a whole chunk before they are prepared.
+// What bounds it is issue (a wave alone issues a vector instruction every 5.5 cycles, three together every 2.7) and, with all CUs busy, the rows that all ask for at
+// once; so a workgroup has three waves per SIMD and takes 16 CW columns: queries and keys are prepared once for all of them (the 64-column walk below prepares them
+// for every 64).  A chunk takes 3.8 us alone and 5.4 on all CUs, 9.1 for two workgroups of the 64-column walk; 16 prompts of 1024 tokens on average, 16 heads of
+// 128: 251 -> 113 us; 40 prompts of 410: 302 -> 165.  Measured and not better: eight waves with 32 columns each (121), sixteen waves (114), fragments read a step
+// ahead by hand (121).
+template <int DK, int CW>
+constexpr size_t pair_lds_bytes(bool summary) {
+    return (size_t)2 * C * (DK * (summary ? 1 : 2) + 16 * CW) * 2 + (summary ? 0 : (size_t)2 * C * PLD * 2);
+}
+
+template <int DK, int CW, int PW, bool SUMMARY>
+__global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const LightningArgs a) {
+    constexpr int T = 64 * PW, VW = 16 * CW, KP = DK / 8, KROW = DK * 2, VP = VW / 8, VROW = VW * 2, NQ = C * KP / T, NV = C * VP / T, DT = DK / 16, PT = PW / 4;
+    constexpr int KIMG = C * KROW, VIMG = C * VROW;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    unsigned char* kimg0 = smem;                                               // [2][C][DK] keys
+    unsigned char* vimg0 = kimg0 + 2 * KIMG;                                   // [2][C][VW] values
+    unsigned char* qimg0 = vimg0 + 2 * VIMG;                                   // [2][C][DK] queries
+    uint16_t* p_lds = reinterpret_cast<uint16_t*>(qimg0 + 2 * KIMG);           // [hi | lo][C][PLD] weights
+    __shared__ __attribute__((aligned(16))) float pw[C + 1], fall_s[C];        // decay^0 .. decay^C; decay^(C - 1 - key)
+    auto swz = [](int r) { return KROW == 128 ? (r >> 1) & 7 : r & 15; };      // rows of 256 bytes span all banks: 16 of them apart, not 8
+    auto swzv = [](int r) { return VROW == 128 ? (r >> 1) & 7 : (2 * r) & 14; };
+    const int seg = blockIdx.y + blockIdx.z * gridDim.y;
+    if (seg >= a.n_chunks) return;
+    const int32_t* ch = a.chunks + 4 * seg;
+    const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
+    const int slices = a.dv / VW, head = blockIdx.x / slices, v0 = (blockIdx.x - head * slices) * VW;
+    const bool last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;
+    if (SUMMARY && last) return;                     // (nothing follows it)
+    const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lq = lane & 15, lg = lane >> 4;
+    const bool prepares = wave_id >= CW;
+    const int wave = prepares ? wave_id - CW : wave_id;
+    const int64_t slot = a.state_slots[seq];
+    const int64_t head_state = (int64_t)a.dk * a.dv;
+    if (threadIdx.x <= C) {
+        const float p = powf(a.decay[head], (float)threadIdx.x);
+        pw[threadIdx.x] = p;
+        if (threadIdx.x < C) fall_s[C - 1 - threadIdx.x] = p;
+    }
+    __syncthreads();
+
+    if (prepares) {
+        const int tid = threadIdx.x - 64 * CW;
+        const uint16_t* qkv = reinterpret_cast<const uint16_t*>(a.qkv);
+        const int64_t k_off = (int64_t)a.heads * a.dk + head * DK, v_off = 2 * (int64_t)a.heads * a.dk + (int64_t)head * a.dv + v0, q_off = (int64_t)head * DK;
+        u32x4 qr[NQ], kr[NQ], vr[NV];
+        const u32x4 zero = {0u, 0u, 0u, 0u};
+        uint32_t at[NQ], atv[NV];                    // bytes from a chunk's first row: one scalar base per chunk, no address arithmetic in the lanes
+        const uint32_t row_bytes = (uint32_t)a.qkv_stride * 2;
+        auto place = [&](int rows) __attribute__((always_inline)) {            // rows past the portion's end read its last one
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) {
+                const int e = j * T + tid, r = e / KP;
+                at[j] = (uint32_t)(r < rows ? r : rows - 1) * row_bytes + (uint32_t)(e - r * KP) * 16;
+            }
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int e = j * T + tid, r = e / VP;
+                atv[j] = (uint32_t)(r < rows ? r : rows - 1) * row_bytes + (uint32_t)(e - r * VP) * 16;
+            }
+        };
+        auto base_of = [&](int t0) __attribute__((always_inline)) { return reinterpret_cast<const unsigned char*>(qkv + (int64_t)(row0 + t0) * a.qkv_stride); };
+        auto fetch_qk = [&](int t0) __attribute__((always_inline)) {
+            if (n_rows - t0 < C) place(n_rows - t0);
+            const unsigned char* base = base_of(t0);
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) {
+                kr[j] = *reinterpret_cast<const u32x4*>(base + 2 * k_off + at[j]);
+                if constexpr (!SUMMARY) qr[j] = *reinterpret_cast<const u32x4*>(base + 2 * q_off + at[j]);
+            }
+        };
+        auto fetch_v = [&](int t0) __attribute__((always_inline)) {
+            const unsigned char* base = base_of(t0);
+#pragma unroll
+            for (int j = 0; j < NV; ++j) vr[j] = *reinterpret_cast<const u32x4*>(base + 2 * v_off + atv[j]);
+        };
+        auto stage_qk = [&](int t0, int buf) __attribute__((always_inline)) {  // rows past the end are zero (as is silu of them)
+            const int n = n_rows - t0;
+            if (n < C) {
+#pragma unroll
+                for (int j = 0; j < NQ; ++j)
+                    if ((j * T + tid) / KP >= n) kr[j] = qr[j] = zero;
+            }
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) {
+                const int e = j * T + tid, r = e / KP, pc = e - r * KP;
+                *reinterpret_cast<u32x4*>(kimg0 + buf * KIMG + r * KROW + (pc ^ swz(r)) * 16) = silu8(kr[j]);
+                if constexpr (!SUMMARY) *reinterpret_cast<u32x4*>(qimg0 + buf * KIMG + r * KROW + (pc ^ swz(r)) * 16) = silu8(qr[j]);
+            }
+        };
+        auto stage_v = [&](int t0, int buf) __attribute__((always_inline)) {
+            const int n = n_rows - t0;
+            if (n < C) {
+#pragma unroll
+                for (int j = 0; j < NV; ++j)
+                    if ((j * T + tid) / VP >= n) vr[j] = zero;
+            }
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int e = j * T + tid, r = e / VP, pc = e - r * VP;
+                *reinterpret_cast<u32x4*>(vimg0 + buf * VIMG + r * VROW + (pc ^ swzv(r)) * 16) = silu8(vr[j]);
+            }
+        };
+        // weights D[key 16 jt + 4 lg + r][query 16 tile + lq]: PT waves share a tile of queries, every PT-th tile of keys each; keys behind all queries stay zero
+        const int tile = wave / PT, Rq = 16 * tile + lq;
+        constexpr int KT = 4 / PT;                   // key tiles a wave may have
+        float fall[KT][4];
+        if constexpr (!SUMMARY) {
+#pragma unroll
+            for (int i = 0; i < KT; ++i) {
+                const int jt = PT * i + wave % PT;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int back = Rq - (16 * jt + 4 * lg + r);
+                    fall[i][r] = pw[back >= 0 ? back : 0];
+                }
+                const int to = Rq * PLD + 32 * (jt >> 1) + 8 * lg + 4 * (jt & 1);
+                if (jt > tile) *reinterpret_cast<u32x2*>(p_lds + to) = *reinterpret_cast<u32x2*>(p_lds + C * PLD + to) = u32x2{0u, 0u};
+            }
+        }
+        auto weights_of = [&](auto nc, int buf) __attribute__((always_inline)) {       // nc key tiles; only the last can be the queries' own
+            constexpr int N = decltype(nc)::value;
+            const unsigned char *kimg = kimg0 + buf * KIMG, *qimg = qimg0 + buf * KIMG;
+            f32x4 s[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int st = 0; st < DK / 32; ++st) {
+                const bf16x8 qf = *reinterpret_cast<const bf16x8*>(qimg + Rq * KROW + ((4 * st + lg) ^ swz(Rq)) * 16);
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    const int Rk = 16 * (PT * i + wave % PT) + lq;
+                    const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kimg + Rk * KROW + ((4 * st + lg) ^ swz(Rk)) * 16);
+                    s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf, s[i], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const int jt = PT * i + wave % PT;
+                float p[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    p[r] = s[i][r] * fall[i][r];
+                    if (i == N - 1 && 16 * jt + 4 * lg + r > Rq) p[r] = 0.f;
+                }
+                const u32x2 hi = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+                const u32x2 lo = {pack_bf16x2(p[0] - bf16_lo(hi[0]), p[1] - bf16_hi(hi[0])), pack_bf16x2(p[2] - bf16_lo(hi[1]), p[3] - bf16_hi(hi[1]))};
+                const int to = Rq * PLD + 32 * (jt >> 1) + 8 * lg + 4 * (jt & 1);
+                *reinterpret_cast<u32x2*>(p_lds + to) = hi;
+                *reinterpret_cast<u32x2*>(p_lds + C * PLD + to) = lo;
+            }
+        };
+        const int mine = (tile - wave % PT + PT) / PT;       // key tiles wave % PT, + PT, .. up to `tile`
+        auto weights = [&](int buf) __attribute__((always_inline)) {
+            if constexpr (!SUMMARY) {
+                if (mine == 1) weights_of(std::integral_constant<int, 1>{}, buf);
+                else if (mine == 2) weights_of(std::integral_constant<int, 2>{}, buf);
+                if constexpr (PT == 1) {
+                    if (mine == 3) weights_of(std::integral_constant<int, 3>{}, buf);
+                    else if (mine == 4) weights_of(std::integral_constant<int, 4>{}, buf);
+                }
+            }
+        };
+        place(C);
+        fetch_qk(0);
+        fetch_v(0);
+        stage_qk(0, 0);
+        if (C < n_rows) fetch_qk(C);
+        stage_v(0, 0);
+        if (C < n_rows) fetch_v(C);
+        lds_only_barrier();
+        weights(0);
+        lds_only_barrier();
+        for (int t0 = 0, buf = 0; t0 < n_rows; t0 += C, buf ^= 1) {
+            const bool next = t0 + C < n_rows, after = t0 + 2 * C < n_rows;
+            if (next) stage_qk(t0 + C, buf ^ 1);
+            if (after) fetch_qk(t0 + 2 * C);
+            lds_only_barrier();
+            if (next) {
+                weights(buf ^ 1);
+                stage_v(t0 + C, buf ^ 1);
+            }
+            if (after) fetch_v(t0 + 2 * C);
+            lds_only_barrier();
+        }
+        return;
+    }
+
+    // state: value column v0 + 16 wave + lq, key rows 16 t + 4 lg + r
+    f32x4 S[DT];
+    const int sv = v0 + 16 * wave + lq;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) S[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (!SUMMARY) {
+        const float* src = nullptr;
+        if (a.summaries) src = a.seg_state + ((int64_t)seg * a.heads + head) * head_state;
+        else if (slot >= 0 && a.positions[row0] > 0) src = a.state + (slot * a.heads + head) * head_state;
+        if (src) {
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) S[t][r] = src[(int64_t)(16 * t + 4 * lg + r) * a.dv + sv];
+        }
+    }
+    const int tr = 4 * lg + (lq >> 2), tp = lq & 3;  // transposed reads: row and column quarter this lane addresses
+    lds_only_barrier();
+    lds_only_barrier();
+    for (int t0 = 0, buf = 0; t0 < n_rows; t0 += C, buf ^= 1) {
+        const int n = n_rows - t0 < C ? n_rows - t0 : C;
+        const unsigned char *kimg = kimg0 + buf * KIMG, *qimg = qimg0 + buf * KIMG, *vimg = vimg0 + buf * VIMG;
+        // value fragments: lane = column 16 wave + lq, slots = keys 32 hh + 4 lg + 0..3 and the same + 16
+        bf16x8 vf[2];
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+            const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * wave + (tp >> 1);
+            const u32x2 lo = lds_tr16(vimg + ra * VROW + (pc ^ swzv(ra)) * 16 + (tp & 1) * 8), hi = lds_tr16(vimg + rb * VROW + (pc ^ swzv(rb)) * 16 + (tp & 1) * 8);
+            const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
+            vf[hh] = *reinterpret_cast<const bf16x8*>(&raw);
+        }
+        if constexpr (!SUMMARY) {
+            unsigned char* out = reinterpret_cast<unsigned char*>(a.out) + 2 * ((int64_t)(row0 + t0) * a.out_stride + (int64_t)head * a.dv + v0 + 16 * wave + 4 * lg);
+            const uint32_t out_bytes = (uint32_t)a.out_stride * 2;
+            // what the state gives: slots of a 32-wide step are key rows 16 (2 st) + 4 lg + 0..3 and 16 (2 st + 1) + 4 lg + 0..3
+            f32x4 o[4];                              // o^T: value 16 wave + 4 lg + r, token 16 it + lq
+#pragma unroll
+            for (int it = 0; it < 4; ++it) o[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int st = 0; st < DK / 32; ++st) {
+                const f32x4 s0 = S[2 * st], s1 = S[2 * st + 1];
+                const float v[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+                bf16x8 hi, lo;
+                split_hi_lo(v, hi, lo);
+#pragma unroll
+                for (int it = 0; it < 4; ++it) {
+                    const int R = 16 * it + lq;
+                    const unsigned char* qrow = qimg + R * KROW + (lg & 1) * 8;
+                    const u32x2 qa = *reinterpret_cast<const u32x2*>(qrow + ((4 * st + (lg >> 1)) ^ swz(R)) * 16);
+                    const u32x2 qb = *reinterpret_cast<const u32x2*>(qrow + ((4 * st + 2 + (lg >> 1)) ^ swz(R)) * 16);
+                    const u32x4 raw = {qa[0], qa[1], qb[0], qb[1]};
+                    const bf16x8 qf = *reinterpret_cast<const bf16x8*>(&raw);
+                    o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, qf, o[it], 0, 0, 0);
+                    o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, qf, o[it], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int it = 0; it < 4; ++it) o[it] *= pw[16 * it + lq + 1];
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+#pragma unroll
+                for (int hh = 0; hh <= it / 2; ++hh) {
+                    const uint16_t* pr = p_lds + (16 * it + lq) * PLD + 32 * hh + 8 * lg;
+                    o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(pr), o[it], 0, 0, 0);
+                    o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(pr + C * PLD), o[it], 0, 0, 0);
+                }
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+                if (16 * it + lq < n) act_st4(reinterpret_cast<uint16_t*>(out + (uint32_t)(16 * it + lq) * out_bytes), o[it]);
+        }
+        lds_only_barrier();                          // the weights may be replaced
+        // ---- the state behind these tokens
+        const float decayed = pw[n];
+#pragma unroll
+        for (int t = 0; t < DT; ++t) S[t] *= decayed;
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+            const u32x4 raw = *reinterpret_cast<const u32x4*>(&vf[hh]);
+            f32x4 fall[2];                           // what a value decays by until the chunk's end
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int key = 32 * hh + 16 * q + 4 * lg;
+                if (n == C) {
+                    fall[q] = *reinterpret_cast<const f32x4*>(fall_s + key);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) fall[q][r] = pw[key + r < n ? n - 1 - key - r : 0];
+                }
+            }
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = (j & 1 ? bf16_hi(raw[j >> 1]) : bf16_lo(raw[j >> 1])) * fall[j >> 2][j & 3];
+            bf16x8 hi, lo;
+            split_hi_lo(v, hi, lo);
+            const int ra = 32 * hh + tr, rb = ra + 16;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                const int pc = 2 * t + (tp >> 1);
+                const u32x2 klo = lds_tr16(kimg + ra * KROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8), khi = lds_tr16(kimg + rb * KROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8);
+                const u32x4 kraw = {klo[0], klo[1], khi[0], khi[1]};
+                const bf16x8 kf = *reinterpret_cast<const bf16x8*>(&kraw);
+                S[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, hi, S[t], 0, 0, 0);
+                S[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, lo, S[t], 0, 0, 0);
+            }
+        }
+        lds_only_barrier();                          // this chunk's images may be replaced
+    }
+    float* dst = nullptr;
+    if constexpr (SUMMARY) dst = a.seg_state + ((int64_t)seg * a.heads + head) * head_state;
+    else if (last && slot >= 0) dst = a.state + (slot * a.heads + head) * head_state;
+    if (dst) {
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dst[(int64_t)(16 * t + 4 * lg + r) * a.dv + sv] = S[t][r];
+    }
+}
+
 // contributions of the segments -> states at their starts, in place; one thread per state element, walking the segments of every portion
 __global__ __launch_bounds__(256) void lightning_starts_kernel(const LightningArgs a) {
     const int64_t head_state = (int64_t)a.dk * a.dv, per = a.heads * head_state, e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -420,6 +735,29 @@ int walk_dk(const LightningArgs& a, hipStream_t stream) {
     return check_launch("lightning walk");
 }
 
+template <int DK, int CW, int PW>
+int pair_dk(const LightningArgs& a, hipStream_t stream) {
+    constexpr size_t sum_lds = pair_lds_bytes<DK, CW>(true), lds = pair_lds_bytes<DK, CW>(false);
+    if (lds > 64 * 1024)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (sum_lds > 64 * 1024)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sum_lds);
+    // heads run fastest: workgroups are dealt round-robin over the 8 XCDs, and segments differ in length while the heads of one do not
+    const unsigned deep = (a.n_chunks + 65534) / 65535;
+    const dim3 grid(a.heads * (a.dv / (16 * CW)), (a.n_chunks + deep - 1) / deep, deep);
+    if (a.summaries) {
+        lightning_pair_kernel<DK, CW, PW, true><<<grid, 64 * (CW + PW), sum_lds, stream>>>(a);
+        int rc = check_launch("lightning summary");
+        if (rc) return rc;
+        const int64_t per = (int64_t)a.heads * a.dk * a.dv;
+        lightning_starts_kernel<<<dim3((unsigned)((per + 255) / 256), a.n_chunks), 256, 0, stream>>>(a);
+        rc = check_launch("lightning starts");
+        if (rc) return rc;
+    }
+    lightning_pair_kernel<DK, CW, PW, false><<<grid, 64 * (CW + PW), lds, stream>>>(a);
+    return check_launch("lightning walk");
+}
+
 template <typename T>
 void norm_gate_t(void* out, void* packed, const void* x, const void* gate, const float* w, float eps, int rows, int cols, int n, int64_t xs, int64_t gs, int64_t os,
                  hipStream_t stream) {
@@ -441,8 +779,8 @@ bool lightning_supported(int dk, int dv) { return (dk == 64 || dk == 128 || dk =
 int launch_lightning_chunks(const LightningArgs& a, int f32, int generic, hipStream_t stream) {
     if (!f32 && !generic && lightning_supported(a.dk, a.dv)) {
         switch (a.dk) {
-            case 64: return walk_dk<64>(a, stream);
-            case 128: return walk_dk<128>(a, stream);
+            case 64: return a.dv % 128 == 0 ? pair_dk<64, 8, 4>(a, stream) : pair_dk<64, 4, 4>(a, stream);
+            case 128: return a.dv % 128 == 0 ? pair_dk<128, 8, 4>(a, stream) : pair_dk<128, 4, 4>(a, stream);
             default: return walk_dk<256>(a, stream);
         }
     }

@@ -12,7 +12,8 @@ from .linear import linear, padded, round_up
 
 
 class LightningAttention(nn.Module):
-    segment_units = property(lambda self: self.heads * max(1, self.dv // 64))     # workgroups that walk one segment
+    # workgroups that walk one segment: one per head and 128 value columns, 64 where the columns or the keys' width leave no other choice
+    segment_units = property(lambda self: self.heads * max(1, self.dv // (128 if self.dv % 128 == 0 and self.dk <= 128 else 64)))
 
     def __init__(self, in_width, in_cols, heads, dim, vdim, decay, eps, dtype, passes=1):
         super().__init__()

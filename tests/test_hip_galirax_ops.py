@@ -246,6 +246,27 @@ def test_lightning_portions(heads, dk, dv, segment, dtype, generic):
     assert (state[1] == 1e4).all()
 
 
+@pytest.mark.parametrize("heads,dk,dv", [(2, 64, 64), (2, 64, 256), (2, 128, 128), (1, 128, 192), (1, 128, 256)])
+def test_lightning_chunk_borders_behind_a_state(heads, dk, dv):
+    """Portions of one row, a chunk and one to either side, behind states that are not zero, in rows of wider tensors; every number of 64-column groups."""
+    from nanovllm_hip import ops
+    lengths, decay = [1, 63, 64, 65, 128, 129, 320], DECAYS[:heads]
+    rows, cols = sum(lengths), heads * (2 * dk + dv)
+    x = randn(rows, cols + 64, seed=3)
+    start = randn(len(lengths), heads, dk, dv, seed=4, dtype=F32)
+    first = [sum(lengths[:i]) for i in range(len(lengths))]
+    pos = torch.cat([torch.arange(5, 5 + n) for n in lengths]).cuda()
+    chunks = torch.tensor([(f, n, i, 0) for i, (f, n) in enumerate(zip(first, lengths))], dtype=torch.int32).cuda()
+    state, out = start.cuda(), torch.full((rows, heads * dv + 32), 7.0, dtype=BF16, device="cuda")
+    ops.lightning_chunks(x.cuda()[:, :cols], torch.tensor(decay, dtype=F32).cuda(), pos, torch.arange(len(lengths), dtype=torch.int32).cuda(), chunks, False, state,
+                         out=out[:, :heads * dv])
+    assert (out[:, heads * dv:] == 7).all()
+    for i, (f, n) in enumerate(zip(first, lengths)):
+        o, s = lightning_ref(x[f:f + n, :cols], heads, dk, dv, decay, BF16, start[i])
+        close(out[f:f + n, :heads * dv], o, BF16, f"portion {i}", slack=4)
+        close(state[i], s, BF16, f"state {i}", slack=0.05)
+
+
 @pytest.mark.parametrize("heads,dk,dv,rows", [(3, 64, 64, 4), (2, 128, 128, 5), (4, 256, 64, 2), (16, 64, 64, 40)])
 def test_lightning_step(heads, dk, dv, rows):
     """Token by token: the step form against the recurrence, from garbage-filled slots on; long enough that a slow head remembers and a fast one forgets."""

@@ -263,8 +263,8 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
 // Images are double (chunk parity), the weights are written in the half in which nobody reads them; rows are asked for a whole chunk before they are prepared.
 // What bounds it is issue (a wave alone issues a vector instruction every 5.5 cycles, three together every 2.7) and, with all CUs busy, the rows that all ask for at
 // once; so a workgroup has three waves per SIMD and takes 16 CW columns: queries and keys are prepared once for all of them (the 64-column walk below prepares them
-// for every 64).  A chunk takes 3.8 us alone and 5.4 on all CUs, 9.1 for two workgroups of the 64-column walk; 16 prompts of 1024 tokens on average, 16 heads of
-// 128: 251 -> 113 us; 40 prompts of 410: 302 -> 165.  Measured and not better: eight waves with 32 columns each (121), sixteen waves (114), fragments read a step
+// for every 64).  A chunk takes 3.8 us alone and 5.0 on all CUs, 9.1 for two workgroups of the 64-column walk; 16 prompts of 1024 tokens on average, 16 heads of
+// 128: 251 -> 108 us; 40 prompts of 410: 302 -> 157.  Measured and not better: eight waves with 32 columns each (121), sixteen waves (114), fragments read a step
 // ahead by hand (121).
 template <int DK, int CW>
 constexpr size_t pair_lds_bytes(bool summary) {
@@ -323,7 +323,11 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
             }
         };
         auto base_of = [&](int t0) __attribute__((always_inline)) { return reinterpret_cast<const unsigned char*>(qkv + (int64_t)(row0 + t0) * a.qkv_stride); };
-        auto fetch_qk = [&](int t0) __attribute__((always_inline)) {
+        // (every chunk asks for as many rows as any other, in straight line, the last one's again behind the end: behind a branch around loads the compiler waits
+        // for all that are in flight instead of the ones it needs)
+        const int t_last = (n_rows - 1) / C * C;
+        auto fetch_qk = [&](int t) __attribute__((always_inline)) {
+            const int t0 = t < t_last ? t : t_last;
             if (n_rows - t0 < C) place(n_rows - t0);
             const unsigned char* base = base_of(t0);
 #pragma unroll
@@ -332,8 +336,8 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
                 if constexpr (!SUMMARY) qr[j] = *reinterpret_cast<const u32x4*>(base + 2 * q_off + at[j]);
             }
         };
-        auto fetch_v = [&](int t0) __attribute__((always_inline)) {
-            const unsigned char* base = base_of(t0);
+        auto fetch_v = [&](int t) __attribute__((always_inline)) {
+            const unsigned char* base = base_of(t < t_last ? t : t_last);
 #pragma unroll
             for (int j = 0; j < NV; ++j) vr[j] = *reinterpret_cast<const u32x4*>(base + 2 * v_off + atv[j]);
         };
@@ -428,22 +432,22 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
         fetch_qk(0);
         fetch_v(0);
         stage_qk(0, 0);
-        if (C < n_rows) fetch_qk(C);
+        fetch_qk(C);
         stage_v(0, 0);
-        if (C < n_rows) fetch_v(C);
+        fetch_v(C);
         lds_only_barrier();
         weights(0);
         lds_only_barrier();
         for (int t0 = 0, buf = 0; t0 < n_rows; t0 += C, buf ^= 1) {
-            const bool next = t0 + C < n_rows, after = t0 + 2 * C < n_rows;
+            const bool next = t0 + C < n_rows;
             if (next) stage_qk(t0 + C, buf ^ 1);
-            if (after) fetch_qk(t0 + 2 * C);
+            fetch_qk(t0 + 2 * C);
             lds_only_barrier();
             if (next) {
                 weights(buf ^ 1);
                 stage_v(t0 + C, buf ^ 1);
             }
-            if (after) fetch_v(t0 + 2 * C);
+            fetch_v(t0 + 2 * C);
             lds_only_barrier();
         }
         return;

@@ -14,6 +14,8 @@
 // segment starts, and the second walk begins there.
 // Decoding (launch_wkv_step): one workgroup per (sequence, head) computes the decays from the low-rank row, streams the state once, norms and gates.
 // A sequence's first token (position 0) takes the state as zero instead of reading it: slots need no clearing when reused.
+#include <type_traits>
+
 #include "api_common.h"
 #include "attend_tile.h"
 #include "mixers.h"
@@ -40,43 +42,253 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& 
     lo = *reinterpret_cast<const bf16x8*>(&l);
 }
 
+// the same number as one the compiler has not seen yet: what is computed from it is computed where it stands, not held in a register over the whole walk
+__device__ __forceinline__ int fresh(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 template <int DIM>
 struct WkvLds {
     static constexpr int WAVES = DIM / 16, ROW = DIM * 2, IMG = C * ROW;
     unsigned char r_hi[IMG], r_lo[IMG], k_hi[IMG], k_lo[IMG], v[IMG];          // (token by token: w as fp32 over r_hi and r_lo, k and r as they came over k_hi and k_lo)
     uint16_t p[2][C][PLD];                                                     // weights, hi | lo (token by token: outputs, [wave][16][16] fp32)
     float tot[8][DIM];                                                         // log decays by groups of 8 tokens
-    float mid[DIM], full[DIM];
+    float to_mid[DIM], to_end[DIM], mid_to_end[DIM];                           // what a channel decays by up to m, over the chunk, from m on
     float bonus[C];
     float red[WAVES][C];
+    int strong;
 };
 
-// DIM / 16 waves; wave w holds value columns 16 w ..
+// DIM / 16 waves consume: wave w holds value columns 16 w .., state and outputs of this chunk.  As many prepare the next one: log decays and their sums, r~ and k~,
+// weights.  Three parts a chunk, one barrier behind each; the images are written when this chunk's consumers are done with them:
+//   consume: outputs, state, sums of squares | norm, gate, store          |
+//   prepare: log decays of chunk i + 1       | images, tables of i + 1    | weights of i + 1
+// What bounds it is issue and latency, not memory: a wave alone issues a vector instruction every 5.5 cycles, four together every 2.3 to 3.3, so two workgroups per CU
+// (heads of 64: 62 KB and 128 registers each) keep four waves on every SIMD; no register may be spilled inside the loop, a reload waits for every row in flight.
+// A chunk of a head of 64 takes 4.0 us alone and 7.8 beside a second one (6.8 and 13.9 with one kind of wave, 275 registers and one workgroup per CU); 11 portions of
+// 1090 tokens on average, 32 heads: 274 -> 153 us, 40 prompts of 410: 384 -> 166; heads of 128 about half the time.
 template <int DIM, bool SUMMARY>
-__global__ __launch_bounds__(DIM * 4) void wkv_walk_kernel(const WkvArgs a) {
+__global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(const WkvArgs a) {
     using Lds = WkvLds<DIM>;
-    constexpr int ROW = DIM * 2, DT = DIM / 16, CP = DIM / 2, WAVES = Lds::WAVES;
-    constexpr bool kOdd = ((ROW / 128) & 1) != 0;
+    constexpr int ROW = DIM * 2, DT = DIM / 16, CP = DIM / 2, WAVES = Lds::WAVES, T = DIM * 4;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     Lds& lds = *reinterpret_cast<Lds*>(smem);
-    auto swz = [](int r) { return kOdd ? ((r >> 1) & 7) : (r & 7); };
-    const int32_t* ch = a.chunks + 4 * blockIdx.x;
+    auto swz = [](int r) { return ROW == 128 ? (r >> 1) & 7 : r & 15; };       // rows of 256 bytes span all banks
+    const int head = blockIdx.x, seg = blockIdx.y;   // heads run fastest: workgroups are dealt round-robin over the XCDs, and segments differ in length
+    const int32_t* ch = a.chunks + 4 * seg;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
-    const int head = blockIdx.y;
-    const bool last = blockIdx.x + 1 == (unsigned)a.n_chunks || a.chunks[4 * (blockIdx.x + 1) + 3] == 0;
+    const bool last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;
     if (SUMMARY && last) return;                     // (nothing follows it)
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4;
+    const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lq = lane & 15, lg = lane >> 4;
     const int64_t slot = a.state_slots[seq];
     constexpr int64_t head_state = (int64_t)DIM * DIM;
 
+    if (wave_id >= WAVES) {
+        // ---- this thread's rows of a chunk: channels 2 cp, 2 cp + 1 of tokens 8 tg ..; two 16-byte pieces of values
+        const int tid = threadIdx.x - T, wave = wave_id - WAVES, cp = tid % CP, tg = tid / CP;
+        const int hc = head * DIM + 2 * cp;
+        const float w0a = a.w0[hc], w0b = a.w0[hc + 1];
+        float ua = 0.f, ub = 0.f;
+        if constexpr (!SUMMARY) {
+            ua = a.u[hc];
+            ub = a.u[hc + 1];
+        }
+        uint32_t rr[8], kk[8], zz[8];
+        u32x4 vv[2];
+        // a chunk's rows, past the segment's end its last one.  Every chunk asks for as many rows as any other, in straight line: behind a branch around loads the
+        // compiler waits for all that are in flight instead of the ones it needs
+        const uint32_t row_bytes = (uint32_t)a.stride * 2, z_bytes = (uint32_t)a.z_stride * 2;
+        const int t_last = (n_rows - 1) / C * C;
+        auto rows_of = [&](const void* p, int64_t stride, int t0) __attribute__((always_inline)) {
+            return reinterpret_cast<const unsigned char*>(p) + 2 * ((int64_t)(row0 + t0) * stride + head * DIM);
+        };
+        auto fetch_z = [&](int t) __attribute__((always_inline)) {
+            const int t0 = t < t_last ? t : t_last, top = n_rows - t0 - 1, tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
+            const unsigned char* zb = rows_of(a.z, a.z_stride, t0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) zz[i] = *reinterpret_cast<const uint32_t*>(zb + ((uint32_t)(8 * tg + i < top ? 8 * tg + i : top) * z_bytes + 4 * cp));
+        };
+        auto fetch = [&](int t) __attribute__((always_inline)) {
+            const int t0 = t < t_last ? t : t_last, top = n_rows - t0 - 1, tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
+            const unsigned char *kb = rows_of(a.k, a.stride, t0), *rb = rows_of(a.r, a.stride, t0), *vb = rows_of(a.v, a.stride, t0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t at = (uint32_t)(8 * tg + i < top ? 8 * tg + i : top) * row_bytes + 4 * cp;
+                kk[i] = *reinterpret_cast<const uint32_t*>(kb + at);
+                if constexpr (!SUMMARY) rr[i] = *reinterpret_cast<const uint32_t*>(rb + at);
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int e = j * T + tid, r = e / (DIM / 8);
+                vv[j] = *reinterpret_cast<const u32x4*>(vb + ((uint32_t)(r < top ? r : top) * row_bytes + e % (DIM / 8) * 16));
+            }
+        };
+        float la[8], lb[8];                          // sums of log decays up to and with token i of the group
+        auto decays = [&](int n) __attribute__((always_inline)) {
+            float sa = 0.f, sb = 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float da = log2_decay(bf16_lo(zz[i]) + w0a), db = log2_decay(bf16_hi(zz[i]) + w0b);
+                const bool ok = 8 * tg + i < n;
+                sa += ok ? da : 0.f;
+                sb += ok ? db : 0.f;
+                la[i] = sa;
+                lb[i] = sb;
+            }
+            *reinterpret_cast<f32x2*>(&lds.tot[tg][2 * cp]) = f32x2{sa, sb};
+        };
+        float dec_a = 0.f, dec_b = 0.f;
+        bool strong = false;
+        auto images = [&](int t0, int n) __attribute__((always_inline)) {
+            const int tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
+            if (n < C) {                             // keys and values past the end count nothing
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (8 * tg + i >= n) kk[i] = 0u;
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    if ((j * T + tid) / (DIM / 8) >= n) vv[j] = u32x4{0u, 0u, 0u, 0u};
+            }
+            float oa = 0.f, ob = 0.f, ma = 0.f, mb = 0.f, fa = 0.f, fb = 0.f;
+#pragma unroll
+            for (int g = 0; g < 8; ++g) {
+                const f32x2 s = *reinterpret_cast<const f32x2*>(&lds.tot[g][2 * cp]);
+                oa += g < tg ? s[0] : 0.f;
+                ob += g < tg ? s[1] : 0.f;
+                if (g < 4) {
+                    ma += s[0];
+                    mb += s[1];
+                }
+                fa += s[0];
+                fb += s[1];
+            }
+            dec_a += fa;
+            dec_b += fb;
+            // (every wave holds all channels: they agree)
+            strong = __builtin_amdgcn_ballot_w64(!(fminf(fminf(ma, fa - ma), fminf(mb, fb - mb)) >= -kMaxDecay)) != 0;
+            const int pofs = (cp & 3) * 4;
+            if (!strong) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int t = 8 * tg + i, at = t * ROW + (((cp >> 2) ^ swz(t)) * 16) + pofs;
+                    const float ia = oa + la[i], ib = ob + lb[i];
+                    const float ka = bf16_lo(kk[i]) * fast_exp2(ma - ia), kb = bf16_hi(kk[i]) * fast_exp2(mb - ib);
+                    const uint32_t kh = pack_bf16x2(ka, kb);
+                    *reinterpret_cast<uint32_t*>(lds.k_hi + at) = kh;
+                    *reinterpret_cast<uint32_t*>(lds.k_lo + at) = pack_bf16x2(ka - bf16_lo(kh), kb - bf16_hi(kh));
+                    if constexpr (!SUMMARY) {
+                        const float ea = oa + (i ? la[i ? i - 1 : 0] : 0.f), eb = ob + (i ? lb[i ? i - 1 : 0] : 0.f);
+                        const float ra = bf16_lo(rr[i]) * fast_exp2(ea - ma), rb = bf16_hi(rr[i]) * fast_exp2(eb - mb);
+                        const uint32_t rh = pack_bf16x2(ra, rb);
+                        *reinterpret_cast<uint32_t*>(lds.r_hi + at) = rh;
+                        *reinterpret_cast<uint32_t*>(lds.r_lo + at) = pack_bf16x2(ra - bf16_lo(rh), rb - bf16_hi(rh));
+                    }
+                }
+            } else {
+                // (rare: z is read again, its registers hold the next chunk's)
+                float* w_f = reinterpret_cast<float*>(lds.r_hi);
+                const unsigned char* zb = rows_of(a.z, a.z_stride, t0);
+#pragma unroll 1
+                for (int i = 0; i < 8; ++i) {
+                    const int t = 8 * tg + i;
+                    const uint32_t z = *reinterpret_cast<const uint32_t*>(zb + ((uint32_t)(t < n ? t : n - 1) * z_bytes + 4 * cp));
+                    *reinterpret_cast<f32x2*>(w_f + t * DIM + 2 * cp) = f32x2{fast_exp2(log2_decay(bf16_lo(z) + w0a)), fast_exp2(log2_decay(bf16_hi(z) + w0b))};
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int t = 8 * tg + i;
+                    *reinterpret_cast<uint32_t*>(lds.k_hi + t * ROW + 4 * cp) = kk[i];
+                    if constexpr (!SUMMARY) *reinterpret_cast<uint32_t*>(lds.k_lo + t * ROW + 4 * cp) = rr[i];
+                }
+            }
+            if constexpr (!SUMMARY) {                // r . u k of the 8 tokens: over the lanes that hold a token's channels
+                float d[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    d[i] = bf16_lo(rr[i]) * ua * bf16_lo(kk[i]) + bf16_hi(rr[i]) * ub * bf16_hi(kk[i]);
+                    d[i] = sum_xor16(group_sum<16>(d[i]));
+                    if constexpr (CP == 64) d[i] = sum_xor32(d[i]);
+                }
+                if (cp == 0) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) lds.bonus[8 * tg + i] = d[i];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int e = j * T + tid, t = e / (DIM / 8), pc = e % (DIM / 8);
+                *reinterpret_cast<u32x4*>(lds.v + t * ROW + (pc ^ swz(t)) * 16) = vv[j];
+            }
+            if (tg == 0) {
+                *reinterpret_cast<f32x2*>(&lds.to_mid[2 * cp]) = f32x2{fast_exp2(ma), fast_exp2(mb)};
+                *reinterpret_cast<f32x2*>(&lds.to_end[2 * cp]) = f32x2{fast_exp2(fa), fast_exp2(fb)};
+                *reinterpret_cast<f32x2*>(&lds.mid_to_end[2 * cp]) = f32x2{fast_exp2(fa - ma), fast_exp2(fb - mb)};
+                if (cp == 0) lds.strong = strong;
+            }
+        };
+        // weights D[key 16 jt + 4 lg + r][query 16 qg + lq]: the twelve 16 x 16 tiles the outputs read, dealt to the waves
+        auto weights = [&]() __attribute__((always_inline)) {
+            if (SUMMARY || strong) return;
+            const int lane_ = fresh(lane), lq = lane_ & 15, lg = lane_ >> 4;
+#pragma unroll
+            for (int x0 = 0; x0 < 12; x0 += WAVES) {
+                const int x = x0 + wave;
+                if (x >= 12) break;
+                const int qg = x < 4 ? x >> 1 : 2 + ((x - 4) >> 2), jt = x < 4 ? x & 1 : (x - 4) & 3, Rq = 16 * qg + lq, Rk = 16 * jt + lq;
+                f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int st = 0; st < DIM / 32; ++st) {
+                    const int qat = Rq * ROW + ((4 * st + lg) ^ swz(Rq)) * 16, kat = Rk * ROW + ((4 * st + lg) ^ swz(Rk)) * 16;
+                    const bf16x8 qh = *reinterpret_cast<const bf16x8*>(lds.r_hi + qat), ql = *reinterpret_cast<const bf16x8*>(lds.r_lo + qat);
+                    const bf16x8 kh = *reinterpret_cast<const bf16x8*>(lds.k_hi + kat), kl = *reinterpret_cast<const bf16x8*>(lds.k_lo + kat);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh, s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, ql, s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qh, s, 0, 0, 0);
+                }
+                const float bonus = lds.bonus[Rq];
+                float p[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int back = Rq - (16 * jt + 4 * lg + r);
+                    p[r] = back > 0 ? s[r] : back == 0 ? bonus : 0.f;
+                }
+                const u32x2 hi = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+                const u32x2 lo = {pack_bf16x2(p[0] - bf16_lo(hi[0]), p[1] - bf16_hi(hi[0])), pack_bf16x2(p[2] - bf16_lo(hi[1]), p[3] - bf16_hi(hi[1]))};
+                const int at = 32 * (jt >> 1) + 8 * lg + 4 * (jt & 1);
+                *reinterpret_cast<u32x2*>(&lds.p[0][Rq][at]) = hi;
+                *reinterpret_cast<u32x2*>(&lds.p[1][Rq][at]) = lo;
+            }
+        };
+        fetch_z(0);
+        fetch(0);
+        auto rows = [&](int t0) { return n_rows - t0 < C ? n_rows - t0 : C; };
+        for (int t0 = 0; t0 < n_rows + C; t0 += C) {         // prepares the chunk at t0 while the one in front of it is consumed
+            const bool there = t0 < n_rows;
+            if (there) decays(rows(t0));
+            fetch_z(t0 + C);
+            lds_only_barrier();
+            if (there) images(t0, rows(t0));
+            fetch(t0 + C);
+            lds_only_barrier();
+            if (there) weights();
+            lds_only_barrier();
+        }
+        if constexpr (SUMMARY) {
+            if (tg == 0) *reinterpret_cast<f32x2*>(a.seg_decay + (int64_t)seg * a.heads * DIM + hc) = f32x2{dec_a, dec_b};
+        }
+        return;
+    }
+
     // state: value column 16 wave + lq, key rows 16 t + 4 lg + r
+    const int wave = wave_id;
     f32x4 S[DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t) S[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int sv = 16 * wave + lq;
     if constexpr (!SUMMARY) {
         const float* src = nullptr;
-        if (a.summaries) src = a.seg_state + ((int64_t)blockIdx.x * a.heads + head) * head_state;
+        if (a.summaries) src = a.seg_state + ((int64_t)seg * a.heads + head) * head_state;
         else if (slot >= 0 && a.positions[row0] > 0) src = a.state + (slot * a.heads + head) * head_state;
         if (src) {
 #pragma unroll
@@ -85,175 +297,38 @@ __global__ __launch_bounds__(DIM * 4) void wkv_walk_kernel(const WkvArgs a) {
                 for (int r = 0; r < 4; ++r) S[t][r] = src[(16 * t + 4 * lg + r) * DIM + sv];
         }
     }
-    // ---- this thread's rows of a chunk: channels 2 cp, 2 cp + 1 of tokens 8 tg ..; two 16-byte pieces of values; 4 gates of four tokens
-    const int cp = tid % CP, tg = tid / CP;
-    const int hc = head * DIM + 2 * cp;
-    const float w0a = a.w0[hc], w0b = a.w0[hc + 1];
-    float ua = 0.f, ub = 0.f;
-    if constexpr (!SUMMARY) {
-        ua = a.u[hc];
-        ub = a.u[hc + 1];
-    }
-    uint32_t rr[8], kk[8], zz[8];
-    u32x4 vv[2];
-    u32x2 gg[4];
-    auto fetch = [&](int t0) {                       // rows past the segment's end are zero (zz: not used)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int t = t0 + 8 * tg + i;
-            const bool ok = t < n_rows;
-            const int64_t row = row0 + (ok ? t : 0);
-            kk[i] = ok ? *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(a.k) + row * a.stride + hc) : 0u;
-            zz[i] = ok ? *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(a.z) + row * a.z_stride + hc) : 0u;
-            if constexpr (!SUMMARY) rr[i] = ok ? *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(a.r) + row * a.stride + hc) : 0u;
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int e = j * DIM * 4 + tid, t = t0 + e / (DIM / 8), c = e % (DIM / 8) * 8;
-            const bool ok = t < n_rows;
-            vv[j] = ok ? *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(a.v) + (int64_t)(row0 + t) * a.stride + head * DIM + c) : u32x4{0u, 0u, 0u, 0u};
-        }
-        if constexpr (!SUMMARY) {
-#pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                const int t = t0 + 16 * it + lq;
-                gg[it] = t < n_rows ? *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(a.g) + (int64_t)(row0 + t) * a.stride + head * DIM + 16 * wave + 4 * lg)
-                                    : u32x2{0u, 0u};
-            }
-        }
-    };
     f32x4 nw = {0.f, 0.f, 0.f, 0.f};
     if constexpr (!SUMMARY) nw = *reinterpret_cast<const f32x4*>(a.norm + head * DIM + 16 * wave + 4 * lg);
-    float dec_a = 0.f, dec_b = 0.f;
-    fetch(0);
+    const float inv_n = 1.f / a.n;
+    u32x2 gate[4];                                   // gates of four tokens, 4 columns
+    const uint32_t g_bytes = (uint32_t)a.stride * 2, out_bytes = (uint32_t)a.out_stride * 2;
+    auto fetch_gate = [&](int t0) __attribute__((always_inline)) {
+        if constexpr (!SUMMARY) {
+            const unsigned char* gb = reinterpret_cast<const unsigned char*>(a.g) + 2 * ((int64_t)(row0 + t0) * a.stride + head * DIM);
+            const int top = n_rows - t0 - 1, lane_ = fresh(lane), lq = lane_ & 15, col_bytes = 2 * (16 * wave + 4 * (lane_ >> 4));
+#pragma unroll
+            for (int it = 0; it < 4; ++it) gate[it] = *reinterpret_cast<const u32x2*>(gb + ((uint32_t)(16 * it + lq < top ? 16 * it + lq : top) * g_bytes + col_bytes));
+        }
+    };
+    const int tr = 4 * lg + (lq >> 2), tp = lq & 3;  // transposed reads: row and column quarter this lane addresses
+    fetch_gate(0);
+    lds_only_barrier();
+    lds_only_barrier();
+    lds_only_barrier();
     for (int t0 = 0; t0 < n_rows; t0 += C) {
         const int n = n_rows - t0 < C ? n_rows - t0 : C;
-        // ---- log decays of this thread's tokens, summed up
-        float la[8], lb[8];                          // sums up to and with token i of the group
-        {
-            float sa = 0.f, sb = 0.f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const bool ok = 8 * tg + i < n;
-                sa += ok ? log2_decay(bf16_lo(zz[i]) + w0a) : 0.f;
-                sb += ok ? log2_decay(bf16_hi(zz[i]) + w0b) : 0.f;
-                la[i] = sa;
-                lb[i] = sb;
-            }
-            *reinterpret_cast<f32x2*>(&lds.tot[tg][2 * cp]) = f32x2{sa, sb};
-        }
-        lds_only_barrier();
-        float oa = 0.f, ob = 0.f, ma = 0.f, mb = 0.f, fa = 0.f, fb = 0.f;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const f32x2 s = *reinterpret_cast<const f32x2*>(&lds.tot[g][2 * cp]);
-            oa += g < tg ? s[0] : 0.f;
-            ob += g < tg ? s[1] : 0.f;
-            if (g < 4) {
-                ma += s[0];
-                mb += s[1];
-            }
-            fa += s[0];
-            fb += s[1];
-        }
-        dec_a += fa;
-        dec_b += fb;
-        // (every wave holds all channels: they agree)
-        const bool strong = __builtin_amdgcn_ballot_w64(!(fminf(fminf(ma, fa - ma), fminf(mb, fb - mb)) >= -kMaxDecay)) != 0;
-        const int pofs = (cp & 3) * 4;
-        if (!strong) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int t = 8 * tg + i, at = t * ROW + (((cp >> 2) ^ swz(t)) * 16) + pofs;
-                const float ia = oa + la[i], ib = ob + lb[i];
-                const float ka = bf16_lo(kk[i]) * fast_exp2(ma - ia), kb = bf16_hi(kk[i]) * fast_exp2(mb - ib);
-                const uint32_t kh = pack_bf16x2(ka, kb);
-                *reinterpret_cast<uint32_t*>(lds.k_hi + at) = kh;
-                *reinterpret_cast<uint32_t*>(lds.k_lo + at) = pack_bf16x2(ka - bf16_lo(kh), kb - bf16_hi(kh));
-                if constexpr (!SUMMARY) {
-                    const float ea = oa + (i ? la[i ? i - 1 : 0] : 0.f), eb = ob + (i ? lb[i ? i - 1 : 0] : 0.f);
-                    const float ra = bf16_lo(rr[i]) * fast_exp2(ea - ma), rb = bf16_hi(rr[i]) * fast_exp2(eb - mb);
-                    const uint32_t rh = pack_bf16x2(ra, rb);
-                    *reinterpret_cast<uint32_t*>(lds.r_hi + at) = rh;
-                    *reinterpret_cast<uint32_t*>(lds.r_lo + at) = pack_bf16x2(ra - bf16_lo(rh), rb - bf16_hi(rh));
-                }
-            }
-        } else {
-            float* w_f = reinterpret_cast<float*>(lds.r_hi);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int t = 8 * tg + i;
-                *reinterpret_cast<f32x2*>(w_f + t * DIM + 2 * cp) = f32x2{fast_exp2(log2_decay(bf16_lo(zz[i]) + w0a)), fast_exp2(log2_decay(bf16_hi(zz[i]) + w0b))};
-                *reinterpret_cast<uint32_t*>(lds.k_hi + t * ROW + 4 * cp) = kk[i];
-                if constexpr (!SUMMARY) *reinterpret_cast<uint32_t*>(lds.k_lo + t * ROW + 4 * cp) = rr[i];
-            }
-        }
-        if constexpr (!SUMMARY) {                    // r . u k of the 8 tokens: over the lanes that hold a token's channels
-            float d[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                d[i] = bf16_lo(rr[i]) * ua * bf16_lo(kk[i]) + bf16_hi(rr[i]) * ub * bf16_hi(kk[i]);
-                d[i] = sum_xor16(group_sum<16>(d[i]));
-                if constexpr (CP == 64) d[i] = sum_xor32(d[i]);
-            }
-            if (cp == 0) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) lds.bonus[8 * tg + i] = d[i];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int e = j * DIM * 4 + tid, t = e / (DIM / 8), pc = e % (DIM / 8);
-            *reinterpret_cast<u32x4*>(lds.v + t * ROW + (pc ^ swz(t)) * 16) = vv[j];
-        }
-        if (tg == 0) {
-            *reinterpret_cast<f32x2*>(&lds.mid[2 * cp]) = f32x2{ma, mb};
-            *reinterpret_cast<f32x2*>(&lds.full[2 * cp]) = f32x2{fa, fb};
-        }
-        u32x2 gate[4] = {gg[0], gg[1], gg[2], gg[3]};
-        if (t0 + C < n_rows) fetch(t0 + C);
-        lds_only_barrier();
         f32x4 o[4];                                  // o^T: value 16 wave + 4 lg + r, token 16 it + lq
-        if (!strong) {
-            const int tr = 4 * lg + (lq >> 2), tp = lq & 3;                    // transposed reads: row and column quarter this lane addresses
+        if (!__builtin_amdgcn_readfirstlane(lds.strong)) {
+            // value fragments: lane = column 16 wave + lq, slots = keys 32 hh + 4 lg + 0..3 and the same + 16
+            bf16x8 vf[2];
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * wave + (tp >> 1);
+                const u32x2 lo = lds_tr16(lds.v + ra * ROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8), hi = lds_tr16(lds.v + rb * ROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8);
+                const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
+                vf[hh] = *reinterpret_cast<const bf16x8*>(&raw);
+            }
             if constexpr (!SUMMARY) {
-                // weights: D[key 16 jt + 4 lg + r][query 16 qg + lq]; with 8 waves, two share a group of queries
-                const int qg = wave & 3, Rq = 16 * qg + lq;
-                f32x4 s[4];
-#pragma unroll
-                for (int jt = 0; jt < 4; ++jt) s[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int st = 0; st < DIM / 32; ++st) {
-                    const int qat = Rq * ROW + ((4 * st + lg) ^ swz(Rq)) * 16;
-                    const bf16x8 qh = *reinterpret_cast<const bf16x8*>(lds.r_hi + qat), ql = *reinterpret_cast<const bf16x8*>(lds.r_lo + qat);
-#pragma unroll
-                    for (int jt = 0; jt < 4; ++jt) {
-                        if (jt > qg || (WAVES == 8 && (jt & 1) != wave >> 2)) continue;
-                        const int Rk = 16 * jt + lq, kat = Rk * ROW + ((4 * st + lg) ^ swz(Rk)) * 16;
-                        const bf16x8 kh = *reinterpret_cast<const bf16x8*>(lds.k_hi + kat), kl = *reinterpret_cast<const bf16x8*>(lds.k_lo + kat);
-                        s[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh, s[jt], 0, 0, 0);
-                        s[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, ql, s[jt], 0, 0, 0);
-                        s[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qh, s[jt], 0, 0, 0);
-                    }
-                }
-                // products behind a branch: hipcc counts the wait states to their readers along one path into the join only
-                asm volatile("s_nop 7" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
-                const float bonus = lds.bonus[Rq];
-#pragma unroll
-                for (int jt = 0; jt < 4; ++jt) {
-                    if (WAVES == 8 && (jt & 1) != wave >> 2) continue;
-                    float p[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int back = Rq - (16 * jt + 4 * lg + r);
-                        p[r] = back > 0 ? s[jt][r] : back == 0 ? bonus : 0.f;
-                    }
-                    const u32x2 hi = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
-                    const u32x2 lo = {pack_bf16x2(p[0] - bf16_lo(hi[0]), p[1] - bf16_hi(hi[0])), pack_bf16x2(p[2] - bf16_lo(hi[1]), p[3] - bf16_hi(hi[1]))};
-                    const int at = 32 * (jt >> 1) + 8 * lg + 4 * (jt & 1);
-                    *reinterpret_cast<u32x2*>(&lds.p[0][Rq][at]) = hi;
-                    *reinterpret_cast<u32x2*>(&lds.p[1][Rq][at]) = lo;
-                }
                 // what the state gives: slots of a 32-wide step are key rows 16 (2 st) + 4 lg + 0..3 and 16 (2 st + 1) + 4 lg + 0..3
 #pragma unroll
                 for (int it = 0; it < 4; ++it) o[it] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -262,9 +337,9 @@ __global__ __launch_bounds__(DIM * 4) void wkv_walk_kernel(const WkvArgs a) {
                     float sc[8];
 #pragma unroll
                     for (int q = 0; q < 2; ++q) {
-                        const f32x4 m4 = *reinterpret_cast<const f32x4*>(&lds.mid[16 * (2 * st + q) + 4 * lg]);
+                        const f32x4 m4 = *reinterpret_cast<const f32x4*>(&lds.to_mid[16 * (2 * st + q) + 4 * lg]);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) sc[4 * q + r] = S[2 * st + q][r] * fast_exp2(m4[r]);
+                        for (int r = 0; r < 4; ++r) sc[4 * q + r] = S[2 * st + q][r] * m4[r];
                     }
                     bf16x8 hi, lo;
                     split8(sc, hi, lo);
@@ -280,73 +355,39 @@ __global__ __launch_bounds__(DIM * 4) void wkv_walk_kernel(const WkvArgs a) {
                         o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, qh, o[it], 0, 0, 0);
                     }
                 }
-                lds_only_barrier();                  // all weights are in LDS
-            }
-            // value fragments: lane = column 16 wave + lq, slots = keys 32 hh + 4 lg + 0..3 and the same + 16
-            u32x2 vlo[2], vhi[2];
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * wave + (tp >> 1);
-                vlo[hh] = ds_read_tr16<0>(lds_addr_of(lds.v + ra * ROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8));
-                vhi[hh] = ds_read_tr16<0>(lds_addr_of(lds.v + rb * ROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8));
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-            bf16x8 vf[2];
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const u32x4 raw = {vlo[hh][0], vlo[hh][1], vhi[hh][0], vhi[hh][1]};
-                vf[hh] = *reinterpret_cast<const bf16x8*>(&raw);
-            }
-            if constexpr (!SUMMARY) {
 #pragma unroll
                 for (int it = 0; it < 4; ++it)
 #pragma unroll
-                    for (int hh = 0; hh < 2; ++hh) {
-                        if (32 * hh > 16 * it + 15) continue;
+                    for (int hh = 0; hh <= it / 2; ++hh) {
                         o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(&lds.p[0][16 * it + lq][32 * hh + 8 * lg]), o[it], 0, 0, 0);
                         o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(&lds.p[1][16 * it + lq][32 * hh + 8 * lg]), o[it], 0, 0, 0);
                     }
             }
-            // ---- the state behind these tokens, four key tiles at a time
+            // ---- the state behind these tokens
 #pragma unroll
-            for (int tb = 0; tb < DT; tb += 4) {
-                f32x4 M[4];
-#pragma unroll
-                for (int t = 0; t < 4; ++t) M[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < DT; ++t) {
+                f32x4 M = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int hh = 0; hh < 2; ++hh) {
-                    const int ra = 32 * hh + tr, rb = ra + 16;
-                    u32x2 ka[2][4], kb[2][4];
+                    const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * t + (tp >> 1);
+                    const int pa = ra * ROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8, pb = rb * ROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8;
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const int pc = 2 * (tb + t) + (tp >> 1), pa = ra * ROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8, pb = rb * ROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8;
-                        ka[0][t] = ds_read_tr16<0>(lds_addr_of(lds.k_hi + pa));
-                        kb[0][t] = ds_read_tr16<0>(lds_addr_of(lds.k_hi + pb));
-                        ka[1][t] = ds_read_tr16<0>(lds_addr_of(lds.k_lo + pa));
-                        kb[1][t] = ds_read_tr16<0>(lds_addr_of(lds.k_lo + pb));
+                    for (int q = 0; q < 2; ++q) {
+                        const unsigned char* img = q ? lds.k_lo : lds.k_hi;
+                        const u32x2 ka = lds_tr16(img + pa), kb = lds_tr16(img + pb);
+                        const u32x4 kraw = {ka[0], ka[1], kb[0], kb[1]};
+                        M = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&kraw), vf[hh], M, 0, 0, 0);
                     }
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-#pragma unroll
-                        for (int q = 0; q < 2; ++q) {
-                            const u32x4 kraw = {ka[q][t][0], ka[q][t][1], kb[q][t][0], kb[q][t][1]};
-                            M[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&kraw), vf[hh], M[t], 0, 0, 0);
-                        }
                 }
+                const f32x4 e4 = *reinterpret_cast<const f32x4*>(&lds.to_end[16 * t + 4 * lg]), f4 = *reinterpret_cast<const f32x4*>(&lds.mid_to_end[16 * t + 4 * lg]);
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const f32x4 m4 = *reinterpret_cast<const f32x4*>(&lds.mid[16 * (tb + t) + 4 * lg]), f4 = *reinterpret_cast<const f32x4*>(&lds.full[16 * (tb + t) + 4 * lg]);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) S[tb + t][r] = fast_exp2(f4[r]) * S[tb + t][r] + fast_exp2(f4[r] - m4[r]) * M[t][r];
-                }
+                for (int r = 0; r < 4; ++r) S[t][r] = e4[r] * S[t][r] + f4[r] * M[r];
             }
         } else {
             // ---- token by token; outputs of 16 tokens change lanes through a few LDS words of the wave
             const float* w_f = reinterpret_cast<const float*>(lds.r_hi);
             float* obuf = reinterpret_cast<float*>(lds.p) + wave * 256;
+            const int lane_ = fresh(lane), lq = lane_ & 15, lg = lane_ >> 4, sv = 16 * wave + lq;
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
                 o[it] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -375,7 +416,6 @@ __global__ __launch_bounds__(DIM * 4) void wkv_walk_kernel(const WkvArgs a) {
             }
         }
         if constexpr (!SUMMARY) {
-            // ---- norm over the head's columns, gate
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
                 float ss = sum4(o[it] * o[it]);
@@ -383,29 +423,32 @@ __global__ __launch_bounds__(DIM * 4) void wkv_walk_kernel(const WkvArgs a) {
                 ss = sum_xor32(ss);
                 if (lg == 0) lds.red[wave][16 * it + lq] = ss;
             }
-            lds_only_barrier();
+        }
+        lds_only_barrier();                          // this chunk's images may be replaced; sums of squares are there
+        if constexpr (!SUMMARY) {
+            // ---- norm over the head's columns, gate
+            const int lane_ = fresh(lane), lq = lane_ & 15, lg = lane_ >> 4, col_bytes = 2 * (16 * wave + 4 * lg);
+            unsigned char* out = reinterpret_cast<unsigned char*>(a.out) + 2 * ((int64_t)(row0 + t0) * a.out_stride + head * DIM) + col_bytes;
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
                 float ss = 0.f;
 #pragma unroll
                 for (int w = 0; w < WAVES; ++w) ss += lds.red[w][16 * it + lq];
-                const float inv = 1.f / sqrtf(ss / a.n + a.eps);
-                const int t = t0 + 16 * it + lq;
+                const float inv = __builtin_amdgcn_rsqf(ss * inv_n + a.eps);
                 const float g[4] = {bf16_lo(gate[it][0]), bf16_hi(gate[it][0]), bf16_lo(gate[it][1]), bf16_hi(gate[it][1])};
                 f32x4 r;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) r[k] = o[it][k] * inv * nw[k] * silu_f(g[k]);
-                if (t < n_rows) act_st4(reinterpret_cast<uint16_t*>(a.out) + (int64_t)(row0 + t) * a.out_stride + head * DIM + 16 * wave + 4 * lg, r);
+                for (int k = 0; k < 4; ++k) r[k] = o[it][k] * inv * nw[k] * (g[k] * fast_rcp(1.f + fast_exp2(-kLog2e * g[k])));
+                if (16 * it + lq < n) act_st4(reinterpret_cast<uint16_t*>(out + (uint32_t)(16 * it + lq) * out_bytes), r);
             }
+            fetch_gate(t0 + C < n_rows ? t0 + C : t0);
         }
+        lds_only_barrier();
+        lds_only_barrier();
     }
     float* dst = nullptr;
-    if constexpr (SUMMARY) {
-        dst = a.seg_state + ((int64_t)blockIdx.x * a.heads + head) * head_state;
-        if (tg == 0) *reinterpret_cast<f32x2*>(a.seg_decay + (int64_t)blockIdx.x * a.heads * DIM + hc) = f32x2{dec_a, dec_b};
-    } else if (last && slot >= 0) {
-        dst = a.state + (slot * a.heads + head) * head_state;
-    }
+    if constexpr (SUMMARY) dst = a.seg_state + ((int64_t)seg * a.heads + head) * head_state;
+    else if (last && slot >= 0) dst = a.state + (slot * a.heads + head) * head_state;
     if (dst) {
 #pragma unroll
         for (int t = 0; t < DT; ++t)
@@ -564,9 +607,9 @@ int walk_dim(const WkvArgs& a, hipStream_t stream) {
     constexpr size_t lds = sizeof(WkvLds<DIM>);
     for (const void* fn : {reinterpret_cast<const void*>(wkv_walk_kernel<DIM, true>), reinterpret_cast<const void*>(wkv_walk_kernel<DIM, false>)})
         if (lds > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    const dim3 grid(a.n_chunks, a.heads);
+    const dim3 grid(a.heads, a.n_chunks);
     if (a.summaries) {
-        wkv_walk_kernel<DIM, true><<<grid, DIM * 4, lds, stream>>>(a);
+        wkv_walk_kernel<DIM, true><<<grid, DIM * 8, lds, stream>>>(a);
         int rc = check_launch("wkv summary");
         if (rc) return rc;
         const int64_t per = (int64_t)a.heads * DIM * DIM;
@@ -574,7 +617,7 @@ int walk_dim(const WkvArgs& a, hipStream_t stream) {
         rc = check_launch("wkv starts");
         if (rc) return rc;
     }
-    wkv_walk_kernel<DIM, false><<<grid, DIM * 4, lds, stream>>>(a);
+    wkv_walk_kernel<DIM, false><<<grid, DIM * 8, lds, stream>>>(a);
     return check_launch("wkv walk");
 }
 

@@ -311,6 +311,19 @@ def test_wkv_portions(heads, dim, dk, dtype, generic, decay):
         assert (state[1] == 30).all()
 
 
+@pytest.mark.parametrize("decay", ["usual", "some chunks strong"])
+@pytest.mark.parametrize("heads,dim,dk", [(9, 64, 64), (3, 128, 128)])
+def test_wkv_chunk_borders(heads, dim, dk, decay):
+    """Portions that end on a chunk, one row in front of it and one behind it, the later ones behind a state, in segments and whole."""
+    lengths, cuts, slots = [63, 65, 129, 320], [[63], [64], [128], [64, 127, 64]], [3, 1, 0, 2]
+    layer = Wkv(lengths, heads, dim, dk, BF16, DECAYS[decay])
+    for segment in (64, 512):
+        got, state = feed_wkv(layer, lengths, cuts, slots, segment)
+        for i, (o, s) in enumerate(layer.want):
+            close(got[i], o, BF16, f"segment {segment} sequence {i}", slack=2)
+            close(state[slots[i], :, :dim, :dim], s, F32, f"state {i}", slack=64)
+
+
 @pytest.mark.parametrize("decay", ["usual", "slow", "strong"])
 @pytest.mark.parametrize("heads,dim,dk", WKV_SHAPES)
 def test_wkv_step(heads, dim, dk, decay):

@@ -9,7 +9,10 @@
 // launch turns those into states at segment starts, and the second walk begins there.
 // Decoding (launch_scan_step): four states per lane, dt from the projection's low-rank row on the spot, several rows per workgroup so that its weights are read
 // once for all of them.
-// Per (token, channel, state): one transcendental and four vector instructions: issue-bound, not HBM-bound.
+// Per (token, channel, state): one transcendental and four vector instructions: issue-bound, not HBM-bound.  So the walk is written for few instructions and no
+// waits: every load is unconditional (rows past the end repeat the last one; a load behind a branch makes the compiler wait for all of them), dt comes without
+// division and without a branch, and up to 16 states B and C stay in the activation type in LDS, one 16-byte read per token.  Channels run fastest over the grid,
+// or whole segments of different lengths fall on single XCDs.  16384 tokens of 16 sequences, 4096 channels of 16 states: 613 -> 409 us as whole portions.
 // A sequence's first token (position 0) takes the state as zero instead of reading it: slots need no clearing when reused.
 #include <type_traits>
 
@@ -26,9 +29,10 @@ constexpr int min3(int x, int y, int z) { return x < y ? (x < z ? x : z) : (y < 
 
 // log(1 + e^z); by the series of log(1 + e) where 1 + e would round
 __device__ __forceinline__ float softplus_f(float z) {
-    const float e = __expf(z);
+    const float e = fast_exp2(kLog2e * z);
     const float small = e * (1.f - e * (1.f / 2 - e * (1.f / 3 - e * (1.f / 4 - e * (1.f / 5)))));
-    return z > 20.f ? z : e < 0.0625f ? small : __logf(1.f + e);
+    const float large = 0.6931471805599453f * __builtin_amdgcn_logf(1.f + e);  // (v_log_f32: both are always taken, a branch costs more)
+    return z > 20.f ? z : e < 0.0625f ? small : large;
 }
 
 __device__ __forceinline__ float gate_f(float z) { return z * fast_rcp(1.f + fast_exp2(-kLog2e * z)); }         // silu
@@ -44,96 +48,149 @@ __device__ __forceinline__ float sum_lanes(float v) {        // over aligned gro
     return v;
 }
 
+// B and C of a token as a lane's NS states read them from LDS: [lane of the channel][B (NS) | C (NS)]
+template <typename T, int NS>
+struct StatePairs {
+    float b[NS], c[NS];
+    __device__ __forceinline__ void read(const T* p) {
+        if constexpr (sizeof(T) == 2) {
+            uint32_t raw[NS];
+#pragma unroll
+            for (int i = 0; i < NS; i += 4) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(p + 2 * i);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) raw[i + k] = v[k];
+            }
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                b[i] = i & 1 ? bf16_hi(raw[i >> 1]) : bf16_lo(raw[i >> 1]);
+                c[i] = i & 1 ? bf16_hi(raw[(NS + i) >> 1]) : bf16_lo(raw[(NS + i) >> 1]);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NS; i += 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(p + i), w = *reinterpret_cast<const f32x4*>(p + NS + i);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    b[i + k] = v[k];
+                    c[i + k] = w[k];
+                }
+            }
+        }
+    }
+};
+
 template <typename T, int NS, int NL, bool SUMMARY>
 __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
-    constexpr int NP = NS * NL, CHN = 256 / NL, TT = min3(TILE / CHN, 64, 4096 / NP), PIECES = TT * CHN / 8;     // (PIECES <= 256)
-    constexpr int BCP = (TT * 2 * NP / 8 + 255) / 256;                         // pieces of B | C per thread
-    __shared__ __attribute__((aligned(16))) float dt_s[TT * CHN], dx_s[TT * CHN], y_s[SUMMARY ? 8 : TT * CHN], bc_s[TT * 2 * NP];
-    const int32_t* ch = a.chunks + 4 * blockIdx.x;
+    constexpr int NP = NS * NL, CHN = 256 / NL, TT = min3(TILE / CHN, 64, 4096 / NP), PIECES = TT * CHN / 8;        // (PIECES <= 256)
+    constexpr int BCP = (TT * 2 * NP / 8 + 255) / 256, U = NS < 8 ? NS : 8;    // pieces of B | C per thread; states of a lane a piece holds
+    __shared__ __attribute__((aligned(16))) float dt_s[TT * CHN], dx_s[TT * CHN], y_s[SUMMARY ? 8 : TT * CHN];
+    // B and C in LDS: widened on every read where a lane has few states to do it for (16 sequences of 512 tokens, 4096 channels: 190 us against 213 at 16 states),
+    // once on the way in at 32 and 64 (242 against 296, 414 against 494); beyond that the wider rows' bank conflicts cost more than widening (928 against 1021)
+    using L = typename std::conditional<NP == 32 || NP == 64, float, T>::type;
+    __shared__ __attribute__((aligned(16))) L bc_s[TT * 2 * NP];
+    const int seg = blockIdx.y;                      // channels run fastest: workgroups are dealt round-robin over the XCDs, and segments differ in length
+    const int32_t* ch = a.chunks + 4 * seg;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
-    const bool last = blockIdx.x + 1 == (unsigned)a.n_chunks || a.chunks[4 * (blockIdx.x + 1) + 3] == 0;
+    const bool last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;
     if (SUMMARY && last) return;                     // (nothing follows it)
-    const int tid = threadIdx.x, c0 = blockIdx.y * CHN, lane_ch = tid / NL, sl = tid % NL;
-    const int my = c0 + lane_ch < a.inner ? c0 + lane_ch : a.inner - 1;        // channel this lane scans (a last group may be short)
+    const int tid = threadIdx.x, c0 = blockIdx.x * CHN, lane_ch = tid / NL, sl = tid % NL;
     const int64_t slot = a.state_slots[seq];
+    const int my = c0 + lane_ch < a.inner ? c0 + lane_ch : a.inner - 1;          // the channel this lane scans (a last group may be short)
     float A[NS], S[NS], dt_sum = 0.f;
+    const float* src = nullptr;
+    if constexpr (!SUMMARY) {
+        if (a.summaries) src = a.seg_state + ((int64_t)seg * a.inner + my) * NP;
+        else if (slot >= 0 && a.positions[row0] > 0) src = a.state + (slot * a.inner + my) * NP;
+    }
 #pragma unroll
     for (int s = 0; s < NS; s += 4) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(a.a_log2 + (int64_t)my * NP + sl * NS + s);
+        f32x4 w = {0.f, 0.f, 0.f, 0.f};
+        if (src) w = *reinterpret_cast<const f32x4*>(src + sl * NS + s);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             A[s + k] = v[k];
-            S[s + k] = 0.f;
-        }
-    }
-    if constexpr (!SUMMARY) {
-        const float* src = nullptr;
-        if (a.summaries) src = a.seg_state + ((int64_t)blockIdx.x * a.inner + my) * NP;
-        else if (slot >= 0 && a.positions[row0] > 0) src = a.state + (slot * a.inner + my) * NP;
-        if (src) {
-#pragma unroll
-            for (int s = 0; s < NS; s += 4) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(src + sl * NS + s);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) S[s + k] = v[k];
-            }
+            S[s + k] = w[k];
         }
     }
     // ---- this thread's piece of the tile: token pt, channels pc .. pc + 7
     const int pt = tid / (CHN / 8), pc = c0 + tid % (CHN / 8) * 8;
     const bool piece = tid < PIECES && pc < a.inner;
-    const f32x8 bias = piece ? act_ld8(a.dt_bias + pc) : f32x8{f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    const int pcc = pc < a.inner ? pc : a.inner - 8; // (channels come in eights)
+    const f32x8 bias = act_ld8(a.dt_bias + pcc);
     f32x8 D = bias;
-    if (!SUMMARY && piece) D = act_ld8(a.d + pc);
-    f32x8 xr, dr, zr, bc[BCP];
-    const f32x8 zero = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    auto fetch = [&](int t0) {
-        const bool ok = piece && t0 + pt < n_rows;
-        const int64_t r = row0 + t0 + pt;
-        xr = ok ? act_ld8(reinterpret_cast<const T*>(a.x) + r * a.x_stride + pc) : zero;
-        dr = ok ? act_ld8(reinterpret_cast<const T*>(a.dt) + r * a.dt_stride + pc) : zero;
-        if constexpr (!SUMMARY) zr = ok ? act_ld8(reinterpret_cast<const T*>(a.z) + r * a.z_stride + pc) : zero;
+    if (!SUMMARY) D = act_ld8(a.d + pcc);
+    using Raw = typename std::conditional<sizeof(T) == 2, u32x4, f32x8>::type;
+    auto widen = [](const Raw& r) {
+        if constexpr (sizeof(T) == 2) return unpack8(r);
+        else return r;
+    };
+    Raw xr, dr, zr, bc[BCP];
+    auto fetch = [&](int t0) __attribute__((always_inline)) {                  // rows past the end: the last one again
+        const int top = n_rows - 1;
+        const int64_t r = row0 + (t0 + pt < top ? t0 + pt : top);
+        xr = *reinterpret_cast<const Raw*>(reinterpret_cast<const T*>(a.x) + r * a.x_stride + pcc);
+        dr = *reinterpret_cast<const Raw*>(reinterpret_cast<const T*>(a.dt) + r * a.dt_stride + pcc);
+        if constexpr (!SUMMARY) zr = *reinterpret_cast<const Raw*>(reinterpret_cast<const T*>(a.z) + r * a.z_stride + pcc);
 #pragma unroll
         for (int j = 0; j < BCP; ++j) {
-            const int e = j * 256 + tid, t = e / (2 * NP / 8), p = e - t * (2 * NP / 8);
-            bc[j] = e < TT * 2 * NP / 8 && t0 + t < n_rows ? act_ld8(reinterpret_cast<const T*>(a.bc) + (int64_t)(row0 + t0 + t) * a.bc_stride + p * 8) : zero;
+            const int e = j * 256 + tid, t = t0 + e / (2 * NP / 8), p = e % (2 * NP / 8);
+            bc[j] = *reinterpret_cast<const Raw*>(reinterpret_cast<const T*>(a.bc) + (int64_t)(row0 + (t < top ? t : top)) * a.bc_stride + p * 8);
         }
     };
     fetch(0);
     for (int t0 = 0; t0 < n_rows; t0 += TT) {
         const int n = n_rows - t0 < TT ? n_rows - t0 : TT;
-        const f32x8 xk = xr, zk = zr;
+        const f32x8 xk = widen(xr);
+        const Raw zk = SUMMARY ? xr : zr;
         if (tid < PIECES) {
+            const f32x8 dk = widen(dr);
             f32x8 dt;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                dt.a[k] = pt < n ? softplus_f(dr.a[k] + bias.a[k]) : 0.f;      // (a token past the end leaves the state alone)
-                dt.b[k] = pt < n ? softplus_f(dr.b[k] + bias.b[k]) : 0.f;
+                dt.a[k] = pt < n ? softplus_f(dk.a[k] + bias.a[k]) : 0.f;      // (a token past the end leaves the state alone)
+                dt.b[k] = pt < n ? softplus_f(dk.b[k] + bias.b[k]) : 0.f;
             }
+            f32x8 dx = {dt.a * xk.a, dt.b * xk.b};
+            if (pt >= n) dx = f32x8{f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
             act_st8(dt_s + tid * 8, dt);
-            act_st8(dx_s + tid * 8, f32x8{dt.a * xk.a, dt.b * xk.b});
+            act_st8(dx_s + tid * 8, dx);
         }
 #pragma unroll
-        for (int j = 0; j < BCP; ++j)
-            if (j * 256 + tid < TT * 2 * NP / 8) act_st8(bc_s + (j * 256 + tid) * 8, bc[j]);
+        for (int j = 0; j < BCP; ++j) {
+            const int e = j * 256 + tid, t = e / (2 * NP / 8), p = e % (2 * NP / 8), half = p / (NP / 8), s0 = p % (NP / 8) * 8;       // states s0 .. s0 + 7 of B or C
+            if (e < TT * 2 * NP / 8) {
+                L* row = bc_s + t * 2 * NP + half * NS;
+                if constexpr (sizeof(L) == sizeof(T)) {
+                    const L* from = reinterpret_cast<const L*>(&bc[j]);
+#pragma unroll
+                    for (int u = 0; u < 8; u += U) {
+                        L* dst = row + (s0 + u) / NS * 2 * NS + (s0 + u) % NS;
+                        if constexpr (U * sizeof(L) == 8) *reinterpret_cast<u32x2*>(dst) = *reinterpret_cast<const u32x2*>(from + u);
+                        else if constexpr (U * sizeof(L) == 16) *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(from + u);
+                        else act_st8(dst, *reinterpret_cast<const f32x8*>(from + u));
+                    }
+                } else {
+                    const f32x8 v = widen(bc[j]);
+                    *reinterpret_cast<f32x4*>(row + s0 / NS * 2 * NS + s0 % NS) = v.a;
+                    *reinterpret_cast<f32x4*>(row + (s0 + 4) / NS * 2 * NS + (s0 + 4) % NS) = v.b;
+                }
+            }
+        }
         __syncthreads();
-        if (t0 + TT < n_rows) fetch(t0 + TT);
+        fetch(t0 + TT);
         for (int tb = 0; tb < n; tb += 4) {
 #pragma unroll
             for (int t = tb; t < tb + 4; ++t) {
                 const float dt = dt_s[t * CHN + lane_ch], dx = dx_s[t * CHN + lane_ch];
-                const float* b = bc_s + t * 2 * NP + sl * NS;
+                StatePairs<L, NS> v;
+                v.read(bc_s + t * 2 * NP + sl * 2 * NS);
                 float y = 0.f;
 #pragma unroll
-                for (int s = 0; s < NS; s += 4) {
-                    const f32x4 bv = *reinterpret_cast<const f32x4*>(b + s);
-                    f32x4 cv = bv;
-                    if constexpr (!SUMMARY) cv = *reinterpret_cast<const f32x4*>(b + NP + s);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        S[s + k] = fast_exp2(dt * A[s + k]) * S[s + k] + dx * bv[k];
-                        if constexpr (!SUMMARY) y += S[s + k] * cv[k];
-                    }
+                for (int s = 0; s < NS; ++s) {
+                    S[s] = fast_exp2(dt * A[s]) * S[s] + dx * v.b[s];
+                    if constexpr (!SUMMARY) y += S[s] * v.c[s];
                 }
                 if constexpr (SUMMARY) {
                     dt_sum += dt;
@@ -147,12 +204,13 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
         if constexpr (!SUMMARY) {
             if (piece && pt < n) {
                 f32x8 y = act_ld8(y_s + tid * 8);
+                const f32x8 z = widen(zk);
                 y.a += D.a * xk.a;
                 y.b += D.b * xk.b;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    y.a[k] *= gate_f(zk.a[k]);
-                    y.b[k] *= gate_f(zk.b[k]);
+                    y.a[k] *= gate_f(z.a[k]);
+                    y.b[k] *= gate_f(z.b[k]);
                 }
                 act_st8(reinterpret_cast<T*>(a.out) + (int64_t)(row0 + t0 + pt) * a.out_stride + pc, y);
             }
@@ -162,15 +220,14 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
     if (c0 + lane_ch >= a.inner) return;
     float* dst = nullptr;
     if constexpr (SUMMARY) {
-        dst = a.seg_state + ((int64_t)blockIdx.x * a.inner + my) * NP;
-        if (sl == 0) a.seg_dt[(int64_t)blockIdx.x * a.inner + my] = dt_sum;
+        dst = a.seg_state + ((int64_t)seg * a.inner + my) * NP;
+        if (sl == 0) a.seg_dt[(int64_t)seg * a.inner + my] = dt_sum;
     } else if (last && slot >= 0) {
         dst = a.state + (slot * a.inner + my) * NP;
     }
-    if (dst) {
+    if (!dst) return;
 #pragma unroll
-        for (int s = 0; s < NS; s += 4) *reinterpret_cast<f32x4*>(dst + sl * NS + s) = f32x4{S[s], S[s + 1], S[s + 2], S[s + 3]};
-    }
+    for (int s = 0; s < NS; s += 4) *reinterpret_cast<f32x4*>(dst + sl * NS + s) = f32x4{S[s], S[s + 1], S[s + 2], S[s + 3]};
 }
 
 // contributions of the segments -> states at their starts, in place; one thread per state, walking the segments of every portion
@@ -251,7 +308,7 @@ __global__ __launch_bounds__(256) void scan_step_kernel(const ScanArgs a) {
 template <typename T, int NS, int NL>
 int walk_ns(const ScanArgs& a, hipStream_t stream) {
     constexpr int CHN = 256 / NL;
-    const dim3 grid(a.n_chunks, (a.inner + CHN - 1) / CHN);
+    const dim3 grid((a.inner + CHN - 1) / CHN, a.n_chunks);
     if (a.summaries) {
         scan_walk_kernel<T, NS, NL, true><<<grid, 256, 0, stream>>>(a);
         int rc = check_launch("scan summary");
@@ -267,12 +324,13 @@ int walk_ns(const ScanArgs& a, hipStream_t stream) {
 
 template <typename T>
 int walk_t(const ScanArgs& a, hipStream_t stream) {
-    // states per lane: fewer lanes per channel cost less, but two waves per SIMD of the 256 CUs should be there
-    const int64_t waves = (int64_t)a.n_chunks * ((a.inner + 63) / 64);
+    // Lanes per channel: more of them add up y over more lanes and read dt and dt x again, fewer keep the chip busy with fewer workgroups and hold A, S, B and C in
+    // more registers.  16 sequences of 512 tokens, 4096 channels: 8 states 147 us with 4 lanes, 171 with 8; 16 states 190 and 202; 32 states 244 with 8 lanes,
+    // 314 with 4; 64 states 420 with 16 lanes, 506 with 8.
     switch (a.n) {
-        case 8: return waves >= 2048 ? walk_ns<T, 8, 1>(a, stream) : walk_ns<T, 4, 2>(a, stream);
-        case 16: return waves >= 2048 ? walk_ns<T, 16, 1>(a, stream) : waves >= 1024 ? walk_ns<T, 8, 2>(a, stream) : walk_ns<T, 4, 4>(a, stream);
-        case 32: return waves >= 1024 ? walk_ns<T, 16, 2>(a, stream) : walk_ns<T, 8, 4>(a, stream);
+        case 8: return walk_ns<T, 4, 2>(a, stream);
+        case 16: return walk_ns<T, 4, 4>(a, stream);
+        case 32: return walk_ns<T, 8, 4>(a, stream);
         case 64: return walk_ns<T, 16, 4>(a, stream);
         case 128: return walk_ns<T, 16, 8>(a, stream);
         default: return walk_ns<T, 16, 16>(a, stream);

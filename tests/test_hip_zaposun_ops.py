@@ -216,6 +216,19 @@ def test_scan_portions(inner, n, rank, dtype):
         assert (state[1] == 30).all()
 
 
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("inner,n", [(72, 8), (136, 16), (200, 32), (24, 64), (24, 128)])
+def test_scan_tile_borders(inner, n, dtype):
+    """Portions that end on a tile of tokens, one row in front of it and one behind it, the later ones behind a state; a last group of channels that is not full."""
+    lengths, cuts, slots = [63, 65, 128, 257], [[63], [64], [127], [32, 161, 64]], [3, 1, 0, 2]
+    layer = Scan(lengths, inner, n, 8, dtype)
+    for segment in (64, 512):
+        got, state = feed_scan(layer, lengths, cuts, slots, segment)
+        for i, (y, s) in enumerate(layer.want):
+            close(got[i], y, dtype, f"segment {segment} sequence {i}")
+            close(state[slots[i], :, :n], s, F32, f"state {i}", slack=4)
+
+
 @pytest.mark.parametrize("inner,n,rank", [(72, 5, 16), (64, 16, 64), (8192, 16, 128), (320, 30, 24), (64, 50, 8), (40, 100, 72), (24, 256, 8)])
 def test_scan_step(inner, n, rank):
     """Single tokens behind portions; many channels take several rows per workgroup."""

@@ -28,14 +28,15 @@ constexpr int kGroup = 256;                          // channels one walking wor
 __device__ __forceinline__ float fast_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ float fast_sigmoid(float x) { return fast_rcp(1.f + fast_exp2(-kLog2e * x)); }
 __device__ __forceinline__ float fast_gelu(float z) {
-    const float t = (2.f * kLog2e * 0.7978845608028654f) * (z + 0.044715f * z * z * z);
+    constexpr float c = 2.f * kLog2e * 0.7978845608028654f;
+    const float t = z * (c + c * 0.044715f * (z * z));
     return z - z * fast_rcp(1.f + fast_exp2(t));
 }
 // decay a = exp(-rate r) and input sqrt(1 - a^2) i u; 1 - a^2 by its series where it would cancel
 __device__ __forceinline__ void decay_and_input(float rate, float r, float ig, float u, float& a, float& b) {
-    const float x = rate * r, y = 2.f * x;
-    a = fast_exp2(-kLog2e * x);
-    const float series = y * (1.f - y * (1.f / 2) * (1.f - y * (1.f / 3) * (1.f - y * (1.f / 4))));
+    const float y = (2.f * rate) * r;
+    a = fast_exp2((-kLog2e * rate) * r);
+    const float series = y * (1.f + y * (-1.f / 2 + y * (1.f / 6 - y * (1.f / 24))));
     b = fast_sqrt(y < 0.06f ? series : 1.f - a * a) * ig * u;
 }
 
@@ -244,10 +245,21 @@ __global__ __launch_bounds__(1024) void rglru_walk_kernel(const RglruArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------ prompt portions, blocks of up to 256 channels
-// The same walk with everything in flight early: x of the next 64 tokens and y of these travel by LDS-DMA under this step's arithmetic, both gates' weights
-// of a wave's channels stay in registers for the whole segment (8 waves, 16 or 32 channels each), and u and y come into the accumulator layout through an
-// MFMA with a 0/1 selection matrix (exact) instead of single-element LDS reads.
+// The same walk with everything in flight early: x and y of the next 64 tokens travel by LDS-DMA under this step's arithmetic, both gates' weights of a wave's
+// 16 channels stay in registers for the whole segment, and u and y come into the accumulator layout through an MFMA with a 0/1 selection matrix (exact)
+// instead of single-element LDS reads.
+// Eight transcendentals and about 25 vector instructions per (token, channel) bound it (the vector units issue three quarters of the time at a block of 256), so
+// a block has a wave for every 16 channels, four on each SIMD at 256: 128 registers a lane, addresses computed again (fresh) instead of held.  Rows are
+// reached by 32-bit offsets from a step's first one; the 16-token passes are unrolled and find everything at fixed distances.  One barrier behind the scan frees u and
+// makes out whole, one behind the rows' way out and the next convolution frees x.
+// Four blocks of 256 channels, 16 sequences of 1024 tokens as whole portions: 200 -> 148 us; of 32 channels 66 -> 59; 16384 tokens of 16 uneven sequences, 10 blocks
+// of 256, split: 302 -> 230.
 constexpr int HALO = 8;                              // rows in front of a step's 64 in the x image: taps <= HALO + 1
+
+__device__ __forceinline__ int fresh(int v) {         // computed again from here on instead of held in registers across the loop
+    asm volatile("" : "+v"(v));
+    return v;
+}
 
 __device__ __forceinline__ void lds_barrier() {      // (a __syncthreads() would drain the DMA in flight)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -256,22 +268,27 @@ __device__ __forceinline__ void lds_barrier() {      // (a __syncthreads() would
 }
 
 template <int KS> constexpr size_t scan_x_bytes() { return (size_t)(CH + HALO) * KS * 64 + 1024; }     // (the last DMA instruction may run over)
+template <int KS> constexpr int scan_y_dma() { return 512 + (KS & (KS - 1) ? 0 : 16); }                 // elements between the pieces of two DMA instructions
+template <int KS> constexpr size_t scan_y_bytes() { return (size_t)4 * KS * scan_y_dma<KS>() * 2; }
 template <int KS> constexpr size_t scan_lds_bytes(int taps) {
-    return 2 * scan_x_bytes<KS>() + (size_t)CH * (KS * 32 + 8) * 2 + (size_t)CH * KS * 64 + (size_t)(taps + 1) * KS * 128;
+    return scan_x_bytes<KS>() + (size_t)CH * (KS * 32 + 8) * 2 + 2 * scan_y_bytes<KS>() + (size_t)(taps + 1) * KS * 128;
 }
 
-template <int KS, bool SUMMARY>                      // block = 32 KS
-__global__ __launch_bounds__(512) void rglru_scan_kernel(const RglruArgs a) {
-    constexpr int BLOCK = 32 * KS, OCT = 4 * KS, TILES = 2 * KS, NTW = (TILES + 7) / 8, LD = BLOCK + 8;
-    constexpr int SWZ = OCT % 8 == 0 ? 7 : 3;        // y image: piece p of row r sits at p ^ (r & SWZ)
-    constexpr int XINS = ((CH + HALO) * OCT + 63) / 64, YINS = OCT;
+template <int KS, bool SUMMARY>                      // block = 32 KS; grid (blocks, segments)
+__global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs a) {
+    constexpr int BLOCK = 32 * KS, OCT = 4 * KS, WAVES = 2 * KS, THREADS = 64 * WAVES, LD = BLOCK + 8;
+    constexpr int XINS = ((CH + HALO) * OCT + 63) / 64;                        // DMA instructions; y has two a wave
+    // y image: pieces of 8 channels in order, odd rows' swapped in pairs, 32 spare bytes behind 64 where a row is a power of two: 16 rows' pieces miss each
+    // other's banks, and the four rows of a lane lie at fixed distances
+    constexpr int YDMA = scan_y_dma<KS>(), YBUF = 4 * KS * YDMA;
+    static_assert(XINS <= 3 * WAVES && CH * OCT == 2 * THREADS);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    uint16_t* x_lds = reinterpret_cast<uint16_t*>(smem);                       // [2][HALO + CH][BLOCK]
-    constexpr int XBUF = scan_x_bytes<KS>() / 2;
-    uint16_t* u_lds = x_lds + 2 * XBUF;                                        // [CH][LD]
-    uint16_t* y_lds = u_lds + CH * LD;                                         // [CH][BLOCK] swizzled; out after the scan
-    float* w_lds = reinterpret_cast<float*>(y_lds + CH * BLOCK);               // [taps + 1][BLOCK]: taps, then the bias
-    const int seg = blockIdx.x, blk = blockIdx.y, c0 = blk * BLOCK;
+    uint16_t* x_lds = reinterpret_cast<uint16_t*>(smem);                       // [HALO + CH][BLOCK]
+    uint16_t* u_lds = x_lds + scan_x_bytes<KS>() / 2;                          // [CH][LD]
+    uint16_t* y_lds = u_lds + CH * LD;                                         // [2][YBUF]; out after the scan
+    float* w_lds = reinterpret_cast<float*>(y_lds + 2 * YBUF);                 // [taps + 1][BLOCK]: taps, then the bias
+    const int seg = blockIdx.y + blockIdx.z * gridDim.y, blk = blockIdx.x, c0 = blk * BLOCK;
+    if (seg >= a.n_chunks) return;
     const int row0 = a.chunks[seg * 4], n = a.chunks[seg * 4 + 1], seq = a.chunks[seg * 4 + 2], kth = a.chunks[seg * 4 + 3];
     const bool more = seg + 1 < a.n_chunks && a.chunks[seg * 4 + 6] == seq;
     if (SUMMARY && !more) return;
@@ -280,191 +297,191 @@ __global__ __launch_bounds__(512) void rglru_scan_kernel(const RglruArgs a) {
     const int64_t pos0 = a.positions[seq_row0];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4;
     const uint16_t* yx = reinterpret_cast<const uint16_t*>(a.yx);
-    const uint16_t* xcol = yx + a.width + c0;
-    auto dma = [&](const uint16_t* src, void* dst) {
+    auto dma = [&](const char* src, void* dst) __attribute__((always_inline)) {
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
     };
-    auto stage_x = [&](int t0, int buf) {            // rows t0 - HALO .. t0 + CH - 1 of the segment, clamped to the portion's rows that exist
-        const int lo = -off0, hi = n - 1;
+    const uint32_t stride = (uint32_t)a.yx_stride * 2;                         // bytes; a step's 72 rows are reached by 32-bit offsets from its first one
+    auto stage_x = [&](int t0) __attribute__((always_inline)) {                // rows t0 - HALO .. t0 + CH - 1 of the segment, clamped to the portion's rows that exist
+        const char* base = reinterpret_cast<const char*>(yx + (int64_t)(row0 + t0 - HALO) * a.yx_stride + a.width + c0);
+        const int lo = HALO - off0 - t0, hi = n - 1 + HALO - t0;
 #pragma unroll
-        for (int j = 0; j < (XINS + 7) / 8; ++j) {
-            const int ins = wave + 8 * j;
+        for (int j = 0; j < 3; ++j) {
+            const int ins = wave + WAVES * j;
             if (ins < XINS) {
-                const int s = ins * 64 + lane;
-                int t = t0 - HALO + s / OCT;
-                t = t < lo ? lo : (t > hi ? hi : t);
-                dma(xcol + (int64_t)(row0 + t) * a.yx_stride + (s % OCT) * 8, x_lds + buf * XBUF + ins * 512);
+                const int s = ins * 64 + fresh(lane), r = s / OCT, d = r < lo ? lo : (r > hi ? hi : r);
+                dma(base + ((uint32_t)d * stride + (uint32_t)(s % OCT) * 16), x_lds + ins * 512);
             }
         }
     };
-    auto stage_y = [&](int t0) {
+    auto stage_y = [&](int t0, uint16_t* image) __attribute__((always_inline)) {
+        const char* base = reinterpret_cast<const char*>(yx + (int64_t)(row0 + t0) * a.yx_stride + c0);
+        const int hi = n - 1 - t0;
 #pragma unroll
-        for (int j = 0; j < (YINS + 7) / 8; ++j) {
-            const int ins = wave + 8 * j;
-            if (ins < YINS) {
-                const int s = ins * 64 + lane, r = s / OCT, t = t0 + r < n ? t0 + r : n - 1;
-                dma(yx + (int64_t)(row0 + t) * a.yx_stride + c0 + ((s % OCT) ^ (r & SWZ)) * 8, y_lds + ins * 512);
-            }
+        for (int j = 0; j < 2; ++j) {
+            const int ins = wave + WAVES * j, s = ins * 64 + fresh(lane), r = s / OCT, d = r < hi ? r : hi;
+            dma(base + ((uint32_t)d * stride + (uint32_t)((s % OCT) ^ (r & 1)) * 16), image + ins * YDMA);
         }
     };
-    stage_x(0, 0);
-    for (int e = tid; e < (a.taps + 1) * BLOCK; e += 512) w_lds[e] = e < a.taps * BLOCK ? a.conv_w[(int64_t)(e / BLOCK) * a.width + c0 + e % BLOCK] : a.conv_b[c0 + e % BLOCK];
+    stage_x(0);
+    if (!SUMMARY) stage_y(0, y_lds);
+    for (int e = tid; e < (a.taps + 1) * BLOCK; e += THREADS)
+        w_lds[e] = e < a.taps * BLOCK ? a.conv_w[(int64_t)(e / BLOCK) * a.width + c0 + e % BLOCK] : a.conv_b[c0 + e % BLOCK];
 
-    // ---- this wave's channels: 16-channel tiles wave, wave + 8
-    bf16x8 wr[NTW][KS], wi[NTW][KS], sel;
-    float ca[NTW], cs[NTW], rb[NTW], ib[NTW], rate[NTW];
+    // ---- this wave's 16 channels
+    const int cb = 16 * wave + lq, ch = c0 + cb;
+    bf16x8 wr[KS], wi[KS], sel;
     {
-        u32x4 one;                                   // 1.0 where this lane's k-slot is its own channel (tiles wave and wave + 8: the same half of a k-step)
+        u32x4 one;                                   // 1.0 where this lane's k-slot is its own channel (tile `wave` is one half of a k-step)
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int want = 16 * (wave & 1) + lq - 8 * lg - 2 * k;
             one[k] = want == 0 ? 0x3F80u : (want == 1 ? 0x3F800000u : 0u);
         }
         sel = __builtin_bit_cast(bf16x8, one);
-    }
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) {
-        const int nt = wave + 8 * j < TILES ? wave + 8 * j : 0, cb = 16 * nt + lq, ch = c0 + cb;
-        const uint16_t* pr = reinterpret_cast<const uint16_t*>(a.ra) + ((int64_t)c0 + cb) * BLOCK + 8 * lg;
-        const uint16_t* pi = reinterpret_cast<const uint16_t*>(a.ri) + ((int64_t)c0 + cb) * BLOCK + 8 * lg;
+        const uint16_t* pr = reinterpret_cast<const uint16_t*>(a.ra) + (int64_t)ch * BLOCK + 8 * lg;
+        const uint16_t* pi = reinterpret_cast<const uint16_t*>(a.ri) + (int64_t)ch * BLOCK + 8 * lg;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
-            wr[j][k] = *reinterpret_cast<const bf16x8*>(pr + 32 * k);
-            wi[j][k] = *reinterpret_cast<const bf16x8*>(pi + 32 * k);
+            wr[k] = *reinterpret_cast<const bf16x8*>(pr + 32 * k);
+            wi[k] = *reinterpret_cast<const bf16x8*>(pi + 32 * k);
         }
-        rb[j] = -kLog2e * a.ra_b[ch], ib[j] = -kLog2e * a.ri_b[ch], rate[j] = a.rate[ch];
-        ca[j] = 1.f;
-        cs[j] = walk_start(a, SUMMARY, more, seg, kth, slot, pos0, ch);
-        if (SUMMARY && kth == 0 && wave + 8 * j < TILES && lg == 0) a.a_cum[(int64_t)seg * a.width + ch] = cs[j];
     }
+    const float rb = -kLog2e * a.ra_b[ch], ib = -kLog2e * a.ri_b[ch], rate = a.rate[ch];
+    float ca = 1.f, cs = walk_start(a, SUMMARY, more, seg, kth, slot, pos0, ch);
+    if (SUMMARY && kth == 0 && lg == 0) a.a_cum[(int64_t)seg * a.width + ch] = cs;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
     if (off0 == 0)                                   // inputs in front of the portion: from the ring, zero in front of the sequence
-        for (int e = tid; e < (a.taps - 1) * OCT; e += 512) {
+        for (int e = tid; e < (a.taps - 1) * OCT; e += THREADS) {
             const int back = e / OCT + 1, o = e % OCT;
             const uint16_t* p = conv_input<uint16_t>(a, seq_row0, -back, pos0, slot, c0 + o * 8);
             *reinterpret_cast<u32x4*>(x_lds + (HALO - back) * BLOCK + o * 8) = p ? *reinterpret_cast<const u32x4*>(p) : u32x4{0, 0, 0, 0};
         }
 
-    for (int t0 = 0, buf = 0; t0 < n; t0 += CH, buf ^= 1) {
-        const int cnt = n - t0 < CH ? n - t0 : CH;
-        // x of this step was asked for a step ago; only that step's own stores were issued behind it (vector-memory operations complete in order)
-        if (t0 > 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SUMMARY ? 0 : KS / 2) : "memory");
-        lds_barrier();                               // x is in LDS for everyone; the last step's reads of u and y are done
-        if (!SUMMARY) stage_y(t0);
-        if (t0 + CH < n) stage_x(t0 + CH, buf ^ 1);
-        // ---- u, four tokens x 8 channels a time
-        const uint16_t* xs = x_lds + buf * XBUF;
-        for (int e = tid; e < CH / 4 * OCT; e += 512) {
-            const int t = 4 * (e / OCT), o = e % OCT;
-            const float* wp = w_lds + o * 8;
-            float acc[4][8];
-            {
-                const f32x4 b0 = *reinterpret_cast<const f32x4*>(wp + a.taps * BLOCK), b1 = *reinterpret_cast<const f32x4*>(wp + a.taps * BLOCK + 4);
+    auto convolve = [&]() __attribute__((always_inline)) {                     // x -> u, eight tokens x 2 channels a thread
+        const int id = fresh(tid), o = 2 * (id % (16 * KS)), t = 8 * (id / (16 * KS));
+        const uint16_t* xp = x_lds + (HALO + t - (a.taps - 1)) * BLOCK + o;
+        const float* wp = w_lds + o;
+        const f32x2 bias = *reinterpret_cast<const f32x2*>(wp + a.taps * BLOCK);
+        float acc[8][2];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i) acc[i][0] = bias[0], acc[i][1] = bias[1];
+        if (a.taps == 4) {
+            f32x2 w[4];
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) acc[i][k] = k < 4 ? b0[k] : b1[k - 4];
-            }
-            const uint16_t* xp = xs + (HALO + t - (a.taps - 1)) * BLOCK + o * 8;
-            if (a.taps == 4) {
-                u32x4 v[7];
+            for (int j = 0; j < 4; ++j) w[j] = *reinterpret_cast<const f32x2*>(wp + j * BLOCK);
 #pragma unroll
-                for (int j = 0; j < 7; ++j) v[j] = *reinterpret_cast<const u32x4*>(xp + j * BLOCK);
+            for (int s = 0; s < 11; ++s) {
+                const uint32_t v = *reinterpret_cast<const uint32_t*>(xp + s * BLOCK);
+                const float lo = bf16_lo(v), hi = bf16_hi(v);
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) fma8(acc[i], v[i + j], wp + j * BLOCK);
-            } else {
-                for (int j = 0; j < a.taps; ++j)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) fma8(acc[i], *reinterpret_cast<const u32x4*>(xp + (i + j) * BLOCK), wp + j * BLOCK);
+                    if (s - j >= 0 && s - j < 8) {
+                        acc[s - j][0] += w[j][0] * lo;
+                        acc[s - j][1] += w[j][1] * hi;
+                    }
             }
+        } else {
+            for (int j = 0; j < a.taps; ++j) {
+                const f32x2 w = *reinterpret_cast<const f32x2*>(wp + j * BLOCK);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(u_lds + (t + i) * LD + o * 8) = pack8(acc[i]);
+                for (int i = 0; i < 8; ++i) {
+                    const uint32_t v = *reinterpret_cast<const uint32_t*>(xp + (i + j) * BLOCK);
+                    acc[i][0] += w[0] * bf16_lo(v);
+                    acc[i][1] += w[1] * bf16_hi(v);
+                }
+            }
         }
-        lds_barrier();
-#pragma unroll 1
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<uint32_t*>(u_lds + (t + i) * LD + o) = pack_bf16x2(acc[i][0], acc[i][1]);
+    };
+    lds_barrier();                                   // (what came out of the ring)
+    convolve();
+    lds_barrier();
+    for (int t0 = 0; t0 < n; t0 += CH) {
+        const int cnt = n - t0 < CH ? n - t0 : CH;
+        uint16_t* y_now = y_lds + (t0 / CH & 1) * YBUF;
+        if (t0 + CH < n) {                           // x has become u, and the other y image went out before the barrier
+            stage_x(t0 + CH);
+            if (!SUMMARY) stage_y(t0 + CH, y_lds + ((t0 / CH + 1) & 1) * YBUF);
+        }
+        const int ln = fresh(lane), lq = ln & 15, lg = ln >> 4, piece = 2 * wave + (lq >> 3);
+        const auto at = [](int row, int p) { const int s = row * OCT + p; return s / 64 * YDMA + s % 64 * 8; };
+        const uint16_t* u_row = u_lds + lq * LD + 8 * lg;
+        const uint16_t* y_row = y_now + at(lq, ((wave >> 1) * 4 + lg) ^ (lq & 1));
+        uint16_t* y_even = y_now + at(4 * lg, piece) + (lq & 7);               // this lane's channel in rows 4 lg and, by fixed distances, 4 lg + 2
+        uint16_t* y_odd = y_now + at(4 * lg, piece ^ 1) + (lq & 7);            // ... and, likewise, in 4 lg + 1 and 4 lg + 3
+#pragma unroll
         for (int tm = 0; tm < CH; tm += 16) {        // 16 tokens at a time
             if (tm > 0 && tm >= cnt) break;
-            f32x4 gr[NTW], gi[NTW];
-#pragma unroll
-            for (int j = 0; j < NTW; ++j) gr[j] = gi[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const uint16_t* u_row = u_lds + (tm + lq) * LD + 8 * lg;
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+            f32x4 gr = zero, gi = zero;
 #pragma unroll
             for (int k = 0; k < KS; ++k) {
-                const bf16x8 ua = *reinterpret_cast<const bf16x8*>(u_row + 32 * k);
+                const bf16x8 ua = *reinterpret_cast<const bf16x8*>(u_row + tm * LD + 32 * k);
+                gr = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua, wr[k], gr, 0, 0, 0);
+                gi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua, wi[k], gi, 0, 0, 0);
+            }
+            const f32x4 uu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(u_row + tm * LD + 32 * (wave >> 1)), sel, zero, 0, 0, 0);
+            f32x4 yv = zero;
+            if (!SUMMARY) yv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(y_row + tm / 16 * KS * YDMA), sel, zero, 0, 0, 0);
+            float av[4], sv[4];
 #pragma unroll
-                for (int j = 0; j < NTW; ++j) {
-                    gr[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua, wr[j][k], gr[j], 0, 0, 0);
-                    gi[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua, wi[j][k], gi[j], 0, 0, 0);
+            for (int i = 0; i < 4; ++i) {
+                const float rg = fast_rcp(1.f + fast_exp2(gr[i] * -kLog2e + rb)), ig = fast_rcp(1.f + fast_exp2(gi[i] * -kLog2e + ib));
+                decay_and_input(rate, rg, ig, uu[i], av[i], sv[i]);
+            }
+            if (tm + 16 > cnt) {                     // (tokens past the end leave the state alone)
+                asm volatile("");                    // (a branch: the comparisons are wanted in the last step only)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (tm + 4 * lg + i >= cnt) av[i] = 1.f, sv[i] = 0.f;
+            }
+#pragma unroll
+            for (int i = 1; i < 4; ++i) {            // inclusive inside the lane
+                sv[i] += av[i] * sv[i - 1];
+                av[i] *= av[i - 1];
+            }
+            // across the four lane groups (4 tokens each): e = the even group of the pair, then both pairs' totals to everyone
+            const auto swap16 = [](float v) { return __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false); };
+            const auto swap32 = [](float v) { return __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false); };
+            const bool odd = lg & 1;
+            const float pa = av[3], ps = sv[3];
+            const float ea = __uint_as_float(swap16(pa)[0]), es = __uint_as_float(swap16(ps)[0]);
+            const float ia = odd ? pa * ea : pa, is = odd ? pa * es + ps : ps;                      // inclusive inside the pair
+            const auto ha = swap32(__uint_as_float(swap16(ia)[1])), hs = swap32(__uint_as_float(swap16(is)[1]));
+            const float la = __uint_as_float(ha[0]), ls = __uint_as_float(hs[0]), ua_ = __uint_as_float(ha[1]), us_ = __uint_as_float(hs[1]);
+            if (!SUMMARY) {
+                float before = lg >= 2 ? la * cs + ls : cs;
+                before = odd ? ea * before + es : before;                                           // the state in front of this lane's first token
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    const uint32_t two = pack_bf16x2((av[i] * before + sv[i]) * fast_gelu(yv[i]), (av[i + 1] * before + sv[i + 1]) * fast_gelu(yv[i + 1]));
+                    const int off = tm / 16 * KS * YDMA + (KS == 8 ? i / 2 * YDMA : i * BLOCK);
+                    y_even[off] = (uint16_t)two;
+                    y_odd[off + BLOCK] = (uint16_t)(two >> 16);
                 }
             }
-            if (!SUMMARY && tm == 0) {               // y of this step is in LDS; x of the next may still travel
-                if (t0 + CH < n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(XINS / 8) : "memory");
-                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                lds_barrier();
-            }
-#pragma unroll
-            for (int j = 0; j < NTW; ++j) {
-                if (wave + 8 * j >= TILES) break;
-                const int nt = wave + 8 * j, cb = 16 * nt + lq, r = tm + lq;
-                const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-                const f32x4 uu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(u_row + 32 * (nt >> 1)), sel, zero, 0, 0, 0);
-                f32x4 yv = zero;
-                if (!SUMMARY)
-                    yv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(y_lds + r * BLOCK + (((nt >> 1) * 4 + lg) ^ (r & SWZ)) * 8), sel, zero,
-                                                                 0, 0, 0);
-                float av[4], sv[4];
-                float pa = 1.f, ps = 0.f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float rg = fast_rcp(1.f + fast_exp2(gr[j][i] * -kLog2e + rb[j])), ig = fast_rcp(1.f + fast_exp2(gi[j][i] * -kLog2e + ib[j]));
-                    float dec, inp;
-                    decay_and_input(rate[j], rg, ig, uu[i], dec, inp);
-                    if (tm + 4 * lg + i >= cnt) dec = 1.f, inp = 0.f;
-                    ps = dec * ps + inp;
-                    pa *= dec;
-                    av[i] = pa;
-                    sv[i] = ps;
-                }
-                // across the four lane groups (4 tokens each): e = the even group of the pair, then both pairs' totals to everyone
-                const auto swap16 = [](float v) { return __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false); };
-                const auto swap32 = [](float v) { return __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false); };
-                const bool odd = lg & 1;
-                const float ea = __uint_as_float(swap16(pa)[0]), es = __uint_as_float(swap16(ps)[0]);
-                const float ia = odd ? pa * ea : pa, is = odd ? pa * es + ps : ps;                  // inclusive inside the pair
-                const auto ha = swap32(__uint_as_float(swap16(ia)[1])), hs = swap32(__uint_as_float(swap16(is)[1]));
-                const float la = __uint_as_float(ha[0]), ls = __uint_as_float(hs[0]), ua_ = __uint_as_float(ha[1]), us_ = __uint_as_float(hs[1]);
-                if (!SUMMARY) {
-                    float before = lg >= 2 ? la * cs[j] + ls : cs[j];
-                    before = odd ? ea * before + es : before;                                       // the state in front of this lane's first token
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int ro = tm + 4 * lg + i;
-                        act_st(y_lds + ro * BLOCK + ((cb >> 3) ^ (ro & SWZ)) * 8 + (cb & 7), (av[i] * before + sv[i]) * fast_gelu(yv[i]));
-                    }
-                }
-                cs[j] = ua_ * (la * cs[j] + ls) + us_;
-                ca[j] *= la * ua_;
-            }
+            cs = ua_ * (la * cs + ls) + us_;
+            if (SUMMARY) ca *= la * ua_;
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the next step's x and y, asked for a step ago
+        lds_barrier();                               // they are in LDS for everyone; u is free and out is whole
         if (!SUMMARY) {
-            lds_barrier();
-            for (int e = tid; e < cnt * OCT; e += 512) {
-                const int r = e / OCT, p = e % OCT;
-                *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(a.out) + (int64_t)(row0 + t0 + r) * a.out_stride + c0 + p * 8) =
-                    *reinterpret_cast<const u32x4*>(y_lds + r * BLOCK + (p ^ (r & SWZ)) * 8);
+            char* out = reinterpret_cast<char*>(reinterpret_cast<uint16_t*>(a.out) + (int64_t)(row0 + t0) * a.out_stride + c0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int e = fresh(tid) + j * THREADS, r = e / OCT, p = e % OCT;
+                if (r < cnt)
+                    *reinterpret_cast<u32x4*>(out + ((uint32_t)r * (uint32_t)(a.out_stride * 2) + (uint32_t)p * 16)) = *reinterpret_cast<const u32x4*>(y_now + at(r, p ^ (r & 1)));
             }
         }
+        if (t0 + CH < n) convolve();
+        lds_barrier();
     }
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) {
-        const int nt = wave + 8 * j, ch = c0 + 16 * nt + lq;
-        if (nt < TILES && lg == 0 && (SUMMARY || !more)) {
-            a.s_loc[(int64_t)seg * a.width + ch] = cs[j];
-            if (SUMMARY && kth) a.a_cum[(int64_t)seg * a.width + ch] = ca[j];
-        }
+    if (lg == 0 && (SUMMARY || !more)) {
+        a.s_loc[(int64_t)seg * a.width + ch] = cs;
+        if (SUMMARY && kth) a.a_cum[(int64_t)seg * a.width + ch] = ca;
     }
 }
 
@@ -684,12 +701,15 @@ template <bool SUMMARY, int KS>
 bool scan_ks(const RglruArgs& a, hipStream_t stream) {
     const size_t lds = scan_lds_bytes<KS>(a.taps);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rglru_scan_kernel<KS, SUMMARY>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
-    rglru_scan_kernel<KS, SUMMARY><<<dim3(a.n_chunks, a.blocks), 512, lds, stream>>>(a);
+    // blocks run fastest: workgroups are dealt round-robin over the 8 XCDs, and segments differ in length while the blocks of one do not
+    const int deep = (a.n_chunks + 65534) / 65535;
+    rglru_scan_kernel<KS, SUMMARY><<<dim3(a.blocks, (a.n_chunks + deep - 1) / deep, deep), 128 * KS, lds, stream>>>(a);
     return true;
 }
 template <bool SUMMARY>
 bool scan(const RglruArgs& a, hipStream_t stream) {
-    if (a.taps > HALO + 1 || scan_lds_bytes<8>(a.taps) > kMaxLds) return false;
+    // (32-bit row offsets: 72 rows of less than 2^25 bytes)
+    if (a.taps > HALO + 1 || a.yx_stride >= 1 << 24 || a.out_stride >= 1 << 24 || scan_lds_bytes<8>(a.taps) > kMaxLds) return false;
     switch (a.block / 32) {
         case 1: return scan_ks<SUMMARY, 1>(a, stream);
         case 2: return scan_ks<SUMMARY, 2>(a, stream);

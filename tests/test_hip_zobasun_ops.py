@@ -186,6 +186,32 @@ def test_recurrence_portions(blocks, size, block, taps, dtype, generic, segment)
     close(r.unspread(r.state[[2, 0]].cpu()), torch.stack([la, lb]), torch.float32, 40 if dtype == torch.bfloat16 else 3)
 
 
+@pytest.mark.parametrize("segment", [64, 4096])
+@pytest.mark.parametrize("blocks,block,taps", [(2, 32, 4), (2, 96, 4), (2, 128, 4), (2, 192, 3), (1, 256, 9)])
+def test_recurrence_row_edges(blocks, block, taps, segment):
+    """Portions that end on, in front of and behind 16 and 64 tokens, then their last tokens from the state."""
+    r = Recurrence(blocks, block, block, taps, torch.bfloat16, slots=8)
+    lengths = [15, 16, 17, 48, 63, 64, 65, 129]
+    data = [r.yx(n, i) for i, n in enumerate(lengths)]
+    want = [r.plain(y, x) for y, x in data]
+    for cut in (slice(0, -3), slice(-3, None)):
+        got = r.run([(i, range(n)[cut][0], y[cut], x[cut]) for i, (n, (y, x)) in enumerate(zip(lengths, data))], segment=segment)
+        for g, (w, _) in zip(got, want):
+            close(g, w[cut], torch.bfloat16)
+    close(r.unspread(r.state.cpu()), torch.stack([s for _, s in want]), torch.float32, 40)
+
+
+def test_recurrence_rows_far_apart():
+    """Rows too far apart for 32-bit offsets."""
+    from nanovllm_hip import ops
+    r = Recurrence(2, 64, 64, 4, torch.bfloat16)
+    y, x = r.yx(3, 1)
+    rows = torch.zeros((3, 1 << 24), dtype=torch.bfloat16, device="cuda")[:, :2 * r.cols].copy_(r.rows(y, x))
+    out = ops.rglru_chunks(rows, r.params, torch.arange(3).cuda(), torch.zeros(1, dtype=torch.int32, device="cuda"), torch.tensor([[0, 3, 0, 0]], dtype=torch.int32, device="cuda"),
+                           64, False, r.state, r.conv_state)
+    close(out.cpu(), r.plain(y, x)[0], torch.bfloat16)
+
+
 @pytest.mark.parametrize("blocks,size,block,taps", SHAPES)
 def test_recurrence_step_follows_portions(blocks, size, block, taps):
     """Prompt by the chunked form, then single tokens by the step form (one sequence steps from its very first token)."""

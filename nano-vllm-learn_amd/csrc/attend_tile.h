@@ -1,5 +1,5 @@
 // The MFMA tile of the prompt-attention kernels that read keys and values from LDS images of 64 rows (unequal widths DK, DV):
-// 4 waves x QT x 16 query rows, S^T = K Q^T and O^T = V^T P^T with the weights as bf16 hi + lo halves, online softmax in the log2 domain.
+// WV waves x QT x 16 query rows, S^T = K Q^T and O^T = V^T P^T with the weights as bf16 hi + lo halves, online softmax in the log2 domain.
 // A kernel stages the images (16-byte pieces swizzled by swz_k / swz_v), fills the query fragments and says which keys a query sees.
 #pragma once
 #include <type_traits>
@@ -45,17 +45,17 @@ template <int W>
 __device__ __forceinline__ int swz_v(int row) { return W == 64 ? (row & 6) : ((2 * row) & 14); }
 
 // LDS of a tile walk: V images of both buffers, then their K images (V offsets fit a DS immediate)
-template <int DK, int DV>
+template <int DK, int DV, int WV = 4>
 struct TileImages {
     static constexpr int BN = 64, KROW = DK * 2, VROW = DV * 2, KIMG = BN * KROW, VIMG = BN * VROW;
     static constexpr int KP = DK / 8, VP = DV / 8;   // 16-byte pieces per row == DMA instructions per image
-    static constexpr int NK = KP / 4, NV = VP / 4;   // ... per wave
+    static constexpr int NK = KP / WV, NV = VP / WV; // ... per wave
     static constexpr size_t BYTES = (size_t)2 * (KIMG + VIMG);
     static __device__ __forceinline__ unsigned char* k(unsigned char* lds, int buf) { return lds + 2 * VIMG + buf * KIMG; }
     static __device__ __forceinline__ unsigned char* v(unsigned char* lds, int buf) { return lds + buf * VIMG; }
 };
 
-// One workgroup's attention over n_tiles tiles of 64 keys; wave w holds query rows 16 QT w .. of the workgroup's 64 QT.  The kernel says
+// One workgroup's attention over n_tiles tiles of 64 keys; wave w holds query rows 16 QT w .. of the workgroup's 16 WV QT.  The kernel says
 //   stage(it, buf)       starts the NK + NV DMA instructions per wave that fill buffer `buf` with tile `it`
 //   query(qs, st)        query fragment: row lq of sub-tile qs, columns 32 st + 8 lg .. (B operand of S^T)
 //   first_key(it)        key of the tile's first row; covers(kv0): this wave sees something of that tile; masked(kv0): but not all of it:
@@ -63,11 +63,13 @@ struct TileImages {
 //   row(qs)              where the lane's query of sub-tile qs goes, or null; last(qs, d, v): what becomes of its 4 output columns from d on
 // start: score (log2 domain) of a softmax entry without key and value, -inf for none.
 // (The sums, the fragments and the tile loop live in ONE function: split up, the same code takes 32 registers more.)
-template <int DK, int DV, int QT, typename Stage, typename Query, typename FirstKey, typename Covers, typename Masked, typename Sees, typename Row, typename Last>
+template <int DK, int DV, int QT, int WV, typename Stage, typename Query, typename FirstKey, typename Covers, typename Masked, typename Sees, typename Row, typename Last>
 __device__ __forceinline__ void attend_walk(unsigned char* lds, int n_tiles, float scale_log2, float start, int lane, Stage stage, Query query, FirstKey first_key, Covers covers,
                                             Masked need_mask, Sees sees, Row row, Last last) {
-    using Images = TileImages<DK, DV>;
+    using Images = TileImages<DK, DV, WV>;
     constexpr int BN = Images::BN, KROW = Images::KROW, VROW = Images::VROW, KIMG = Images::KIMG, VIMG = Images::VIMG, NK = Images::NK, NV = Images::NV;
+    static_assert((DV & (DV - 1)) == 0 && VROW <= 512);
+    constexpr int VBATCH = WV == 8 ? 4 : 16;         // (eight waves live on 128 registers)
     constexpr int STEPS = DK / 32, DT = DV / 16, NT = BN / 16;
     const int lq = lane & 15, lg = lane >> 4;
     f32x4 o[QT][DT];
@@ -85,11 +87,15 @@ __device__ __forceinline__ void attend_walk(unsigned char* lds, int n_tiles, flo
     for (int qs = 0; qs < QT; ++qs)
 #pragma unroll
         for (int st = 0; st < STEPS; ++st) qf[qs][st] = query(qs, st);
-    uint32_t vaddr[DT];
-    {
-        const int R0 = 4 * lg + (lq >> 2), p = lq & 3, swz = swz_v<DV>(R0);    // rows R0, R0 + 16, R0 + 32 share a swizzle
+    // waited for here: left to the loop, the wait for these loads would drain the DMA in flight in every tile
 #pragma unroll
-        for (int t = 0; t < DT; ++t) vaddr[t] = lds_addr_of(lds + R0 * VROW + (p & 1) * 8 + (((2 * t + (p >> 1)) ^ swz) * 16));
+    for (int qs = 0; qs < QT; ++qs)
+#pragma unroll
+        for (int st = 0; st < STEPS; ++st) asm volatile("" : "+v"(qf[qs][st]));
+    uint32_t vbase;                                  // of this lane's transposed reads; piece t of a row is an exclusive or away (swizzles are even)
+    {
+        const int R0 = 4 * lg + (lq >> 2), p = lq & 3;                         // rows R0, R0 + 16, R0 + 32 share a swizzle
+        vbase = lds_addr_of(lds + R0 * VROW + (p & 1) * 8 + (((p >> 1) ^ swz_v<DV>(R0)) * 16));
     }
     auto tile_body = [&](auto bufc, const int it) {
         constexpr int buf = decltype(bufc)::value;
@@ -140,7 +146,7 @@ __device__ __forceinline__ void attend_walk(unsigned char* lds, int n_tiles, flo
                 mx = max_xor16(mx);
                 mx = max_xor32(mx);
                 mx *= scale_log2;                                                  // (the host admits positive scales only)
-                const float m_new = max2(m[qs], mx);
+                const float m_new = moved_max(m[qs], mx);
                 const float m_use = m_new == -INFINITY ? 0.f : m_new;
                 float psum = 0.f;
 #pragma unroll
@@ -175,36 +181,38 @@ __device__ __forceinline__ void attend_walk(unsigned char* lds, int n_tiles, flo
                     p_hi[qs] = *reinterpret_cast<const bf16x8*>(&hraw);
                     p_lo[qs] = *reinterpret_cast<const bf16x8*>(&lraw);
                 }
-                u32x2 vlo[DT], vhi[DT];
-                if (hh == 0) {
+                constexpr int VB = DT < VBATCH ? DT : VBATCH;                      // pieces whose reads are in flight together
 #pragma unroll
-                    for (int t = 0; t < DT; ++t) {
-                        vlo[t] = ds_read_tr16<buf * VIMG>(vaddr[t]);
-                        vhi[t] = ds_read_tr16<buf * VIMG + 16 * VROW>(vaddr[t]);
+                for (int tb = 0; tb < DT; tb += VB) {
+                    u32x2 vlo[VB], vhi[VB];
+#pragma unroll
+                    for (int t = 0; t < VB; ++t) {
+                        const uint32_t at = vbase ^ ((tb + t) * 32);
+                        if (hh == 0) {
+                            vlo[t] = ds_read_tr16<buf * VIMG>(at);
+                            vhi[t] = ds_read_tr16<buf * VIMG + 16 * VROW>(at);
+                        } else {
+                            vlo[t] = ds_read_tr16<buf * VIMG + 32 * VROW>(at);
+                            vhi[t] = ds_read_tr16<buf * VIMG + 48 * VROW>(at);
+                        }
                     }
-                } else {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                    bf16x8 vf[VB];
 #pragma unroll
-                    for (int t = 0; t < DT; ++t) {
-                        vlo[t] = ds_read_tr16<buf * VIMG + 32 * VROW>(vaddr[t]);
-                        vhi[t] = ds_read_tr16<buf * VIMG + 48 * VROW>(vaddr[t]);
+                    for (int t = 0; t < VB; ++t) {
+                        const u32x4 raw = {vlo[t][0], vlo[t][1], vhi[t][0], vhi[t][1]};
+                        vf[t] = *reinterpret_cast<const bf16x8*>(&raw);
                     }
+#pragma unroll
+                    for (int t = 0; t < VB; ++t)
+#pragma unroll
+                        for (int qs = 0; qs < QT; ++qs) o[qs][tb + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], p_hi[qs], o[qs][tb + t], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < VB; ++t)
+#pragma unroll
+                        for (int qs = 0; qs < QT; ++qs) o[qs][tb + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], p_lo[qs], o[qs][tb + t], 0, 0, 0);
                 }
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-                bf16x8 vf[DT];
-#pragma unroll
-                for (int t = 0; t < DT; ++t) {
-                    const u32x4 raw = {vlo[t][0], vlo[t][1], vhi[t][0], vhi[t][1]};
-                    vf[t] = *reinterpret_cast<const bf16x8*>(&raw);
-                }
-#pragma unroll
-                for (int t = 0; t < DT; ++t)
-#pragma unroll
-                    for (int qs = 0; qs < QT; ++qs) o[qs][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], p_hi[qs], o[qs][t], 0, 0, 0);
-#pragma unroll
-                for (int t = 0; t < DT; ++t)
-#pragma unroll
-                    for (int qs = 0; qs < QT; ++qs) o[qs][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], p_lo[qs], o[qs][t], 0, 0, 0);
             }
         }
         lds_only_barrier();                                                    // everyone's reads of this buffer are done

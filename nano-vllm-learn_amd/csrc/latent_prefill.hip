@@ -15,7 +15,7 @@ template <int DK, int DV, int QT>
 __global__ __launch_bounds__(256, DK + DV <= 320 ? 2 : 1) void latent_prefill_kernel(const LatentPrefillArgs a) {
     using Images = TileImages<DK, DV>;
     constexpr int BM = 64 * QT, WR = 16 * QT, BN = Images::BN, KP = Images::KP, VP = Images::VP, NK = Images::NK, NV = Images::NV;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    extern __shared__ __attribute__((aligned(512))) unsigned char lds[];
     int qt, head, b;
     attend_unit(a.heads, qt, head, b);
     const int q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, k_beg = a.cu_k[b], sk = a.cu_k[b + 1] - k_beg;
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256, DK + DV <= 320 ? 2 : 1) void latent_prefill_ke
         }
         return *reinterpret_cast<const bf16x8*>(&raw);
     };
-    attend_walk<DK, DV, QT>(
+    attend_walk<DK, DV, QT, 4>(
         lds, n_tiles, a.scale_log2, -INFINITY, lane, stage, query, [&](int it) { return it * BN; }, [&](int kv0) { return kv0 <= wave_last_key; },
         [&](int kv0) { return kv0 + BN - 1 > wave_first_key || kv0 + BN > sk; },
         [&](int kv0, int qs, int off) { return off <= (my_q[qs] + shift < sk - 1 ? my_q[qs] + shift : sk - 1) - kv0 - 4 * lg; },

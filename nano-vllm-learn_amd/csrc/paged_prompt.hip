@@ -9,11 +9,11 @@ namespace nvh {
 
 namespace {
 
-template <int DK, int DV, int QT>
-__global__ __launch_bounds__(256, DK + DV <= 320 ? 2 : 1) void paged_prompt_kernel(const PagedAttendArgs a) {
-    using Images = TileImages<DK, DV>;
-    constexpr int BM = 64 * QT, WR = 16 * QT, BN = Images::BN, KP = Images::KP, VP = Images::VP, NK = Images::NK, NV = Images::NV;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+template <int DK, int DV, int QT, int WV>
+__global__ __launch_bounds__(64 * WV, WV == 8 ? 4 : DK + DV <= 320 ? 2 : 1) void paged_prompt_kernel(const PagedAttendArgs a) {
+    using Images = TileImages<DK, DV, WV>;
+    constexpr int BM = 16 * WV * QT, WR = 16 * QT, BN = Images::BN, KP = Images::KP, VP = Images::VP, NK = Images::NK, NV = Images::NV;
+    extern __shared__ __attribute__((aligned(512))) unsigned char lds[];
     int qt, head, b;
     attend_unit(a.heads, qt, head, b);
     const int q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, sk = a.cu_k[b + 1] - a.cu_k[b];
@@ -31,33 +31,43 @@ __global__ __launch_bounds__(256, DK + DV <= 320 ? 2 : 1) void paged_prompt_kern
     // ---- staging: this lane's piece of each DMA instruction: row of the tile and offset inside it
     const uint16_t* cache = reinterpret_cast<const uint16_t*>(a.cache) + (int64_t)g * a.block_size * (DK + DV);
     const int64_t page_elems = (int64_t)a.kv_heads * a.block_size * (DK + DV);
-    const int32_t* table = a.block_tables + (int64_t)b * a.bt_stride;
-    int kr[NK], kc[NK], vr[NV], vc[NV];
+    PageNumbers pages{a.block_tables + (int64_t)b * a.bt_stride, (sk - 1) / a.block_size};
+    uint32_t koff[NK], voff[NV];                     // of a full tile, in bytes from its first row
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
         const int s = (wave * NK + j) * 64 + lane, R = s / KP;
-        kr[j] = R;
-        kc[j] = ((s - R * KP) ^ swz_k<DK>(R)) * 8;
+        koff[j] = (R * DK + ((s - R * KP) ^ swz_k<DK>(R)) * 8) * 2;
     }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const int s = (wave * NV + j) * 64 + lane, R = s / VP;
-        vr[j] = R;
-        vc[j] = ((s - R * VP) ^ swz_v<DV>(R)) * 8;
+        voff[j] = (R * DV + ((s - R * VP) ^ swz_v<DV>(R)) * 8) * 2;
     }
-    auto page_of = [&](int it) { return it < n_tiles ? table[vis.tile(it) * BN / a.block_size] : 0; };
-    int page = page_of(0);                           // of the tile that is staged next
-    auto stage = [&](int it, int buf) {
+    auto stage = [&](int it, int buf) __attribute__((always_inline)) {
         unsigned char* kimg = Images::k(lds, buf);
         unsigned char* vimg = Images::v(lds, buf);
-        const int kv0 = vis.tile(it) * BN, off = kv0 % a.block_size, live = sk - kv0 < BN ? sk - kv0 : BN;
-        const uint16_t* kb = cache + page * page_elems + (int64_t)off * DK;
-        const uint16_t* vb = cache + page * page_elems + (int64_t)a.block_size * DK + (int64_t)off * DV;
+        const int kv0 = vis.tile(it) * BN, page = kv0 / a.block_size, off = kv0 - page * a.block_size, live = sk - kv0 < BN ? sk - kv0 : BN;
+        const uint16_t* head = cache + pages.at(page, lane) * page_elems;
+        const char* kb = reinterpret_cast<const char*>(head + (int64_t)off * DK);
+        const char* vb = reinterpret_cast<const char*>(head + (int64_t)a.block_size * DK + (int64_t)off * DV);
 #pragma unroll
-        for (int j = 0; j < NK; ++j) dma16(kb + (kr[j] < live ? kr[j] : live - 1) * DK + kc[j], kimg + (wave * NK + j) * 1024);   // rows past the end repeat the last key: masked
+        for (int j = 0; j < NK; ++j) {
+            uint32_t at = koff[j];
+            if (live < BN) {                         // rows past the end repeat the last key: masked
+                const int s = (wave * NK + j) * 64 + lane, R = s / KP;
+                at = ((R < live ? R : live - 1) * DK + ((s - R * KP) ^ swz_k<DK>(R)) * 8) * 2;
+            }
+            dma16(kb + at, kimg + (wave * NK + j) * 1024);
+        }
 #pragma unroll
-        for (int j = 0; j < NV; ++j) dma16(vb + (vr[j] < live ? vr[j] : live - 1) * DV + vc[j], vimg + (wave * NV + j) * 1024);
-        page = page_of(it + 1);
+        for (int j = 0; j < NV; ++j) {
+            uint32_t at = voff[j];
+            if (live < BN) {
+                const int s = (wave * NV + j) * 64 + lane, R = s / VP;
+                at = ((R < live ? R : live - 1) * DV + ((s - R * VP) ^ swz_v<DV>(R)) * 8) * 2;
+            }
+            dma16(vb + at, vimg + (wave * NV + j) * 1024);
+        }
     };
     int my_q[QT], lo[QT];
     bool q_ok[QT];
@@ -69,7 +79,7 @@ __global__ __launch_bounds__(256, DK + DV <= 320 ? 2 : 1) void paged_prompt_kern
         lo[qs] = first_seen(my_q[qs] + shift, a.window, a.chunk);
         qp[qs] = reinterpret_cast<const uint16_t*>(a.q) + (int64_t)(q_beg + (q_ok[qs] ? my_q[qs] : sq - 1)) * a.q_stride + (int64_t)head * DK + lg * 8;
     }
-    attend_walk<DK, DV, QT>(
+    attend_walk<DK, DV, QT, WV>(
         lds, n_tiles, a.scale * kLog2e, a.sink ? a.sink[head] * kLog2e : -INFINITY, lane, stage,
         [&](int qs, int st) { return *reinterpret_cast<const bf16x8*>(qp[qs] + st * 32); }, [&](int it) { return vis.tile(it) * BN; },
         [&](int kv0) { return kv0 <= wave_last && (kv0 + BN > lo_first || kv0 < a.keep_first); },
@@ -82,19 +92,24 @@ __global__ __launch_bounds__(256, DK + DV <= 320 ? 2 : 1) void paged_prompt_kern
         [&](int qs, int d, f32x4 v) { return a.o_cos_sin ? turn_back(v, a.o_cos_sin, my_q[qs] + shift, a.max_position, a.o_rot, d) : v; });
 }
 
-template <int DK, int DV, int QT>
+template <int DK, int DV, int QT, int WV>
 int launch_one(const PagedAttendArgs& a, hipStream_t stream) {
-    constexpr size_t lds = TileImages<DK, DV>::BYTES;
-    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paged_prompt_kernel<DK, DV, QT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    paged_prompt_kernel<DK, DV, QT><<<dim3(a.heads, a.batch, (a.max_q + 64 * QT - 1) / (64 * QT)), 256, lds, stream>>>(a);
+    constexpr size_t lds = TileImages<DK, DV, WV>::BYTES;
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paged_prompt_kernel<DK, DV, QT, WV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    paged_prompt_kernel<DK, DV, QT, WV><<<dim3(a.heads, a.batch, (a.max_q + 16 * WV * QT - 1) / (16 * WV * QT)), 64 * WV, lds, stream>>>(a);
     return check_launch("paged_attend_prompt");
 }
 template <int DK, int DV>
 int launch_dims(const PagedAttendArgs& a, hipStream_t stream) {
     if constexpr (DV <= 128) {
-        if (a.max_q > 256) return launch_one<DK, DV, 2>(a, stream);
+        // 128 rows per workgroup.  Two sub-tiles per wave read a key or value fragment for 32 queries; where that leaves two waves on a SIMD (192 registers and more),
+        // eight waves of one sub-tile, four on a SIMD, fill each other's waits better.  14 sequences of 1170 tokens, 16 heads of 128 / 128: 183 us against
+        // 191, one of 2000 62 against 72; of 192 / 64: 166 and 62 against 171 and 70; but of 128 / 64 (three waves on a SIMD either way) 145 against 125,
+        // and of 192 / 128 and wider, where one sub-tile does not fit 128 registers, 236 against 213.
+        constexpr bool eight = DK + 2 * DV >= 320 && DK + DV <= 256;
+        if (a.max_q > 256) return launch_one<DK, DV, eight ? 1 : 2, eight ? 8 : 4>(a, stream);
     }
-    return launch_one<DK, DV, 1>(a, stream);
+    return launch_one<DK, DV, 1, 4>(a, stream);
 }
 
 }  // namespace

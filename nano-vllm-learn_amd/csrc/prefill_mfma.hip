@@ -218,14 +218,15 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         koff[j] = (uint32_t)(R * kstride + (dp ^ chunk_swz<LPT>(R)) * 8);
         voff[j] = (uint32_t)(R * vstride + (dp ^ chunk_swz_v<LPT>(R)) * 8);
     }
-    auto stage = [&](int tile, int buf, const bool do_k = true, const bool do_v = true) {
+    PageNumbers pages{PAGED ? a.block_tables + (int64_t)b * a.bt_row_stride : nullptr, PAGED ? (sk - 1) / a.block_size : 0};
+    auto stage = [&](int tile, int buf, const bool do_k = true, const bool do_v = true) __attribute__((always_inline)) {
         unsigned char* kimg = lds + buf * 2 * IMG;
         unsigned char* vimg = kimg + IMG;
         const int kv0 = tile * BN;
         const uint16_t *kb, *vb;                     // wave-uniform bases of the tile's first key row, this kv head
         if constexpr (PAGED) {                       // BN divides block_size: one block per tile
             const int blk = kv0 / a.block_size;
-            const int bid = a.block_tables[(int64_t)b * a.bt_row_stride + blk];
+            const int bid = pages.at(blk, lane);
             const int64_t base = (((int64_t)bid * a.block_size + (kv0 - blk * a.block_size)) * a.kvh + kh) * D;
             kb = a.k + base;
             vb = a.v + base;
@@ -293,6 +294,11 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
             qf[qs][st] = *reinterpret_cast<const bf16x8*>(&raw);
         }
     }
+    // waited for here: left to the loop, the wait for these loads would drain the DMA in flight in every tile
+#pragma unroll
+    for (int qs = 0; qs < QT; ++qs)
+#pragma unroll
+        for (int st = 0; st < STEPS; ++st) asm volatile("" : "+v"(qf[qs][st]));
     PF_STAMP(0);
     // tr-read: lane 4q+p of its group addresses key row q, dims 4p..4p+3.  The per-lane part of the address (row 4*lg+q,
     // swizzled chunk of dim tile t) is loop invariant: DT registers; buffer, image, 32-key half and the +16-row partner are
@@ -375,7 +381,7 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
                 mx = max_xor16(mx);
                 mx = max_xor32(mx);
                 mx *= a.scale_log2;                                              // scale > 0: max commutes with the scaling
-                const float m_new = max2(m_run[qs], mx);
+                const float m_new = moved_max(m_run[qs], mx);
                 // rows that have seen no key yet keep m = -inf; use 0 as the reference point so exp2 stays finite
                 const float m_use = m_new == -INFINITY ? 0.f : m_new;
                 // scale-and-subtract and the row sum on element pairs (plain fp32 instructions: packed ones are switched off in the build), exp2 per element
@@ -726,7 +732,7 @@ void prefill_short_kernel(const PrefillArgs a) {
             mx = max_xor16(mx);
             mx = max_xor32(mx);
             mx *= a.scale_log2;
-            const float m_new = max2(m_run, mx);
+            const float m_new = moved_max(m_run, mx);
             const float m_use = m_new == -INFINITY ? 0.f : m_new;                // rows that have seen no key yet
             const f32x2 sc2 = {a.scale_log2, a.scale_log2}, mm2 = {-m_use, -m_use};
             f32x2 psum2 = {0.f, 0.f};

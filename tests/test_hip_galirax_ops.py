@@ -115,6 +115,25 @@ def test_prompt(heads, kvh, dim, vdim, window, keep):
             at += r
 
 
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128), (192, 64)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (70, 0), (300, 70)])
+def test_prompt_over_many_pages(window, keep, dim, vdim):
+    """More than 64 pages of a sequence, with kept ones behind which the window starts in another group of 64; scores that rise from tile to tile, by less
+    and by more than what moves the reference point of the softmax."""
+    from nanovllm_hip import ops
+    heads, kvh, rows, keys = 4, 2, 300, 65 * 64 + 40
+    pg = Pages([keys], kvh, dim, vdim, BF16, seed=3)
+    q = randn(1, kvh, dim, seed=8).repeat_interleave(heads // kvh, dim=1).expand(rows, -1, -1).contiguous()
+    steps = (torch.arange(keys) // 64).float()
+    for slope in (0.5, 20.0):                        # of the score, per tile, in units of the softmax's exponent
+        pg.k[0] = ((0.05 * randn(keys, kvh, dim, seed=9, dtype=F32)) + (slope * steps[:, None] / (0.2 * (q[0, ::heads // kvh].float() ** 2).sum(-1)))[..., None]
+                   * q[0, ::heads // kvh].float()).bfloat16()
+        cu = lambda n: torch.tensor([0, n], dtype=torch.int32).cuda()
+        got = pg.unpad(ops.paged_attend_prompt(pg.pad_q(q), pg.cache(), pg.tables.cuda(), cu(rows), cu(keys), rows, heads, kvh, pg.dk, pg.dv, 0.2, window, keep), heads)
+        for t in (0, 1, 23, 24, 128, 299):
+            close(got[t], attend_ref(q[t], pg.k[0], pg.v[0], keys - rows + t, 0.2, window, keep, None), BF16, f"slope {slope} row {t}")
+
+
 @pytest.mark.parametrize("window,keep", [(0, 0), (64, 0), (65, 1), (130, 4), (40, 70)])
 @pytest.mark.parametrize("portion", [2, 40, 200])
 def test_prompt_one_key_stands_out(window, keep, portion):

@@ -319,6 +319,30 @@ def test_paged_prefill_prefix_cache_vs_oracle(ops):
     check_close(o32.cpu().numpy(), o16.float().cpu().numpy(), exp, "paged prefill")
 
 
+@pytest.mark.parametrize("D,sq", [(64, 40), (128, 140)])
+@pytest.mark.parametrize("slope", [0.5, 20.0])
+def test_paged_prefill_over_many_pages(ops, D, sq, slope):
+    """More than 64 pages of a sequence; scores that rise from 64 keys to the next by less and by more than what moves the softmax's reference point."""
+    H, KVH, bs, sk = 4, 2, 64, 65 * 64 + 40
+    nb = (sk + bs - 1) // bs
+    bt = np.zeros((1, nb), np.int32)
+    bt[0] = np.random.default_rng(5).permutation(nb)
+    gen = torch.Generator().manual_seed(6)
+    q1 = torch.randn(1, KVH, D, generator=gen).bfloat16()
+    q = q1.repeat_interleave(H // KVH, 1).expand(sq, -1, -1).contiguous()
+    rise = slope * (torch.arange(sk) // 64)[:, None] / ((q1[0].float() ** 2).sum(-1) * D ** -0.5)
+    k = (rise[..., None] * q1.float() + 0.1 * torch.randn(sk, KVH, D, generator=gen)).bfloat16()
+    v = torch.randn(sk, KVH, D, generator=gen).bfloat16()
+    kc, vc = torch.zeros(nb, bs, KVH, D).bfloat16(), torch.zeros(nb, bs, KVH, D).bfloat16()
+    for t in range(sk):
+        kc[bt[0, t // bs], t % bs], vc[bt[0, t // bs], t % bs] = k[t], v[t]
+    cu_q, cu_k = np.array([0, sq], np.int32), np.array([0, sk], np.int32)
+    exp = O.paged_prefill(q.float().numpy(), kc.float().numpy(), vc.float().numpy(), cu_q, cu_k, bt)
+    o32, o16 = [ops.flash_attn_varlen_func(q.cuda(), kc.cuda(), vc.cuda(), sq, dev_i32(cu_q), sk, dev_i32(cu_k), block_table=dev_i32(bt), out_dtype=t)
+                for t in (torch.float32, torch.bfloat16)]
+    check_close(o32.cpu().numpy(), o16.float().cpu().numpy(), exp, f"slope {slope}")
+
+
 def test_chunked_prefill_equals_one_shot(ops):
     """SURVEY §8f row 4 (chunked prefill): a prompt prefilled in chunks — each chunk's K/V stored into the paged cache
     (store_kvcache), its queries attending to the cache so far (paged prefill, Sq < Sk, bottom-right causal mask) — gives the

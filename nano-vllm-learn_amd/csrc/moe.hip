@@ -310,7 +310,9 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
     const int expert = a.tiles[4 * mt], first = a.tiles[4 * mt + 1], live = a.tiles[4 * mt + 2];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4, wm = wave / NW, wn = wave % NW;
     const uint16_t* w = reinterpret_cast<const uint16_t*>(a.w) + (int64_t)expert * (GLU ? 2 : 1) * a.n * a.k;
-    auto swz = [](int r) { return (r >> 2) & 3; };   // 16-byte pieces of a row are xor-ed: 16 rows read at one column spread over all banks
+    // 16-byte pieces of a row are xor-ed with 0, 2, 3, 1 for rows 0-3, 4-7, 8-11, 12-15: a 16-byte read takes lanes 0-3, 12-15 and 20-27 of 32 in one cycle, the others
+    // in the next, and either set of 16 (8 rows at one column, the 8 other rows at the next one) then spreads over all banks
+    auto swz = [](int r) { return (0x78 >> ((r >> 1) & 6)) & 3; };
     // this lane's piece of each DMA instruction: 16 rows of 64 bytes
     const uint16_t* src[DMA];
 #pragma unroll
@@ -325,7 +327,9 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
             src[j] = reinterpret_cast<const uint16_t*>(a.x) + (GLU ? (int64_t)(pair / a.top) * a.x_stride : (int64_t)pair * a.k) + piece;
         }
     }
+    const bool feeds = wave * DMA * 16 < TN + live;  // a wave whose pieces are of pairs that do not exist leaves them out (weights come first)
     auto stage = [&](int it, int buf) {
+        if (!feeds) return;
 #pragma unroll
         for (int j = 0; j < DMA; ++j) dma16(src[j] + it * TK, lds + buf * G::IMG + (wave * DMA + j) * 1024);
     };
@@ -339,61 +343,79 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
     auto stage_next = [&](int it) { stage(it < iters ? it : iters - 1, it % kRing); };
 #pragma unroll
     for (int it = 0; it < kRing; ++it) stage_next(it);
-    struct Operands {
-        bf16x8 w[NT], x[MT];
-    };
-    Operands even, odd;                              // of the image being multiplied and of the next one, read meanwhile
-    auto read = [&](int it, Operands& f) {
-        const int at = (it % kRing) * G::IMG + lq * 64 + (lg ^ swz(lq)) * 16;
-        const unsigned char* wimg = lds + at + wn * NT * 16 * 64;
-        const unsigned char* ximg = lds + at + (TN + wm * MT * 16) * 64;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) f.w[t] = *reinterpret_cast<const bf16x8*>(wimg + t * 16 * 64);
-#pragma unroll
-        for (int t = 0; t < MT; ++t) f.x[t] = *reinterpret_cast<const bf16x8*>(ximg + t * 16 * 64);
-    };
     // the oldest image in flight has landed (`younger` behind it), and everyone has read the one before it
     auto arrive = [&](auto younger) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(younger)::value * DMA) : "memory");
         lds_only_barrier();
     };
-    // reads and loads spread between the products
-    auto spread = [] {
+    constexpr std::integral_constant<int, kRing - 2> in_flight{};
+    // the products of this wave's first MTU tiles of pairs
+    auto run = [&](auto mtu) __attribute__((always_inline)) {
+        constexpr int MTU = decltype(mtu)::value;
+        struct Operands {
+            bf16x8 w[NT], x[MTU];
+        };
+        Operands even, odd;                          // of the image being multiplied and of the next one, read meanwhile
+        auto read = [&](int it, Operands& f) __attribute__((always_inline)) {
+            const int at = (it % kRing) * G::IMG + lq * 64 + (lg ^ swz(lq)) * 16;
+            const unsigned char* wimg = lds + at + wn * NT * 16 * 64;
+            const unsigned char* ximg = lds + at + (TN + wm * MT * 16) * 64;
 #pragma unroll
-        for (int k = 0; k < NT + MT; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                 // LDS read
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                 // MFMA
+            for (int t = 0; t < NT; ++t) f.w[t] = *reinterpret_cast<const bf16x8*>(wimg + t * 16 * 64);
+#pragma unroll
+            for (int t = 0; t < MTU; ++t) f.x[t] = *reinterpret_cast<const bf16x8*>(ximg + t * 16 * 64);
+        };
+        // reads and loads spread between the products
+        auto spread = []() __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < NT + MTU; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);             // LDS read
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA
+            }
+#pragma unroll
+            for (int k = 0; k < DMA; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);             // load
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            }
+        };
+        auto multiply = [&](const Operands& f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < MTU; ++j)
+#pragma unroll
+                for (int i = 0; i < NT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[i], f.x[j], acc[i][j], 0, 0, 0);
+        };
+        read(0, even);
+        for (int it = 0; it < iters; it += 2) {
+            arrive(in_flight);
+            read(it + 1, odd);
+            stage_next(it + kRing);
+            multiply(even);
+            spread();
+            arrive(in_flight);
+            read(it + 2, even);                      // (behind the last image: read and not used)
+            stage_next(it + 1 + kRing);
+            multiply(odd);
+            spread();
         }
-#pragma unroll
-        for (int k = 0; k < DMA; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);                 // load
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        }
-    };
-    auto multiply = [&](const Operands& f) {
-#pragma unroll
-        for (int j = 0; j < MT; ++j)
-#pragma unroll
-            for (int i = 0; i < NT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[i], f.x[j], acc[i][j], 0, 0, 0);
     };
     arrive(std::integral_constant<int, kRing - 1>{});
-    read(0, even);
-    constexpr std::integral_constant<int, kRing - 2> in_flight{};
-    for (int it = 0; it < iters; it += 2) {
-        arrive(in_flight);
-        read(it + 1, odd);
-        stage_next(it + kRing);
-        multiply(even);
-        spread();
-        arrive(in_flight);
-        read(it + 2, even);                          // (behind the last image: read and not used)
-        stage_next(it + 1 + kRing);
-        multiply(odd);
-        spread();
+    // Rows of pairs that do not exist are not multiplied, in steps of half a wave's rows: the waves beside get the matrix cores.  (100 tokens' pairs in tiles of 256:
+    // 207 -> 179 us; in tiles of 128: 167 -> 160; of 16384 tokens, 8 tiles of 256 an expert: 1367 -> 1340.)
+    const int mine = live - wm * MT * 16;            // pairs from this wave's first one on
+    if (mine > MT * 8) {
+        run(std::integral_constant<int, MT>{});
+    } else if (mine > 0) {
+        run(std::integral_constant<int, MT / 2>{});
+    } else {
+        for (int it = 0; it < iters; ++it) {
+            arrive(in_flight);
+            stage_next(it + kRing);
+        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // ---- results through LDS (the images are done with): a wave's MT * 16 pairs by CW columns, then whole rows of them to memory
     lds_only_barrier();
+    if (mine <= 0) return;
     constexpr int CW = GLU ? NT * 8 : NT * 16, CP = CW / 8;                    // columns of a wave, 16-byte pieces of a row
     unsigned char* tile = lds + wave * MT * 16 * CW * 2;
     auto put = [&](int r, int col, f32x4 v) {        // columns col .. + 3 of row r
@@ -634,7 +656,14 @@ int launch_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, con
     return check_launch("moe_scatter");
 }
 
-int moe_tile_rows(int pairs, int experts, int f32) { return f32 ? FM : pairs / experts >= 256 ? 256 : 128; }
+// Rows of a tile.  From 256 pairs an expert on, 256: twice the products per byte of weights and rows read.  From 100 to 192 too: an expert's pairs mostly fit one tile, whose
+// missing rows cost little, where many take two of 128.  2048 wide, 32 experts of 1536, softmax router: 125 pairs an expert 203 us against 254, 187
+// 234 against 268; 1024 wide, 187: 88 against 96.  Below, 128: 75 pairs 197 both (1024 wide 72 against 68); in between many an expert needs a second tile of 256: 250 pairs
+// 321 against 319 (1024 wide 122 against 109).
+int moe_tile_rows(int pairs, int experts, int f32) {
+    const int mean = pairs / experts;
+    return f32 ? FM : mean >= 256 || (mean >= 100 && mean <= 192) ? 256 : 128;
+}
 
 int launch_moe_gemm(const MoeGemmArgs& a, int f32, hipStream_t stream) {
     if (f32) {

@@ -416,6 +416,26 @@ def test_expert_products(rows, top, experts, n, k, dtype):
                 close(out[p.cuda()], f64(act)[p] @ f64(dn[e]).T, dtype, f"out {e}", slack=2)
 
 
+@pytest.mark.parametrize("tile", [128, 256])
+def test_expert_tiles_that_are_not_full(tile):
+    """Experts whose last tile ends on, in front of and behind what a wave multiplies and half of it; columns that end inside a tile."""
+    from nanovllm_hip import ops
+    counts, n, k = [1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 0, 191, 192, 193, 255, 256, 257], 192, 128
+    flat = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))[torch.randperm(sum(counts), generator=torch.Generator().manual_seed(1))]
+    ids = flat.int()[:, None]
+    x = randn(len(flat), k, seed=1)
+    gu, dn = randn(len(counts), 2 * n, k, seed=2, scale=k ** -0.5), randn(len(counts), k, n, seed=3, scale=n ** -0.5)
+    dispatch = ops.moe_dispatch(ids.cuda(), len(counts), BF16, tile)
+    act = ops.moe_gemm(x.cuda(), gu.cuda(), ids.cuda(), True, dispatch)
+    out = ops.moe_gemm(act, dn.cuda(), ids.cuda(), False, dispatch)
+    for e in range(len(counts)):
+        p = (flat == e).nonzero().flatten()
+        if len(p):
+            want = G.silu(f64(x)[p] @ f64(gu[e, :n]).T) * (f64(x)[p] @ f64(gu[e, n:]).T)
+            close(act[p.cuda()], want, BF16, f"act {e}", slack=2)
+            close(out[p.cuda()], f64(act)[p] @ f64(dn[e]).T, BF16, f"out {e}", slack=2)
+
+
 # ------------------------------------------------------------------------------------------------ residual, norm, cap
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,cols,n,top", [(3, 64, 64, 0), (5, 320, 300, 4), (17, 2048, 2048, 8), (2, 8192, 8190, 3)])

@@ -224,7 +224,7 @@ def galirax_kernels(size, batch=32, ctx=1536, seqs=16, prompt=1024):
     slots = torch.arange(max(seqs, batch), dtype=torch.int32, device="cuda")
     state = torch.zeros(max(seqs, batch), h, d, d, device="cuda")
     o = torch.empty(rows, h * d, device="cuda", dtype=torch.bfloat16)
-    seg = choose_segment([prompt] * seqs, h * 2)
+    seg = choose_segment([prompt] * seqs, h)
     chunks = torch.tensor([c for i in range(seqs) for c in recurrence_chunks(i * prompt, prompt, i, seg)], dtype=torch.int32, device="cuda")
     us = _time([lambda a=a: ops.lightning_chunks(a, decay, pos, slots, chunks, seg < prompt, state, out=o) for a in x] * 2)
     out["lightning_chunks"] = _line(us, rows * 8 * h * d, 4 * rows * h * d * d)
@@ -493,7 +493,7 @@ def zaposun_kernels(size, batch=32, ctx=1536, seqs=16, prompt=1024):
     p = dict(w0=torch.rand(width, device="cuda") * 5 - 6, u=_randn(width, dtype=f32), norm=one, w2=_randn(width, 64) * 0.05)
     o = torch.empty(rows, width, device="cuda", dtype=torch.bfloat16)
     state = torch.zeros(max(seqs, batch), hw, 64, 64, device="cuda")
-    chunks, more = segments(hw)
+    chunks, more = segments(max(1, hw // 2))
     us = _time([lambda a=a: ops.wkv_chunks(*a, p, 1e-6, 64, pos, slots, chunks, more, state, out=o) for a in x] * 2)
     out["wkv_chunks"] = _line(us, rows * 12 * width, 4 * rows * width * 64)
     x1 = [_randn(batch, width) for _ in range(4)]
@@ -505,7 +505,7 @@ def zaposun_kernels(size, batch=32, ctx=1536, seqs=16, prompt=1024):
     x = [_randn(rows, 4 * h * d) for _ in range(2)]
     decay, state = torch.linspace(0.8, 0.999, h, device="cuda"), torch.zeros(max(seqs, batch), h, d, d, device="cuda")
     o = torch.empty(rows, h * d, device="cuda", dtype=torch.bfloat16)
-    chunks, more = segments(h * 2)
+    chunks, more = segments(h)
     us = _time([lambda a=a: ops.lightning_chunks(a, decay, pos, slots, chunks, more, state, out=o) for a in x] * 2)
     out["galirax lightning_chunks"] = _line(us, rows * 8 * h * d, 4 * rows * h * d * d)
     x1 = _randn(batch, 4 * h * d)
@@ -523,7 +523,7 @@ def zaposun_kernels(size, batch=32, ctx=1536, seqs=16, prompt=1024):
     p = dict(a_log2=-torch.rand(inner, STATES, device="cuda") * 4, d=torch.ones(inner, device="cuda"), dt_bias=torch.rand(inner, device="cuda") * 4 - 5, w_dt=_randn(inner, (rank + 63) // 64 * 64) * 0.1)
     o = torch.empty(rows, inner, device="cuda", dtype=torch.bfloat16)
     state = torch.zeros(max(seqs, batch), inner, STATES, device="cuda")
-    chunks, more = segments(inner // 192)
+    chunks, more = segments(inner // 256)
     us = _time([lambda a=a: ops.scan_chunks(a[:, :inner], dt, bc, a[:, inner:], p, pos, slots, chunks, more, state, out=o) for a in xz] * 2)
     out["scan_chunks"] = _line(us, rows * inner * 8)
     x1, low, bc1 = _randn(batch, 2 * inner), _randn(batch, p["w_dt"].shape[1]), _randn(batch, 64)

@@ -15,20 +15,34 @@ from .linear import linear, padded, round_up
 CUS = 256                     # compute units of an MI355X: one walking workgroup keeps one busy
 
 
-SEGMENT_OVERHEAD = 0.8        # start of a walk (gate weights into registers, first rows) in units of one 64-token step
+SEGMENT_OVERHEAD = 1.2        # start of a walk (gate weights into registers, first rows) in units of one 64-token step
+SPLIT_OVERHEAD = 3.0          # two launches more, the states of segments written and read
 SUMMARY_SHARE = 0.7           # a summary walk's step against a full one's
+LATE_SHARE = 0.7              # of a longest walk that still runs alone when the others are done
 
 
 def choose_segment(portions, blocks, chunk=64):
-    """Tokens per segment for portions of these lengths: one workgroup walks one (segment, diagonal block), and cutting a portion into more than one
-    costs a summary walk over all its segments but the last.  Returns the cheapest multiple of `chunk` among about ten per octave of lengths."""
+    """Tokens per segment for portions of these lengths: `blocks` workgroups walk each segment, and cutting a portion into more than one
+    costs a summary walk over all its segments but the last.  Returns the cheapest multiple of `chunk` among about ten per octave of lengths.
+
+    Walks of different lengths share the CUs: beyond one a CU, the launch takes as long as the even load and most of a longest walk, or as so many rounds
+    of longest walks, whichever is less.  (Counted in rounds alone, forty prompts of 6 to 13 steps were cut up: whole, lightning attention takes them in 67 us against
+    117, the scan in 214 against 308.)  Over ten mixes of 1 to 40 sequences the choice costs 1.03 times the best segment's walks for lightning attention, time mixing and
+    the gated recurrence, 1.07 for the scan; counted in rounds 1.16, 1.10, 1.11 and 1.14."""
     longest = max(portions, default=1)
-    last = -(-longest // chunk)
+    last, total = -(-longest // chunk), sum(portions) / chunk
+
+    def launch(walks, steps, k):                     # `walks` of at most k steps each, `steps` in all
+        if walks * blocks <= CUS:
+            return k + SEGMENT_OVERHEAD
+        rounds, load = -(-walks * blocks // CUS), (steps + walks * SEGMENT_OVERHEAD) * blocks / CUS
+        return min(rounds * (k + SEGMENT_OVERHEAD), load + LATE_SHARE * (k + SEGMENT_OVERHEAD))
 
     def cost(k):
-        pieces = [-(-n // (k * chunk)) for n in portions]
-        walk, summary = -(-sum(pieces) * blocks // CUS), -(-sum(p - 1 for p in pieces) * blocks // CUS)
-        return (walk + SUMMARY_SHARE * summary) * (min(k, last) + SEGMENT_OVERHEAD)
+        walks = sum(-(-n // (k * chunk)) for n in portions)
+        ahead = walks - len(portions)                # segments in front of others
+        walk = launch(walks, total, min(k, last))
+        return walk + SPLIT_OVERHEAD + SUMMARY_SHARE * launch(ahead, ahead * k, k) if ahead else walk
     steps, k = [last], 1
     while k < last:
         steps.append(k)

@@ -16,7 +16,8 @@ MIXES = ("r", "k", "v", "g", "w")
 
 class TimeMixing(nn.Module):
     mixes = MIXES
-    segment_units = property(lambda self: self.heads)        # workgroups that walk one segment
+    # what choose_segment takes for workgroups that walk one segment: it counts one per CU, and two of these (a head each) share one
+    segment_units = property(lambda self: max(1, self.heads // 2))
 
     def __init__(self, in_width, in_cols, heads, dim, eps, dtype):
         super().__init__()

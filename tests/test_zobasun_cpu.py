@@ -192,6 +192,16 @@ def test_segment_choice():
     assert all(choose_segment([n] * m, b) % 64 == 0 for n in (63, 65, 1000, 30000) for m in (1, 7) for b in (1, 10))
 
 
+@pytest.mark.parametrize("portions,blocks,whole", [([400 + 11 * i for i in range(40)], 8, True), ([512] * 32, 8, True), ([1170] * 14, 16, True), ([4096, 2000, 3000], 8, False),
+                                                   ([4096] + [64] * 40, 4, False)])
+def test_segments_of_uneven_portions(portions, blocks, whole):
+    """More walks than compute units stay whole where their even load fills the GPU; a few long portions are cut, also among many short ones."""
+    from nanovllm_hip.layers.rglru import choose_segment
+    segment = choose_segment(portions, blocks)
+    assert segment % 64 == 0 and (segment >= max(portions)) == whole
+
+
+
 # ------------------------------------------------------------------------------------------------ scheduler
 def _scheduler(blocks, slots=4, mixed=True, **kw):
     from nanovllm_hip.engine.block_manager import BlockManager, StateSlots

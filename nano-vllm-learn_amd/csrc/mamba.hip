@@ -11,8 +11,8 @@
 // once for all of them.
 // Per (token, channel, state): one transcendental and four vector instructions: issue-bound, not HBM-bound.  So the walk is written for few instructions and no
 // waits: every load is unconditional (rows past the end repeat the last one; a load behind a branch makes the compiler wait for all of them), dt comes without
-// division and without a branch, and up to 16 states B and C stay in the activation type in LDS, one 16-byte read per token.  Channels run fastest over the grid,
-// or whole segments of different lengths fall on single XCDs.  16384 tokens of 16 sequences, 4096 channels of 16 states: 613 -> 409 us as whole portions.
+// division and without a branch, and no branch parts the tokens of a tile, so that the operands of eight are read from LDS ahead of their arithmetic.
+// Channels run fastest over the grid, or whole segments of different lengths fall on single XCDs.  16384 tokens of 16 sequences, 4096 channels of 16 states: 613 -> 316 us as whole portions.
 // A sequence's first token (position 0) takes the state as zero instead of reading it: slots need no clearing when reused.
 #include <type_traits>
 
@@ -85,9 +85,9 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
     constexpr int NP = NS * NL, CHN = 256 / NL, TT = min3(TILE / CHN, 64, 4096 / NP), PIECES = TT * CHN / 8;        // (PIECES <= 256)
     constexpr int BCP = (TT * 2 * NP / 8 + 255) / 256, U = NS < 8 ? NS : 8;    // pieces of B | C per thread; states of a lane a piece holds
     __shared__ __attribute__((aligned(16))) float dt_s[TT * CHN], dx_s[TT * CHN], y_s[SUMMARY ? 8 : TT * CHN];
-    // B and C in LDS: widened on every read where a lane has few states to do it for (16 sequences of 512 tokens, 4096 channels: 190 us against 213 at 16 states),
-    // once on the way in at 32 and 64 (242 against 296, 414 against 494); beyond that the wider rows' bank conflicts cost more than widening (928 against 1021)
-    using L = typename std::conditional<NP == 32 || NP == 64, float, T>::type;
+    // B and C in LDS: widened once on the way in up to 64 states (16 sequences of 512 tokens, 4096 channels: 157 us against 177 at 16 states, 242 against 296 at 32,
+    // 414 against 494 at 64); beyond that the wider rows' bank conflicts cost more than widening on every read (1021 against 928 at 128)
+    using L = typename std::conditional<NP <= 64, float, T>::type;
     __shared__ __attribute__((aligned(16))) L bc_s[TT * 2 * NP];
     const int seg = blockIdx.y + blockIdx.z * gridDim.y;         // channels run fastest: workgroups are dealt round-robin over the XCDs, and segments differ in length
     if (seg >= a.n_chunks) return;
@@ -181,9 +181,11 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
         }
         __syncthreads();
         fetch(t0 + TT);
-        for (int tb = 0; tb < n; tb += 4) {
+        constexpr int UN = NS <= 4 ? 8 : 4;          // tokens whose operands are on their way from LDS together
+        static_assert(TT % UN == 0);
+        for (int tb = 0; tb < n; tb += UN) {
 #pragma unroll
-            for (int t = tb; t < tb + 4; ++t) {
+            for (int t = tb; t < tb + UN; ++t) {
                 const float dt = dt_s[t * CHN + lane_ch], dx = dx_s[t * CHN + lane_ch];
                 StatePairs<L, NS> v;
                 v.read(bc_s + t * 2 * NP + sl * 2 * NS);
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
                     dt_sum += dt;
                 } else {
                     y = sum_lanes<NL>(y);
-                    if (sl == 0) y_s[t * CHN + lane_ch] = y;
+                    y_s[t * CHN + lane_ch] = y;      // (all the channel's lanes hold the sum: a branch here would end the block that reads ahead)
                 }
             }
         }
@@ -326,9 +328,9 @@ int walk_ns(const ScanArgs& a, hipStream_t stream) {
 
 template <typename T>
 int walk_t(const ScanArgs& a, hipStream_t stream) {
-    // Lanes per channel: more of them add up y over more lanes and read dt and dt x again, fewer keep the chip busy with fewer workgroups and hold A, S, B and C in
-    // more registers.  16 sequences of 512 tokens, 4096 channels: 8 states 147 us with 4 lanes, 171 with 8; 16 states 190 and 202; 32 states 244 with 8 lanes,
-    // 314 with 4; 64 states 420 with 16 lanes, 506 with 8.
+    // Lanes per channel: more of them add up y over more lanes and read dt and dt x again, fewer make fewer waves, each with more registers.  16 sequences of 512
+    // tokens, 4096 channels: 8 states 122 us with 2 lanes, 159 with 1; 16 states 153 with 4 lanes, 164 with 2; 32 states 244 with 4 lanes, 314 with 8;
+    // 64 states 420 with 4 lanes, 506 with 8.
     switch (a.n) {
         case 8: return walk_ns<T, 4, 2>(a, stream);
         case 16: return walk_ns<T, 4, 4>(a, stream);

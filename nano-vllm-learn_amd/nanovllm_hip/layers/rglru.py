@@ -27,8 +27,8 @@ def choose_segment(portions, blocks, chunk=64):
 
     Walks of different lengths share the CUs: beyond one a CU, the launch takes as long as the even load and most of a longest walk, or as so many rounds
     of longest walks, whichever is less.  (Counted in rounds alone, forty prompts of 6 to 13 steps were cut up: whole, lightning attention takes them in 67 us against
-    117, the scan in 214 against 308.)  Over ten mixes of 1 to 40 sequences the choice costs 1.03 times the best segment's walks for lightning attention, time mixing and
-    the gated recurrence, 1.07 for the scan; counted in rounds 1.16, 1.10, 1.11 and 1.14."""
+    117, the scan in 155 against 265.)  Over ten mixes of 1 to 40 sequences the choice costs 1.03 times the best segment's walks for lightning attention, time mixing and
+    the gated recurrence, 1.04 for the scan; counted in rounds 1.16, 1.10, 1.11 and 1.14."""
     longest = max(portions, default=1)
     last, total = -(-longest // chunk), sum(portions) / chunk
 

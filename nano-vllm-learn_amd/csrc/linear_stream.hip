@@ -707,6 +707,116 @@ int launch_mt(const LinearArgs& a, hipStream_t stream) {
     return -100;
 }
 
+// ------------------------------------------------------------------------------------------------ residual add, at most four rows, K beyond one workgroup of the tiles above
+// The tiles above share a long K over workgroups and add the parts up behind tickets: a drain, an atomic round trip and a round of loads, about a third of such a launch.  One to
+// four rows are few enough for the vector pipe to take a column's products as they arrive, so a workgroup has four columns and all of K: no tickets, no partial records, no LDS
+// image of the weights.  16 lanes share a column: lane q holds pieces q, q + 16, ... (16 bytes) of its wave's part of the weight row, all of them asked for at once; x waits in
+// LDS, widened (products and sums in fp32).
+constexpr int FW = 8;                              // waves of a workgroup: they share K
+template <int R, int CH>
+__global__ __launch_bounds__(64 * FW) void linear_few_kernel(const uint16_t* __restrict__ p_w, const uint16_t* __restrict__ p_x, const int p_K, const int p_N, const int p_M,
+                                                             const int p_xs /* row stride of x, 0: packed */, const int p_stride, void* const p_out, uint16_t* const p_packed, const LinearArgs a) {
+    constexpr int TPB = 64 * FW, XP = (CH * R + 3) / 4;               // 16-byte pieces of x per thread
+    extern __shared__ __attribute__((aligned(16))) unsigned char few_lds[];
+    float* const xs = reinterpret_cast<float*>(few_lds);                       // [R][K]
+    float* const part = xs + R * p_K;                                          // [waves][4 columns][R], then a spare piece
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane & 15, tiles = p_N / 4;
+    if ((int)blockIdx.x >= tiles) {
+        const int idx = (int)blockIdx.x - tiles, n = (int)gridDim.x - tiles;
+        if (a.pf_kv.k_cache) prefetch_kv_images(a.pf_kv, idx, n, tid, TPB, few_lds);
+        if (a.pf_ptr) prefetch_lines(a.pf_ptr, a.pf_bytes, idx, n, tid, TPB);
+        return;
+    }
+    const int col = 4 * (int)blockIdx.x + (lane >> 4), steps = p_K / 128, s0 = steps * wave / FW, s1 = steps * (wave + 1) / FW;
+    // ---- x is asked for first: the wait for it leaves the weights in flight
+    const int pieces = p_K / 8 * R;
+    u32x4 xr[XP];
+#pragma unroll
+    for (int j = 0; j < XP; ++j) {
+        const int p = tid + j * TPB < pieces ? tid + j * TPB : pieces - 1, row = p % R < p_M ? p % R : p_M - 1, c = p / R;
+        xr[j] = *reinterpret_cast<const u32x4*>(p_x + (p_xs ? row * p_xs + c * 8 : ((c >> 2) * 64 + (c & 3) * 16 + row) * 8));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 w[CH];
+    const uint16_t* const wp = p_w + (int64_t)col * p_K + q * 8;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp + (s0 + i < s1 ? s0 + i : s0) * 128));      // (past the end: the first again, not used)
+    __builtin_amdgcn_sched_barrier(0);
+    const uint16_t resid = reinterpret_cast<const uint16_t*>(p_out)[(int64_t)(q < p_M ? q : 0) * p_stride + col];
+#pragma unroll
+    for (int j = 0; j < XP; ++j) {
+        // (past the end: into the spare piece; a branch here would take the load along, behind the weights)
+        const int p = tid + j * TPB;
+        float* const to = p < pieces ? xs + p % R * p_K + p / R * 8 : part + FW * 4 * R;
+        *reinterpret_cast<f32x4*>(to) = f32x4{bf16_lo(xr[j][0]), bf16_hi(xr[j][0]), bf16_lo(xr[j][1]), bf16_hi(xr[j][1])};
+        *reinterpret_cast<f32x4*>(to + 4) = f32x4{bf16_lo(xr[j][2]), bf16_hi(xr[j][2]), bf16_lo(xr[j][3]), bf16_hi(xr[j][3])};
+    }
+    lds_barrier();                                   // (a __syncthreads() would wait for the weights)
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        if (s0 + i < s1) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float* const xp = xs + r * p_K + (s0 + i) * 128 + q * 8;
+                const f32x4 x0 = *reinterpret_cast<const f32x4*>(xp), x1 = *reinterpret_cast<const f32x4*>(xp + 4);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const float wf = k & 1 ? bf16_hi(w[i][k >> 1]) : bf16_lo(w[i][k >> 1]);
+                    acc[r] = __builtin_fmaf(wf, k < 4 ? x0[k] : x1[k - 4], acc[r]);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        acc[r] += pair_in_row<1>(acc[r]);
+        acc[r] += pair_in_row<2>(acc[r]);
+        acc[r] += pair_in_row<4>(acc[r]);
+        acc[r] += pair_in_row<8>(acc[r]);
+        if (q == 0) part[(wave * 4 + (lane >> 4)) * R + r] = acc[r];
+    }
+    __syncthreads();
+    if (wave > 0 || q >= p_M) return;                // lane q < M of a column's lanes finishes row q
+    float sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < FW; ++k) sum += part[(k * 4 + (lane >> 4)) * R + q];
+    const __bf16 o = (__bf16)(sum + __builtin_bit_cast(float, (uint32_t)resid << 16));
+    reinterpret_cast<__bf16*>(p_out)[(int64_t)q * p_stride + col] = o;
+    if (p_packed) p_packed[pack_index(q, col, p_N)] = __builtin_bit_cast(uint16_t, o);
+}
+
+template <int R, int CH>
+int few_launch(const LinearArgs& a, hipStream_t stream) {
+    const size_t lds = (size_t)(R * a.K + FW * 4 * R + 8) * 4;
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(linear_few_kernel<R, CH>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const bool ahead = (a.pf_ptr && a.pf_bytes >= 128) || a.pf_kv.k_cache;       // (workgroups that only prefetch share the CUs: 128 of them end no later than the others)
+    linear_few_kernel<R, CH><<<a.N / 4 + (ahead ? 128 : 0), 64 * FW, lds, stream>>>(a.w, a.x, a.K, a.N, a.M, a.x_packed ? 0 : a.M == 1 ? a.K : (int)a.x_stride, (int)a.out_stride, a.out, a.out_packed,
+                                                                                       a);
+    return check_launch("linear_few");
+}
+template <int R>
+int few_rows(const LinearArgs& a, hipStream_t stream) {
+    const int steps = a.K / 128;
+    if (steps <= 2 * FW) return few_launch<R, 2>(a, stream);
+    if (steps <= 3 * FW) return few_launch<R, 3>(a, stream);
+    if (steps <= 5 * FW) return few_launch<R, 5>(a, stream);
+    if (steps <= 8 * FW) return few_launch<R, 8>(a, stream);
+    return few_launch<R, 12>(a, stream);
+}
+// Residual adds of up to 12288 activations (rows x K) whose K the tiles would split.  Decode steps of one row: 28 layers of K = 2048 and 3072, 1024 columns 798 -> 735 us; 24 layers
+// with K = 4864, 896 columns 616 -> 603.  Three rows of the former 806 -> 756; but four of the latter 605 -> 628, widening x takes longer than the tickets: left to the tiles,
+// as are shorter K (no tickets: 3.5 us either way) and wider products (gate | up of one row 7.5 us against 7.2).
+bool few_takes(const LinearArgs& a) {
+    return a.epi == EPI_RESADD && a.norm_mode == 0 && a.M <= 4 && a.K % 128 == 0 && a.ksplit > 1 && a.M * a.K <= 12288 && a.N % 4 == 0 && a.out_stride < 1ll << 31 &&
+           (a.x_packed || a.M == 1 || (a.x_stride > 0 && a.x_stride < 1 << 28));
+}
+int launch_few(const LinearArgs& a, hipStream_t stream) {
+    return a.M == 1 ? few_rows<1>(a, stream) : a.M == 2 ? few_rows<2>(a, stream) : few_rows<4>(a, stream);
+}
+
 int tiles_of(int n, int inter, int h, int kvh, int hd, int epi) {
     if (epi == EPI_ROPE) return (h + 2 * kvh) * (hd / 32);
     if (epi == EPI_SILU) return inter / 16;
@@ -750,6 +860,7 @@ int launch_linear_stream(const LinearArgs& a_in, hipStream_t stream) {
         a.counters = reinterpret_cast<unsigned*>(a.ws_raw);
         a.ws = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(a.ws_raw) + kTicketHeader);
     }
+    if (few_takes(a)) return launch_few(a, stream);
     switch ((a.M + 15) / 16) {
         case 1: return launch_mt<1>(a, stream);
         case 2: return launch_mt<2>(a, stream);

@@ -290,6 +290,31 @@ def test_stream_linear_split_k_residual_add(m, n, k):
     assert int(ws[: tiles * 128].view(torch.int32).abs().sum()) == 0       # one ticket per 128-byte line, all back at zero
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 32, 1152), (2, 64, 2048), (3, 1024, 3072), (4, 512, 3072), (1, 896, 4864), (2, 896, 4864), (1, 96, 6272), (1, 64, 8192), (1, 32, 12288), (2, 32, 6144)])
+def test_stream_linear_few_rows_residual_add(m, n, k):
+    """Up to four rows of a long K: within one bf16 rounding of the fp32 reference, the same bits from packed and row-major rows and beside a prefetch, no ticket
+    touched, packed rows past the last one left alone."""
+    from nanovllm_hip import ops
+    g = torch.Generator().manual_seed(n + k)
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    w = (torch.randn(n, k, generator=g) * 0.02).bfloat16().cuda()
+    res0 = torch.randn(m, n, generator=g).bfloat16().cuda()
+    ws = _zero_ws(ops.linear_workspace_bytes(m, n, k, "residual_add"))
+    ref = torch.nn.functional.linear(x.float(), w.float()) + res0.float()
+    xp = ops.pack_rows(torch.cat([x, torch.full((16 - m, k), float("nan"), dtype=torch.bfloat16, device="cuda")]))
+    outs, packs = [], []
+    for packed, hint in ((True, None), (False, None), (True, w.view(torch.uint8).flatten()[:60000])):
+        res, op = res0.clone(), torch.full((16 * n,), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.fused_linear(xp if packed else x, w, epilogue="residual_add", out=res, out_packed=op, workspace=ws, prefetch=hint, x_packed_rows=m if packed else None)
+        outs.append(res)
+        packs.append(op)
+    _close(outs[0], ref)
+    assert all(torch.equal(o, outs[0]) for o in outs) and not ws.any()
+    for op in packs:
+        rows = ops.unpack_rows(op, 16, n)
+        assert torch.equal(rows[:m], outs[0]) and (rows[m:] == 7.0).all()
+
+
 def test_stream_linear_shapes_share_a_workspace():
     """Split-K launches of different tile counts and splits, interleaved on ONE workspace: a launch's partial sums must not land on another's tickets."""
     from nanovllm_hip import ops

@@ -60,7 +60,7 @@ struct TileImages {
 //   query(qs, st)        query fragment: row lq of sub-tile qs, columns 32 st + 8 lg .. (B operand of S^T)
 //   first_key(it)        key of the tile's first row; covers(kv0): this wave sees something of that tile; masked(kv0): but not all of it:
 //   sees(kv0, qs, off)   key kv0 + 4 lg + off counts for the lane's query of sub-tile qs
-//   row(qs)              where the lane's query of sub-tile qs goes, or null; last(qs, d, v): what becomes of its 4 output columns from d on
+//   row(qs)              where the lane's query of sub-tile qs goes, or null; last(qs, v): changes its output columns 16 t + 4 lg .. of all t, v[t]
 // start: score (log2 domain) of a softmax entry without key and value, -inf for none.
 // (The sums, the fragments and the tile loop live in ONE function: split up, the same code takes 32 registers more.)
 template <int DK, int DV, int QT, int WV, typename Stage, typename Query, typename FirstKey, typename Covers, typename Masked, typename Sees, typename Row, typename Last>
@@ -229,7 +229,10 @@ __device__ __forceinline__ void attend_walk(unsigned char* lds, int n_tiles, flo
         if (!out) continue;
         const float inv = sum > 0.f ? 1.f / sum : 0.f;
 #pragma unroll
-        for (int t = 0; t < DT; ++t) act_st4(out + 16 * t + 4 * lg, last(qs, 16 * t + 4 * lg, o[qs][t] * inv));
+        for (int t = 0; t < DT; ++t) o[qs][t] *= inv;
+        last(qs, o[qs]);
+#pragma unroll
+        for (int t = 0; t < DT; ++t) act_st4(out + 16 * t + 4 * lg, o[qs][t]);
     }
 }
 

@@ -89,7 +89,9 @@ __global__ __launch_bounds__(64 * WV, WV == 8 ? 4 : DK + DV <= 320 ? 2 : 1) void
             return at <= (pos < sk - 1 ? pos : sk - 1) && (at >= lo[qs] || at < a.keep_first);
         },
         [&](int qs) { return q_ok[qs] ? reinterpret_cast<uint16_t*>(a.out) + (int64_t)(q_beg + my_q[qs]) * a.out_stride + head * DV : nullptr; },
-        [&](int qs, int d, f32x4 v) { return a.o_cos_sin ? turn_back(v, a.o_cos_sin, my_q[qs] + shift, a.max_position, a.o_rot, d) : v; });
+        [&](int qs, f32x4 (&v)[DV / 16]) {
+            if (a.o_cos_sin) turn_back_tiles(v, a.o_cos_sin, my_q[qs] + shift, a.max_position, a.o_rot, lg);
+        });
 }
 
 template <int DK, int DV, int QT, int WV>

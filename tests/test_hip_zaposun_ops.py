@@ -449,6 +449,20 @@ def test_prompt_in_chunks(heads, kvh, dim, vdim, chunk, keep):
             at += r
 
 
+@pytest.mark.parametrize("vdim,turned,shift", [(128, 2, 0), (128, 6, 0), (128, 64, 0), (128, 128, 1), (64, 36, 1), (64, 4, 0), (256, 200, 0)])
+def test_prompt_turned_widths(vdim, turned, shift):
+    """Widths whose pairs come in twos and others, fewer columns turned than there are; a table that starts `shift` floats behind a border of 8 bytes."""
+    heads, kvh, dim, rows, keys = 4, 2, 64 if vdim < 256 else 256, 150, 170
+    whole = table_of(turned)
+    table = torch.cat([whole.new_zeros(shift), whole.flatten()])[shift:].view_as(whole)
+    pg = Pages([keys], kvh, dim, vdim, BF16, seed=3)
+    q = randn(rows, heads, dim, seed=8)
+    cu = lambda n: torch.tensor([0, n], dtype=torch.int32).cuda()
+    got = pg.unpad(ops().paged_attend_prompt(pg.pad_q(q), pg.cache(), pg.tables.cuda(), cu(rows), cu(keys), rows, heads, kvh, pg.dk, pg.dv, 0.2, 0, 0, chunk=100, turn=table), heads)
+    for t in range(0, rows, 7):
+        close(got[t], turned_back(attend_ref(q[t], pg.k[0], pg.v[0], keys - rows + t, 0.2, 100, 0), keys - rows + t, table), BF16, f"row {t}")
+
+
 @pytest.mark.parametrize("chunk", [1, 64, 65, 40, 100, 128])
 @pytest.mark.parametrize("portion", [1, 2, 40, 200])
 def test_one_key_stands_out_at_chunk_borders(chunk, portion):

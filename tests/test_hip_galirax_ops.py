@@ -286,6 +286,26 @@ def test_lightning_chunk_borders_behind_a_state(heads, dk, dv):
         close(state[i], s, BF16, f"state {i}", slack=0.05)
 
 
+@pytest.mark.parametrize("stride", [(1 << 25) - 8, 34_100_000])
+@pytest.mark.parametrize("heads,dk,dv", [(2, 64, 64), (1, 64, 128), (1, 128, 64), (2, 128, 128)])
+def test_lightning_rows_far_apart(heads, dk, dv, stride):
+    """Rows as far apart as 32-bit offsets reach, and further (the 64th one starts more than 4 GiB behind the first): the same bits as of rows side by side,
+    whole and in segments."""
+    from nanovllm_hip import ops
+    rows, cols, decay = 130, heads * (2 * dk + dv), torch.tensor(DECAYS[:heads], dtype=F32).cuda()
+    x, pos, slots = randn(rows, cols, seed=3).cuda(), torch.arange(5, 5 + rows).cuda(), torch.zeros(1, dtype=torch.int32, device="cuda")
+    start = randn(1, heads, dk, dv, seed=4, dtype=F32).cuda()
+    far = torch.empty((rows, stride), dtype=BF16, device="cuda")[:, :2 * cols]
+    far[:, :cols] = x
+    for chunks in ([(0, rows, 0, 0)], [(0, 64, 0, 0), (64, 66, 0, 1)]):
+        table, near_state, far_state = torch.tensor(chunks, dtype=torch.int32).cuda(), start.clone(), start.clone()
+        far[:, cols:] = 7.0
+        want = ops.lightning_chunks(x, decay, pos, slots, table, len(chunks) > 1, near_state)
+        ops.lightning_chunks(far[:, :cols], decay, pos, slots, table, len(chunks) > 1, far_state, out=far[:, cols:cols + heads * dv])
+        assert torch.equal(far[:, cols:cols + heads * dv], want) and torch.equal(far_state, near_state)
+        assert (far[:, cols + heads * dv:] == 7).all() and torch.equal(far[:, :cols], x)
+
+
 @pytest.mark.parametrize("heads,dk,dv,rows", [(3, 64, 64, 4), (2, 128, 128, 5), (4, 256, 64, 2), (16, 64, 64, 40)])
 def test_lightning_step(heads, dk, dv, rows):
     """Token by token: the step form against the recurrence, from garbage-filled slots on; long enough that a slow head remembers and a fast one forgets."""

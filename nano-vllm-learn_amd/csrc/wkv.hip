@@ -68,7 +68,8 @@ struct WkvLds {
 // (heads of 64: 62 KB and 128 registers each) keep four waves on every SIMD; no register may be spilled inside the loop, a reload waits for every row in flight.
 // A chunk of a head of 64 takes 4.0 us alone and 7.8 beside a second one (6.8 and 13.9 with one kind of wave, 275 registers and one workgroup per CU); 11 portions of
 // 1090 tokens on average, 32 heads: 274 -> 153 us, 40 prompts of 410: 384 -> 166; heads of 128 about half the time.
-template <int DIM, bool SUMMARY>
+// Off: bytes from a chunk's first row.  32 bits where 64 rows fit them: a sequence of 1536 tokens takes 102.5 us against 106.1 in 64 bits, eight of them 122.5 against 128.
+template <int DIM, bool SUMMARY, typename Off>
 __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(const WkvArgs a) {
     using Lds = WkvLds<DIM>;
     constexpr int ROW = DIM * 2, DT = DIM / 16, CP = DIM / 2, WAVES = Lds::WAVES, T = DIM * 4;
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
         u32x4 vv[2];
         // a chunk's rows, past the segment's end its last one.  Every chunk asks for as many rows as any other, in straight line: behind a branch around loads the
         // compiler waits for all that are in flight instead of the ones it needs
-        const uint32_t row_bytes = (uint32_t)a.stride * 2, z_bytes = (uint32_t)a.z_stride * 2;
+        const Off row_bytes = (Off)a.stride * 2, z_bytes = (Off)a.z_stride * 2;
         const int t_last = (n_rows - 1) / C * C;
         auto rows_of = [&](const void* p, int64_t stride, int t0) __attribute__((always_inline)) {
             return reinterpret_cast<const unsigned char*>(p) + 2 * ((int64_t)(row0 + t0) * stride + head * DIM);
@@ -108,21 +109,21 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
             const int t0 = t < t_last ? t : t_last, top = n_rows - t0 - 1, tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
             const unsigned char* zb = rows_of(a.z, a.z_stride, t0);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) zz[i] = *reinterpret_cast<const uint32_t*>(zb + ((uint32_t)(8 * tg + i < top ? 8 * tg + i : top) * z_bytes + 4 * cp));
+            for (int i = 0; i < 8; ++i) zz[i] = *reinterpret_cast<const uint32_t*>(zb + ((Off)(8 * tg + i < top ? 8 * tg + i : top) * z_bytes + 4 * cp));
         };
         auto fetch = [&](int t) __attribute__((always_inline)) {
             const int t0 = t < t_last ? t : t_last, top = n_rows - t0 - 1, tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
             const unsigned char *kb = rows_of(a.k, a.stride, t0), *rb = rows_of(a.r, a.stride, t0), *vb = rows_of(a.v, a.stride, t0);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const uint32_t at = (uint32_t)(8 * tg + i < top ? 8 * tg + i : top) * row_bytes + 4 * cp;
+                const Off at = (Off)(8 * tg + i < top ? 8 * tg + i : top) * row_bytes + 4 * cp;
                 kk[i] = *reinterpret_cast<const uint32_t*>(kb + at);
                 if constexpr (!SUMMARY) rr[i] = *reinterpret_cast<const uint32_t*>(rb + at);
             }
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int e = j * T + tid, r = e / (DIM / 8);
-                vv[j] = *reinterpret_cast<const u32x4*>(vb + ((uint32_t)(r < top ? r : top) * row_bytes + e % (DIM / 8) * 16));
+                vv[j] = *reinterpret_cast<const u32x4*>(vb + ((Off)(r < top ? r : top) * row_bytes + e % (DIM / 8) * 16));
             }
         };
         float la[8], lb[8];                          // sums of log decays up to and with token i of the group
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
 #pragma unroll 1
                 for (int i = 0; i < 8; ++i) {
                     const int t = 8 * tg + i;
-                    const uint32_t z = *reinterpret_cast<const uint32_t*>(zb + ((uint32_t)(t < n ? t : n - 1) * z_bytes + 4 * cp));
+                    const uint32_t z = *reinterpret_cast<const uint32_t*>(zb + ((Off)(t < n ? t : n - 1) * z_bytes + 4 * cp));
                     *reinterpret_cast<f32x2*>(w_f + t * DIM + 2 * cp) = f32x2{fast_exp2(log2_decay(bf16_lo(z) + w0a)), fast_exp2(log2_decay(bf16_hi(z) + w0b))};
                 }
 #pragma unroll
@@ -302,13 +303,13 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
     if constexpr (!SUMMARY) nw = *reinterpret_cast<const f32x4*>(a.norm + head * DIM + 16 * wave + 4 * lg);
     const float inv_n = 1.f / a.n;
     u32x2 gate[4];                                   // gates of four tokens, 4 columns
-    const uint32_t g_bytes = (uint32_t)a.stride * 2, out_bytes = (uint32_t)a.out_stride * 2;
+    const Off g_bytes = (Off)a.stride * 2, out_bytes = (Off)a.out_stride * 2;
     auto fetch_gate = [&](int t0) __attribute__((always_inline)) {
         if constexpr (!SUMMARY) {
             const unsigned char* gb = reinterpret_cast<const unsigned char*>(a.g) + 2 * ((int64_t)(row0 + t0) * a.stride + head * DIM);
             const int top = n_rows - t0 - 1, lane_ = fresh(lane), lq = lane_ & 15, col_bytes = 2 * (16 * wave + 4 * (lane_ >> 4));
 #pragma unroll
-            for (int it = 0; it < 4; ++it) gate[it] = *reinterpret_cast<const u32x2*>(gb + ((uint32_t)(16 * it + lq < top ? 16 * it + lq : top) * g_bytes + col_bytes));
+            for (int it = 0; it < 4; ++it) gate[it] = *reinterpret_cast<const u32x2*>(gb + ((Off)(16 * it + lq < top ? 16 * it + lq : top) * g_bytes + col_bytes));
         }
     };
     const int tr = 4 * lg + (lq >> 2), tp = lq & 3;  // transposed reads: row and column quarter this lane addresses
@@ -440,7 +441,7 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
                 f32x4 r;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) r[k] = o[it][k] * inv * nw[k] * (g[k] * fast_rcp(1.f + fast_exp2(-kLog2e * g[k])));
-                if (16 * it + lq < n) act_st4(reinterpret_cast<uint16_t*>(out + (uint32_t)(16 * it + lq) * out_bytes), r);
+                if (16 * it + lq < n) act_st4(reinterpret_cast<uint16_t*>(out + (Off)(16 * it + lq) * out_bytes), r);
             }
             fetch_gate(t0 + C < n_rows ? t0 + C : t0);
         }
@@ -603,15 +604,15 @@ __global__ __launch_bounds__(256) void wkv_step_kernel(const WkvArgs a) {
     }
 }
 
-template <int DIM>
-int walk_dim(const WkvArgs& a, hipStream_t stream) {
+template <int DIM, typename Off>
+int walk_off(const WkvArgs& a, hipStream_t stream) {
     constexpr size_t lds = sizeof(WkvLds<DIM>);
-    for (const void* fn : {reinterpret_cast<const void*>(wkv_walk_kernel<DIM, true>), reinterpret_cast<const void*>(wkv_walk_kernel<DIM, false>)})
+    for (const void* fn : {reinterpret_cast<const void*>(wkv_walk_kernel<DIM, true, Off>), reinterpret_cast<const void*>(wkv_walk_kernel<DIM, false, Off>)})
         if (lds > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const unsigned deep = (a.n_chunks + 65534) / 65535;
     const dim3 grid(a.heads, (a.n_chunks + deep - 1) / deep, deep);
     if (a.summaries) {
-        wkv_walk_kernel<DIM, true><<<grid, DIM * 8, lds, stream>>>(a);
+        wkv_walk_kernel<DIM, true, Off><<<grid, DIM * 8, lds, stream>>>(a);
         int rc = check_launch("wkv summary");
         if (rc) return rc;
         const int64_t per = (int64_t)a.heads * DIM * DIM;
@@ -619,8 +620,14 @@ int walk_dim(const WkvArgs& a, hipStream_t stream) {
         rc = check_launch("wkv starts");
         if (rc) return rc;
     }
-    wkv_walk_kernel<DIM, false><<<grid, DIM * 8, lds, stream>>>(a);
+    wkv_walk_kernel<DIM, false, Off><<<grid, DIM * 8, lds, stream>>>(a);
     return check_launch("wkv walk");
+}
+
+template <int DIM>
+int walk_dim(const WkvArgs& a, hipStream_t stream) {
+    constexpr int64_t kNear = 1 << 25;               // row strides with which 63 rows and a piece stay below 2^32 bytes
+    return a.stride < kNear && a.z_stride < kNear && a.out_stride < kNear ? walk_off<DIM, uint32_t>(a, stream) : walk_off<DIM, int64_t>(a, stream);
 }
 
 template <typename T>

@@ -337,6 +337,30 @@ def test_wkv_chunk_borders(heads, dim, dk, decay):
             close(state[slots[i], :, :dim, :dim], s, F32, f"state {i}", slack=64)
 
 
+@pytest.mark.parametrize("stride", [(1 << 25) - 8, 34_100_000])
+@pytest.mark.parametrize("decay", ["usual", "strong"])
+@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 128)])
+def test_wkv_rows_far_apart(heads, dim, decay, stride):
+    """Rows as far apart as 32-bit offsets reach, and further (the 64th one starts more than 4 GiB behind the first): the same bits as of rows side by side,
+    whole and in segments."""
+    rows, cols = 130, heads * dim
+    layer = Wkv([rows], heads, dim, dim, BF16, DECAYS[decay])
+    batch, start = [(0, 0, rows, 0)], randn(1, heads, dim, dim, seed=4, dtype=F32).cuda()
+    near = [layer.rows(w, batch) for w in ("r", "k", "v", "g", "z")]
+    far = torch.empty((rows, stride), dtype=BF16, device="cuda")[:, :7 * cols]
+    for i, t in enumerate(near):
+        far[:, i * cols:(i + 1) * cols] = t
+    pos, slots = torch.arange(5, 5 + rows).cuda(), torch.zeros(1, dtype=torch.int32, device="cuda")
+    for chunks in ([(0, rows, 0, 0)], [(0, 64, 0, 0), (64, 66, 0, 1)]):
+        states = start.clone(), start.clone()
+        far[:, 5 * cols:] = 7.0
+        how = layer.params, layer.eps, dim, pos, slots, torch.tensor(chunks, dtype=torch.int32).cuda(), len(chunks) > 1
+        want = ops().wkv_chunks(*near, *how, states[0])
+        ops().wkv_chunks(*(far[:, i * cols:(i + 1) * cols] for i in range(5)), *how, states[1], out=far[:, 5 * cols:6 * cols])
+        assert torch.equal(far[:, 5 * cols:6 * cols], want) and torch.equal(states[0], states[1])
+        assert (far[:, 6 * cols:] == 7).all() and all(torch.equal(far[:, i * cols:(i + 1) * cols], t) for i, t in enumerate(near))
+
+
 @pytest.mark.parametrize("decay", ["usual", "slow", "strong"])
 @pytest.mark.parametrize("heads,dim,dk", WKV_SHAPES)
 def test_wkv_step(heads, dim, dk, decay):

@@ -60,6 +60,11 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4;
     const int64_t slot = a.state_slots[seq];
     const int64_t head_state = (int64_t)a.dk * a.dv;
+    if (n_rows <= 0) {
+        if (SUMMARY || (last && slot >= 0 && ch[3] > 0))
+            pass_segment<SUMMARY>(a.seg_state + ((int64_t)blockIdx.x * a.heads + head) * head_state + v0, a.state + (slot * a.heads + head) * head_state + v0, DK, VS, a.dv);
+        return;
+    }
     if (tid <= C) pw[tid] = powf(a.decay[head], (float)tid);
 
     // state: value column v0 + 16 wave + lq, key rows 16 t + 4 lg + r
@@ -295,6 +300,11 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
     const int wave = prepares ? wave_id - CW : wave_id;
     const int64_t slot = a.state_slots[seq];
     const int64_t head_state = (int64_t)a.dk * a.dv;
+    if (n_rows <= 0) {
+        if (SUMMARY || (last && slot >= 0 && ch[3] > 0))
+            pass_segment<SUMMARY>(a.seg_state + ((int64_t)seg * a.heads + head) * head_state + v0, a.state + (slot * a.heads + head) * head_state + v0, DK, VW, a.dv);
+        return;
+    }
     if (threadIdx.x <= C) {
         const float p = powf(a.decay[head], (float)threadIdx.x);
         pw[threadIdx.x] = p;
@@ -579,7 +589,7 @@ __global__ __launch_bounds__(256) void lightning_starts_kernel(const LightningAr
     if (e >= per || a.chunks[4 * first + 3] != 0) return;
     const float d = a.decay[e / head_state];
     const int64_t slot = a.state_slots[a.chunks[4 * first + 2]];
-    float cur = slot >= 0 && a.positions[a.chunks[4 * first]] > 0 ? a.state[slot * per + e] : 0.f;
+    float cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? a.state[slot * per + e] : 0.f;
     for (int c = first; c < a.n_chunks && (c == first || a.chunks[4 * c + 3] != 0); ++c) {
         const bool more = c + 1 < a.n_chunks && a.chunks[4 * (c + 1) + 3] != 0;        // (the last segment left no contribution)
         const float own = more ? a.seg_state[c * per + e] : 0.f;
@@ -602,7 +612,7 @@ __global__ __launch_bounds__(256) void lightning_generic_kernel(const LightningA
     const int64_t slot = a.state_slots[a.chunks[4 * first + 2]], head_state = (int64_t)a.dk * a.dv;
     const bool ok = col < a.dv;
     float* pool = slot >= 0 ? a.state + (slot * a.heads + head) * head_state : nullptr;
-    const bool carry = pool && a.positions[row0] > 0;
+    const bool carry = pool && portion_carries(a.chunks, a.n_chunks, first, a.positions);
     for (int r = rg; r < a.dk; r += 8) S[r * 32 + c] = carry && ok ? pool[(int64_t)r * a.dv + col] : 0.f;
     const float d = a.decay[head];
     for (int t = 0; t < n_rows; ++t) {

@@ -176,4 +176,22 @@ __device__ __forceinline__ void turn_back_tiles(f32x4 (&v)[DT], const float* tab
     }
 }
 
+// ---- segment tables of the recurrent mechanisms: [first row, rows, sequence, index in its portion].  A segment may have no rows: it is left out of the
+// walks (which ask for rows before they count them), and a portion of such segments leaves its state as it is.
+// Whether a portion goes on from its slot's state: not where its first token is at position 0.
+__device__ __forceinline__ bool portion_carries(const int32_t* chunks, int n_chunks, int first, const int64_t* positions) {
+    for (int c = first; c < n_chunks && (c == first || chunks[4 * c + 3] != 0); ++c)
+        if (chunks[4 * c + 1] > 0) return positions[chunks[4 * c]] > 0;
+    return true;
+}
+// What a workgroup leaves of `rows` x `cols` state elements behind a segment without rows: a summary of nothing, or the state at its start.
+template <bool SUMMARY>
+__device__ __forceinline__ void pass_segment(float* seg_state, float* state, int rows, int cols, int64_t stride) {
+    for (int e = threadIdx.x; e < rows * cols; e += blockDim.x) {
+        const int64_t at = e / cols * stride + e % cols;
+        if constexpr (SUMMARY) seg_state[at] = 0.f;
+        else state[at] = seg_state[at];
+    }
+}
+
 }  // namespace nvh

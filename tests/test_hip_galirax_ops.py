@@ -306,6 +306,30 @@ def test_lightning_rows_far_apart(heads, dk, dv, stride):
         assert (far[:, cols + heads * dv:] == 7).all() and torch.equal(far[:, :cols], x)
 
 
+@pytest.mark.parametrize("dtype,generic", [(BF16, False), (BF16, True), (F32, False)])
+@pytest.mark.parametrize("heads,dk,dv", [(2, 64, 64), (1, 128, 128), (1, 256, 64)])
+def test_lightning_segments_without_rows(heads, dk, dv, dtype, generic):
+    """A segment without rows first, between and last in its portion gives what the table without it gives; a portion without rows, one segment or several, in
+    front of others or behind the last row, leaves its state as it is.  (Behind a last segment without rows the state comes from the summaries of the ones in
+    front: the same products, whose halves round at other places, 2^-17 of each.)"""
+    from nanovllm_hip import ops
+    rows, decay = 130 + 65, torch.tensor(DECAYS[:heads], dtype=F32).cuda()
+    x, start = randn(rows, heads * (2 * dk + dv), seed=3, dtype=dtype).cuda(), randn(5, heads, dk, dv, seed=4, dtype=F32).cuda()
+    pos, slots = torch.cat([torch.arange(5, 135), torch.arange(65)]).cuda(), torch.tensor([3, 0, 2, 4], dtype=torch.int32).cuda()
+
+    def run(chunks):
+        state = start.clone()
+        return ops.lightning_chunks(x, decay, pos, slots, torch.tensor(chunks, dtype=torch.int32).cuda(), any(c[3] for c in chunks), state, generic=generic), state
+    a, b = [(0, 64, 0, 0), (64, 66, 0, 1)], [(130, 65, 1, 0)]
+    whole, cut = run([(0, 130, 0, 0), *b]), run(a + b)
+    for chunks, (want, state), exact in (([(0, 130, 0, 0), (130, 0, 2, 0), *b, (195, 0, 3, 0)], whole, True),
+                                         ([*a, (130, 0, 2, 0), (130, 0, 2, 1), *b, (195, 0, 3, 0), (195, 0, 3, 1)], cut, True),
+                                         ([(0, 0, 0, 0), (0, 64, 0, 1), (64, 0, 0, 2), (64, 66, 0, 3), *b], cut, True),
+                                         ([(0, 64, 0, 0), (64, 66, 0, 1), (130, 0, 0, 2), (130, 0, 1, 0), (130, 65, 1, 1), (195, 0, 1, 2)], cut, False)):
+        got, after = run(chunks)
+        assert torch.equal(got, want) and (torch.equal(after, state) if exact or generic or dtype == F32 else (after - state).abs().max() < 1e-4 * state.abs().max())
+
+
 @pytest.mark.parametrize("heads,dk,dv,rows", [(3, 64, 64, 4), (2, 128, 128, 5), (4, 256, 64, 2), (16, 64, 64, 40)])
 def test_lightning_step(heads, dk, dv, rows):
     """Token by token: the step form against the recurrence, from garbage-filled slots on; long enough that a slow head remembers and a fast one forgets."""

@@ -85,6 +85,12 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
     const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lq = lane & 15, lg = lane >> 4;
     const int64_t slot = a.state_slots[seq];
     constexpr int64_t head_state = (int64_t)DIM * DIM;
+    if (n_rows <= 0) {
+        if (SUMMARY || (last && slot >= 0 && ch[3] > 0))
+            pass_segment<SUMMARY>(a.seg_state + ((int64_t)seg * a.heads + head) * head_state, a.state + (slot * a.heads + head) * head_state, DIM, DIM, DIM);
+        if (SUMMARY && threadIdx.x < DIM) a.seg_decay[((int64_t)seg * a.heads + head) * DIM + threadIdx.x] = 0.f;
+        return;
+    }
 
     if (wave_id >= WAVES) {
         // ---- this thread's rows of a chunk: channels 2 cp, 2 cp + 1 of tokens 8 tg ..; two 16-byte pieces of values
@@ -465,7 +471,7 @@ __global__ __launch_bounds__(256) void wkv_starts_kernel(const WkvArgs a) {
     const int first = blockIdx.y;                    // only a portion's first segment starts a walk
     if (e >= per || a.chunks[4 * first + 3] != 0) return;
     const int64_t ch = e / a.dim, slot = a.state_slots[a.chunks[4 * first + 2]];
-    float cur = slot >= 0 && a.positions[a.chunks[4 * first]] > 0 ? a.state[slot * per + e] : 0.f;
+    float cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? a.state[slot * per + e] : 0.f;
     for (int c = first; c < a.n_chunks && (c == first || a.chunks[4 * c + 3] != 0); ++c) {
         const bool more = c + 1 < a.n_chunks && a.chunks[4 * (c + 1) + 3] != 0;        // (the last segment left no contribution)
         const float own = more ? a.seg_state[c * per + e] : 0.f;
@@ -488,7 +494,7 @@ __global__ __launch_bounds__(256) void wkv_generic_kernel(const WkvArgs a) {
     const int64_t slot = a.state_slots[a.chunks[4 * first + 2]], head_state = (int64_t)a.dim * a.dim;
     const bool ok = col < a.dim;
     float* pool = slot >= 0 ? a.state + (slot * a.heads + head) * head_state : nullptr;
-    const bool carry = pool && a.positions[row0] > 0;
+    const bool carry = pool && portion_carries(a.chunks, a.n_chunks, first, a.positions);
     for (int r = rg; r < a.dim; r += 8) S[r * 32 + c] = carry && ok ? pool[(int64_t)r * a.dim + col] : 0.f;
     for (int i = tid; i < a.dim; i += 256) wkr[3 * a.dim + i] = a.u[head * a.dim + i];
     for (int t = 0; t < n_rows; ++t) {

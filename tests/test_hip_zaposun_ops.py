@@ -361,6 +361,35 @@ def test_wkv_rows_far_apart(heads, dim, decay, stride):
         assert (far[:, 6 * cols:] == 7).all() and all(torch.equal(far[:, i * cols:(i + 1) * cols], t) for i, t in enumerate(near))
 
 
+def segments_without_rows(run, exact):
+    """run(chunks) -> outputs, state, over 130 rows of sequence 0 and 65 of sequence 1.  A segment without rows first, between and last in its portion gives what the
+    table without it gives; a portion without rows, in front of others or behind the last row, leaves its state as it is.  (Behind a last segment without rows
+    the state comes from the summaries of the ones in front: the same sums, put together in another order.)"""
+    a, b = [(0, 64, 0, 0), (64, 66, 0, 1)], [(130, 65, 1, 0)]
+    whole, cut = run([(0, 130, 0, 0), *b]), run(a + b)
+    for chunks, (want, state), same in (([(0, 130, 0, 0), (130, 0, 2, 0), *b, (195, 0, 3, 0)], whole, True),
+                                        ([*a, (130, 0, 2, 0), (130, 0, 2, 1), *b, (195, 0, 3, 0), (195, 0, 3, 1)], cut, True),
+                                        ([(0, 0, 0, 0), (0, 64, 0, 1), (64, 0, 0, 2), (64, 66, 0, 3), *b], cut, True),
+                                        ([(0, 64, 0, 0), (64, 66, 0, 1), (130, 0, 0, 2), (130, 0, 1, 0), (130, 65, 1, 1), (195, 0, 1, 2)], cut, exact)):
+        got, after = run(chunks)
+        assert torch.equal(got, want) and (torch.equal(after, state) if same else (after - state).abs().max() < 1e-4 * state.abs().max())
+
+
+@pytest.mark.parametrize("heads,dim,dtype,generic", [(3, 64, BF16, False), (2, 128, BF16, False), (2, 64, BF16, True), (2, 24, F32, True)])
+@pytest.mark.parametrize("decay", ["usual", "strong"])
+def test_wkv_segments_without_rows(heads, dim, dtype, generic, decay):
+    layer = Wkv([130, 65], heads, dim, dim, dtype, DECAYS[decay])
+    args = [layer.rows(w, [(0, 0, 130, 0), (1, 0, 65, 0)]) for w in ("r", "k", "v", "g", "z")]
+    pos, slots = torch.cat([torch.arange(5, 135), torch.arange(65)]).cuda(), torch.tensor([3, 0, 2, 4], dtype=torch.int32).cuda()
+    start = randn(5, heads, dim, dim, seed=4, dtype=F32).cuda()
+
+    def run(chunks):
+        state = start.clone()
+        return ops().wkv_chunks(*args, layer.params, layer.eps, dim, pos, slots, torch.tensor(chunks, dtype=torch.int32).cuda(), any(c[3] for c in chunks), state,
+                                generic=generic), state
+    segments_without_rows(run, generic)
+
+
 @pytest.mark.parametrize("decay", ["usual", "slow", "strong"])
 @pytest.mark.parametrize("heads,dim,dk", WKV_SHAPES)
 def test_wkv_step(heads, dim, dk, decay):

@@ -97,6 +97,13 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
     if (SUMMARY && last) return;                     // (nothing follows it)
     const int tid = threadIdx.x, c0 = blockIdx.x * CHN, lane_ch = tid / NL, sl = tid % NL;
     const int64_t slot = a.state_slots[seq];
+    if (n_rows <= 0) {
+        const int mine = a.inner - c0 < CHN ? a.inner - c0 : CHN;
+        if (SUMMARY || (last && slot >= 0 && ch[3] > 0))
+            pass_segment<SUMMARY>(a.seg_state + ((int64_t)seg * a.inner + c0) * NP, a.state + (slot * a.inner + c0) * NP, mine, NP, NP);
+        if (SUMMARY && tid < mine) a.seg_dt[(int64_t)seg * a.inner + c0 + tid] = 0.f;
+        return;
+    }
     const int my = c0 + lane_ch < a.inner ? c0 + lane_ch : a.inner - 1;          // the channel this lane scans (a last group may be short)
     float A[NS], S[NS], dt_sum = 0.f;
     const float* src = nullptr;
@@ -240,7 +247,7 @@ __global__ __launch_bounds__(256) void scan_starts_kernel(const ScanArgs a) {
     if (e >= per || a.chunks[4 * first + 3] != 0) return;
     const float A = a.a_log2[e];
     const int64_t c = e / a.n, slot = a.state_slots[a.chunks[4 * first + 2]];
-    float cur = slot >= 0 && a.positions[a.chunks[4 * first]] > 0 ? a.state[slot * per + e] : 0.f;
+    float cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? a.state[slot * per + e] : 0.f;
     for (int k = first; k < a.n_chunks && (k == first || a.chunks[4 * k + 3] != 0); ++k) {
         const bool more = k + 1 < a.n_chunks && a.chunks[4 * (k + 1) + 3] != 0;        // (the last segment left no contribution)
         const float own = more ? a.seg_state[k * per + e] : 0.f;

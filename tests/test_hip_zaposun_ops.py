@@ -158,6 +158,20 @@ def test_causal_conv(taps, dtype):
         close(torch.cat(g), t, dtype)
 
 
+def segments_without_rows(run, exact):
+    """run(chunks) -> outputs, state, over 130 rows of sequence 0 and 65 of sequence 1.  A segment without rows first, between and last in its portion gives what the
+    table without it gives; a portion without rows, in front of others or behind the last row, leaves its state as it is.  (Behind a last segment without rows
+    the state comes from the summaries of the ones in front: the same sums, put together in another order.)"""
+    a, b = [(0, 64, 0, 0), (64, 66, 0, 1)], [(130, 65, 1, 0)]
+    whole, cut = run([(0, 130, 0, 0), *b]), run(a + b)
+    for chunks, (want, state), same in (([(0, 130, 0, 0), (130, 0, 2, 0), *b, (195, 0, 3, 0)], whole, True),
+                                        ([*a, (130, 0, 2, 0), (130, 0, 2, 1), *b, (195, 0, 3, 0), (195, 0, 3, 1)], cut, True),
+                                        ([(0, 0, 0, 0), (0, 64, 0, 1), (64, 0, 0, 2), (64, 66, 0, 3), *b], cut, True),
+                                        ([(0, 64, 0, 0), (64, 66, 0, 1), (130, 0, 0, 2), (130, 0, 1, 0), (130, 65, 1, 1), (195, 0, 1, 2)], cut, exact)):
+        got, after = run(chunks)
+        assert torch.equal(got, want) and (torch.equal(after, state) if same else (after - state).abs().max() < 1e-4 * state.abs().max())
+
+
 # ------------------------------------------------------------------------------------------------ selective scan
 class Scan:
     """Random operands of one scan layer and the plain result for several sequences."""
@@ -227,6 +241,20 @@ def test_scan_tile_borders(inner, n, dtype):
         for i, (y, s) in enumerate(layer.want):
             close(got[i], y, dtype, f"segment {segment} sequence {i}")
             close(state[slots[i], :, :n], s, F32, f"state {i}", slack=4)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("inner,n", [(72, 8), (136, 16), (24, 256)])
+def test_scan_segments_without_rows(inner, n, dtype):
+    layer = Scan([130, 65], inner, n, 8, dtype)
+    x, dt, bc, z = (layer.rows(w, [(0, 0, 130, 0), (1, 0, 65, 0)]) for w in ("x", "dt", "bc", "z"))
+    pos, slots = torch.cat([torch.arange(5, 135), torch.arange(65)]).cuda(), torch.tensor([3, 0, 2, 4], dtype=torch.int32).cuda()
+    start = randn(5, inner, n, seed=4, dtype=F32).cuda()
+
+    def run(chunks):
+        state = start.clone()
+        return ops().scan_chunks(x, dt, bc, z, layer.params, pos, slots, torch.tensor(chunks, dtype=torch.int32).cuda(), any(c[3] for c in chunks), state), state
+    segments_without_rows(run, False)
 
 
 @pytest.mark.parametrize("inner,n,rank", [(72, 5, 16), (64, 16, 64), (8192, 16, 128), (320, 30, 24), (64, 50, 8), (40, 100, 72), (24, 256, 8)])
@@ -359,20 +387,6 @@ def test_wkv_rows_far_apart(heads, dim, decay, stride):
         ops().wkv_chunks(*(far[:, i * cols:(i + 1) * cols] for i in range(5)), *how, states[1], out=far[:, 5 * cols:6 * cols])
         assert torch.equal(far[:, 5 * cols:6 * cols], want) and torch.equal(states[0], states[1])
         assert (far[:, 6 * cols:] == 7).all() and all(torch.equal(far[:, i * cols:(i + 1) * cols], t) for i, t in enumerate(near))
-
-
-def segments_without_rows(run, exact):
-    """run(chunks) -> outputs, state, over 130 rows of sequence 0 and 65 of sequence 1.  A segment without rows first, between and last in its portion gives what the
-    table without it gives; a portion without rows, in front of others or behind the last row, leaves its state as it is.  (Behind a last segment without rows
-    the state comes from the summaries of the ones in front: the same sums, put together in another order.)"""
-    a, b = [(0, 64, 0, 0), (64, 66, 0, 1)], [(130, 65, 1, 0)]
-    whole, cut = run([(0, 130, 0, 0), *b]), run(a + b)
-    for chunks, (want, state), same in (([(0, 130, 0, 0), (130, 0, 2, 0), *b, (195, 0, 3, 0)], whole, True),
-                                        ([*a, (130, 0, 2, 0), (130, 0, 2, 1), *b, (195, 0, 3, 0), (195, 0, 3, 1)], cut, True),
-                                        ([(0, 0, 0, 0), (0, 64, 0, 1), (64, 0, 0, 2), (64, 66, 0, 3), *b], cut, True),
-                                        ([(0, 64, 0, 0), (64, 66, 0, 1), (130, 0, 0, 2), (130, 0, 1, 0), (130, 65, 1, 1), (195, 0, 1, 2)], cut, exact)):
-        got, after = run(chunks)
-        assert torch.equal(got, want) and (torch.equal(after, state) if same else (after - state).abs().max() < 1e-4 * state.abs().max())
 
 
 @pytest.mark.parametrize("heads,dim,dtype,generic", [(3, 64, BF16, False), (2, 128, BF16, False), (2, 64, BF16, True), (2, 24, F32, True)])

@@ -165,6 +165,11 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
             act_st8(dt_s + tid * 8, dt);
             act_st8(dx_s + tid * 8, dx);
         }
+        if (n < TT) {                                // rows past the end count nothing, not even infinite ones
+#pragma unroll
+            for (int j = 0; j < BCP; ++j)
+                if ((j * 256 + tid) / (2 * NP / 8) >= n) bc[j] = Raw{};
+        }
 #pragma unroll
         for (int j = 0; j < BCP; ++j) {
             const int e = j * 256 + tid, t = e / (2 * NP / 8), p = e % (2 * NP / 8), half = p / (NP / 8), s0 = p % (NP / 8) * 8;       // states s0 .. s0 + 7 of B or C

@@ -257,6 +257,22 @@ def test_scan_segments_without_rows(inner, n, dtype):
     segments_without_rows(run, False)
 
 
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("inner,n", [(72, 8), (136, 16), (24, 64), (24, 128)])
+def test_scan_infinite_last_row(inner, n, dtype):
+    """A last row whose B is infinite for one state: that state becomes infinite, not a number made of it and rows past the end; the others are what they were."""
+    rows, one = 61, n // 2 + 1
+    layer, states = Scan([rows], inner, n, 8, dtype), []
+    for last in (1.0, float("inf")):
+        layer.bc[0][-1, 0, one] = last
+        states.append(torch.zeros(1, inner, n, device="cuda"))
+        layer.run([(0, 0, rows, 0)], states[-1])
+    was, now = states
+    assert torch.equal(now[0, :, one].cpu(), layer.x[0][-1].float().sign() * float("inf"))
+    was[0, :, one] = now[0, :, one] = 0
+    assert torch.equal(was, now)
+
+
 @pytest.mark.parametrize("inner,n,rank", [(72, 5, 16), (64, 16, 64), (8192, 16, 128), (320, 30, 24), (64, 50, 8), (40, 100, 72), (24, 256, 8)])
 def test_scan_step(inner, n, rank):
     """Single tokens behind portions; many channels take several rows per workgroup."""

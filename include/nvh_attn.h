@@ -470,7 +470,8 @@ int nvh_clamped_glu(void* out, const void* gate_up, int rows, int inter, int64_t
 int nvh_gelu_glu(void* out, const void* gate_up, int rows, int inter, int64_t gate_up_row_stride, int64_t out_row_stride, int dtype, void* stream);
 /* Real-gated linear recurrent unit behind a causal depthwise convolution: log a = -rate sigmoid(ra u), S = a S + sqrt(1 - a^2) sigmoid(ri u) u,
  * out = S gelu(y).  nvh_rglru_chunks: portions of prompts (and single tokens), cut by the caller into segments that are
- * scanned side by side; segments of one portion are consecutive.  nvh_rglru_step: row i is one new token of sequence i (bf16; nvh_rglru_step_supported(block)).
+ * scanned side by side; segments of one portion are consecutive.  A portion's last segment may have no rows; a portion without rows leaves state and ring as they are.
+ * nvh_rglru_step: row i is one new token of sequence i (bf16; nvh_rglru_step_supported(block)).
  * generic: 0 = the fastest form the shape allows, 1 = the plain kernel, 2 = the MFMA walk without LDS-DMA (tests). */
 typedef struct nvh_rglru_desc {
     const void* yx;              /* [rows, 2 * width]: gate branch | recurrent branch (biases added), row stride yx_stride */
@@ -653,7 +654,8 @@ int nvh_talk_prompt_supported(int heads, int kv_heads, int dk, int dv, int block
 int nvh_talk_prompt(const nvh_paged_attend_desc* d, int dtype, void* stream);
 
 /* Lightning attention: per head S = decay S + k v^T, o = S^T q with q, k, v = silu of the projection's columns (rounded to the activation type);
- * the state is fp32.  nvh_lightning_chunks: portions cut into segments as for nvh_rglru_chunks; nvh_lightning_step: row i is one new token of
+ * the state is fp32.  nvh_lightning_chunks: portions cut into segments as for nvh_rglru_chunks, of any number of
+ * rows, none included; nvh_lightning_step: row i is one new token of
  * sequence i.  A token at position 0 takes the state as zero.  generic (chunks): the plain token-by-token kernel, any width; the MFMA form and the step need
  * nvh_lightning_supported(dk, dv). */
 typedef struct nvh_lightning_desc {
@@ -844,7 +846,7 @@ int nvh_causal_conv(const nvh_causal_conv_desc* d, int dtype, void* stream);
 
 /* Selective scan: S[c][n] <- exp(dt_c A[c][n]) S[c][n] + dt_c x_c B[n], y_c = sum_n S[c][n] C[n] + d_c x_c, out = y silu(z), dt = softplus(. + dt_bias).  The state is
  * fp32; a token at position 0 takes it as zero.  nvh_scan_states(n): the number of states kept for n of them (0: too many).
- *   portions (nvh_scan_chunks)  dt [rows, inner]; cut into segments as for nvh_rglru_chunks
+ *   portions (nvh_scan_chunks)  dt [rows, inner]; cut into segments as for nvh_lightning_chunks
  *   single   (nvh_scan_step)    bf16; row i is one new token of sequence i; dt [rows, rank] is multiplied by w_dt [inner, rank] first */
 typedef struct nvh_scan_desc {
     const void* x;               /* [rows, inner] */
@@ -879,7 +881,7 @@ int nvh_scan_step(const nvh_scan_desc* d, int dtype, void* stream);
 
 /* Time mixing: per head o = (S + diag(u) k v^T)^T r, S <- diag(w) S + k v^T with w = exp(-exp(z + w0)) per token and key channel, then
  * out = o / sqrt(mean over n columns of o^2 + eps) * norm * silu(g).  The state is fp32; a token at position 0 takes it as zero.
- *   portions (nvh_wkv_chunks)  z [rows, heads * dim]; cut into segments as for nvh_rglru_chunks; generic: the plain token-by-token kernel, any width
+ *   portions (nvh_wkv_chunks)  z [rows, heads * dim]; cut into segments as for nvh_lightning_chunks; generic: the plain token-by-token kernel, any width
  *   single   (nvh_wkv_step)    bf16; row i is one new token of sequence i; z [rows, rank]: w2 tanh(z) is computed first; nvh_wkv_supported(dim) */
 typedef struct nvh_wkv_desc {
     const void* r;               /* r, k, v, g: [rows, heads * dim], one row stride */

@@ -101,6 +101,9 @@ __device__ __forceinline__ void conv_run(const RglruArgs& a, int ch, int taps_rt
     }
 }
 
+// Only a portion's last segment may have no rows; where that is its only one, nothing is walked and the slot keeps what it holds.
+__device__ __forceinline__ bool portion_without_rows(int n, int kth) { return n <= 0 && kth == 0; }
+
 // what a segment starts from (segment table index `seg`, channel ch)
 __device__ __forceinline__ float walk_start(const RglruArgs& a, bool summary, bool more, int seg, int kth, int slot, int64_t pos0, int ch) {
     float cs = 0.f;
@@ -123,7 +126,7 @@ __global__ __launch_bounds__(1024) void rglru_walk_kernel(const RglruArgs a) {
     const int groups = (a.block + kGroup - 1) / kGroup, seg = blockIdx.x, blk = blockIdx.y / groups, g0 = (blockIdx.y - blk * groups) * kGroup;
     const int row0 = a.chunks[seg * 4], n = a.chunks[seg * 4 + 1], seq = a.chunks[seg * 4 + 2], kth = a.chunks[seg * 4 + 3];
     const bool more = seg + 1 < a.n_chunks && a.chunks[seg * 4 + 6] == seq;    // another segment of this sequence follows
-    if (SUMMARY && !more) return;
+    if ((SUMMARY && !more) || portion_without_rows(n, kth)) return;
     const int off0 = kth * a.segment, seq_row0 = row0 - off0;
     const int slot = a.state_slots[seq];
     const int64_t pos0 = a.positions[seq_row0];
@@ -291,7 +294,7 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs
     if (seg >= a.n_chunks) return;
     const int row0 = a.chunks[seg * 4], n = a.chunks[seg * 4 + 1], seq = a.chunks[seg * 4 + 2], kth = a.chunks[seg * 4 + 3];
     const bool more = seg + 1 < a.n_chunks && a.chunks[seg * 4 + 6] == seq;
-    if (SUMMARY && !more) return;
+    if ((SUMMARY && !more) || portion_without_rows(n, kth)) return;
     const int off0 = kth * a.segment, seq_row0 = row0 - off0;
     const int slot = a.state_slots[seq];
     const int64_t pos0 = a.positions[seq_row0];
@@ -323,7 +326,7 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs
         }
     };
     stage_x(0);
-    if (!SUMMARY) stage_y(0, y_lds);
+    if (!SUMMARY && n > 0) stage_y(0, y_lds);        // (a last segment without rows has some of x in front of it, but none of y)
     for (int e = tid; e < (a.taps + 1) * BLOCK; e += THREADS)
         w_lds[e] = e < a.taps * BLOCK ? a.conv_w[(int64_t)(e / BLOCK) * a.width + c0 + e % BLOCK] : a.conv_b[c0 + e % BLOCK];
 
@@ -497,7 +500,7 @@ __global__ __launch_bounds__(256) void rglru_walk_generic_kernel(const RglruArgs
     const int tiles = (a.block + 63) / 64, blk = blockIdx.y / tiles, n0 = (blockIdx.y % tiles) * 64;
     const int row0 = a.chunks[seg * 4], n = a.chunks[seg * 4 + 1], seq = a.chunks[seg * 4 + 2], kth = a.chunks[seg * 4 + 3];
     const bool more = seg + 1 < a.n_chunks && a.chunks[seg * 4 + 6] == seq;
-    if (SUMMARY && !more) return;
+    if ((SUMMARY && !more) || portion_without_rows(n, kth)) return;
     const int off0 = kth * a.segment, seq_row0 = row0 - off0;
     const int slot = a.state_slots[seq];
     const int64_t pos0 = a.positions[seq_row0];
@@ -585,7 +588,7 @@ __global__ __launch_bounds__(256) void rglru_keep_kernel(const RglruArgs a) {
     const int seg = blockIdx.x, ch = (blockIdx.y * 256 + threadIdx.x) * 4;
     const int row0 = a.chunks[seg * 4], n = a.chunks[seg * 4 + 1], seq = a.chunks[seg * 4 + 2], kth = a.chunks[seg * 4 + 3];
     const int slot = a.state_slots[seq];
-    if (ch >= a.width || slot < 0 || (seg + 1 < a.n_chunks && a.chunks[seg * 4 + 6] == seq)) return;
+    if (ch >= a.width || slot < 0 || portion_without_rows(n, kth) || (seg + 1 < a.n_chunks && a.chunks[seg * 4 + 6] == seq)) return;
     *reinterpret_cast<f32x4*>(a.state + (int64_t)slot * a.width + ch) = *reinterpret_cast<const f32x4*>(a.s_loc + (int64_t)seg * a.width + ch);
     const int portion = kth * a.segment + n, keep = portion < a.taps ? portion : a.taps;
     for (int j = 0; j < keep; ++j) {

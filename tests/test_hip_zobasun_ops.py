@@ -212,6 +212,27 @@ def test_recurrence_rows_far_apart():
     close(out.cpu(), r.plain(y, x)[0], torch.bfloat16)
 
 
+@pytest.mark.parametrize("dtype,generic", WALKS)
+@pytest.mark.parametrize("blocks,block", [(2, 64), (2, 160)])
+def test_recurrence_segments_without_rows(blocks, block, dtype, generic):
+    """A last segment without rows gives what the table without it gives (the state from the summaries of the ones in front: the same decays, multiplied in another
+    order); portions without rows, in front of others or behind the last row, leave state and ring as they are."""
+    from nanovllm_hip import ops
+    r = Recurrence(blocks, block, block, 4, dtype, slots=5)
+    yx, pos, slots = r.rows(*r.yx(193, 1)), torch.cat([torch.arange(5, 133), torch.arange(65)]).cuda(), torch.tensor([3, 0, 2, 4], dtype=torch.int32, device="cuda")
+    r.state.normal_(), r.conv_state.normal_()
+
+    def run(chunks):
+        pools = r.state.clone(), r.conv_state.clone()
+        return ops.rglru_chunks(yx, r.params, pos, slots, torch.tensor(chunks, dtype=torch.int32, device="cuda"), 64, any(c[3] for c in chunks), *pools, generic=generic), *pools
+    a, b = [(0, 64, 0, 0), (64, 64, 0, 1)], [(128, 64, 1, 0), (192, 1, 1, 1)]
+    want, state, ring = run(a + b)
+    for chunks, same in (([*a, (128, 0, 2, 0), *b, (193, 0, 3, 0)], True), ([*a, (128, 0, 0, 2), *b], False)):
+        got, after, kept = run(chunks)
+        assert torch.equal(got, want) and torch.equal(kept, ring)
+        assert torch.equal(after, state) if same else (after - state).abs().max() < 1e-4 * state.abs().max()
+
+
 @pytest.mark.parametrize("blocks,size,block,taps", SHAPES)
 def test_recurrence_step_follows_portions(blocks, size, block, taps):
     """Prompt by the chunked form, then single tokens by the step form (one sequence steps from its very first token)."""

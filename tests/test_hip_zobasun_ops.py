@@ -201,15 +201,25 @@ def test_recurrence_row_edges(blocks, block, taps, segment):
     close(r.unspread(r.state.cpu()), torch.stack([s for _, s in want]), torch.float32, 40)
 
 
-def test_recurrence_rows_far_apart():
-    """Rows too far apart for 32-bit offsets."""
+@pytest.mark.parametrize("stride", [(1 << 24) - 8, 34_100_000])
+def test_recurrence_rows_far_apart(stride):
+    """Rows as far apart as 32-bit offsets are used for, and too far for them (the 64th one starts more than 4 GiB behind the first): the same bits as of rows side
+    by side in the form that takes them, whole and in segments."""
     from nanovllm_hip import ops
-    r = Recurrence(2, 64, 64, 4, torch.bfloat16)
-    y, x = r.yx(3, 1)
-    rows = torch.zeros((3, 1 << 24), dtype=torch.bfloat16, device="cuda")[:, :2 * r.cols].copy_(r.rows(y, x))
-    out = ops.rglru_chunks(rows, r.params, torch.arange(3).cuda(), torch.zeros(1, dtype=torch.int32, device="cuda"), torch.tensor([[0, 3, 0, 0]], dtype=torch.int32, device="cuda"),
-                           64, False, r.state, r.conv_state)
-    close(out.cpu(), r.plain(y, x)[0], torch.bfloat16)
+    r, n = Recurrence(2, 64, 64, 4, torch.bfloat16), 130
+    near, form = r.rows(*r.yx(n, 1)), 0 if stride < 1 << 24 else 2
+    far = torch.empty((n, stride), dtype=torch.bfloat16, device="cuda")[:, :4 * r.cols]
+    far[:, :2 * r.cols] = near
+    pos, slot = torch.arange(5, 5 + n).cuda(), torch.ones(1, dtype=torch.int32, device="cuda")
+    r.state.normal_(), r.conv_state.normal_()
+    for chunks in ([(0, n, 0, 0)], [(0, 64, 0, 0), (64, 64, 0, 1), (128, 2, 0, 2)]):
+        far[:, 2 * r.cols:] = 7.0
+        table, pools = torch.tensor(chunks, dtype=torch.int32, device="cuda"), [(r.state.clone(), r.conv_state.clone()) for _ in range(2)]
+        how = r.params, pos, slot, table, 64 * (3 - len(chunks)) + 64, len(chunks) > 1
+        want = ops.rglru_chunks(near, *how, *pools[0], generic=form)
+        ops.rglru_chunks(far[:, :2 * r.cols], *how, *pools[1], out=far[:, 2 * r.cols:3 * r.cols])
+        assert torch.equal(far[:, 2 * r.cols:3 * r.cols], want) and all(torch.equal(a, b) for a, b in zip(*pools))
+        assert (far[:, 3 * r.cols:] == 7).all() and torch.equal(far[:, :2 * r.cols], near)
 
 
 @pytest.mark.parametrize("dtype,generic", WALKS)
@@ -231,6 +241,18 @@ def test_recurrence_segments_without_rows(blocks, block, dtype, generic):
         got, after, kept = run(chunks)
         assert torch.equal(got, want) and torch.equal(kept, ring)
         assert torch.equal(after, state) if same else (after - state).abs().max() < 1e-4 * state.abs().max()
+
+
+def test_recurrence_many_segments():
+    """More segments than one dimension of a grid holds."""
+    from nanovllm_hip import ops
+    n = 65541
+    r = Recurrence(2, 32, 32, 4, torch.bfloat16, slots=1)
+    yx = r.rows(*r.yx(7, 1)).repeat(n // 7 + 1, 1)[:n].contiguous()
+    table = torch.tensor([(i, 1, i, 0) for i in range(n)], dtype=torch.int32, device="cuda")
+    out = ops.rglru_chunks(yx, r.params, torch.zeros(n, dtype=torch.int64, device="cuda"), torch.full((n,), -1, dtype=torch.int32, device="cuda"), table, 64, False, r.state, r.conv_state)
+    few = ops.rglru_chunks(yx[:7], r.params, torch.zeros(7, dtype=torch.int64, device="cuda"), torch.full((7,), -1, dtype=torch.int32, device="cuda"), table[:7], 64, False, r.state, r.conv_state)
+    assert torch.equal(out, few.repeat(n // 7 + 1, 1)[:n]) and few.any(dim=1).all()
 
 
 @pytest.mark.parametrize("blocks,size,block,taps", SHAPES)

@@ -300,3 +300,13 @@ def test_which_kernels_take_which_layers():
     assert all(l.mixer.step_ok for l in layers["wide"]) and all(l.mixer.left.fast_prompt for l in layers["wide"] if hasattr(l.mixer, "left"))
     assert [l.mixer.step_ok for l in layers["plain"]] == [False, False, True, False]
     assert wkv(2, 3)["mlp"] is None
+
+
+@pytest.mark.parametrize("heads,dim,units,whole", [(32, 64, 16, True), (16, 40, 8, False), (1, 64, 1, False), (16, 128, 16, True), (8, 100, 8, False)])
+def test_time_mixing_segments(heads, dim, units, whole):
+    """Heads of 64 share a compute unit by two, wider ones have one each: sixteen portions stay whole where that many of their walks fill the GPU."""
+    from nanovllm_hip.layers.rglru import choose_segment
+    from nanovllm_hip.layers.wkv import TimeMixing
+    portions = [200 + 95 * i for i in range(16)]
+    assert (got := TimeMixing(64, 64, heads, dim, 1e-5, torch.bfloat16).segment_units) == units
+    assert (choose_segment(portions, got) >= max(portions)) == whole

@@ -12,9 +12,11 @@ from .linear import linear, padded, round_up
 
 
 class SelectiveScan(nn.Module):
-    # what choose_segment takes for workgroups that walk one segment: it counts one per CU, and four of the scan's (64 channels each) share one.
-    # Over ten mixes of 1 to 40 sequences the choice costs 1.04 times the best segment's walks; counted by 192 channels 1.07, by 128 1.10, by 512 1.07
-    segment_units = property(lambda self: max(1, self.inner_cols // 256))
+    # What choose_segment takes for workgroups that walk one segment: it counts one per CU, and many of the scan's small ones share one (of 128 channels at 8 states, 64
+    # up to 64, 32 at 128, 16 at 256).  By states: times 1024 channels.  Over ten mixes of 1 to 40 sequences the choice costs, times the best segment's walks, for
+    # 4096 / 2048 channels: 8 states 1.01 / 1.01 (counted as 16 states 1.16 / 1.10), 16 to 64 states 1.07 to 1.08 / 1.09 to 1.12 at 32 and 64 (6 units instead of 4:
+    # 1.03 / 1.15), 128 states 1.01 / 1.03 (as 16: 1.14 / 1.09); 2048 / 1024 channels of 256 states 1.01 / 1.03 (as 16: 1.23 / 1.06)
+    segment_units = property(lambda self: max(1, self.inner_cols * {8: 1, 128: 12, 256: 24}.get(self.n, 4) // 1024))
 
     def __init__(self, in_width, in_cols, inner, states, rank, taps, dtype):
         super().__init__()

@@ -310,3 +310,10 @@ def test_time_mixing_segments(heads, dim, units, whole):
     portions = [200 + 95 * i for i in range(16)]
     assert (got := TimeMixing(64, 64, heads, dim, 1e-5, torch.bfloat16).segment_units) == units
     assert (choose_segment(portions, got) >= max(portions)) == whole
+
+
+@pytest.mark.parametrize("inner,states,units", [(4096, 8, 4), (64, 5, 1), (2048, 16, 8), (4096, 64, 16), (2048, 100, 24), (1024, 256, 24)])
+def test_scan_segments(inner, states, units):
+    """The more states a channel has, the fewer channels' walks keep a compute unit busy."""
+    from nanovllm_hip.layers.mamba import SelectiveScan
+    assert SelectiveScan(64, 64, inner, states, 16, 4, torch.bfloat16).segment_units == units

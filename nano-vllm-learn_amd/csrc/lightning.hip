@@ -288,8 +288,7 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
     __shared__ __attribute__((aligned(16))) float pw[C + 1], fall_s[C];        // decay^0 .. decay^C; decay^(C - 1 - key)
     auto swz = [](int r) { return KROW == 128 ? (r >> 1) & 7 : r & 15; };      // rows of 256 bytes span all banks: 16 of them apart, not 8
     auto swzv = [](int r) { return VROW == 128 ? (r >> 1) & 7 : (2 * r) & 14; };
-    const int seg = blockIdx.y + blockIdx.z * gridDim.y;
-    if (seg >= a.n_chunks) return;
+    const int seg = blockIdx.y;
     const int32_t* ch = a.chunks + 4 * seg;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
     const int slices = a.dv / VW, head = blockIdx.x / slices, v0 = (blockIdx.x - head * slices) * VW;
@@ -758,8 +757,7 @@ int pair_dk(const LightningArgs& a, hipStream_t stream) {
     if (sum_lds > 64 * 1024)
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sum_lds);
     // heads run fastest: workgroups are dealt round-robin over the 8 XCDs, and segments differ in length while the heads of one do not
-    const unsigned deep = (a.n_chunks + 65534) / 65535;
-    const dim3 grid(a.heads * (a.dv / (16 * CW)), (a.n_chunks + deep - 1) / deep, deep);
+    const dim3 grid(a.heads * (a.dv / (16 * CW)), a.n_chunks);
     if (a.summaries) {
         lightning_pair_kernel<DK, CW, PW, true><<<grid, 64 * (CW + PW), sum_lds, stream>>>(a);
         int rc = check_launch("lightning summary");

@@ -89,8 +89,7 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
     // 414 against 494 at 64); beyond that the wider rows' bank conflicts cost more than widening on every read (1021 against 928 at 128)
     using L = typename std::conditional<NP <= 64, float, T>::type;
     __shared__ __attribute__((aligned(16))) L bc_s[TT * 2 * NP];
-    const int seg = blockIdx.y + blockIdx.z * gridDim.y;         // channels run fastest: workgroups are dealt round-robin over the XCDs, and segments differ in length
-    if (seg >= a.n_chunks) return;
+    const int seg = blockIdx.y;                      // channels run fastest: workgroups are dealt round-robin over the XCDs, and segments differ in length
     const int32_t* ch = a.chunks + 4 * seg;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
     const bool last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;
@@ -323,8 +322,7 @@ __global__ __launch_bounds__(256) void scan_step_kernel(const ScanArgs a) {
 template <typename T, int NS, int NL>
 int walk_ns(const ScanArgs& a, hipStream_t stream) {
     constexpr int CHN = 256 / NL;
-    const unsigned deep = (a.n_chunks + 65534) / 65535;
-    const dim3 grid((a.inner + CHN - 1) / CHN, (a.n_chunks + deep - 1) / deep, deep);
+    const dim3 grid((a.inner + CHN - 1) / CHN, a.n_chunks);
     if (a.summaries) {
         scan_walk_kernel<T, NS, NL, true><<<grid, 256, 0, stream>>>(a);
         int rc = check_launch("scan summary");

@@ -76,8 +76,7 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     Lds& lds = *reinterpret_cast<Lds*>(smem);
     auto swz = [](int r) { return ROW == 128 ? (r >> 1) & 7 : r & 15; };       // rows of 256 bytes span all banks
-    const int head = blockIdx.x, seg = blockIdx.y + blockIdx.z * gridDim.y;      // heads run fastest: workgroups are dealt round-robin over the XCDs, and segments differ in length
-    if (seg >= a.n_chunks) return;
+    const int head = blockIdx.x, seg = blockIdx.y;   // heads run fastest: workgroups are dealt round-robin over the XCDs, and segments differ in length
     const int32_t* ch = a.chunks + 4 * seg;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
     const bool last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;
@@ -615,8 +614,7 @@ int walk_off(const WkvArgs& a, hipStream_t stream) {
     constexpr size_t lds = sizeof(WkvLds<DIM>);
     for (const void* fn : {reinterpret_cast<const void*>(wkv_walk_kernel<DIM, true, Off>), reinterpret_cast<const void*>(wkv_walk_kernel<DIM, false, Off>)})
         if (lds > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    const unsigned deep = (a.n_chunks + 65534) / 65535;
-    const dim3 grid(a.heads, (a.n_chunks + deep - 1) / deep, deep);
+    const dim3 grid(a.heads, a.n_chunks);
     if (a.summaries) {
         wkv_walk_kernel<DIM, true, Off><<<grid, DIM * 8, lds, stream>>>(a);
         int rc = check_launch("wkv summary");

@@ -16,7 +16,7 @@ namespace nvh {
 
 namespace {
 
-constexpr int C = kLightningChunk, VS = 64;          // tokens per step, value columns per workgroup
+constexpr int C = kLightningChunk, VS = 64;          // tokens per step; value columns of a workgroup of keys of 256
 constexpr int PLD = C + 8;                           // row of the weights in LDS
 
 __device__ __forceinline__ void split_hi_lo(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
@@ -38,19 +38,19 @@ __device__ __forceinline__ u32x4 silu8(u32x4 r) {
     return r;
 }
 
-// (keys wider than 128: two images of each kind would not fit the LDS)
-template <int DK, bool SUMMARY>
+// Keys of 256 (two images of each kind, as the walk below holds, would not fit the LDS, nor rows of a step ahead the registers)
+constexpr int kWide = 256;
+template <bool SUMMARY>
 __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs a) {
-    constexpr int KP = DK / 8, KROW = DK * 2, NQ = C * KP / 256, NV = C * (VS / 8) / 256, DT = DK / 16;
-    constexpr bool kOdd = ((KROW / 128) & 1) != 0, kAhead = DK <= 128;         // (wider: no registers to fetch a step ahead)
-    constexpr int TB = DT < 8 ? DT : 8;              // key tiles read at a time
+    constexpr int DK = kWide, KP = DK / 8, KROW = DK * 2, NQ = C * KP / 256, NV = C * (VS / 8) / 256, DT = DK / 16;
+    constexpr int TB = 8;                            // key tiles read at a time
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* kimg = smem;                                                // [C][DK] keys
     unsigned char* vimg = kimg + C * KROW;                                     // [C][VS] values
     unsigned char* qimg = vimg + C * VS * 2;                                   // [C][DK] queries
     uint16_t* p_lds = reinterpret_cast<uint16_t*>(qimg + C * KROW);            // [hi | lo][C][PLD] weights
     __shared__ float pw[C + 1];                                                // decay^0 .. decay^C
-    auto swz = [](int r) { return kOdd ? ((r >> 1) & 7) : (r & 7); };
+    auto swz = [](int r) { return r & 7; };
     auto swzv = [](int r) { return (r >> 1) & 7; };
     const int32_t* ch = a.chunks + 4 * blockIdx.x;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
@@ -103,10 +103,9 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
             vr[j] = ok ? *reinterpret_cast<const u32x4*>(qkv + (int64_t)(row0 + t0 + r) * a.qkv_stride + v_off + c) : zero;
         }
     };
-    if constexpr (kAhead) fetch(0);
     for (int t0 = 0; t0 < n_rows; t0 += C) {
         const int n = n_rows - t0 < C ? n_rows - t0 : C;
-        if constexpr (!kAhead) fetch(t0);
+        fetch(t0);
         // (silu(0) = 0: rows past the end stay zero)
 #pragma unroll
         for (int j = 0; j < NQ; ++j) {
@@ -118,9 +117,6 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
         for (int j = 0; j < NV; ++j) {
             const int e = j * 256 + tid, r = e >> 3, pc = e & 7;
             *reinterpret_cast<u32x4*>(vimg + r * VS * 2 + (pc ^ swzv(r)) * 16) = silu8(vr[j]);
-        }
-        if constexpr (kAhead) {
-            if (t0 + C < n_rows) fetch(t0 + C);
         }
         lds_only_barrier();
         const int tr = 4 * lg + (lq >> 2), tp = lq & 3;                        // transposed reads: row and column quarter this lane addresses
@@ -261,14 +257,14 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
 }
 
 // ------------------------------------------------------------------------------------------------ the same walk with two kinds of waves
-// Half of the waves prepare: rows of the next chunk from registers through silu into the images, its weights.  The others consume: 16 value columns each, state
-// and outputs of this chunk.  Two halves a chunk, one barrier behind each:
+// Four waves prepare: rows of the next chunk from registers through silu into the images, its weights.  The others, four or eight, consume: 16 value columns each,
+// state and outputs of this chunk.  Two halves a chunk, one barrier behind each:
 //   consume: o(i) = S^T q + weights v                | S(i) behind the chunk
 //   prepare: q, k of chunk i + 1 into its images     | weights of chunk i + 1, its values
 // Images are double (chunk parity), the weights are written in the half in which nobody reads them; rows are asked for a whole chunk before they are prepared.
 // What bounds it is issue (a wave alone issues a vector instruction every 5.5 cycles, three together every 2.7) and, with all CUs busy, the rows that all ask for at
-// once; so a workgroup has three waves per SIMD and takes 16 CW columns: queries and keys are prepared once for all of them (the 64-column walk below prepares them
-// for every 64).  A chunk takes 3.8 us alone and 5.0 on all CUs, 9.1 for two workgroups of the 64-column walk; 16 prompts of 1024 tokens on average, 16 heads of
+// once; so a workgroup has three waves per SIMD and takes 16 CW columns, 128 where they come in such numbers: queries and keys are prepared once for all of them,
+// not for every 64.  A chunk takes 3.8 us alone and 5.0 on all CUs, 9.1 for two workgroups of the 64-column walk; 16 prompts of 1024 tokens on average, 16 heads of
 // 128: 251 -> 108 us; 40 prompts of 410: 302 -> 157.  Measured and not better: eight waves with 32 columns each (121), sixteen waves (114), fragments read a step
 // ahead by hand (121).
 template <int DK, int CW>
@@ -730,14 +726,13 @@ __global__ __launch_bounds__(256) void norm_gate_kernel(T* __restrict__ out, uin
     }
 }
 
-template <int DK>
-int walk_dk(const LightningArgs& a, hipStream_t stream) {
-    constexpr size_t sum_lds = (size_t)C * (DK + VS) * 2, lds = sum_lds + (size_t)C * DK * 2 + (size_t)2 * C * PLD * 2;
+int walk_wide(const LightningArgs& a, hipStream_t stream) {
+    constexpr size_t sum_lds = (size_t)C * (kWide + VS) * 2, lds = sum_lds + (size_t)C * kWide * 2 + (size_t)2 * C * PLD * 2;
     if (lds > 64 * 1024)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_walk_kernel<DK, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_walk_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const dim3 grid(a.n_chunks, a.heads, a.dv / VS);
     if (a.summaries) {
-        lightning_walk_kernel<DK, true><<<grid, 256, sum_lds, stream>>>(a);
+        lightning_walk_kernel<true><<<grid, 256, sum_lds, stream>>>(a);
         int rc = check_launch("lightning summary");
         if (rc) return rc;
         const int64_t per = (int64_t)a.heads * a.dk * a.dv;
@@ -745,7 +740,7 @@ int walk_dk(const LightningArgs& a, hipStream_t stream) {
         rc = check_launch("lightning starts");
         if (rc) return rc;
     }
-    lightning_walk_kernel<DK, false><<<grid, 256, lds, stream>>>(a);
+    lightning_walk_kernel<false><<<grid, 256, lds, stream>>>(a);
     return check_launch("lightning walk");
 }
 
@@ -794,7 +789,7 @@ int launch_lightning_chunks(const LightningArgs& a, int f32, int generic, hipStr
         switch (a.dk) {
             case 64: return a.dv % 128 == 0 ? pair_dk<64, 8, 4>(a, stream) : pair_dk<64, 4, 4>(a, stream);
             case 128: return a.dv % 128 == 0 ? pair_dk<128, 8, 4>(a, stream) : pair_dk<128, 4, 4>(a, stream);
-            default: return walk_dk<256>(a, stream);
+            default: return walk_wide(a, stream);
         }
     }
     const size_t lds = ((size_t)a.dk * 34 + 256) * 4;

@@ -722,9 +722,7 @@ __global__ __launch_bounds__(64 * FW) void linear_few_kernel(const uint16_t* __r
     float* const part = xs + R * p_K;                                          // [waves][4 columns][R], then a spare piece
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane & 15, tiles = p_N / 4;
     if ((int)blockIdx.x >= tiles) {
-        const int idx = (int)blockIdx.x - tiles, n = (int)gridDim.x - tiles;
-        if (a.pf_kv.k_cache) prefetch_kv_images(a.pf_kv, idx, n, tid, TPB, few_lds);
-        if (a.pf_ptr) prefetch_lines(a.pf_ptr, a.pf_bytes, idx, n, tid, TPB);
+        prefetch_lines(a.pf_ptr, a.pf_bytes, (int)blockIdx.x - tiles, (int)gridDim.x - tiles, tid, TPB);
         return;
     }
     const int col = 4 * (int)blockIdx.x + (lane >> 4), steps = p_K / 128, s0 = steps * wave / FW, s1 = steps * (wave + 1) / FW;
@@ -792,7 +790,7 @@ template <int R, int CH>
 int few_launch(const LinearArgs& a, hipStream_t stream) {
     const size_t lds = (size_t)(R * a.K + FW * 4 * R + 8) * 4;
     if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(linear_few_kernel<R, CH>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    const bool ahead = (a.pf_ptr && a.pf_bytes >= 128) || a.pf_kv.k_cache;       // (workgroups that only prefetch share the CUs: 128 of them end no later than the others)
+    const bool ahead = a.pf_ptr && a.pf_bytes >= 128;            // (workgroups that only prefetch share the CUs: 128 of them end no later than the others)
     linear_few_kernel<R, CH><<<a.N / 4 + (ahead ? 128 : 0), 64 * FW, lds, stream>>>(a.w, a.x, a.K, a.N, a.M, a.x_packed ? 0 : a.M == 1 ? a.K : (int)a.x_stride, (int)a.out_stride, a.out, a.out_packed,
                                                                                        a);
     return check_launch("linear_few");

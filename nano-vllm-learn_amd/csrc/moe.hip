@@ -657,9 +657,10 @@ int launch_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, con
 }
 
 // Rows of a tile.  From 256 pairs an expert on, 256: twice the products per byte of weights and rows read.  From 100 to 192 too: an expert's pairs mostly fit one tile, whose
-// missing rows cost little, where many take two of 128.  2048 wide, 32 experts of 1536, softmax router: 125 pairs an expert 203 us against 254, 187
-// 234 against 268; 1024 wide, 187: 88 against 96.  Below, 128: 75 pairs 197 both (1024 wide 72 against 68); in between many an expert needs a second tile of 256: 250 pairs
-// 321 against 319 (1024 wide 122 against 109).
+// missing rows cost little, where many take two of 128.  2048 wide, 32 experts of 1536, softmax router: 100 pairs an expert 194 us against 220, 125
+// 217 against 252, 187 240 against 269; 1024 wide (768): 77 against 80, 80 against 91, 87 against 95.  Below, 128: 75 pairs 197 both (1024 wide 72 against 68).  From 193 to 255
+// an expert's pairs come out on either side of 256, and a second, mostly empty tile costs what the first one gives: 200 pairs still 262 against 285 (1024 wide
+// 89 against 104), 250 pairs 315 against 323 but 1024 wide 122 against 109; there 128 stays.
 int moe_tile_rows(int pairs, int experts, int f32) {
     const int mean = pairs / experts;
     return f32 ? FM : mean >= 256 || (mean >= 100 && mean <= 192) ? 256 : 128;

@@ -14,7 +14,7 @@
 // Decode (launch_rglru_step): one workgroup per 16 channels and 32 sequences does all of it in one launch.  Convolution inputs live in a ring of
 // `taps` entries (input of position p at entry p % taps): the entry a step writes is the one no workgroup of that step reads.
 // A sequence's first token (position 0) takes state and earlier inputs as zero instead of reading them: slots need no clearing when reused.
-// Bytes per (token, channel) of a walk: 2 (x) + 2 (y) + 2 (out); about 50 vector instructions, 8 of them transcendental: issue-bound.
+// Bytes per (token, channel) of a walk: 2 (x) + 2 (y) + 2 (out); about 25 vector instructions and 8 transcendentals: issue-bound.
 #include "hybrid.h"
 
 namespace nvh {
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(1024) void rglru_walk_kernel(const RglruArgs a) {
 // reached by 32-bit offsets from a step's first one; the 16-token passes are unrolled and find everything at fixed distances.  One barrier behind the scan frees u and
 // makes out whole, one behind the rows' way out and the next convolution frees x.
 // Four blocks of 256 channels, 16 sequences of 1024 tokens as whole portions: 200 -> 148 us; of 32 channels 66 -> 59; 16384 tokens of 16 uneven sequences, 10 blocks
-// of 256, split: 302 -> 230.
+// of 256, split: 316 -> 250 (230 to 260, with the lengths).
 constexpr int HALO = 8;                              // rows in front of a step's 64 in the x image: taps <= HALO + 1
 
 __device__ __forceinline__ int fresh(int v) {         // computed again from here on instead of held in registers across the loop

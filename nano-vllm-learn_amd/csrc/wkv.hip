@@ -65,7 +65,8 @@ struct WkvLds {
 //   consume: outputs, state, sums of squares | norm, gate, store          |
 //   prepare: log decays of chunk i + 1       | images, tables of i + 1    | weights of i + 1
 // What bounds it is issue and latency, not memory: a wave alone issues a vector instruction every 5.5 cycles, four together every 2.3 to 3.3, so two workgroups per CU
-// (heads of 64: 62 KB and 128 registers each) keep four waves on every SIMD; no register may be spilled inside the loop, a reload waits for every row in flight.
+// (heads of 64: 62 KB and 128 registers each) keep four waves on every SIMD; no register of theirs may be spilled inside the loop, a reload waits for every row in
+// flight.  (Heads of 128: 16 waves and 108 KB, one workgroup per CU; at 128 registers some are spilled.)
 // A chunk of a head of 64 takes 4.0 us alone and 7.8 beside a second one (6.8 and 13.9 with one kind of wave, 275 registers and one workgroup per CU); 11 portions of
 // 1090 tokens on average, 32 heads: 274 -> 153 us, 40 prompts of 410: 384 -> 166; heads of 128 about half the time.
 // Off: bytes from a chunk's first row.  32 bits where 64 rows fit them: a sequence of 1536 tokens takes 102.5 us against 106.1 in 64 bits, eight of them 122.5 against 128.

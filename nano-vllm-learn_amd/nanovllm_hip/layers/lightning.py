@@ -12,7 +12,8 @@ from .linear import linear, padded, round_up
 
 
 class LightningAttention(nn.Module):
-    # workgroups that walk one segment: one per head and 128 value columns, 64 where the columns or the keys' width leave no other choice
+    # Workgroups that walk one segment: one per head and 128 value columns, 64 where the columns or the keys' width leave no other choice.  (Of 64 keys and 64 columns two
+    # fit a CU, but counting pairs of them chooses worse: over ten mixes of 1 to 40 sequences 1.09 to 1.10 times the best segment's walks at 8 and 16 heads, counted singly 1.01 to 1.02)
     segment_units = property(lambda self: self.heads * max(1, self.dv // (128 if self.dv % 128 == 0 and self.dk <= 128 else 64)))
 
     def __init__(self, in_width, in_cols, heads, dim, vdim, decay, eps, dtype, passes=1):

@@ -17,7 +17,7 @@ MIXES = ("r", "k", "v", "g", "w")
 class TimeMixing(nn.Module):
     mixes = MIXES
     # What choose_segment takes for workgroups that walk one segment: it counts one per CU.  A workgroup has a head: of 64 channels, two share a CU; of 128, one
-    # needs 16 waves and 110 KB of LDS.  Over ten mixes of 1 to 40 sequences the choice costs 1.04 times the best segment's walks for 32 heads of 64 (counted
+    # needs 16 waves and 108 KB of LDS.  Over ten mixes of 1 to 40 sequences the choice costs 1.04 times the best segment's walks for 32 heads of 64 (counted
     # by heads 1.09), 1.01 for 8 and 16 heads of 128 (counted by pairs of heads 1.10 and 1.12: 16 sequences of 1024 tokens on average were cut, 739 us against 498)
     segment_units = property(lambda self: self.heads if self.dk > 64 else max(1, self.heads // 2))
 

@@ -290,7 +290,7 @@ def test_stream_linear_split_k_residual_add(m, n, k):
     assert int(ws[: tiles * 128].view(torch.int32).abs().sum()) == 0       # one ticket per 128-byte line, all back at zero
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 32, 1152), (2, 64, 2048), (3, 1024, 3072), (4, 512, 3072), (1, 896, 4864), (2, 896, 4864), (1, 96, 6272), (1, 64, 8192), (1, 32, 12288), (2, 32, 6144)])
+@pytest.mark.parametrize("m,n,k", [(1, 32, 1152), (2, 64, 2048), (3, 1024, 3072), (4, 512, 3072), (1, 896, 4864), (2, 896, 4864), (1, 96, 6272), (1, 64, 8192), (1, 32, 12288), (2, 32, 6144), (3, 64, 4096)])
 def test_stream_linear_few_rows_residual_add(m, n, k):
     """Up to four rows of a long K: within one bf16 rounding of the fp32 reference, the same bits from packed and row-major rows and beside a prefetch, no ticket
     touched, packed rows past the last one left alone."""

@@ -27,12 +27,17 @@ extern "C" {
 int nvh_rglru_chunk_tokens(void) { return kRglruChunk; }
 int nvh_rglru_step_supported(int block) { return block > 0 && block % 32 == 0 && rglru_step_supported(block); }
 
+int64_t nvh_rglru_link_bytes(int block, int blocks, int taps, int max_steps, int dtype) {
+    return block > 0 && blocks > 0 && taps >= 1 ? rglru_link_bytes(block, blocks, taps, max_steps, dtype == NVH_F32) : 0;
+}
+
 int nvh_rglru_chunks(const nvh_rglru_desc* d, int generic, int dtype, void* stream) {
     REQUIRE(d, NVH_E_NULL, "rglru_chunks: null descriptor");
     if (d->n_chunks == 0) return 0;
     const int rc = check_rglru("rglru_chunks", d, dtype);
     if (rc) return rc;
     REQUIRE(d->chunks && d->s_loc && d->a_cum && d->out && d->n_chunks > 0, NVH_E_NULL, "rglru_chunks: null pointer");
+    REQUIRE(!d->links || aligned16(d->links), NVH_E_ALIGN, "rglru_chunks: scratch must be 16-byte aligned");
     REQUIRE(d->segment > 0 && d->segment % kRglruChunk == 0, NVH_E_SHAPE, "rglru_chunks: segment %d must be a positive multiple of %d", d->segment, kRglruChunk);
     REQUIRE(!d->out_packed, NVH_E_SHAPE, "rglru_chunks: packed output belongs to the step form");
     REQUIRE(aligned16(d->s_loc) && aligned16(d->a_cum), NVH_E_ALIGN, "rglru_chunks: scratch must be 16-byte aligned");

@@ -49,6 +49,7 @@ using RglruArgs = nvh_rglru_desc;
 int launch_rglru_chunks(const RglruArgs& a, int f32, int generic, hipStream_t stream);
 int launch_rglru_step(const RglruArgs& a, int rows, hipStream_t stream);
 bool rglru_step_supported(int block);
+int64_t rglru_link_bytes(int block, int blocks, int taps, int max_steps, int f32);   // 0: the chained form does not take it
 
 // ---- latent attention (latent_attention.hip, latent_prefill.hip)
 using LatentPrepArgs = nvh_latent_prep_desc;

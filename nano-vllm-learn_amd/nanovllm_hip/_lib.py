@@ -47,7 +47,8 @@ class RglruDesc(ctypes.Structure):
                 ("ra", ctypes.c_void_p), ("ri", ctypes.c_void_p), ("ra_b", ctypes.c_void_p), ("ri_b", ctypes.c_void_p),
                 ("rate", ctypes.c_void_p), ("chunks", ctypes.c_void_p), ("n_chunks", ctypes.c_int32), ("segment", ctypes.c_int32), ("summaries", ctypes.c_int32), ("positions", ctypes.c_void_p),
                 ("state_slots", ctypes.c_void_p), ("state", ctypes.c_void_p), ("conv_state", ctypes.c_void_p), ("s_loc", ctypes.c_void_p),
-                ("a_cum", ctypes.c_void_p), ("out", ctypes.c_void_p), ("out_stride", ctypes.c_int64), ("out_packed", ctypes.c_void_p)]
+                ("a_cum", ctypes.c_void_p), ("out", ctypes.c_void_p), ("out_stride", ctypes.c_int64), ("out_packed", ctypes.c_void_p),
+                ("links", ctypes.c_void_p), ("max_steps", ctypes.c_int32)]
 
 
 class LatentPrepDesc(ctypes.Structure):
@@ -273,6 +274,7 @@ _SIGS = {
     "nvh_gelu_glu": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 + [ctypes.c_int64] * 2 + [ctypes.c_int, ctypes.c_void_p]),
     "nvh_rglru_chunk_tokens": (ctypes.c_int, []),
     "nvh_rglru_step_supported": (ctypes.c_int, [ctypes.c_int]),
+    "nvh_rglru_link_bytes": (ctypes.c_int64, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "nvh_rglru_chunks": (ctypes.c_int, [ctypes.POINTER(RglruDesc), ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
     "nvh_rglru_step": (ctypes.c_int, [ctypes.POINTER(RglruDesc), ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
     "nvh_latent_prep": (ctypes.c_int, [ctypes.POINTER(LatentPrepDesc), ctypes.c_int, ctypes.c_void_p]),

@@ -717,7 +717,11 @@ def rglru_chunks(yx, params, positions, state_slots, chunks, segment, summaries,
     d.chunks, d.n_chunks, d.s_loc, d.a_cum = chunks.data_ptr(), chunks.shape[0], scratch[0].data_ptr(), scratch[1].data_ptr()
     d.segment, d.summaries = int(segment), int(summaries)
     d.out, d.out_stride = out.data_ptr(), out.stride(0)
-    _lib.check(_lib.load().nvh_rglru_chunks(ctypes.byref(d), int(generic), code, _stream()), "nvh_rglru_chunks")
+    lib = _lib.load()
+    steps = chunks.shape[0] + rows // lib.nvh_rglru_chunk_tokens()
+    links = torch.empty(lib.nvh_rglru_link_bytes(d.block, d.blocks, d.taps, steps, code), dtype=torch.uint8, device=yx.device)
+    d.links, d.max_steps = links.data_ptr() if links.numel() else None, steps
+    _lib.check(lib.nvh_rglru_chunks(ctypes.byref(d), int(generic), code, _stream()), "nvh_rglru_chunks")
     return out
 
 

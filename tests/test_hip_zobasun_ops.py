@@ -255,6 +255,53 @@ def test_recurrence_many_segments():
     assert torch.equal(out, few.repeat(n // 7 + 1, 1)[:n]) and few.any(dim=1).all()
 
 
+@pytest.mark.parametrize("blocks,block,taps", [(2, 32, 4), (2, 96, 9), (2, 160, 1), (3, 256, 4), (12, 256, 8)])
+@pytest.mark.parametrize("lengths", [(4500,), (300, 1, 64, 129, 700, 65, 128), (70,) * 300], ids=["one", "uneven", "many"])
+def test_recurrence_steps_by_any_workgroup(blocks, block, taps, lengths):
+    """Steps that workgroups draw against the walks: one portion of more steps than a look back covers, uneven ones, more segments than are ordered by step; in segments
+    and whole, from states of their own, some infinite.  What a step starts from is summed in one order, so that runs and replays of a graph agree bit for bit."""
+    from nanovllm_hip import ops
+    from nanovllm_hip.engine.model_runner import recurrence_chunks
+    n, total = len(lengths), sum(lengths)
+    r = Recurrence(blocks, block, block, taps, torch.bfloat16, slots=n + 1)
+    r.state.normal_(), r.conv_state.normal_()
+    r.state[n // 2, 5] = float("inf")
+    yx, first = r.rows(*r.yx(total, 1)), [sum(lengths[:i]) for i in range(n)]
+    pos = torch.cat([torch.arange(i % 3, i % 3 + m) for i, m in enumerate(lengths)]).cuda()
+    slots = torch.arange(n, dtype=torch.int32, device="cuda").flip(0).contiguous()
+
+    def run(segment, form, pools):
+        table = [c for i, m in enumerate(lengths) for c in recurrence_chunks(first[i], m, i, segment)]
+        chunks = torch.tensor(table, dtype=torch.int32, device="cuda")
+        return lambda: ops.rglru_chunks(yx, r.params, pos, slots, chunks, segment, any(k for *_, k in table), *pools, generic=form)
+
+    def pools():
+        return r.state.clone(), r.conv_state.clone()
+    wanted = pools()
+    want = run(64, 2, wanted)()
+    first_run = None
+    for segment in (64, 8192):
+        after = pools()
+        go = run(segment, 0, after)
+        got = go()
+        infinite = ~torch.isfinite(want)                        # (walks lose an infinite state to NaN where decays multiply to zero)
+        assert ((got - want)[~infinite].abs() <= 2 ** -7 * want[~infinite].abs() + 1e-3).all() and (~torch.isfinite(got[infinite])).all()
+        fine = torch.isfinite(wanted[0])
+        assert (after[0] - wanted[0])[fine].abs().max() <= 2e-5 * wanted[0][fine].abs().max() and torch.equal(after[1], wanted[1]) and not torch.isnan(after[0]).any()
+        if first_run is not None and max(lengths) > 320:        # (otherwise whole portions may be walked)
+            assert torch.equal(got, first_run[0]) and torch.equal(after[0], first_run[1])
+        first_run = got.clone(), after[0].clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            again = go()
+        for _ in range(3):
+            for p, start in zip(after, pools()):
+                p.copy_(start)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(again, first_run[0]) and torch.equal(after[0], first_run[1])
+
+
 @pytest.mark.parametrize("blocks,size,block,taps", SHAPES)
 def test_recurrence_step_follows_portions(blocks, size, block, taps):
     """Prompt by the chunked form, then single tokens by the step form (one sequence steps from its very first token)."""

@@ -244,6 +244,128 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
     for (int s = 0; s < NS; s += 4) *reinterpret_cast<f32x4*>(dst + sl * NS + s) = f32x4{S[s], S[s + 1], S[s + 2], S[s + 3]};
 }
 
+// ------------------------------------------------------------------------------------------------ whole portions, 16 states (bf16)
+// Where the waves of whole portions, with four states a lane, would leave the GPU idle: a state per lane, four times as many waves and no pass over segments in front.
+// A row of 16 lanes is a channel, a wave four of them.  dt and dt x of 16 tokens lie one per lane of the row and reach all of it as an operand's row broadcast; a
+// token's 16 products with C are added up for 16 tokens at once, so that each lane ends with its token's y, and D x, gate and store follow there.
+// Bound by vector issue (a lane-crossing addition takes as long as two plain ones, so that a filled GPU is 6 to 13 % slower with it than with four states a lane) and, for few
+// portions, by a wave's own pace: 42 ns a token.  16384 tokens of 5 sequences, 2048 channels: 280 (segments, two passes) -> 230 us; of 16: 252 -> 198; 7000 tokens
+// of 5, 4096 channels: 225 -> 161; 2400 of 9, 2048 channels: 52 -> 35.
+constexpr int ROW_TT = 64, ROW_CHN = 16, ROW_LD = ROW_TT + 4;
+
+template <int J>
+__device__ __forceinline__ float row_lane(float v) { return dpp_f32<0x150 + J>(v); }           // lane J of the row
+
+// lane i of each row: the sum over the row of p[i].  Two tokens share a register from the first addition on (banks of four lanes that an addition leaves alone keep the other
+// token's sum); in front of the block and inside it two instructions or more lie between a register's write and its reading across lanes.
+__device__ __forceinline__ float row_sums(float (&p)[16], int lane) {
+    asm("s_nop 1\n"
+        "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+        "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+        "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+        "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+        "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %4, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+        "v_add_f32_dpp %5, %5, %5 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %5, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+        "v_add_f32_dpp %6, %6, %6 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %6, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+        "v_add_f32_dpp %7, %7, %7 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %7, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+        "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0x5\n v_add_f32_dpp %0, %4, %4 row_half_mirror row_mask:0xf bank_mask:0xa\n"
+        "v_add_f32_dpp %1, %1, %1 row_half_mirror row_mask:0xf bank_mask:0x5\n v_add_f32_dpp %1, %5, %5 row_half_mirror row_mask:0xf bank_mask:0xa\n"
+        "v_add_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0x5\n v_add_f32_dpp %2, %6, %6 row_half_mirror row_mask:0xf bank_mask:0xa\n"
+        "v_add_f32_dpp %3, %3, %3 row_half_mirror row_mask:0xf bank_mask:0x5\n v_add_f32_dpp %3, %7, %7 row_half_mirror row_mask:0xf bank_mask:0xa\n"
+        "s_nop 1"
+        : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7])
+        : "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
+    const bool b1 = lane & 1, b2 = lane & 2;
+    float u[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const float lo = p[2 * t] + dpp_f32<0xB1>(p[2 * t]), hi = p[2 * t + 1] + dpp_f32<0xB1>(p[2 * t + 1]);    // quad_perm [1,0,3,2]
+        u[t] = b1 ? hi : lo;
+    }
+    const float lo = u[0] + dpp_f32<0x4E>(u[0]), hi = u[1] + dpp_f32<0x4E>(u[1]);                                // quad_perm [2,3,0,1]
+    return b2 ? hi : lo;
+}
+
+__global__ __launch_bounds__(256) void scan_rows_kernel(const ScanArgs a) {
+    __shared__ __attribute__((aligned(16))) uint16_t x_s[ROW_TT * ROW_CHN], d_s[ROW_TT * ROW_CHN], z_s[ROW_TT * ROW_CHN];
+    __shared__ __attribute__((aligned(16))) float bc_s[32 * ROW_LD];           // [B 0..15 | C 0..15][token]
+    const int seg = blockIdx.y, groups = gridDim.x;
+    const int32_t* chk = a.chunks + 4 * seg;
+    const int row0 = chk[0], n_rows = chk[1];
+    if (n_rows <= 0) return;
+    const int64_t slot = a.state_slots[chk[2]];
+    // neighbouring channels' 32-byte pieces of a row share lines: they go to one XCD (workgroups are dealt round-robin)
+    const int g = groups % 8 ? blockIdx.x : blockIdx.x % 8 * (groups / 8) + blockIdx.x / 8, c0 = g * ROW_CHN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, st = lane & 15, lc = 4 * wave + (lane >> 4);
+    const int my = c0 + lc < a.inner ? c0 + lc : a.inner - 1;
+    const float A = a.a_log2[(int64_t)my * 16 + st], bias = a.dt_bias[my], D = a.d[my];
+    float S = 0.f;
+    if (slot >= 0 && a.positions[row0] > 0) S = a.state[(slot * a.inner + my) * 16 + st];
+    // ---- this thread's pieces: x and z (tid < 128), dt; and 8 of a token's B | C
+    const int pt = (tid & 127) >> 1, pc = c0 + (tid & 1) * 8, pcc = pc < a.inner ? pc : a.inner - 8, bt = tid >> 2, bp = tid & 3;
+    const bool low = tid < 128;
+    const uint16_t* from = reinterpret_cast<const uint16_t*>(low ? a.x : a.dt) + pcc;
+    const int64_t from_stride = low ? a.x_stride : a.dt_stride;
+    u32x4 r0, r1, rb;
+    auto fetch = [&](int t0) __attribute__((always_inline)) {                  // rows past the end: the last one again
+        const int top = n_rows - 1;
+        const int64_t r = row0 + (t0 + pt < top ? t0 + pt : top);
+        r0 = *reinterpret_cast<const u32x4*>(from + r * from_stride);
+        r1 = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(a.z) + r * a.z_stride + pcc);
+        rb = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(a.bc) + (int64_t)(row0 + (t0 + bt < top ? t0 + bt : top)) * a.bc_stride + bp * 8);
+    };
+    fetch(0);
+    for (int t0 = 0; t0 < n_rows; t0 += ROW_TT) {
+        const int n = n_rows - t0 < ROW_TT ? n_rows - t0 : ROW_TT;
+        *reinterpret_cast<u32x4*>((low ? x_s : d_s) + (tid & 127) * 8) = r0;
+        if (low) *reinterpret_cast<u32x4*>(z_s + tid * 8) = r1;
+        if (bt >= n) rb = u32x4{0, 0, 0, 0};                     // rows past the end count nothing, not even infinite ones
+        {
+            const f32x8 v = unpack8(rb);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                bc_s[(8 * bp + i) * ROW_LD + bt] = v.a[i];
+                bc_s[(8 * bp + 4 + i) * ROW_LD + bt] = v.b[i];
+            }
+        }
+        __syncthreads();
+        fetch(t0 + ROW_TT);
+        for (int k = 0; k < n; k += 16) {
+            const int e = (k + st) * ROW_CHN + lc;
+            const float xv = act_ld(x_s + e), zv = act_ld(z_s + e);
+            float dt = softplus_f(act_ld(d_s + e) + bias), dx = dt * xv;
+            if (k + st >= n) dt = 0.f, dx = 0.f;     // (a token past the end leaves the state alone)
+            const float* b_row = bc_s + st * ROW_LD + k;
+            float p[16];
+            auto token = [&](auto j, float b, float c) __attribute__((always_inline)) {
+                constexpr int J = decltype(j)::value;
+                float in = row_lane<J>(dx) * b;      // (the broadcast is an operand of the multiplication, as long as that is not merged into the sum)
+                asm("" : "+v"(in));
+                S = fast_exp2(row_lane<J>(dt) * A) * S + in;
+                p[J] = S * c;
+            };
+            auto four = [&](auto q) __attribute__((always_inline)) {
+                constexpr int Q = decltype(q)::value;
+                const f32x4 b = *reinterpret_cast<const f32x4*>(b_row + 4 * Q), c = *reinterpret_cast<const f32x4*>(b_row + 16 * ROW_LD + 4 * Q);
+                token(std::integral_constant<int, 4 * Q>(), b[0], c[0]);
+                token(std::integral_constant<int, 4 * Q + 1>(), b[1], c[1]);
+                token(std::integral_constant<int, 4 * Q + 2>(), b[2], c[2]);
+                token(std::integral_constant<int, 4 * Q + 3>(), b[3], c[3]);
+            };
+            four(std::integral_constant<int, 0>());
+            four(std::integral_constant<int, 1>());
+            four(std::integral_constant<int, 2>());
+            four(std::integral_constant<int, 3>());
+            act_st(z_s + e, (row_sums(p, lane) + D * xv) * gate_f(zv));
+        }
+        __syncthreads();
+        if (low && pt < n && pc < a.inner)
+            *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(a.out) + (int64_t)(row0 + t0 + pt) * a.out_stride + pc) = *reinterpret_cast<const u32x4*>(z_s + tid * 8);
+        // (this thread puts the next z where it has just read)
+    }
+    if (c0 + lc < a.inner && slot >= 0) a.state[(slot * a.inner + my) * 16 + st] = S;
+}
+
 // contributions of the segments -> states at their starts, in place; one thread per state, walking the segments of every portion
 __global__ __launch_bounds__(256) void scan_starts_kernel(const ScanArgs a) {
     const int64_t per = (int64_t)a.inner * a.n, e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -343,7 +465,18 @@ int walk_t(const ScanArgs& a, hipStream_t stream) {
     // 64 states 420 with 4 lanes, 506 with 8.
     switch (a.n) {
         case 8: return walk_ns<T, 4, 2>(a, stream);
-        case 16: return walk_ns<T, 4, 4>(a, stream);
+        case 16:
+            // Four states a lane fill the GPU from about four waves on every SIMD on (portions x channels / 16384), with long portions from two and a half.
+            // Whole portions, one against four states a lane: 23 of 200 tokens, 2048 channels (2.9 waves) 59 to 64 us; 13 of 250, 4096 channels (3.25) 74 to 77; 31 of 100 (3.9) 41 to 40; 17
+            // of 200, 4096 channels (4.25) 82 to 71; 8 of 600 (2.0) 108 to 116, 10 of 790 (2.5) 180 to 173.
+            if constexpr (sizeof(T) == 2) {
+                const int64_t fill = (int64_t)a.n_chunks * a.inner;
+                if (!a.summaries && (fill < 40960 || (fill < 65536 && a.rows / a.n_chunks < 512))) {
+                    scan_rows_kernel<<<dim3((a.inner + 15) / 16, a.n_chunks), 256, 0, stream>>>(a);
+                    return check_launch("scan rows");
+                }
+            }
+            return walk_ns<T, 4, 4>(a, stream);
         case 32: return walk_ns<T, 8, 4>(a, stream);
         case 64: return walk_ns<T, 16, 4>(a, stream);
         case 128: return walk_ns<T, 16, 8>(a, stream);

@@ -11,12 +11,30 @@ from .. import ops
 from .linear import linear, padded, round_up
 
 
+class ScanUnits(int):
+    """What choose_segment takes for workgroups that walk one segment, of a layer whose whole portions have a kernel of their own."""
+
+    def __new__(cls, units, channels):
+        self = super().__new__(cls, units)
+        self.channels = channels
+        return self
+
+    def whole(self, portions):
+        """Portions few enough for a state per lane that are scanned as fast in one pass as in segments: in microseconds 42 ns a token of the longest, or the load of all and part of
+        that, against two passes over the load.  Over 44 mixes the choice costs 1.002 times the faster of both, and takes 0.86 of the time of segments alone."""
+        total, longest = sum(portions) * self.channels, max(portions)
+        return len(portions) * self.channels < 40960 and max(0.042 * longest, 4.6e-6 * total + 0.0168 * longest) < 22 + 7.2e-6 * total
+
+
 class SelectiveScan(nn.Module):
     # What choose_segment takes for workgroups that walk one segment: it counts one per CU, and many of the scan's small ones share one (of 128 channels at 8 states, 64
     # up to 64, 32 at 128, 16 at 256).  By states: times 1024 channels.  Over ten mixes of 1 to 40 sequences the choice costs, times the best segment's walks, for
     # 4096 / 2048 channels: 8 states 1.01 / 1.01 (counted as 16 states 1.16 / 1.10), 16 to 64 states 1.07 to 1.08 / 1.09 to 1.12 at 32 and 64 (6 units instead of 4:
     # 1.03 / 1.15), 128 states 1.01 / 1.03 (as 16: 1.14 / 1.09); 2048 / 1024 channels of 256 states 1.01 / 1.03 (as 16: 1.23 / 1.06)
-    segment_units = property(lambda self: max(1, self.inner_cols * {8: 1, 128: 12, 256: 24}.get(self.n, 4) // 1024))
+    @property
+    def segment_units(self):
+        units = max(1, self.inner_cols * {8: 1, 128: 12, 256: 24}.get(self.n, 4) // 1024)
+        return ScanUnits(units, self.inner_cols) if self.n == 16 and self.dtype == torch.bfloat16 else units
 
     def __init__(self, in_width, in_cols, inner, states, rank, taps, dtype):
         super().__init__()

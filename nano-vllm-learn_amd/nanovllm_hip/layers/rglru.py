@@ -43,6 +43,8 @@ def choose_segment(portions, blocks, chunk=64):
         ahead = walks - len(portions)                # segments in front of others
         walk = launch(walks, total, min(k, last))
         return walk + SPLIT_OVERHEAD + SUMMARY_SHARE * launch(ahead, ahead * k, k) if ahead else walk
+    if hasattr(blocks, "whole") and portions and blocks.whole(portions):
+        return chunk * last                          # (a kernel of its own for them)
     steps, k = [last], 1
     while k < last:
         steps.append(k)

@@ -243,6 +243,17 @@ def test_scan_tile_borders(inner, n, dtype):
             close(state[slots[i], :, :n], s, F32, f"state {i}", slack=4)
 
 
+@pytest.mark.parametrize("inner,n", [(128, 16), (8, 9), (264, 13)])
+def test_scan_a_state_per_lane(inner, n):
+    """Whole portions around 16 and 64 tokens, from the start and behind a state; groups of channels that are dealt over the XCDs, one and a last one that are not full."""
+    lengths, cuts, slots = [1, 15, 16, 17, 65, 129, 80], [[1], [15], [16], [17], [63, 2], [64, 65], [33, 47]], [3, 1, 0, 2, 6, 5, 4]
+    layer = Scan(lengths, inner, n, 8, BF16)
+    got, state = feed_scan(layer, lengths, cuts, slots, 1024)
+    for i, (y, s) in enumerate(layer.want):
+        close(got[i], y, BF16, f"sequence {i}")
+        close(state[slots[i], :, :n], s, F32, f"state {i}", slack=4)
+
+
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("inner,n", [(72, 8), (136, 16), (24, 256)])
 def test_scan_segments_without_rows(inner, n, dtype):

@@ -317,3 +317,14 @@ def test_scan_segments(inner, states, units):
     """The more states a channel has, the fewer channels' walks keep a compute unit busy."""
     from nanovllm_hip.layers.mamba import SelectiveScan
     assert SelectiveScan(64, 64, inner, states, 16, 4, torch.bfloat16).segment_units == units
+
+
+def test_scan_whole_portions():
+    """16 states in bfloat16: portions whose waves leave the GPU idle stay whole unless one is long for what there is to do; many are cut as other layers' are."""
+    from nanovllm_hip.layers.mamba import SelectiveScan
+    from nanovllm_hip.layers.rglru import choose_segment
+    one, other = (SelectiveScan(64, 64, 2048, 16, 16, 4, d).segment_units for d in (torch.bfloat16, torch.float32))
+    for portions, whole in (([4096, 3000, 3000, 3000, 3000], True), ([400] * 9, True), ([3848], False), ([1000] * 18, True), ([4096, *[60] * 17], False), ([], True)):
+        assert (choose_segment(portions, one) >= max(portions, default=0)) == whole
+    long = [4096, *[200] * 39]
+    assert one == other and choose_segment(long, one) == choose_segment(long, other) < 4096

@@ -166,4 +166,23 @@ struct PageNumbers {
     }
 };
 
+// Lane with the nth largest of the values (0 .. 2^BITS - 1) in lanes 0 .. count - 1, equal ones in order; the same in all lanes.  One ballot and a few scalar instructions a bit.
+template <int BITS>
+__device__ __forceinline__ int nth_largest(int value, int count, int nth) {
+    uint64_t in = count >= 64 ? ~0ull : (1ull << count) - 1;
+#pragma unroll
+    for (int bit = BITS - 1; bit >= 0; --bit) {
+        const uint64_t ones = __builtin_amdgcn_ballot_w64(value >> bit & 1) & in;
+        const int c = __builtin_popcountll(ones);
+        if (nth < c) {
+            in = ones;
+        } else {
+            nth -= c;
+            in &= ~ones;
+        }
+    }
+    for (; nth > 0; --nth) in &= in - 1;
+    return __builtin_ctzll(in);
+}
+
 }  // namespace nvh

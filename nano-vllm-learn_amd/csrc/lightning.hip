@@ -284,7 +284,7 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
     __shared__ __attribute__((aligned(16))) float pw[C + 1], fall_s[C];        // decay^0 .. decay^C; decay^(C - 1 - key)
     auto swz = [](int r) { return KROW == 128 ? (r >> 1) & 7 : r & 15; };      // rows of 256 bytes span all banks: 16 of them apart, not 8
     auto swzv = [](int r) { return VROW == 128 ? (r >> 1) & 7 : (2 * r) & 14; };
-    const int seg = blockIdx.y;
+    const int seg = longest_first(a, a.heads * (a.dv / VW));
     const int32_t* ch = a.chunks + 4 * seg;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
     const int slices = a.dv / VW, head = blockIdx.x / slices, v0 = (blockIdx.x - head * slices) * VW;

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
     // 414 against 494 at 64); beyond that the wider rows' bank conflicts cost more than widening on every read (1021 against 928 at 128)
     using L = typename std::conditional<NP <= 64, float, T>::type;
     __shared__ __attribute__((aligned(16))) L bc_s[TT * 2 * NP];
-    const int seg = blockIdx.y;                      // channels run fastest: workgroups are dealt round-robin over the XCDs, and segments differ in length
+    const int seg = longest_first(a, a.inner / CHN);        // channels run fastest: workgroups are dealt round-robin over the XCDs
     const int32_t* ch = a.chunks + 4 * seg;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
     const bool last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;
@@ -289,7 +289,7 @@ __device__ __forceinline__ float row_sums(float (&p)[16], int lane) {
 __global__ __launch_bounds__(256) void scan_rows_kernel(const ScanArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t x_s[ROW_TT * ROW_CHN], d_s[ROW_TT * ROW_CHN], z_s[ROW_TT * ROW_CHN];
     __shared__ __attribute__((aligned(16))) float bc_s[32 * ROW_LD];           // [B 0..15 | C 0..15][token]
-    const int seg = blockIdx.y, groups = gridDim.x;
+    const int seg = longest_first(a, a.inner / ROW_CHN), groups = gridDim.x;
     const int32_t* chk = a.chunks + 4 * seg;
     const int row0 = chk[0], n_rows = chk[1];
     if (n_rows <= 0) return;

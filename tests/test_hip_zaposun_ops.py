@@ -654,3 +654,41 @@ def test_operand_checks():
     assert [ops().scan_states(n) for n in (1, 8, 9, 256, 257)] == [8, 8, 16, 256, 0] and not ops().wkv_supported(96)
     with pytest.raises(RuntimeError, match="x groups"):
         ops().fused_linear(torch.zeros(5 * 16 * 64, dtype=BF16, device="cuda"), torch.zeros(100, 64, dtype=BF16, device="cuda")[:96], x_packed_rows=1, x_groups=(5, 24))
+
+
+@pytest.mark.parametrize("portions", [40, 64, 65])
+@pytest.mark.parametrize("kind", ["scan", "time mixing", "lightning"])
+def test_portions_longest_first(kind, portions):
+    """Portions whose walks do not all have a compute unit of their own start the longest first: each of them once, equal lengths and ones without rows among them, with the bits
+    that it has alone."""
+    gen, rng = torch.Generator().manual_seed(portions), torch.Generator().manual_seed(7)
+    lengths = [(0, 1, 16, 17, 130, 130, 700)[int(torch.randint(7, (1,), generator=rng))] for _ in range(portions)]
+    total, heads, f = sum(lengths), 8, dict(generator=gen)
+    slots, first = torch.randperm(portions, **f).int().cuda(), [sum(lengths[:i]) for i in range(portions)]
+    pos = torch.cat([torch.arange(i % 2 * 5, i % 2 * 5 + n) for i, n in enumerate(lengths)]).cuda()
+
+    def bf16(*shape):
+        return torch.randn(*shape, **f).bfloat16().cuda()
+
+    def f32(*shape):
+        return torch.randn(*shape, **f).cuda()
+    if kind == "scan":
+        x, dt, bc, z, state = bf16(total, 128), bf16(total, 128), bf16(total, 32), bf16(total, 128), f32(portions, 128, 16)
+        p = dict(a_log2=-f32(128, 16).abs(), d=f32(128), dt_bias=f32(128) - 3)
+        def run(rows, *at): return ops().scan_chunks(x[rows], dt[rows], bc[rows], z[rows], p, *at)
+    elif kind == "time mixing":
+        x, state = [bf16(total, 64 * heads) * s for s in (1, 1, 1, 1, 0.3)], f32(portions, heads, 64, 64)
+        p = dict(w0=f32(64 * heads) - 3, u=f32(64 * heads), norm=f32(64 * heads))
+        def run(rows, *at): return ops().wkv_chunks(*(t[rows] for t in x), p, 1e-6, 64, *at)
+    else:
+        x, state, decay = bf16(total, 4 * heads * 128), f32(portions, heads, 128, 128), torch.rand(heads, **f).cuda()
+        def run(rows, *at): return ops().lightning_chunks(x[rows], decay, *at)
+    after, alone = state.clone(), state.clone()
+    table = torch.tensor([(a, n, i, 0) for i, (a, n) in enumerate(zip(first, lengths))], dtype=torch.int32).cuda()
+    got = run(slice(None), pos, slots, table, False, after)
+    for i, (a, n) in enumerate(zip(first, lengths)):
+        if n:
+            rows = slice(a, a + n)
+            want = run(rows, pos[rows], slots[i:i + 1], torch.tensor([(0, n, 0, 0)], dtype=torch.int32).cuda(), False, alone)
+            assert torch.equal(got[rows], want), (i, n)
+    assert torch.equal(after, alone)

@@ -126,6 +126,14 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float a, float b) {
 // and strides), P is rounded to fp16 and P V is ONE v_mfma_f32_16x16x32_f16 per operand pair — no lo half.  Everything else is the same code.
 typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+// Sequence with the `rank`th most work of up to 64 (more: in order): queries times the keys they see, in blocks of 64.
+__device__ __forceinline__ int by_work(const PrefillArgs& a, int rank) {
+    if (a.batch > 64) return rank;
+    const int lane = threadIdx.x & 63, i = lane < a.batch ? lane : 0, q = a.cu_q[i + 1] - a.cu_q[i], k = a.cu_k[i + 1] - a.cu_k[i];
+    const uint32_t work = (uint32_t)((q + 63) >> 6) * (uint32_t)((2 * k - q + 127) >> 7);
+    return nth_largest<14>((int)(work < 16383u ? work : 16383u), a.batch, rank);
+}
+
 // grid (H, B, q-tiles) -> this workgroup's (q-tile, head, sequence).  Workgroups are dispatched x-fastest, so the q-tile index is the SLOW dimension
 // and runs backwards: under the causal mask tile t costs t+1 key tiles, and dispatching the heaviest tiles of every (sequence, head) first leaves
 // the light ones for the tail (census in tools/probes/stamp_prefill.py: the old x = q-tile order spent the last 40 % of the launch draining a
@@ -136,9 +144,11 @@ __device__ __forceinline__ void prefill_tile_of_block(const PrefillArgs& a, int&
     {
         // XCD-aware order (speed only; any mapping is correct): workgroups are dealt round-robin over the 8 XCDs, each with an L2 of its
         // own, so in the plain order the G heads x q-tiles that stream the SAME K/V rows of a (sequence, kv head) pair land on all eight
-        // and each L2 fetches those rows for itself.  Re-deal: linear workgroup id -> (XCD = id % 8, index on that XCD); pair u lives on
-        // XCD u % 8, and on its XCD the order is heads of the group fastest, then the XCD's pairs, then q-tiles heaviest first — so every
-        // XCD still works through the same mix of heavy and light tiles.
+        // and each L2 fetches those rows for itself.  Re-deal: linear workgroup id -> (XCD = id % 8, index on that XCD); the pairs, those of the sequence with the most work
+        // first, are dealt to the XCDs back and forth, and on an XCD the order is heads of the group fastest, then the XCD's pairs, then q-tiles heaviest first — so every
+        // XCD works through as much as any other, and the same mix of heavy and light tiles.  (In the order of the batch an XCD's six of 48 pairs are more or less work by
+        // chance: 24 uneven prompts of 16384 tokens, 14 / 2 heads of 64, 73.6 -> 67.0 us; 16 of 12000, 7 / 1 heads of 128, 63.2 -> 54.8; 8 of 8192 behind cached keys, 28 / 4
+        // heads of 128, 325 -> 309.)
         const int G = a.h / a.kvh, units = (int)gridDim.y * a.kvh, total = (int)(gridDim.x * gridDim.y * gridDim.z);
         if ((units & 7) == 0 && (total & 7) == 0) {
             const int lin = (int)blockIdx.x + (int)gridDim.x * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
@@ -146,10 +156,11 @@ __device__ __forceinline__ void prefill_tile_of_block(const PrefillArgs& a, int&
 #ifdef NVH_PREFILL_PAIR_MAJOR                 // A/B builds: one pair after the other on an XCD (its K/V alone in the L2) instead of all of the XCD's pairs per q-tile rank
             const int g_in = idx % G, r = idx / G, zs = (int)gridDim.z, u = xcd + 8 * (r / zs), z = r % zs;
 #else
-            const int g_in = idx % G, r = idx / G, u = xcd + 8 * (r % per), z = r / per;
+            const int g_in = idx % G, r = idx / G, j = r % per, u = 8 * j + (j & 1 ? 7 - xcd : xcd), z = r / per;
 #endif
             b = u / a.kvh;
             head = (u - b * a.kvh) * G + g_in;
+            b = by_work(a, b);
             qt = (int)gridDim.z - 1 - z;
         }
     }

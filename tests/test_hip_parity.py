@@ -1012,3 +1012,34 @@ def test_attention_module_fp16_pv_prefill_rule():
             outs[tuple(lens), opt] = o
     assert not np.array_equal(outs[(1100, 37), None], outs[(1100, 37), False])       # the long batch took the fp16 form
     assert np.array_equal(outs[(200, 90), None], outs[(200, 90), False])             # the short one did not
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("batch,h,kvh,d", [(8, 2, 1, 64), (24, 6, 2, 64), (64, 2, 1, 128), (72, 1, 1, 64)])
+def test_prefill_sequences_by_work(ops, batch, h, kvh, d, paged):
+    """Sequences are dealt to the XCDs by their work: each of them once, equal ones and ones without rows or without earlier keys among them, with the bits that it has alone."""
+    gen = torch.Generator().manual_seed(batch)
+    new = [(0, 1, 63, 64, 65, 200, 513)[int(i)] for i in torch.randint(7, (batch,), generator=gen)]
+    old = [(0, 0, 70, 300)[int(i)] if paged and n else 0 for i, n in zip(torch.randint(4, (batch,), generator=gen), new)]
+    total, starts = sum(new), [sum(new[:i]) for i in range(batch + 1)]
+    q = torch.randn(total, h, d, generator=gen).bfloat16().cuda()
+    width = 4
+    tables = torch.randperm(batch * width, generator=gen).view(batch, width).int().cuda()
+    if paged:
+        k, v = (torch.randn(batch * width, 256, kvh, d, generator=gen).bfloat16().cuda() for _ in range(2))
+    else:
+        k, v = (torch.randn(total, kvh, d, generator=gen).bfloat16().cuda() for _ in range(2))
+    most = dict(max_seqlen_q=max(new), max_seqlen_k=max(n + o for n, o in zip(new, old)))
+
+    def cu(lengths):
+        return torch.tensor([sum(lengths[:i]) for i in range(len(lengths) + 1)], dtype=torch.int32).cuda()
+
+    def run(rows, one):
+        keys = (k, v) if paged else (k[rows], v[rows])
+        return ops.flash_attn_varlen_func(q[rows], *keys, cu_seqlens_q=cu(new[one]), cu_seqlens_k=cu([n + o for n, o in zip(new[one], old[one])]),
+                                          block_table=tables[one] if paged else None, **most)
+    got = run(slice(None), slice(None))
+    for i in range(batch):
+        if new[i]:
+            rows = slice(starts[i], starts[i + 1])
+            assert torch.equal(got[rows], run(rows, slice(i, i + 1))), (i, new[i], old[i])

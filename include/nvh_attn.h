@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 207          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links */
+#define NVH_VERSION 207          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -214,6 +214,16 @@ int nvh_prefill_varlen_pv16(void* out, const void* q, const void* k, const void*
                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int batch, int max_seqlen_q, int max_seqlen_k, int total_k,
                             int h, int kvh, int hd, int64_t q_row_stride, int64_t k_row_stride, int64_t v_row_stride,
                             float scale, int dtype, int out_dtype, void* scratch, size_t scratch_bytes, void* stream);
+
+/*
+ * nvh_store_kvcache of all total_k rows of k / v (slot_mapping [total_k]), then nvh_prefill_varlen over the packed rows, or nvh_prefill_varlen_pv16 where pv16 != 0 (scratch as
+ * there): same results.  Where that form takes fp16 rows of V, one launch stores the rows and converts V.
+ * Replaces: the pair of calls at nanovllm/layers/attention.py:84-86 and :93-96.
+ */
+int nvh_prefill_step(void* out, const void* q, const void* k, const void* v, void* k_cache, void* v_cache, const int32_t* slot_mapping,
+                     const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int batch, int max_seqlen_q, int max_seqlen_k, int total_k,
+                     int h, int kvh, int hd, int64_t q_row_stride, int64_t k_row_stride, int64_t v_row_stride,
+                     float scale, int dtype, int out_dtype, int pv16, void* scratch, size_t scratch_bytes, void* stream);
 
 /*
  * "Next" row: the step immediately before attention, fused into one launch.

@@ -196,13 +196,19 @@ int nvh_decode_step(void* out, const void* q, const void* k_new, const void* v_n
                             workspace, workspace_bytes, stream);
 }
 
+// rows of K and V that go to the cache in front of the attention launch
+struct StoreRows {
+    void *k_cache, *v_cache;
+    const int32_t* slots;
+    int rows;
+};
 static int prefill_varlen_impl(int kernel, int short_waves, void* out, const void* q, const void* k, const void* v,
                        const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                        const int32_t* block_tables, int batch, int max_seqlen_q, int max_seqlen_k,
                        int h, int kvh, int hd, int block_size, int max_blocks,
                        int64_t q_row_stride, int64_t k_row_stride, int64_t v_row_stride,
                        int64_t bt_row_stride, float scale, int dtype, int out_dtype, void* stream,
-                       bool pv16 = false, int total_k = 0, void* pv16_scratch = nullptr, size_t pv16_scratch_bytes = 0) {
+                       bool pv16 = false, int total_k = 0, void* pv16_scratch = nullptr, size_t pv16_scratch_bytes = 0, const StoreRows* store = nullptr) {
     if (batch == 0 || max_seqlen_q == 0) return 0;
     if (kernel < 0 || kernel > 3 || (kernel == 3 && block_tables) || (short_waves != 0 && short_waves != 8 && short_waves != 16)) {
         set_error("prefill_varlen: kernel %d / short_waves %d not supported", kernel, short_waves);
@@ -262,11 +268,17 @@ static int prefill_varlen_impl(int kernel, int short_waves, void* out, const voi
             }
             int32_t* flags = (int32_t*)pv16_scratch;
             uint16_t* v16 = (uint16_t*)((char*)pv16_scratch + pv16_header_bytes(total_k));
-            rc = launch_bf16_rows_to_f16(v16, v, total_k, kvh * hd, v_row_stride, (int64_t)kvh * hd, flags, (hipStream_t)stream);
+            rc = store ? launch_store_rows_f16(k, v, store->k_cache, store->v_cache, store->slots, v16, flags, total_k, kvh * hd, k_row_stride, v_row_stride, (hipStream_t)stream)
+                       : launch_bf16_rows_to_f16(v16, v, total_k, kvh * hd, v_row_stride, (int64_t)kvh * hd, flags, (hipStream_t)stream);
             if (rc) return rc;
+            store = nullptr;
             a.v16 = v16; a.v16_row_stride = (int64_t)kvh * hd; a.pv16_flags = flags; a.pv16_rows = total_k;
             a.kernel = 1;                                        // the tiled kernel
         }
+    }
+    if (store) {
+        rc = launch_store_kvcache(k, v, store->k_cache, store->v_cache, store->slots, store->rows, kvh, hd, k_row_stride, v_row_stride, (hipStream_t)stream);
+        if (rc) return rc;
     }
     return launch_prefill_varlen(a, (hipStream_t)stream);
 }
@@ -289,6 +301,20 @@ int nvh_prefill_varlen_pv16(void* out, const void* q, const void* k, const void*
     if (batch == 0 || max_seqlen_q == 0) return 0;
     return prefill_varlen_impl(0, 0, out, q, k, v, cu_seqlens_q, cu_seqlens_k, nullptr, batch, max_seqlen_q, max_seqlen_k, h, kvh, hd,
                                0, 0, q_row_stride, k_row_stride, v_row_stride, 0, scale, dtype, out_dtype, stream, true, total_k, scratch, scratch_bytes);
+}
+
+int nvh_prefill_step(void* out, const void* q, const void* k, const void* v, void* k_cache, void* v_cache, const int32_t* slot_mapping,
+                     const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int batch, int max_seqlen_q, int max_seqlen_k, int total_k,
+                     int h, int kvh, int hd, int64_t q_row_stride, int64_t k_row_stride, int64_t v_row_stride,
+                     float scale, int dtype, int out_dtype, int pv16, void* scratch, size_t scratch_bytes, void* stream) {
+    if (batch == 0 || max_seqlen_q == 0)                                 // no attention: the rows are stored all the same
+        return nvh_store_kvcache(k, v, k_cache, v_cache, slot_mapping, total_k, kvh, hd, k_row_stride, v_row_stride, dtype, stream);
+    if (!k_cache || !v_cache || !slot_mapping) { set_error("prefill_step: null pointer"); return NVH_E_NULL; }
+    if (total_k < 0) { set_error("prefill_step: negative size"); return NVH_E_SHAPE; }
+    if (!aligned16(k_cache) || !aligned16(v_cache)) { set_error("prefill_step: pointers must be 16-byte aligned"); return NVH_E_ALIGN; }
+    const StoreRows store{k_cache, v_cache, slot_mapping, total_k};
+    return prefill_varlen_impl(0, 0, out, q, k, v, cu_seqlens_q, cu_seqlens_k, nullptr, batch, max_seqlen_q, max_seqlen_k, h, kvh, hd,
+                               0, 0, q_row_stride, k_row_stride, v_row_stride, 0, scale, dtype, out_dtype, stream, pv16 != 0, total_k, scratch, scratch_bytes, &store);
 }
 
 int nvh_prefill_varlen(void* out, const void* q, const void* k, const void* v,

@@ -11,6 +11,8 @@ int launch_store_kvcache(const void* k, const void* v, void* k_cache, void* v_ca
                          int64_t k_row_stride, int64_t v_row_stride, hipStream_t stream);
 
 constexpr int kPv16GroupRows = 64;   // rows per range flag of the bf16 -> fp16 conversion (one conversion workgroup per group)
+int launch_store_rows_f16(const void* k, const void* v, void* k_cache, void* v_cache, const int32_t* slot_mapping, void* v16, int32_t* group_flags, int n_rows, int row_elems,
+                          int64_t k_row_stride, int64_t v_row_stride, hipStream_t stream);
 int launch_bf16_rows_to_f16(void* out, const void* in, int n_rows, int row_elems, int64_t in_row_stride, int64_t out_row_stride, int32_t* group_flags, hipStream_t stream);
 
 struct DecodeArgs {

@@ -76,7 +76,10 @@ class Attention(nn.Module):
         have_cache = k_cache.numel() > 0 and v_cache.numel() > 0       # warmup prefill runs before allocation
         store = store and have_cache and context.slot_mapping is not None   # attention.py:84, attention_sdpa.py:242
 
-        if context.is_prefill:
+        if context.is_prefill and store and context.block_tables is None:
+            o = ops.prefill_step(q, k, v, k_cache, v_cache, context.slot_mapping, context.max_seqlen_q, context.cu_seqlens_q, context.max_seqlen_k,
+                                 context.cu_seqlens_k, self.scale, pv_fp16=self.prefill_pv_fp16)
+        elif context.is_prefill:
             if store:
                 ops.store_kvcache(k, v, k_cache, v_cache, context.slot_mapping)
             if context.block_tables is not None:                        # prefix-cache hit: read K/V from the cache

@@ -184,6 +184,40 @@ def decode_step(q, k_new, v_new, k_cache, v_cache, slot_mapping, cache_seqlens, 
 PV16_MIN_KEYS = 512       # fp16 P V (nvh_prefill_varlen_pv16) by default from this many keys per sequence on (40.5 vs 42.0 us at 32 x 512; below, the conversion launch costs what it saves)
 
 
+def _pv16_pays(head_dim, kv_heads, batch, max_seqlen_q, max_seqlen_k):
+    # from PV16_MIN_KEYS on, or on the short-sequence kernel's shapes (it converts its resident V images itself: no extra launch; the library's rule, prefill_mfma.hip launch_short)
+    return max_seqlen_k >= PV16_MIN_KEYS or (head_dim == 64 and 64 < max_seqlen_k <= 128 and max_seqlen_q <= max_seqlen_k and batch * kv_heads >= 128)
+
+
+def _pv16_scratch(lib, batch, max_seqlen_q, max_seqlen_k, rows, kvh, hd, device):
+    """(pointer, bytes, the tensor that owns them): none where the short-sequence kernel converts V in LDS."""
+    if max_seqlen_k <= 128 and not lib.nvh_prefill_pv16_uses_scratch(batch, max_seqlen_q, max_seqlen_k, kvh, hd):
+        return None, 0, None
+    scratch = torch.empty(lib.nvh_prefill_pv16_scratch_bytes(rows, kvh, hd), dtype=torch.uint8, device=device)
+    return scratch.data_ptr(), scratch.numel(), scratch
+
+
+def prefill_step(q, k, v, k_cache, v_cache, slot_mapping, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k, softmax_scale, pv_fp16=None):
+    """store_kvcache(k, v, ...) followed by flash_attn_varlen_func(q, k, v, ...) over the packed rows as one C-ABI call (the two calls at attention.py:84-86 and :93-96)."""
+    (tq, h, hd), (n, kvh, _) = q.shape, k.shape
+    batch, max_q, max_k, d = cu_seqlens_q.numel() - 1, int(max_seqlen_q), int(max_seqlen_k), kvh * hd
+    _require_gpu_bf16(q=q, k=k, v=v, k_cache=k_cache, v_cache=v_cache)
+    _require_i32(slot_mapping=slot_mapping, cu_seqlens_q=cu_seqlens_q, cu_seqlens_k=cu_seqlens_k)
+    (q0, q1, q2), (k0, k1, k2), (v0, v1, v2) = q.stride(), k.stride(), v.stride()
+    assert k.shape[2] == hd and v.shape == k.shape and q2 == k2 == v2 == 1 and q1 == k1 == v1 == hd
+    assert k_cache.stride(1) == d and v_cache.stride(1) == d and k_cache.is_contiguous() and v_cache.is_contiguous()
+    assert slot_mapping.numel() == n and slot_mapping.is_contiguous() and cu_seqlens_k.numel() == batch + 1
+    if pv_fp16 is None:
+        pv_fp16 = _pv16_pays(hd, kvh, batch, max_q, max_k)
+    lib, out = _lib.load(), torch.empty((tq, h, hd), dtype=torch.bfloat16, device=q.device)
+    sc_ptr, sc_bytes, _scratch = _pv16_scratch(lib, batch, max_q, max_k, n, kvh, hd, q.device) if pv_fp16 else (None, 0, None)
+    rc = lib.nvh_prefill_step(out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), slot_mapping.data_ptr(),
+                              cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), batch, max_q, max_k, n, h, kvh, hd, q0, k0, v0, float(softmax_scale),
+                              NVH_BF16, NVH_BF16, int(pv_fp16), sc_ptr, sc_bytes, _stream())
+    _lib.check(rc, "nvh_prefill_step")
+    return out
+
+
 def flash_attn_varlen_func(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k, softmax_scale=None,
                            causal=True, block_table=None, out_dtype=None, kernel=None, short_waves=0, pv_fp16=None):
     """Packed varlen causal attention, drop-in for the call at attention.py:93-96.
@@ -201,10 +235,7 @@ def flash_attn_varlen_func(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu
         assert not pv_fp16 or kernel == "tiled_f16v", "pv_fp16 goes with the default kernel choice and packed k / v rows"
         pv_fp16 = False
     elif pv_fp16 is None:
-        # ... or on the short-sequence kernel's shapes (it converts its resident V images itself: no extra launch; the library's rule, prefill_mfma.hip launch_short)
-        short = (q.shape[2] == 64 and 64 < int(max_seqlen_k) <= 128 and int(max_seqlen_q) <= int(max_seqlen_k)
-                 and (cu_seqlens_q.numel() - 1) * k.shape[1] >= 128)
-        pv_fp16 = (out_dtype in (None, torch.bfloat16)) and (int(max_seqlen_k) >= PV16_MIN_KEYS or short)
+        pv_fp16 = out_dtype in (None, torch.bfloat16) and _pv16_pays(q.shape[2], k.shape[1], cu_seqlens_q.numel() - 1, int(max_seqlen_q), int(max_seqlen_k))
     if not causal:
         raise NotImplementedError("the reference only ever calls this with causal=True (attention.py:96)")
     tq, h, hd = q.shape
@@ -238,11 +269,7 @@ def flash_attn_varlen_func(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu
             float(softmax_scale), NVH_BF16, _out_code(out.dtype), _stream())
     if pv_fp16:
         lib = _lib.load()
-        if int(max_seqlen_k) <= 128 and not lib.nvh_prefill_pv16_uses_scratch(batch, int(max_seqlen_q), int(max_seqlen_k), kvh, hd):
-            sc_ptr, sc_bytes = None, 0                           # the short-sequence kernel converts V in LDS: one launch, no scratch
-        else:
-            scratch = torch.empty(lib.nvh_prefill_pv16_scratch_bytes(tk, kvh, hd), dtype=torch.uint8, device=q.device)
-            sc_ptr, sc_bytes = scratch.data_ptr(), scratch.numel()
+        sc_ptr, sc_bytes, _scratch = _pv16_scratch(lib, batch, int(max_seqlen_q), int(max_seqlen_k), tk, kvh, hd, q.device)
         rc = lib.nvh_prefill_varlen_pv16(out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), batch,
                                          int(max_seqlen_q), int(max_seqlen_k), tk, h, kvh, hd, q.stride(0), k_stride, v_stride, float(softmax_scale),
                                          NVH_BF16, _out_code(out.dtype), sc_ptr, sc_bytes, _stream())

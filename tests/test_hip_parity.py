@@ -1043,3 +1043,24 @@ def test_prefill_sequences_by_work(ops, batch, h, kvh, d, paged):
         if new[i]:
             rows = slice(starts[i], starts[i + 1])
             assert torch.equal(got[rows], run(rows, slice(i, i + 1))), (i, new[i], old[i])
+
+
+@pytest.mark.parametrize("h,kvh,d,lens,pv", [(4, 2, 64, (513, 1, 64), None), (2, 2, 128, (700, 65), None), (14, 2, 64, (300, 40), None), (2, 1, 64, (130, 3), True), (2, 2, 64, (100,) * 64, None)])
+def test_prefill_step_is_store_then_attend(ops, h, kvh, d, lens, pv):
+    """Output and cache bit for bit those of the two calls: rows of whole and ragged groups, skipped slots, views of a fused projection, V that does not fit fp16."""
+    gen, n = torch.Generator().manual_seed(sum(lens)), sum(lens)
+    qkv = torch.randn(n, (h + 2 * kvh) * d, generator=gen).bfloat16()
+    qkv[n // 2, -3] = 1e5
+    q, k, v = (t.view(n, -1, d) for t in qkv.cuda().split([h * d, kvh * d, kvh * d], dim=-1))
+    blocks = -(-n // 256) + 1
+    slots = torch.randperm(blocks * 256, generator=gen)[:n].int()
+    slots[::7] = -1
+    slots = slots.cuda()
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32).cuda()
+    start = torch.randn(2, blocks, 256, kvh, d, generator=gen).bfloat16().cuda()
+    want_kv, got_kv = start.clone(), start.clone()
+    how = dict(max_seqlen_q=max(lens), cu_seqlens_q=cu, max_seqlen_k=max(lens), cu_seqlens_k=cu, softmax_scale=d ** -0.5, pv_fp16=pv)
+    ops.store_kvcache(k, v, *want_kv, slots)
+    want = ops.flash_attn_varlen_func(q, k, v, **how)
+    got = ops.prefill_step(q, k, v, *got_kv, slots, **how)
+    assert torch.equal(got, want) and torch.equal(got_kv, want_kv) and not torch.equal(got_kv, start)

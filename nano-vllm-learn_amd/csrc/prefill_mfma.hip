@@ -149,8 +149,11 @@ __device__ __forceinline__ void prefill_tile_of_block(const PrefillArgs& a, int&
         // XCD works through as much as any other, and the same mix of heavy and light tiles.  (In the order of the batch an XCD's six of 48 pairs are more or less work by
         // chance: 24 uneven prompts of 16384 tokens, 14 / 2 heads of 64, 73.6 -> 67.0 us; 16 of 12000, 7 / 1 heads of 128, 63.2 -> 54.8; 8 of 8192 behind cached keys, 28 / 4
         // heads of 128, 325 -> 309.)
+        // One pair an XCD (8 pairs) is no balance at all where sequences differ, and so few keys that each L2 may well read them for itself: plain order.  4 prompts of 12000 tokens,
+        // 14 / 2 heads, 142 -> 110 us, behind cached keys 259 -> 190; 2 of 5000, 28 / 4 heads, 190 -> 142 (of 8000, as long as each other: 268 -> 270 to 285).  From 16 pairs on the
+        // plain order is slower: up to 5 % without, 5 to 20 % with cached keys.
         const int G = a.h / a.kvh, units = (int)gridDim.y * a.kvh, total = (int)(gridDim.x * gridDim.y * gridDim.z);
-        if ((units & 7) == 0 && (total & 7) == 0) {
+        if ((units & 7) == 0 && (total & 7) == 0 && units >= 16) {
             const int lin = (int)blockIdx.x + (int)gridDim.x * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
             const int xcd = lin & 7, idx = lin >> 3, per = units >> 3;
 #ifdef NVH_PREFILL_PAIR_MAJOR                 // A/B builds: one pair after the other on an XCD (its K/V alone in the L2) instead of all of the XCD's pairs per q-tile rank
@@ -171,8 +174,9 @@ __device__ __forceinline__ void prefill_tile_of_block(const PrefillArgs& a, int&
 // GUARD (nvh_prefill_varlen_pv16): `a.v` is the fp16 copy of V; the range flags of this sequence's rows are fetched FIRST, the first K image's DMA is
 // issued behind them, and only then are they looked at — so the check costs no memory latency of its own.  Returns false (nothing but that K image
 // touched) when a flag is set: the caller runs the exact body instead.
-template <int D, bool PAGED, int QT, bool F16V, bool GUARD = false>
-__device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsigned char* const lds, const int qt, const int head, const int b) {
+// KS groups of four waves work on the same rows, each on every KS-th tile of keys with images of its own; the first adds up their sums at the end.
+template <int D, bool PAGED, int QT, bool F16V, bool GUARD, int KS>
+__device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsigned char* const lds_all, const int qt, const int head, const int b) {
     constexpr int BM = 64 * QT;                      // query rows per workgroup (4 waves x QT x 16)
     constexpr int ROWB = D * 2;                      // LDS row, bytes
     constexpr int LPT = D / 8;                       // 16-byte chunks per row
@@ -194,7 +198,9 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;              // ... of its group
+    const int grp = KS > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
+    unsigned char* const lds = lds_all + grp * 4 * IMG;
     const int lq = lane & 15;                        // query column of this lane
     const int lg = lane >> 4;                        // lane group: k-block of the operands / key rows of C
 
@@ -263,6 +269,7 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         }
     };
 
+    const int first = grp < n_tiles ? grp : n_tiles - 1;         // (a group without a tile stages one all the same: the waits count on it)
     if constexpr (GUARD) {
         // one flag per kPv16GroupRows rows of V; lane l looks at groups g0 + l, + 64, + 128, + 192 (16384 rows: the largest prefill batch), a plain loop
         // takes longer sequences.  The loads are inline asm so that no compiler-placed wait sits between them and the K image's DMA.
@@ -276,7 +283,7 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
             const int32_t* p = a.pv16_flags + (g < last ? g : last);
             asm volatile("global_load_dword %0, %1, off" : "=v"(fl[i]) : "v"(p) : "memory");
         }
-        stage(0, 0, true, false);
+        stage(first, 0, true, false);
         asm volatile("s_waitcnt vmcnt(%4)" : "+v"(fl[0]), "+v"(fl[1]), "+v"(fl[2]), "+v"(fl[3]) : "n"(NIW) : "memory");
         bool bad = k_end > a.pv16_rows;              // (a caller whose total_k was short of cu_seqlens_k[batch]: no fp16 copy of those rows)
 #pragma unroll
@@ -284,9 +291,9 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         for (int g = g0 + 256 + lane; __builtin_amdgcn_ballot_w64(g < g1) != 0; g += 64)
             bad |= __builtin_amdgcn_ballot_w64(g < g1 && a.pv16_flags[g < g1 ? g : last] != 0) != 0;
         if (bad) return false;
-        stage(0, 0, false, true);
+        stage(first, 0, false, true);
     } else {
-        stage(0, 0);
+        stage(first, 0);
     }
     // ---- Q fragments (B operand of S^T): Q[row][32*step + 8*lg .. +8]; plain loads issued BEHIND the first tile's DMA, so that a workgroup
     // pays one memory latency at its start, not two in a row (the counted wait of the first tile body leaves only tile 1's DMA in flight:
@@ -324,9 +331,9 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
     }
     auto tile_body = [&](auto bufc, const int it) {
         constexpr int buf = decltype(bufc)::value;
-        if (it + 1 < n_tiles) {
-            stage(it + 1, buf ^ 1);
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NIW) : "memory");       // tile `it` landed, tile it+1 in flight
+        if (it + KS < n_tiles) {
+            stage(it + KS, buf ^ 1);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NIW) : "memory");       // tile `it` landed, the group's next in flight
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
@@ -336,7 +343,7 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         PF_STAMP(3 + 3 * it);
         const unsigned char* kimg = lds + buf * 2 * IMG;
         const int kv0 = it * BN;
-        if (kv0 <= wave_last_key) {                                              // wave-uniform: tile not entirely above the diagonal
+        if (kv0 <= wave_last_key && (KS == 1 || it < n_tiles)) {                 // wave-uniform: tile not entirely above the diagonal
             // ---- S^T for the four 16-key tiles of both query sub-tiles: each K fragment is read once, used QT times
             // (skipping the 16-key groups above the wave's diagonal, as the short-sequence kernel below does, measured 2-5 % SLOWER
             // here at every S >= 256, same-box A/B: the interior tiles pay for the extra branches and live ranges)
@@ -495,12 +502,45 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         __builtin_amdgcn_s_barrier();                                            // ... and everyone's: tile it+2 may overwrite it
         asm volatile("" ::: "memory");
     };
-    for (int it = 0; it < n_tiles; it += 2) {
-        tile_body(std::integral_constant<int, 0>{}, it);
-        if (it + 1 < n_tiles) tile_body(std::integral_constant<int, 1>{}, it + 1);
+    for (int it = 0; it < n_tiles; it += 2 * KS) {                               // (the groups share the barriers: as many rounds for each)
+        tile_body(std::integral_constant<int, 0>{}, it + grp);
+        if (it + KS < n_tiles) tile_body(std::integral_constant<int, 1>{}, it + KS + grp);
     }
 
     PF_STAMP(31);
+    if constexpr (KS == 2) {                                                     // sums of the second group to the first, through the images' memory
+        float* at = reinterpret_cast<float*>(lds_all) + 64 * wave + lane;
+        constexpr int STEP = 256;
+        static_assert((QT * (4 * DT + 2)) * STEP * 4 <= KS * 4 * IMG);
+        if (grp == 1) {
+#pragma unroll
+            for (int qs = 0; qs < QT; ++qs) {
+                float* p = at + qs * (4 * DT + 2) * STEP;
+                p[0] = m_run[qs];
+                p[STEP] = l_run[qs];
+#pragma unroll
+                for (int t = 0; t < DT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) p[(2 + 4 * t + r) * STEP] = o[qs][t][r];
+            }
+        }
+        __syncthreads();
+        if (grp == 0) {
+#pragma unroll
+            for (int qs = 0; qs < QT; ++qs) {
+                const float* p = at + qs * (4 * DT + 2) * STEP;
+                const float m1 = p[0], m = max2(m_run[qs], m1), m_use = m == -INFINITY ? 0.f : m;
+                const float w0 = fast_exp2(m_run[qs] - m_use), w1 = fast_exp2(m1 - m_use);
+                l_run[qs] = l_run[qs] * w0 + p[STEP] * w1;
+#pragma unroll
+                for (int t = 0; t < DT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[qs][t][r] = o[qs][t][r] * w0 + p[(2 + 4 * t + r) * STEP] * w1;
+            }
+        }
+        __syncthreads();
+        if (grp == 1) return true;
+    }
     // ---- finalise: total row sum over the 4 lane groups, normalise, store 4 contiguous dims per tile
 #pragma unroll
     for (int qs = 0; qs < QT; ++qs) {
@@ -529,11 +569,11 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
 // conversion launch ahead of this one flagged a 64-row group of THIS sequence's V rows (a finite |v| > 65504 does not fit fp16): then the hi + lo form
 // on the caller's own rows.  Every conversion workgroup writes its group's flag unconditionally (nothing to clear); a wave ORs the flags that cover its
 // sequence behind the first K image's DMA (GUARD above); both bodies are instantiations of the same code.
-template <int D, bool PAGED, int QT, int PV = 0>
-__global__ __launch_bounds__(256)
+template <int D, bool PAGED, int QT, int PV, int KS>
+__global__ __launch_bounds__(256 * KS)
 __attribute__((amdgpu_waves_per_eu(PV == 2 && D == 64 && QT == 2 ? 4 : 1)))         // (the guarded kernel at the fp16 body's 128 registers: hipcc gives it 134 otherwise)
 void prefill_varlen_kernel(const PrefillArgs a) {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * 2 * BN * D * 2];     // [buffer][K | V]
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];          // [group][buffer][K | V]
     int qt, head, b;
     prefill_tile_of_block(a, qt, head, b);
     if constexpr (PV == 2) {
@@ -541,7 +581,7 @@ void prefill_varlen_kernel(const PrefillArgs a) {
         PrefillArgs f = a;
         f.v = a.v16;
         f.v_row_stride = a.v16_row_stride;
-        if (!prefill_varlen_body<D, false, QT, true, true>(f, lds, qt, head, b)) {
+        if (!prefill_varlen_body<D, false, QT, true, true, KS>(f, lds, qt, head, b)) {
             // the fall-back runs the one-sub-tile-per-wave body QT times over the workgroup's rows: its registers stay below the fp16 body's, so the
             // guard costs the fast path no occupancy (D = 64, QT = 2: 128 registers = 4 waves per SIMD; the QT = 2 hi + lo body needs 136).  The
             // abandoned K image's DMA is drained first (the exact body stages it again).
@@ -549,10 +589,10 @@ void prefill_varlen_kernel(const PrefillArgs a) {
             __builtin_amdgcn_s_barrier();
             int qt2 = qt, head2 = head, b2 = b;      // (laundered: the exact body shares no value with the abandoned one, so the fast path's registers
             asm volatile("" : "+s"(qt2), "+s"(head2), "+s"(b2));     //  are not held across the branch for its sake)
-            for (int sub = 0; sub < QT; ++sub) prefill_varlen_body<D, false, 1, false>(a, lds, qt2 * QT + sub, head2, b2);
+            for (int sub = 0; sub < QT; ++sub) prefill_varlen_body<D, false, 1, false, false, KS>(a, lds, qt2 * QT + sub, head2, b2);
         }
     } else {
-        prefill_varlen_body<D, PAGED, QT, PV == 1>(a, lds, qt, head, b);
+        prefill_varlen_body<D, PAGED, QT, PV == 1, false, KS>(a, lds, qt, head, b);
     }
 }
 
@@ -865,20 +905,28 @@ void prefill_short_kernel(const PrefillArgs a) {
     SK_STAMP(15);
 }
 
-template <int D, int QT>
+template <int D, bool PAGED, int QT, int PV, int KS>
+int launch_one(const PrefillArgs& a, hipStream_t stream, const char* what) {
+    constexpr int lds = KS * 2 * 2 * BN * D * 2;
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_varlen_kernel<D, PAGED, QT, PV, KS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    const dim3 grid(a.h, a.batch, (a.max_seqlen_q + 64 * QT - 1) / (64 * QT));
+    prefill_varlen_kernel<D, PAGED, QT, PV, KS><<<grid, 256 * KS, lds, stream>>>(a);
+    return check_launch(what);
+}
+
+// QT sub-tiles of 16 rows a wave, KS groups of four waves
+template <int D, int QT, int KS>
 int launch_q(const PrefillArgs& a, hipStream_t stream) {
-    dim3 grid(a.h, a.batch, (a.max_seqlen_q + 64 * QT - 1) / (64 * QT));
-    if (a.kernel == 3) {                                         // NVH_PREFILL_TILED_F16V: v holds fp16 rows (measurement variant; never paged)
-        hipLaunchKernelGGL((prefill_varlen_kernel<D, false, QT, 1>), grid, dim3(256), 0, stream, a);
-        return check_launch("prefill_varlen_f16v");
-    }
-    if (a.v16) {                                                 // nvh_prefill_varlen_pv16: fp16 P V unless the conversion raised the guard
-        hipLaunchKernelGGL((prefill_varlen_kernel<D, false, QT, 2>), grid, dim3(256), 0, stream, a);
-        return check_launch("prefill_varlen_pv16");
-    }
-    if (a.block_tables) hipLaunchKernelGGL((prefill_varlen_kernel<D, true, QT>), grid, dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL((prefill_varlen_kernel<D, false, QT>), grid, dim3(256), 0, stream, a);
-    return check_launch("prefill_varlen");
+    if (a.kernel == 3) return launch_one<D, false, QT, 1, 1>(a, stream, "prefill_varlen_f16v");      // NVH_PREFILL_TILED_F16V: v holds fp16 rows (measurement variant; never paged)
+    // nvh_prefill_varlen_pv16: fp16 P V unless the conversion raised the guard
+    if (a.v16) return launch_one<D, false, QT, 2, KS>(a, stream, "prefill_varlen_pv16");
+    if (a.block_tables) return launch_one<D, true, QT, 0, KS>(a, stream, "prefill_varlen");
+    return launch_one<D, false, QT, 0, KS>(a, stream, "prefill_varlen");
+}
+
+// How full a launch of 64-row workgroups leaves the 256 CUs: the tiles of keys that a CU gets over those of the longest walk
+double prefill_fill(const PrefillArgs& a, double rows) {
+    return a.max_seqlen_k > 0 ? a.h * rows / (64.0 * 256.0) * (1.0 - 0.5 * a.max_seqlen_q / a.max_seqlen_k) : 0.0;
 }
 
 // a.kernel (nvh_prefill_varlen_variant): 1 = never, 2 = whenever the shape allows (tests), 0 = when it also fills the chip
@@ -923,7 +971,16 @@ int launch_d(const PrefillArgs& a, hipStream_t stream) {
                                              // S = 512 42.5 -> 40.5 us, S = 1024 62.8 -> 58.8, S = 1536 77.8 -> 74.0; profiles/r03_prefill_qt2_pv16_ab.txt)
 #endif
     const bool two = D == 128 ? a.max_seqlen_q > 128 : a.max_seqlen_q >= (a.v16 ? NVH_PREFILL_QT2_FROM_PV16 : NVH_PREFILL_QT2_FROM);
-    return two ? launch_q<D, 2>(a, stream) : launch_q<D, 1>(a, stream);
+    // A launch that leaves CUs idle takes as long as its longest walk over the keys: half the rows a workgroup, and where even those are few two groups of waves that
+    // share the walk (each tile costs more with them, and a start that nothing hides: 1024 keys at least).  us with 128 rows / 64 rows / two groups, by fill:
+    // 14 / 2 heads of 64: 0.9 43 / 31 / 26.5, 1.3 61 / 47 / 38.5, 1.5 36 / 30 / 38, 2.6 77 / 65 / 70, 3.4 90 / 98 / 101; heads of 128: 7 / 1 0.4 57 / 43 / 34, 0.85 103 / 79 / 61,
+    // 1.1 46 / 35 / 38, 1.7 101 / 82 / 106; 16 / 8 1.0 64 / 53 / 49, 1.9 82 / 91 / 116; 28 / 4 1.7 33 / 30 / 40, 2.5 42 / 45 / 62.
+    // The rows are known where V was copied; otherwise uneven sequences are taken to have half of the longest on average (for the two groups always: which of them adds what
+    // shows in the last bits, and a sequence whose V does not fit fp16 keeps those of the exact form).
+    const double all = (double)a.max_seqlen_q * a.batch, guess = 0.5 * (all + a.max_seqlen_q);
+    if (two && prefill_fill(a, a.v16 && a.pv16_rows < all ? a.pv16_rows : guess) >= (D == 64 ? 3.0 : 1.8)) return launch_q<D, 2, 1>(a, stream);
+    if (a.max_seqlen_k >= 1024 && prefill_fill(a, guess) < (D == 64 ? 1.3 : 1.0)) return launch_q<D, 1, 2>(a, stream);
+    return launch_q<D, 1, 1>(a, stream);
 }
 
 }  // namespace

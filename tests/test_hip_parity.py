@@ -1045,6 +1045,38 @@ def test_prefill_sequences_by_work(ops, batch, h, kvh, d, paged):
             assert torch.equal(got[rows], run(rows, slice(i, i + 1))), (i, new[i], old[i])
 
 
+@pytest.mark.parametrize("h,kvh,d,new,old,paged,large", [
+    (2, 1, 64, (1024,), (0,), False, False), (2, 2, 128, (1025, 1, 63), (0, 0, 0), False, False), (3, 1, 64, (1100, 65, 0, 130), (0, 0, 0, 0), False, True),
+    (2, 1, 128, (1031, 70), (0, 0), False, True), (2, 1, 128, (65, 1), (1215, 0), True, False), (2, 2, 64, (129, 64, 1), (900, 960, 1023), True, False)])
+def test_prefill_two_groups_share_the_keys(ops, h, kvh, d, new, old, paged, large):
+    """Few rows and long walks: two groups of waves take every other tile of keys; odd and even numbers of tiles, one tile, rows behind cached keys, V that does not fit fp16.
+    Against 64 bits: P and V are rounded to 11 bits (each to half of 2^-10 of itself, so the weighted mean of |v| bounds the error), the output to 8."""
+    gen, total = torch.Generator().manual_seed(sum(new)), sum(new)
+    q = torch.randn(total, h, d, generator=gen).bfloat16().cuda()
+    n_keys = [n + o if n else 0 for n, o in zip(new, old)]
+    assert max(n_keys) >= 1024
+    tables = torch.randperm(len(new) * 6, generator=gen).view(len(new), 6).int().cuda()
+    k, v = (torch.randn(*((len(new) * 6, 256) if paged else (total,)), kvh, d, generator=gen).bfloat16().cuda() for _ in range(2))
+    if large:
+        v[total // 2, 0, 3] = 1e5
+
+    def cu(lengths):
+        return torch.tensor([sum(lengths[:i]) for i in range(len(lengths) + 1)], dtype=torch.int32).cuda()
+    got = ops.flash_attn_varlen_func(q, k, v, max_seqlen_q=max(new), cu_seqlens_q=cu(new), max_seqlen_k=max(n_keys), cu_seqlens_k=cu(n_keys), softmax_scale=d ** -0.5,
+                                     block_table=tables if paged else None, pv_fp16=None if paged else True)
+    at = 0
+    for i, (n, m) in enumerate(zip(new, n_keys)):
+        if not n:
+            continue
+        ks, vs = ((t[tables[i].long()].flatten(0, 1)[:m] if paged else t[at:at + n]).double() for t in (k, v))
+        seen = torch.arange(m, device="cuda")[None] <= torch.arange(n, device="cuda")[:, None] + (m - n)
+        for j in range(h):
+            p = (q[at:at + n, j].double() @ ks[:, j * kvh // h].T * d ** -0.5).masked_fill(~seen, float("-inf")).softmax(dim=-1)
+            want, spread = p @ vs[:, j * kvh // h], p @ vs[:, j * kvh // h].abs()
+            assert ((got[at:at + n, j].double() - want).abs() <= want.abs() * 2 ** -8 + spread * 2 ** -10 + 1e-5).all(), (i, j)
+        at += n
+
+
 @pytest.mark.parametrize("h,kvh,d,lens,pv", [(4, 2, 64, (513, 1, 64), None), (2, 2, 128, (700, 65), None), (14, 2, 64, (300, 40), None), (2, 1, 64, (130, 3), True), (2, 2, 64, (100,) * 64, None)])
 def test_prefill_step_is_store_then_attend(ops, h, kvh, d, lens, pv):
     """Output and cache bit for bit those of the two calls: rows of whole and ragged groups, skipped slots, views of a fused projection, V that does not fit fp16."""

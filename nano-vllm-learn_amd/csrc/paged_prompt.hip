@@ -109,7 +109,10 @@ int launch_dims(const PagedAttendArgs& a, hipStream_t stream) {
         // 191, one of 2000 62 against 72; of 192 / 64: 166 and 62 against 171 and 70; but of 128 / 64 (three waves on a SIMD either way) 145 against 125,
         // and of 192 / 128 and wider, where one sub-tile does not fit 128 registers, 236 against 213.
         constexpr bool eight = DK + 2 * DV >= 320 && DK + DV <= 256;
-        if (a.max_q > 256) return launch_one<DK, DV, eight ? 1 : 2, eight ? 8 : 4>(a, stream);
+        // Up to 2.2 workgroups of 64 rows a CU, those: a launch that leaves CUs idle takes as long as its longest walk over the keys.  8 heads of 128 / 128, us with 128 and with
+        // 64 rows: one prompt of 2414 tokens 72 and 59, 12 later portions of 3013 with a window 41 and 34, 5 of 3648 with chunks 36 and 29; 16 heads, 4 of 2183 33 and 27; but
+        // 2 later portions of 2415 (2.4 a CU, walks of equal length) 92 and 106, 2 of 4140 103 and 116.
+        if (a.max_q > 256 && (int64_t)a.rows * a.heads > 36044) return launch_one<DK, DV, eight ? 1 : 2, eight ? 8 : 4>(a, stream);
     }
     return launch_one<DK, DV, 1, 4>(a, stream);
 }

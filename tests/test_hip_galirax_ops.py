@@ -115,6 +115,28 @@ def test_prompt(heads, kvh, dim, vdim, window, keep):
             at += r
 
 
+@pytest.mark.parametrize("window,keep,chunk", [(0, 0, 0), (70, 0, 0), (200, 66, 0), (0, 0, 100)])
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (64, 128), (128, 64), (128, 128), (192, 64), (192, 128), (256, 64), (256, 128)])
+def test_prompt_of_many_rows(dim, vdim, window, keep, chunk):
+    """As many rows and heads as fill the GPU with 128 rows a workgroup: the bits of each sequence alone (64 rows a workgroup), and those near the reference."""
+    from nanovllm_hip import ops
+    heads, kvh, portions = 48, 2, [(300, 300), (3, 400), (130, 190), (327, 600)]
+    pg = Pages([k for _, k in portions], kvh, dim, vdim, BF16, seed=3)
+    q, sink = randn(sum(r for r, _ in portions), heads, dim, seed=8), None if chunk else randn(heads, seed=6, dtype=F32).cuda()
+    cu = lambda lengths: torch.tensor([0] + list(lengths)).cumsum(0).int().cuda()
+
+    def run(rows, some):
+        return pg.unpad(ops.paged_attend_prompt(pg.pad_q(q[rows]), pg.cache(), pg.tables[some].contiguous().cuda(), cu(r for r, _ in portions[some]), cu(k for _, k in portions[some]), 327,
+                                                heads, kvh, pg.dk, pg.dv, 0.2, window, keep, sink, chunk=chunk), heads)
+    got, at = run(slice(None), slice(None)), 0
+    for i, (r, k) in enumerate(portions):
+        assert torch.equal(got[at:at + r], run(slice(at, at + r), slice(i, i + 1))), i
+        if not chunk:
+            for t in {0, r // 2, r - 1}:
+                close(got[at + t], attend_ref(q[at + t], pg.k[i], pg.v[i], k - r + t, 0.2, window, keep, sink.cpu()), BF16, f"portion {i} row {t}")
+        at += r
+
+
 @pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128), (192, 64)])
 @pytest.mark.parametrize("window,keep", [(0, 0), (70, 0), (300, 70)])
 def test_prompt_over_many_pages(window, keep, dim, vdim):

@@ -1045,25 +1045,28 @@ def test_prefill_sequences_by_work(ops, batch, h, kvh, d, paged):
             assert torch.equal(got[rows], run(rows, slice(i, i + 1))), (i, new[i], old[i])
 
 
-@pytest.mark.parametrize("h,kvh,d,new,old,paged,large", [
-    (2, 1, 64, (1024,), (0,), False, False), (2, 2, 128, (1025, 1, 63), (0, 0, 0), False, False), (3, 1, 64, (1100, 65, 0, 130), (0, 0, 0, 0), False, True),
-    (2, 1, 128, (1031, 70), (0, 0), False, True), (2, 1, 128, (65, 1), (1215, 0), True, False), (2, 2, 64, (129, 64, 1), (900, 960, 1023), True, False)])
-def test_prefill_two_groups_share_the_keys(ops, h, kvh, d, new, old, paged, large):
-    """Few rows and long walks: two groups of waves take every other tile of keys; odd and even numbers of tiles, one tile, rows behind cached keys, V that does not fit fp16.
-    Against 64 bits: P and V are rounded to 11 bits (each to half of 2^-10 of itself, so the weighted mean of |v| bounds the error), the output to 8."""
+@pytest.mark.parametrize("h,kvh,d,new,old,form,large", [
+    (2, 1, 64, (1024,), (0,), "fp16", False), (2, 2, 128, (1025, 1, 63), (0, 0, 0), "fp16", False), (3, 1, 64, (1100, 65, 0, 130), (0, 0, 0, 0), "fp16", True),
+    (2, 1, 128, (1031, 70), (0, 0), "fp16", True), (2, 1, 64, (1030,), (0,), "exact", False), (2, 1, 128, (65, 1), (1215, 0), "pages", False),
+    (2, 2, 64, (129, 64, 1), (900, 960, 1023), "pages", False),
+    (48, 2, 64, (2050, 70), (0, 0), "fp16", False), (48, 2, 64, (2050, 70), (0, 0), "exact", False), (48, 2, 64, (2049,), (100,), "pages", False),
+    (48, 2, 128, (700, 577), (0, 0), "fp16", True), (48, 2, 128, (700, 577), (0, 0), "exact", False), (48, 2, 128, (1050,), (300,), "pages", False)])
+def test_prefill_rows_of_a_workgroup_by_fill(ops, h, kvh, d, new, old, form, large):
+    """Few rows and long walks: two groups of waves take every other tile of keys (odd and even numbers of tiles, one tile, rows behind cached keys, V that does not fit fp16);
+    many rows: 128 a workgroup.  Against 64 bits: P and V are rounded to 11 bits (each to half of 2^-10 of itself, so the weighted mean of |v| bounds the error), the output to 8."""
     gen, total = torch.Generator().manual_seed(sum(new)), sum(new)
     q = torch.randn(total, h, d, generator=gen).bfloat16().cuda()
     n_keys = [n + o if n else 0 for n, o in zip(new, old)]
-    assert max(n_keys) >= 1024
-    tables = torch.randperm(len(new) * 6, generator=gen).view(len(new), 6).int().cuda()
-    k, v = (torch.randn(*((len(new) * 6, 256) if paged else (total,)), kvh, d, generator=gen).bfloat16().cuda() for _ in range(2))
+    paged = form == "pages"
+    tables = torch.randperm(len(new) * 9, generator=gen).view(len(new), 9).int().cuda()
+    k, v = (torch.randn(*((len(new) * 9, 256) if paged else (total,)), kvh, d, generator=gen).bfloat16().cuda() for _ in range(2))
     if large:
         v[total // 2, 0, 3] = 1e5
 
     def cu(lengths):
         return torch.tensor([sum(lengths[:i]) for i in range(len(lengths) + 1)], dtype=torch.int32).cuda()
     got = ops.flash_attn_varlen_func(q, k, v, max_seqlen_q=max(new), cu_seqlens_q=cu(new), max_seqlen_k=max(n_keys), cu_seqlens_k=cu(n_keys), softmax_scale=d ** -0.5,
-                                     block_table=tables if paged else None, pv_fp16=None if paged else True)
+                                     block_table=tables if paged else None, pv_fp16=None if paged else form == "fp16")
     at = 0
     for i, (n, m) in enumerate(zip(new, n_keys)):
         if not n:

@@ -719,7 +719,7 @@ int nvh_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, const 
  * g sigmoid(alpha g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit); otherwise
  * out[p] = x[p] . w_e, w = [experts, n, k].
  * tiles == NULL: small batches (bf16, at most 64 rows), the pairs of an expert found from ids; otherwise tiles of tile_rows from
- * nvh_moe_dispatch (bf16: 128 or 256, f32: 64; nvh_moe_tile_rows picks).  n and k multiples of 64. */
+ * nvh_moe_dispatch (bf16: 64, 128 or 256, f32: 64; nvh_moe_tile_rows picks).  n and k multiples of 64. */
 typedef struct nvh_moe_gemm_desc {
     void* out;                   /* [pairs, n] */
     const void* x;               /* glu: [rows, k], row stride x_stride; otherwise [pairs, k] */

@@ -656,14 +656,15 @@ int launch_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, con
     return check_launch("moe_scatter");
 }
 
-// Rows of a tile.  From 256 pairs an expert on, 256: twice the products per byte of weights and rows read.  From 100 to 192 too: an expert's pairs mostly fit one tile, whose
-// missing rows cost little, where many take two of 128.  2048 wide, 32 experts of 1536, softmax router: 100 pairs an expert 194 us against 220, 125
-// 217 against 252, 187 240 against 269; 1024 wide (768): 77 against 80, 80 against 91, 87 against 95.  Below, 128: 75 pairs 197 both (1024 wide 72 against 68).  From 193 to 255
-// an expert's pairs come out on either side of 256, and a second, mostly empty tile costs what the first one gives: 200 pairs still 262 against 285 (1024 wide
-// 89 against 104), 250 pairs 315 against 323 but 1024 wide 122 against 109; there 128 stays.
+// Rows of a tile, by the pairs an expert has on average (us at 2048 wide, 32 experts of 1536, and 1024 wide, of 768; softmax router).  Few: 64, whose images leave room for three
+// workgroups on a CU, as the weight stream wants: 8 pairs 138 against 147 with 128 rows, 16 155 against 167, 25 158 against 170 (1024 wide equal), 41 166 against 162; but where a router crowds them on some experts 31 are
+// 178 against 169.
+// 256, twice the products per byte of weights and rows read, where an expert's pairs mostly fit one such tile: 125 206 against 230 and 80 against 84, 150 212 against 244 and
+// 84 against 88, 237 267 against 284 and 92 against 100, but 100 209 against 210 and 78 against 72; or fill several: 350 316 against 375 and 122 against 123, 500 418 against 485.
+// In between the second tile is mostly empty: 262 316 against 309 and 123 against 104.
 int moe_tile_rows(int pairs, int experts, int f32) {
     const int mean = pairs / experts;
-    return f32 ? FM : mean >= 256 || (mean >= 100 && mean <= 192) ? 256 : 128;
+    return f32 ? FM : mean >= 288 || (mean >= 110 && mean <= 240) ? 256 : mean <= 25 ? 64 : 128;
 }
 
 int launch_moe_gemm(const MoeGemmArgs& a, int f32, hipStream_t stream) {
@@ -683,9 +684,14 @@ int launch_moe_gemm(const MoeGemmArgs& a, int f32, hipStream_t stream) {
         if (a.tile_rows == 256) {
             if (a.glu) gemm_shape<true, 2, 4, 8, 4>(a, stream);
             else gemm_shape<false, 2, 4, 8, 4>(a, stream);
+        } else if (a.tile_rows == 64) {
+            if (a.glu) gemm_shape<true, 2, 2, 2, 4>(a, stream);
+            else gemm_shape<false, 2, 2, 2, 4>(a, stream);
         } else {
-            if (a.glu) gemm_shape<true, 2, 2, 4, 4>(a, stream);
-            else gemm_shape<false, 2, 2, 4, 4>(a, stream);
+            // eight waves of 32 x 64 (94 registers: four on a SIMD) against four of 64 x 64 (146): the rows of pairs that do not exist idle smaller parts, and more waves cover the
+            // loads.  50 pairs an expert 189 -> 169 us, 75 196 -> 173, 100 217 -> 209 (1024 wide 64 -> 59, 67 -> 62, 80 -> 73)
+            if (a.glu) gemm_shape<true, 4, 2, 2, 4>(a, stream);
+            else gemm_shape<false, 4, 2, 2, 4>(a, stream);
         }
     }
     return check_launch("moe_gemm");

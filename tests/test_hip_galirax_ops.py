@@ -502,6 +502,29 @@ def test_expert_tiles_that_are_not_full(tile):
             close(out[p.cuda()], f64(act)[p] @ f64(dn[e]).T, BF16, f"out {e}", slack=2)
 
 
+@pytest.mark.parametrize("tile", [64, 128])
+def test_expert_tiles_by_half_waves(tile):
+    """Last tiles that end around every 16 rows, a wave's whole 32 and half of them, and every tile size the same bits."""
+    from nanovllm_hip import ops
+    counts, n, k = [0, 15, 16, 17, 47, 48, 49, 64, 79, 80, 81, 0, 95, 96, 97, 111, 112, 113, 128, 144, 145], 192, 128
+    flat = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))[torch.randperm(sum(counts), generator=torch.Generator().manual_seed(2))]
+    ids = flat.int()[:, None].cuda()
+    x = randn(len(flat), k, seed=1)
+    gu, dn = randn(len(counts), 2 * n, k, seed=2, scale=k ** -0.5), randn(len(counts), k, n, seed=3, scale=n ** -0.5)
+    got = []
+    for rows in (tile, 256):
+        dispatch = ops.moe_dispatch(ids, len(counts), BF16, rows)
+        act = ops.moe_gemm(x.cuda(), gu.cuda(), ids, True, dispatch)
+        got.append((act, ops.moe_gemm(act, dn.cuda(), ids, False, dispatch)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    act, out = got[0]
+    for e in range(len(counts)):
+        p = (flat == e).nonzero().flatten()
+        if len(p):
+            close(act[p.cuda()], G.silu(f64(x)[p] @ f64(gu[e, :n]).T) * (f64(x)[p] @ f64(gu[e, n:]).T), BF16, f"act {e}", slack=2)
+            close(out[p.cuda()], f64(act)[p] @ f64(dn[e]).T, BF16, f"out {e}", slack=2)
+
+
 # ------------------------------------------------------------------------------------------------ residual, norm, cap
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,cols,n,top", [(3, 64, 64, 0), (5, 320, 300, 4), (17, 2048, 2048, 8), (2, 8192, 8190, 3)])

@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 207          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step */
+#define NVH_VERSION 207          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -734,6 +734,23 @@ typedef struct nvh_moe_gemm_desc {
 } nvh_moe_gemm_desc;
 int nvh_moe_tile_rows(int pairs, int experts, int dtype);
 int nvh_moe_gemm(const nvh_moe_gemm_desc* d, int dtype, void* stream);
+/* Route, dispatch (the small form up to 64 rows in bf16: none) and both products in one call: the launches of the four entries above, in their order. */
+typedef struct nvh_moe_experts_desc {
+    const void* x;               /* [rows, cols], row stride x_stride */
+    int64_t x_stride;
+    const void* router;          /* [experts, cols] */
+    const float* correction;     /* [experts] */
+    const void* gate_up;         /* [experts, 2 * n, cols] */
+    const void* down;            /* [experts, cols, n] */
+    int32_t rows, cols, n, experts, top, groups, keep, softmax;
+    float scale, limit, alpha;
+    void* scratch;               /* nvh_moe_experts_scratch_bytes, 16-byte aligned */
+    size_t scratch_bytes;
+    void* out;                   /* [rows * top, cols] */
+    float* weights;              /* [rows, top] */
+} nvh_moe_experts_desc;
+size_t nvh_moe_experts_scratch_bytes(int rows, int top, int experts, int n, int dtype);
+int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream);
 
 /* x (fp32 stream) += mult * P(y + sum_k ew[row, k] * e[row * top + k])  (each part nullable; P: the layer norm with post_w and post_b where given, nothing
  * otherwise), x += base, x += shift, then, with w given, the layer norm of the new row: (x - mean) / sqrt(var + eps) * w + b. */

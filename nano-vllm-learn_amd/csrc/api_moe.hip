@@ -48,4 +48,63 @@ int nvh_moe_gemm(const nvh_moe_gemm_desc* d, int dtype, void* stream) {
     return launch_moe_gemm(*d, dtype == NVH_F32, (hipStream_t)stream);
 }
 
+// scratch of nvh_moe_experts in 32-bit words: units of the experts | chosen experts | pairs by expert | tiles | counts
+struct MoeScratch {
+    int rows, max_tiles;                             // of a tile; tiles at most (rows 0: the small form, no tiles)
+    size_t ids, slots, tiles, counts, words;
+    MoeScratch(int tokens, int top, int experts, int n, int dtype) {
+        const size_t pairs = (size_t)tokens * top, part = (pairs + 3) / 4 * 4;
+        const bool small = dtype == NVH_BF16 && tokens <= 64;
+        rows = small ? 0 : moe_tile_rows((int)pairs, experts, dtype == NVH_F32);
+        max_tiles = small ? 0 : (int)pairs / rows + experts;
+        ids = pairs * n / (dtype == NVH_F32 ? 1 : 2);
+        slots = ids + part;
+        tiles = slots + (small ? 0 : part);
+        counts = tiles + 4 * (size_t)max_tiles;
+        words = counts + (small ? 0 : (size_t)moe_dispatch_blocks((int)pairs) * experts);
+    }
+};
+static bool moe_sizes_ok(int rows, int top, int experts, int n) {
+    return rows > 0 && top > 0 && experts > 0 && experts <= kMoeMaxExperts && (int64_t)rows * top <= 0x7fffffff && n > 0 && n % 64 == 0;
+}
+
+size_t nvh_moe_experts_scratch_bytes(int rows, int top, int experts, int n, int dtype) {
+    return moe_sizes_ok(rows, top, experts, n) ? 4 * MoeScratch(rows, top, experts, n, dtype).words : 0;
+}
+
+int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream) {
+    REQUIRE(d, NVH_E_NULL, "moe_experts: null descriptor");
+    if (d->rows == 0) return 0;
+    DTYPE("moe_experts");
+    REQUIRE(moe_sizes_ok(d->rows, d->top, d->experts, d->n), NVH_E_SHAPE, "moe_experts: %d rows, top %d of %d experts (<= %d), n %d (%%64)", d->rows, d->top, d->experts, kMoeMaxExperts,
+            d->n);
+    const MoeScratch s(d->rows, d->top, d->experts, d->n, dtype);
+    REQUIRE(d->scratch, NVH_E_NULL, "moe_experts: null pointer");
+    REQUIRE(aligned16(d->scratch), NVH_E_ALIGN, "moe_experts: scratch must be 16-byte aligned");
+    REQUIRE(d->scratch_bytes >= 4 * s.words, NVH_E_WORKSPACE, "moe_experts: scratch %zu B < required %zu B", d->scratch_bytes, 4 * s.words);
+    int32_t* at = reinterpret_cast<int32_t*>(d->scratch);
+    int32_t* const ids = at + s.ids;
+    const int pairs = d->rows * d->top;
+    nvh_moe_route_desc route{};
+    route.x = d->x; route.x_stride = d->x_stride; route.router = d->router; route.correction = d->correction;
+    route.rows = d->rows; route.cols = d->cols; route.experts = d->experts; route.top = d->top; route.groups = d->groups; route.keep = d->keep;
+    route.scale = d->scale; route.ids = ids; route.weights = d->weights; route.softmax = d->softmax;
+    int rc = nvh_moe_route(&route, dtype, stream);
+    if (rc) return rc;
+    nvh_moe_gemm_desc g{};
+    g.out = at; g.x = d->x; g.x_stride = d->x_stride; g.w = d->gate_up;
+    g.pairs = pairs; g.top = d->top; g.experts = d->experts; g.n = d->n; g.k = d->cols; g.glu = 1; g.limit = d->limit; g.alpha = d->alpha;
+    g.ids = ids;
+    if (s.rows) {
+        rc = nvh_moe_dispatch(at + s.slots, at + s.tiles, at + s.counts, ids, pairs, d->experts, s.rows, s.max_tiles, stream);
+        if (rc) return rc;
+        g.slot_pair = at + s.slots; g.tiles = at + s.tiles; g.tile_rows = s.rows;
+        g.max_tiles = s.max_tiles - d->experts + (d->experts < pairs ? d->experts : pairs);
+    }
+    rc = nvh_moe_gemm(&g, dtype, stream);
+    if (rc) return rc;
+    g.out = d->out; g.x = at; g.w = d->down; g.n = d->cols; g.k = d->n; g.glu = 0; g.limit = g.alpha = 0.f;
+    return nvh_moe_gemm(&g, dtype, stream);
+}
+
 }  // extern "C"

@@ -130,6 +130,16 @@ class MoeGemmDesc(ctypes.Structure):
                 ("limit", ctypes.c_float), ("alpha", ctypes.c_float)]
 
 
+class MoeExpertsDesc(ctypes.Structure):
+    """nvh_moe_experts_desc (include/nvh_attn.h)."""
+    _fields_ = [("x", ctypes.c_void_p), ("x_stride", ctypes.c_int64), ("router", ctypes.c_void_p), ("correction", ctypes.c_void_p),
+                ("gate_up", ctypes.c_void_p), ("down", ctypes.c_void_p), ("rows", ctypes.c_int32), ("cols", ctypes.c_int32),
+                ("n", ctypes.c_int32), ("experts", ctypes.c_int32), ("top", ctypes.c_int32), ("groups", ctypes.c_int32),
+                ("keep", ctypes.c_int32), ("softmax", ctypes.c_int32), ("scale", ctypes.c_float), ("limit", ctypes.c_float),
+                ("alpha", ctypes.c_float), ("scratch", ctypes.c_void_p), ("scratch_bytes", ctypes.c_size_t), ("out", ctypes.c_void_p),
+                ("weights", ctypes.c_void_p)]
+
+
 class ResidualNormDesc(ctypes.Structure):
     """nvh_residual_norm_desc (include/nvh_attn.h)."""
     _fields_ = [("x", ctypes.c_void_p), ("y", ctypes.c_void_p), ("y_stride", ctypes.c_int64), ("e", ctypes.c_void_p),
@@ -305,6 +315,8 @@ _SIGS = {
     "nvh_moe_dispatch": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 + [ctypes.c_void_p]),
     "nvh_moe_tile_rows": (ctypes.c_int, [ctypes.c_int] * 3),
     "nvh_moe_gemm": (ctypes.c_int, [ctypes.POINTER(MoeGemmDesc), ctypes.c_int, ctypes.c_void_p]),
+    "nvh_moe_experts_scratch_bytes": (ctypes.c_size_t, [ctypes.c_int] * 5),
+    "nvh_moe_experts": (ctypes.c_int, [ctypes.POINTER(MoeExpertsDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_residual_norm": (ctypes.c_int, [ctypes.POINTER(ResidualNormDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_poly_norm": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_float] + [ctypes.c_int] * 3 + [ctypes.c_int64] * 2 + [ctypes.c_int, ctypes.c_void_p]),
     "nvh_softcap": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),

@@ -35,8 +35,5 @@ class MixtureOfExperts(nn.Module):
 
     def forward(self, x):
         """x [rows, in_cols] -> (expert outputs [rows * top, in_cols], weights fp32 [rows, top])."""
-        ids, weights = ops.moe_route(x, self.router, self.correction, self.top, self.groups, self.keep, self.scale, self.softmax)
-        small = x.dtype == torch.bfloat16 and x.shape[0] <= ops.LINEAR_SMALL_M_MAX
-        dispatch = None if small else ops.moe_dispatch(ids, self.experts, x.dtype)
-        act = ops.moe_gemm(x, self.w_gate_up, ids, True, dispatch, self.unit)
-        return ops.moe_gemm(act, self.w_down, ids, False, dispatch), weights
+        b = self._buffers                             # (past nn.Module's attribute lookup: 0.6 us each)
+        return ops.moe_experts(x, b["router"], b["correction"], b["w_gate_up"], b["w_down"], self.top, self.groups, self.keep, self.scale, self.softmax, self.unit)

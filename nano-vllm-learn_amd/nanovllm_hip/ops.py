@@ -1485,6 +1485,29 @@ def moe_gemm(x, weight, ids, glu, dispatch=None, unit=None):
     return out
 
 
+def moe_experts(x, router, correction, gate_up, down, top, groups=1, keep=1, scale=1.0, softmax=False, unit=None):
+    """(expert outputs [rows * top, cols], weights fp32 [rows, top]): moe_route, moe_dispatch (up to LINEAR_SMALL_M_MAX rows in bf16: none) and both moe_gemm in one
+    call, the same launches.  (Four calls with a descriptor each took the host 40 to 59 us, more than the kernels of up to some 400
+    tokens at 1024 wide; this one takes 22 to 29: 5 tokens 38.5 -> 25 us a pass, 100 55 -> 41.)"""
+    code = _act_code(x, router, gate_up, down)
+    _require_f32(correction=correction)
+    rows, cols = x.shape
+    experts, n, k = down.shape[0], down.shape[2], gate_up.shape[2]
+    assert router.is_contiguous() and router.shape == (experts, cols) and x.stride(1) == 1 and correction.numel() == experts
+    assert gate_up.is_contiguous() and down.is_contiguous() and k == cols and gate_up.shape[:2] == (experts, 2 * n) and down.shape[1] == cols
+    limit, alpha = (0.0, 0.0) if unit is None else (float(unit[0]), float(unit[1]))
+    assert unit is None or alpha != 0.0
+    lib, top = _lib.load(), int(top)
+    words = lib.nvh_moe_experts_scratch_bytes(rows, top, experts, n, code) >> 2
+    scratch = torch.empty(words, dtype=torch.int32, device=x.device)
+    weights = torch.empty((rows, top), dtype=torch.float32, device=x.device)
+    out = torch.empty((rows * top, cols), dtype=x.dtype, device=x.device)
+    d = _lib.MoeExpertsDesc(x.data_ptr(), x.stride(0), router.data_ptr(), correction.data_ptr(), gate_up.data_ptr(), down.data_ptr(), rows, cols, n, experts, top, int(groups),
+                            int(keep), int(softmax), float(scale), limit, alpha, scratch.data_ptr(), 4 * words, out.data_ptr(), weights.data_ptr())
+    _lib.check(lib.nvh_moe_experts(ctypes.byref(d), code, _stream()), "nvh_moe_experts")
+    return out, weights
+
+
 # --------------------------------------------------------------------------------------- residual and output of models with one norm per layer
 def residual_norm(x, dtype, y=None, experts=None, weight=None, bias=None, eps=0.0, n=0, packed=None, want_rows=True, post=None, mult=1.0, base=None, shift=None):
     """x (fp32 stream, in place) += y + the weighted sum of experts = (outputs [rows * top, cols], weights [rows, top]), or mult times the layer norm of that sum

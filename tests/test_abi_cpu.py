@@ -98,6 +98,22 @@ def test_argument_validation_without_gpu(lib):
     assert lib.nvh_prefill_varlen_pv16(p, p, p, p, p, p, 0, 0, 0, 0, 14, 2, 64, 896, 128, 128, 0.125, 0, 0, None, 0, None) == 0   # empty batch
 
 
+def test_experts_in_one_call_refuse_scratch_that_is_too_small(lib):
+    """Scratch is a pure function of the sizes (no tiles up to 64 rows in bf16, always some in fp32); nothing is launched without all of it."""
+    from nanovllm_hip import _lib
+    p = ctypes.c_void_p(4096)
+    assert [lib.nvh_moe_experts_scratch_bytes(*a) for a in ((0, 2, 8, 64, 0), (5, 2, 8, 60, 0), (5, 2, 4096, 64, 0), (5, 0, 8, 64, 0))] == [0] * 4
+    assert lib.nvh_moe_experts_scratch_bytes(5, 2, 8, 64, 0) == 4 * (10 * 64 // 2 + 12)
+    assert lib.nvh_moe_experts_scratch_bytes(100, 2, 8, 64, 0) == 4 * (200 * 64 // 2 + 2 * 200 + 4 * (200 // 64 + 8) + 8)
+    assert lib.nvh_moe_experts_scratch_bytes(5, 2, 8, 64, 1) == 4 * (10 * 64 + 2 * 12 + 4 * 8 + 8)
+    d = _lib.MoeExpertsDesc(p, 64, p, p, p, p, 100, 64, 64, 8, 2, 1, 1, 0, 1.0, 0.0, 0.0, p, lib.nvh_moe_experts_scratch_bytes(100, 2, 8, 64, 0) - 4, p, p)
+    assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == -4 and b"scratch" in lib.nvh_last_error()
+    d.scratch_bytes, d.scratch = 1 << 20, None
+    assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == -5
+    d.scratch, d.scratch_bytes, d.rows = p, 0, 0
+    assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == 0
+
+
 def test_ops_refuse_cpu_tensors():
     """No CPU fallback: the product path must fail loudly off-GPU."""
     from nanovllm_hip import ops

@@ -525,6 +525,38 @@ def test_expert_tiles_by_half_waves(tile):
             close(out[p.cuda()], f64(act)[p] @ f64(dn[e]).T, BF16, f"out {e}", slack=2)
 
 
+@pytest.mark.parametrize("rows,experts,top,dtype,softmax", [(1, 8, 2, BF16, True), (64, 5, 3, BF16, False), (65, 6, 1, BF16, True), (300, 16, 3, BF16, False), (900, 4, 2, BF16, True),
+                                                            (1, 3, 3, F32, False), (130, 7, 2, F32, True)])
+def test_experts_in_one_call(rows, experts, top, dtype, softmax):
+    """Bit for bit the four calls one after the other; eager, and from a graph with other rows behind it; no rows at all."""
+    from nanovllm_hip import ops
+    cols, n, unit = 128, 192, (7.0, 1.702) if softmax else None
+    x = randn(rows, 2 * cols, seed=1, dtype=dtype).cuda()[:, :cols]
+    router, bias = randn(experts, cols, seed=2, dtype=dtype).cuda(), randn(experts, seed=3, dtype=F32).cuda()
+    gu, dn = (randn(experts, *shape, seed=4, scale=shape[1] ** -0.5, dtype=dtype).cuda() for shape in ((2 * n, cols), (cols, n)))
+
+    def one():
+        return ops.moe_experts(x, router, bias, gu, dn, top, softmax=softmax, unit=unit)
+
+    def four():
+        ids, weights = ops.moe_route(x, router, bias, top, softmax=softmax)
+        dispatch = None if dtype == BF16 and rows <= 64 else ops.moe_dispatch(ids, experts, dtype)
+        return ops.moe_gemm(ops.moe_gemm(x, gu, ids, True, dispatch, unit), dn, ids, False, dispatch), weights
+    for got, want in zip(one(), four()):
+        assert torch.equal(got, want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        kept = one()
+    for seed in (5, 6, 7):
+        x.copy_(randn(rows, cols, seed=seed, dtype=dtype).cuda())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(got, want) for got, want in zip(kept, four()))
+    out, weights = ops.moe_experts(x[:0], router, bias, gu, dn, top, softmax=softmax, unit=unit)
+    assert out.shape == (0, cols) and weights.shape == (0, top)
+
+
 # ------------------------------------------------------------------------------------------------ residual, norm, cap
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,cols,n,top", [(3, 64, 64, 0), (5, 320, 300, 4), (17, 2048, 2048, 8), (2, 8192, 8190, 3)])

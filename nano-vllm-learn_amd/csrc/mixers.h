@@ -77,10 +77,17 @@ __device__ __forceinline__ float wave_sum64(float v) {
 // alike).  Workgroups start in the order of their numbers, all of them at once where they fit: the last ones share a compute unit with others, which should be short, and where some
 // wait, the long ones should not.  Uneven portions: 11 of 1090 tokens on average, time mixing with 32 heads 160 -> 137 us; 24 of 670, lightning attention with 16 heads 120 -> 102;
 // 30 of 300, scan of 4096 channels 170 -> 158; 5 of 3277, 2048 channels, a state per lane 223 -> 215.  With a compute unit each any order does.
-template <typename Args>
+// Two workgroups a compute unit (PAIRS) and fewer than two for each: the longest portions go to the units that get one, and of the others the longest starts beside the shortest (a
+// unit takes another workgroup once each has one, in the same order; were it not so, the order would only be another one).  11 portions, 32 heads: 139 -> 130 us; 14 of 857, 120 -> 109;
+// 16 of 1000, 146 -> 138.
+template <bool PAIRS = false, typename Args>
 __device__ __forceinline__ int longest_first(const Args& a, int walks_each) {
-    const int nth = blockIdx.y;
+    int nth = blockIdx.y;
     if (a.n_chunks > 64 || a.summaries || a.n_chunks * walks_each <= 256) return nth;
+    if constexpr (PAIRS) {
+        const int each = 256 / walks_each, two = a.n_chunks - each;            // portions whose walks come first, and that share
+        if (two <= each) nth = nth < two ? each - two + nth : nth < each ? nth - two : a.n_chunks - 1 - (nth - each);
+    }
     const int lane = threadIdx.x & 63, n = a.chunks[4 * (lane < a.n_chunks ? lane : 0) + 1], steps = n > 0 ? (n + 15) >> 4 : 0;
     return nth_largest<10>(steps < 1023 ? steps : 1023, a.n_chunks, nth);
 }

@@ -77,7 +77,7 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     Lds& lds = *reinterpret_cast<Lds*>(smem);
     auto swz = [](int r) { return ROW == 128 ? (r >> 1) & 7 : r & 15; };       // rows of 256 bytes span all banks
-    const int head = blockIdx.x, seg = longest_first(a, a.heads);    // heads run fastest: workgroups are dealt round-robin over the XCDs
+    const int head = blockIdx.x, seg = longest_first<DIM == 64>(a, a.heads);    // heads run fastest: workgroups are dealt round-robin over the XCDs
     const int32_t* ch = a.chunks + 4 * seg;
     const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
     const bool last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;

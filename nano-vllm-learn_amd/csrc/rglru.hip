@@ -412,7 +412,7 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs
         const int ln = fresh(lane), lq = ln & 15, lg = ln >> 4, piece = 2 * wave + (lq >> 3);
         const auto at = [](int row, int p) { const int s = row * OCT + p; return s / 64 * YDMA + s % 64 * 8; };
         const uint16_t* u_row = u_lds + lq * LD + 8 * lg;
-        const uint16_t* y_row = y_now + at(lq, ((wave >> 1) * 4 + lg) ^ (lq & 1));
+        const uint16_t* y_row = y_now + at(lq, (2 * wave + (lg & 1)) ^ (lq & 1));        // (its own channels' pieces, twice: the other half's are on their way out)
         uint16_t* y_even = y_now + at(4 * lg, piece) + (lq & 7);               // this lane's channel in rows 4 lg and, by fixed distances, 4 lg + 2
         uint16_t* y_odd = y_now + at(4 * lg, piece ^ 1) + (lq & 7);            // ... and, likewise, in 4 lg + 1 and 4 lg + 3
 #pragma unroll
@@ -895,7 +895,8 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_chain_kernel(const RglruArg
         }
         {
             const int ln = lane_now(), lq = ln & 15, lg = ln >> 4, piece = 2 * wave + (lq >> 3);
-            const uint16_t* y_row = y_now + place(lq, ((wave >> 1) * 4 + lg) ^ (lq & 1));
+            // This wave's pieces, twice.  (The other half's, which the selection multiplies by zero, its wave replaces by what goes out, and zero times an infinity is none.)
+            const uint16_t* y_row = y_now + place(lq, (2 * wave + (lg & 1)) ^ (lq & 1));
             uint16_t* y_even = y_now + place(4 * lg, piece) + (lq & 7);        // this lane's channel in rows 4 lg and, by fixed distances, 4 lg + 2
             uint16_t* y_odd = y_now + place(4 * lg, piece ^ 1) + (lq & 7);     // ... and, likewise, in 4 lg + 1 and 4 lg + 3
             const bf16x8 sel = selection(ln);

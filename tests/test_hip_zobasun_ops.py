@@ -286,6 +286,7 @@ def test_recurrence_steps_by_any_workgroup(blocks, block, taps, lengths):
         got = go()
         infinite = ~torch.isfinite(want)                        # (walks lose an infinite state to NaN where decays multiply to zero)
         assert ((got - want)[~infinite].abs() <= 2 ** -7 * want[~infinite].abs() + 1e-3).all() and (~torch.isfinite(got[infinite])).all()
+        assert (~torch.isfinite(got)).any(dim=0).nonzero().flatten().tolist() in ([], [5])         # an infinity stays in its channel
         fine = torch.isfinite(wanted[0])
         assert (after[0] - wanted[0])[fine].abs().max() <= 2e-5 * wanted[0][fine].abs().max() and torch.equal(after[1], wanted[1]) and not torch.isnan(after[0]).any()
         if first_run is not None and max(lengths) > 320:        # (otherwise whole portions may be walked)
@@ -300,6 +301,23 @@ def test_recurrence_steps_by_any_workgroup(blocks, block, taps, lengths):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(again, first_run[0]) and torch.equal(after[0], first_run[1])
+
+
+@pytest.mark.parametrize("form", [0, 2])
+@pytest.mark.parametrize("blocks,block", [(2, 32), (3, 256)])
+def test_recurrence_infinity_stays_in_its_channel(blocks, block, form):
+    """Rows go out in the place of the gate's rows, which the waves of neighbouring channels read as multiplied by zero: many portions, each from an infinite state of one channel."""
+    from nanovllm_hip import ops
+    from nanovllm_hip.engine.model_runner import recurrence_chunks
+    n, m = 200, 70
+    r = Recurrence(blocks, block, block, 4, torch.bfloat16, slots=n)
+    r.state.zero_(), r.conv_state.zero_()
+    r.state[:, 5] = float("inf")
+    yx, chunks = r.rows(*r.yx(n * m, 1)), [c for i in range(n) for c in recurrence_chunks(i * m, m, i, 64)]
+    pos, slots, table = (torch.arange(n * m) % m + 1).cuda(), torch.arange(n, dtype=torch.int32, device="cuda"), torch.tensor(chunks, dtype=torch.int32, device="cuda")
+    for _ in range(6):
+        out = ops.rglru_chunks(yx, r.params, pos, slots, table, 64, True, r.state.clone(), r.conv_state.clone(), generic=form)
+        assert (~torch.isfinite(out)).any(dim=0).nonzero().flatten().tolist() == [5]
 
 
 @pytest.mark.parametrize("blocks,size,block,taps", SHAPES)

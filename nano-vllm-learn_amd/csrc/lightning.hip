@@ -577,20 +577,25 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
     }
 }
 
-// contributions of the segments -> states at their starts, in place; one thread per state element, walking the segments of every portion
+// contributions of the segments -> states at their starts, in place; a thread per four state elements of a portion, walking its segments
 __global__ __launch_bounds__(256) void lightning_starts_kernel(const LightningArgs a) {
-    const int64_t head_state = (int64_t)a.dk * a.dv, per = a.heads * head_state, e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t head_state = (int64_t)a.dk * a.dv, per = a.heads * head_state, e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     const int first = blockIdx.y;                    // only a portion's first segment starts a walk
-    if (e >= per || a.chunks[4 * first + 3] != 0) return;
+    if (a.chunks[4 * first + 3] != 0) return;
+    const int count = portion_segments(a.chunks, a.n_chunks, first);
+    if (e >= per) return;
     const float d = a.decay[e / head_state];
     const int64_t slot = a.state_slots[a.chunks[4 * first + 2]];
-    float cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? a.state[slot * per + e] : 0.f;
-    for (int c = first; c < a.n_chunks && (c == first || a.chunks[4 * c + 3] != 0); ++c) {
-        const bool more = c + 1 < a.n_chunks && a.chunks[4 * (c + 1) + 3] != 0;        // (the last segment left no contribution)
-        const float own = more ? a.seg_state[c * per + e] : 0.f;
-        a.seg_state[c * per + e] = cur;
-        cur = powf(d, (float)a.chunks[4 * c + 1]) * cur + own;
-    }
+    const f32x4 cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? *reinterpret_cast<const f32x4*>(a.state + slot * per + e) : f32x4{};
+    float of = 0.f, power = 1.f;                     // (segments but the last are of one length)
+    segment_starts(a.seg_state + first * per + e, per, count, cur, [&](int k) { return (float)a.chunks[4 * (first + k) + 1]; },
+                   [&](float tokens) {
+                       if (tokens != of) {
+                           of = tokens;
+                           power = powf(d, tokens);
+                       }
+                       return power;
+                   });
 }
 
 // ------------------------------------------------------------------------------------------------ token by token, any type and size
@@ -736,7 +741,7 @@ int walk_wide(const LightningArgs& a, hipStream_t stream) {
         int rc = check_launch("lightning summary");
         if (rc) return rc;
         const int64_t per = (int64_t)a.heads * a.dk * a.dv;
-        lightning_starts_kernel<<<dim3((unsigned)((per + 255) / 256), a.n_chunks), 256, 0, stream>>>(a);
+        lightning_starts_kernel<<<dim3((unsigned)((per + 1023) / 1024), a.n_chunks), 256, 0, stream>>>(a);
         rc = check_launch("lightning starts");
         if (rc) return rc;
     }
@@ -758,7 +763,7 @@ int pair_dk(const LightningArgs& a, hipStream_t stream) {
         int rc = check_launch("lightning summary");
         if (rc) return rc;
         const int64_t per = (int64_t)a.heads * a.dk * a.dv;
-        lightning_starts_kernel<<<dim3((unsigned)((per + 255) / 256), a.n_chunks), 256, 0, stream>>>(a);
+        lightning_starts_kernel<<<dim3((unsigned)((per + 1023) / 1024), a.n_chunks), 256, 0, stream>>>(a);
         rc = check_launch("lightning starts");
         if (rc) return rc;
     }

@@ -366,20 +366,21 @@ __global__ __launch_bounds__(256) void scan_rows_kernel(const ScanArgs a) {
     if (c0 + lc < a.inner && slot >= 0) a.state[(slot * a.inner + my) * 16 + st] = S;
 }
 
-// contributions of the segments -> states at their starts, in place; one thread per state, walking the segments of every portion
+// contributions of the segments -> states at their starts, in place; a thread per four states of a portion, walking its segments
 __global__ __launch_bounds__(256) void scan_starts_kernel(const ScanArgs a) {
-    const int64_t per = (int64_t)a.inner * a.n, e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t per = (int64_t)a.inner * a.n, e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     const int first = blockIdx.y;                    // only a portion's first segment starts a walk
-    if (e >= per || a.chunks[4 * first + 3] != 0) return;
-    const float A = a.a_log2[e];
+    if (a.chunks[4 * first + 3] != 0) return;
+    const int count = portion_segments(a.chunks, a.n_chunks, first);
+    if (e >= per) return;
+    const f32x4 A = *reinterpret_cast<const f32x4*>(a.a_log2 + e);
     const int64_t c = e / a.n, slot = a.state_slots[a.chunks[4 * first + 2]];
-    float cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? a.state[slot * per + e] : 0.f;
-    for (int k = first; k < a.n_chunks && (k == first || a.chunks[4 * k + 3] != 0); ++k) {
-        const bool more = k + 1 < a.n_chunks && a.chunks[4 * (k + 1) + 3] != 0;        // (the last segment left no contribution)
-        const float own = more ? a.seg_state[k * per + e] : 0.f;
-        a.seg_state[k * per + e] = cur;
-        if (more) cur = fast_exp2(A * a.seg_dt[k * a.inner + c]) * cur + own;
-    }
+    const f32x4 cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? *reinterpret_cast<const f32x4*>(a.state + slot * per + e) : f32x4{};
+    segment_starts(a.seg_state + first * per + e, per, count, cur, [&](int k) { return a.seg_dt[(int64_t)(first + k) * a.inner + c]; },
+                   [&](float dt) {
+                       const f32x4 p = A * dt;
+                       return f32x4{fast_exp2(p[0]), fast_exp2(p[1]), fast_exp2(p[2]), fast_exp2(p[3])};
+                   });
 }
 
 // one new token per sequence (bf16): grid (channel groups, groups of R rows), LN = n / 4 lanes per channel
@@ -450,7 +451,7 @@ int walk_ns(const ScanArgs& a, hipStream_t stream) {
         int rc = check_launch("scan summary");
         if (rc) return rc;
         const int64_t per = (int64_t)a.inner * a.n;
-        scan_starts_kernel<<<dim3((unsigned)((per + 255) / 256), a.n_chunks), 256, 0, stream>>>(a);
+        scan_starts_kernel<<<dim3((unsigned)((per + 1023) / 1024), a.n_chunks), 256, 0, stream>>>(a);
         rc = check_launch("scan starts");
         if (rc) return rc;
     }

@@ -203,6 +203,49 @@ __device__ __forceinline__ bool portion_carries(const int32_t* chunks, int n_chu
         if (chunks[4 * c + 1] > 0) return positions[chunks[4 * c]] > 0;
     return true;
 }
+
+// Segments of the portion whose first one is row `first` of the table (all lanes of a wave ask).
+__device__ __forceinline__ int portion_segments(const int32_t* chunks, int n_chunks, int first) {
+    int count = 1, run;
+    do {
+        const int c = first + count + (int)(threadIdx.x & 63);
+        const uint64_t others = ~__builtin_amdgcn_ballot_w64(c < n_chunks && chunks[4 * c + 3] != 0);
+        run = others ? __builtin_ctzll(others) : 64;
+        count += run;
+    } while (run == 64);
+    return count;
+}
+
+// Contributions of a portion's `count` segments -> states at their starts, in place, of the four neighbouring state elements at own: own[k * per ..] of segment k, `cur` in front
+// of the first (the last segment left no contribution).  ahead(k) is what the factor of segment k comes from, factor() of it the factor.
+// Nothing a segment reads depends on the one before, but its store might be the next one's load for all the compiler knows: one at a time a segment cost a trip to
+// memory.  Up to 16 of them are asked for together.  33 segments, 8 heads of 128 x 128 states: 25.8 -> 10.2 us (one element a thread 12.6); 16 of 64 x 64 16.4 -> 8.6; 2048 channels
+// of 16 states 15.8 -> 6.6.  3 portions of 5 segments, 16 heads of 128 x 128: 18.6 -> 7.8.
+template <int U, typename Ahead, typename Factor>
+__device__ __forceinline__ void segment_starts_of(float* own, int64_t per, int k0, f32x4& cur, Ahead ahead, Factor factor) {
+    f32x4 mine[U];
+    float raw[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        mine[u] = *reinterpret_cast<const f32x4*>(own + (k0 + u) * per);
+        raw[u] = ahead(k0 + u);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        *reinterpret_cast<f32x4*>(own + (k0 + u) * per) = cur;
+        cur = factor(raw[u]) * cur + mine[u];
+    }
+}
+template <typename Ahead, typename Factor>
+__device__ __forceinline__ void segment_starts(float* own, int64_t per, int count, f32x4 cur, Ahead ahead, Factor factor) {
+    int k = 0;
+    for (; k + 16 < count; k += 16) segment_starts_of<16>(own, per, k, cur, ahead, factor);
+    if (k + 8 < count) segment_starts_of<8>(own, per, k, cur, ahead, factor), k += 8;
+    if (k + 4 < count) segment_starts_of<4>(own, per, k, cur, ahead, factor), k += 4;
+    if (k + 2 < count) segment_starts_of<2>(own, per, k, cur, ahead, factor), k += 2;
+    if (k + 1 < count) segment_starts_of<1>(own, per, k, cur, ahead, factor), k += 1;
+    *reinterpret_cast<f32x4*>(own + k * per) = cur;
+}
 // What a workgroup leaves of `rows` x `cols` state elements behind a segment without rows: a summary of nothing, or the state at its start.
 template <bool SUMMARY>
 __device__ __forceinline__ void pass_segment(float* seg_state, float* state, int rows, int cols, int64_t stride) {

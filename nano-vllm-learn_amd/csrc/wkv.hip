@@ -465,19 +465,16 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
     }
 }
 
-// contributions of the segments -> states at their starts, in place; one thread per state element, walking the segments of every portion
+// contributions of the segments -> states at their starts, in place; a thread per four state elements of a portion, walking its segments
 __global__ __launch_bounds__(256) void wkv_starts_kernel(const WkvArgs a) {
-    const int64_t per = (int64_t)a.heads * a.dim * a.dim, e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t per = (int64_t)a.heads * a.dim * a.dim, e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     const int first = blockIdx.y;                    // only a portion's first segment starts a walk
-    if (e >= per || a.chunks[4 * first + 3] != 0) return;
-    const int64_t ch = e / a.dim, slot = a.state_slots[a.chunks[4 * first + 2]];
-    float cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? a.state[slot * per + e] : 0.f;
-    for (int c = first; c < a.n_chunks && (c == first || a.chunks[4 * c + 3] != 0); ++c) {
-        const bool more = c + 1 < a.n_chunks && a.chunks[4 * (c + 1) + 3] != 0;        // (the last segment left no contribution)
-        const float own = more ? a.seg_state[c * per + e] : 0.f;
-        a.seg_state[c * per + e] = cur;
-        if (more) cur = fast_exp2(a.seg_decay[(int64_t)c * a.heads * a.dim + ch]) * cur + own;
-    }
+    if (a.chunks[4 * first + 3] != 0) return;
+    const int count = portion_segments(a.chunks, a.n_chunks, first);
+    if (e >= per) return;
+    const int64_t ch = e / a.dim, slot = a.state_slots[a.chunks[4 * first + 2]], channels = (int64_t)a.heads * a.dim;
+    const f32x4 cur = slot >= 0 && portion_carries(a.chunks, a.n_chunks, first, a.positions) ? *reinterpret_cast<const f32x4*>(a.state + slot * per + e) : f32x4{};
+    segment_starts(a.seg_state + first * per + e, per, count, cur, [&](int k) { return a.seg_decay[(first + k) * channels + ch]; }, [](float decay) { return fast_exp2(decay); });
 }
 
 // ------------------------------------------------------------------------------------------------ token by token, any type and size
@@ -621,7 +618,7 @@ int walk_off(const WkvArgs& a, hipStream_t stream) {
         int rc = check_launch("wkv summary");
         if (rc) return rc;
         const int64_t per = (int64_t)a.heads * DIM * DIM;
-        wkv_starts_kernel<<<dim3((unsigned)((per + 255) / 256), a.n_chunks), 256, 0, stream>>>(a);
+        wkv_starts_kernel<<<dim3((unsigned)((per + 1023) / 1024), a.n_chunks), 256, 0, stream>>>(a);
         rc = check_launch("wkv starts");
         if (rc) return rc;
     }

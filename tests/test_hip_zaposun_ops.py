@@ -692,3 +692,38 @@ def test_portions_longest_first(kind, portions):
             want = run(rows, pos[rows], slots[i:i + 1], torch.tensor([(0, n, 0, 0)], dtype=torch.int32).cuda(), False, alone)
             assert torch.equal(got[rows], want), (i, n)
     assert torch.equal(after, alone)
+
+
+# segments of a portion that are asked for together: 16, then 8, 4, 2 and 1 of those that follow; 64 rows of the table at a time
+SEGMENT_COUNTS = [1, 2, 3, 4, 8, 9, 16, 17, 18, 33, 48, 64, 65, 66, 130]
+
+
+@pytest.mark.parametrize("mechanism", ["scan", "time mixing", "lightning"])
+def test_states_at_the_starts_of_many_segments(mechanism):
+    """Portions of 1 to 130 segments, every other one behind a state, against the same portions whole: sums of 64 tokens' contributions in another order."""
+    lengths = [64 * (n - 1) + 1 + 7 * i % 64 for i, n in enumerate(SEGMENT_COUNTS)]
+    first, rows, count = [sum(lengths[:i]) for i in range(len(lengths))], sum(lengths), len(lengths)
+    pos = torch.cat([torch.arange(n) + (0 if i % 2 else 100) for i, n in enumerate(lengths)]).cuda()
+    slots = torch.randperm(count, generator=torch.Generator().manual_seed(0)).int().cuda()
+    if mechanism == "scan":
+        layer = Scan([1], 72, 8, 8, BF16)
+        args = [randn(rows, w, seed=s, dtype=BF16).cuda() for s, w in ((1, 72), (2, 72), (3, 16), (4, 72))]
+        args, state = (*args, layer.params, pos, slots), randn(count, 72, 8, seed=5, dtype=F32).cuda()
+        run = lambda chunks, s: ops().scan_chunks(*args, chunks, chunks.shape[0] > count, s)
+    elif mechanism == "time mixing":
+        layer = Wkv([1], 2, 64, 64, BF16, DECAYS["slow"])
+        args = [randn(rows, 128, seed=s, dtype=BF16).cuda() for s in (1, 2, 3, 4)] + [randn(rows, 128, seed=5, dtype=BF16, scale=0.3).cuda()]
+        args, state = (*args, layer.params, layer.eps, layer.dim, pos, slots), randn(count, 2, 64, 64, seed=6, dtype=F32).cuda()
+        run = lambda chunks, s: ops().wkv_chunks(*args, chunks, chunks.shape[0] > count, s)
+    else:
+        decay = torch.tensor([0.97, 0.9995], dtype=F32).cuda()
+        args, state = (randn(rows, 2 * 192, seed=1, dtype=BF16).cuda(), decay, pos, slots), randn(count, 2, 64, 64, seed=2, dtype=F32).cuda()
+        run = lambda chunks, s: ops().lightning_chunks(*args, chunks, chunks.shape[0] > count, s)
+
+    def table(segment):
+        return torch.tensor([(f + a, min(segment, n - a), i, a // segment) for i, (f, n) in enumerate(zip(first, lengths)) for a in range(0, n, segment)], dtype=torch.int32).cuda()
+    one, many = state.clone(), state.clone()
+    want, got = run(table(64 * max(SEGMENT_COUNTS)), one), run(table(64), many)
+    for i, (f, n) in enumerate(zip(first, lengths)):
+        close(got[f:f + n], f64(want[f:f + n]), BF16, f"{SEGMENT_COUNTS[i]} segments")
+        close(many[slots[i]], f64(one[slots[i]]), F32, f"state behind {SEGMENT_COUNTS[i]} segments", slack=64)

@@ -456,6 +456,21 @@ def test_dispatch(pairs_shape, experts, dtype):
     assert seen.all() and all(t[3] == used for t in tiles.tolist())
 
 
+# pairs on both sides of what a workgroup takes (2048) and of what is counted without a launch of its own (8192); experts up to the most
+@pytest.mark.parametrize("pairs,experts", [(2047, 7), (2048, 1), (2049, 33), (6145, 1024), (8191, 32), (8192, 64), (8193, 32)])
+def test_dispatch_counts(pairs, experts):
+    from nanovllm_hip import ops
+    ids = (torch.randint(0, experts, (pairs, 1), generator=torch.Generator().manual_seed(pairs)) * torch.linspace(1, 0.3, pairs)[:, None]).int()      # (uneven, also from workgroup to workgroup)
+    slots, tiles, rows = ops.moe_dispatch(ids.cuda(), experts, BF16)
+    counts, flat = torch.bincount(ids.flatten(), minlength=experts).tolist(), ids.flatten().long()
+    assert flat[slots.cpu().long()].tolist() == sorted(flat.tolist()) and sorted(slots.tolist()) == list(range(pairs))
+    want, first = [], 0
+    for e, n in enumerate(counts):
+        want += [[e, first + t, min(rows, n - t)] for t in range(0, n, rows)]
+        first += n
+    assert [t[:3] for t in tiles.tolist()[:len(want)]] == want and all(t[2:] == [0, len(want)] for t in tiles.tolist()[len(want):])
+
+
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,top,experts,n,k", [(1, 2, 4, 64, 64), (5, 4, 8, 128, 320), (33, 8, 16, 192, 128), (64, 1, 2, 64, 1088), (40, 3, 3, 2112, 192), (65, 2, 9, 64, 128),
                                                   (300, 4, 8, 192, 256), (700, 2, 3, 128, 64)])

@@ -155,7 +155,7 @@ int nvh_decode_step(void* out, const void* q, const void* k_new, const void* v_n
  *   cu_seqlens_q/k int32 [batch+1] on device; max_seqlen_q bounds the launch grid (host int, as in
  *                  model_runner.py:204-207).  The causal mask is bottom-right aligned: query row r
  *                  of a sequence sees keys 0 .. r + (Sk - Sq)  (flash-attn semantics; equals the
- *                  oracle's top-left mask whenever Sq == Sk).
+ *                  oracle's top-left mask whenever Sq == Sk); rows that see none (Sq > Sk) come out as zeros.
  *                  CONTRACT: max_seqlen_q / max_seqlen_k must bound every sequence in cu_seqlens_q/k (as the reference's
  *                  runner guarantees).  The library cannot check device data without a host sync; rows / keys beyond an
  *                  understated maximum are not processed (never an out-of-bounds access).

@@ -170,6 +170,17 @@ __device__ __forceinline__ void prefill_tile_of_block(const PrefillArgs& a, int&
 #endif
 }
 
+// rows row0 .. of one head that see no key
+template <int D, int THREADS>
+__device__ __forceinline__ void zero_rows(const PrefillArgs& a, int row0, int n, int head, int tid) {
+    const int64_t at = ((int64_t)row0 * a.h + head) * D, stride = (int64_t)a.h * D;
+    for (int e = tid; e < n * (D / 4); e += THREADS) {
+        const int64_t o = at + e / (D / 4) * stride + e % (D / 4) * 4;
+        if (a.out_f32) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + o) = f32x4{0.f, 0.f, 0.f, 0.f};
+        else *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.out) + o) = u32x2{0u, 0u};
+    }
+}
+
 // One workgroup's tile: query rows qt * 64 * QT .. of (sequence b, head), all the keys they can see.
 // GUARD (nvh_prefill_varlen_pv16): `a.v` is the fp16 copy of V; the range flags of this sequence's rows are fetched FIRST, the first K image's DMA is
 // issued behind them, and only then are they looked at — so the check costs no memory latency of its own.  Returns false (nothing but that K image
@@ -192,11 +203,19 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
     const int k_beg = a.cu_k[b], k_end = a.cu_k[b + 1];
     const int sq = q_end - q_beg, sk = k_end - k_beg;
     const int q0 = qt * BM;
-    if (q0 >= sq || sk <= 0) return true;
+    if (q0 >= sq) return true;
     const int kh = head / (a.h / a.kvh);
     const int shift = sk - sq;                       // bottom-right alignment: query r sees keys <= r + shift
 
     const int tid = threadIdx.x;
+    // keys any row of this workgroup can see: 0 .. min(sk, q0 + BM + shift) - 1
+    int kv_end = q0 + BM + shift;
+    if (kv_end > sk) kv_end = sk;
+    if (kv_end <= 0) {                               // none (more queries than keys): zeros, and no tile to stage
+        zero_rows<D, 256 * KS>(a, q_beg + q0, sq - q0 < BM ? sq - q0 : BM, head, tid);
+        return true;
+    }
+    const int n_tiles = (kv_end + BN - 1) / BN;      // one at least
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;              // ... of its group
     const int grp = KS > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
@@ -214,10 +233,6 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         for (int t = 0; t < DT; ++t) o[qs][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    // keys any row of this workgroup can see: 0 .. min(sk, q0 + BM + shift) - 1
-    int kv_end = q0 + BM + shift;
-    if (kv_end > sk) kv_end = sk;
-    const int n_tiles = (kv_end + BN - 1) / BN;
     const int wave_first_key = q0 + wave * WR + shift;            // last key the wave's FIRST row may see
     const int wave_last_key = wave_first_key + WR - 1;            // last key ANY row of this wave may see
 
@@ -627,7 +642,7 @@ void prefill_short_kernel(const PrefillArgs a) {
     const int q_beg = a.cu_q[b], q_end = a.cu_q[b + 1];
     const int k_beg = a.cu_k[b], k_end = a.cu_k[b + 1];
     const int sq = q_end - q_beg, sk = k_end - k_beg;
-    if (sq <= 0 || sk <= 0) return;                  // whole workgroup, before the barrier
+    if (sq <= 0) return;                             // whole workgroup, before the barrier
     const int G = a.h / a.kvh;
     const int shift = sk - sq;                       // bottom-right alignment: query r sees keys <= r + shift
     const int tid = threadIdx.x;

@@ -1099,3 +1099,36 @@ def test_prefill_step_is_store_then_attend(ops, h, kvh, d, lens, pv):
     want = ops.flash_attn_varlen_func(q, k, v, **how)
     got = ops.prefill_step(q, k, v, *got_kv, slots, **how)
     assert torch.equal(got, want) and torch.equal(got_kv, want_kv) and not torch.equal(got_kv, start)
+
+
+@pytest.mark.parametrize("form", ["exact", "fp16", "pages"])
+@pytest.mark.parametrize("h,kvh,d,new,keys", [(2, 1, 64, (200, 1, 65), (64, 3, 1)), (2, 2, 128, (130, 1024, 70), (2, 512, 0)), (14, 2, 64, (2000, 40, 300), (1000, 1100, 13)),
+                                              (48, 2, 64, (2113, 2050), (65, 2050)), (48, 2, 128, (700, 577), (300, 513)), (2, 64, 64, (100, 70, 90), (20, 0, 128))])
+def test_prefill_more_queries_than_keys(ops, h, kvh, d, new, keys, form):
+    """Rows in front of the first one that sees a key are zeros, and nothing in front of a sequence's keys counts: NaN stands there, within the same allocation.  One and two
+    groups of waves, 64 and 128 rows, keys that stay in LDS (the bound on those with keys: as where rows are chosen by fill)."""
+    h = max(h, kvh)
+    gen, paged, front = torch.Generator().manual_seed(sum(new)), form == "pages", 2048
+    q = torch.randn(sum(new), h, d, generator=gen).bfloat16().cuda()
+    width = -(-max(keys) // 256)
+    tables = (torch.randperm(len(new) * width, generator=gen) + front // 256).view(len(new), width).int().cuda()
+    k, v = (torch.randn(*((front // 256 + len(new) * width, 256) if paged else (front + sum(keys),)), kvh, d, generator=gen).bfloat16().cuda() for _ in range(2))
+    for t in (k, v):
+        t[:front // 256 if paged else front] = float("nan")
+    packed = [t if paged else t[front:] for t in (k, v)]
+
+    def cu(lengths):
+        return torch.tensor([sum(lengths[:i]) for i in range(len(lengths) + 1)], dtype=torch.int32).cuda()
+    got = ops.flash_attn_varlen_func(q, *packed, max_seqlen_q=max(new), cu_seqlens_q=cu(new), max_seqlen_k=max(keys), cu_seqlens_k=cu(keys), softmax_scale=d ** -0.5,
+                                     block_table=tables if paged else None, pv_fp16=None if paged else form == "fp16")
+    for i, (n, m) in enumerate(zip(new, keys)):
+        at, blind = sum(new[:i]), max(n - m, 0)
+        assert (got[at:at + blind] == 0).all(), i
+        if m == 0:
+            continue
+        ks, vs = ((t[tables[i].long()].flatten(0, 1)[:m] if paged else t[sum(keys[:i]):sum(keys[:i]) + m]).double() for t in packed)
+        seen = torch.arange(m, device="cuda")[None] <= torch.arange(blind, n, device="cuda")[:, None] + (m - n)
+        for j in range(h):
+            p = (q[at + blind:at + n, j].double() @ ks[:, j * kvh // h].T * d ** -0.5).masked_fill(~seen, float("-inf")).softmax(dim=-1)
+            want, spread = p @ vs[:, j * kvh // h], p @ vs[:, j * kvh // h].abs()
+            assert ((got[at + blind:at + n, j].double() - want).abs() <= want.abs() * 2 ** -8 + spread * 2 ** -10 + 1e-5).all(), (i, j)

@@ -1,5 +1,7 @@
 """GPU: the recurrent and latent-attention layer ops, one mechanism at a time, against plain equations on the CPU (oracle/zobasun_ref.py, float64):
 bf16 on the MFMA kernels, bf16 and fp32 on the plain ones.  Inputs are given in the compared type, so fp32 results are held to fp32 rounding."""
+import contextlib
+
 import pytest
 import torch
 
@@ -159,15 +161,29 @@ class Recurrence:
             for j, (_, _, y, _) in enumerate(portions):
                 table += recurrence_chunks(row, y.shape[0], j, segment)
                 row += y.shape[0]
-            out = ops.rglru_chunks(yx, self.params, pos, slots, torch.tensor(table, dtype=torch.int32, device="cuda"), segment, any(k for *_, k in table),
-                                   self.state, self.conv_state, generic=generic)
+            with taking(generic) as form:
+                out = ops.rglru_chunks(yx, self.params, pos, slots, torch.tensor(table, dtype=torch.int32, device="cuda"), segment, any(k for *_, k in table),
+                                       self.state, self.conv_state, generic=form)
         out = self.unspread(out.cpu())
         return out.split([y.shape[0] for _, _, y, _ in portions])
 
 
 SHAPES = [(1, 32, 64, 1), (3, 44, 64, 4), (2, 96, 96, 2), (4, 256, 256, 4), (1, 640, 640, 5), (5, 13, 64, 7), (2, 160, 160, 9), (2, 224, 224, 12)]
 FORMS = [(torch.bfloat16, False), (torch.bfloat16, True), (torch.float32, False)]
-WALKS = [(torch.bfloat16, 0), (torch.bfloat16, 1), (torch.bfloat16, 2), (torch.float32, 0)]      # fastest, plain, MFMA without LDS-DMA
+WALKS = [(torch.bfloat16, 0), (torch.bfloat16, 1), (torch.bfloat16, 2), (torch.bfloat16, 3), (torch.float32, 0)]      # fastest, plain, MFMA without LDS-DMA, walks
+
+
+@contextlib.contextmanager
+def taking(form):
+    """What ops.rglru_chunks takes as `generic`; 3: the fastest form of a caller that brings no scratch for steps, which is a walk of each segment."""
+    from nanovllm_hip import _lib
+    lib = _lib.load()
+    link_bytes = lib.nvh_rglru_link_bytes
+    lib.nvh_rglru_link_bytes = (lambda *sizes: 0) if form == 3 else link_bytes
+    try:
+        yield 0 if form == 3 else form
+    finally:
+        lib.nvh_rglru_link_bytes = link_bytes
 
 
 @pytest.mark.parametrize("segment", [64, 128, 4096])
@@ -186,23 +202,25 @@ def test_recurrence_portions(blocks, size, block, taps, dtype, generic, segment)
     close(r.unspread(r.state[[2, 0]].cpu()), torch.stack([la, lb]), torch.float32, 40 if dtype == torch.bfloat16 else 3)
 
 
+@pytest.mark.parametrize("form", [0, 3])
 @pytest.mark.parametrize("segment", [64, 4096])
-@pytest.mark.parametrize("blocks,block,taps", [(2, 32, 4), (2, 96, 4), (2, 128, 4), (2, 192, 3), (1, 256, 9)])
-def test_recurrence_row_edges(blocks, block, taps, segment):
+@pytest.mark.parametrize("blocks,block,taps", [(2, 32, 4), (2, 64, 4), (2, 96, 4), (2, 128, 4), (2, 160, 4), (2, 192, 3), (2, 224, 4), (1, 256, 9)])
+def test_recurrence_row_edges(blocks, block, taps, segment, form):
     """Portions that end on, in front of and behind 16 and 64 tokens, then their last tokens from the state."""
     r = Recurrence(blocks, block, block, taps, torch.bfloat16, slots=8)
     lengths = [15, 16, 17, 48, 63, 64, 65, 129]
     data = [r.yx(n, i) for i, n in enumerate(lengths)]
     want = [r.plain(y, x) for y, x in data]
     for cut in (slice(0, -3), slice(-3, None)):
-        got = r.run([(i, range(n)[cut][0], y[cut], x[cut]) for i, (n, (y, x)) in enumerate(zip(lengths, data))], segment=segment)
+        got = r.run([(i, range(n)[cut][0], y[cut], x[cut]) for i, (n, (y, x)) in enumerate(zip(lengths, data))], form, segment=segment)
         for g, (w, _) in zip(got, want):
             close(g, w[cut], torch.bfloat16)
     close(r.unspread(r.state.cpu()), torch.stack([s for _, s in want]), torch.float32, 40)
 
 
+@pytest.mark.parametrize("walks", [False, True])
 @pytest.mark.parametrize("stride", [(1 << 24) - 8, 34_100_000])
-def test_recurrence_rows_far_apart(stride):
+def test_recurrence_rows_far_apart(stride, walks):
     """Rows as far apart as 32-bit offsets are used for, and too far for them (the 64th one starts more than 4 GiB behind the first): the same bits as of rows side
     by side in the form that takes them, whole and in segments."""
     from nanovllm_hip import ops
@@ -216,8 +234,9 @@ def test_recurrence_rows_far_apart(stride):
         far[:, 2 * r.cols:] = 7.0
         table, pools = torch.tensor(chunks, dtype=torch.int32, device="cuda"), [(r.state.clone(), r.conv_state.clone()) for _ in range(2)]
         how = r.params, pos, slot, table, 64 * (3 - len(chunks)) + 64, len(chunks) > 1
-        want = ops.rglru_chunks(near, *how, *pools[0], generic=form)
-        ops.rglru_chunks(far[:, :2 * r.cols], *how, *pools[1], out=far[:, 2 * r.cols:3 * r.cols])
+        with taking(3 if walks else 0):
+            want = ops.rglru_chunks(near, *how, *pools[0], generic=form)
+            ops.rglru_chunks(far[:, :2 * r.cols], *how, *pools[1], out=far[:, 2 * r.cols:3 * r.cols])
         assert torch.equal(far[:, 2 * r.cols:3 * r.cols], want) and all(torch.equal(a, b) for a, b in zip(*pools))
         assert (far[:, 3 * r.cols:] == 7).all() and torch.equal(far[:, :2 * r.cols], near)
 
@@ -234,7 +253,8 @@ def test_recurrence_segments_without_rows(blocks, block, dtype, generic):
 
     def run(chunks):
         pools = r.state.clone(), r.conv_state.clone()
-        return ops.rglru_chunks(yx, r.params, pos, slots, torch.tensor(chunks, dtype=torch.int32, device="cuda"), 64, any(c[3] for c in chunks), *pools, generic=generic), *pools
+        with taking(generic) as form:
+            return ops.rglru_chunks(yx, r.params, pos, slots, torch.tensor(chunks, dtype=torch.int32, device="cuda"), 64, any(c[3] for c in chunks), *pools, generic=form), *pools
     a, b = [(0, 64, 0, 0), (64, 64, 0, 1)], [(128, 64, 1, 0), (192, 1, 1, 1)]
     want, state, ring = run(a + b)
     for chunks, same in (([*a, (128, 0, 2, 0), *b, (193, 0, 3, 0)], True), ([*a, (128, 0, 0, 2), *b], False)):
@@ -243,15 +263,17 @@ def test_recurrence_segments_without_rows(blocks, block, dtype, generic):
         assert torch.equal(after, state) if same else (after - state).abs().max() < 1e-4 * state.abs().max()
 
 
-def test_recurrence_many_segments():
+@pytest.mark.parametrize("walks", [False, True])
+def test_recurrence_many_segments(walks):
     """More segments than one dimension of a grid holds."""
     from nanovllm_hip import ops
     n = 65541
     r = Recurrence(2, 32, 32, 4, torch.bfloat16, slots=1)
     yx = r.rows(*r.yx(7, 1)).repeat(n // 7 + 1, 1)[:n].contiguous()
     table = torch.tensor([(i, 1, i, 0) for i in range(n)], dtype=torch.int32, device="cuda")
-    out = ops.rglru_chunks(yx, r.params, torch.zeros(n, dtype=torch.int64, device="cuda"), torch.full((n,), -1, dtype=torch.int32, device="cuda"), table, 64, False, r.state, r.conv_state)
-    few = ops.rglru_chunks(yx[:7], r.params, torch.zeros(7, dtype=torch.int64, device="cuda"), torch.full((7,), -1, dtype=torch.int32, device="cuda"), table[:7], 64, False, r.state, r.conv_state)
+    with taking(3 if walks else 0):
+        out = ops.rglru_chunks(yx, r.params, torch.zeros(n, dtype=torch.int64, device="cuda"), torch.full((n,), -1, dtype=torch.int32, device="cuda"), table, 64, False, r.state, r.conv_state)
+        few = ops.rglru_chunks(yx[:7], r.params, torch.zeros(7, dtype=torch.int64, device="cuda"), torch.full((7,), -1, dtype=torch.int32, device="cuda"), table[:7], 64, False, r.state, r.conv_state)
     assert torch.equal(out, few.repeat(n // 7 + 1, 1)[:n]) and few.any(dim=1).all()
 
 
@@ -303,7 +325,7 @@ def test_recurrence_steps_by_any_workgroup(blocks, block, taps, lengths):
             assert torch.equal(again, first_run[0]) and torch.equal(after[0], first_run[1])
 
 
-@pytest.mark.parametrize("form", [0, 2])
+@pytest.mark.parametrize("form", [0, 2, 3])
 @pytest.mark.parametrize("blocks,block", [(2, 32), (3, 256)])
 def test_recurrence_infinity_stays_in_its_channel(blocks, block, form):
     """Rows go out in the place of the gate's rows, which the waves of neighbouring channels read as multiplied by zero: many portions, each from an infinite state of one channel."""
@@ -316,7 +338,8 @@ def test_recurrence_infinity_stays_in_its_channel(blocks, block, form):
     yx, chunks = r.rows(*r.yx(n * m, 1)), [c for i in range(n) for c in recurrence_chunks(i * m, m, i, 64)]
     pos, slots, table = (torch.arange(n * m) % m + 1).cuda(), torch.arange(n, dtype=torch.int32, device="cuda"), torch.tensor(chunks, dtype=torch.int32, device="cuda")
     for _ in range(6):
-        out = ops.rglru_chunks(yx, r.params, pos, slots, table, 64, True, r.state.clone(), r.conv_state.clone(), generic=form)
+        with taking(form) as generic:
+            out = ops.rglru_chunks(yx, r.params, pos, slots, table, 64, True, r.state.clone(), r.conv_state.clone(), generic=generic)
         assert (~torch.isfinite(out)).any(dim=0).nonzero().flatten().tolist() == [5]
 
 

@@ -250,8 +250,8 @@ __global__ __launch_bounds__(1024) void rglru_walk_kernel(const RglruArgs a) {
 
 // ------------------------------------------------------------------------------------------------ prompt portions, blocks of up to 256 channels
 // The same walk with everything in flight early: x and y of the next 64 tokens travel by LDS-DMA under this step's arithmetic, both gates' weights of a wave's
-// 16 channels stay in registers for the whole segment, and u and y come into the accumulator layout through an MFMA with a 0/1 selection matrix (exact)
-// instead of single-element LDS reads.
+// 16 channels stay in registers for the whole segment, and u and y come into the accumulator layout by single elements (through an MFMA with a 0/1 selection matrix
+// a gate without a number took its 15 neighbours' with it).
 // Eight transcendentals and about 25 vector instructions per (token, channel) bound it (the vector units issue three quarters of the time at a block of 256), so
 // a block has a wave for every 16 channels, four on each SIMD at 256: 128 registers a lane, addresses computed again (fresh) instead of held.  Rows are
 // reached by 32-bit offsets from a step's first one; the 16-token passes are unrolled and find everything at fixed distances.  One barrier behind the scan frees u and
@@ -333,15 +333,8 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs
 
     // ---- this wave's 16 channels
     const int cb = 16 * wave + lq, ch = c0 + cb;
-    bf16x8 wr[KS], wi[KS], sel;
+    bf16x8 wr[KS], wi[KS];
     {
-        u32x4 one;                                   // 1.0 where this lane's k-slot is its own channel (tile `wave` is one half of a k-step)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int want = 16 * (wave & 1) + lq - 8 * lg - 2 * k;
-            one[k] = want == 0 ? 0x3F80u : (want == 1 ? 0x3F800000u : 0u);
-        }
-        sel = __builtin_bit_cast(bf16x8, one);
         const uint16_t* pr = reinterpret_cast<const uint16_t*>(a.ra) + (int64_t)ch * BLOCK + 8 * lg;
         const uint16_t* pi = reinterpret_cast<const uint16_t*>(a.ri) + (int64_t)ch * BLOCK + 8 * lg;
 #pragma unroll
@@ -411,8 +404,7 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs
         }
         const int ln = fresh(lane), lq = ln & 15, lg = ln >> 4, piece = 2 * wave + (lq >> 3);
         const auto at = [](int row, int p) { const int s = row * OCT + p; return s / 64 * YDMA + s % 64 * 8; };
-        const uint16_t* u_row = u_lds + lq * LD + 8 * lg;
-        const uint16_t* y_row = y_now + at(lq, (2 * wave + (lg & 1)) ^ (lq & 1));        // (its own channels' pieces, twice: the other half's are on their way out)
+        const uint16_t *u_row = u_lds + lq * LD + 8 * lg, *u_own = u_lds + 4 * lg * LD + cb;
         uint16_t* y_even = y_now + at(4 * lg, piece) + (lq & 7);               // this lane's channel in rows 4 lg and, by fixed distances, 4 lg + 2
         uint16_t* y_odd = y_now + at(4 * lg, piece ^ 1) + (lq & 7);            // ... and, likewise, in 4 lg + 1 and 4 lg + 3
 #pragma unroll
@@ -426,10 +418,15 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs
                 gr = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua, wr[k], gr, 0, 0, 0);
                 gi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua, wi[k], gi, 0, 0, 0);
             }
-            const f32x4 uu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(u_row + tm * LD + 32 * (wave >> 1)), sel, zero, 0, 0, 0);
-            f32x4 yv = zero;
-            if (!SUMMARY) yv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(y_row + tm / 16 * KS * YDMA), sel, zero, 0, 0, 0);
-            float av[4], sv[4];
+            float uu[4], yv[4], av[4], sv[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) uu[i] = act_ld(u_own + (tm + i) * LD);
+            if (!SUMMARY)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int off = tm / 16 * KS * YDMA + (KS == 8 ? i / 2 * YDMA : i / 2 * 2 * BLOCK);
+                    yv[i] = act_ld(i & 1 ? y_odd + off + BLOCK : y_even + off);
+                }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float rg = fast_rcp(1.f + fast_exp2(gr[i] * -kLog2e + rb)), ig = fast_rcp(1.f + fast_exp2(gi[i] * -kLog2e + ib));
@@ -497,8 +494,7 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs
 // state behind it, and from there the published pairs one by one (always this order of sums, whoever was first).
 // A drawn step waits for steps drawn before it only, and those are in the hands of workgroups that run: no assumption on how many are resident or on their order.  The
 // wait is bounded all the same (a state of NaN behind it).
-// x travels by LDS-DMA under a step's products, y a step ahead; u and y come into the accumulator layout through an MFMA with a 0/1 selection matrix (exact) instead
-// of single-element LDS reads.  Rows lie so that a lane of the accumulators holds 16 consecutive tokens of a channel: one composition across lanes a step, not four.
+// x travels by LDS-DMA under a step's products, y a step ahead; u and y come into the accumulator layout by single elements.  Rows lie so that a lane of the accumulators holds 16 consecutive tokens of a channel: one composition across lanes a step, not four.
 // Both gates' products of all 64 tokens come first and decays and inputs take their place: 64 registers of weights and 32 of these leave room for rows asked for ahead.
 // 128 registers a lane (four waves on each SIMD at 256 channels): addresses are computed again (fresh) instead of held.
 // Bound by the issue of vector instructions (about 60 and 8 transcendentals per element, 80 % of the time) on 250 of 256 CUs; a step takes 11 us whoever takes it, of which the state
@@ -718,15 +714,6 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_chain_kernel(const RglruArg
         for (int i = 0; i < 8; ++i) *reinterpret_cast<uint32_t*>(u_lds + (4 * (t & 8) + t / 16 * 4 + 16 * (i / 4) + i % 4) * LD + o) = pack_bf16x2(acc[i][0], acc[i][1]);
     };
 
-    auto selection = [&](int ln) __attribute__((always_inline)) {              // 1.0 where this lane's k-slot is its own channel (tile `wave` is one half of a k-step)
-        u32x4 one;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int want = 16 * (wave & 1) + (ln & 15) - 8 * (ln >> 4) - 2 * k;
-            one[k] = want == 0 ? 0x3F80u : (want == 1 ? 0x3F800000u : 0u);
-        }
-        return __builtin_bit_cast(bf16x8, one);
-    };
     if (wave == 0) {
         const int first = draw();
         note(first, look_up(first), 0);
@@ -895,28 +882,32 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_chain_kernel(const RglruArg
         }
         {
             const int ln = lane_now(), lq = ln & 15, lg = ln >> 4, piece = 2 * wave + (lq >> 3);
-            // This wave's pieces, twice.  (The other half's, which the selection multiplies by zero, its wave replaces by what goes out, and zero times an infinity is none.)
-            const uint16_t* y_row = y_now + place(lq, (2 * wave + (lg & 1)) ^ (lq & 1));
             uint16_t* y_even = y_now + place(4 * lg, piece) + (lq & 7);        // this lane's channel in rows 4 lg and, by fixed distances, 4 lg + 2
             uint16_t* y_odd = y_now + place(4 * lg, piece ^ 1) + (lq & 7);     // ... and, likewise, in 4 lg + 1 and 4 lg + 3
-            const bf16x8 sel = selection(ln);
+            const auto off = [](int m, int i) { return m * KS * YDMA + (KS == 8 ? i / 2 * YDMA : i / 2 * 2 * BLOCK); };
             const float before = ba * h + bs;
+            float yv[4], yn[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) yv[i] = act_ld(i & 1 ? y_odd + off(0, i) + BLOCK : y_even + off(0, i));
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
-                const f32x4 yv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(y_row + m * KS * YDMA), sel, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                if (m < 3)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) yn[i] = act_ld(i & 1 ? y_odd + off(m + 1, i) + BLOCK : y_even + off(m + 1, i));
 #pragma unroll
                 for (int i = 0; i < 4; i += 2) {
                     const uint32_t two = pack_bf16x2((av[m][i] * before + sv[m][i]) * fast_gelu(yv[i]), (av[m][i + 1] * before + sv[m][i + 1]) * fast_gelu(yv[i + 1]));
-                    const int off = m * KS * YDMA + (KS == 8 ? i / 2 * YDMA : i * BLOCK);
-                    y_even[off] = (uint16_t)two;
-                    y_odd[off + BLOCK] = (uint16_t)(two >> 16);
+                    y_even[off(m, i)] = (uint16_t)two;
+                    y_odd[off(m, i) + BLOCK] = (uint16_t)(two >> 16);
                 }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) yv[i] = yn[i];
             }
         }
         if (now.last) {
             const int slot = now.slot, ln = lane_now();
             if (slot >= 0) {
-                                if (ln < 16) a.state[(int64_t)slot * a.width + c0 + 16 * wave + ln] = ca * h + cs;
+                if (ln < 16) a.state[(int64_t)slot * a.width + c0 + 16 * wave + ln] = ca * h + cs;
                 const int portion = now.off + now.cnt, keep = portion < a.taps ? portion : a.taps;
                 for (int e = fresh(tid); e < keep * OCT; e += THREADS) {       // (its first step, which has read the ring, has published)
                     const int row = now.row + now.cnt - 1 - e / OCT, c = c0 + e % OCT * 8;

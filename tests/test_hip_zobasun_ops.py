@@ -343,6 +343,35 @@ def test_recurrence_infinity_stays_in_its_channel(blocks, block, form):
         assert (~torch.isfinite(out)).any(dim=0).nonzero().flatten().tolist() == [5]
 
 
+@pytest.mark.parametrize("form", [0, 2, 3])
+@pytest.mark.parametrize("blocks,block", [(2, 32), (2, 96), (3, 256)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_recurrence_inputs_without_a_number_stay_in_their_channel(blocks, block, form, value):
+    """An infinite or missing gate value reaches its own output (none: -inf times nothing is no number) and no other channel's, an infinite input what the plain kernel's reaches (both gates of its whole block saturate)."""
+    from nanovllm_hip import ops
+    from nanovllm_hip.engine.model_runner import recurrence_chunks
+    r, n = Recurrence(blocks, block, block, 4, torch.bfloat16, slots=1), 150
+    r.state.normal_(), r.conv_state.normal_()
+    slot, pos = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.arange(3, 3 + n).cuda()
+    chunks = torch.tensor(recurrence_chunks(0, n, 0, 64), dtype=torch.int32, device="cuda")
+
+    def run(yx, form):
+        with taking(form) as generic:
+            return ops.rglru_chunks(yx, r.params, pos, slot, chunks, 64, True, r.state.clone(), r.conv_state.clone(), generic=generic)
+    yx, gates = r.rows(*r.yx(n, 1)), [(0, 7), (21, 8), (40, r.cols - 1), (63, 0), (64, 15), (149, 16)]
+    want = run(yx, form)
+    for t, c in gates:
+        yx[t, c] = value
+    got, one = run(yx, form), torch.zeros_like(want, dtype=torch.bool)
+    for t, c in gates:
+        one[t, c] = True
+    assert torch.equal(got[~one], want[~one]) and not torch.isfinite(got[one]).any()
+    if value == float("inf"):
+        yx = r.rows(*r.yx(n, 1))
+        yx[70, r.cols + 9] = value
+        assert torch.equal(torch.isfinite(run(yx, form)), torch.isfinite(run(yx, 1)))
+
+
 @pytest.mark.parametrize("blocks,size,block,taps", SHAPES)
 def test_recurrence_step_follows_portions(blocks, size, block, taps):
     """Prompt by the chunked form, then single tokens by the step form (one sequence steps from its very first token)."""

@@ -273,7 +273,7 @@ __device__ __forceinline__ float row_sums(float (&p)[16], int lane) {
         "v_add_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0x5\n v_add_f32_dpp %2, %6, %6 row_half_mirror row_mask:0xf bank_mask:0xa\n"
         "v_add_f32_dpp %3, %3, %3 row_half_mirror row_mask:0xf bank_mask:0x5\n v_add_f32_dpp %3, %7, %7 row_half_mirror row_mask:0xf bank_mask:0xa\n"
         "s_nop 1"
-        : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7])
+        : "+&v"(p[0]), "+&v"(p[1]), "+&v"(p[2]), "+&v"(p[3]), "+&v"(p[4]), "+&v"(p[5]), "+&v"(p[6]), "+&v"(p[7])        // (written while the others are still to be read)
         : "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
     const bool b1 = lane & 1, b2 = lane & 2;
     float u[2];

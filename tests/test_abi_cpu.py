@@ -114,6 +114,23 @@ def test_experts_in_one_call_refuse_scratch_that_is_too_small(lib):
     assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == 0
 
 
+def test_asm_of_several_instructions_shares_no_register():
+    """An output that is written while inputs are still to be read must not share a register with one: the compiler may give equal values the same unless it is told (&)."""
+    seen = 0
+    for root, _, names in os.walk(os.path.join(ROOT, "nano-vllm-learn_amd", "csrc")):
+        for name in names:
+            text = re.sub(r"//.*", "", open(os.path.join(root, name)).read())
+            for body in re.findall(r"\basm(?: volatile)?\s*\((.*?)\)\s*;", text, re.S):
+                strings = []
+                marked = re.sub(r'"((?:[^"\\]|\\.)*)"', lambda m: strings.append(m[1]) or f"#{len(strings) - 1} ", body)
+                code, outputs, inputs = ([strings[int(i)] for i in re.findall(r"#(\d+)", part)] for part in (marked.split(":") + ["", ""])[:3])
+                lines = [i for i in re.split(r"\\n|\\t|;", "".join(code)) if i.strip()]
+                if len(lines) > 1 and any(re.search("[vsa]", i) for i in inputs):
+                    seen += 1
+                    assert all("&" in o for o in outputs), f"{name}: {lines[0]}"
+    assert seen >= 3
+
+
 def test_ops_refuse_cpu_tensors():
     """No CPU fallback: the product path must fail loudly off-GPU."""
     from nanovllm_hip import ops

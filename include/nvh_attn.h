@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 207          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts */
+#define NVH_VERSION 208          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -509,10 +509,13 @@ typedef struct nvh_rglru_desc {
     int64_t out_stride;
     void* out_packed;            /* nullable (bf16, step form): the result in MFMA-fragment order */
     void* links;                 /* nullable (chunks form): scratch of nvh_rglru_link_bytes(); what it holds does not matter */
-    int32_t max_steps;           /* steps of nvh_rglru_chunk_tokens() that `links` has room for: at least those of all segments (n_chunks + rows / 64 are always enough) */
+    int32_t max_steps;           /* steps of nvh_rglru_chunk_tokens() that `links` has room for: n_chunks + rows / 64, or the segments are walked without it */
+    int32_t rows;                /* rows of all segments together */
+    int64_t links_bytes;         /* at least nvh_rglru_link_bytes() of max_steps */
 } nvh_rglru_desc;
 int nvh_rglru_chunk_tokens(void);
-/* Bytes of `links` for these sizes; 0: the form that needs them does not take this block, these taps or this type (s_loc and a_cum do then). */
+/* Bytes of `links` for these sizes; 0: the form that needs them does not take this block, these taps or this type (s_loc and a_cum do then).
+ * In that form a step waits for earlier ones that other workgroups have in hand; a wait that came to its limit of some seconds would leave NaN in output and state. */
 int64_t nvh_rglru_link_bytes(int block, int blocks, int taps, int max_steps, int dtype);
 int nvh_rglru_chunks(const nvh_rglru_desc* d, int generic, int dtype, void* stream);
 int nvh_rglru_step(const nvh_rglru_desc* d, int rows, int dtype, void* stream);

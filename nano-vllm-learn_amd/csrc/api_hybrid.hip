@@ -38,6 +38,9 @@ int nvh_rglru_chunks(const nvh_rglru_desc* d, int generic, int dtype, void* stre
     if (rc) return rc;
     REQUIRE(d->chunks && d->s_loc && d->a_cum && d->out && d->n_chunks > 0, NVH_E_NULL, "rglru_chunks: null pointer");
     REQUIRE(!d->links || aligned16(d->links), NVH_E_ALIGN, "rglru_chunks: scratch must be 16-byte aligned");
+    REQUIRE(d->rows >= 0 && d->max_steps >= 0, NVH_E_SHAPE, "rglru_chunks: negative size");
+    const int64_t need = d->links ? nvh_rglru_link_bytes(d->block, d->blocks, d->taps, d->max_steps, dtype) : 0;
+    REQUIRE(d->links_bytes >= need || !d->links, NVH_E_WORKSPACE, "rglru_chunks: scratch %lld B < required %lld B", (long long)d->links_bytes, (long long)need);
     REQUIRE(d->segment > 0 && d->segment % kRglruChunk == 0, NVH_E_SHAPE, "rglru_chunks: segment %d must be a positive multiple of %d", d->segment, kRglruChunk);
     REQUIRE(!d->out_packed, NVH_E_SHAPE, "rglru_chunks: packed output belongs to the step form");
     REQUIRE(aligned16(d->s_loc) && aligned16(d->a_cum), NVH_E_ALIGN, "rglru_chunks: scratch must be 16-byte aligned");

@@ -1189,7 +1189,8 @@ void chain_ks(const RglruArgs& a, hipStream_t stream) {
     rglru_chain_kernel<KS><<<a.blocks * each, 128 * KS, lds, stream>>>(a);
 }
 bool chain(const RglruArgs& a, hipStream_t stream) {
-    if (!a.links || a.max_steps <= 0 || !near_rows(a) || !scan_takes(a.block, a.taps)) return false;
+    // (a segment of n rows is ceil(n / CH) steps; the device counts them, so there has to be room for as many as there can be)
+    if (!a.links || a.max_steps <= 0 || a.max_steps < a.n_chunks + (int64_t)a.rows / CH || !near_rows(a) || !scan_takes(a.block, a.taps)) return false;
     switch (a.block / 32) {
         case 1: chain_ks<1>(a, stream); break;
         case 2: chain_ks<2>(a, stream); break;

@@ -48,7 +48,7 @@ class RglruDesc(ctypes.Structure):
                 ("rate", ctypes.c_void_p), ("chunks", ctypes.c_void_p), ("n_chunks", ctypes.c_int32), ("segment", ctypes.c_int32), ("summaries", ctypes.c_int32), ("positions", ctypes.c_void_p),
                 ("state_slots", ctypes.c_void_p), ("state", ctypes.c_void_p), ("conv_state", ctypes.c_void_p), ("s_loc", ctypes.c_void_p),
                 ("a_cum", ctypes.c_void_p), ("out", ctypes.c_void_p), ("out_stride", ctypes.c_int64), ("out_packed", ctypes.c_void_p),
-                ("links", ctypes.c_void_p), ("max_steps", ctypes.c_int32)]
+                ("links", ctypes.c_void_p), ("max_steps", ctypes.c_int32), ("rows", ctypes.c_int32), ("links_bytes", ctypes.c_int64)]
 
 
 class LatentPrepDesc(ctypes.Structure):

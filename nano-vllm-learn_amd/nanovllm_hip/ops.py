@@ -747,7 +747,7 @@ def rglru_chunks(yx, params, positions, state_slots, chunks, segment, summaries,
     lib = _lib.load()
     steps = chunks.shape[0] + rows // lib.nvh_rglru_chunk_tokens()
     links = torch.empty(lib.nvh_rglru_link_bytes(d.block, d.blocks, d.taps, steps, code), dtype=torch.uint8, device=yx.device)
-    d.links, d.max_steps = links.data_ptr() if links.numel() else None, steps
+    d.links, d.links_bytes, d.max_steps, d.rows = links.data_ptr() if links.numel() else None, links.numel(), steps, rows
     _lib.check(lib.nvh_rglru_chunks(ctypes.byref(d), int(generic), code, _stream()), "nvh_rglru_chunks")
     return out
 

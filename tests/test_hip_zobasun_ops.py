@@ -372,6 +372,30 @@ def test_recurrence_inputs_without_a_number_stay_in_their_channel(blocks, block,
         assert torch.equal(torch.isfinite(run(yx, form)), torch.isfinite(run(yx, 1)))
 
 
+@pytest.mark.parametrize("steps", [0, 1, 5, 6])
+def test_recurrence_with_room_for_fewer_steps(steps, monkeypatch):
+    """300 and 70 rows are 7 steps, and scratch for all that two segments of 370 rows can be has room for 7: with less, every row comes out all the same, walked."""
+    from nanovllm_hip import _lib, ops
+    r = Recurrence(2, 64, 64, 4, torch.bfloat16, slots=2)
+    yx, pos, slots = r.rows(*r.yx(370, 1)), torch.cat([torch.arange(300), torch.arange(70)]).cuda(), torch.tensor([1, 0], dtype=torch.int32, device="cuda")
+    chunks, lib = torch.tensor([(0, 300, 0, 0), (300, 70, 1, 0)], dtype=torch.int32, device="cuda"), _lib.load()
+
+    def run():
+        pools = torch.zeros_like(r.state), torch.zeros_like(r.conv_state)
+        out = torch.full((370, r.cols), float("nan"), dtype=torch.bfloat16, device="cuda")
+        return ops.rglru_chunks(yx, r.params, pos, slots, chunks, 320, False, *pools, out=out), *pools
+    with taking(3):
+        want = run()
+    call = lib.nvh_rglru_chunks
+
+    def fewer(d, *how):
+        d._obj.max_steps = steps
+        return call(d, *how)
+    monkeypatch.setattr(lib, "nvh_rglru_chunks", fewer)
+    for got, wanted in zip(run(), want):
+        assert torch.equal(got, wanted)
+
+
 @pytest.mark.parametrize("blocks,size,block,taps", SHAPES)
 def test_recurrence_step_follows_portions(blocks, size, block, taps):
     """Prompt by the chunked form, then single tokens by the step form (one sequence steps from its very first token)."""

@@ -314,3 +314,25 @@ def test_entry_points_refuse_bad_arguments():
     assert lib.nvh_latent_prefill_supported(192, 128) and not lib.nvh_latent_prefill_supported(320, 128)
     assert lib.nvh_latent_attend_mfma(512, 64, 64) and not lib.nvh_latent_attend_mfma(640, 64, 64) and not lib.nvh_latent_attend_mfma(512, 64, 32)
     assert config(8, 8, [recurrent(8, 1, 1), latent(1, 8, 8, 8, 8, 8, 1.0)])["layers"][1]["mixer"]["heads"] == 1
+
+
+def test_recurrence_refuses_scratch_that_is_too_small():
+    """Scratch for steps is a pure function of sizes; less of it than max_steps asks for is refused before anything is launched."""
+    import ctypes
+    from nanovllm_hip import _lib
+    lib, p, d = _lib.load(), 4096, _lib.RglruDesc()
+    for name, kind in d._fields_:
+        if kind is ctypes.c_void_p:
+            setattr(d, name, p)
+    d.out_packed, d.width, d.block, d.blocks, d.taps, d.yx_stride, d.out_stride = None, 64, 64, 1, 4, 128, 64
+    d.n_chunks, d.segment, d.rows, d.max_steps = 2, 64, 300, 6
+    need = lib.nvh_rglru_link_bytes(64, 1, 4, 6, 0)
+    assert need == 4 * (64 + 8 * 6) + 12 * 64 * 6 and lib.nvh_rglru_link_bytes(64, 1, 4, 6, 1) == 0 and lib.nvh_rglru_link_bytes(64, 1, 12, 6, 0) == 0
+    for have in (0, need - 1):
+        d.links_bytes = have
+        assert lib.nvh_rglru_chunks(ctypes.byref(d), 0, 0, None) == -4 and b"scratch" in lib.nvh_last_error()
+    for name in ("rows", "max_steps"):
+        before = getattr(d, name)
+        setattr(d, name, -1)
+        assert lib.nvh_rglru_chunks(ctypes.byref(d), 0, 0, None) == -2
+        setattr(d, name, before)

@@ -278,3 +278,20 @@ def test_every_model_has_its_sources():
     names = sorted(f for f in os.listdir(build.CSRC) if f.endswith(".hip"))
     assert sorted(build.SOURCES) == names and len(set(build.SOURCES)) == len(build.SOURCES)
     assert all(os.path.exists(os.path.join(build.CSRC, h)) for h in build.HEADERS)
+
+
+def test_experts_take_weights_however_they_are_held(monkeypatch):
+    """Buffers, and parameters or plain attributes in the place of one (a module that was wrapped or shares weights)."""
+    from nanovllm_hip import ops
+    from nanovllm_hip.layers.moe import MixtureOfExperts
+    m, gen = MixtureOfExperts(64, 64, 64, 3, 2, torch.float32), torch.Generator().manual_seed(0)
+    m.load(lambda n: torch.randn({"router": (3, 64), "correction": (3,)}.get(n, (64, 64)), generator=gen))
+    monkeypatch.setattr(ops, "moe_experts", lambda x, *weights: weights[:4])
+    names = ("router", "correction", "w_gate_up", "w_down")
+    held = [getattr(m, n) for n in names]
+    assert all(a is b for a, b in zip(m(None), held))
+    m.router = torch.nn.Parameter(held[0].clone())
+    del m.w_down
+    object.__setattr__(m, "w_down", held[3].clone())
+    m.correction = held[1] + 1
+    assert all(a is getattr(m, n) for a, n in zip(m(None), names)) and torch.equal(m(None)[1], held[1] + 1)

@@ -197,7 +197,7 @@ def _pv16_scratch(lib, batch, max_seqlen_q, max_seqlen_k, rows, kvh, hd, device)
     return scratch.data_ptr(), scratch.numel(), scratch
 
 
-def prefill_step(q, k, v, k_cache, v_cache, slot_mapping, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k, softmax_scale, pv_fp16=None):
+def prefill_step(q, k, v, k_cache, v_cache, slot_mapping, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k, softmax_scale=None, pv_fp16=None):
     """store_kvcache(k, v, ...) followed by flash_attn_varlen_func(q, k, v, ...) over the packed rows as one C-ABI call (the two calls at attention.py:84-86 and :93-96)."""
     (tq, h, hd), (n, kvh, _) = q.shape, k.shape
     batch, max_q, max_k, d = cu_seqlens_q.numel() - 1, int(max_seqlen_q), int(max_seqlen_k), kvh * hd
@@ -209,6 +209,8 @@ def prefill_step(q, k, v, k_cache, v_cache, slot_mapping, max_seqlen_q, cu_seqle
     assert slot_mapping.numel() == n and slot_mapping.is_contiguous() and cu_seqlens_k.numel() == batch + 1
     if pv_fp16 is None:
         pv_fp16 = _pv16_pays(hd, kvh, batch, max_q, max_k)
+    if softmax_scale is None:
+        softmax_scale = hd ** -0.5
     lib, out = _lib.load(), torch.empty((tq, h, hd), dtype=torch.bfloat16, device=q.device)
     sc_ptr, sc_bytes, _scratch = _pv16_scratch(lib, batch, max_q, max_k, n, kvh, hd, q.device) if pv_fp16 else (None, 0, None)
     rc = lib.nvh_prefill_step(out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), slot_mapping.data_ptr(),

@@ -1101,6 +1101,22 @@ def test_prefill_step_is_store_then_attend(ops, h, kvh, d, lens, pv):
     assert torch.equal(got, want) and torch.equal(got_kv, want_kv) and not torch.equal(got_kv, start)
 
 
+def test_attention_module_without_a_scale_stores_and_attends(ops):
+    """No softmax scale is head_dim ** -0.5, packed prompts with a cache included."""
+    from nanovllm_hip import reset_context, set_context
+    from nanovllm_hip.layers.attention_hip import Attention
+    gen = torch.Generator().manual_seed(4)
+    q, k, v = torch.randn(3, 70, 128, generator=gen).bfloat16().cuda().unbind()
+    cu, slots, outs = torch.tensor([0, 70], dtype=torch.int32).cuda(), torch.arange(70, dtype=torch.int32).cuda(), []
+    for scale in (None, 64 ** -0.5):
+        attn = Attention(2, 64, scale, 2)
+        attn.k_cache, attn.v_cache = torch.zeros(2, 1, 256, 2, 64, dtype=torch.bfloat16, device="cuda")
+        set_context(True, cu_seqlens_q=cu, cu_seqlens_k=cu, max_seqlen_q=70, max_seqlen_k=70, slot_mapping=slots)
+        outs += [attn(q, k, v), attn.k_cache, attn.v_cache]
+        reset_context()
+    assert all(torch.equal(a, b) for a, b in zip(outs[:3], outs[3:])) and outs[0].any()
+
+
 @pytest.mark.parametrize("form", ["exact", "fp16", "pages"])
 @pytest.mark.parametrize("h,kvh,d,new,keys", [(2, 1, 64, (200, 1, 65), (64, 3, 1)), (2, 2, 128, (130, 1024, 70), (2, 512, 0)), (14, 2, 64, (2000, 40, 300), (1000, 1100, 13)),
                                               (48, 2, 64, (2113, 2050), (65, 2050)), (48, 2, 128, (700, 577), (300, 513)), (2, 64, 64, (100, 70, 90), (20, 0, 128))])

@@ -92,9 +92,9 @@ def recurrence_chunks(first_row, rows, seq, segment):
     return [(first_row + k, min(segment, rows - k), seq, k // segment) for k in range(0, rows, segment)]
 
 
-def build_step_meta(portions, block_size, segment=64):
+def build_step_meta(portions, block_size, segment=64, whole=False):
     """Rows of a mixed batch.  portions: [(sequence, tokens)] — the sequence's next tokens behind its num_cached_tokens.  Sequences that bring one
-    token come first (`order` gives the places in `portions`); returns host tensors."""
+    token come first (`order` gives the places in `portions`); whole: if any is cut into segments, a second table (`whole`) has them uncut.  Returns host tensors."""
     _check_block_size([s for s, _ in portions], block_size)
     order = sorted(range(len(portions)), key=lambda i: portions[i][1] > 1)
     input_ids, positions, slots, row_seq, chunks = [], [], [], [], []
@@ -116,12 +116,13 @@ def build_step_meta(portions, block_size, segment=64):
             cu_k.append(cu_k[-1] + hi)
             max_q = max(max_q, n)
     seqs = [portions[i][0] for i in order]
+    cut = any(k for *_, k in chunks)
 
     def i32(v):
         return torch.tensor(v, dtype=torch.int32)
     return dict(order=order, input_ids=torch.tensor(input_ids, dtype=torch.int64), positions=torch.tensor(positions, dtype=torch.int64), num_decode=num_decode,
                 slot_mapping=i32(slots), block_tables=build_block_tables(seqs, pad=0), state_slots=i32([s.state_slot for s in seqs]), chunks=i32(chunks), segment=segment,
-                summaries=any(k for *_, k in chunks),
+                summaries=cut, whole=i32([(first, portions[i][1], j, 0) for j, (first, i) in enumerate(zip(cu_rows, order))]) if whole and cut else None,
                 row_seq=i32(row_seq), cu_rows=i32(cu_rows), cu_q=i32(cu_q), cu_k=i32(cu_k), max_q=max_q, total_k=cu_k[-1], max_context=max(positions) + 1)
 
 
@@ -196,7 +197,8 @@ class ModelRunner:
         """One batch of a model that takes mixed batches.  portions: [(sequence, tokens)]; want: per portion, the places among its tokens whose
         logits are asked for (default: the last).  Returns logits rows in the order of `portions` and `want` (None when nothing is wanted) and
         advances num_cached_tokens."""
-        m = build_step_meta(portions, self.block_size, self.model.recurrence_segment([n for _, n in portions if n > 1]))
+        lengths, scans_whole = [n for _, n in portions if n > 1], getattr(self.model, "scans_whole", None)
+        m = build_step_meta(portions, self.block_size, self.model.recurrence_segment(lengths), scans_whole is not None and scans_whole(lengths))
         assert int(m["positions"].max()) < self.max_model_len, "a sequence exceeds max_model_len"
         assert 0 <= int(m["input_ids"].min()) and int(m["input_ids"].max()) < self.cfg.vocab_size, "a token id is outside the vocabulary"
         first, row = {}, 0
@@ -208,7 +210,7 @@ class ModelRunner:
         assert all(0 <= p < portions[i][1] for i, places in enumerate(want) for p in places), "a wanted place is outside its portion"
         decode_only = m["num_decode"] == row
         step = StepMeta(m["num_decode"], self._dev(m["slot_mapping"]), self._dev(m["block_tables"]), self._dev(m["state_slots"]), self._dev(m["chunks"]),
-                        m["segment"], m["summaries"], m["max_context"], *([] if decode_only else [self._dev(m["row_seq"]), self._dev(m["cu_rows"]), self._dev(m["cu_q"]), self._dev(m["cu_k"]), m["max_q"], m["total_k"]]))
+                        m["segment"], m["summaries"], m["max_context"], *([] if decode_only else [self._dev(m["row_seq"]), self._dev(m["cu_rows"]), self._dev(m["cu_q"]), self._dev(m["cu_k"]), m["max_q"], m["total_k"], self._dev(m["whole"])]))
         hidden = self.model(self._dev(m["input_ids"]), self._dev(m["positions"]), step)
         for seq, n in portions:
             seq.num_cached_tokens += n

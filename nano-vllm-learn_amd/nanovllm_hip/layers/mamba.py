@@ -91,7 +91,8 @@ class SelectiveScan(nn.Module):
         if n:
             ops.scan_step(x[:n], low[:n], bc[:n], z[:n], self.params, positions[:n], step.state_slots, self.state, out=out[:n])
         if n < rows:
-            ops.scan_chunks(x, linear(low, self.w_dt), bc, z, self.params, positions, step.state_slots, step.chunks[n:], step.summaries, self.state, out=out)
+            chunks, cut = (step.chunks, step.summaries) if step.whole is None else (step.whole, False)
+            ops.scan_chunks(x, linear(low, self.w_dt), bc, z, self.params, positions, step.state_slots, chunks[n:], cut, self.state, out=out)
         return out
 
     def decode_scan(self, xz, rows, positions, step, bufs):

@@ -185,8 +185,13 @@ class ZaposunForCausalLM(nn.Module):
 
     def recurrence_segment(self, portions):
         """Tokens per recurrence segment for portions of these lengths (the layer with the fewest workgroups fills the GPU last)."""
-        units = [layer.mixer.segment_units for layer in self.layers]
+        units = [int(layer.mixer.segment_units) for layer in self.layers]
         return choose_segment(portions, min(units)) if units and portions else 64
+
+    def scans_whole(self, portions):
+        """Whether the scans take portions of these lengths whole, however time mixing cuts them."""
+        units = [layer.mixer.segment_units for layer in self.layers if isinstance(layer.mixer, ParallelMixer)]
+        return bool(units and portions) and all(hasattr(u, "whole") and u.whole(portions) for u in units)
 
     def compute_logits(self, x):
         """Logits [rows, vocab] (a view of padded rows) of residual-stream sums."""

@@ -21,3 +21,4 @@ class StepMeta:
     cu_k: torch.Tensor | None = None                # int32 [portions + 1] offsets of the keys the portions see
     max_q: int = 0
     total_k: int = 0
+    whole: torch.Tensor | None = None               # int32 [sequences, 4] what `chunks` cuts, uncut, where scans take it so (None: they take `chunks`)

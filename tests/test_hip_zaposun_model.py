@@ -81,6 +81,25 @@ def test_prompts_portions_and_decoding(folder, name, dtype):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("name", ["odd", "plain"])
+def test_scans_take_whole_what_time_mixing_cuts(folder, name, dtype, monkeypatch):
+    """Two tables of one batch: portions beside a single token, in segments for time mixing and whole for the scans."""
+    from nanovllm_hip import ops
+    from nanovllm_hip.models.zaposun import ZaposunForCausalLM
+    seen, scan = [], ops.scan_chunks
+    monkeypatch.setattr(ZaposunForCausalLM, "recurrence_segment", lambda self, portions: 64)
+    monkeypatch.setattr(ZaposunForCausalLM, "scans_whole", lambda self, portions: True)
+    monkeypatch.setattr(ops, "scan_chunks", lambda *a, **kw: seen.append(a[7:9]) or scan(*a, **kw))
+    eng, vocab = engine(folder, name, dtype), CONFIGS[name]["vocab"]
+    prompts = [tokens(n, vocab, 40 + i) for i, n in enumerate((1, 203, 70, 129))]
+    seqs = [eng.sequence(p) for p in prompts]
+    got = eng.feed([(s, len(s)) for s in seqs], [list(range(len(s))) for s in seqs])
+    assert seen and all(not cut and (table[:, 3] == 0).all() and table[-3:, 1].tolist() == [203, 70, 129] for table, cut in seen)
+    for p, rows in zip(prompts, got.split([len(p) for p in prompts])):
+        check(rows, plain(name, p), dtype)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("name", ["odd", "plain", "strong", "wide"])
 def test_mixed_batches_with_reuse(folder, name, dtype):
     """Unequal requests in one batch — portions beside single tokens, requests left out of steps — on pages and state slots that are handed on several times; every

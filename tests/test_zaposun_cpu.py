@@ -328,3 +328,31 @@ def test_scan_whole_portions():
         assert (choose_segment(portions, one) >= max(portions, default=0)) == whole
     long = [4096, *[200] * 39]
     assert one == other and choose_segment(long, one) == choose_segment(long, other) < 4096
+
+
+@pytest.mark.parametrize("heads,inner,order", [(16, 2048, ("wkv", "parallel")), (16, 2048, ("parallel", "wkv")), (32, 2048, ("wkv", "parallel")), (32, 2048, ("parallel",) * 2), (8, 2048, ("wkv",))])
+def test_segments_by_kind_of_layer(heads, inner, order):
+    """Scans that take few portions whole do so whatever the other layers' order and units are, and time mixing is cut as without them."""
+    from nanovllm_hip.engine.model_runner import build_step_meta
+    from nanovllm_hip.engine.sequence import Sequence
+    from nanovllm_hip.layers.rglru import choose_segment
+    from nanovllm_hip.models import build_model
+    from nanovllm_hip.models.zaposun import ZaposunConfig
+    mixers = {"wkv": dict(heads=heads, dim=64), "parallel": dict(left=dict(heads=1, kv_heads=1, dim=64, vdim=64, scale=0.1, rot=dict(base=100.0, dims=0), mask=dict(size=64)),
+                                                                 right=dict(inner=inner, state=16, dt_rank=16, conv=4))}
+    cfg = ZaposunConfig.from_json(dict(width=64, vocab=16, norm=dict(eps=1e-6, groups=1), streams=1, logit_scale=1.0, embedding=dict(bigram=dict(buckets=3, mul_prev=1, mul_cur=1)),
+                                       layers=[dict(type=t, mixer=mixers[t], mlp=None) for t in order]))
+    model, units = build_model(cfg), [{"wkv": heads // 2, "parallel": inner // 256}[t] for t in order]
+    few, many = [3277] * 5, [300] * 60
+    assert [model.recurrence_segment(p) for p in (few, many)] == [choose_segment(p, min(units)) for p in (few, many)]
+    assert [model.scans_whole(p) for p in (few, many, [])] == ["parallel" in order, False, False]
+    seqs = [Sequence(list(range(n)), block_size=64) for n in (1, 130, 64)]
+    for i, s in enumerate(seqs):
+        s.num_cached_tokens, s.block_table, s.state_slot = 0, [0, 1, 2], i
+    for segment in (64, 192):
+        m = build_step_meta([(seqs[1], 130), (seqs[0], 1), (seqs[2], 64)], 64, segment, True)
+        if segment == 64:
+            assert m["summaries"] and m["whole"].tolist() == [[0, 1, 0, 0], [1, 130, 1, 0], [131, 64, 2, 0]]
+        else:
+            assert not m["summaries"] and m["whole"] is None and m["chunks"].tolist() == [[0, 1, 0, 0], [1, 130, 1, 0], [131, 64, 2, 0]]
+    assert build_step_meta([(seqs[1], 130)], 64, 64)["whole"] is None

@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 208          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes */
+#define NVH_VERSION 208          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -910,6 +910,8 @@ typedef struct nvh_scan_desc {
     void* out_packed;            /* nullable (single tokens): the same in MFMA-fragment order */
 } nvh_scan_desc;
 int nvh_scan_states(int n);
+/* Portions times channels below which uncut portions of 16 states (bf16) are scanned with a state per lane, of any length. */
+int nvh_scan_whole_channels(void);
 int nvh_scan_chunks(const nvh_scan_desc* d, int dtype, void* stream);
 int nvh_scan_step(const nvh_scan_desc* d, int dtype, void* stream);
 

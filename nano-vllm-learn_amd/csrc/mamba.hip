@@ -459,6 +459,7 @@ int walk_ns(const ScanArgs& a, hipStream_t stream) {
     return check_launch("scan walk");
 }
 
+constexpr int kWholeChannels = 40960;                // (the host's choice of segments asks for it: nvh_scan_whole_channels)
 template <typename T>
 int walk_t(const ScanArgs& a, hipStream_t stream) {
     // Lanes per channel: more of them add up y over more lanes and read dt and dt x again, fewer make fewer waves, each with more registers.  16 sequences of 512
@@ -472,7 +473,7 @@ int walk_t(const ScanArgs& a, hipStream_t stream) {
             // of 200, 4096 channels (4.25) 82 to 71; 8 of 600 (2.0) 108 to 116, 10 of 790 (2.5) 180 to 173.
             if constexpr (sizeof(T) == 2) {
                 const int64_t fill = (int64_t)a.n_chunks * a.inner;
-                if (!a.summaries && (fill < 40960 || (fill < 65536 && a.rows / a.n_chunks < 512))) {
+                if (!a.summaries && (fill < kWholeChannels || (fill < 65536 && a.rows / a.n_chunks < 512))) {
                     scan_rows_kernel<<<dim3((a.inner + 15) / 16, a.n_chunks), 256, 0, stream>>>(a);
                     return check_launch("scan rows");
                 }
@@ -517,6 +518,8 @@ int nvh_scan_states(int n) {
         if (n > 0 && n <= p) return p;
     return 0;
 }
+
+int nvh_scan_whole_channels(void) { return kWholeChannels; }
 
 int nvh_scan_chunks(const nvh_scan_desc* d, int dtype, void* stream) {
     REQUIRE(d, NVH_E_NULL, "scan_chunks: null descriptor");

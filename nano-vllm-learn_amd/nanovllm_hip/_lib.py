@@ -325,6 +325,7 @@ _SIGS = {
     "nvh_token_shift": (ctypes.c_int, [ctypes.POINTER(TokenShiftDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_causal_conv": (ctypes.c_int, [ctypes.POINTER(CausalConvDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_scan_states": (ctypes.c_int, [ctypes.c_int]),
+    "nvh_scan_whole_channels": (ctypes.c_int, []),
     "nvh_scan_chunks": (ctypes.c_int, [ctypes.POINTER(ScanDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_scan_step": (ctypes.c_int, [ctypes.POINTER(ScanDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_wkv_supported": (ctypes.c_int, [ctypes.c_int]),

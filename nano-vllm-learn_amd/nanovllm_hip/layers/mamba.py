@@ -23,7 +23,7 @@ class ScanUnits(int):
         """Portions few enough for a state per lane that are scanned as fast in one pass as in segments: in microseconds 42 ns a token of the longest, or the load of all and part of
         that, against two passes over the load.  Over 44 mixes the choice costs 1.002 times the faster of both, and takes 0.86 of the time of segments alone."""
         total, longest = sum(portions) * self.channels, max(portions)
-        return len(portions) * self.channels < 40960 and max(0.042 * longest, 4.6e-6 * total + 0.0168 * longest) < 22 + 7.2e-6 * total
+        return len(portions) * self.channels < ops.scan_whole_channels() and max(0.042 * longest, 4.6e-6 * total + 0.0168 * longest) < 22 + 7.2e-6 * total
 
 
 class SelectiveScan(nn.Module):

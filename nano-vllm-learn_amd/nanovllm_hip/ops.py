@@ -1317,6 +1317,11 @@ def scan_states(n) -> int:
     return int(_lib.load().nvh_scan_states(int(n)))
 
 
+def scan_whole_channels() -> int:
+    """Portions times channels below which uncut portions of 16 states (bf16) are scanned with a state per lane."""
+    return int(_lib.load().nvh_scan_whole_channels())
+
+
 def _scan_desc(x, dt, bc, z, p, positions, state_slots, state, out):
     code = _act_code(x, dt, bc, z)
     rows, (inner, n) = x.shape[0], p["a_log2"].shape

@@ -319,8 +319,9 @@ def test_scan_segments(inner, states, units):
     assert SelectiveScan(64, 64, inner, states, 16, 4, torch.bfloat16).segment_units == units
 
 
-def test_scan_whole_portions():
+def test_scan_whole_portions(monkeypatch):
     """16 states in bfloat16: portions whose waves leave the GPU idle stay whole unless one is long for what there is to do; many are cut as other layers' are."""
+    from nanovllm_hip import ops
     from nanovllm_hip.layers.mamba import SelectiveScan
     from nanovllm_hip.layers.rglru import choose_segment
     one, other = (SelectiveScan(64, 64, 2048, 16, 16, 4, d).segment_units for d in (torch.bfloat16, torch.float32))
@@ -328,6 +329,8 @@ def test_scan_whole_portions():
         assert (choose_segment(portions, one) >= max(portions, default=0)) == whole
     long = [4096, *[200] * 39]
     assert one == other and choose_segment(long, one) == choose_segment(long, other) < 4096
+    monkeypatch.setattr(ops, "scan_whole_channels", lambda: 18 * 2048)          # (the kernel's own number, not one like it)
+    assert not one.whole([1000] * 18) and one.whole([1000] * 17)
 
 
 @pytest.mark.parametrize("heads,inner,order", [(16, 2048, ("wkv", "parallel")), (16, 2048, ("parallel", "wkv")), (32, 2048, ("wkv", "parallel")), (32, 2048, ("parallel",) * 2), (8, 2048, ("wkv",))])

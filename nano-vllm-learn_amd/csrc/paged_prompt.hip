@@ -112,7 +112,12 @@ int launch_dims(const PagedAttendArgs& a, hipStream_t stream) {
         // Up to 2.2 workgroups of 64 rows a CU, those: a launch that leaves CUs idle takes as long as its longest walk over the keys.  8 heads of 128 / 128, us with 128 and with
         // 64 rows: one prompt of 2414 tokens 72 and 59, 12 later portions of 3013 with a window 41 and 34, 5 of 3648 with chunks 36 and 29; 16 heads, 4 of 2183 33 and 27; but
         // 2 later portions of 2415 (2.4 a CU, walks of equal length) 92 and 106, 2 of 4140 103 and 116.
-        if (a.max_q > 256 && (int64_t)a.rows * a.heads > 36044) return launch_one<DK, DV, eight ? 1 : 2, eight ? 8 : 4>(a, stream);
+        // But only where all of them run at once, ragged last ones included: wide images leave room for two on a CU (one of 256 / 128), and with 128 rows a second round is
+        // shorter.  2 later portions of 1100 and 3 windowed ones of 730, 16 heads: 128 / 128 104 and 131, 37 and 40; 192 / 64 100 and 125, 35 and 43; 192 / 128 123 and 145; 256 / 128
+        // at half as many rows 123 and 138; where all fit it is 0.98 to 1.6 times as fast, 1.2 in the mean.
+        constexpr int64_t at_once = 163840 / TileImages<DK, DV, 4>::BYTES * 256;
+        const bool few = (int64_t)a.rows * a.heads <= 36044 && ((int64_t)a.rows + 63 * (int64_t)a.batch) * a.heads <= 64 * at_once;
+        if (a.max_q > 256 && !few) return launch_one<DK, DV, eight ? 1 : 2, eight ? 8 : 4>(a, stream);
     }
     return launch_one<DK, DV, 1, 4>(a, stream);
 }

@@ -31,7 +31,7 @@ int nvh_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, const 
     return launch_moe_dispatch(slot_pair, tiles, counts, ids, pairs, experts, tile_rows, max_tiles, (hipStream_t)stream);
 }
 
-int nvh_moe_tile_rows(int pairs, int experts, int dtype) { return pairs > 0 && experts > 0 ? moe_tile_rows(pairs, experts, dtype == NVH_F32) : 0; }
+int nvh_moe_tile_rows(int pairs, int experts, int dtype) { return pairs > 0 && experts > 0 ? moe_tile_rows(pairs, experts, 1024, dtype == NVH_F32) : 0; }
 
 int nvh_moe_gemm(const nvh_moe_gemm_desc* d, int dtype, void* stream) {
     REQUIRE(d, NVH_E_NULL, "moe_gemm: null descriptor");
@@ -55,7 +55,7 @@ struct MoeScratch {
     MoeScratch(int tokens, int top, int experts, int n, int dtype) {
         const size_t pairs = (size_t)tokens * top, part = (pairs + 3) / 4 * 4;
         const bool small = dtype == NVH_BF16 && tokens <= 64;
-        rows = small ? 0 : moe_tile_rows((int)pairs, experts, dtype == NVH_F32);
+        rows = small ? 0 : moe_tile_rows((int)pairs, experts, n, dtype == NVH_F32);
         max_tiles = small ? 0 : (int)pairs / rows + experts;
         ids = pairs * n / (dtype == NVH_F32 ? 1 : 2);
         slots = ids + part;

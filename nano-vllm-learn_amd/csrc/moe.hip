@@ -698,15 +698,22 @@ int launch_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, con
     return check_launch("moe_scatter");
 }
 
-// Rows of a tile, by the pairs an expert has on average (us at 2048 wide, 32 experts of 1536, and 1024 wide, of 768; softmax router).  Few: 64, whose images leave room for three
-// workgroups on a CU, as the weight stream wants: 8 pairs 138 against 147 with 128 rows, 16 155 against 167, 25 158 against 170 (1024 wide equal), 41 166 against 162; but where a router crowds them on some experts 31 are
-// 178 against 169.
-// 256, twice the products per byte of weights and rows read, where an expert's pairs mostly fit one such tile: 125 206 against 230 and 80 against 84, 150 212 against 244 and
-// 84 against 88, 237 267 against 284 and 92 against 100, but 100 209 against 210 and 78 against 72; or fill several: 350 316 against 375 and 122 against 123, 500 418 against 485.
-// In between the second tile is mostly empty: 262 316 against 309 and 123 against 104.
-int moe_tile_rows(int pairs, int experts, int f32) {
+// Rows of a tile, by the pairs an expert has on average and by all columns of the experts (`wide`: how many workgroups a row of tiles is).  us at 2048 wide, experts of 1536, and
+// at 1024, of 768; 8 to 128 experts, even and crowded (the k-th one k^-0.6 as often) routes:
+// - few pairs: 64, whose images leave room for three workgroups on a CU, as the weight stream wants: 32 experts of 1536, 8 pairs 138 against 147 with 128 rows, 16 155 against 167.
+//   From 17 to 25 pairs many wide experts lose with them where a route crowds some (0.92 to 0.95 of the speed); up to 36864 columns in all it is the same or better.
+// - 256, twice the products per byte of weights and rows read, where an expert's pairs mostly fit one such tile or fill several, and there are tiles enough:
+//   from 110 pairs on, 32 experts of 1536, 125 206 against 230, 150 212 against 244; with 98304 columns already from 100 on (64 experts of 1536 0.90 to 0.96 with 128);
+//   193 to 240, below 24576 columns half the CUs and more would get none: 8 experts 1.28 to 2.1 times as fast with 128, 16 of 768 1.3 to 1.65;
+//   256 to 287, where the second tile is mostly empty, 128 is 1.0 to 1.9 times as fast up to 36864 columns (24 of 1536, 48 of 768), 256 from 49152 on (128 experts 0.79 to 0.93 with 128);
+//   more: 32 of 1536, 350 316 against 375, 500 418 against 485.
+int moe_tile_rows(int pairs, int experts, int n, int f32) {
+    if (f32) return FM;
     const int mean = pairs / experts;
-    return f32 ? FM : mean >= 288 || (mean >= 110 && mean <= 240) ? 256 : mean <= 25 ? 64 : 128;
+    const int64_t wide = (int64_t)experts * n;
+    if (mean <= 16 || (mean <= 25 && wide < 49152)) return 64;
+    const bool large = mean >= 288 ? true : mean >= 256 ? wide >= 49152 : mean > 240 ? false : mean >= 193 ? wide >= 24576 : mean >= 110 || (mean >= 100 && wide >= 98304);
+    return large ? 256 : 128;
 }
 
 int launch_moe_gemm(const MoeGemmArgs& a, int f32, hipStream_t stream) {

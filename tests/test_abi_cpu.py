@@ -114,6 +114,15 @@ def test_experts_in_one_call_refuse_scratch_that_is_too_small(lib):
     assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == 0
 
 
+@pytest.mark.parametrize("experts,rows", [(8, {16: 64, 25: 64, 26: 128, 109: 128, 110: 256, 192: 256, 193: 128, 240: 128, 256: 128, 287: 128, 288: 256}),
+                                          (32, {25: 64, 100: 128, 192: 256, 193: 256, 240: 256, 241: 128, 256: 128, 288: 256}),
+                                          (64, {16: 64, 17: 128, 25: 128, 100: 128, 240: 256, 241: 128, 255: 128, 256: 256}), (96, {99: 128, 100: 256, 109: 256, 241: 128, 256: 256})])
+def test_rows_of_expert_tiles(lib, experts, rows):
+    """By the pairs of an expert and by how wide all of them are (1024 columns each); fp32 has one size."""
+    assert {mean: lib.nvh_moe_tile_rows(mean * experts, experts, 0) for mean in rows} == rows
+    assert all(lib.nvh_moe_tile_rows(mean * experts, experts, 1) == 64 for mean in rows)
+
+
 def test_asm_of_several_instructions_shares_no_register():
     """An output that is written while inputs are still to be read must not share a register with one: the compiler may give equal values the same unless it is told (&)."""
     seen = 0

@@ -290,7 +290,7 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         // takes longer sequences.  The loads are inline asm so that no compiler-placed wait sits between them and the K image's DMA.
         const int rows_ok = k_end < a.pv16_rows ? k_end : a.pv16_rows;
         const int g0 = k_beg / kPv16GroupRows, g1 = (rows_ok + kPv16GroupRows - 1) / kPv16GroupRows;
-        const int last = g1 > g0 ? g1 - 1 : g0;
+        const int last = g1 > g0 ? g1 - 1 : 0;       // (rows past the copy have no flags: the first one is read, and does not count)
         int fl[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {

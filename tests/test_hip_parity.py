@@ -1014,6 +1014,21 @@ def test_attention_module_fp16_pv_prefill_rule():
     assert np.array_equal(outs[(200, 90), None], outs[(200, 90), False])             # the short one did not
 
 
+@pytest.mark.parametrize("h,kvh,d", [(2, 1, 64), (14, 2, 64), (4, 2, 128)])
+def test_prefill_pv16_of_fewer_rows_than_sequences_have(ops, h, kvh, d):
+    """Sequences past total_k have no fp16 rows and no range flags: they take the exact form, however far behind the copy they begin."""
+    from nanovllm_hip import _lib
+    lib, lens, copied, gen = _lib.load(), (70, 20000, 700, 5), 70, torch.Generator().manual_seed(d)
+    q, k, v = (torch.randn(sum(lens), n, d, generator=gen).bfloat16().cuda() for n in (h, kvh, kvh))
+    cu = dev_i32([0, 70, 20070, 20770, 20775])
+    how = dict(max_seqlen_q=max(lens), cu_seqlens_q=cu, max_seqlen_k=max(lens), cu_seqlens_k=cu, softmax_scale=d ** -0.5)
+    fast, exact = (ops.flash_attn_varlen_func(q, k, v, **how, pv_fp16=form) for form in (True, False))
+    got, scratch = torch.zeros_like(q), torch.empty(lib.nvh_prefill_pv16_scratch_bytes(copied, kvh, d), dtype=torch.uint8, device="cuda")
+    assert lib.nvh_prefill_varlen_pv16(got.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), cu.data_ptr(), cu.data_ptr(), len(lens), max(lens), max(lens), copied, h, kvh, d,
+                                       h * d, kvh * d, kvh * d, d ** -0.5, 0, 0, scratch.data_ptr(), scratch.numel(), torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(got[:copied], fast[:copied]) and torch.equal(got[copied:], exact[copied:])
+
+
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("batch,h,kvh,d", [(8, 2, 1, 64), (24, 6, 2, 64), (64, 2, 1, 128), (72, 1, 1, 64)])
 def test_prefill_sequences_by_work(ops, batch, h, kvh, d, paged):

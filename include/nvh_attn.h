@@ -715,7 +715,7 @@ typedef struct nvh_moe_route_desc {
 int nvh_moe_route(const nvh_moe_route_desc* d, int dtype, void* stream);
 /* Pairs sorted by expert: slot_pair[slot], tiles [max_tiles][4] = (expert, first slot, slots, tiles in use), unused ones with
  * 0 slots, tile_rows slots each;
- * counts: [nvh_moe_dispatch_blocks(pairs), experts] scratch.  max_tiles >= pairs / tile_rows + experts. */
+ * counts: [nvh_moe_dispatch_blocks(pairs), experts] scratch (up to 8192 pairs left as it is).  max_tiles >= pairs / tile_rows + experts. */
 int nvh_moe_dispatch_blocks(int pairs);
 int nvh_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, const int32_t* ids, int pairs, int experts, int tile_rows, int max_tiles, void* stream);
 /* Expert products.  glu: act[p] = silu(x[p / top] . gate_e) * (x . up_e), w = [experts, 2 * n, k] (gate rows, then up rows), or with alpha != 0 the clamped unit

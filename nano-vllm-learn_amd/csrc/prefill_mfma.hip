@@ -991,7 +991,8 @@ int launch_d(const PrefillArgs& a, hipStream_t stream) {
     // 14 / 2 heads of 64: 0.9 43 / 31 / 26.5, 1.3 61 / 47 / 38.5, 1.5 36 / 30 / 38, 2.6 77 / 65 / 70, 3.4 90 / 98 / 101; heads of 128: 7 / 1 0.4 57 / 43 / 34, 0.85 103 / 79 / 61,
     // 1.1 46 / 35 / 38, 1.7 101 / 82 / 106; 16 / 8 1.0 64 / 53 / 49, 1.9 82 / 91 / 116; 28 / 4 1.7 33 / 30 / 40, 2.5 42 / 45 / 62.
     // The rows are known where V was copied; otherwise uneven sequences are taken to have half of the longest on average (for the two groups always: which of them adds what
-    // shows in the last bits, and a sequence whose V does not fit fp16 keeps those of the exact form).
+    // shows in the last bits, and a sequence whose V does not fit fp16 keeps those of the exact form, but for ten and more prompts of nearly one length at heads of 128 that
+    // just reach the line for 128 rows).  By the longest prompt and their number, so these bits depend on what else is in the batch.
     const double all = (double)a.max_seqlen_q * a.batch, guess = 0.5 * (all + a.max_seqlen_q);
     if (two && prefill_fill(a, a.v16 && a.pv16_rows < all ? a.pv16_rows : guess) >= (D == 64 ? 3.0 : 1.8)) return launch_q<D, 2, 1>(a, stream);
     if (a.max_seqlen_k >= 1024 && prefill_fill(a, guess) < (D == 64 ? 1.3 : 1.0)) return launch_q<D, 1, 2>(a, stream);

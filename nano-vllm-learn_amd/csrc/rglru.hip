@@ -4,14 +4,15 @@
 //   log a = -rate r ; S = a S + sqrt(1 - a^2) i u ; out = S gelu(y)
 // The recurrence and everything that enters it besides u is fp32; u is rounded once to the activation type.
 //
-// Prompt portions (launch_rglru_chunks): the host cuts a portion into segments; a workgroup owns one (segment, diagonal block) and walks the segment 64
-// tokens at a time with the state in registers: convolution into LDS, both gates on MFMA tiles, and the scan of the 64 tokens IN the accumulator
-// layout (a lane holds 4 consecutive tokens of one channel, the 4 lane groups 16 consecutive ones: compose 4 in the lane, two shuffles across the
-// groups, a carry over the 16-token tiles), then S gelu(y) back out through LDS.
-// A portion of one segment (many sequences at once) is one such walk.  Otherwise a SUMMARY walk first leaves (product of decays, end value) of every
-// segment but the last, and the second walk of a segment starts from the composition of the ones before it.
-// Blocks of up to 256 channels whose walks would not fill the GPU evenly take the same steps of 64 tokens in any workgroup (rglru_chain_kernel).
-// State and convolution ring are read by the walks and written by a small launch behind them: no workgroup can see a half-updated one.
+// Prompt portions (launch_rglru_chunks) come cut into segments by the host and are worked through 64 tokens at a time, by workgroups that own a diagonal block:
+// convolution into LDS, both gates on MFMA tiles, and the scan of the 64 tokens IN the accumulator layout, then S gelu(y) back out through LDS.
+// - Blocks of up to 256 channels (bf16) mostly: any workgroup of the block takes any step, and the state in front of a step comes from the ones before it
+//   (rglru_chain_kernel; a lane holds 16 consecutive tokens).  Cut or whole portions, the steps are the same.
+// - Otherwise a workgroup walks a segment with the state in registers (rglru_scan_kernel; larger blocks rglru_walk_kernel; a lane holds 4 consecutive tokens of one
+//   channel, the 4 lane groups 16: compose 4 in the lane, two shuffles across the groups, a carry over the 16-token tiles).  A portion of one segment is one such walk.
+//   Of a cut one a SUMMARY walk first leaves (product of decays, end value) of every segment but the last, and the second walk of a segment starts from the composition
+//   of the ones before it.  Blocks of up to 256 channels come here where walks of whole portions are faster (whole_walks), and of cut ones from callers without `links`.
+// State and convolution ring are read by the walks and written by a small launch behind them, by the steps in a portion's last one: nobody sees a half-updated one.
 // Decode (launch_rglru_step): one workgroup per 16 channels and 32 sequences does all of it in one launch.  Convolution inputs live in a ring of
 // `taps` entries (input of position p at entry p % taps): the entry a step writes is the one no workgroup of that step reads.
 // A sequence's first token (position 0) takes state and earlier inputs as zero instead of reading them: slots need no clearing when reused.
@@ -256,8 +257,8 @@ __global__ __launch_bounds__(1024) void rglru_walk_kernel(const RglruArgs a) {
 // a block has a wave for every 16 channels, four on each SIMD at 256: 128 registers a lane, addresses computed again (fresh) instead of held.  Rows are
 // reached by 32-bit offsets from a step's first one; the 16-token passes are unrolled and find everything at fixed distances.  One barrier behind the scan frees u and
 // makes out whole, one behind the rows' way out and the next convolution frees x.
-// Four blocks of 256 channels, 16 sequences of 1024 tokens as whole portions: 200 -> 148 us; of 32 channels 66 -> 59; 16384 tokens of 16 uneven sequences, 10 blocks
-// of 256, split: 316 -> 250 (230 to 260, with the lengths).
+// Against the walk without LDS-DMA, four blocks of 256 channels, 16 sequences of 1024 tokens as whole portions: 200 -> 148 us (144 since elements are read singly); of
+// 32 channels 66 -> 59 (56).  What runs in their place now (whole_walks says where not) takes 70 and 30 there.
 constexpr int HALO = 8;                              // rows in front of a step's 64 in the x image: taps <= HALO + 1
 
 __device__ __forceinline__ int fresh(int v) {         // computed again from here on instead of held in registers across the loop
@@ -489,16 +490,18 @@ __global__ __launch_bounds__(128 * KS, 4) void rglru_scan_kernel(const RglruArgs
 // ------------------------------------------------------------------------------------------------ the same blocks, any workgroup any 64 tokens
 // The same arithmetic, cut into steps of 64 tokens that any workgroup of the block can take: what enters the recurrence needs no state, so a step's decays and
 // inputs are composed from its first token on, and only the state in front of it comes from elsewhere: out = (A h + S) gelu(y).  A workgroup keeps both gates'
-// weights of its block in registers (a wave its 16 channels') and draws steps by ticket, in the order of the segment table.  Per step and wave: products, gates, scan -> (product of
-// decays, end value) of its 16 channels published; the next step's convolution; then the state in front: the nearest step of the portion that has published the
-// state behind it, and from there the published pairs one by one (always this order of sums, whoever was first).
+// weights of its block in registers (a wave its 16 channels') and draws steps by ticket, in the order of rglru_steps_kernel's list.  The state in front is found by decoupled
+// look-back (Merrill and Garland, single-pass parallel prefix scan, 2016).  Per step and wave: products, gates, scan -> (product of decays, end value) of its 16 channels published;
+// then the state in front: the nearest step of the portion that has published the state behind it, and from there the published pairs one by one (always this order of sums,
+// whoever was first); then the output, and the next step's convolution.
 // A drawn step waits for steps drawn before it only, and those are in the hands of workgroups that run: no assumption on how many are resident or on their order.  The
 // wait is bounded all the same (a state of NaN behind it).
-// x travels by LDS-DMA under a step's products, y a step ahead; u and y come into the accumulator layout by single elements.  Rows lie so that a lane of the accumulators holds 16 consecutive tokens of a channel: one composition across lanes a step, not four.
+// x travels by LDS-DMA under a step's products, y a step ahead; u and y come into the accumulator layout by single elements.  Rows lie so that a lane of the accumulators
+// holds 16 consecutive tokens of a channel: one composition across lanes a step, not four.
 // Both gates' products of all 64 tokens come first and decays and inputs take their place: 64 registers of weights and 32 of these leave room for rows asked for ahead.
 // 128 registers a lane (four waves on each SIMD at 256 channels): addresses are computed again (fresh) instead of held.
 // Bound by the issue of vector instructions (about 60 and 8 transcendentals per element, 80 % of the time) on 250 of 256 CUs; a step takes 11 us whoever takes it, of which the state
-// in front costs 1.  16384 tokens of 16 uneven sequences, 10 blocks of 256: walks 224 us on 160 CUs, the longest 28 steps; steps by any workgroup 148.  5 sequences, 4 blocks: 106 -> 91 (in
+// in front costs 1.  16384 tokens of 16 uneven sequences, 10 blocks of 256: walks 224 us on 160 CUs, the longest 28 steps; steps by any workgroup 135.  5 sequences, 4 blocks: 106 -> 91 (in
 // segments with a summary pass before).  One sequence of 2000 tokens, 4 blocks: 45 -> 38.
 constexpr int kWaitLimit = 1 << 22;                  // polls of about a microsecond
 constexpr int kAhead = 2;                            // rows of u asked for ahead of the products that take them

@@ -23,12 +23,13 @@ LATE_SHARE = 0.7              # of a longest walk that still runs alone when the
 
 def choose_segment(portions, blocks, chunk=64):
     """Tokens per segment for portions of these lengths: `blocks` workgroups walk each segment, and cutting a portion into more than one
-    costs a summary walk over all its segments but the last.  Returns the cheapest multiple of `chunk` among about ten per octave of lengths.
+    costs a summary walk over all its segments but the last.  (The gated recurrence in bf16 with blocks of up to 256 channels takes steps of 64 tokens by any workgroup however
+    portions are cut: there the choice only says that it does, where it cuts.)  Returns the cheapest multiple of `chunk` among about ten per octave of lengths.
 
     Walks of different lengths share the CUs: beyond one a CU, the launch takes as long as the even load and most of a longest walk, or as so many rounds
     of longest walks, whichever is less.  (Counted in rounds alone, forty prompts of 6 to 13 steps were cut up: whole, lightning attention takes them in 67 us against
     117, the scan in 155 against 265.)  Over ten mixes of 1 to 40 sequences the choice costs 1.03 times the best segment's walks for lightning attention, time mixing and
-    the gated recurrence, 1.04 for the scan; counted in rounds 1.16, 1.10, 1.11 and 1.14."""
+    the gated recurrence (walked: larger blocks), 1.04 for the scan; counted in rounds 1.16, 1.10, 1.11 and 1.14."""
     longest = max(portions, default=1)
     last, total = -(-longest // chunk), sum(portions) / chunk
 

@@ -1032,7 +1032,8 @@ def test_prefill_pv16_of_fewer_rows_than_sequences_have(ops, h, kvh, d):
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("batch,h,kvh,d", [(8, 2, 1, 64), (24, 6, 2, 64), (64, 2, 1, 128), (72, 1, 1, 64)])
 def test_prefill_sequences_by_work(ops, batch, h, kvh, d, paged):
-    """Sequences are dealt to the XCDs by their work: each of them once, equal ones and ones without rows or without earlier keys among them, with the bits that it has alone."""
+    """Sequences are dealt to the XCDs by their work: each of them once, equal ones and ones without rows or without earlier keys among them, with the bits that it has alone (up
+    to 813 keys; from 1024 on a launch of few rows joins the sums of two groups of waves: test_prefill_rows_of_a_workgroup_by_fill)."""
     gen = torch.Generator().manual_seed(batch)
     new = [(0, 1, 63, 64, 65, 200, 513)[int(i)] for i in torch.randint(7, (batch,), generator=gen)]
     old = [(0, 0, 70, 300)[int(i)] if paged and n else 0 for i, n in zip(torch.randint(4, (batch,), generator=gen), new)]

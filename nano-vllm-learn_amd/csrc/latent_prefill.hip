@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256, DK + DV <= 320 ? 2 : 1) void latent_prefill_ke
         }
         return *reinterpret_cast<const bf16x8*>(&raw);
     };
-    attend_walk<DK, DV, QT, 4>(
+    attend_walk<DK, DV, QT>(
         lds, n_tiles, a.scale_log2, -INFINITY, lane, stage, query, [&](int it) { return it * BN; }, [&](int kv0) { return kv0 <= wave_last_key; },
         [&](int kv0) { return kv0 + BN - 1 > wave_first_key || kv0 + BN > sk; },
         [&](int kv0, int qs, int off) { return off <= (my_q[qs] + shift < sk - 1 ? my_q[qs] + shift : sk - 1) - kv0 - 4 * lg; },

@@ -164,28 +164,28 @@ __device__ __forceinline__ f32x4 turn_back(f32x4 v, const float* table, int64_t 
     }
     return v;
 }
-// the same for columns 16 t + 4 lg .. of all t: where a lane's two pairs lie side by side in the table on 8 bytes (every usual width), everything
+// the same for columns COLS t + 4 lg .. of all t: where a lane's two pairs lie side by side in the table on 8 bytes (every usual width), everything
 // is asked of the table before anything is turned, two pairs a load.  Tile by tile each turn waited for its own four loads, DT round trips to the
 // cache one behind the other at the end of every block: paged_prompt_kernel over 16384 new tokens, chunk mask, 128 columns turned:
 // 16 heads 79.7 -> 71.2 us (16 sequences) and 71.7 -> 64.7 (5), 32 heads 131.7 -> 116.5 (30).
-template <int DT>
+template <int COLS = 16, int DT>
 __device__ __forceinline__ void turn_back_tiles(f32x4 (&v)[DT], const float* table, int64_t pos, int max_position, int rot, int lg) {
     if (rot & 3 || reinterpret_cast<uintptr_t>(table) & 7) {
 #pragma unroll
-        for (int t = 0; t < DT; ++t) v[t] = turn_back(v[t], table, pos, max_position, rot, 16 * t + 4 * lg);
+        for (int t = 0; t < DT; ++t) v[t] = turn_back(v[t], table, pos, max_position, rot, COLS * t + 4 * lg);
         return;
     }
     const float* cs = table + (pos < max_position ? pos : max_position - 1) * rot;
     f32x2 c[DT], s[DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
-        const int i = 8 * t + 2 * lg, at = 2 * i < rot ? i : 0;
+        const int i = COLS / 2 * t + 2 * lg, at = 2 * i < rot ? i : 0;
         c[t] = *reinterpret_cast<const f32x2*>(cs + at);
         s[t] = *reinterpret_cast<const f32x2*>(cs + rot / 2 + at);
     }
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
-        const bool turned = 16 * t + 4 * lg < rot;
+        const bool turned = COLS * t + 4 * lg < rot;
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             const float x = v[t][2 * p], y = v[t][2 * p + 1];

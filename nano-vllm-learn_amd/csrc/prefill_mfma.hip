@@ -5,8 +5,8 @@
 //                   bottom-right aligned causal mask; parity unpinned by the reference)
 //
 // Dense contraction -> MFMA (v_mfma_f32_16x16x32_bf16), flash-style online softmax, fp32 accumulate.
-// Workgroup = 4 waves = a tile of BM = 64*QT query rows of one (sequence, q head); wave w owns rows 16*QT*w .. +16*QT-1 as QT
-// sub-tiles of 16 rows (QT = 1 or 2, picked per launch from head_dim and the longest sequence).
+// Workgroup = 4 waves = a tile of 64 query rows of one (sequence, q head), wave w rows 16 w .. 16 w + 15; or of 128 rows, 32 a wave on 32 x 32 tiles (attend_walk32, the
+// same sums to the bit), where the launch fills the chip with those.
 // K/V tiles of BN = 64 keys are staged through LDS by LDS-DMA (global_load_lds_dwordx4: one instruction = 1 KiB of
 // whole, coalesced key rows, no VGPR round trip), DOUBLE-BUFFERED: the DMA of tile i+1 is in flight while tile i is
 // computed; waves wait with a counted vmcnt and meet at raw s_barriers (a __syncthreads() would drain the prefetch).
@@ -32,7 +32,7 @@
 // Algorithmic flops per launch: sum_seq 4*D*H*(causal pairs); bytes: Tq*H*D*2*2 + Tk*KVH*D*2*2.
 #include <type_traits>
 
-#include "common.h"
+#include "attend_tile.h"
 #include "kernels.h"
 
 namespace nvh {
@@ -69,9 +69,6 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 #define SK_STAMP(k) do {} while (0)
 #endif
 
-// QT = 16-row query sub-tiles per wave (template parameter): with QT = 2 every K / V fragment read from LDS feeds both
-// sub-tiles' MFMAs and the per-tile scalar / DMA / barrier work is halved per flop, at half the occupancy.  Measured (lean
-// loop, heaviest-first grid): D=128 +18.5 % (482 -> 571 TFLOP/s at S=4096), D=64 +6.6 % at S=4096, neutral at S=1024.
 constexpr int BN = 64;      // keys per LDS tile
 
 // ds_read_b64_tr_b16 through inline asm: the builtin form makes hipcc wait vmcnt(0) before the read (it cannot prove the read
@@ -170,6 +167,13 @@ __device__ __forceinline__ void prefill_tile_of_block(const PrefillArgs& a, int&
 #endif
 }
 
+__device__ __forceinline__ bool prefill_tile(const PrefillArgs& a, int* words, PromptTile& t) {
+    if (a.batch <= kFewPrompts) return few_prompts_tile<128>(a.cu_q, a.cu_k, a.batch, a.h, a.kvh, 0, words, t);
+    prefill_tile_of_block(a, t.qt, t.head, t.b);
+    prompt_rows(a.cu_q, a.cu_k, t);
+    return t.qt * 128 < t.sq;
+}
+
 // rows row0 .. of one head that see no key
 template <int D, int THREADS>
 __device__ __forceinline__ void zero_rows(const PrefillArgs& a, int row0, int n, int head, int tid) {
@@ -181,14 +185,35 @@ __device__ __forceinline__ void zero_rows(const PrefillArgs& a, int row0, int n,
     }
 }
 
-// One workgroup's tile: query rows qt * 64 * QT .. of (sequence b, head), all the keys they can see.
-// GUARD (nvh_prefill_varlen_pv16): `a.v` is the fp16 copy of V; the range flags of this sequence's rows are fetched FIRST, the first K image's DMA is
-// issued behind them, and only then are they looked at — so the check costs no memory latency of its own.  Returns false (nothing but that K image
-// touched) when a flag is set: the caller runs the exact body instead.
+// Range flags of one sequence's rows of V, one per kPv16GroupRows rows: asked for ahead of the first tile's DMA and the queries and looked at behind them, so that the check costs no
+// memory latency of its own.  Lane l holds groups g0 + l, + 64, + 128, + 192 (16384 rows: the largest prefill batch); a plain loop takes longer sequences.
+struct RangeFlags {
+    int held[4], g0, g1;
+    // false: rows without a copy (a caller whose total_k was short of cu_seqlens_k[batch])
+    __device__ __forceinline__ bool ask(const PrefillArgs& a, int k_beg, int k_end, int lane) {
+        if (k_end > a.pv16_rows) return false;
+        g0 = k_beg / kPv16GroupRows;
+        g1 = (k_end + kPv16GroupRows - 1) / kPv16GroupRows;                      // (one group at least: a tile is staged for keys only)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) held[i] = a.pv16_flags[min(g0 + lane + 64 * i, g1 - 1)];
+        return true;
+    }
+    __device__ __forceinline__ bool clear(const PrefillArgs& a, int lane) const {
+        uint64_t bad = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bad |= __builtin_amdgcn_ballot_w64(held[i] != 0);
+        for (int g = g0 + 256; g < g1; g += 64) bad |= __builtin_amdgcn_ballot_w64(a.pv16_flags[min(g + lane, g1 - 1)] != 0);
+        return bad == 0;
+    }
+};
+
+// One workgroup's tile: query rows qt * 64 .. of (sequence b, head), all the keys they can see.
+// GUARD (nvh_prefill_varlen_pv16): `a.v` is the fp16 copy of V.  Returns false, with nothing but the first images touched, when a range flag is set: the caller runs the exact body
+// instead.
 // KS groups of four waves work on the same rows, each on every KS-th tile of keys with images of its own; the first adds up their sums at the end.
-template <int D, bool PAGED, int QT, bool F16V, bool GUARD, int KS>
+template <int D, bool PAGED, bool F16V, bool GUARD, int KS>
 __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsigned char* const lds_all, const int qt, const int head, const int b) {
-    constexpr int BM = 64 * QT;                      // query rows per workgroup (4 waves x QT x 16)
+    constexpr int BM = 64;                           // query rows per workgroup (4 waves x 16)
     constexpr int ROWB = D * 2;                      // LDS row, bytes
     constexpr int LPT = D / 8;                       // 16-byte chunks per row
     constexpr int TPI = 64 / LPT;                    // rows per DMA instruction
@@ -198,7 +223,7 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
     constexpr int STEPS = D / 32;                    // k-steps of the QK^T contraction
     constexpr int DT = D / 16;                       // 16-dim output tiles
     constexpr int NT = BN / 16;                      // 16-key tiles of S^T per LDS tile
-    constexpr int WR = 16 * QT;                      // query rows per wave
+    constexpr int WR = 16;                           // query rows per wave
     const int q_beg = a.cu_q[b], q_end = a.cu_q[b + 1];
     const int k_beg = a.cu_k[b], k_end = a.cu_k[b + 1];
     const int sq = q_end - q_beg, sk = k_end - k_beg;
@@ -223,15 +248,12 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
     const int lq = lane & 15;                        // query column of this lane
     const int lg = lane >> 4;                        // lane group: k-block of the operands / key rows of C
 
-    f32x4 o[QT][DT];
-    float m_run[QT], l_run[QT];                      // per query column; l_run is this lane group's share
+    f32x4 o[DT];
+    float m_run, l_run;                      // per query column; l_run is this lane group's share
+    m_run = -INFINITY;
+    l_run = 0.f;
 #pragma unroll
-    for (int qs = 0; qs < QT; ++qs) {
-        m_run[qs] = -INFINITY;
-        l_run[qs] = 0.f;
-#pragma unroll
-        for (int t = 0; t < DT; ++t) o[qs][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int wave_first_key = q0 + wave * WR + shift;            // last key the wave's FIRST row may see
     const int wave_last_key = wave_first_key + WR - 1;            // last key ANY row of this wave may see
@@ -251,7 +273,7 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         voff[j] = (uint32_t)(R * vstride + (dp ^ chunk_swz_v<LPT>(R)) * 8);
     }
     PageNumbers pages{PAGED ? a.block_tables + (int64_t)b * a.bt_row_stride : nullptr, PAGED ? (sk - 1) / a.block_size : 0};
-    auto stage = [&](int tile, int buf, const bool do_k = true, const bool do_v = true) __attribute__((always_inline)) {
+    auto stage = [&](int tile, int buf) __attribute__((always_inline)) {
         unsigned char* kimg = lds + buf * 2 * IMG;
         unsigned char* vimg = kimg + IMG;
         const int kv0 = tile * BN;
@@ -277,61 +299,37 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
                 ko = (uint32_t)(Rc * kstride + (dp ^ chunk_swz<LPT>(R)) * 8);
                 vo = (uint32_t)(Rc * vstride + (dp ^ chunk_swz_v<LPT>(R)) * 8);
             }
-            if (do_k) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kb + ko),
-                                                       (__attribute__((address_space(3))) void*)(kimg + ins * 1024), 16, 0, 0);
-            if (do_v) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vb + vo),
-                                                       (__attribute__((address_space(3))) void*)(vimg + ins * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kb + ko),
+                                             (__attribute__((address_space(3))) void*)(kimg + ins * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vb + vo),
+                                             (__attribute__((address_space(3))) void*)(vimg + ins * 1024), 16, 0, 0);
         }
     };
 
     const int first = grp < n_tiles ? grp : n_tiles - 1;         // (a group without a tile stages one all the same: the waits count on it)
+    RangeFlags flags;
     if constexpr (GUARD) {
-        // one flag per kPv16GroupRows rows of V; lane l looks at groups g0 + l, + 64, + 128, + 192 (16384 rows: the largest prefill batch), a plain loop
-        // takes longer sequences.  The loads are inline asm so that no compiler-placed wait sits between them and the K image's DMA.
-        const int rows_ok = k_end < a.pv16_rows ? k_end : a.pv16_rows;
-        const int g0 = k_beg / kPv16GroupRows, g1 = (rows_ok + kPv16GroupRows - 1) / kPv16GroupRows;
-        const int last = g1 > g0 ? g1 - 1 : 0;       // (rows past the copy have no flags: the first one is read, and does not count)
-        int fl[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int g = g0 + lane + 64 * i;
-            const int32_t* p = a.pv16_flags + (g < last ? g : last);
-            asm volatile("global_load_dword %0, %1, off" : "=v"(fl[i]) : "v"(p) : "memory");
-        }
-        stage(first, 0, true, false);
-        asm volatile("s_waitcnt vmcnt(%4)" : "+v"(fl[0]), "+v"(fl[1]), "+v"(fl[2]), "+v"(fl[3]) : "n"(NIW) : "memory");
-        bool bad = k_end > a.pv16_rows;              // (a caller whose total_k was short of cu_seqlens_k[batch]: no fp16 copy of those rows)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) bad |= __builtin_amdgcn_ballot_w64(g0 + lane + 64 * i < g1 && fl[i] != 0) != 0;
-        for (int g = g0 + 256 + lane; __builtin_amdgcn_ballot_w64(g < g1) != 0; g += 64)
-            bad |= __builtin_amdgcn_ballot_w64(g < g1 && a.pv16_flags[g < g1 ? g : last] != 0) != 0;
-        if (bad) return false;
-        stage(first, 0, false, true);
-    } else {
-        stage(first, 0);
+        if (!flags.ask(a, k_beg, k_end, lane)) return false;
     }
+    stage(first, 0);
     // ---- Q fragments (B operand of S^T): Q[row][32*step + 8*lg .. +8]; plain loads issued BEHIND the first tile's DMA, so that a workgroup
     // pays one memory latency at its start, not two in a row (the counted wait of the first tile body leaves only tile 1's DMA in flight:
     // vector-memory operations complete in order, so tile 0 and these loads have landed by then)
-    int my_q[QT];                                    // query index inside the sequence, per sub-tile
-    bool q_ok[QT];
-    bf16x8 qf[QT][STEPS];
+    const int my_q = q0 + wave * WR + lq;            // query index inside the sequence
+    const bool q_ok = my_q < sq;
+    bf16x8 qf[STEPS];
+    const uint16_t* qp = a.q + (int64_t)(q_beg + (q_ok ? my_q : sq - 1)) * a.q_row_stride + (int64_t)head * D + lg * 8;
 #pragma unroll
-    for (int qs = 0; qs < QT; ++qs) {
-        my_q[qs] = q0 + wave * WR + 16 * qs + lq;
-        q_ok[qs] = my_q[qs] < sq;
-        const uint16_t* qp = a.q + (int64_t)(q_beg + (q_ok[qs] ? my_q[qs] : sq - 1)) * a.q_row_stride + (int64_t)head * D + lg * 8;
-#pragma unroll
-        for (int st = 0; st < STEPS; ++st) {
-            const u32x4 raw = *reinterpret_cast<const u32x4*>(qp + st * 32);
-            qf[qs][st] = *reinterpret_cast<const bf16x8*>(&raw);
-        }
+    for (int st = 0; st < STEPS; ++st) {
+        const u32x4 raw = *reinterpret_cast<const u32x4*>(qp + st * 32);
+        qf[st] = *reinterpret_cast<const bf16x8*>(&raw);
+    }
+    if constexpr (GUARD) {
+        if (!flags.clear(a, lane)) return false;
     }
     // waited for here: left to the loop, the wait for these loads would drain the DMA in flight in every tile
 #pragma unroll
-    for (int qs = 0; qs < QT; ++qs)
-#pragma unroll
-        for (int st = 0; st < STEPS; ++st) asm volatile("" : "+v"(qf[qs][st]));
+    for (int st = 0; st < STEPS; ++st) asm volatile("" : "+v"(qf[st]));
     PF_STAMP(0);
     // tr-read: lane 4q+p of its group addresses key row q, dims 4p..4p+3.  The per-lane part of the address (row 4*lg+q,
     // swizzled chunk of dim tile t) is loop invariant: DT registers; buffer, image, 32-key half and the +16-row partner are
@@ -359,116 +357,106 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
         const unsigned char* kimg = lds + buf * 2 * IMG;
         const int kv0 = it * BN;
         if (kv0 <= wave_last_key && (KS == 1 || it < n_tiles)) {                 // wave-uniform: tile not entirely above the diagonal
-            // ---- S^T for the four 16-key tiles of both query sub-tiles: each K fragment is read once, used QT times
+            // ---- S^T for the four 16-key tiles
             // (skipping the 16-key groups above the wave's diagonal, as the short-sequence kernel below does, measured 2-5 % SLOWER
             // here at every S >= 256, same-box A/B: the interior tiles pay for the extra branches and live ranges)
-            f32x4 sT[QT][NT];
+            f32x4 sT[NT];
 #pragma unroll
             for (int tt = 0; tt < NT; ++tt) {
-#pragma unroll
-                for (int qs = 0; qs < QT; ++qs) sT[qs][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                sT[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
                 const int R = 16 * tt + lq;
 #pragma unroll
                 for (int st = 0; st < STEPS; ++st) {
                     const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kimg + R * ROWB + (((4 * st + lg) ^ chunk_swz<LPT>(R)) * 16));
-#pragma unroll
-                    for (int qs = 0; qs < QT; ++qs) sT[qs][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[qs][st], sT[qs][tt], 0, 0, 0);
+                    sT[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[st], sT[tt], 0, 0, 0);
                 }
             }
             // The max chain reads the accumulators through inline asm, which hipcc does not pad with the wait states a VALU read of
             // a fresh MFMA result needs; one statement that takes every accumulator as an operand (so it follows every MFMA of the
             // tile) carries them (see the same guard in paged_decode.hip, where a 16-key tile exposed the hazard).
-            if constexpr (QT == 1) asm volatile("s_nop 7" : "+v"(sT[0][0]), "+v"(sT[0][1]), "+v"(sT[0][2]), "+v"(sT[0][3]));
-            else asm volatile("s_nop 7" : "+v"(sT[0][0]), "+v"(sT[0][1]), "+v"(sT[0][2]), "+v"(sT[0][3]), "+v"(sT[1][0]), "+v"(sT[1][1]), "+v"(sT[1][2]), "+v"(sT[1][3]));
-            static_assert(QT == 1 || QT == 2, "query sub-tiles per wave");
+            asm volatile("s_nop 7" : "+v"(sT[0]), "+v"(sT[1]), "+v"(sT[2]), "+v"(sT[3]));
             // ---- online softmax in the log2 domain.  Masking only where it can matter: tiles that reach past this wave's
             // first row's diagonal or past the sequence end (wave-uniform test); interior tiles skip the per-element work.
             const bool need_mask = kv0 + BN - 1 > wave_first_key || kv0 + BN > sk;
+            if (need_mask) {
+                // element (tt, r) of this lane is key kv0 + 16 tt + 4 lg + r; it is visible iff key <= min(q_pos, sk - 1), i.e. iff the
+                // CONSTANT 16 tt + r is <= a per-lane limit: one compare against an inline constant + one select per element — and only
+                // in the 16-key groups that reach past what the sub-tile's FIRST row may see (wave-uniform test): the groups below the
+                // diagonal block of a diagonal tile are visible to every row
+                const int q_pos = my_q + shift;                          // last key this lane's query may see
+                const int limit = (q_pos < sk - 1 ? q_pos : sk - 1) - kv0 - 4 * lg;
+                const int first_row_key = wave_first_key;
+                const int all_see = (first_row_key < sk - 1 ? first_row_key : sk - 1) - kv0;      // keys kv0 .. kv0 + all_see: no mask needed
 #pragma unroll
-            for (int qs = 0; qs < QT; ++qs) {
-                if (need_mask) {
-                    // element (tt, r) of this lane is key kv0 + 16 tt + 4 lg + r; it is visible iff key <= min(q_pos, sk - 1), i.e. iff the
-                    // CONSTANT 16 tt + r is <= a per-lane limit: one compare against an inline constant + one select per element — and only
-                    // in the 16-key groups that reach past what the sub-tile's FIRST row may see (wave-uniform test): the groups below the
-                    // diagonal block of a diagonal tile are visible to every row
-                    const int q_pos = my_q[qs] + shift;                          // last key this lane's query may see
-                    const int limit = (q_pos < sk - 1 ? q_pos : sk - 1) - kv0 - 4 * lg;
-                    const int first_row_key = wave_first_key + 16 * qs;
-                    const int all_see = (first_row_key < sk - 1 ? first_row_key : sk - 1) - kv0;      // keys kv0 .. kv0 + all_see: no mask needed
+                for (int tt = 0; tt < NT; ++tt) {
+                    if (16 * tt + 15 > all_see) {
 #pragma unroll
-                    for (int tt = 0; tt < NT; ++tt) {
-                        if (16 * tt + 15 > all_see) {
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) sT[qs][tt][r] = (16 * tt + r <= limit) ? sT[qs][tt][r] : -INFINITY;
-                        }
+                        for (int r = 0; r < 4; ++r) sT[tt][r] = (16 * tt + r <= limit) ? sT[tt][r] : -INFINITY;
                     }
                 }
-                float mx = max3(sT[qs][0][0], sT[qs][0][1], sT[qs][0][2]);
-                mx = max3(mx, sT[qs][0][3], sT[qs][1][0]);
-                mx = max3(mx, sT[qs][1][1], sT[qs][1][2]);
-                mx = max3(mx, sT[qs][1][3], sT[qs][2][0]);
-                mx = max3(mx, sT[qs][2][1], sT[qs][2][2]);
-                mx = max3(mx, sT[qs][2][3], sT[qs][3][0]);
-                mx = max3(mx, sT[qs][3][1], sT[qs][3][2]);
-                mx = max2(mx, sT[qs][3][3]);
-                mx = max_xor16(mx);
-                mx = max_xor32(mx);
-                mx *= a.scale_log2;                                              // scale > 0: max commutes with the scaling
-                const float m_new = moved_max(m_run[qs], mx);
-                // rows that have seen no key yet keep m = -inf; use 0 as the reference point so exp2 stays finite
-                const float m_use = m_new == -INFINITY ? 0.f : m_new;
-                // scale-and-subtract and the row sum on element pairs (plain fp32 instructions: packed ones are switched off in the build), exp2 per element
-                const f32x2 sc2 = {a.scale_log2, a.scale_log2}, mm2 = {-m_use, -m_use};
-                f32x2 psum2 = {0.f, 0.f};
-#pragma unroll
-                for (int tt = 0; tt < NT; ++tt)
-#pragma unroll
-                    for (int r = 0; r < 4; r += 2) {
-                        const f32x2 sv = {sT[qs][tt][r], sT[qs][tt][r + 1]};
-                        const f32x2 z = __builtin_elementwise_fma(sv, sc2, mm2);
-                        const f32x2 e = {fast_exp2(z[0]), fast_exp2(z[1])};
-                        sT[qs][tt][r] = e[0];
-                        sT[qs][tt][r + 1] = e[1];
-                        psum2 += e;
-                    }
-                const float psum = psum2[0] + psum2[1];
-                if (__builtin_amdgcn_ballot_w64(m_new != m_run[qs]) != 0) {      // some row's max moved: rescale (wave-uniform branch)
-                    const float alpha = fast_exp2(m_run[qs] - m_use);            // m_run = -inf -> 0
-                    l_run[qs] *= alpha;
-#pragma unroll
-                    for (int t = 0; t < DT; ++t) o[qs][t] *= alpha;
-                }
-                l_run[qs] += psum;
-                m_run[qs] = m_new;
             }
-            // ---- O^T += V^T P^T, 32 keys at a time, P as hi + lo bf16; each V fragment is read once, used 2*QT times
+            float mx = max3(sT[0][0], sT[0][1], sT[0][2]);
+            mx = max3(mx, sT[0][3], sT[1][0]);
+            mx = max3(mx, sT[1][1], sT[1][2]);
+            mx = max3(mx, sT[1][3], sT[2][0]);
+            mx = max3(mx, sT[2][1], sT[2][2]);
+            mx = max3(mx, sT[2][3], sT[3][0]);
+            mx = max3(mx, sT[3][1], sT[3][2]);
+            mx = max2(mx, sT[3][3]);
+            mx = max_xor16(mx);
+            mx = max_xor32(mx);
+            mx *= a.scale_log2;                                              // scale > 0: max commutes with the scaling
+            const float m_new = moved_max(m_run, mx);
+            // rows that have seen no key yet keep m = -inf; use 0 as the reference point so exp2 stays finite
+            const float m_use = m_new == -INFINITY ? 0.f : m_new;
+            // scale-and-subtract and the row sum on element pairs (plain fp32 instructions: packed ones are switched off in the build), exp2 per element
+            const f32x2 sc2 = {a.scale_log2, a.scale_log2}, mm2 = {-m_use, -m_use};
+            f32x2 psum2 = {0.f, 0.f};
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    const f32x2 sv = {sT[tt][r], sT[tt][r + 1]};
+                    const f32x2 z = __builtin_elementwise_fma(sv, sc2, mm2);
+                    const f32x2 e = {fast_exp2(z[0]), fast_exp2(z[1])};
+                    sT[tt][r] = e[0];
+                    sT[tt][r + 1] = e[1];
+                    psum2 += e;
+                }
+            const float psum = psum2[0] + psum2[1];
+            if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {      // some row's max moved: rescale (wave-uniform branch)
+                const float alpha = fast_exp2(m_run - m_use);            // m_run = -inf -> 0
+                l_run *= alpha;
+#pragma unroll
+                for (int t = 0; t < DT; ++t) o[t] *= alpha;
+            }
+            l_run += psum;
+            m_run = m_new;
+            // ---- O^T += V^T P^T, 32 keys at a time, P as hi + lo bf16; each V fragment is read once, used twice
 #pragma unroll
             for (int hh = 0; hh < BN / 32; ++hh) {
-                bf16x8 p_hi[QT], p_lo[QT];
-                f16x8 p16[QT];
+                bf16x8 p_hi, p_lo;
+                f16x8 p16;
+                // five VALU instructions per element PAIR: pack hi, two unpacks, one packed (exact) subtract, pack lo
+                u32x4 hraw, lraw;
 #pragma unroll
-                for (int qs = 0; qs < QT; ++qs) {
-                    // five VALU instructions per element PAIR: pack hi, two unpacks, one packed (exact) subtract, pack lo
-                    u32x4 hraw, lraw;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const f32x2 pv = {sT[qs][2 * hh + (j >> 1)][2 * (j & 1)], sT[qs][2 * hh + (j >> 1)][2 * (j & 1) + 1]};
-                        if constexpr (F16V) {
-                            hraw[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pv, f16x2v));   // v_cvt_pk_f16_f32 (round to nearest even)
-                        } else {
-                            const uint32_t hp = cvt_pk_bf16(pv[0], pv[1]);
-                            const f32x2 hf = {__builtin_bit_cast(float, hp << 16), __builtin_bit_cast(float, hp & 0xffff0000u)};
-                            const f32x2 lo = pv - hf;
-                            hraw[j] = hp;
-                            lraw[j] = cvt_pk_bf16(lo[0], lo[1]);
-                        }
-                    }
+                for (int j = 0; j < 4; ++j) {
+                    const f32x2 pv = {sT[2 * hh + (j >> 1)][2 * (j & 1)], sT[2 * hh + (j >> 1)][2 * (j & 1) + 1]};
                     if constexpr (F16V) {
-                        p16[qs] = __builtin_bit_cast(f16x8, hraw);
+                        hraw[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pv, f16x2v));   // v_cvt_pk_f16_f32 (round to nearest even)
                     } else {
-                        p_hi[qs] = *reinterpret_cast<const bf16x8*>(&hraw);
-                        p_lo[qs] = *reinterpret_cast<const bf16x8*>(&lraw);
+                        const uint32_t hp = cvt_pk_bf16(pv[0], pv[1]);
+                        const f32x2 hf = {__builtin_bit_cast(float, hp << 16), __builtin_bit_cast(float, hp & 0xffff0000u)};
+                        const f32x2 lo = pv - hf;
+                        hraw[j] = hp;
+                        lraw[j] = cvt_pk_bf16(lo[0], lo[1]);
                     }
+                }
+                if constexpr (F16V) {
+                    p16 = __builtin_bit_cast(f16x8, hraw);
+                } else {
+                    p_hi = *reinterpret_cast<const bf16x8*>(&hraw);
+                    p_lo = *reinterpret_cast<const bf16x8*>(&lraw);
                 }
                 u32x2 vlo[DT], vhi[DT];
                 if (hh == 0) {
@@ -490,8 +478,7 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
 #pragma unroll
                     for (int t = 0; t < DT; ++t) {
                         const u32x4 raw = {vlo[t][0], vlo[t][1], vhi[t][0], vhi[t][1]};
-#pragma unroll
-                        for (int qs = 0; qs < QT; ++qs) o[qs][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, raw), p16[qs], o[qs][t], 0, 0, 0);
+                        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, raw), p16, o[t], 0, 0, 0);
                     }
                 } else {
                 bf16x8 vf[DT];
@@ -500,15 +487,13 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
                     const u32x4 raw = {vlo[t][0], vlo[t][1], vhi[t][0], vhi[t][1]};
                     vf[t] = *reinterpret_cast<const bf16x8*>(&raw);
                 }
-                // all hi products, then all lo: the two MFMAs on one accumulator are QT*DT-1 independent MFMAs apart
+                // all hi products, then all lo: the two MFMAs on one accumulator are DT-1 independent MFMAs apart
 #pragma unroll
                 for (int t = 0; t < DT; ++t)
-#pragma unroll
-                    for (int qs = 0; qs < QT; ++qs) o[qs][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], p_hi[qs], o[qs][t], 0, 0, 0);
+                    o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], p_hi, o[t], 0, 0, 0);
 #pragma unroll
                 for (int t = 0; t < DT; ++t)
-#pragma unroll
-                    for (int qs = 0; qs < QT; ++qs) o[qs][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], p_lo[qs], o[qs][t], 0, 0, 0);
+                    o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], p_lo, o[t], 0, 0, 0);
                 }
             }
         }
@@ -526,54 +511,45 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
     if constexpr (KS == 2) {                                                     // sums of the second group to the first, through the images' memory
         float* at = reinterpret_cast<float*>(lds_all) + 64 * wave + lane;
         constexpr int STEP = 256;
-        static_assert((QT * (4 * DT + 2)) * STEP * 4 <= KS * 4 * IMG);
+        static_assert((4 * DT + 2) * STEP * 4 <= KS * 4 * IMG);
         if (grp == 1) {
+            float* p = at;
+            p[0] = m_run;
+            p[STEP] = l_run;
 #pragma unroll
-            for (int qs = 0; qs < QT; ++qs) {
-                float* p = at + qs * (4 * DT + 2) * STEP;
-                p[0] = m_run[qs];
-                p[STEP] = l_run[qs];
+            for (int t = 0; t < DT; ++t)
 #pragma unroll
-                for (int t = 0; t < DT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) p[(2 + 4 * t + r) * STEP] = o[qs][t][r];
-            }
+                for (int r = 0; r < 4; ++r) p[(2 + 4 * t + r) * STEP] = o[t][r];
         }
         __syncthreads();
         if (grp == 0) {
+            const float* p = at;
+            const float m1 = p[0], m = max2(m_run, m1), m_use = m == -INFINITY ? 0.f : m;
+            const float w0 = fast_exp2(m_run - m_use), w1 = fast_exp2(m1 - m_use);
+            l_run = l_run * w0 + p[STEP] * w1;
 #pragma unroll
-            for (int qs = 0; qs < QT; ++qs) {
-                const float* p = at + qs * (4 * DT + 2) * STEP;
-                const float m1 = p[0], m = max2(m_run[qs], m1), m_use = m == -INFINITY ? 0.f : m;
-                const float w0 = fast_exp2(m_run[qs] - m_use), w1 = fast_exp2(m1 - m_use);
-                l_run[qs] = l_run[qs] * w0 + p[STEP] * w1;
+            for (int t = 0; t < DT; ++t)
 #pragma unroll
-                for (int t = 0; t < DT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) o[qs][t][r] = o[qs][t][r] * w0 + p[(2 + 4 * t + r) * STEP] * w1;
-            }
+                for (int r = 0; r < 4; ++r) o[t][r] = o[t][r] * w0 + p[(2 + 4 * t + r) * STEP] * w1;
         }
         __syncthreads();
         if (grp == 1) return true;
     }
     // ---- finalise: total row sum over the 4 lane groups, normalise, store 4 contiguous dims per tile
+    float l = sum_xor16(l_run);
+    l = sum_xor32(l);
+    if (!q_ok) return true;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const int64_t orow = ((int64_t)(q_beg + my_q) * a.h + head) * D;
 #pragma unroll
-    for (int qs = 0; qs < QT; ++qs) {
-        float l = sum_xor16(l_run[qs]);
-        l = sum_xor32(l);
-        if (!q_ok[qs]) continue;
-        const float inv = l > 0.f ? 1.f / l : 0.f;
-        const int64_t orow = ((int64_t)(q_beg + my_q[qs]) * a.h + head) * D;
-#pragma unroll
-        for (int t = 0; t < DT; ++t) {
-            const int d0 = 16 * t + 4 * lg;
-            const f32x4 r = o[qs][t] * inv;
-            if (a.out_f32) {
-                *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + orow + d0) = r;
-            } else {
-                u32x2 pk = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
-                *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.out) + orow + d0) = pk;
-            }
+    for (int t = 0; t < DT; ++t) {
+        const int d0 = 16 * t + 4 * lg;
+        const f32x4 r = o[t] * inv;
+        if (a.out_f32) {
+            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + orow + d0) = r;
+        } else {
+            u32x2 pk = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
+            *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.out) + orow + d0) = pk;
         }
     }
     return true;
@@ -583,11 +559,9 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
 // handed over in `v` (NVH_PREFILL_TILED_F16V, measurement variant), 2 = nvh_prefill_varlen_pv16: fp16 P against the fp16 copy of V in `v16` UNLESS the
 // conversion launch ahead of this one flagged a 64-row group of THIS sequence's V rows (a finite |v| > 65504 does not fit fp16): then the hi + lo form
 // on the caller's own rows.  Every conversion workgroup writes its group's flag unconditionally (nothing to clear); a wave ORs the flags that cover its
-// sequence behind the first K image's DMA (GUARD above); both bodies are instantiations of the same code.
-template <int D, bool PAGED, int QT, int PV, int KS>
-__global__ __launch_bounds__(256 * KS)
-__attribute__((amdgpu_waves_per_eu(PV == 2 && D == 64 && QT == 2 ? 4 : 1)))         // (the guarded kernel at the fp16 body's 128 registers: hipcc gives it 134 otherwise)
-void prefill_varlen_kernel(const PrefillArgs a) {
+// sequence (GUARD above).
+template <int D, bool PAGED, int PV, int KS>
+__global__ __launch_bounds__(256 * KS) void prefill_varlen_kernel(const PrefillArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];          // [group][buffer][K | V]
     int qt, head, b;
     prefill_tile_of_block(a, qt, head, b);
@@ -596,18 +570,123 @@ void prefill_varlen_kernel(const PrefillArgs a) {
         PrefillArgs f = a;
         f.v = a.v16;
         f.v_row_stride = a.v16_row_stride;
-        if (!prefill_varlen_body<D, false, QT, true, true, KS>(f, lds, qt, head, b)) {
-            // the fall-back runs the one-sub-tile-per-wave body QT times over the workgroup's rows: its registers stay below the fp16 body's, so the
-            // guard costs the fast path no occupancy (D = 64, QT = 2: 128 registers = 4 waves per SIMD; the QT = 2 hi + lo body needs 136).  The
-            // abandoned K image's DMA is drained first (the exact body stages it again).
+        if (!prefill_varlen_body<D, false, true, true, KS>(f, lds, qt, head, b)) {
+            // the abandoned first tile's DMA is drained first (the exact body stages it again)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             int qt2 = qt, head2 = head, b2 = b;      // (laundered: the exact body shares no value with the abandoned one, so the fast path's registers
             asm volatile("" : "+s"(qt2), "+s"(head2), "+s"(b2));     //  are not held across the branch for its sake)
-            for (int sub = 0; sub < QT; ++sub) prefill_varlen_body<D, false, 1, false, false, KS>(a, lds, qt2 * QT + sub, head2, b2);
+            prefill_varlen_body<D, false, false, false, KS>(a, lds, qt2, head2, b2);
         }
     } else {
-        prefill_varlen_body<D, PAGED, QT, PV == 1, false, KS>(a, lds, qt, head, b);
+        prefill_varlen_body<D, PAGED, PV == 1, false, KS>(a, lds, qt, head, b);
+    }
+}
+
+// 128 query rows of one (sequence, q head) on 32 x 32 tiles (attend_walk32), four waves of 32.  Against 32 rows a wave on 16 x 16 tiles: 8 prompts of 8192 tokens, 1024 cached keys
+// each, 28 / 4 heads of 128, 264 -> 254 us; 20 of 7426, 28 / 4, 77.4 -> 71.7; 9 of 9000 behind cached keys, 7 / 1, 109 -> 100; 24 of 16384, 14 / 2 heads of 64, 60.7 -> 59.0 (there
+// vector issue binds, and the clock that power leaves).  F16V: `a.v` holds fp16 rows; GUARD as in prefill_varlen_body.
+template <int D, bool PAGED, bool F16V, bool GUARD>
+__device__ __forceinline__ bool prefill32_body(const PrefillArgs& a, unsigned char* const lds, const PromptTile& at) {
+    using Images = TileImages<D, D>;
+    constexpr int BM = 128, WR = 32, LPT = D / 8, TPI = 64 / LPT, NK = Images::NK;
+    const int head = at.head, b = at.b, q_beg = at.q_beg, sq = at.sq, k_beg = at.k_beg, sk = at.sk, q0 = at.qt * BM;
+    if (q0 >= sq) return true;
+    const int kh = head / (a.h / a.kvh), shift = sk - sq, tid = threadIdx.x;
+    const int kv_end = q0 + BM + shift < sk ? q0 + BM + shift : sk;              // keys any row of this workgroup can see
+    if (kv_end <= 0) {
+        zero_rows<D, 256>(a, q_beg + q0, sq - q0 < BM ? sq - q0 : BM, head, tid);
+        return true;
+    }
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 31, lh = lane >> 5;
+    const int wave_first_key = q0 + wave * WR + shift, wave_last_key = wave_first_key + WR - 1;
+    const int dp = lane % LPT, dr = lane / LPT;
+    const int64_t kstride = PAGED ? (int64_t)a.kvh * D : a.k_row_stride, vstride = PAGED ? (int64_t)a.kvh * D : a.v_row_stride;
+    uint32_t koff[NK], voff[NK];                     // this lane's piece of each DMA instruction of a full tile, in bytes from the tile's first row
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+        const int R = (wave * NK + j) * TPI + dr;
+        koff[j] = (uint32_t)(R * kstride + (dp ^ swz_k<D>(R)) * 8) * 2;
+        voff[j] = (uint32_t)(R * vstride + (dp ^ swz_v32<D>(R)) * 8) * 2;
+    }
+    PageNumbers pages{PAGED ? a.block_tables + (int64_t)b * a.bt_row_stride : nullptr, PAGED ? (sk - 1) / a.block_size : 0};
+    auto stage = [&](int tile, int buf) __attribute__((always_inline)) {
+        unsigned char *kimg = Images::k(lds, buf), *vimg = Images::v(lds, buf);
+        const int kv0 = tile * BN;
+        const uint16_t *kb, *vb;                     // wave-uniform bases of the tile's first key row, this kv head
+        if constexpr (PAGED) {                       // BN divides block_size: one block per tile
+            const int blk = kv0 / a.block_size;
+            const int64_t base = (((int64_t)pages.at(blk, lane) * a.block_size + (kv0 - blk * a.block_size)) * a.kvh + kh) * D;
+            kb = a.k + base;
+            vb = a.v + base;
+        } else {
+            kb = a.k + (int64_t)(k_beg + kv0) * kstride + (int64_t)kh * D;
+            vb = a.v + (int64_t)(k_beg + kv0) * vstride + (int64_t)kh * D;
+        }
+        const bool ragged = kv0 + BN > sk;           // wave-uniform: rows past the end repeat the last key (masked)
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+            uint32_t ko = koff[j], vo = voff[j];
+            if (ragged) {
+                const int R = (wave * NK + j) * TPI + dr, Rc = kv0 + R < sk ? R : sk - 1 - kv0;
+                ko = (uint32_t)(Rc * kstride + (dp ^ swz_k<D>(R)) * 8) * 2;
+                vo = (uint32_t)(Rc * vstride + (dp ^ swz_v32<D>(R)) * 8) * 2;
+            }
+            dma16_uncounted(kb, ko, kimg + (wave * NK + j) * 1024);
+            dma16_uncounted(vb, vo, vimg + (wave * NK + j) * 1024);
+        }
+    };
+    RangeFlags flags;
+    if constexpr (GUARD) {
+        if (!flags.ask(a, k_beg, k_beg + sk, lane)) return false;
+    }
+    stage(0, 0);
+    const int my_q = q0 + wave * WR + lq, pos = my_q + shift < sk - 1 ? my_q + shift : sk - 1;    // the last key this lane's query may see
+    const uint16_t* qp = a.q + (int64_t)(q_beg + (my_q < sq ? my_q : sq - 1)) * a.q_row_stride + (int64_t)head * D + lh * 8;
+    u32x4 qf[D / 16];
+#pragma unroll
+    for (int st = 0; st < D / 16; ++st) qf[st] = *reinterpret_cast<const u32x4*>(qp + st * 16);
+    if constexpr (GUARD) {
+        if (!flags.clear(a, lane)) return false;
+    }
+    attend_walk32<D, D, F16V, true>(
+        lds, (kv_end + BN - 1) / BN, a.scale_log2, -INFINITY, lane, qf, stage, [](int it) { return it * BN; },
+        [&](int key) { return key <= wave_last_key && key < sk; },
+        [&](int key, auto& s) {
+            constexpr int N = 32 * (sizeof(s) / sizeof(s[0]));
+            const int limit = pos - key - 4 * lh;
+            if (key + N - 1 > wave_first_key || key + N > sk) hide_scores(s, [&](int at) { return at <= limit; });
+        },
+        [&](f32x4 (&v)[D / 8]) {
+            if (my_q >= sq) return;
+            const int64_t at = ((int64_t)(q_beg + my_q) * a.h + head) * D + 4 * lh;
+#pragma unroll
+            for (int u = 0; u < D / 8; ++u) {
+                if (a.out_f32) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + at + 8 * u) = v[u];
+                else act_st4(reinterpret_cast<uint16_t*>(a.out) + at + 8 * u, v[u]);
+            }
+        });
+    return true;
+}
+
+template <int D, bool PAGED, int PV>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 && PV != 0 ? 4 : 2))) void prefill32_kernel(const PrefillArgs a) {
+    extern __shared__ __attribute__((aligned(512))) unsigned char lds[];
+    PromptTile at;
+    if (!prefill_tile(a, reinterpret_cast<int*>(lds), at)) return;
+    if constexpr (PV == 2) {
+        PrefillArgs f = a;
+        f.v = a.v16;
+        f.v_row_stride = a.v16_row_stride;
+        if (!prefill32_body<D, false, true, true>(f, lds, at)) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            int qt = at.qt, head = at.head, b = at.b;
+            asm volatile("" : "+s"(qt), "+s"(head), "+s"(b));        // (the exact body shares no value with the abandoned one)
+            for (int sub = 0; sub < 2; ++sub) prefill_varlen_body<D, false, false, false, 1>(a, lds, qt * 2 + sub, head, b);
+        }
+    } else {
+        prefill32_body<D, PAGED, PV == 1, false>(a, lds, at);
     }
 }
 
@@ -920,23 +999,37 @@ void prefill_short_kernel(const PrefillArgs a) {
     SK_STAMP(15);
 }
 
-template <int D, bool PAGED, int QT, int PV, int KS>
+template <int D, bool PAGED, int PV, int KS>
 int launch_one(const PrefillArgs& a, hipStream_t stream, const char* what) {
     constexpr int lds = KS * 2 * 2 * BN * D * 2;
-    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_varlen_kernel<D, PAGED, QT, PV, KS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    const dim3 grid(a.h, a.batch, (a.max_seqlen_q + 64 * QT - 1) / (64 * QT));
-    prefill_varlen_kernel<D, PAGED, QT, PV, KS><<<grid, 256 * KS, lds, stream>>>(a);
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_varlen_kernel<D, PAGED, PV, KS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    const dim3 grid(a.h, a.batch, (a.max_seqlen_q + 63) / 64);
+    prefill_varlen_kernel<D, PAGED, PV, KS><<<grid, 256 * KS, lds, stream>>>(a);
     return check_launch(what);
 }
 
-// QT sub-tiles of 16 rows a wave, KS groups of four waves
-template <int D, int QT, int KS>
+template <int D, bool PAGED, int PV>
+int launch_one32(const PrefillArgs& a, hipStream_t stream, const char* what) {
+    constexpr int lds = (int)TileImages<D, D>::BYTES;
+    prefill32_kernel<D, PAGED, PV><<<dim3(a.h, a.batch, (a.max_seqlen_q + 127) / 128), 256, lds, stream>>>(a);
+    return check_launch(what);
+}
+template <int D>
+int launch_32(const PrefillArgs& a, hipStream_t stream) {
+    if (a.kernel == 3) return launch_one32<D, false, 1>(a, stream, "prefill_varlen_f16v");
+    if (a.v16) return launch_one32<D, false, 2>(a, stream, "prefill_varlen_pv16");
+    if (a.block_tables) return launch_one32<D, true, 0>(a, stream, "prefill_varlen");
+    return launch_one32<D, false, 0>(a, stream, "prefill_varlen");
+}
+
+// 64 rows a workgroup, KS groups of four waves
+template <int D, int KS>
 int launch_q(const PrefillArgs& a, hipStream_t stream) {
-    if (a.kernel == 3) return launch_one<D, false, QT, 1, 1>(a, stream, "prefill_varlen_f16v");      // NVH_PREFILL_TILED_F16V: v holds fp16 rows (measurement variant; never paged)
+    if (a.kernel == 3) return launch_one<D, false, 1, 1>(a, stream, "prefill_varlen_f16v");      // NVH_PREFILL_TILED_F16V: v holds fp16 rows (measurement variant; never paged)
     // nvh_prefill_varlen_pv16: fp16 P V unless the conversion raised the guard
-    if (a.v16) return launch_one<D, false, QT, 2, KS>(a, stream, "prefill_varlen_pv16");
-    if (a.block_tables) return launch_one<D, true, QT, 0, KS>(a, stream, "prefill_varlen");
-    return launch_one<D, false, QT, 0, KS>(a, stream, "prefill_varlen");
+    if (a.v16) return launch_one<D, false, 2, KS>(a, stream, "prefill_varlen_pv16");
+    if (a.block_tables) return launch_one<D, true, 0, KS>(a, stream, "prefill_varlen");
+    return launch_one<D, false, 0, KS>(a, stream, "prefill_varlen");
 }
 
 // How full a launch of 64-row workgroups leaves the 256 CUs: the tiles of keys that a CU gets over those of the longest walk
@@ -978,14 +1071,6 @@ int launch_d(const PrefillArgs& a, hipStream_t stream) {
     const int rc = launch_short<D>(a, stream, taken);
     if (taken) return rc;
     if (a.kernel == 2) { set_error("prefill_varlen: the short-sequence kernel needs max_seqlen_q <= max_seqlen_k <= 128 and no block table"); return -2; }
-#ifndef NVH_PREFILL_QT2_FROM
-#define NVH_PREFILL_QT2_FROM 2048            // D = 64: two 16-row sub-tiles per wave from this many query rows on (A/B builds change it)
-#endif
-#ifndef NVH_PREFILL_QT2_FROM_PV16
-#define NVH_PREFILL_QT2_FROM_PV16 512        // ... in the fp16 P V form: its two-sub-tile body fits 128 registers = 4 waves per SIMD (same-box A/B against 2048:
-                                             // S = 512 42.5 -> 40.5 us, S = 1024 62.8 -> 58.8, S = 1536 77.8 -> 74.0; profiles/r03_prefill_qt2_pv16_ab.txt)
-#endif
-    const bool two = D == 128 ? a.max_seqlen_q > 128 : a.max_seqlen_q >= (a.v16 ? NVH_PREFILL_QT2_FROM_PV16 : NVH_PREFILL_QT2_FROM);
     // A launch that leaves CUs idle takes as long as its longest walk over the keys: half the rows a workgroup, and where even those are few two groups of waves that
     // share the walk (each tile costs more with them, and a start that nothing hides: 1024 keys at least).  us with 128 rows / 64 rows / two groups, by fill:
     // 14 / 2 heads of 64: 0.9 43 / 31 / 26.5, 1.3 61 / 47 / 38.5, 1.5 36 / 30 / 38, 2.6 77 / 65 / 70, 3.4 90 / 98 / 101; heads of 128: 7 / 1 0.4 57 / 43 / 34, 0.85 103 / 79 / 61,
@@ -993,10 +1078,14 @@ int launch_d(const PrefillArgs& a, hipStream_t stream) {
     // The rows are known where V was copied; otherwise uneven sequences are taken to have half of the longest on average (for the two groups always: which of them adds what
     // shows in the last bits, and a sequence whose V does not fit fp16 keeps those of the exact form, but for ten and more prompts of nearly one length at heads of 128 that
     // just reach the line for 128 rows).  By the longest prompt and their number, so these bits depend on what else is in the batch.
+    // 128 rows a workgroup, 32 a wave: from 129 rows on at heads of 128; at heads of 64, where a tile is little work, from 512 with fp16 P and from 2048 with exact P (from 512: 8 of
+    // 6000 tokens behind 1024 cached, 69.7 -> 80.0 us).  (Its DMA addresses rows of a tile by 32 bits of bytes.)
+    constexpr int64_t far = 1 << 24;
+    const bool two = (D == 128 ? a.max_seqlen_q > 128 : a.max_seqlen_q >= (a.v16 ? 512 : 2048)) && a.k_row_stride <= far && a.v_row_stride <= far;
     const double all = (double)a.max_seqlen_q * a.batch, guess = 0.5 * (all + a.max_seqlen_q);
-    if (two && prefill_fill(a, a.v16 && a.pv16_rows < all ? a.pv16_rows : guess) >= (D == 64 ? 3.0 : 1.8)) return launch_q<D, 2, 1>(a, stream);
-    if (a.max_seqlen_k >= 1024 && prefill_fill(a, guess) < (D == 64 ? 1.3 : 1.0)) return launch_q<D, 1, 2>(a, stream);
-    return launch_q<D, 1, 1>(a, stream);
+    if (two && prefill_fill(a, a.v16 && a.pv16_rows < all ? a.pv16_rows : guess) >= (D == 64 ? 3.0 : 1.8)) return launch_32<D>(a, stream);
+    if (a.max_seqlen_k >= 1024 && prefill_fill(a, guess) < (D == 64 ? 1.3 : 1.0)) return launch_q<D, 2>(a, stream);
+    return launch_q<D, 1>(a, stream);
 }
 
 }  // namespace

@@ -27,12 +27,20 @@ using ScanArgs = nvh_scan_desc;
 constexpr int TILE = 2048;                           // (token, channel) pairs a workgroup stages at a time
 constexpr int min3(int x, int y, int z) { return x < y ? (x < z ? x : z) : (y < z ? y : z); }
 
-// log(1 + e^z); by the series of log(1 + e) where 1 + e would round
+// log(1 + e^z) = max(z, 0) + log(1 + e), e = e^-|z|, without a branch or a selection: log(1 + e) / e on [0, 1] by its minimax polynomial of degree 8 (relative error 3e-8, 1.7e-7 with
+// 32-bit rounding)
 __device__ __forceinline__ float softplus_f(float z) {
-    const float e = fast_exp2(kLog2e * z);
-    const float small = e * (1.f - e * (1.f / 2 - e * (1.f / 3 - e * (1.f / 4 - e * (1.f / 5)))));
-    const float large = 0.6931471805599453f * __builtin_amdgcn_logf(1.f + e);  // (v_log_f32: both are always taken, a branch costs more)
-    return z > 20.f ? z : e < 0.0625f ? small : large;
+    const float e = fast_exp2(-kLog2e * __builtin_fabsf(z));
+    float p = 0.005232693627476692f;
+    p = p * e - 0.02950523979961872f;
+    p = p * e + 0.07822596281766891f;
+    p = p * e - 0.13663247227668762f;
+    p = p * e + 0.19106008112430573f;
+    p = p * e - 0.2484298199415207f;
+    p = p * e + 0.3331909775733948f;
+    p = p * e - 0.4999949336051941f;
+    p = p * e + 0.9999999403953552f;
+    return p * e + max2(z, 0.f);
 }
 
 __device__ __forceinline__ float gate_f(float z) { return z * fast_rcp(1.f + fast_exp2(-kLog2e * z)); }         // silu
@@ -249,7 +257,10 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const ScanArgs a) {
 // A row of 16 lanes is a channel, a wave four of them.  dt and dt x of 16 tokens lie one per lane of the row and reach all of it as an operand's row broadcast; a
 // token's 16 products with C are added up for 16 tokens at once, so that each lane ends with its token's y, and D x, gate and store follow there.
 // Bound by vector issue (a lane-crossing addition takes as long as two plain ones, so that a filled GPU is 6 to 13 % slower with it than with four states a lane) and, for few
-// portions, by a wave's own pace: 42 ns a token.  16384 tokens of 5 sequences, 2048 channels: 280 (segments, two passes) -> 230 us; of 16: 252 -> 198; 7000 tokens
+// portions, by a wave's own pace.  That: 35 ns a token with the step sizes computed in front of each 16 tokens and dt A multiplied by the lanes, 31 with the next 16 tokens' step sizes in
+// between and dt A from the matrix cores, one product of a 4 x 1 and a 1 x 4 matrix a row and four tokens (four waves on a SIMD, issue: 85 -> 80 ns); no token past the end is
+// told apart in the loop.  A layer of 16384 tokens of 5 sequences, 2048 channels: 195 -> 187 us.
+// Against segments in two passes: 16384 tokens of 5 sequences, 2048 channels: 280 (segments, two passes) -> 230 us; of 16: 252 -> 198; 7000 tokens
 // of 5, 4096 channels: 225 -> 161; 2400 of 9, 2048 channels: 52 -> 35.
 constexpr int ROW_TT = 64, ROW_CHN = 16, ROW_LD = ROW_TT + 4;
 
@@ -317,9 +328,11 @@ __global__ __launch_bounds__(256) void scan_rows_kernel(const ScanArgs a) {
     fetch(0);
     for (int t0 = 0; t0 < n_rows; t0 += ROW_TT) {
         const int n = n_rows - t0 < ROW_TT ? n_rows - t0 : ROW_TT;
+        // rows past the end count nothing, not even infinite ones: a step of softplus(-inf) = 0 leaves the state alone
+        if (pt >= n) r0 = low ? u32x4{0, 0, 0, 0} : u32x4{0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u};
+        if (bt >= n) rb = u32x4{0, 0, 0, 0};
         *reinterpret_cast<u32x4*>((low ? x_s : d_s) + (tid & 127) * 8) = r0;
         if (low) *reinterpret_cast<u32x4*>(z_s + tid * 8) = r1;
-        if (bt >= n) rb = u32x4{0, 0, 0, 0};                     // rows past the end count nothing, not even infinite ones
         {
             const f32x8 v = unpack8(rb);
 #pragma unroll
@@ -330,33 +343,56 @@ __global__ __launch_bounds__(256) void scan_rows_kernel(const ScanArgs a) {
         }
         __syncthreads();
         fetch(t0 + ROW_TT);
-        for (int k = 0; k < n; k += 16) {
+        // token k + st of this lane's channel: its steps, and what the output needs
+        float xv, zv, dt, dx;
+        auto steps = [&](int k, float& xv, float& zv, float& dt, float& dx) __attribute__((always_inline)) {
             const int e = (k + st) * ROW_CHN + lc;
-            const float xv = act_ld(x_s + e), zv = act_ld(z_s + e);
-            float dt = softplus_f(act_ld(d_s + e) + bias), dx = dt * xv;
-            if (k + st >= n) dt = 0.f, dx = 0.f;     // (a token past the end leaves the state alone)
+            xv = act_ld(x_s + e), zv = act_ld(z_s + e);
+            dt = softplus_f(act_ld(d_s + e) + bias);
+            dx = dt * xv;
+        };
+        steps(0, xv, zv, dt, dx);
+#pragma unroll
+        for (int k = 0; k < ROW_TT; k += 16) {
+            if (k >= n) break;
+            float xn = 0.f, zn = 0.f, dtn = 0.f, dxn = 0.f;      // the next 16 tokens', in between these ones' chain
+            if (k + 16 < ROW_TT) steps(k + 16, xn, zn, dtn, dxn);
             const float* b_row = bc_s + st * ROW_LD + k;
             float p[16];
-            auto token = [&](auto j, float b, float c) __attribute__((always_inline)) {
+            auto token = [&](auto j, float at, float b, float c) __attribute__((always_inline)) {
                 constexpr int J = decltype(j)::value;
                 float in = row_lane<J>(dx) * b;      // (the broadcast is an operand of the multiplication, as long as that is not merged into the sum)
                 asm("" : "+v"(in));
-                S = fast_exp2(row_lane<J>(dt) * A) * S + in;
+                S = fast_exp2(at) * S + in;
                 p[J] = S * c;
             };
+            f32x4 at[4], b[4], c[4];
             auto four = [&](auto q) __attribute__((always_inline)) {
                 constexpr int Q = decltype(q)::value;
-                const f32x4 b = *reinterpret_cast<const f32x4*>(b_row + 4 * Q), c = *reinterpret_cast<const f32x4*>(b_row + 16 * ROW_LD + 4 * Q);
-                token(std::integral_constant<int, 4 * Q>(), b[0], c[0]);
-                token(std::integral_constant<int, 4 * Q + 1>(), b[1], c[1]);
-                token(std::integral_constant<int, 4 * Q + 2>(), b[2], c[2]);
-                token(std::integral_constant<int, 4 * Q + 3>(), b[3], c[3]);
+                token(std::integral_constant<int, 4 * Q>(), at[Q][0], b[Q][0], c[Q][0]);
+                token(std::integral_constant<int, 4 * Q + 1>(), at[Q][1], b[Q][1], c[Q][1]);
+                token(std::integral_constant<int, 4 * Q + 2>(), at[Q][2], b[Q][2], c[Q][2]);
+                token(std::integral_constant<int, 4 * Q + 3>(), at[Q][3], b[Q][3], c[Q][3]);
             };
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                b[q] = *reinterpret_cast<const f32x4*>(b_row + 4 * q);
+                c[q] = *reinterpret_cast<const f32x4*>(b_row + 16 * ROW_LD + 4 * q);
+            }
+            // dt of tokens 4 q .. times this lane's A: block q of the row's four holds those tokens and is every block's left operand
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+            at[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(dt, A, zero, 2, 0, 0);
+            at[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(dt, A, zero, 2, 1, 0);
+            at[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(dt, A, zero, 2, 2, 0);
+            at[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(dt, A, zero, 2, 3, 0);
             four(std::integral_constant<int, 0>());
             four(std::integral_constant<int, 1>());
             four(std::integral_constant<int, 2>());
             four(std::integral_constant<int, 3>());
-            act_st(z_s + e, (row_sums(p, lane) + D * xv) * gate_f(zv));
+            __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);   // (everything asked for before the chain)
+            __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
+            act_st(z_s + (k + st) * ROW_CHN + lc, (row_sums(p, lane) + D * xv) * gate_f(zv));
+            xv = xn, zv = zn, dt = dtn, dx = dxn;
         }
         __syncthreads();
         if (low && pt < n && pc < a.inner)

@@ -284,6 +284,21 @@ def test_scan_infinite_last_row(inner, n, dtype):
     assert torch.equal(was, now)
 
 
+@pytest.mark.parametrize("dtype,n,step", [(BF16, 16, False), (BF16, 16, True), (BF16, 64, False), (F32, 16, False)])
+def test_scan_step_sizes(dtype, n, step):
+    """softplus of arguments from -80 to 80, read from the state behind one token whose x and B are 1.  Off by the argument's rounding in e^-|z| (its product with log2 e, and that constant:
+    1.5 |z| of 2^-24), e^-|z| itself (4), and the polynomial with its rounding (3), of which e is at most a factor."""
+    z = torch.cat([torch.linspace(-80, 80, 1600), torch.linspace(-0.1, 0.1, 448)])
+    one, none = torch.ones(1, z.numel(), dtype=dtype).cuda(), torch.zeros(1, z.numel(), dtype=dtype).cuda()
+    params = dict(a_log2=torch.full((z.numel(), n), -1.0).cuda(), d=z.cuda(), dt_bias=z.cuda(), w_dt=torch.zeros(z.numel(), 8, dtype=dtype).cuda())
+    state, p = torch.full((1, z.numel(), n), 30.0).cuda(), Portions([(0, 1, 0)])
+    bc = torch.ones(1, 2 * n, dtype=dtype).cuda()
+    if step: ops().scan_step(one, none[:, :8], bc, one, params, p.positions, p.slots, state)
+    else: ops().scan_chunks(one, none, bc, one, params, p.positions, p.slots, *p.chunks(64), state)
+    want = Z.softplus(f64(z))
+    assert ((f64(state[0].cpu()) - want[:, None]).abs() <= ((1.5 * f64(z).abs() + 8) * 2 ** -24 * want)[:, None]).all()
+
+
 @pytest.mark.parametrize("inner,n,rank", [(72, 5, 16), (64, 16, 64), (8192, 16, 128), (320, 30, 24), (64, 50, 8), (40, 100, 72), (24, 256, 8)])
 def test_scan_step(inner, n, rank):
     """Single tokens behind portions; many channels take several rows per workgroup."""

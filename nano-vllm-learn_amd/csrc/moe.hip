@@ -335,18 +335,42 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
     using G = GemmShape<MW, NW, MT, NT>;
     constexpr int TN = G::TN, DMA = G::DMA, OUTS = GLU ? TN / 2 : TN;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];        // [ring][TN weight rows | TM pairs][64 bytes]
-    int nt, mt;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4, wm = wave / NW, wn = wave % NW;
+    int nt, expert, first, live;
     {
-        // one XCD takes a run of the tiles, eight row tiles times the columns at a time, rows first: what runs at once shares rows and weights in its L2
+        // One XCD takes a run of the tiles: an expert's, up to eight row tiles times the columns at a time, rows first.  What runs at once shares rows and weights in its L2
+        // (eight row tiles whosever they are, as it was, share less: 12000 tokens, 32 experts of 1536, 1000 -> 955 us, 3000 385 -> 371; 1500 at 1024 wide 74 -> 73)
         const int nx = gridDim.x, tiles = a.tiles[3], total = nx * tiles, lin = (int)(blockIdx.x + gridDim.x * blockIdx.y), per = total >> 3;
         if (lin >= total) return;
         const int idx = lin < per * 8 ? (lin & 7) * per + (lin >> 3) : lin;
-        const int g = idx / (8 * nx), in = idx - g * 8 * nx, gm = tiles - 8 * g < 8 ? tiles - 8 * g : 8;
+        const int m = idx / nx, at = m - 32 + lane;  // a tile of this workgroup's expert, and 63 around it
+        const int4 t = reinterpret_cast<const int4*>(a.tiles)[at < 0 ? 0 : at < tiles ? at : tiles - 1];
+        expert = __builtin_amdgcn_readlane(t.x, 32);
+        const uint64_t same = __builtin_amdgcn_ballot_w64(at >= 0 && at < tiles && t.x == expert);
+        const int back = __builtin_clz(~(uint32_t)same | 1), ahead = __builtin_ctz(~(uint32_t)(same >> 33));
+        int t0 = m - back, n = back + 1 + ahead;     // the expert's tiles, if it has fewer than 32: lane 0's and lane 63's are not of it then
+        const bool all_seen = n < 32;
+        if (!all_seen) {                             // the eight around this one that are of it
+            const int lo = m & ~7;
+            n = (m + ahead < lo + 7 ? m + ahead : lo + 7) + 1;
+            t0 = t0 > lo ? t0 : lo;
+            n -= t0;
+        }
+        int in = idx - t0 * nx;
+        const int g = in / (8 * nx), gm = n - 8 * g < 8 ? n - 8 * g : 8;
+        in -= g * 8 * nx;
         nt = in / gm;
-        mt = 8 * g + in - nt * gm;
+        const int mine = 8 * g + in - nt * gm, of = t0 - m + 32;               // lane of the first one
+        first = __builtin_amdgcn_readlane(t.y, of + mine);
+        live = __builtin_amdgcn_readlane(t.z, of + mine);
+        // The tiles of an expert share its pairs evenly, in steps of a row of every wave's tiles, instead of all but the last being full: workgroups of one length fill the rounds
+        // that the CUs take them in better.  (1024 wide, 3000 tokens 132 -> 129 us)
+        if (all_seen && n > 1) {
+            const int all = (n - 1) * G::TM + __builtin_amdgcn_readlane(t.z, of + n - 1), each = (all + n * 16 * MW - 1) / (n * 16 * MW) * 16 * MW;
+            first += mine * (each - G::TM);
+            live = all - mine * each < each ? all - mine * each : each;
+        }
     }
-    const int expert = a.tiles[4 * mt], first = a.tiles[4 * mt + 1], live = a.tiles[4 * mt + 2];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4, wm = wave / NW, wn = wave % NW;
     const uint16_t* w = reinterpret_cast<const uint16_t*>(a.w) + (int64_t)expert * (GLU ? 2 : 1) * a.n * a.k;
     // 16-byte pieces of a row are xor-ed with 0, 2, 3, 1 for rows 0-3, 4-7, 8-11, 12-15: a 16-byte read takes lanes 0-3, 12-15 and 20-27 of 32 in one cycle, the others
     // in the next, and either set of 16 (8 rows at one column, the 8 other rows at the next one) then spreads over all banks
@@ -387,6 +411,11 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
         lds_only_barrier();
     };
     constexpr std::integral_constant<int, kRing - 2> in_flight{};
+    // Rows of pairs that do not exist are not multiplied: the waves along the rows share the tiles of 16 that there are.  (100 tokens' pairs in tiles of 256: 207 -> 179 us; in tiles of
+    // 128: 167 -> 160; of 16384 tokens, 8 tiles of 256 an expert: 1367 -> 1340, when the first waves were full and the last ones did without; shared evenly, 25 pairs an expert in tiles of
+    // 128: 162 -> 155)
+    const int part = ((live + 15) / 16 + MW - 1) / MW, row0 = 16 * wm * part;
+    const int mine = live - row0 < 16 * part ? live - row0 : 16 * part;        // pairs of this wave, from row0 on (none: <= 0)
     // the products of this wave's first MTU tiles of pairs
     auto run = [&](auto mtu) __attribute__((always_inline)) {
         constexpr int MTU = decltype(mtu)::value;
@@ -397,7 +426,7 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
         auto read = [&](int it, Operands& f) __attribute__((always_inline)) {
             const int at = (it % kRing) * G::IMG + lq * 64 + (lg ^ swz(lq)) * 16;
             const unsigned char* wimg = lds + at + wn * NT * 16 * 64;
-            const unsigned char* ximg = lds + at + (TN + wm * MT * 16) * 64;
+            const unsigned char* ximg = lds + at + (TN + row0) * 64;
 #pragma unroll
             for (int t = 0; t < NT; ++t) f.w[t] = *reinterpret_cast<const bf16x8*>(wimg + t * 16 * 64);
 #pragma unroll
@@ -437,13 +466,15 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
         }
     };
     arrive(std::integral_constant<int, kRing - 1>{});
-    // Rows of pairs that do not exist are not multiplied, in steps of half a wave's rows: the waves beside get the matrix cores.  (100 tokens' pairs in tiles of 256:
-    // 207 -> 179 us; in tiles of 128: 167 -> 160; of 16384 tokens, 8 tiles of 256 an expert: 1367 -> 1340.)
-    const int mine = live - wm * MT * 16;            // pairs from this wave's first one on
-    if (mine > MT * 8) {
+    constexpr int STEP = MT >= 4 ? MT / 4 : 1;       // (in quarters: a copy of the loop for each)
+    if (mine > (MT - STEP) * 16) {
         run(std::integral_constant<int, MT>{});
-    } else if (mine > 0) {
+    } else if (MT > 2 && mine > (MT - 2 * STEP) * 16) {
+        run(std::integral_constant<int, MT - STEP>{});
+    } else if (MT > 2 && mine > STEP * 16) {
         run(std::integral_constant<int, MT / 2>{});
+    } else if (mine > 0) {
+        run(std::integral_constant<int, STEP>{});
     } else {
         for (int it = 0; it < iters; ++it) {
             arrive(in_flight);
@@ -479,8 +510,8 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
     if (col < a.n) {                                 // (n is a multiple of 64: whole pieces)
 #pragma unroll
         for (int k = 0; k < MT * 16 * CP / 64; ++k) {
-            const int r = (k * 64 + lane) / CP, R = wm * MT * 16 + r;
-            if (R < live)
+            const int r = (k * 64 + lane) / CP, R = row0 + r;
+            if (r < mine)
                 *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(a.out) + (int64_t)a.slot_pair[first + R] * a.n + col) =
                     *reinterpret_cast<const u32x4*>(tile + r * CW * 2 + ((lane % CP) ^ (r & (CP - 1))) * 16);
         }

@@ -540,6 +540,25 @@ def test_expert_tiles_by_half_waves(tile):
             close(out[p.cuda()], f64(act)[p] @ f64(dn[e]).T, BF16, f"out {e}", slack=2)
 
 
+@pytest.mark.parametrize("tile", [64, 128, 256])
+@pytest.mark.parametrize("counts", [[300, 2500, 1, 513, 0, 4700], [1984, 64, 1985, 2049], [9000], [575, 576, 577, 0, 449]])
+def test_experts_of_many_tiles(counts, tile):
+    """Tiles that share an expert's pairs evenly: two to 31 of an expert, around 16 rows of every wave; experts of more tiles than a workgroup looks at, and where the next one begins."""
+    from nanovllm_hip import ops
+    n, k = 192, 64
+    flat = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))[torch.randperm(sum(counts), generator=torch.Generator().manual_seed(3))]
+    ids = flat.int()[:, None].cuda()
+    x, gu, dn = randn(len(flat), k, seed=1).cuda(), randn(len(counts), 2 * n, k, seed=2, scale=k ** -0.5).cuda(), randn(len(counts), k, n, seed=3, scale=n ** -0.5).cuda()
+    dispatch = ops.moe_dispatch(ids, len(counts), BF16, tile)
+    act = ops.moe_gemm(x, gu, ids, True, dispatch)
+    out = ops.moe_gemm(act, dn, ids, False, dispatch)
+    for e in range(len(counts)):
+        p = (flat == e).nonzero().flatten().cuda()
+        if len(p):
+            close(act[p], (G.silu(x[p].double() @ gu[e, :n].double().T) * (x[p].double() @ gu[e, n:].double().T)).cpu(), BF16, f"act {e}", slack=2)
+            close(out[p], (act[p].double() @ dn[e].double().T).cpu(), BF16, f"out {e}", slack=2)
+
+
 @pytest.mark.parametrize("rows,experts,top,dtype,softmax", [(1, 8, 2, BF16, True), (64, 5, 3, BF16, False), (65, 6, 1, BF16, True), (300, 16, 3, BF16, False), (900, 4, 2, BF16, True),
                                                             (1, 3, 3, F32, False), (130, 7, 2, F32, True)])
 def test_experts_in_one_call(rows, experts, top, dtype, softmax):

@@ -737,7 +737,8 @@ typedef struct nvh_moe_gemm_desc {
 } nvh_moe_gemm_desc;
 int nvh_moe_tile_rows(int pairs, int experts, int dtype);     /* for experts of about 1024 columns (nvh_moe_experts goes by its own) */
 int nvh_moe_gemm(const nvh_moe_gemm_desc* d, int dtype, void* stream);
-/* Route, dispatch (the small form up to 64 rows in bf16: none) and both products in one call: the launches of the four entries above, in their order. */
+/* Route, dispatch (the small form up to 64 rows in bf16: none) and both products in one call: the launches of the four entries above, in their order
+   (large batches: both products in one launch, the same results bit for bit). */
 typedef struct nvh_moe_experts_desc {
     const void* x;               /* [rows, cols], row stride x_stride */
     int64_t x_stride;

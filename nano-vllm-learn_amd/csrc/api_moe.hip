@@ -28,14 +28,12 @@ int nvh_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, const 
     REQUIRE(pairs > 0 && experts > 0 && experts <= kMoeMaxExperts && tile_rows > 0 && max_tiles >= pairs / tile_rows + experts, NVH_E_SHAPE,
             "moe_dispatch: %d pairs %d experts: room for %d tiles of %d", pairs, experts, max_tiles, tile_rows);
     REQUIRE(aligned16(tiles), NVH_E_ALIGN, "moe_dispatch: tiles must be 16-byte aligned");
-    return launch_moe_dispatch(slot_pair, tiles, counts, ids, pairs, experts, tile_rows, max_tiles, (hipStream_t)stream);
+    return launch_moe_dispatch(slot_pair, tiles, counts, ids, pairs, experts, tile_rows, max_tiles, nullptr, 0, (hipStream_t)stream);
 }
 
 int nvh_moe_tile_rows(int pairs, int experts, int dtype) { return pairs > 0 && experts > 0 ? moe_tile_rows(pairs, experts, 1024, dtype == NVH_F32) : 0; }
 
-int nvh_moe_gemm(const nvh_moe_gemm_desc* d, int dtype, void* stream) {
-    REQUIRE(d, NVH_E_NULL, "moe_gemm: null descriptor");
-    if (d->pairs == 0) return 0;
+static int moe_gemm_ok(const nvh_moe_gemm_desc* d, int dtype) {
     DTYPE("moe_gemm");
     REQUIRE(d->out && d->x && d->w && (d->tiles ? d->slot_pair != nullptr : d->ids != nullptr), NVH_E_NULL, "moe_gemm: null pointer");
     REQUIRE(d->pairs > 0 && d->top > 0 && d->pairs % d->top == 0 && d->experts > 0 && d->experts <= kMoeMaxExperts && d->n > 0 && d->n % 64 == 0 && d->k > 0 && d->k % 64 == 0,
@@ -45,13 +43,20 @@ int nvh_moe_gemm(const nvh_moe_gemm_desc* d, int dtype, void* stream) {
             "moe_gemm: %d tiles, or the small form with more than 64 rows", d->max_tiles);
     REQUIRE(!d->glu || (d->x_stride % 8 == 0 && d->x_stride >= d->k), NVH_E_STRIDE, "moe_gemm: row stride");
     REQUIRE(aligned16(d->out) && aligned16(d->x) && aligned16(d->w) && aligned16(d->tiles), NVH_E_ALIGN, "moe_gemm: pointers must be 16-byte aligned");
-    return launch_moe_gemm(*d, dtype == NVH_F32, (hipStream_t)stream);
+    return 0;
 }
 
-// scratch of nvh_moe_experts in 32-bit words: units of the experts | chosen experts | pairs by expert | tiles | counts
+int nvh_moe_gemm(const nvh_moe_gemm_desc* d, int dtype, void* stream) {
+    REQUIRE(d, NVH_E_NULL, "moe_gemm: null descriptor");
+    if (d->pairs == 0) return 0;
+    const int rc = moe_gemm_ok(d, dtype);
+    return rc ? rc : launch_moe_gemm(*d, dtype == NVH_F32, (hipStream_t)stream);
+}
+
+// scratch of nvh_moe_experts in 32-bit words: units of the experts | chosen experts | pairs by expert | tiles | counts | links of the launch of both products
 struct MoeScratch {
     int rows, max_tiles;                             // of a tile; tiles at most (rows 0: the small form, no tiles)
-    size_t ids, slots, tiles, counts, words;
+    size_t ids, slots, tiles, counts, links, link_words, words;
     MoeScratch(int tokens, int top, int experts, int n, int dtype) {
         const size_t pairs = (size_t)tokens * top, part = (pairs + 3) / 4 * 4;
         const bool small = dtype == NVH_BF16 && tokens <= 64;
@@ -61,7 +66,9 @@ struct MoeScratch {
         slots = ids + part;
         tiles = slots + (small ? 0 : part);
         counts = tiles + 4 * (size_t)max_tiles;
-        words = counts + (small ? 0 : (size_t)moe_dispatch_blocks((int)pairs) * experts);
+        links = counts + (small ? 0 : (size_t)moe_dispatch_blocks((int)pairs) * experts);
+        link_words = small || dtype != NVH_BF16 ? 0 : moe_links_words(rows, max_tiles);
+        words = links + link_words;
     }
 };
 static bool moe_sizes_ok(int rows, int top, int experts, int n) {
@@ -95,16 +102,23 @@ int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream) {
     g.out = at; g.x = d->x; g.x_stride = d->x_stride; g.w = d->gate_up;
     g.pairs = pairs; g.top = d->top; g.experts = d->experts; g.n = d->n; g.k = d->cols; g.glu = 1; g.limit = d->limit; g.alpha = d->alpha;
     g.ids = ids;
+    // both products in one launch: what the second one reads has lines of its own in the scratch
+    const bool both = s.link_words && ((uintptr_t)d->scratch & 127) == 0 && moe_one_launch(pairs, d->experts, d->n, d->cols, s.rows);
+    uint32_t* const links = reinterpret_cast<uint32_t*>(at + s.links);
     if (s.rows) {
-        rc = nvh_moe_dispatch(at + s.slots, at + s.tiles, at + s.counts, ids, pairs, d->experts, s.rows, s.max_tiles, stream);
+        rc = launch_moe_dispatch(at + s.slots, at + s.tiles, at + s.counts, ids, pairs, d->experts, s.rows, s.max_tiles, both ? links : nullptr, both ? s.link_words : 0, (hipStream_t)stream);
         if (rc) return rc;
         g.slot_pair = at + s.slots; g.tiles = at + s.tiles; g.tile_rows = s.rows;
         g.max_tiles = s.max_tiles - d->experts + (d->experts < pairs ? d->experts : pairs);
     }
+    nvh_moe_gemm_desc down = g;
+    down.out = d->out; down.x = at; down.w = d->down; down.n = d->cols; down.k = d->n; down.glu = 0; down.limit = down.alpha = 0.f;
+    if (both) {
+        if ((rc = moe_gemm_ok(&g, dtype)) || (rc = moe_gemm_ok(&down, dtype))) return rc;
+        return launch_moe_both(g, down, links, (hipStream_t)stream);
+    }
     rc = nvh_moe_gemm(&g, dtype, stream);
-    if (rc) return rc;
-    g.out = d->out; g.x = at; g.w = d->down; g.n = d->cols; g.k = d->n; g.glu = 0; g.limit = g.alpha = 0.f;
-    return nvh_moe_gemm(&g, dtype, stream);
+    return rc ? rc : nvh_moe_gemm(&down, dtype, stream);
 }
 
 }  // extern "C"

@@ -185,4 +185,8 @@ __device__ __forceinline__ int nth_largest(int value, int count, int nth) {
     return __builtin_ctzll(in);
 }
 
+// 16 bytes written through to memory.  (A store of more than 8 bytes reads its registers once more behind the next instruction, which must not write them: the compiler knows that
+// of its own stores, not of one in an asm statement.)
+__device__ __forceinline__ void st16_global_sc1(void* p, u32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off sc1\n s_nop 1" ::"v"(p), "v"(v) : "memory"); }
+
 }  // namespace nvh

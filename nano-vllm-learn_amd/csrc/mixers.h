@@ -41,7 +41,10 @@ int launch_norm_gate(void* out, void* packed, const void* x, const void* gate, c
 int launch_moe_route(const MoeRouteArgs& a, int f32, hipStream_t stream);
 int moe_dispatch_blocks(int pairs);
 int launch_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, const int32_t* ids, int pairs, int experts, int tile_rows, int max_tiles,
-                        hipStream_t stream);
+                        uint32_t* clear, size_t clear_words, hipStream_t stream);      // (clear: words set to zero besides)
+bool moe_one_launch(int pairs, int experts, int n, int cols, int tile_rows);
+size_t moe_links_words(int tile_rows, int max_tiles);    // of that launch
+int launch_moe_both(const MoeGemmArgs& up, const MoeGemmArgs& down, uint32_t* tickets, hipStream_t stream);
 int moe_tile_rows(int pairs, int experts, int n, int f32);
 int launch_moe_gemm(const MoeGemmArgs& a, int f32, hipStream_t stream);
 

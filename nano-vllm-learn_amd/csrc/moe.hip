@@ -2,7 +2,7 @@
 //   route     32-bit logits of a row tile against every expert (MFMA for bf16), group and expert choice, weights: one launch
 //   dispatch  pairs (row, chosen expert) sorted by expert and cut into tiles of one expert each: two launches, no host round trip
 //   gemm      expert products: gate | up with the gated unit in the epilogue, and down.  Large batches: 128 x 128 or 256 x 256 MFMA tiles over the
-//             sorted pairs, the rows gathered by the DMA that fills LDS.  At most 64 rows: every wave streams 16 weight rows once for all the rows that chose the expert.
+//             sorted pairs, the rows gathered by the DMA that fills LDS; both products in one launch where that fills the CUs better.  At most 64 rows: every wave streams 16 weight rows once for all the rows that chose the expert.
 // Outputs stay per pair; the weighted sum over a row's experts belongs to the residual add (hybrid_ops.hip).
 #include "attend_tile.h"
 #include "mixers.h"
@@ -232,11 +232,12 @@ __global__ __launch_bounds__(256) void moe_count_kernel(int32_t* __restrict__ co
 constexpr int kCountHere = 4 * DP;
 template <bool COUNTED>
 __global__ __launch_bounds__(256) void moe_scatter_kernel(int32_t* __restrict__ slot_pair, int32_t* __restrict__ tiles, const int32_t* __restrict__ counts,
-                                                          const int32_t* __restrict__ ids, int pairs, int experts, int tile_rows, int max_tiles) {
+                                                          const int32_t* __restrict__ ids, int pairs, int experts, int tile_rows, int max_tiles, uint32_t* __restrict__ clear, int clear_words) {
     __shared__ int at[kMoeMaxExperts], total[kMoeMaxExperts], start[kMoeMaxExperts], tile0[kMoeMaxExperts];
     __shared__ int n_tiles;
     constexpr int PER = DP / 256;
     const int p0 = blockIdx.x * DP;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < clear_words; i += gridDim.x * 256) clear[i] = 0;            // (for the launch behind this one)
     auto take = [&](int first, int (&id)[PER]) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < PER; ++u) {
@@ -325,52 +326,65 @@ constexpr int TK = 32, kRing = 4;
 __device__ __forceinline__ float expert_unit(const MoeGemmArgs& a, float g, float u) { return a.alpha != 0.f ? clamped_glu(g, u, a.limit, a.alpha) : silu_f(g) * u; }
 template <int MW, int NW, int MT, int NT>
 struct GemmShape {
-    static constexpr int WAVES = MW * NW, TM = MW * MT * 16, TN = NW * NT * 16, ROWS = TM + TN, IMG = ROWS * TK * 2, DMA = IMG / 1024 / WAVES;
+    static constexpr int WAVES = MW * NW, TM = MW * MT * 16, TN = NW * NT * 16, ROWS = TM + TN, STEP = MT >= 4 ? MT / 4 : 1, UNIT = MW * STEP * 16, IMG = ROWS * TK * 2, DMA = IMG / 1024 / WAVES;
     static constexpr size_t LDS = (size_t)kRing * IMG;
     static_assert(IMG % (1024 * WAVES) == 0 && NT % 2 == 0, "DMA instructions and gate/up tiles divide evenly");
 };
 
-template <bool GLU, int MW, int NW, int MT, int NT>
-__global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArgs a) {
+// A workgroup's part of a product: rows of tile mt (pairs first .. of an expert, `live` of them) and columns nt.
+struct ExpertTile {
+    int nt, mt, expert, first, live;
+};
+// The idx-th one of the row tiles lo .. hi - 1 times nx columns: an expert's, up to eight row tiles times the columns at a time, rows first.  What runs at once shares rows and weights
+// in an XCD's L2.  (Eight row tiles whosever they are share less: 12000 tokens, 32 experts of 1536, 1000 -> 955 us, 3000 385 -> 371; 1500 at 1024 wide 74 -> 73)
+// The tiles of an expert share its pairs evenly, in units of what the waves multiply at a time, instead of all but the last being full: workgroups of one length fill the rounds that the
+// CUs take them in better.  (1024 wide, 3000 tokens 132 -> 129 us.  In units of a row of every wave's tiles a tile of 240 would multiply 256, eight times an expert: 16384 tokens at
+// 2048 wide 1155 -> 1160)
+template <int TM, int UNIT>
+__device__ __forceinline__ ExpertTile find_tile(const int32_t* table, int tiles, int nx, int idx, int lo, int hi, int rows, int lane) {
+    ExpertTile to;
+    const int m = lo + idx / nx, at = m - 32 + lane; // a tile of the expert, and 63 around it
+    const int4 t = reinterpret_cast<const int4*>(table)[at < 0 ? 0 : at < tiles ? at : tiles - 1];
+    to.expert = __builtin_amdgcn_readlane(t.x, 32);
+    const uint64_t same = __builtin_amdgcn_ballot_w64(at >= 0 && at < tiles && t.x == to.expert);
+    const int back = __builtin_clz(~(uint32_t)same | 1), ahead = __builtin_ctz(~(uint32_t)(same >> 33));
+    const bool all_seen = back + 1 + ahead < 32;     // (lane 0's and lane 63's are not of it then); otherwise the eight around this one that are
+    int from = m - back, to_end = m + ahead + 1;
+    const int n = to_end - from, t0 = from;
+    if (!all_seen) {
+        from = from > (m & ~7) ? from : m & ~7;
+        to_end = to_end < (m | 7) + 1 ? to_end : (m | 7) + 1;
+    }
+    from = from > lo ? from : lo;
+    to_end = to_end < hi ? to_end : hi;
+    int in = idx - (from - lo) * nx;
+    const int span = to_end - from, groups = (span + rows - 1) / rows;
+    rows = (span + groups - 1) / groups;    // nine tiles: five and four
+    const int g = in / (rows * nx), left = span - rows * g, gm = left < rows ? left : rows;
+    in -= g * rows * nx;
+    to.nt = in / gm;
+    to.mt = from + rows * g + in - to.nt * gm;
+    to.first = __builtin_amdgcn_readlane(t.y, to.mt - m + 32);
+    to.live = __builtin_amdgcn_readlane(t.z, to.mt - m + 32);
+    if (all_seen && n > 1) {
+        const int all = (n - 1) * TM + __builtin_amdgcn_readlane(t.z, t0 + n - 1 - m + 32), each = (all + n * UNIT - 1) / (n * UNIT) * UNIT, nth = to.mt - t0;
+        to.first += nth * (each - TM);
+        to.live = all - nth * each < each ? all - nth * each : each;
+    }
+    return to;
+}
+
+// LINKED: a part of the launch of both products: what is stored for the second one goes through to memory.
+// ready(): the second product's rows are there (a barrier).  landed(): behind the barrier after it, by when all earlier stores of the workgroup have arrived.
+template <bool GLU, bool LINKED, int MW, int NW, int MT, int NT, class Ready, class Landed>
+__device__ __forceinline__ void expert_product(const MoeGemmArgs& a, const ExpertTile& to, unsigned char* lds, Ready ready, Landed landed) {
     using G = GemmShape<MW, NW, MT, NT>;
     constexpr int TN = G::TN, DMA = G::DMA, OUTS = GLU ? TN / 2 : TN;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];        // [ring][TN weight rows | TM pairs][64 bytes]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4, wm = wave / NW, wn = wave % NW;
-    int nt, expert, first, live;
-    {
-        // One XCD takes a run of the tiles: an expert's, up to eight row tiles times the columns at a time, rows first.  What runs at once shares rows and weights in its L2
-        // (eight row tiles whosever they are, as it was, share less: 12000 tokens, 32 experts of 1536, 1000 -> 955 us, 3000 385 -> 371; 1500 at 1024 wide 74 -> 73)
-        const int nx = gridDim.x, tiles = a.tiles[3], total = nx * tiles, lin = (int)(blockIdx.x + gridDim.x * blockIdx.y), per = total >> 3;
-        if (lin >= total) return;
-        const int idx = lin < per * 8 ? (lin & 7) * per + (lin >> 3) : lin;
-        const int m = idx / nx, at = m - 32 + lane;  // a tile of this workgroup's expert, and 63 around it
-        const int4 t = reinterpret_cast<const int4*>(a.tiles)[at < 0 ? 0 : at < tiles ? at : tiles - 1];
-        expert = __builtin_amdgcn_readlane(t.x, 32);
-        const uint64_t same = __builtin_amdgcn_ballot_w64(at >= 0 && at < tiles && t.x == expert);
-        const int back = __builtin_clz(~(uint32_t)same | 1), ahead = __builtin_ctz(~(uint32_t)(same >> 33));
-        int t0 = m - back, n = back + 1 + ahead;     // the expert's tiles, if it has fewer than 32: lane 0's and lane 63's are not of it then
-        const bool all_seen = n < 32;
-        if (!all_seen) {                             // the eight around this one that are of it
-            const int lo = m & ~7;
-            n = (m + ahead < lo + 7 ? m + ahead : lo + 7) + 1;
-            t0 = t0 > lo ? t0 : lo;
-            n -= t0;
-        }
-        int in = idx - t0 * nx;
-        const int g = in / (8 * nx), gm = n - 8 * g < 8 ? n - 8 * g : 8;
-        in -= g * 8 * nx;
-        nt = in / gm;
-        const int mine = 8 * g + in - nt * gm, of = t0 - m + 32;               // lane of the first one
-        first = __builtin_amdgcn_readlane(t.y, of + mine);
-        live = __builtin_amdgcn_readlane(t.z, of + mine);
-        // The tiles of an expert share its pairs evenly, in steps of a row of every wave's tiles, instead of all but the last being full: workgroups of one length fill the rounds
-        // that the CUs take them in better.  (1024 wide, 3000 tokens 132 -> 129 us)
-        if (all_seen && n > 1) {
-            const int all = (n - 1) * G::TM + __builtin_amdgcn_readlane(t.z, of + n - 1), each = (all + n * 16 * MW - 1) / (n * 16 * MW) * 16 * MW;
-            first += mine * (each - G::TM);
-            live = all - mine * each < each ? all - mine * each : each;
-        }
-    }
+    int tid = threadIdx.x;
+    if (LINKED) asm volatile("" : "+v"(tid));        // (what hangs on it is computed for each part: held over the loop around it would take too many registers)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4, wm = wave / NW, wn = wave % NW;
+    const auto same = [](int v) { return __builtin_amdgcn_readfirstlane(v); };           // (they are: inside the loop over parts the compiler does not see it)
+    const int nt = same(to.nt), expert = same(to.expert), first = same(to.first), live = same(to.live);
     const uint16_t* w = reinterpret_cast<const uint16_t*>(a.w) + (int64_t)expert * (GLU ? 2 : 1) * a.n * a.k;
     // 16-byte pieces of a row are xor-ed with 0, 2, 3, 1 for rows 0-3, 4-7, 8-11, 12-15: a 16-byte read takes lanes 0-3, 12-15 and 20-27 of 32 in one cycle, the others
     // in the next, and either set of 16 (8 rows at one column, the 8 other rows at the next one) then spreads over all banks
@@ -395,16 +409,26 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
 #pragma unroll
         for (int j = 0; j < DMA; ++j) dma16(src[j] + it * TK, lds + buf * G::IMG + (wave * DMA + j) * 1024);
     };
+    const int iters = a.k / TK;                      // (k is a multiple of 64: even)
+    // (images past the last one are asked for again: every iteration leaves the same number of loads in flight, without a branch)
+    auto stage_next = [&](int it) { stage(it < iters ? it : iters - 1, it % kRing); };
+    auto begin = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int it = 0; it < kRing; ++it) stage_next(it);
+    };
+    float start = 0.f;
+    if constexpr (!LINKED) {
+        begin();
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // (this wave's earlier stores)
+        if (!ready()) start = __uint_as_float(0x7FC00000u);                    // (a bounded wait that ended: no number)
+        begin();
+    }
     f32x4 acc[NT][MT];                               // D[weight row 16 i + 4 lg + r][pair 16 j + lq]
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int iters = a.k / TK;                      // (k is a multiple of 64: even)
-    // (images past the last one are asked for again: every iteration leaves the same number of loads in flight, without a branch)
-    auto stage_next = [&](int it) { stage(it < iters ? it : iters - 1, it % kRing); };
-#pragma unroll
-    for (int it = 0; it < kRing; ++it) stage_next(it);
+        for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{start, start, start, start};
     // the oldest image in flight has landed (`younger` behind it), and everyone has read the one before it
     auto arrive = [&](auto younger) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(younger)::value * DMA) : "memory");
@@ -466,7 +490,8 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
         }
     };
     arrive(std::integral_constant<int, kRing - 1>{});
-    constexpr int STEP = MT >= 4 ? MT / 4 : 1;       // (in quarters: a copy of the loop for each)
+    landed();
+    constexpr int STEP = G::STEP;                    // (in quarters: a copy of the loop for each)
     if (mine > (MT - STEP) * 16) {
         run(std::integral_constant<int, MT>{});
     } else if (MT > 2 && mine > (MT - 2 * STEP) * 16) {
@@ -511,10 +536,128 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
 #pragma unroll
         for (int k = 0; k < MT * 16 * CP / 64; ++k) {
             const int r = (k * 64 + lane) / CP, R = row0 + r;
-            if (r < mine)
-                *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(a.out) + (int64_t)a.slot_pair[first + R] * a.n + col) =
-                    *reinterpret_cast<const u32x4*>(tile + r * CW * 2 + ((lane % CP) ^ (r & (CP - 1))) * 16);
+            if (r < mine) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(tile + r * CW * 2 + ((lane % CP) ^ (r & (CP - 1))) * 16);
+                uint16_t* dst = reinterpret_cast<uint16_t*>(a.out) + (int64_t)a.slot_pair[first + R] * a.n + col;
+                if (GLU && LINKED) st16_global_sc1(dst, v);
+                else *reinterpret_cast<u32x4*>(dst) = v;
+            }
         }
+    }
+}
+
+template <bool GLU, int MW, int NW, int MT, int NT>
+__global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArgs a) {
+    using G = GemmShape<MW, NW, MT, NT>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];        // [ring][TN weight rows | TM pairs][64 bytes]
+    // one XCD takes a run of the parts
+    const int nx = gridDim.x, tiles = a.tiles[3], total = nx * tiles, lin = (int)(blockIdx.x + gridDim.x * blockIdx.y), per = total >> 3;
+    if (lin >= total) return;
+    const int idx = lin < per * 8 ? (lin & 7) * per + (lin >> 3) : lin;
+    expert_product<GLU, false, MW, NW, MT, NT>(a, find_tile<G::TM, G::UNIT>(a.tiles, tiles, nx, idx, 0, tiles, 8, threadIdx.x & 63), lds, [] { return true; }, [] {});
+}
+
+// Both products in one launch of workgroups that stay: the parts of the second one fill the CUs that the last round of the first one leaves idle, and the other way round at its head.
+// A row of tiles is split over eight lists, one for the workgroups of an XCD; a list is its tiles' parts of the first product and behind them those of the second one, drawn by ticket.
+// Whose list is at an end draws from the next one's.  A part of the second product waits until all columns of its row tile are stored, and those were drawn before it
+// from the same list: they are in the hands of workgroups that run, and never wait.  (No assumption on how many are resident, on their order, or on who runs where; the wait is
+// bounded all the same, and numbers of none behind it.)
+// What the second product reads is stored through to memory, announced behind the stores' arrival, and lies in lines of its own (rows of whole 128 bytes): no cache holds an older copy.
+constexpr int kListWords = 32, kWaitLimit = 1 << 22; // tickets a line each; polls of about a microsecond
+struct MoeBothArgs {
+    MoeGemmArgs up, down;
+    uint32_t* tickets;                               // [8][kListWords], zero; then per row tile its stored columns, [tiles][kListWords], zero
+};
+template <int MW, int NW, int MT, int NT>
+__global__ __launch_bounds__(64 * MW * NW) void moe_both_kernel(const MoeBothArgs a) {
+    using G = GemmShape<MW, NW, MT, NT>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    int* const next = reinterpret_cast<int*>(lds + G::LDS);                    // list (-1: at the end), number in it; whether a wait ended well
+    uint32_t* const stored = a.tickets + 8 * kListWords;
+    const int tiles = a.up.tiles[3], nx = (a.up.n + G::TN / 2 - 1) / (G::TN / 2), ny = (a.down.n + G::TN - 1) / G::TN;
+    const int rows = tiles < 128 ? 4 : 8;
+    const auto begin = [&](int list) { return (int)((int64_t)tiles * list >> 3); };
+    const auto parts = [&](int list) { return (begin(list + 1) - begin(list)) * (nx + ny); };
+    const auto draw = [&](int list) {                // (a wave)
+        uint32_t t = 0;
+        if ((threadIdx.x & 63) == 0) t = __hip_atomic_fetch_add(a.tickets + list * kListWords, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return t;
+    };
+    const auto settle = [&](int list, uint32_t ticket) {                       // (a wave) that ticket, or one of the first later list that has any
+        int number = __builtin_amdgcn_readfirstlane(ticket);
+        if (number >= parts(list)) {                 // (all lists' tickets at once, one per lane: what is at an end stays there)
+            const uint32_t seen = __hip_atomic_load(a.tickets + (threadIdx.x & 7) * kListWords, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t open = (uint32_t)__builtin_amdgcn_ballot_w64((int)seen < parts(threadIdx.x & 7)) & 0xFF;
+            uint32_t later = (open | open << 8) >> (list + 1) & 0x7F;          // list + 1, list + 2, ..
+            const int was = list;
+            list = -1;
+            while (later) {
+                const int next_one = (was + 1 + __builtin_ctz(later)) & 7;
+                number = __builtin_amdgcn_readfirstlane(draw(next_one));
+                if (number < parts(next_one)) {
+                    list = next_one;
+                    break;
+                }
+                later &= later - 1;
+            }
+        }
+        if ((threadIdx.x & 63) == 0) {
+            next[0] = list;
+            next[1] = number;
+        }
+    };
+    if (threadIdx.x < 64) settle(blockIdx.x & 7, draw(blockIdx.x & 7));
+    int announce = -1;                               // a row tile whose columns are on their way to memory
+    const auto announce_it = [&]() {
+        if (announce >= 0) __hip_atomic_fetch_add(stored + announce * kListWords, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    while (true) {
+        lds_only_barrier();                          // (the next part is known, and the images are done with)
+        const int list = __builtin_amdgcn_readfirstlane(next[0]), number = __builtin_amdgcn_readfirstlane(next[1]);
+        if (list < 0) break;
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63;
+        const int lo = begin(list), hi = begin(list + 1), first = (hi - lo) * nx;
+        // The part behind it: drawn beside the look into the table.  (Behind the first images instead, these are held up: loads arrive in the order in which they were asked for.)
+        uint32_t drawn = 0;
+        if (tid < 64 && number < first) drawn = draw(list);
+        const auto landed = [&]() {
+            if (tid < 64) {
+                if (tid == 0) announce_it();
+                settle(list, drawn);
+            }
+        };
+        if (number < first) {
+            const ExpertTile to = find_tile<G::TM, G::UNIT>(a.up.tiles, tiles, nx, number, lo, hi, rows, lane);
+            expert_product<true, true, MW, NW, MT, NT>(a.up, to, lds, [] { return true; }, landed);
+            announce = to.mt;
+        } else {
+            if (announce >= 0) {                     // before it waits for anyone
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                lds_only_barrier();
+                if (tid == 0) announce_it();
+                announce = -1;
+            }
+            const ExpertTile to = find_tile<G::TM, G::UNIT>(a.up.tiles, tiles, ny, number - first, lo, hi, rows, lane);
+            const uint32_t* const word = stored + to.mt * kListWords;
+            const auto ready = [&]() {
+                if (tid == 0) {
+                    int tries = 0;
+                    while (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (uint32_t)nx && ++tries < kWaitLimit) __builtin_amdgcn_s_sleep(8);
+                    next[2] = tries < kWaitLimit;
+                }
+                if (tid < 64) drawn = draw(list);    // (not before: a workgroup that waits keeps no other part waiting)
+                lds_only_barrier();
+                return next[2] != 0;
+            };
+            expert_product<false, true, MW, NW, MT, NT>(a.down, to, lds, ready, landed);
+        }
+    }
+    if (announce >= 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_only_barrier();
+        if (threadIdx.x == 0) announce_it();
     }
 }
 
@@ -716,16 +859,16 @@ int launch_moe_route(const MoeRouteArgs& a, int f32, hipStream_t stream) {
 int moe_dispatch_blocks(int pairs) { return (pairs + DP - 1) / DP; }
 
 int launch_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, const int32_t* ids, int pairs, int experts, int tile_rows, int max_tiles,
-                        hipStream_t stream) {
+                        uint32_t* clear, size_t clear_words, hipStream_t stream) {
     const int grid = moe_dispatch_blocks(pairs);
     if (pairs <= kCountHere) {
-        moe_scatter_kernel<false><<<grid, 256, 0, stream>>>(slot_pair, tiles, counts, ids, pairs, experts, tile_rows, max_tiles);
+        moe_scatter_kernel<false><<<grid, 256, 0, stream>>>(slot_pair, tiles, counts, ids, pairs, experts, tile_rows, max_tiles, clear, (int)clear_words);
         return check_launch("moe_scatter");
     }
     moe_count_kernel<<<grid, 256, 0, stream>>>(counts, ids, pairs, experts);
     const int rc = check_launch("moe_count");
     if (rc) return rc;
-    moe_scatter_kernel<true><<<grid, 256, 0, stream>>>(slot_pair, tiles, counts, ids, pairs, experts, tile_rows, max_tiles);
+    moe_scatter_kernel<true><<<grid, 256, 0, stream>>>(slot_pair, tiles, counts, ids, pairs, experts, tile_rows, max_tiles, clear, (int)clear_words);
     return check_launch("moe_scatter");
 }
 
@@ -745,6 +888,39 @@ int moe_tile_rows(int pairs, int experts, int n, int f32) {
     if (mean <= 16 || (mean <= 25 && wide < 49152)) return 64;
     const bool large = mean >= 288 ? true : mean >= 256 ? wide >= 49152 : mean > 240 ? false : mean >= 193 ? wide >= 24576 : mean >= 110 || (mean >= 100 && wide >= 98304);
     return large ? 256 : 128;
+}
+
+// compute units of the current device (256 on MI355X), read once
+static int device_cus() {
+    static const int n = [] {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
+        return v;
+    }();
+    return n;
+}
+
+// Whether both products go in one launch: tiles of 256 rows (a workgroup a CU) that are enough, as far as the pairs tell, for two and a half rounds of the CUs, and a second product
+// whose parts, which come last, are not the longer ones.  us at 32 experts, four routes each, two launches against one: 2048 wide, experts of 1536, 130 pairs an expert (2.5
+// rounds) 199 against 198, 190 246 against 211, 220 247 against 214, 290 286 against 271, 375 329 against 310, 430 384 against 340, 600 453 against 433, 1000 688 against 661;
+// 1024 wide, of 768, 240 (1.8) 84 against 102, 290 (2.0) 102 against 104, 375 (2.4) 109 against 111, 400 (2.6) 123 against 111, 460 131 against 113, 1000 234 against 205.
+// 4096 wide, of 512, 375 pairs 304 against 258.  Where the parts of either product are just whole rounds, one launch takes up to 3 % longer; 768 wide, of 2048, 16 experts of 600 pairs:
+// 154 against 167.  From 20 rounds on the idle ends are little against what each part's hand-over costs: 2048 wide, 16384 tokens by sigmoids 1151 against 1156 (12000, 16 rounds, 982
+// against 960).  Tiles of 128 rows, two workgroups a CU, fill their rounds better as they are: 32 experts of 2048 and 1536, 60 pairs 158 against 164.
+bool moe_one_launch(int pairs, int experts, int n, int cols, int tile_rows) {
+    if (tile_rows != 256 || n > cols) return false;
+    const int64_t tiles = pairs / 256 + experts / 2, parts = tiles * ((n + 127) / 128 + (cols + 255) / 256);
+    return 2 * parts >= 5 * device_cus() && parts < 20 * device_cus();
+}
+size_t moe_links_words(int tile_rows, int max_tiles) { return tile_rows == 256 ? (size_t)(8 + max_tiles) * kListWords : 0; }
+
+int launch_moe_both(const MoeGemmArgs& up, const MoeGemmArgs& down, uint32_t* tickets, hipStream_t stream) {
+    using G = GemmShape<2, 4, 8, 4>;
+    const size_t lds = G::LDS + 16;
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(moe_both_kernel<2, 4, 8, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const int64_t parts = (int64_t)up.max_tiles * ((up.n + G::TN / 2 - 1) / (G::TN / 2) + (down.n + G::TN - 1) / G::TN);
+    moe_both_kernel<2, 4, 8, 4><<<(int)(parts < device_cus() ? parts : device_cus()), 64 * G::WAVES, lds, stream>>>(MoeBothArgs{up, down, tickets});
+    return check_launch("moe_both");
 }
 
 int launch_moe_gemm(const MoeGemmArgs& a, int f32, hipStream_t stream) {

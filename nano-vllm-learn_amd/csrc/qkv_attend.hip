@@ -48,10 +48,6 @@ struct QkvAttendArgs {
     int bs_shift;                // log2(block_size) or -1
 };
 
-__device__ __forceinline__ void st16_global_sc1(void* p, u32x4 v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
-}
-
 // Diagnostic build only (-DNVH_STAMPS, tools/probes/stamp_qkv_attend.py): clock stamps of the producer role, [tile][wave][8], behind the
 // consumers' region of the debug buffer.  Never compiled into the shipped library.
 #ifdef NVH_STAMPS

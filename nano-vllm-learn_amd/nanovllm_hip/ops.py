@@ -1494,7 +1494,7 @@ def moe_gemm(x, weight, ids, glu, dispatch=None, unit=None):
 
 def moe_experts(x, router, correction, gate_up, down, top, groups=1, keep=1, scale=1.0, softmax=False, unit=None):
     """(expert outputs [rows * top, cols], weights fp32 [rows, top]): moe_route, moe_dispatch (up to LINEAR_SMALL_M_MAX rows in bf16: none) and both moe_gemm in one
-    call, the same launches.  (Four calls with a descriptor each took the host 40 to 59 us, more than the kernels of up to some 400
+    call: the same launches, or, where many tiles of 256 rows fill the GPU better so, both products in one, with the same bits.  (Four calls with a descriptor each took the host 40 to 59 us, more than the kernels of up to some 400
     tokens at 1024 wide; this one takes 22 to 29: 5 tokens 38.5 -> 25 us a pass, 100 55 -> 41.)"""
     code = _act_code(x, router, gate_up, down)
     _require_f32(correction=correction)

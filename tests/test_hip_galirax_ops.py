@@ -591,6 +591,39 @@ def test_experts_in_one_call(rows, experts, top, dtype, softmax):
     assert out.shape == (0, cols) and weights.shape == (0, top)
 
 
+@pytest.mark.parametrize("rows,experts,top,cols,n", [(9000, 24, 4, 1024, 64), (3100, 33, 4, 2048, 320), (11000, 3, 2, 1536, 192), (4100, 9, 3, 2240, 640)])
+def test_experts_in_one_launch(rows, experts, top, cols, n):
+    """Enough tiles for both products to share a launch: bit for bit two launches, alone, two calls at once on two streams, and from a graph with other rows behind it.  Experts of a few
+    tiles and of more than a workgroup looks at; columns of either product that end inside a tile."""
+    from nanovllm_hip import ops
+    xs = [randn(rows, cols, seed=s).cuda() for s in (1, 2)]
+    router, bias = randn(experts, cols, seed=3, scale=cols ** -0.5).cuda(), randn(experts, seed=4, dtype=F32).cuda()
+    gu, dn = (randn(experts, *shape, seed=5, scale=shape[1] ** -0.5).cuda() for shape in ((2 * n, cols), (cols, n)))
+
+    def four(x):
+        ids, _ = ops.moe_route(x, router, bias, top)
+        dispatch = ops.moe_dispatch(ids, experts, BF16, 256)
+        return ops.moe_gemm(ops.moe_gemm(x, gu, ids, True, dispatch), dn, ids, False, dispatch)
+    want = [four(x) for x in xs]
+    assert torch.equal(ops.moe_experts(xs[0], router, bias, gu, dn, top)[0], want[0])
+    streams, got = [torch.cuda.Stream() for _ in xs], [[], []]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for i, stream in enumerate(streams):
+            with torch.cuda.stream(stream):
+                got[i].append(ops.moe_experts(xs[i], router, bias, gu, dn, top)[0])
+    torch.cuda.synchronize()
+    assert all(torch.equal(g, want[i]) for i in (0, 1) for g in got[i])
+    x, graph = xs[0].clone(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        kept, _ = ops.moe_experts(x, router, bias, gu, dn, top)
+    for i in (1, 0, 1):
+        x.copy_(xs[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(kept, want[i])
+
+
 # ------------------------------------------------------------------------------------------------ residual, norm, cap
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,cols,n,top", [(3, 64, 64, 0), (5, 320, 300, 4), (17, 2048, 2048, 8), (2, 8192, 8190, 3)])

@@ -343,7 +343,13 @@ struct ExpertTile {
 template <int TM, int UNIT>
 __device__ __forceinline__ ExpertTile find_tile(const int32_t* table, int tiles, int nx, int idx, int lo, int hi, int rows, int lane) {
     ExpertTile to;
-    const int m = lo + idx / nx, at = m - 32 + lane; // a tile of the expert, and 63 around it
+    const int m = lo + idx / nx;
+    {   // the only tile of its expert: nothing to order or share (100 tokens, 32 experts, a call 39.8 -> 39.4 us)
+        const int4 own = reinterpret_cast<const int4*>(table)[m];
+        const int before = table[4 * (m ? m - 1 : 0)], behind = table[4 * (m + 1 < tiles ? m + 1 : m)];
+        if ((!m || before != own.x) && (m + 1 == tiles || behind != own.x)) return ExpertTile{idx - (m - lo) * nx, m, own.x, own.y, own.z};
+    }
+    const int at = m - 32 + lane;                    // a tile of the expert, and 63 around it
     const int4 t = reinterpret_cast<const int4*>(table)[at < 0 ? 0 : at < tiles ? at : tiles - 1];
     to.expert = __builtin_amdgcn_readlane(t.x, 32);
     const uint64_t same = __builtin_amdgcn_ballot_w64(at >= 0 && at < tiles && t.x == to.expert);
@@ -374,57 +380,65 @@ __device__ __forceinline__ ExpertTile find_tile(const int32_t* table, int tiles,
     return to;
 }
 
-// LINKED: a part of the launch of both products: what is stored for the second one goes through to memory.
-// ready(): the second product's rows are there (a barrier).  landed(): behind the barrier after it, by when all earlier stores of the workgroup have arrived.
-template <bool GLU, bool LINKED, int MW, int NW, int MT, int NT, class Ready, class Landed>
-__device__ __forceinline__ void expert_product(const MoeGemmArgs& a, const ExpertTile& to, unsigned char* lds, Ready ready, Landed landed) {
-    using G = GemmShape<MW, NW, MT, NT>;
-    constexpr int TN = G::TN, DMA = G::DMA, OUTS = GLU ? TN / 2 : TN;
-    int tid = threadIdx.x;
-    if (LINKED) asm volatile("" : "+v"(tid));        // (what hangs on it is computed for each part: held over the loop around it would take too many registers)
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & 15, lg = lane >> 4, wm = wave / NW, wn = wave % NW;
-    const auto same = [](int v) { return __builtin_amdgcn_readfirstlane(v); };           // (they are: inside the loop over parts the compiler does not see it)
-    const int nt = same(to.nt), expert = same(to.expert), first = same(to.first), live = same(to.live);
-    const uint16_t* w = reinterpret_cast<const uint16_t*>(a.w) + (int64_t)expert * (GLU ? 2 : 1) * a.n * a.k;
-    // 16-byte pieces of a row are xor-ed with 0, 2, 3, 1 for rows 0-3, 4-7, 8-11, 12-15: a 16-byte read takes lanes 0-3, 12-15 and 20-27 of 32 in one cycle, the others
-    // in the next, and either set of 16 (8 rows at one column, the 8 other rows at the next one) then spreads over all banks
-    auto swz = [](int r) { return (0x78 >> ((r >> 1) & 6)) & 3; };
-    // this lane's piece of each DMA instruction: 16 rows of 64 bytes
-    const uint16_t* src[DMA];
+// 16-byte pieces of an image's row are xor-ed with 0, 2, 3, 1 for rows 0-3, 4-7, 8-11, 12-15: a 16-byte read takes lanes 0-3, 12-15 and 20-27 of 32 in one cycle, the others
+// in the next, and either set of 16 (8 rows at one column, the 8 other rows at the next one) then spreads over all banks
+__device__ __forceinline__ int image_swizzle(int r) { return (0x78 >> ((r >> 1) & 6)) & 3; }
+
+// What a lane asks for: its piece of each DMA instruction of an image, 16 rows of 64 bytes.  A wave whose pieces are of pairs that do not exist leaves them out (weights come first).
+template <class G>
+struct ExpertFeed {
+    const uint16_t* src[G::DMA];
+    bool feeds;
+    __device__ __forceinline__ void aim(bool glu, const MoeGemmArgs& a, const ExpertTile& to, int wave, int lane) {
+        const uint16_t* w = reinterpret_cast<const uint16_t*>(a.w) + (int64_t)to.expert * (glu ? 2 : 1) * a.n * a.k;
+        const int col0 = to.nt * (glu ? G::TN / 2 : G::TN);
 #pragma unroll
-    for (int j = 0; j < DMA; ++j) {
-        const int R = (wave * DMA + j) * 16 + (lane >> 2), piece = ((lane & 3) ^ swz(R)) * 8;
-        if (R < TN) {
-            int col = nt * OUTS + (GLU ? (R >> 5) * 16 + (R & 15) : R);
-            if (col >= a.n) col = a.n - 1;
-            src[j] = w + (int64_t)(GLU && (R & 16) ? a.n + col : col) * a.k + piece;
-        } else {
-            const int r = R - TN, pair = a.slot_pair[first + (r < live ? r : live - 1)];
-            src[j] = reinterpret_cast<const uint16_t*>(a.x) + (GLU ? (int64_t)(pair / a.top) * a.x_stride : (int64_t)pair * a.k) + piece;
+        for (int j = 0; j < G::DMA; ++j) {
+            const int R = (wave * G::DMA + j) * 16 + (lane >> 2), piece = ((lane & 3) ^ image_swizzle(R)) * 8;
+            if (R < G::TN) {
+                int col = col0 + (glu ? (R >> 5) * 16 + (R & 15) : R);
+                if (col >= a.n) col = a.n - 1;
+                src[j] = w + (int64_t)(glu && (R & 16) ? a.n + col : col) * a.k + piece;
+            } else {
+                const int r = R - G::TN, pair = a.slot_pair[to.first + (r < to.live ? r : to.live - 1)];
+                src[j] = reinterpret_cast<const uint16_t*>(a.x) + (glu ? (int64_t)(pair / a.top) * a.x_stride : (int64_t)pair * a.k) + piece;
+            }
         }
+        feeds = wave * G::DMA * 16 < G::TN + to.live;
     }
-    const bool feeds = wave * DMA * 16 < TN + live;  // a wave whose pieces are of pairs that do not exist leaves them out (weights come first)
-    auto stage = [&](int it, int buf) {
+    __device__ __forceinline__ void stage(unsigned char* lds, int it, int buf, int wave) const {
         if (!feeds) return;
 #pragma unroll
-        for (int j = 0; j < DMA; ++j) dma16(src[j] + it * TK, lds + buf * G::IMG + (wave * DMA + j) * 1024);
-    };
-    const int iters = a.k / TK;                      // (k is a multiple of 64: even)
-    // (images past the last one are asked for again: every iteration leaves the same number of loads in flight, without a branch)
-    auto stage_next = [&](int it) { stage(it < iters ? it : iters - 1, it % kRing); };
-    auto begin = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int it = 0; it < kRing; ++it) stage_next(it);
-    };
-    float start = 0.f;
-    if constexpr (!LINKED) {
-        begin();
-    } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // (this wave's earlier stores)
-        if (!ready()) start = __uint_as_float(0x7FC00000u);                    // (a bounded wait that ended: no number)
-        begin();
+        for (int j = 0; j < G::DMA; ++j) dma16(src[j] + it * TK, lds + buf * G::IMG + (wave * G::DMA + j) * 1024);
     }
-    f32x4 acc[NT][MT];                               // D[weight row 16 i + 4 lg + r][pair 16 j + lq]
+    // (images past the last one are asked for again: every iteration leaves the same number of loads in flight, without a branch)
+    __device__ __forceinline__ void stage_next(unsigned char* lds, int it, int iters, int wave) const { stage(lds, it < iters ? it : iters - 1, it % kRing, wave); }
+    __device__ __forceinline__ void begin(unsigned char* lds, int iters, int wave) const {
+#pragma unroll
+        for (int it = 0; it < kRing; ++it) stage_next(lds, it, iters, wave);
+    }
+};
+
+// Rows of pairs that do not exist are not multiplied: the waves along the rows share the tiles of 16 that there are.  (100 tokens' pairs in tiles of 256: 207 -> 179 us; in tiles of
+// 128: 167 -> 160; of 16384 tokens, 8 tiles of 256 an expert: 1367 -> 1340, when the first waves were full and the last ones did without; shared evenly, 25 pairs an expert in tiles of
+// 128: 162 -> 155)
+struct WaveRows {
+    int row0, mine;                                  // pairs of a wave, from row0 on (none: <= 0)
+    __device__ __forceinline__ WaveRows(int live, int wm, int waves) {
+        const int part = ((live + 15) / 16 + waves - 1) / waves;
+        row0 = 16 * wm * part;
+        mine = live - row0 < 16 * part ? live - row0 : 16 * part;
+    }
+};
+
+// D[weight row 16 i + 4 lg + r][pair 16 j + lq] of a wave, behind start (0); the images have been begun.
+// landed(): behind the barrier after the first image.  fourth(): behind that after the fourth, by when all that was stored in front of the fifth's loads has arrived.
+template <int MW, int NW, int MT, int NT, class Landed, class Fourth>
+__device__ __forceinline__ void expert_sums(f32x4 (&acc)[NT][MT], const ExpertFeed<GemmShape<MW, NW, MT, NT>>& feed, unsigned char* lds, int iters, const WaveRows& rows, int wave, int lane,
+                                            float start, Landed landed, Fourth fourth) {
+    using G = GemmShape<MW, NW, MT, NT>;
+    constexpr int TN = G::TN, DMA = G::DMA;
+    const int lq = lane & 15, lg = lane >> 4, wn = wave % NW, mine = rows.mine;
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -435,11 +449,8 @@ __device__ __forceinline__ void expert_product(const MoeGemmArgs& a, const Exper
         lds_only_barrier();
     };
     constexpr std::integral_constant<int, kRing - 2> in_flight{};
-    // Rows of pairs that do not exist are not multiplied: the waves along the rows share the tiles of 16 that there are.  (100 tokens' pairs in tiles of 256: 207 -> 179 us; in tiles of
-    // 128: 167 -> 160; of 16384 tokens, 8 tiles of 256 an expert: 1367 -> 1340, when the first waves were full and the last ones did without; shared evenly, 25 pairs an expert in tiles of
-    // 128: 162 -> 155)
-    const int part = ((live + 15) / 16 + MW - 1) / MW, row0 = 16 * wm * part;
-    const int mine = live - row0 < 16 * part ? live - row0 : 16 * part;        // pairs of this wave, from row0 on (none: <= 0)
+    int two = 2;
+    asm("" : "+s"(two));                             // (not a loop peeled for it)
     // the products of this wave's first MTU tiles of pairs
     auto run = [&](auto mtu) __attribute__((always_inline)) {
         constexpr int MTU = decltype(mtu)::value;
@@ -448,9 +459,9 @@ __device__ __forceinline__ void expert_product(const MoeGemmArgs& a, const Exper
         };
         Operands even, odd;                          // of the image being multiplied and of the next one, read meanwhile
         auto read = [&](int it, Operands& f) __attribute__((always_inline)) {
-            const int at = (it % kRing) * G::IMG + lq * 64 + (lg ^ swz(lq)) * 16;
+            const int at = (it % kRing) * G::IMG + lq * 64 + (lg ^ image_swizzle(lq)) * 16;
             const unsigned char* wimg = lds + at + wn * NT * 16 * 64;
-            const unsigned char* ximg = lds + at + (TN + row0) * 64;
+            const unsigned char* ximg = lds + at + (TN + rows.row0) * 64;
 #pragma unroll
             for (int t = 0; t < NT; ++t) f.w[t] = *reinterpret_cast<const bf16x8*>(wimg + t * 16 * 64);
 #pragma unroll
@@ -478,13 +489,14 @@ __device__ __forceinline__ void expert_product(const MoeGemmArgs& a, const Exper
         read(0, even);
         for (int it = 0; it < iters; it += 2) {
             arrive(in_flight);
+            if (it == two) fourth();
             read(it + 1, odd);
-            stage_next(it + kRing);
+            feed.stage_next(lds, it + kRing, iters, wave);
             multiply(even);
             spread();
             arrive(in_flight);
             read(it + 2, even);                      // (behind the last image: read and not used)
-            stage_next(it + 1 + kRing);
+            feed.stage_next(lds, it + 1 + kRing, iters, wave);
             multiply(odd);
             spread();
         }
@@ -503,44 +515,68 @@ __device__ __forceinline__ void expert_product(const MoeGemmArgs& a, const Exper
     } else {
         for (int it = 0; it < iters; ++it) {
             arrive(in_flight);
-            stage_next(it + kRing);
+            if (it == two) fourth();
+            feed.stage_next(lds, it + kRing, iters, wave);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // ---- results through LDS (the images are done with): a wave's MT * 16 pairs by CW columns, then whole rows of them to memory
-    lds_only_barrier();
-    if (mine <= 0) return;
-    constexpr int CW = GLU ? NT * 8 : NT * 16, CP = CW / 8;                    // columns of a wave, 16-byte pieces of a row
-    unsigned char* tile = lds + wave * MT * 16 * CW * 2;
-    auto put = [&](int r, int col, f32x4 v) {        // columns col .. + 3 of row r
-        act_st4(reinterpret_cast<uint16_t*>(tile + r * CW * 2 + (((col >> 3) ^ (r & (CP - 1))) * 16 + (col & 4) * 2)), v);
-    };
+    lds_only_barrier();                              // the images are done with
+}
+
+// Results through LDS (2048 bytes a wave, room), 16 or 32 rows at a time, and whole rows of the wave's columns to memory.  THROUGH: past the caches.  (All rows at once, with what names
+// their places loaded behind: 2048 wide, 16384 tokens 1182 -> 1167 us)
+// between(h): before the first, the third and the fifth eighth of them.
+template <bool GLU, bool THROUGH, int MW, int NW, int MT, int NT, class Between>
+__device__ __forceinline__ void expert_results(const f32x4 (&acc)[NT][MT], const MoeGemmArgs& a, const ExpertTile& to, const WaveRows& rows, unsigned char* room, int wave, int lane,
+                                               Between between) {
+    using G = GemmShape<MW, NW, MT, NT>;
+    constexpr int CW = GLU ? NT * 8 : NT * 16, CP = CW / 8, PR = 1024 / CW, PASSES = MT * 16 / PR;      // columns of a wave, 16-byte pieces of a row; rows of a pass
+    static_assert(PR % 16 == 0 && PR * CP == 128 && PASSES >= 1, "two pieces a lane and pass");
+    const int lq = lane & 15, lg = lane >> 4, wn = wave % NW, mine = rows.mine;
+    const int col = to.nt * (GLU ? G::TN / 2 : G::TN) + wn * CW + (lane % CP) * 8;
+    int pair[2 * PASSES];
 #pragma unroll
-    for (int j = 0; j < MT; ++j) {
-        if constexpr (GLU) {
-#pragma unroll
-            for (int i = 0; i < NT / 2; ++i) {
-                f32x4 v;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = expert_unit(a, acc[2 * i][j][r], acc[2 * i + 1][j][r]);
-                put(16 * j + lq, 16 * i + 4 * lg, v);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < NT; ++i) put(16 * j + lq, 16 * i + 4 * lg, acc[i][j]);
-        }
+    for (int k = 0; k < 2 * PASSES; ++k) {
+        const int r = (k * 64 + lane) / CP;
+        pair[k] = a.slot_pair[to.first + (mine > 0 ? rows.row0 + (r < mine ? r : mine - 1) : 0)];
     }
-    wave_lds_sync();
-    const int col = nt * OUTS + wn * CW + (lane % CP) * 8;
-    if (col < a.n) {                                 // (n is a multiple of 64: whole pieces)
 #pragma unroll
-        for (int k = 0; k < MT * 16 * CP / 64; ++k) {
-            const int r = (k * 64 + lane) / CP, R = row0 + r;
-            if (r < mine) {
-                const u32x4 v = *reinterpret_cast<const u32x4*>(tile + r * CW * 2 + ((lane % CP) ^ (r & (CP - 1))) * 16);
-                uint16_t* dst = reinterpret_cast<uint16_t*>(a.out) + (int64_t)a.slot_pair[first + R] * a.n + col;
-                if (GLU && LINKED) st16_global_sc1(dst, v);
-                else *reinterpret_cast<u32x4*>(dst) = v;
+    for (int p = 0; p < PASSES; ++p) {
+        if (8 * p % (2 * PASSES) == 0 && 8 * p / (2 * PASSES) < 3) between(8 * p / (2 * PASSES));
+        if (mine <= p * PR) continue;
+#pragma unroll
+        for (int jj = 0; jj < PR / 16; ++jj) {
+            const int j = p * (PR / 16) + jj, r = 16 * jj + lq;
+            auto put = [&](int c, f32x4 v) {         // columns c .. + 3 of row r
+                act_st4(reinterpret_cast<uint16_t*>(room + r * CW * 2 + (((c >> 3) ^ (r & (CP - 1))) * 16 + (c & 4) * 2)), v);
+            };
+            if constexpr (GLU) {
+#pragma unroll
+                for (int i = 0; i < NT / 2; ++i) {
+                    f32x4 v;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = expert_unit(a, acc[2 * i][j][q], acc[2 * i + 1][j][q]);
+                    put(16 * i + 4 * lg, v);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < NT; ++i) put(16 * i + 4 * lg, acc[i][j]);
+            }
+        }
+        wave_lds_sync();
+        u32x4 v[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int r = (k * 64 + lane) / CP;
+            v[k] = *reinterpret_cast<const u32x4*>(room + r * CW * 2 + ((lane % CP) ^ (r & (CP - 1))) * 16);
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (p * PR + (k * 64 + lane) / CP < mine && col < a.n) {           // (n is a multiple of 64: whole pieces)
+                uint16_t* dst = reinterpret_cast<uint16_t*>(a.out) + (int64_t)pair[2 * p + k] * a.n + col;
+                if (THROUGH) st16_global_sc1(dst, v[k]);
+                else *reinterpret_cast<u32x4*>(dst) = v[k];
             }
         }
     }
@@ -553,41 +589,65 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
     // one XCD takes a run of the parts
     const int nx = gridDim.x, tiles = a.tiles[3], total = nx * tiles, lin = (int)(blockIdx.x + gridDim.x * blockIdx.y), per = total >> 3;
     if (lin >= total) return;
-    const int idx = lin < per * 8 ? (lin & 7) * per + (lin >> 3) : lin;
-    expert_product<GLU, false, MW, NW, MT, NT>(a, find_tile<G::TM, G::UNIT>(a.tiles, tiles, nx, idx, 0, tiles, 8, threadIdx.x & 63), lds, [] { return true; }, [] {});
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const ExpertTile to = find_tile<G::TM, G::UNIT>(a.tiles, tiles, nx, lin < per * 8 ? (lin & 7) * per + (lin >> 3) : lin, 0, tiles, 8, lane);
+    const int iters = a.k / TK;                      // (k is a multiple of 64: even)
+    ExpertFeed<G> feed;
+    feed.aim(GLU, a, to, wave, lane);
+    feed.begin(lds, iters, wave);
+    const WaveRows rows(to.live, wave / NW, MW);
+    f32x4 acc[NT][MT];
+    expert_sums<MW, NW, MT, NT>(acc, feed, lds, iters, rows, wave, lane, 0.f, [] {}, [] {});
+    expert_results<GLU, false, MW, NW, MT, NT>(acc, a, to, rows, lds + wave * 2048, wave, lane, [](int) {});
 }
 
 // Both products in one launch of workgroups that stay: the parts of the second one fill the CUs that the last round of the first one leaves idle, and the other way round at its head.
 // A row of tiles is split over eight lists, one for the workgroups of an XCD; a list is its tiles' parts of the first product and behind them those of the second one, drawn by ticket.
 // Whose list is at an end draws from the next one's.  A part of the second product waits until all columns of its row tile are stored, and those were drawn before it
-// from the same list: they are in the hands of workgroups that run, and never wait.  (No assumption on how many are resident, on their order, or on who runs where; the wait is
-// bounded all the same, and numbers of none behind it.)
+// from the same list: they are in the hands of workgroups that run, and never wait; who waits keeps no other part waiting.  (No assumption on how many are resident, on their order,
+// or on who runs where; the wait is bounded all the same, and numbers of none behind it.)
 // What the second product reads is stored through to memory, announced behind the stores' arrival, and lies in lines of its own (rows of whole 128 bytes): no cache holds an older copy.
+// The next part is looked up, and its first images asked for if its rows are there, while this one's results leave: the ring is free by then, they have LDS of their own.  A workgroup's
+// loads and stores arrive in the order of their issue, so these stores are there when a later image is.
+// Bound by the products while they run (0.95 us an image of 256 x 256, the rate of a large product at the clock the card keeps under it); a part of 64 images at 2048 wide is 60 us of those
+// and, before, 4.5 of lookups and first images and 6 to 8 of results.  3000 tokens, 32 experts of 1536: 371 us in two launches, 313 with the parts one after the other, 308 overlapped;
+// 12000 966, 935, 930; 1024 wide, of 768, 6000 176, 164, 160.
+// Few operations on shared words: 256 workgroups that look at eight lists when theirs is at an end took 25 us for it.
+// this lane, not held in a register
+__device__ __forceinline__ int lane_now() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n v_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
 constexpr int kListWords = 32, kWaitLimit = 1 << 22; // tickets a line each; polls of about a microsecond
 struct MoeBothArgs {
     MoeGemmArgs up, down;
     uint32_t* tickets;                               // [8][kListWords], zero; then per row tile its stored columns, [tiles][kListWords], zero
 };
 template <int MW, int NW, int MT, int NT>
+constexpr size_t both_lds_bytes() { return GemmShape<MW, NW, MT, NT>::LDS + MW * NW * 2048 + 16; }
+template <int MW, int NW, int MT, int NT>
 __global__ __launch_bounds__(64 * MW * NW) void moe_both_kernel(const MoeBothArgs a) {
     using G = GemmShape<MW, NW, MT, NT>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    int* const next = reinterpret_cast<int*>(lds + G::LDS);                    // list (-1: at the end), number in it; whether a wait ended well
+    int* const next = reinterpret_cast<int*>(lds + G::LDS + G::WAVES * 2048);  // list (-1: at the end), number in it; whether the rows are there
     uint32_t* const stored = a.tickets + 8 * kListWords;
     const int tiles = a.up.tiles[3], nx = (a.up.n + G::TN / 2 - 1) / (G::TN / 2), ny = (a.down.n + G::TN - 1) / G::TN;
-    const int rows = tiles < 128 ? 4 : 8;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned char* const room = lds + G::LDS + wave * 2048;
     const auto begin = [&](int list) { return (int)((int64_t)tiles * list >> 3); };
     const auto parts = [&](int list) { return (begin(list + 1) - begin(list)) * (nx + ny); };
     const auto draw = [&](int list) {                // (a wave)
         uint32_t t = 0;
-        if ((threadIdx.x & 63) == 0) t = __hip_atomic_fetch_add(a.tickets + list * kListWords, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane_now() == 0) t = __hip_atomic_fetch_add(a.tickets + list * kListWords, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return t;
     };
     const auto settle = [&](int list, uint32_t ticket) {                       // (a wave) that ticket, or one of the first later list that has any
         int number = __builtin_amdgcn_readfirstlane(ticket);
         if (number >= parts(list)) {                 // (all lists' tickets at once, one per lane: what is at an end stays there)
-            const uint32_t seen = __hip_atomic_load(a.tickets + (threadIdx.x & 7) * kListWords, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint32_t open = (uint32_t)__builtin_amdgcn_ballot_w64((int)seen < parts(threadIdx.x & 7)) & 0xFF;
+            const int one = lane_now() & 7;
+            const uint32_t seen = __hip_atomic_load(a.tickets + one * kListWords, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t open = (uint32_t)__builtin_amdgcn_ballot_w64((int)seen < parts(one)) & 0xFF;
             uint32_t later = (open | open << 8) >> (list + 1) & 0x7F;          // list + 1, list + 2, ..
             const int was = list;
             list = -1;
@@ -601,64 +661,94 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_both_kernel(const MoeBothArg
                 later &= later - 1;
             }
         }
-        if ((threadIdx.x & 63) == 0) {
+        if (lane_now() == 0) {
             next[0] = list;
             next[1] = number;
         }
     };
-    if (threadIdx.x < 64) settle(blockIdx.x & 7, draw(blockIdx.x & 7));
+    const auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    struct Part {
+        int list;                                    // -1: none
+        bool glu;
+        ExpertTile to;
+    };
+    Part now, then;
+    ExpertFeed<G> feed;
+    const auto take = [&](Part& part, int lane) {    // the one that was settled
+        const int list = uniform(next[0]), number = uniform(next[1]);
+        part.list = list;
+        if (list < 0) return;
+        const int lo = begin(list), hi = begin(list + 1), first = (hi - lo) * nx;
+        part.glu = number < first;
+        const ExpertTile to = find_tile<G::TM, G::UNIT>(a.up.tiles, tiles, part.glu ? nx : ny, part.glu ? number : number - first, lo, hi, tiles < 128 ? 4 : 8, lane);
+        part.to = ExpertTile{uniform(to.nt), uniform(to.mt), uniform(to.expert), uniform(to.first), uniform(to.live)};
+    };
+    const auto columns = [&](int mt) { return __hip_atomic_load(stored + mt * kListWords, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     int announce = -1;                               // a row tile whose columns are on their way to memory
     const auto announce_it = [&]() {
-        if (announce >= 0) __hip_atomic_fetch_add(stored + announce * kListWords, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (announce >= 0 && wave == 0 && lane_now() == 0) __hip_atomic_fetch_add(stored + announce * kListWords, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        announce = -1;
     };
-    while (true) {
-        lds_only_barrier();                          // (the next part is known, and the images are done with)
-        const int list = __builtin_amdgcn_readfirstlane(next[0]), number = __builtin_amdgcn_readfirstlane(next[1]);
-        if (list < 0) break;
-        int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));
-        const int lane = tid & 63;
-        const int lo = begin(list), hi = begin(list + 1), first = (hi - lo) * nx;
-        // The part behind it: drawn beside the look into the table.  (Behind the first images instead, these are held up: loads arrive in the order in which they were asked for.)
-        uint32_t drawn = 0;
-        if (tid < 64 && number < first) drawn = draw(list);
-        const auto landed = [&]() {
-            if (tid < 64) {
-                if (tid == 0) announce_it();
-                settle(list, drawn);
-            }
-        };
-        if (number < first) {
-            const ExpertTile to = find_tile<G::TM, G::UNIT>(a.up.tiles, tiles, nx, number, lo, hi, rows, lane);
-            expert_product<true, true, MW, NW, MT, NT>(a.up, to, lds, [] { return true; }, landed);
-            announce = to.mt;
-        } else {
-            if (announce >= 0) {                     // before it waits for anyone
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                lds_only_barrier();
-                if (tid == 0) announce_it();
-                announce = -1;
-            }
-            const ExpertTile to = find_tile<G::TM, G::UNIT>(a.up.tiles, tiles, ny, number - first, lo, hi, rows, lane);
-            const uint32_t* const word = stored + to.mt * kListWords;
-            const auto ready = [&]() {
-                if (tid == 0) {
-                    int tries = 0;
-                    while (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (uint32_t)nx && ++tries < kWaitLimit) __builtin_amdgcn_s_sleep(8);
-                    next[2] = tries < kWaitLimit;
-                }
-                if (tid < 64) drawn = draw(list);    // (not before: a workgroup that waits keeps no other part waiting)
-                lds_only_barrier();
-                return next[2] != 0;
-            };
-            expert_product<false, true, MW, NW, MT, NT>(a.down, to, lds, ready, landed);
-        }
-    }
-    if (announce >= 0) {
+    const auto arrived = [&]() {                     // all that the workgroup has stored
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_only_barrier();
-        if (threadIdx.x == 0) announce_it();
+        announce_it();
+    };
+    uint32_t drawn = 0;                              // the part behind the one that has begun
+    const auto go = [&](const Part& part) {
+        if (wave == 0) drawn = draw(part.list);
+        feed.begin(lds, (part.glu ? a.up.k : a.down.k) / TK, wave);
+    };
+    if (wave == 0) settle(blockIdx.x & 7, draw(blockIdx.x & 7));
+    lds_only_barrier();
+    take(then, lane_now());
+    bool begun = false;
+    if (then.list >= 0) feed.aim(then.glu, then.glu ? a.up : a.down, then.to, wave, lane_now());
+    while (then.list >= 0) {
+        float start = 0.f;
+        if (!begun) {
+            arrived();                               // (before it waits for anyone)
+            if (!then.glu) {
+                if (wave == 0 && lane_now() == 0) {
+                    int tries = 0;
+                    while (columns(then.to.mt) < (uint32_t)nx && ++tries < kWaitLimit) __builtin_amdgcn_s_sleep(8);
+                    next[2] = tries < kWaitLimit;
+                }
+                lds_only_barrier();
+                if (!uniform(next[2])) start = __uint_as_float(0x7FC00000u);
+            }
+            go(then);
+        }
+        now = then;
+        const int lane = lane_now();                 // (what hangs on it is computed for each part: held over the loop it would take too many registers)
+        const WaveRows rows(now.to.live, wave / NW, MW);
+        f32x4 acc[NT][MT];
+        expert_sums<MW, NW, MT, NT>(
+            acc, feed, lds, (now.glu ? a.up.k : a.down.k) / TK, rows, wave, lane, start,
+            [&] {
+                if (wave == 0) settle(now.list, drawn);
+            },
+            [&] { announce_it(); });
+        const auto between = [&](int h) __attribute__((always_inline)) {
+            if (h == 0) {
+                take(then, lane_now());
+            } else if (h == 1) {
+                if (then.list >= 0) feed.aim(then.glu, then.glu ? a.up : a.down, then.to, wave, lane_now());
+                if (wave == 0 && lane_now() == 0) next[2] = then.list >= 0 && (then.glu || columns(then.to.mt) >= (uint32_t)nx);
+            } else {
+                lds_only_barrier();
+                begun = uniform(next[2]);
+                if (begun) go(then);
+            }
+        };
+        if (now.glu) {
+            expert_results<true, true, MW, NW, MT, NT>(acc, a.up, now.to, rows, room, wave, lane_now(), between);
+            announce = now.to.mt;
+        } else {
+            expert_results<false, false, MW, NW, MT, NT>(acc, a.down, now.to, rows, room, wave, lane_now(), between);
+        }
     }
+    arrived();
 }
 
 template <bool GLU, int MW, int NW, int MT, int NT>
@@ -900,15 +990,16 @@ static int device_cus() {
     return n;
 }
 
-// Whether both products go in one launch: tiles of 256 rows (a workgroup a CU) that are enough, as far as the pairs tell, for two and a half rounds of the CUs, and a second product
-// whose parts, which come last, are not the longer ones.  us at 32 experts, four routes each, two launches against one: 2048 wide, experts of 1536, 130 pairs an expert (2.5
-// rounds) 199 against 198, 190 246 against 211, 220 247 against 214, 290 286 against 271, 375 329 against 310, 430 384 against 340, 600 453 against 433, 1000 688 against 661;
-// 1024 wide, of 768, 240 (1.8) 84 against 102, 290 (2.0) 102 against 104, 375 (2.4) 109 against 111, 400 (2.6) 123 against 111, 460 131 against 113, 1000 234 against 205.
-// 4096 wide, of 512, 375 pairs 304 against 258.  Where the parts of either product are just whole rounds, one launch takes up to 3 % longer; 768 wide, of 2048, 16 experts of 600 pairs:
-// 154 against 167.  From 20 rounds on the idle ends are little against what each part's hand-over costs: 2048 wide, 16384 tokens by sigmoids 1151 against 1156 (12000, 16 rounds, 982
-// against 960).  Tiles of 128 rows, two workgroups a CU, fill their rounds better as they are: 32 experts of 2048 and 1536, 60 pairs 158 against 164.
+// Whether both products go in one launch: tiles of 256 rows (a workgroup a CU) that are enough, as far as the pairs tell, for two and a half rounds of the CUs and some experts with two
+// tiles, and a second product whose parts, which come last, are not the longer ones.  us of four routes each, two launches against one: 2048 wide, 32 experts of 1536, 170 pairs an expert
+// 205 against 212, 190 223 against 220, 220 250 against 223, 290 279 against 272, 375 302 against 295, 430 383 against 339, 600 448 against 435, 1000 681 against 666; 1024 wide, of 768,
+// 240 (1.8 rounds) 85 against 101, 330 (2.2) 105 against 109, 375 (2.4) 112 against 112, 400 (2.6) 126 against 113, 460 136 against 117, 1000 238 against 209; 4096 wide, of 512, 170
+// 177 against 182, 190 193 against 185, 375 269 against 242, 550 362 against 308; 24 experts of 1536 at 2048, 220 202 against 206, 240 220 against 202.  768 wide, 16 experts of 2048,
+// 500 to 600 142 to 150 against 144 to 152, around them up to 1.16 times as fast.  From 20 rounds on the idle ends are little against what each part's hand-over
+// costs: 2048 wide, 16384 tokens by sigmoids 1106 against 1118, by a softmax 1256 against 1240.  Tiles of 128 rows, two workgroups a CU, fill their rounds better as they are:
+// 32 experts of 1536, 2048 wide, 60 pairs 158 against 164.
 bool moe_one_launch(int pairs, int experts, int n, int cols, int tile_rows) {
-    if (tile_rows != 256 || n > cols) return false;
+    if (tile_rows != 256 || pairs / experts < 180 || n > cols || n < 128) return false;       // (n: a part announces the one before it behind its fourth image of 32)
     const int64_t tiles = pairs / 256 + experts / 2, parts = tiles * ((n + 127) / 128 + (cols + 255) / 256);
     return 2 * parts >= 5 * device_cus() && parts < 20 * device_cus();
 }
@@ -916,7 +1007,7 @@ size_t moe_links_words(int tile_rows, int max_tiles) { return tile_rows == 256 ?
 
 int launch_moe_both(const MoeGemmArgs& up, const MoeGemmArgs& down, uint32_t* tickets, hipStream_t stream) {
     using G = GemmShape<2, 4, 8, 4>;
-    const size_t lds = G::LDS + 16;
+    const size_t lds = both_lds_bytes<2, 4, 8, 4>();
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(moe_both_kernel<2, 4, 8, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const int64_t parts = (int64_t)up.max_tiles * ((up.n + G::TN / 2 - 1) / (G::TN / 2) + (down.n + G::TN - 1) / G::TN);
     moe_both_kernel<2, 4, 8, 4><<<(int)(parts < device_cus() ? parts : device_cus()), 64 * G::WAVES, lds, stream>>>(MoeBothArgs{up, down, tickets});

@@ -220,14 +220,20 @@ __global__ __launch_bounds__(256) void moe_count_kernel(int32_t* __restrict__ co
     __shared__ int hist[kMoeMaxExperts];
     for (int e = threadIdx.x; e < experts; e += 256) hist[e] = 0;
     __syncthreads();
-    const int p0 = blockIdx.x * DP;
-    for (int p = p0 + threadIdx.x; p < p0 + DP && p < pairs; p += 256) atomicAdd(&hist[ids[p]], 1);
+    const int p0 = blockIdx.x * DP + threadIdx.x;
+    int id[DP / 256];                                // (all asked for at once)
+#pragma unroll
+    for (int u = 0; u < DP / 256; ++u) id[u] = ids[p0 + 256 * u < pairs ? p0 + 256 * u : pairs - 1];
+#pragma unroll
+    for (int u = 0; u < DP / 256; ++u)
+        if (p0 + 256 * u < pairs) atomicAdd(&hist[id[u]], 1);
     __syncthreads();
     for (int e = threadIdx.x; e < experts; e += 256) counts[(int64_t)blockIdx.x * experts + e] = hist[e];
 }
 
 // Every workgroup sums the counts in front of its own pairs; the first one also writes the tiles.  Up to kCountHere pairs each counts all of them itself: the launch that counts takes
-// longer than that.  300 tokens' 1200 pairs 1.9 + 3.1 us in two launches, 2.4 in one (1024 wide: the call 55 -> 52 us); 7200
+// longer than that.  (Both bound by latency: every load of a thread is asked for at once, and all threads sum the counts.  One by one, 32 threads summing: dispatch of 65536 pairs of 32
+// experts 13.2 -> 6.7 us, 12000 7.1 -> 6.4.)  300 tokens' 1200 pairs 1.9 + 3.1 us in two launches, 2.4 in one (1024 wide: the call 55 -> 52 us); 7200
 // pairs 89 -> 86.
 constexpr int kCountHere = 4 * DP;
 template <bool COUNTED>
@@ -247,20 +253,27 @@ __global__ __launch_bounds__(256) void moe_scatter_kernel(int32_t* __restrict__ 
     };
     int own[PER];                                    // the experts of this workgroup's pairs
     take(p0, own);
-    if constexpr (COUNTED) {
-        for (int e = threadIdx.x; e < experts; e += 256) {
-            int before = 0, all = 0;
-            for (int b = 0; b < (int)gridDim.x; ++b) {
-                const int c = counts[(int64_t)b * experts + e];
-                if (b < (int)blockIdx.x) before += c;
-                all += c;
+    for (int e = threadIdx.x; e < experts; e += 256) at[e] = total[e] = 0;
+    __syncthreads();
+    if constexpr (COUNTED) {                         // (every thread, as the counts lie)
+        const int words = (int)gridDim.x * experts, mine = (int)blockIdx.x * experts;
+        for (int i0 = 0; i0 < words; i0 += 4 * 256) {
+            int c[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = i0 + 256 * u + (int)threadIdx.x;
+                c[u] = counts[i < words ? i : 0];
             }
-            at[e] = before;
-            total[e] = all;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = i0 + 256 * u + (int)threadIdx.x, e = i % experts;
+                if (i < words && c[u]) {
+                    atomicAdd(&total[e], c[u]);
+                    if (i < mine) atomicAdd(&at[e], c[u]);
+                }
+            }
         }
     } else {
-        for (int e = threadIdx.x; e < experts; e += 256) at[e] = total[e] = 0;
-        __syncthreads();
         auto count = [&](int first, const int (&id)[PER]) __attribute__((always_inline)) {
 #pragma unroll
             for (int u = 0; u < PER; ++u)

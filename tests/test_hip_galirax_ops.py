@@ -471,6 +471,12 @@ def test_dispatch_counts(pairs, experts):
     assert [t[:3] for t in tiles.tolist()[:len(want)]] == want and all(t[2:] == [0, len(want)] for t in tiles.tolist()[len(want):])
 
 
+# counts of several workgroups: experts that divide what the threads take at a time and that do not, up to the most; many more counts than threads
+@pytest.mark.parametrize("pairs,experts", [(8193, 1024), (8193, 1000), (20481, 1), (40000, 257), (70001, 33)])
+def test_dispatch_sums_counts(pairs, experts):
+    test_dispatch_counts(pairs, experts)
+
+
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,top,experts,n,k", [(1, 2, 4, 64, 64), (5, 4, 8, 128, 320), (33, 8, 16, 192, 128), (64, 1, 2, 64, 1088), (40, 3, 3, 2112, 192), (65, 2, 9, 64, 128),
                                                   (300, 4, 8, 192, 256), (700, 2, 3, 128, 64)])

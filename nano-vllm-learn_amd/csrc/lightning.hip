@@ -272,7 +272,71 @@ constexpr size_t pair_lds_bytes(bool summary) {
     return (size_t)2 * C * (DK * (summary ? 1 : 2) + 16 * CW) * 2 + (summary ? 0 : (size_t)2 * C * PLD * 2);
 }
 
-template <int DK, int CW, int PW, bool SUMMARY>
+// Whole portions that nothing comes in front of: the longest of them as two pieces of the same length in time.  The second one follows the state over the first one's tokens (keys and
+// values only: kFollow of a chunk) and goes on from there with outputs: the same operations on the same numbers, no summary and no launch in front.  Both would read a state that the
+// second one replaces: portions behind a state stay whole, and with them all of the launch.
+// A workgroup a CU walks at its own pace, so the longest portion sets the time, 1.6 to 1.75 of the mean.  As many pieces are made as bring the longest one (a chunk to start, and those that
+// it takes) and the even load (times kUneven, what the order by length leaves on it) down together.  16384 tokens of 16 uneven sequences, 16 heads of 128: 129 -> 106 us; 9000 of 14
+// 82 -> 64, 5000 of 16 46 -> 42; 8 heads, 9000 of 28 42 -> 37.
+// (a wave) The nth walk, the longest first: portion, tokens followed, end in tokens; portion -1: none.
+constexpr int kSplitPortions = 32;
+constexpr float kFollow = 0.6f, kUneven = 1.2f;
+struct LightningWalk {
+    int seg, from, to;
+};
+__device__ __forceinline__ LightningWalk lightning_walk_of(const LightningArgs& a, int walks_each, int nth) {
+    const int lane = threadIdx.x & 63, i = lane & 31;
+    const int rows = i < a.n_chunks ? a.chunks[4 * i + 1] : 0, length = rows > 0 ? (rows + C - 1) / C : 0;
+    const bool behind = rows > 0 && a.positions[a.chunks[4 * i]] > 0;
+    if (__builtin_amdgcn_ballot_w64(behind)) {
+        if (nth >= a.n_chunks) return LightningWalk{-1, 0, 0};
+        return LightningWalk{nth_largest<10>(length < 1023 ? length : 1023, a.n_chunks, nth), 0, 0x7FFFFFFF};
+    }
+    int rank = 0;                                    // in the order of lengths
+    for (int k = 0; k < a.n_chunks; ++k) {
+        const int other = __builtin_amdgcn_readlane(length, k);
+        rank += other > length || (other == length && k < i);
+    }
+    // lanes p and 32 + p: the p-th longest, in chunks
+    const int lane_of = 4 * (rank + (lane & 32)), mine = __builtin_amdgcn_ds_permute(lane_of, i < a.n_chunks ? length : 0), seg = __builtin_amdgcn_ds_permute(lane_of, i);
+    const int cut = (int)ceilf((float)mine * (1.f / (2.f - kFollow)));
+    const float first = cut + 1.f, second = kFollow * cut + (mine - cut) + 1.f, whole = mine + 1.f;
+    // lane p: the longest p as two pieces (lengths fall with the lane, and with them whole and halves)
+    const bool real = lane < 32 && lane < a.n_chunks;
+    float all = real ? whole : 0.f, added = real ? first + second - whole : 0.f;
+    const float own = added;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const float below = __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane - d), __float_as_uint(added)));
+        all += __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane ^ d), __float_as_uint(all)));
+        added += lane >= d ? below : 0.f;
+    }
+    const float top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(fmaxf(first, second))));
+    const float rest = real ? whole : 0.f, longest = lane ? fmaxf(top, rest) : rest;
+    const int places = 256 / walks_each, most = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < 32 && mine >= 4));
+    const float even = (all + added - own) * kUneven / places;
+    float cost = a.n_chunks + lane > places && even > longest ? even : longest;
+    if (lane > most) cost = INFINITY;
+    if (lane) cost = cost * (1.f / 0.97f);           // (not for little)
+    float least = cost;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) least = fminf(least, __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane ^ d), __float_as_uint(least))));
+    const int split = __builtin_ctzll(__builtin_amdgcn_ballot_w64(cost == least));
+    // pieces: lanes 0 .. 31 the first ones, or whole, 32 .. the second ones
+    const bool two = i < split;
+    const float piece = lane < 32 ? (two ? first : whole) : two ? second : 0.f;
+    LightningWalk to{-1, 0, 0};
+    if (nth >= a.n_chunks + split) return to;
+    const int size = i < a.n_chunks ? (int)(2.f * piece) : 0, at = nth_largest<10>(size < 1023 ? size : 1023, 64, nth), p = at & 31;
+    const int from = C * (int)__builtin_amdgcn_readlane(cut, p);
+    to.seg = __builtin_amdgcn_readlane(seg, p);
+    const bool halves = p < split;
+    to.from = at >= 32 ? from : 0;
+    to.to = halves && at < 32 ? from : 0x7FFFFFFF;
+    return to;
+}
+
+template <int DK, int CW, int PW, bool SUMMARY, bool PIECES>
 __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const LightningArgs a) {
     constexpr int T = 64 * PW, VW = 16 * CW, KP = DK / 8, KROW = DK * 2, VP = VW / 8, VROW = VW * 2, NQ = C * KP / T, NV = C * VP / T, DT = DK / 16, PT = PW / 4;
     constexpr int KIMG = C * KROW, VIMG = C * VROW;
@@ -284,11 +348,28 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
     __shared__ __attribute__((aligned(16))) float pw[C + 1], fall_s[C];        // decay^0 .. decay^C; decay^(C - 1 - key)
     auto swz = [](int r) { return KROW == 128 ? (r >> 1) & 7 : r & 15; };      // rows of 256 bytes span all banks: 16 of them apart, not 8
     auto swzv = [](int r) { return VROW == 128 ? (r >> 1) & 7 : (2 * r) & 14; };
-    const int seg = longest_first(a, a.heads * (a.dv / VW));
-    const int32_t* ch = a.chunks + 4 * seg;
-    const int row0 = ch[0], n_rows = ch[1], seq = ch[2];
+    __shared__ int walk_s[3];
     const int slices = a.dv / VW, head = blockIdx.x / slices, v0 = (blockIdx.x - head * slices) * VW;
-    const bool last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;
+    int seg = blockIdx.y, from = 0, to = 0x7FFFFFFF; // tokens that are only followed; end
+    if constexpr (PIECES) {
+        if (threadIdx.x < 64) {
+            const LightningWalk w = lightning_walk_of(a, a.heads * (a.dv / VW), blockIdx.y);
+            if (threadIdx.x == 0) walk_s[0] = w.seg, walk_s[1] = w.from, walk_s[2] = w.to;
+        } else if (threadIdx.x <= 64 + C) {          // (meanwhile)
+            const int t = threadIdx.x - 64;
+            const float p = powf(a.decay[head], (float)t);
+            pw[t] = p;
+            if (t < C) fall_s[C - 1 - t] = p;
+        }
+        __syncthreads();
+        seg = __builtin_amdgcn_readfirstlane(walk_s[0]), from = __builtin_amdgcn_readfirstlane(walk_s[1]), to = __builtin_amdgcn_readfirstlane(walk_s[2]);
+        if (seg < 0) return;
+    } else {
+        seg = longest_first(a, a.heads * (a.dv / VW));
+    }
+    const int32_t* ch = a.chunks + 4 * seg;
+    const int row0 = ch[0], n_rows = ch[1] < to ? ch[1] : to, seq = ch[2];
+    const bool last = ch[1] <= to && (seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0);
     if (SUMMARY && last) return;                     // (nothing follows it)
     const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lq = lane & 15, lg = lane >> 4;
     const bool prepares = wave_id >= CW;
@@ -300,12 +381,14 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
             pass_segment<SUMMARY>(a.seg_state + ((int64_t)seg * a.heads + head) * head_state + v0, a.state + (slot * a.heads + head) * head_state + v0, DK, VW, a.dv);
         return;
     }
-    if (threadIdx.x <= C) {
-        const float p = powf(a.decay[head], (float)threadIdx.x);
-        pw[threadIdx.x] = p;
-        if (threadIdx.x < C) fall_s[C - 1 - threadIdx.x] = p;
+    if constexpr (!PIECES) {
+        if (threadIdx.x <= C) {
+            const float p = powf(a.decay[head], (float)threadIdx.x);
+            pw[threadIdx.x] = p;
+            if (threadIdx.x < C) fall_s[C - 1 - threadIdx.x] = p;
+        }
+        __syncthreads();
     }
-    __syncthreads();
 
     if (prepares) {
         const int tid = threadIdx.x - 64 * CW;
@@ -333,14 +416,16 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
         // (every chunk asks for as many rows as any other, in straight line, the last one's again behind the end: behind a branch around loads the compiler waits
         // for all that are in flight instead of the ones it needs)
         const int t_last = (n_rows - 1) / C * C;
-        auto fetch_qk = [&](int t) __attribute__((always_inline)) {
+        constexpr std::bool_constant<!SUMMARY> with_q{};
+        constexpr std::bool_constant<false> no_q{};
+        auto fetch_qk = [&](int t, auto q) __attribute__((always_inline)) {
             const int t0 = t < t_last ? t : t_last;
             if (n_rows - t0 < C) place(n_rows - t0);
             const unsigned char* base = base_of(t0);
 #pragma unroll
             for (int j = 0; j < NQ; ++j) {
                 kr[j] = *reinterpret_cast<const u32x4*>(base + 2 * k_off + at[j]);
-                if constexpr (!SUMMARY) qr[j] = *reinterpret_cast<const u32x4*>(base + 2 * q_off + at[j]);
+                if constexpr (decltype(q)::value) qr[j] = *reinterpret_cast<const u32x4*>(base + 2 * q_off + at[j]);
             }
         };
         auto fetch_v = [&](int t) __attribute__((always_inline)) {
@@ -348,18 +433,21 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
 #pragma unroll
             for (int j = 0; j < NV; ++j) vr[j] = *reinterpret_cast<const u32x4*>(base + 2 * v_off + atv[j]);
         };
-        auto stage_qk = [&](int t0, int buf) __attribute__((always_inline)) {  // rows past the end are zero (as is silu of them)
+        auto stage_qk = [&](int t0, int buf, auto q) __attribute__((always_inline)) {    // rows past the end are zero (as is silu of them)
             const int n = n_rows - t0;
             if (n < C) {
 #pragma unroll
                 for (int j = 0; j < NQ; ++j)
-                    if ((j * T + tid) / KP >= n) kr[j] = qr[j] = zero;
+                    if ((j * T + tid) / KP >= n) {
+                        kr[j] = zero;
+                        if constexpr (decltype(q)::value) qr[j] = zero;
+                    }
             }
 #pragma unroll
             for (int j = 0; j < NQ; ++j) {
                 const int e = j * T + tid, r = e / KP, pc = e - r * KP;
                 *reinterpret_cast<u32x4*>(kimg0 + buf * KIMG + r * KROW + (pc ^ swz(r)) * 16) = silu8(kr[j]);
-                if constexpr (!SUMMARY) *reinterpret_cast<u32x4*>(qimg0 + buf * KIMG + r * KROW + (pc ^ swz(r)) * 16) = silu8(qr[j]);
+                if constexpr (decltype(q)::value) *reinterpret_cast<u32x4*>(qimg0 + buf * KIMG + r * KROW + (pc ^ swz(r)) * 16) = silu8(qr[j]);
             }
         };
         auto stage_v = [&](int t0, int buf) __attribute__((always_inline)) {
@@ -436,19 +524,43 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
             }
         };
         place(C);
-        fetch_qk(0);
-        fetch_v(0);
-        stage_qk(0, 0);
-        fetch_qk(C);
-        stage_v(0, 0);
-        fetch_v(C);
-        lds_only_barrier();
-        weights(0);
-        lds_only_barrier();
-        for (int t0 = 0, buf = 0; t0 < n_rows; t0 += C, buf ^= 1) {
+        int t0 = 0, buf = 0;
+        if (PIECES && from) {                        // (at least three chunks)
+            fetch_qk(0, no_q);
+            fetch_v(0);
+            stage_qk(0, 0, no_q);
+            fetch_qk(C, no_q);
+            stage_v(0, 0);
+            fetch_v(C);
+            lds_only_barrier();
+            lds_only_barrier();
+            auto follow = [&](auto q) __attribute__((always_inline)) {
+                stage_qk(t0 + C, buf ^ 1, no_q);
+                fetch_qk(t0 + 2 * C, q);
+                lds_only_barrier();
+                stage_v(t0 + C, buf ^ 1);
+                fetch_v(t0 + 2 * C);
+                lds_only_barrier();
+                t0 += C;
+                buf ^= 1;
+            };
+            while (t0 < from - 2 * C) follow(no_q);
+            follow(with_q);                          // (asks for the first chunk that has outputs)
+        } else {
+            fetch_qk(0, with_q);
+            fetch_v(0);
+            stage_qk(0, 0, with_q);
+            fetch_qk(C, with_q);
+            stage_v(0, 0);
+            fetch_v(C);
+            lds_only_barrier();
+            weights(0);
+            lds_only_barrier();
+        }
+        for (; t0 < n_rows; t0 += C, buf ^= 1) {
             const bool next = t0 + C < n_rows;
-            if (next) stage_qk(t0 + C, buf ^ 1);
-            fetch_qk(t0 + 2 * C);
+            if (next) stage_qk(t0 + C, buf ^ 1, with_q);
+            fetch_qk(t0 + 2 * C, with_q);
             lds_only_barrier();
             if (next) {
                 weights(buf ^ 1);
@@ -479,7 +591,63 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
     const int tr = 4 * lg + (lq >> 2), tp = lq & 3;  // transposed reads: row and column quarter this lane addresses
     lds_only_barrier();
     lds_only_barrier();
-    for (int t0 = 0, buf = 0; t0 < n_rows; t0 += C, buf ^= 1) {
+    // what a followed chunk does to the state: the second half of the loop below.  (Shared with it as a function, that loop loses 1 % of its speed)
+    auto values = [&](bf16x8 (&vf)[2], const unsigned char* vimg) __attribute__((always_inline)) {
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+            const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * wave + (tp >> 1);
+            const u32x2 lo = lds_tr16(vimg + ra * VROW + (pc ^ swzv(ra)) * 16 + (tp & 1) * 8), hi = lds_tr16(vimg + rb * VROW + (pc ^ swzv(rb)) * 16 + (tp & 1) * 8);
+            const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
+            vf[hh] = *reinterpret_cast<const bf16x8*>(&raw);
+        }
+    };
+    auto advance = [&](const bf16x8 (&vf)[2], int n, const unsigned char* kimg) __attribute__((always_inline)) {
+        // ---- the state behind these tokens
+        const float decayed = pw[n];
+#pragma unroll
+        for (int t = 0; t < DT; ++t) S[t] *= decayed;
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+            const u32x4 raw = *reinterpret_cast<const u32x4*>(&vf[hh]);
+            f32x4 fall[2];                           // what a value decays by until the chunk's end
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int key = 32 * hh + 16 * q + 4 * lg;
+                if (n == C) {
+                    fall[q] = *reinterpret_cast<const f32x4*>(fall_s + key);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) fall[q][r] = pw[key + r < n ? n - 1 - key - r : 0];
+                }
+            }
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = (j & 1 ? bf16_hi(raw[j >> 1]) : bf16_lo(raw[j >> 1])) * fall[j >> 2][j & 3];
+            bf16x8 hi, lo;
+            split_hi_lo(v, hi, lo);
+            const int ra = 32 * hh + tr, rb = ra + 16;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                const int pc = 2 * t + (tp >> 1);
+                const u32x2 klo = lds_tr16(kimg + ra * KROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8), khi = lds_tr16(kimg + rb * KROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8);
+                const u32x4 kraw = {klo[0], klo[1], khi[0], khi[1]};
+                const bf16x8 kf = *reinterpret_cast<const bf16x8*>(&kraw);
+                S[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, hi, S[t], 0, 0, 0);
+                S[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, lo, S[t], 0, 0, 0);
+            }
+        }
+    };
+    int t0 = 0, buf = 0;
+    if constexpr (PIECES) {
+        for (; t0 < from; t0 += C, buf ^= 1) {
+            bf16x8 vf[2];
+            values(vf, vimg0 + buf * VIMG);
+            lds_only_barrier();
+            advance(vf, C, kimg0 + buf * KIMG);
+            lds_only_barrier();
+        }
+    }
+    for (; t0 < n_rows; t0 += C, buf ^= 1) {
         const int n = n_rows - t0 < C ? n_rows - t0 : C;
         const unsigned char *kimg = kimg0 + buf * KIMG, *qimg = qimg0 + buf * KIMG, *vimg = vimg0 + buf * VIMG;
         // value fragments: lane = column 16 wave + lq, slots = keys 32 hh + 4 lg + 0..3 and the same + 16
@@ -753,13 +921,14 @@ template <int DK, int CW, int PW>
 int pair_dk(const LightningArgs& a, hipStream_t stream) {
     constexpr size_t sum_lds = pair_lds_bytes<DK, CW>(true), lds = pair_lds_bytes<DK, CW>(false);
     if (lds > 64 * 1024)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, false, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (sum_lds > 64 * 1024)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sum_lds);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, true, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sum_lds);
     // heads run fastest: workgroups are dealt round-robin over the 8 XCDs, and segments differ in length while the heads of one do not
-    const dim3 grid(a.heads * (a.dv / (16 * CW)), a.n_chunks);
+    const int walks = a.heads * (a.dv / (16 * CW));
+    dim3 grid(walks, a.n_chunks);
     if (a.summaries) {
-        lightning_pair_kernel<DK, CW, PW, true><<<grid, 64 * (CW + PW), sum_lds, stream>>>(a);
+        lightning_pair_kernel<DK, CW, PW, true, false><<<grid, 64 * (CW + PW), sum_lds, stream>>>(a);
         int rc = check_launch("lightning summary");
         if (rc) return rc;
         const int64_t per = (int64_t)a.heads * a.dk * a.dv;
@@ -767,7 +936,17 @@ int pair_dk(const LightningArgs& a, hipStream_t stream) {
         rc = check_launch("lightning starts");
         if (rc) return rc;
     }
-    lightning_pair_kernel<DK, CW, PW, false><<<grid, 64 * (CW + PW), lds, stream>>>(a);
+    // The longest portions as two pieces, where whole ones come to 193 to 320 workgroups: fewer are better cut into segments, more fill the CUs more than once and even out.  Choosing takes
+    // 2 us, for nothing where a portion continues (9000 tokens of 16, 16 heads of 128: 73.5 against 74.4); so other launches have a kernel without it, as have those of less than four
+    // chunks a portion (3000 of 20: 29 against 32).
+    if (!a.summaries && a.n_chunks > 1 && a.n_chunks <= kSplitPortions && walks * a.n_chunks > 192 && walks * a.n_chunks <= 320 && a.rows >= 4 * C * a.n_chunks) {
+        grid.y = 2 * a.n_chunks;
+        if (lds > 64 * 1024)
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, false, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        lightning_pair_kernel<DK, CW, PW, false, true><<<grid, 64 * (CW + PW), lds, stream>>>(a);
+    } else {
+        lightning_pair_kernel<DK, CW, PW, false, false><<<grid, 64 * (CW + PW), lds, stream>>>(a);
+    }
     return check_launch("lightning walk");
 }
 

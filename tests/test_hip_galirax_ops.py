@@ -308,6 +308,33 @@ def test_lightning_chunk_borders_behind_a_state(heads, dk, dv):
         close(state[i], s, BF16, f"state {i}", slack=0.05)
 
 
+# a few long portions among short ones, portions of 192, 193, 256 and 257 tokens (the shortest that are cut), without rows, one behind a state, as many as are looked at and one more
+UNEVEN = [1500, 700, 90, 300, 64, 0, 1, 400, 193, 1000, 20, 192, 257, 256]
+@pytest.mark.parametrize("heads,dk,dv,lengths,behind", [
+    (16, 128, 128, UNEVEN, False), (16, 64, 64, UNEVEN, False), (8, 64, 256, UNEVEN, False), (16, 128, 128, UNEVEN, True), (64, 64, 64, [700, 1500, 193, 64], False),
+    (32, 128, 64, [1500, 64, 700, 193, 250, 192, 256, 257], False), (8, 64, 128, [1200, 900] + [257] * 30, False), (8, 64, 128, [1200, 900] + [257] * 31, False)])
+def test_lightning_long_portions_as_two_pieces(heads, dk, dv, lengths, behind):
+    """Bit for bit every portion alone, where it is whole."""
+    from nanovllm_hip import ops
+    n, width, none = len(lengths), heads * (2 * dk + dv), min(4, len(lengths) - 1)
+    x, decay = randn(sum(lengths), width, seed=3).cuda(), torch.linspace(0.9, 0.999, heads).cuda()
+    first = [sum(lengths[:i]) for i in range(n)]
+    pos = torch.cat([torch.arange(m) + (7 if behind and i == 3 else 0) for i, m in enumerate(lengths)]).cuda()
+    slots = torch.tensor([n - 1 - i if i != none else -1 for i in range(n)], dtype=torch.int32).cuda()
+    start = randn(n, heads, dk, dv, seed=4, dtype=F32).cuda()
+
+    def run(table):
+        state = start.clone()
+        return ops.lightning_chunks(x, decay, pos, slots, torch.tensor(table, dtype=torch.int32).cuda(), False, state), state
+    out, state = run([(f, m, i, 0) for i, (f, m) in enumerate(zip(first, lengths))])
+    for i, (f, m) in enumerate(zip(first, lengths)):
+        if m:
+            one, end = run([(f, m, i, 0)])
+            assert torch.equal(out[f:f + m], one[f:f + m])
+            assert i == none or torch.equal(state[n - 1 - i], end[n - 1 - i])
+    assert torch.equal(state[n - 1 - none], start[n - 1 - none])
+
+
 @pytest.mark.parametrize("stride", [(1 << 25) - 8, 34_100_000])
 @pytest.mark.parametrize("heads,dk,dv", [(2, 64, 64), (1, 64, 128), (1, 128, 64), (2, 128, 128)])
 def test_lightning_rows_far_apart(heads, dk, dv, stride):

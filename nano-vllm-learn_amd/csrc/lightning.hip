@@ -276,29 +276,31 @@ constexpr size_t pair_lds_bytes(bool summary) {
 // values only: kFollow of a chunk) and goes on from there with outputs: the same operations on the same numbers, no summary and no launch in front.  Both would read a state that the
 // second one replaces: portions behind a state stay whole, and with them all of the launch.
 // A workgroup a CU walks at its own pace, so the longest portion sets the time, 1.6 to 1.75 of the mean.  As many pieces are made as bring the longest one (a chunk to start, and those that
-// it takes) and the even load (times kUneven, what the order by length leaves on it) down together.  16384 tokens of 16 uneven sequences, 16 heads of 128: 129 -> 106 us; 9000 of 14
-// 82 -> 64, 5000 of 16 46 -> 42; 8 heads, 9000 of 28 42 -> 37.
+// it takes), the even load (times kUneven, what the order by length leaves on it) and the first to wait for a CU down together.  Eight sets of lengths each, 16 heads of 128: 16384 tokens
+// of 16 1.11 times as fast (130 -> 94, 100 -> 95), 9000 of 14 1.18 (82 -> 64), 12000 of 19 1.00 (0.95 to 1.04); 8 heads, 14000 of 28 1.13.  kFollow 0.6: 1.10, 1.17, 1.00, 1.13; kUneven 1.1: 1.11,
+// 1.18, 1.00, 1.12; without the wait for a CU 1.08, 1.13, 1.00, 1.09, one of 32 sets at 0.83.
 // (a wave) The nth walk, the longest first: portion, tokens followed, end in tokens; portion -1: none.
 constexpr int kSplitPortions = 32;
-constexpr float kFollow = 0.6f, kUneven = 1.2f;
+constexpr float kFollow = 0.5f, kUneven = 1.2f;
 struct LightningWalk {
     int seg, from, to;
 };
 __device__ __forceinline__ LightningWalk lightning_walk_of(const LightningArgs& a, int walks_each, int nth) {
     const int lane = threadIdx.x & 63, i = lane & 31;
-    const int rows = i < a.n_chunks ? a.chunks[4 * i + 1] : 0, length = rows > 0 ? (rows + C - 1) / C : 0;
+    const int listed = i < a.n_chunks ? a.chunks[4 * i + 1] : 0, rows = listed > 0 ? listed : 0;
     const bool behind = rows > 0 && a.positions[a.chunks[4 * i]] > 0;
     if (__builtin_amdgcn_ballot_w64(behind)) {
         if (nth >= a.n_chunks) return LightningWalk{-1, 0, 0};
-        return LightningWalk{nth_largest<10>(length < 1023 ? length : 1023, a.n_chunks, nth), 0, 0x7FFFFFFF};
+        const int steps = (rows + 15) >> 4;
+        return LightningWalk{nth_largest<10>(steps < 1023 ? steps : 1023, a.n_chunks, nth), 0, 0x7FFFFFFF};
     }
     int rank = 0;                                    // in the order of lengths
     for (int k = 0; k < a.n_chunks; ++k) {
-        const int other = __builtin_amdgcn_readlane(length, k);
-        rank += other > length || (other == length && k < i);
+        const int other = __builtin_amdgcn_readlane(rows, k);
+        rank += other > rows || (other == rows && k < i);
     }
-    // lanes p and 32 + p: the p-th longest, in chunks
-    const int lane_of = 4 * (rank + (lane & 32)), mine = __builtin_amdgcn_ds_permute(lane_of, i < a.n_chunks ? length : 0), seg = __builtin_amdgcn_ds_permute(lane_of, i);
+    // lanes p and 32 + p: the p-th longest
+    const int lane_of = 4 * (rank + (lane & 32)), mine_rows = __builtin_amdgcn_ds_permute(lane_of, rows), seg = __builtin_amdgcn_ds_permute(lane_of, i), mine = (mine_rows + C - 1) / C;
     const int cut = (int)ceilf((float)mine * (1.f / (2.f - kFollow)));
     const float first = cut + 1.f, second = kFollow * cut + (mine - cut) + 1.f, whole = mine + 1.f;
     // lane p: the longest p as two pieces (lengths fall with the lane, and with them whole and halves)
@@ -315,8 +317,12 @@ __device__ __forceinline__ LightningWalk lightning_walk_of(const LightningArgs& 
     const float rest = real ? whole : 0.f, longest = lane ? fmaxf(top, rest) : rest;
     const int places = 256 / walks_each, most = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < 32 && mine >= 4));
     const float even = (all + added - own) * kUneven / places;
-    float cost = a.n_chunks + lane > places && even > longest ? even : longest;
-    if (lane > most) cost = INFINITY;
+    // more pieces than CUs for them: the largest that waits goes behind the first to end, both of them short whole portions
+    const float waits = __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (places - lane), __float_as_uint(whole))),
+                ends = __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (places - lane - 1), __float_as_uint(whole)));
+    float cost = longest;
+    if (a.n_chunks + lane > places) cost = fmaxf(fmaxf(longest, even), lane ? waits + ends : 0.f);
+    if (lane > most || (lane && a.n_chunks + lane > places && 2 * lane >= places)) cost = INFINITY;
     if (lane) cost = cost * (1.f / 0.97f);           // (not for little)
     float least = cost;
 #pragma unroll
@@ -324,10 +330,10 @@ __device__ __forceinline__ LightningWalk lightning_walk_of(const LightningArgs& 
     const int split = __builtin_ctzll(__builtin_amdgcn_ballot_w64(cost == least));
     // pieces: lanes 0 .. 31 the first ones, or whole, 32 .. the second ones
     const bool two = i < split;
-    const float piece = lane < 32 ? (two ? first : whole) : two ? second : 0.f;
+    const float piece = lane < 32 ? first : two ? second : 0.f;
     LightningWalk to{-1, 0, 0};
     if (nth >= a.n_chunks + split) return to;
-    const int size = i < a.n_chunks ? (int)(2.f * piece) : 0, at = nth_largest<10>(size < 1023 ? size : 1023, 64, nth), p = at & 31;
+    const int size = i >= a.n_chunks ? 0 : lane < 32 && !two ? 4 + ((mine_rows + 15) >> 4) : (int)(4.f * piece), at = nth_largest<10>(size < 1023 ? size : 1023, 64, nth), p = at & 31;
     const int from = C * (int)__builtin_amdgcn_readlane(cut, p);
     to.seg = __builtin_amdgcn_readlane(seg, p);
     const bool halves = p < split;
@@ -937,7 +943,7 @@ int pair_dk(const LightningArgs& a, hipStream_t stream) {
         if (rc) return rc;
     }
     // The longest portions as two pieces, where whole ones come to 193 to 320 workgroups: fewer are better cut into segments, more fill the CUs more than once and even out.  Choosing takes
-    // 2 us, for nothing where a portion continues (9000 tokens of 16, 16 heads of 128: 73.5 against 74.4); so other launches have a kernel without it, as have those of less than four
+    // 2 us, for nothing where a portion continues (9000 tokens of 16, 16 heads of 128: 74.4 us against 73.5); so other launches have a kernel without it, as have those of less than four
     // chunks a portion (3000 of 20: 29 against 32).
     if (!a.summaries && a.n_chunks > 1 && a.n_chunks <= kSplitPortions && walks * a.n_chunks > 192 && walks * a.n_chunks <= 320 && a.rows >= 4 * C * a.n_chunks) {
         grid.y = 2 * a.n_chunks;

@@ -445,10 +445,10 @@ struct WaveRows {
 };
 
 // D[weight row 16 i + 4 lg + r][pair 16 j + lq] of a wave, behind start (0); the images have been begun.
-// landed(): behind the barrier after the first image.  fourth(): behind that after the fourth, by when all that was stored in front of the fifth's loads has arrived.
-template <int MW, int NW, int MT, int NT, class Landed, class Fourth>
+// landed(): behind the barrier after the first image.
+template <int MW, int NW, int MT, int NT, class Landed>
 __device__ __forceinline__ void expert_sums(f32x4 (&acc)[NT][MT], const ExpertFeed<GemmShape<MW, NW, MT, NT>>& feed, unsigned char* lds, int iters, const WaveRows& rows, int wave, int lane,
-                                            float start, Landed landed, Fourth fourth) {
+                                            float start, Landed landed) {
     using G = GemmShape<MW, NW, MT, NT>;
     constexpr int TN = G::TN, DMA = G::DMA;
     const int lq = lane & 15, lg = lane >> 4, wn = wave % NW, mine = rows.mine;
@@ -462,8 +462,6 @@ __device__ __forceinline__ void expert_sums(f32x4 (&acc)[NT][MT], const ExpertFe
         lds_only_barrier();
     };
     constexpr std::integral_constant<int, kRing - 2> in_flight{};
-    int two = 2;
-    asm("" : "+s"(two));                             // (not a loop peeled for it)
     // the products of this wave's first MTU tiles of pairs
     auto run = [&](auto mtu) __attribute__((always_inline)) {
         constexpr int MTU = decltype(mtu)::value;
@@ -502,7 +500,6 @@ __device__ __forceinline__ void expert_sums(f32x4 (&acc)[NT][MT], const ExpertFe
         read(0, even);
         for (int it = 0; it < iters; it += 2) {
             arrive(in_flight);
-            if (it == two) fourth();
             read(it + 1, odd);
             feed.stage_next(lds, it + kRing, iters, wave);
             multiply(even);
@@ -528,7 +525,6 @@ __device__ __forceinline__ void expert_sums(f32x4 (&acc)[NT][MT], const ExpertFe
     } else {
         for (int it = 0; it < iters; ++it) {
             arrive(in_flight);
-            if (it == two) fourth();
             feed.stage_next(lds, it + kRing, iters, wave);
         }
     }
@@ -610,7 +606,7 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
     feed.begin(lds, iters, wave);
     const WaveRows rows(to.live, wave / NW, MW);
     f32x4 acc[NT][MT];
-    expert_sums<MW, NW, MT, NT>(acc, feed, lds, iters, rows, wave, lane, 0.f, [] {}, [] {});
+    expert_sums<MW, NW, MT, NT>(acc, feed, lds, iters, rows, wave, lane, 0.f, [] {});
     expert_results<GLU, false, MW, NW, MT, NT>(acc, a, to, rows, lds + wave * 2048, wave, lane, [](int) {});
 }
 
@@ -620,11 +616,11 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
 // from the same list: they are in the hands of workgroups that run, and never wait; who waits keeps no other part waiting.  (No assumption on how many are resident, on their order,
 // or on who runs where; the wait is bounded all the same, and numbers of none behind it.)
 // What the second product reads is stored through to memory, announced behind the stores' arrival, and lies in lines of its own (rows of whole 128 bytes): no cache holds an older copy.
-// The next part is looked up, and its first images asked for if its rows are there, while this one's results leave: the ring is free by then, they have LDS of their own.  A workgroup's
-// loads and stores arrive in the order of their issue, so these stores are there when a later image is.
+// The next part is looked up, and its first images asked for if its rows are there, while this one's results leave: the ring is free by then, they have LDS of their own.
+// A wave waits for its stores once all are out, beside those images; they are announced behind the next part's first barrier.
 // Bound by the products while they run (0.95 us an image of 256 x 256, the rate of a large product at the clock the card keeps under it); a part of 64 images at 2048 wide is 60 us of those
 // and, before, 4.5 of lookups and first images and 6 to 8 of results.  3000 tokens, 32 experts of 1536: 371 us in two launches, 313 with the parts one after the other, 308 overlapped;
-// 12000 966, 935, 930; 1024 wide, of 768, 6000 176, 164, 160.
+// 12000 966, 935, 930; 1024 wide, of 768, 6000 176, 164, 160.  (Announced from the next part's loop without a wait of its own: 1 % slower, rows came later to those who waited)
 // Few operations on shared words: 256 workgroups that look at eight lists when theirs is at an end took 25 us for it.
 // this lane, not held in a register
 __device__ __forceinline__ int lane_now() {
@@ -739,9 +735,9 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_both_kernel(const MoeBothArg
         expert_sums<MW, NW, MT, NT>(
             acc, feed, lds, (now.glu ? a.up.k : a.down.k) / TK, rows, wave, lane, start,
             [&] {
+                announce_it();
                 if (wave == 0) settle(now.list, drawn);
-            },
-            [&] { announce_it(); });
+            });
         const auto between = [&](int h) __attribute__((always_inline)) {
             if (h == 0) {
                 take(then, lane_now());
@@ -756,6 +752,7 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_both_kernel(const MoeBothArg
         };
         if (now.glu) {
             expert_results<true, true, MW, NW, MT, NT>(acc, a.up, now.to, rows, room, wave, lane_now(), between);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                   // (announced behind the next barrier)
             announce = now.to.mt;
         } else {
             expert_results<false, false, MW, NW, MT, NT>(acc, a.down, now.to, rows, room, wave, lane_now(), between);
@@ -1012,7 +1009,7 @@ static int device_cus() {
 // costs: 2048 wide, 16384 tokens by sigmoids 1106 against 1118, by a softmax 1256 against 1240.  Tiles of 128 rows, two workgroups a CU, fill their rounds better as they are:
 // 32 experts of 1536, 2048 wide, 60 pairs 158 against 164.
 bool moe_one_launch(int pairs, int experts, int n, int cols, int tile_rows) {
-    if (tile_rows != 256 || pairs / experts < 180 || n > cols || n < 128) return false;       // (n: a part announces the one before it behind its fourth image of 32)
+    if (tile_rows != 256 || pairs / experts < 180 || n > cols) return false;
     const int64_t tiles = pairs / 256 + experts / 2, parts = tiles * ((n + 127) / 128 + (cols + 255) / 256);
     return 2 * parts >= 5 * device_cus() && parts < 20 * device_cus();
 }

@@ -624,7 +624,7 @@ def test_experts_in_one_call(rows, experts, top, dtype, softmax):
     assert out.shape == (0, cols) and weights.shape == (0, top)
 
 
-@pytest.mark.parametrize("rows,experts,top,cols,n", [(9000, 24, 4, 1024, 128), (3100, 33, 4, 2048, 320), (11000, 3, 2, 1536, 192), (4100, 9, 3, 2240, 640)])
+@pytest.mark.parametrize("rows,experts,top,cols,n", [(9000, 24, 4, 1024, 64), (3100, 33, 4, 2048, 320), (11000, 3, 2, 1536, 192), (4100, 9, 3, 2240, 640)])
 def test_experts_in_one_launch(rows, experts, top, cols, n):
     """Enough tiles for both products to share a launch: bit for bit two launches, alone, two calls at once on two streams, and from a graph with other rows behind it.  Experts of a few
     tiles and of more than a workgroup looks at; columns of either product that end inside a tile."""

@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 208          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels */
+#define NVH_VERSION 209          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -738,7 +738,7 @@ typedef struct nvh_moe_gemm_desc {
 int nvh_moe_tile_rows(int pairs, int experts, int dtype);     /* for experts of about 1024 columns (nvh_moe_experts goes by its own) */
 int nvh_moe_gemm(const nvh_moe_gemm_desc* d, int dtype, void* stream);
 /* Route, dispatch (the small form up to 64 rows in bf16: none) and both products in one call: the launches of the four entries above, in their order
-   (large batches: both products in one launch, the same results bit for bit). */
+   (large batches: both products in one launch, the same results bit for bit; not where `out` overlaps x or gate_up, which may hold them). */
 typedef struct nvh_moe_experts_desc {
     const void* x;               /* [rows, cols], row stride x_stride */
     int64_t x_stride;
@@ -755,6 +755,7 @@ typedef struct nvh_moe_experts_desc {
 } nvh_moe_experts_desc;
 size_t nvh_moe_experts_scratch_bytes(int rows, int top, int experts, int n, int dtype);
 int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream);
+int nvh_moe_experts_one_launch(const nvh_moe_experts_desc* d, int dtype);      /* 1: that call's products share a launch (host only) */
 
 /* x (fp32 stream) += mult * P(y + sum_k ew[row, k] * e[row * top + k])  (each part nullable; P: the layer norm with post_w and post_b where given, nothing
  * otherwise), x += base, x += shift, then, with w given, the layer norm of the new row: (x - mean) / sqrt(var + eps) * w + b. */

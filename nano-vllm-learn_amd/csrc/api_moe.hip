@@ -75,8 +75,27 @@ static bool moe_sizes_ok(int rows, int top, int experts, int n) {
     return rows > 0 && top > 0 && experts > 0 && experts <= kMoeMaxExperts && (int64_t)rows * top <= 0x7fffffff && n > 0 && n % 64 == 0;
 }
 
+// Both products in one launch: the rule of sizes, what the second one reads in lines of its own in the scratch, and outputs, which are stored while the first product still
+// runs, apart from what that reads (two launches let `out` hold x).
+static bool experts_in_one(const nvh_moe_experts_desc* d, const MoeScratch& s) {
+    const auto apart = [&](const void* p, int64_t elems) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(d->out);
+        return a + 2 * (uintptr_t)elems <= b || b + 2 * (uintptr_t)d->rows * d->top * d->cols <= a;
+    };
+    return s.link_words && (reinterpret_cast<uintptr_t>(d->scratch) & 127) == 0 && moe_one_launch(d->rows * d->top, d->experts, d->n, d->cols, s.rows) &&
+           apart(d->x, (d->rows - 1) * d->x_stride + d->cols) && apart(d->gate_up, (int64_t)d->experts * 2 * d->n * d->cols);
+}
+
 size_t nvh_moe_experts_scratch_bytes(int rows, int top, int experts, int n, int dtype) {
     return moe_sizes_ok(rows, top, experts, n) ? 4 * MoeScratch(rows, top, experts, n, dtype).words : 0;
+}
+
+int nvh_moe_experts_one_launch(const nvh_moe_experts_desc* d, int dtype) {
+    REQUIRE(d, NVH_E_NULL, "moe_experts_one_launch: null descriptor");
+    if (d->rows == 0) return 0;
+    DTYPE("moe_experts_one_launch");
+    REQUIRE(moe_sizes_ok(d->rows, d->top, d->experts, d->n) && d->cols > 0, NVH_E_SHAPE, "moe_experts_one_launch: sizes");
+    return experts_in_one(d, MoeScratch(d->rows, d->top, d->experts, d->n, dtype));
 }
 
 int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream) {
@@ -102,8 +121,7 @@ int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream) {
     g.out = at; g.x = d->x; g.x_stride = d->x_stride; g.w = d->gate_up;
     g.pairs = pairs; g.top = d->top; g.experts = d->experts; g.n = d->n; g.k = d->cols; g.glu = 1; g.limit = d->limit; g.alpha = d->alpha;
     g.ids = ids;
-    // both products in one launch: what the second one reads has lines of its own in the scratch
-    const bool both = s.link_words && ((uintptr_t)d->scratch & 127) == 0 && moe_one_launch(pairs, d->experts, d->n, d->cols, s.rows);
+    const bool both = experts_in_one(d, s);
     uint32_t* const links = reinterpret_cast<uint32_t*>(at + s.links);
     if (s.rows) {
         rc = launch_moe_dispatch(at + s.slots, at + s.tiles, at + s.counts, ids, pairs, d->experts, s.rows, s.max_tiles, both ? links : nullptr, both ? s.link_words : 0, (hipStream_t)stream);

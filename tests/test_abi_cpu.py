@@ -114,6 +114,27 @@ def test_experts_in_one_call_refuse_scratch_that_is_too_small(lib):
     assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == 0
 
 
+def test_experts_share_a_launch_where_nothing_read_is_overwritten(lib):
+    """Both products in one launch store outputs while rows and weights are still read: not where they overlap (two launches let them).  By the rule of sizes; scratch on whole lines."""
+    from nanovllm_hip import _lib
+    rows, cols, n, experts, top = 9000, 1024, 64, 24, 4
+    out, x, w, scratch = 1 << 40, 1 << 41, 1 << 42, 1 << 43
+    size, stride = 2 * rows * top * cols, cols + 64
+
+    def one(dtype=0, **kw):
+        d = _lib.MoeExpertsDesc(x, stride, w, w, w, w, rows, cols, n, experts, top, 1, 1, 0, 1.0, 0.0, 0.0, scratch, lib.nvh_moe_experts_scratch_bytes(rows, top, experts, n, 0), out, w)
+        for name, value in kw.items():
+            setattr(d, name, value)
+        return lib.nvh_moe_experts_one_launch(ctypes.byref(d), dtype)
+    used, weights = 2 * ((rows - 1) * stride + cols), 2 * experts * 2 * n * cols
+    assert one() == 1
+    assert [one(x=out + at) for at in (-used, 16 - used, 0, 4096, size - 16, size)] == [1, 0, 0, 0, 0, 1]
+    assert [one(gate_up=out + at) for at in (-weights, 16 - weights, 0, size - 16, size)] == [1, 0, 0, 0, 1]
+    assert [one(scratch=scratch + at) for at in (16, 64, 128)] == [0, 0, 1]
+    assert one(dtype=1) == 0 and one(rows=60) == 0 and one(rows=700) == 0 and one(rows=0) == 0
+    assert one(dtype=9) == -1 and lib.nvh_moe_experts_one_launch(None, 0) == -5 and one(n=60) == -2
+
+
 @pytest.mark.parametrize("experts,rows", [(8, {16: 64, 25: 64, 26: 128, 109: 128, 110: 256, 192: 256, 193: 128, 240: 128, 256: 128, 287: 128, 288: 256}),
                                           (32, {25: 64, 100: 128, 192: 256, 193: 256, 240: 256, 241: 128, 256: 128, 288: 256}),
                                           (64, {16: 64, 17: 128, 25: 128, 100: 128, 240: 256, 241: 128, 255: 128, 256: 256}), (96, {99: 128, 100: 256, 109: 256, 241: 128, 256: 256})])

@@ -657,6 +657,46 @@ def test_experts_in_one_launch(rows, experts, top, cols, n):
         assert torch.equal(kept, want[i])
 
 
+def experts_call(x, router, bias, gu, dn, top, out, spare=0):
+    """(descriptor, weights, scratch): nvh_moe_experts with outputs, and scratch `spare` bytes behind 256, of the caller's."""
+    from nanovllm_hip import _lib
+    rows, cols, n = x.shape[0], x.shape[1], dn.shape[2]
+    size = _lib.load().nvh_moe_experts_scratch_bytes(rows, top, len(gu), n, 0)
+    scratch, weights = torch.full((size + 512,), 7, dtype=torch.uint8, device="cuda"), torch.empty(rows, top, device="cuda")
+    at = (scratch.data_ptr() + 255) // 256 * 256 + spare
+    d = _lib.MoeExpertsDesc(x.data_ptr(), x.stride(0), router.data_ptr(), bias.data_ptr(), gu.data_ptr(), dn.data_ptr(), rows, cols, n, len(gu), top, 1, 1, 0, 1.0, 0.0, 0.0, at, size,
+                            out.data_ptr(), weights.data_ptr())
+    return d, weights, scratch
+
+
+def run_experts(d):
+    """Whether both products shared a launch."""
+    import ctypes
+    from nanovllm_hip import _lib
+    lib = _lib.load()
+    assert lib.nvh_moe_experts(ctypes.byref(d), 0, torch.cuda.current_stream().cuda_stream) == 0, lib.nvh_last_error()
+    return lib.nvh_moe_experts_one_launch(ctypes.byref(d), 0)
+
+
+ONE_LAUNCH = [(9000, 24, 4, 1024, 64), (3100, 33, 4, 2048, 320), (11000, 3, 2, 1536, 192), (4100, 9, 3, 2240, 640)]
+
+
+@pytest.mark.parametrize("first", [0, 100, 27000])
+def test_experts_whose_rows_lie_in_the_outputs(first):
+    """`out` may hold x: the same bits as apart from it."""
+    from nanovllm_hip import ops
+    rows, experts, top, cols, n = ONE_LAUNCH[0]
+    x, router, bias = randn(rows, cols, seed=1).cuda(), randn(experts, cols, seed=3, scale=cols ** -0.5).cuda(), randn(experts, seed=4, dtype=F32).cuda()
+    gu, dn = (randn(experts, *shape, seed=5, scale=shape[1] ** -0.5).cuda() for shape in ((2 * n, cols), (cols, n)))
+    want, weights = ops.moe_experts(x, router, bias, gu, dn, top)
+    out = torch.empty_like(want)
+    d, got_weights, _ = experts_call(out[first:first + rows], router, bias, gu, dn, top, out)
+    for _ in range(3):
+        out[first:first + rows] = x
+        assert run_experts(d) == 0
+        assert torch.equal(out, want) and torch.equal(got_weights, weights)
+
+
 # ------------------------------------------------------------------------------------------------ residual, norm, cap
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,cols,n,top", [(3, 64, 64, 0), (5, 320, 300, 4), (17, 2048, 2048, 8), (2, 8192, 8190, 3)])

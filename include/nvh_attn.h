@@ -748,7 +748,7 @@ typedef struct nvh_moe_experts_desc {
     const void* down;            /* [experts, cols, n] */
     int32_t rows, cols, n, experts, top, groups, keep, softmax;
     float scale, limit, alpha;
-    void* scratch;               /* nvh_moe_experts_scratch_bytes, 16-byte aligned */
+    void* scratch;               /* nvh_moe_experts_scratch_bytes, 16-byte aligned.  Off 128 bytes, or without the last (8 + tiles) * 128 of those (what two launches need): two launches */
     size_t scratch_bytes;
     void* out;                   /* [rows * top, cols] */
     float* weights;              /* [rows, top] */

@@ -75,14 +75,14 @@ static bool moe_sizes_ok(int rows, int top, int experts, int n) {
     return rows > 0 && top > 0 && experts > 0 && experts <= kMoeMaxExperts && (int64_t)rows * top <= 0x7fffffff && n > 0 && n % 64 == 0;
 }
 
-// Both products in one launch: the rule of sizes, what the second one reads in lines of its own in the scratch, and outputs, which are stored while the first product still
+// Both products in one launch: the rule of sizes, scratch with room for its links and what the second one reads in lines of its own, and outputs, which are stored while the first product still
 // runs, apart from what that reads (two launches let `out` hold x).
 static bool experts_in_one(const nvh_moe_experts_desc* d, const MoeScratch& s) {
     const auto apart = [&](const void* p, int64_t elems) {
         const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(d->out);
         return a + 2 * (uintptr_t)elems <= b || b + 2 * (uintptr_t)d->rows * d->top * d->cols <= a;
     };
-    return s.link_words && (reinterpret_cast<uintptr_t>(d->scratch) & 127) == 0 && moe_one_launch(d->rows * d->top, d->experts, d->n, d->cols, s.rows) &&
+    return s.link_words && d->scratch_bytes >= 4 * s.words && (reinterpret_cast<uintptr_t>(d->scratch) & 127) == 0 && moe_one_launch(d->rows * d->top, d->experts, d->n, d->cols, s.rows) &&
            apart(d->x, (d->rows - 1) * d->x_stride + d->cols) && apart(d->gate_up, (int64_t)d->experts * 2 * d->n * d->cols);
 }
 
@@ -107,7 +107,7 @@ int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream) {
     const MoeScratch s(d->rows, d->top, d->experts, d->n, dtype);
     REQUIRE(d->scratch, NVH_E_NULL, "moe_experts: null pointer");
     REQUIRE(aligned16(d->scratch), NVH_E_ALIGN, "moe_experts: scratch must be 16-byte aligned");
-    REQUIRE(d->scratch_bytes >= 4 * s.words, NVH_E_WORKSPACE, "moe_experts: scratch %zu B < required %zu B", d->scratch_bytes, 4 * s.words);
+    REQUIRE(d->scratch_bytes >= 4 * s.links, NVH_E_WORKSPACE, "moe_experts: scratch %zu B < required %zu B", d->scratch_bytes, 4 * s.links);
     int32_t* at = reinterpret_cast<int32_t*>(d->scratch);
     int32_t* const ids = at + s.ids;
     const int pairs = d->rows * d->top;

@@ -131,6 +131,12 @@ def test_experts_share_a_launch_where_nothing_read_is_overwritten(lib):
     assert [one(x=out + at) for at in (-used, 16 - used, 0, 4096, size - 16, size)] == [1, 0, 0, 0, 0, 1]
     assert [one(gate_up=out + at) for at in (-weights, 16 - weights, 0, size - 16, size)] == [1, 0, 0, 0, 1]
     assert [one(scratch=scratch + at) for at in (16, 64, 128)] == [0, 0, 1]
+    full, least = lib.nvh_moe_experts_scratch_bytes(rows, top, experts, n, 0), 4 * (rows * top * n // 2 + 2 * rows * top + 4 * (rows * top // 256 + experts) + 18 * experts)
+    assert full == least + 128 * (8 + rows * top // 256 + experts) and [one(scratch_bytes=b) for b in (full, full - 4, least)] == [1, 0, 0]
+    d = _lib.MoeExpertsDesc(x, stride, w, w, w, w, rows, cols, n, experts, top, 1, 1, 0, 1.0, 0.0, 0.0, scratch, least - 4, out, None)
+    assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == -4 and str(least).encode() in lib.nvh_last_error()
+    d.scratch_bytes = least
+    assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == -5 and b"moe_route" in lib.nvh_last_error()     # (enough: the next check is another one)
     assert one(dtype=1) == 0 and one(rows=60) == 0 and one(rows=700) == 0 and one(rows=0) == 0
     assert one(dtype=9) == -1 and lib.nvh_moe_experts_one_launch(None, 0) == -5 and one(n=60) == -2
 

@@ -697,6 +697,23 @@ def test_experts_whose_rows_lie_in_the_outputs(first):
         assert torch.equal(out, want) and torch.equal(got_weights, weights)
 
 
+@pytest.mark.parametrize("spare,short,one", [(0, 0, 1), (16, 0, 0), (0, 128 * (8 + 140 + 24), 0)])
+def test_experts_scratch_that_allows_two_launches_only(spare, short, one):
+    """Scratch off whole lines, and as little as two launches need: the same bits, and nothing behind it is touched."""
+    from nanovllm_hip import ops
+    rows, experts, top, cols, n = ONE_LAUNCH[0]
+    x, router, bias = randn(rows, cols, seed=1).cuda(), randn(experts, cols, seed=3, scale=cols ** -0.5).cuda(), randn(experts, seed=4, dtype=F32).cuda()
+    gu, dn = (randn(experts, *shape, seed=5, scale=shape[1] ** -0.5).cuda() for shape in ((2 * n, cols), (cols, n)))
+    want, weights = ops.moe_experts(x, router, bias, gu, dn, top)
+    out = torch.empty_like(want)
+    d, got_weights, scratch = experts_call(x, router, bias, gu, dn, top, out, spare)
+    d.scratch_bytes -= short
+    assert run_experts(d) == one
+    assert torch.equal(out, want) and torch.equal(got_weights, weights)
+    end = d.scratch + d.scratch_bytes - scratch.data_ptr()
+    assert (scratch[:d.scratch - scratch.data_ptr()] == 7).all() and (scratch[end:] == 7).all()
+
+
 # ------------------------------------------------------------------------------------------------ residual, norm, cap
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,cols,n,top", [(3, 64, 64, 0), (5, 320, 300, 4), (17, 2048, 2048, 8), (2, 8192, 8190, 3)])

@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 209          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch */
+#define NVH_VERSION 209          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch, _status, _variant */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -756,6 +756,10 @@ typedef struct nvh_moe_experts_desc {
 size_t nvh_moe_experts_scratch_bytes(int rows, int top, int experts, int n, int dtype);
 int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream);
 int nvh_moe_experts_one_launch(const nvh_moe_experts_desc* d, int dtype);      /* 1: that call's products share a launch (host only) */
+/* There a part of the second product waits (bounded, seconds; for workgroups that run) for rows of the first.  Behind a wait that ran out its outputs are NaN, and the status of that call,
+ * read from its scratch, is 1 (host-synchronous, not capturable; 0 for two launches).  The variant, for tests: wait_limit polls (0: as usual) and so many stores that nobody makes waited for. */
+int nvh_moe_experts_status(const nvh_moe_experts_desc* d, int dtype, uint32_t* ran_out);
+int nvh_moe_experts_variant(uint32_t wait_limit, uint32_t missing, const nvh_moe_experts_desc* d, int dtype, void* stream);
 
 /* x (fp32 stream) += mult * P(y + sum_k ew[row, k] * e[row * top + k])  (each part nullable; P: the layer norm with post_w and post_b where given, nothing
  * otherwise), x += base, x += shift, then, with w given, the layer norm of the new row: (x - mean) / sqrt(var + eps) * w + b. */

@@ -1,5 +1,5 @@
 // C ABI of the mixture of experts (declared in include/nvh_attn.h): argument validation, dispatch.
-// Nothing here allocates, synchronises or reads device memory: every entry point is capture-safe.
+// Nothing here allocates, synchronises or reads device memory, nvh_moe_experts_status aside: every other entry point is capture-safe.
 #include "api_common.h"
 #include "mixers.h"
 
@@ -98,7 +98,7 @@ int nvh_moe_experts_one_launch(const nvh_moe_experts_desc* d, int dtype) {
     return experts_in_one(d, MoeScratch(d->rows, d->top, d->experts, d->n, dtype));
 }
 
-int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream) {
+static int moe_experts(const nvh_moe_experts_desc* d, int dtype, uint32_t wait_limit, uint32_t missing, void* stream) {
     REQUIRE(d, NVH_E_NULL, "moe_experts: null descriptor");
     if (d->rows == 0) return 0;
     DTYPE("moe_experts");
@@ -133,10 +133,26 @@ int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream) {
     down.out = d->out; down.x = at; down.w = d->down; down.n = d->cols; down.k = d->n; down.glu = 0; down.limit = down.alpha = 0.f;
     if (both) {
         if ((rc = moe_gemm_ok(&g, dtype)) || (rc = moe_gemm_ok(&down, dtype))) return rc;
-        return launch_moe_both(g, down, links, (hipStream_t)stream);
+        return launch_moe_both(g, down, links, wait_limit, missing, (hipStream_t)stream);
     }
     rc = nvh_moe_gemm(&g, dtype, stream);
     return rc ? rc : nvh_moe_gemm(&down, dtype, stream);
+}
+
+int nvh_moe_experts(const nvh_moe_experts_desc* d, int dtype, void* stream) { return moe_experts(d, dtype, 0, 0, stream); }
+
+int nvh_moe_experts_variant(uint32_t wait_limit, uint32_t missing, const nvh_moe_experts_desc* d, int dtype, void* stream) { return moe_experts(d, dtype, wait_limit, missing, stream); }
+
+int nvh_moe_experts_status(const nvh_moe_experts_desc* d, int dtype, uint32_t* ran_out) {
+    REQUIRE(ran_out, NVH_E_NULL, "moe_experts_status: null pointer");
+    *ran_out = 0;
+    const int one = nvh_moe_experts_one_launch(d, dtype);
+    if (one <= 0) return one;
+    const MoeScratch s(d->rows, d->top, d->experts, d->n, dtype);
+    hipError_t e = hipDeviceSynchronize();
+    if (e == hipSuccess) e = hipMemcpy(ran_out, moe_ran_out(reinterpret_cast<const uint32_t*>(d->scratch) + s.links), sizeof(uint32_t), hipMemcpyDeviceToHost);
+    REQUIRE(e == hipSuccess, (int)e, "moe_experts_status: %s", hipGetErrorString(e));
+    return 0;
 }
 
 }  // extern "C"

@@ -44,7 +44,8 @@ int launch_moe_dispatch(int32_t* slot_pair, int32_t* tiles, int32_t* counts, con
                         uint32_t* clear, size_t clear_words, hipStream_t stream);      // (clear: words set to zero besides)
 bool moe_one_launch(int pairs, int experts, int n, int cols, int tile_rows);
 size_t moe_links_words(int tile_rows, int max_tiles);    // of that launch
-int launch_moe_both(const MoeGemmArgs& up, const MoeGemmArgs& down, uint32_t* tickets, hipStream_t stream);
+int launch_moe_both(const MoeGemmArgs& up, const MoeGemmArgs& down, uint32_t* tickets, uint32_t wait_limit, uint32_t missing, hipStream_t stream);
+const uint32_t* moe_ran_out(const uint32_t* tickets);    // its word: 1 after a wait that ran out
 int moe_tile_rows(int pairs, int experts, int n, int f32);
 int launch_moe_gemm(const MoeGemmArgs& a, int f32, hipStream_t stream);
 

@@ -614,7 +614,7 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
 // A row of tiles is split over eight lists, one for the workgroups of an XCD; a list is its tiles' parts of the first product and behind them those of the second one, drawn by ticket.
 // Whose list is at an end draws from the next one's.  A part of the second product waits until all columns of its row tile are stored, and those were drawn before it
 // from the same list: they are in the hands of workgroups that run, and never wait; who waits keeps no other part waiting.  (No assumption on how many are resident, on their order,
-// or on who runs where; the wait is bounded all the same, and numbers of none behind it.)
+// or on who runs where; the wait is bounded all the same: behind one that ran out the part's outputs are NaN, and a word beside the tickets says so.)
 // What the second product reads is stored through to memory, announced behind the stores' arrival, and lies in lines of its own (rows of whole 128 bytes): no cache holds an older copy.
 // The next part is looked up, and its first images asked for if its rows are there, while this one's results leave: the ring is free by then, they have LDS of their own.
 // A wave waits for its stores once all are out, beside those images; they are announced behind the next part's first barrier.
@@ -628,10 +628,12 @@ __device__ __forceinline__ int lane_now() {
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n v_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
     return l;
 }
-constexpr int kListWords = 32, kWaitLimit = 1 << 22; // tickets a line each; polls of about a microsecond
+constexpr int kListWords = 32, kRanOut = 16;         // tickets a line each; in the first line, whether a wait ran out
+constexpr uint32_t kWaitLimit = 1 << 22;             // polls of about a microsecond
 struct MoeBothArgs {
     MoeGemmArgs up, down;
     uint32_t* tickets;                               // [8][kListWords], zero; then per row tile its stored columns, [tiles][kListWords], zero
+    uint32_t wait_limit, missing;                    // columns waited for that nobody stores (tests: the wait that runs out)
 };
 template <int MW, int NW, int MT, int NT>
 constexpr size_t both_lds_bytes() { return GemmShape<MW, NW, MT, NT>::LDS + MW * NW * 2048 + 16; }
@@ -692,6 +694,7 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_both_kernel(const MoeBothArg
         const ExpertTile to = find_tile<G::TM, G::UNIT>(a.up.tiles, tiles, part.glu ? nx : ny, part.glu ? number : number - first, lo, hi, tiles < 128 ? 4 : 8, lane);
         part.to = ExpertTile{uniform(to.nt), uniform(to.mt), uniform(to.expert), uniform(to.first), uniform(to.live)};
     };
+    const uint32_t all_columns = (uint32_t)nx + a.missing;
     const auto columns = [&](int mt) { return __hip_atomic_load(stored + mt * kListWords, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     int announce = -1;                               // a row tile whose columns are on their way to memory
     const auto announce_it = [&]() {
@@ -719,9 +722,10 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_both_kernel(const MoeBothArg
             arrived();                               // (before it waits for anyone)
             if (!then.glu) {
                 if (wave == 0 && lane_now() == 0) {
-                    int tries = 0;
-                    while (columns(then.to.mt) < (uint32_t)nx && ++tries < kWaitLimit) __builtin_amdgcn_s_sleep(8);
-                    next[2] = tries < kWaitLimit;
+                    uint32_t tries = 0;
+                    while (columns(then.to.mt) < all_columns && ++tries < a.wait_limit) __builtin_amdgcn_s_sleep(8);
+                    next[2] = tries < a.wait_limit;
+                    if (tries >= a.wait_limit) __hip_atomic_store(a.tickets + kRanOut, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
                 lds_only_barrier();
                 if (!uniform(next[2])) start = __uint_as_float(0x7FC00000u);
@@ -743,7 +747,7 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_both_kernel(const MoeBothArg
                 take(then, lane_now());
             } else if (h == 1) {
                 if (then.list >= 0) feed.aim(then.glu, then.glu ? a.up : a.down, then.to, wave, lane_now());
-                if (wave == 0 && lane_now() == 0) next[2] = then.list >= 0 && (then.glu || columns(then.to.mt) >= (uint32_t)nx);
+                if (wave == 0 && lane_now() == 0) next[2] = then.list >= 0 && (then.glu || columns(then.to.mt) >= all_columns);
             } else {
                 lds_only_barrier();
                 begun = uniform(next[2]);
@@ -1015,12 +1019,15 @@ bool moe_one_launch(int pairs, int experts, int n, int cols, int tile_rows) {
 }
 size_t moe_links_words(int tile_rows, int max_tiles) { return tile_rows == 256 ? (size_t)(8 + max_tiles) * kListWords : 0; }
 
-int launch_moe_both(const MoeGemmArgs& up, const MoeGemmArgs& down, uint32_t* tickets, hipStream_t stream) {
+const uint32_t* moe_ran_out(const uint32_t* tickets) { return tickets + kRanOut; }
+
+int launch_moe_both(const MoeGemmArgs& up, const MoeGemmArgs& down, uint32_t* tickets, uint32_t wait_limit, uint32_t missing, hipStream_t stream) {
     using G = GemmShape<2, 4, 8, 4>;
     const size_t lds = both_lds_bytes<2, 4, 8, 4>();
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(moe_both_kernel<2, 4, 8, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const int64_t parts = (int64_t)up.max_tiles * ((up.n + G::TN / 2 - 1) / (G::TN / 2) + (down.n + G::TN - 1) / G::TN);
-    moe_both_kernel<2, 4, 8, 4><<<(int)(parts < device_cus() ? parts : device_cus()), 64 * G::WAVES, lds, stream>>>(MoeBothArgs{up, down, tickets});
+    moe_both_kernel<2, 4, 8, 4><<<(int)(parts < device_cus() ? parts : device_cus()), 64 * G::WAVES, lds, stream>>>(
+        MoeBothArgs{up, down, tickets, wait_limit ? wait_limit : kWaitLimit, missing});
     return check_launch("moe_both");
 }
 

@@ -318,6 +318,8 @@ _SIGS = {
     "nvh_moe_experts_scratch_bytes": (ctypes.c_size_t, [ctypes.c_int] * 5),
     "nvh_moe_experts": (ctypes.c_int, [ctypes.POINTER(MoeExpertsDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_moe_experts_one_launch": (ctypes.c_int, [ctypes.POINTER(MoeExpertsDesc), ctypes.c_int]),
+    "nvh_moe_experts_status": (ctypes.c_int, [ctypes.POINTER(MoeExpertsDesc), ctypes.c_int, ctypes.POINTER(ctypes.c_uint32)]),
+    "nvh_moe_experts_variant": (ctypes.c_int, [ctypes.c_uint32, ctypes.c_uint32, ctypes.POINTER(MoeExpertsDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_residual_norm": (ctypes.c_int, [ctypes.POINTER(ResidualNormDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_poly_norm": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_float] + [ctypes.c_int] * 3 + [ctypes.c_int64] * 2 + [ctypes.c_int, ctypes.c_void_p]),
     "nvh_softcap": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),

@@ -138,6 +138,9 @@ def test_experts_share_a_launch_where_nothing_read_is_overwritten(lib):
     d.scratch_bytes = least
     assert lib.nvh_moe_experts(ctypes.byref(d), 0, None) == -5 and b"moe_route" in lib.nvh_last_error()     # (enough: the next check is another one)
     assert one(dtype=1) == 0 and one(rows=60) == 0 and one(rows=700) == 0 and one(rows=0) == 0
+    ran_out = ctypes.c_uint32(5)
+    assert lib.nvh_moe_experts_status(None, 0, ctypes.byref(ran_out)) == -5 and lib.nvh_moe_experts_status(ctypes.byref(d), 0, None) == -5
+    assert lib.nvh_moe_experts_status(ctypes.byref(d), 0, ctypes.byref(ran_out)) == 0 and ran_out.value == 0         # (two launches: none waits)
     assert one(dtype=9) == -1 and lib.nvh_moe_experts_one_launch(None, 0) == -5 and one(n=60) == -2
 
 

@@ -624,39 +624,6 @@ def test_experts_in_one_call(rows, experts, top, dtype, softmax):
     assert out.shape == (0, cols) and weights.shape == (0, top)
 
 
-@pytest.mark.parametrize("rows,experts,top,cols,n", [(9000, 24, 4, 1024, 64), (3100, 33, 4, 2048, 320), (11000, 3, 2, 1536, 192), (4100, 9, 3, 2240, 640)])
-def test_experts_in_one_launch(rows, experts, top, cols, n):
-    """Enough tiles for both products to share a launch: bit for bit two launches, alone, two calls at once on two streams, and from a graph with other rows behind it.  Experts of a few
-    tiles and of more than a workgroup looks at; columns of either product that end inside a tile."""
-    from nanovllm_hip import ops
-    xs = [randn(rows, cols, seed=s).cuda() for s in (1, 2)]
-    router, bias = randn(experts, cols, seed=3, scale=cols ** -0.5).cuda(), randn(experts, seed=4, dtype=F32).cuda()
-    gu, dn = (randn(experts, *shape, seed=5, scale=shape[1] ** -0.5).cuda() for shape in ((2 * n, cols), (cols, n)))
-
-    def four(x):
-        ids, _ = ops.moe_route(x, router, bias, top)
-        dispatch = ops.moe_dispatch(ids, experts, BF16, 256)
-        return ops.moe_gemm(ops.moe_gemm(x, gu, ids, True, dispatch), dn, ids, False, dispatch)
-    want = [four(x) for x in xs]
-    assert torch.equal(ops.moe_experts(xs[0], router, bias, gu, dn, top)[0], want[0])
-    streams, got = [torch.cuda.Stream() for _ in xs], [[], []]
-    torch.cuda.synchronize()
-    for _ in range(3):
-        for i, stream in enumerate(streams):
-            with torch.cuda.stream(stream):
-                got[i].append(ops.moe_experts(xs[i], router, bias, gu, dn, top)[0])
-    torch.cuda.synchronize()
-    assert all(torch.equal(g, want[i]) for i in (0, 1) for g in got[i])
-    x, graph = xs[0].clone(), torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        kept, _ = ops.moe_experts(x, router, bias, gu, dn, top)
-    for i in (1, 0, 1):
-        x.copy_(xs[i])
-        graph.replay()
-        torch.cuda.synchronize()
-        assert torch.equal(kept, want[i])
-
-
 def experts_call(x, router, bias, gu, dn, top, out, spare=0):
     """(descriptor, weights, scratch): nvh_moe_experts with outputs, and scratch `spare` bytes behind 256, of the caller's."""
     from nanovllm_hip import _lib
@@ -679,6 +646,41 @@ def run_experts(d):
 
 
 ONE_LAUNCH = [(9000, 24, 4, 1024, 64), (3100, 33, 4, 2048, 320), (11000, 3, 2, 1536, 192), (4100, 9, 3, 2240, 640)]
+
+
+@pytest.mark.parametrize("rows,experts,top,cols,n", ONE_LAUNCH)
+def test_experts_in_one_launch(rows, experts, top, cols, n):
+    """Enough tiles for both products to share a launch: bit for bit two launches, alone, two calls at once on two streams, and from a graph with other rows behind it.  Experts of a few
+    tiles and of more than a workgroup looks at; columns of either product that end inside a tile."""
+    from nanovllm_hip import ops
+    xs = [randn(rows, cols, seed=s).cuda() for s in (1, 2)]
+    router, bias = randn(experts, cols, seed=3, scale=cols ** -0.5).cuda(), randn(experts, seed=4, dtype=F32).cuda()
+    gu, dn = (randn(experts, *shape, seed=5, scale=shape[1] ** -0.5).cuda() for shape in ((2 * n, cols), (cols, n)))
+
+    def four(x):
+        ids, _ = ops.moe_route(x, router, bias, top)
+        dispatch = ops.moe_dispatch(ids, experts, BF16, 256)
+        return ops.moe_gemm(ops.moe_gemm(x, gu, ids, True, dispatch), dn, ids, False, dispatch)
+    want = [four(x) for x in xs]
+    out = torch.empty_like(want[0])
+    assert run_experts(experts_call(xs[0], router, bias, gu, dn, top, out)[0]) == 1 and torch.equal(out, want[0])
+    assert torch.equal(ops.moe_experts(xs[0], router, bias, gu, dn, top)[0], want[0])
+    streams, got = [torch.cuda.Stream() for _ in xs], [[], []]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for i, stream in enumerate(streams):
+            with torch.cuda.stream(stream):
+                got[i].append(ops.moe_experts(xs[i], router, bias, gu, dn, top)[0])
+    torch.cuda.synchronize()
+    assert all(torch.equal(g, want[i]) for i in (0, 1) for g in got[i])
+    x, graph = xs[0].clone(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        kept, _ = ops.moe_experts(x, router, bias, gu, dn, top)
+    for i in (1, 0, 1):
+        x.copy_(xs[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(kept, want[i])
 
 
 @pytest.mark.parametrize("first", [0, 100, 27000])
@@ -712,6 +714,27 @@ def test_experts_scratch_that_allows_two_launches_only(spare, short, one):
     assert torch.equal(out, want) and torch.equal(got_weights, weights)
     end = d.scratch + d.scratch_bytes - scratch.data_ptr()
     assert (scratch[:d.scratch - scratch.data_ptr()] == 7).all() and (scratch[end:] == 7).all()
+
+
+def test_experts_behind_a_wait_that_ran_out():
+    """Told to wait for stores that nobody makes, the second product gives up: NaN everywhere and a status, never a plausible number; the next call with that scratch is clean."""
+    import ctypes
+    from nanovllm_hip import _lib, ops
+    lib, ran_out = _lib.load(), ctypes.c_uint32()
+    rows, experts, top, cols, n = ONE_LAUNCH[0]
+    x, router, bias = randn(rows, cols, seed=1).cuda(), randn(experts, cols, seed=3, scale=cols ** -0.5).cuda(), randn(experts, seed=4, dtype=F32).cuda()
+    gu, dn = (randn(experts, *shape, seed=5, scale=shape[1] ** -0.5).cuda() for shape in ((2 * n, cols), (cols, n)))
+    want = ops.moe_experts(x, router, bias, gu, dn, top)[0]
+    out = torch.zeros_like(want)
+    d, _, _ = experts_call(x, router, bias, gu, dn, top, out)
+
+    def status():
+        assert lib.nvh_moe_experts_status(ctypes.byref(d), 0, ctypes.byref(ran_out)) == 0
+        return ran_out.value
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.nvh_moe_experts_variant(3, 1, ctypes.byref(d), 0, stream) == 0
+    assert status() == 1 and torch.isnan(out).all()
+    assert run_experts(d) == 1 and status() == 0 and torch.equal(out, want)
 
 
 # ------------------------------------------------------------------------------------------------ residual, norm, cap

@@ -166,6 +166,13 @@ struct PageNumbers {
     }
 };
 
+// this lane, not held in a register
+__device__ __forceinline__ int lane_now() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n v_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+
 // Lane with the nth largest of the values (0 .. 2^BITS - 1) in lanes 0 .. count - 1, equal ones in order; the same in all lanes.  One ballot and a few scalar instructions a bit.
 template <int BITS>
 __device__ __forceinline__ int nth_largest(int value, int count, int nth) {

@@ -276,74 +276,90 @@ constexpr size_t pair_lds_bytes(bool summary) {
 // values only: kFollow of a chunk) and goes on from there with outputs: the same operations on the same numbers, no summary and no launch in front.  Both would read a state that the
 // second one replaces: portions behind a state stay whole, and with them all of the launch.
 // A workgroup a CU walks at its own pace, so the longest portion sets the time, 1.6 to 1.75 of the mean.  As many pieces are made as bring the longest one (a chunk to start, and those that
-// it takes), the even load (times kUneven, what the order by length leaves on it) and the first to wait for a CU down together.  Eight sets of lengths each, 16 heads of 128: 16384 tokens
-// of 16 1.11 times as fast (130 -> 94, 100 -> 95), 9000 of 14 1.18 (82 -> 64), 12000 of 19 1.00 (0.95 to 1.04); 8 heads, 14000 of 28 1.13.  kFollow 0.6: 1.10, 1.17, 1.00, 1.13; kUneven 1.1: 1.11,
-// 1.18, 1.00, 1.12; without the wait for a CU 1.08, 1.13, 1.00, 1.09, one of 32 sets at 0.83.
-// (a wave) The nth walk, the longest first: portion, tokens followed, end in tokens; portion -1: none.
+// it takes), the even load (times kUneven, what the order by length leaves on it) and the pairs below down together.
+// A workgroup begins with a portion of its own, whole, while its first wave weighs the lengths, and learns behind the first chunk's images where to stop.  Second pieces go to workgroups
+// without a portion where CUs are left, and in place of the shortest portions where not; those then go behind the next shortest ones, in the same workgroup.  (Chosen first, with a workgroup
+// for every piece that there might be: 2.2 us in front of each, and 1 to 2 at the end of the launch for those that had none; lengths much alike 0.93 to 0.96 of the speed of whole portions,
+// 31 portions of 8 heads 0.88.)
+// Eight sets of lengths each, 16 heads of 128, against whole portions: 16384 tokens of 16 1.21 times as fast (128 -> 106 us), 9000 of 14 1.16, 12000 of 19 1.11; 8 heads, 14000 of 28 1.17.
+// Lengths of 0.9 to 1.1 of their mean, which are not cut, and launches with a portion behind a state: 0.99 (0.9 us, half of it the choice).
 constexpr int kSplitPortions = 32;
-constexpr float kFollow = 0.5f, kUneven = 1.2f;
+constexpr float kFollow = 0.5f, kUneven = 1.2f, kLate = 0.6f;                  // (a second piece starts behind the choice)
+// of the portions that run at once, those cut at most (11)
+__host__ __device__ __forceinline__ int lightning_most_cut(int places) { return places * 5 / 16; }
 struct LightningWalk {
-    int seg, from, to;
+    int seg, from, to, next;                         // portion (-1: none), tokens followed, end in tokens; the portion behind it (-1: none)
+    int row0, rows;                                  // of the portion
 };
-__device__ __forceinline__ LightningWalk lightning_walk_of(const LightningArgs& a, int walks_each, int nth) {
-    const int lane = threadIdx.x & 63, i = lane & 31;
-    const int listed = i < a.n_chunks ? a.chunks[4 * i + 1] : 0, rows = listed > 0 ? listed : 0;
-    const bool behind = rows > 0 && a.positions[a.chunks[4 * i]] > 0;
-    if (__builtin_amdgcn_ballot_w64(behind)) {
-        if (nth >= a.n_chunks) return LightningWalk{-1, 0, 0};
-        const int steps = (rows + 15) >> 4;
-        return LightningWalk{nth_largest<10>(steps < 1023 ? steps : 1023, a.n_chunks, nth), 0, 0x7FFFFFFF};
-    }
-    int rank = 0;                                    // in the order of lengths
-    for (int k = 0; k < a.n_chunks; ++k) {
-        const int other = __builtin_amdgcn_readlane(rows, k);
-        rank += other > rows || (other == rows && k < i);
-    }
+__device__ __forceinline__ float lane_value(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
+// sums of lanes 0 .. l in lanes l < 32
+__device__ __forceinline__ float sum_to_here32(float v) {
+    v += dpp_f32<0x111>(v);                          // row_shr:1, 2, 4, 8
+    v += dpp_f32<0x112>(v);
+    v += dpp_f32<0x114>(v);
+    v += dpp_f32<0x118>(v);
+    return v + (threadIdx.x & 16 ? lane_value(v, 15) : 0.f);
+}
+// (a wave) What workgroup y of a head walks; it has begun with portion `own`, the y-th longest where they are more than run at once.
+__device__ __forceinline__ LightningWalk lightning_walk_of(const LightningArgs& a, int walks_each, int y, int own) {
+    const int lane = threadIdx.x & 63, i = lane & 31, n = a.n_chunks, places = 256 / walks_each;
+    const int32_t* ch = a.chunks + 4 * (i < n ? i : 0);
+    const int first_row = ch[0], listed = ch[1], rows = i < n && listed > 0 ? listed : 0;
+    const int64_t position = a.positions[rows ? first_row : 0];                // (looked at last)
+    const int steps = (rows + 15) >> 4, key = (steps < 1023 ? steps : 1023) * 32 + 31 - i;      // as longest_first orders them
+    int rank = 0;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) rank += __builtin_amdgcn_readlane(key, k) > key ? 1 : 0;
     // lanes p and 32 + p: the p-th longest
-    const int lane_of = 4 * (rank + (lane & 32)), mine_rows = __builtin_amdgcn_ds_permute(lane_of, rows), seg = __builtin_amdgcn_ds_permute(lane_of, i), mine = (mine_rows + C - 1) / C;
-    const int cut = (int)ceilf((float)mine * (1.f / (2.f - kFollow)));
-    const float first = cut + 1.f, second = kFollow * cut + (mine - cut) + 1.f, whole = mine + 1.f;
+    const int lane_of = 4 * (rank + (lane & 32)), seg = __builtin_amdgcn_ds_permute(lane_of, i), mine = __builtin_amdgcn_ds_permute(lane_of, (rows + C - 1) / C);
+    int cut = (int)((mine + kLate) * (1.f / (2.f - kFollow)));
+    if (mine + kLate - (1.f - kFollow) * cut > cut + 1.f) ++cut;               // (the piece that is longer then is shorter)
+    const float first = cut + 1.f, second = kFollow * cut + (mine - cut) + 1.f + kLate, whole = mine + 1.f;
     // lane p: the longest p as two pieces (lengths fall with the lane, and with them whole and halves)
-    const bool real = lane < 32 && lane < a.n_chunks;
-    float all = real ? whole : 0.f, added = real ? first + second - whole : 0.f;
-    const float own = added;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const float below = __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane - d), __float_as_uint(added)));
-        all += __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane ^ d), __float_as_uint(all)));
-        added += lane >= d ? below : 0.f;
-    }
-    const float top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(fmaxf(first, second))));
+    const bool real = lane < 32 && lane < n;
+    const float one = real ? first + second - whole : 0.f, added = sum_to_here32(one), all = lane_value(sum_to_here32(real ? whole : 0.f), 31);
+    const float top = lane_value(fmaxf(first, second), 0);
     const float rest = real ? whole : 0.f, longest = lane ? fmaxf(top, rest) : rest;
-    const int places = 256 / walks_each, most = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < 32 && mine >= 4));
-    const float even = (all + added - own) * kUneven / places;
-    // more pieces than CUs for them: the largest that waits goes behind the first to end, both of them short whole portions
-    const float waits = __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (places - lane), __float_as_uint(whole))),
-                ends = __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (places - lane - 1), __float_as_uint(whole)));
+    const int could = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < 32 && mine >= 4)), most = could < lightning_most_cut(places) ? could : lightning_most_cut(places);
+    const float even = (all + added - one) * kUneven / places;
+    // more pieces than CUs for them: of the places, ranks up to places - lane - 1 have a portion of their own, and the longest of the others goes behind the last of those
+    const auto portion = [&](int p) { return __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * p, __float_as_uint(whole))); };
+    const float pair = portion(places - lane) + portion(places - lane - 1);
+    const int over = n + lane - places;              // portions that go behind others
     float cost = longest;
-    if (a.n_chunks + lane > places) cost = fmaxf(fmaxf(longest, even), lane ? waits + ends : 0.f);
-    if (lane > most || (lane && a.n_chunks + lane > places && 2 * lane >= places)) cost = INFINITY;
+    if (over > 0) cost = fmaxf(fmaxf(longest, even), lane ? pair : 0.f);
+    if (lane > most || (lane && over > 0 && n - 2 * over < lane)) cost = INFINITY;       // (none goes behind a piece)
     if (lane) cost = cost * (1.f / 0.97f);           // (not for little)
-    float least = cost;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) least = fminf(least, __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane ^ d), __float_as_uint(least))));
+    float least = cost;                              // (of the first row of lanes: fewer are cut)
+    least = fminf(least, dpp_f32<0x128>(least));     // row_ror:8, 4, 2, 1
+    least = fminf(least, dpp_f32<0x124>(least));
+    least = fminf(least, dpp_f32<0x122>(least));
+    least = lane_value(fminf(least, dpp_f32<0x121>(least)), 0);
     const int split = __builtin_ctzll(__builtin_amdgcn_ballot_w64(cost == least));
-    // pieces: lanes 0 .. 31 the first ones, or whole, 32 .. the second ones
-    const bool two = i < split;
-    const float piece = lane < 32 ? first : two ? second : 0.f;
-    LightningWalk to{-1, 0, 0};
-    if (nth >= a.n_chunks + split) return to;
-    const int size = i >= a.n_chunks ? 0 : lane < 32 && !two ? 4 + ((mine_rows + 15) >> 4) : (int)(4.f * piece), at = nth_largest<10>(size < 1023 ? size : 1023, 64, nth), p = at & 31;
-    const int from = C * (int)__builtin_amdgcn_readlane(cut, p);
-    to.seg = __builtin_amdgcn_readlane(seg, p);
-    const bool halves = p < split;
-    to.from = at >= 32 ? from : 0;
-    to.to = halves && at < 32 ? from : 0x7FFFFFFF;
+    const int behind = n + split > places ? n + split - places : 0, holders = n - behind;     // portions behind others; workgroups with one of their own
+    // (the other pairs: lane p, the p-th longest that goes behind)
+    const float uncut = lane_value(cost, 0), pairs = portion(holders + lane) + portion(holders - 1 - lane);
+    const bool worse = lane < behind && pairs > uncut;
+    const LightningWalk as_begun{own, 0, 0x7FFFFFFF, -1, 0, 0};
+    if (!split || __builtin_amdgcn_ballot_w64(worse || position > 0)) return as_begun;
+    LightningWalk to{-1, 0, 0x7FFFFFFF, -1, 0, 0};
+    const int r = y >= n ? 0 : n <= places ? __builtin_amdgcn_readlane(rank, y) : y;
+    if (y < n && r < holders) {
+        to.seg = __builtin_amdgcn_readlane(seg, r);
+        if (r < split) to.to = C * __builtin_amdgcn_readlane(cut, r);
+        if (holders - 1 - r < behind) to.next = __builtin_amdgcn_readlane(seg, 2 * holders - 1 - r);
+    } else {
+        const int piece = y < n ? r - holders : behind + y - n;
+        if (piece < split) {
+            to.seg = __builtin_amdgcn_readlane(seg, piece), to.from = C * __builtin_amdgcn_readlane(cut, piece);
+            to.row0 = __builtin_amdgcn_readlane(first_row, to.seg), to.rows = __builtin_amdgcn_readlane(rows, to.seg);
+        }
+    }
     return to;
 }
 
 template <int DK, int CW, int PW, bool SUMMARY, bool PIECES>
-__global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const LightningArgs a) {
+__global__ __launch_bounds__(64 * (CW + PW), DK == 64 && CW == 4 ? 4 : 1) void lightning_pair_kernel(const LightningArgs a) {
     constexpr int T = 64 * PW, VW = 16 * CW, KP = DK / 8, KROW = DK * 2, VP = VW / 8, VROW = VW * 2, NQ = C * KP / T, NV = C * VP / T, DT = DK / 16, PT = PW / 4;
     constexpr int KIMG = C * KROW, VIMG = C * VROW;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -354,40 +370,31 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
     __shared__ __attribute__((aligned(16))) float pw[C + 1], fall_s[C];        // decay^0 .. decay^C; decay^(C - 1 - key)
     auto swz = [](int r) { return KROW == 128 ? (r >> 1) & 7 : r & 15; };      // rows of 256 bytes span all banks: 16 of them apart, not 8
     auto swzv = [](int r) { return VROW == 128 ? (r >> 1) & 7 : (2 * r) & 14; };
-    __shared__ int walk_s[3];
+    __shared__ int walk_s[6];
     const int slices = a.dv / VW, head = blockIdx.x / slices, v0 = (blockIdx.x - head * slices) * VW;
-    int seg = blockIdx.y, from = 0, to = 0x7FFFFFFF; // tokens that are only followed; end
-    if constexpr (PIECES) {
-        if (threadIdx.x < 64) {
-            const LightningWalk w = lightning_walk_of(a, a.heads * (a.dv / VW), blockIdx.y);
-            if (threadIdx.x == 0) walk_s[0] = w.seg, walk_s[1] = w.from, walk_s[2] = w.to;
-        } else if (threadIdx.x <= 64 + C) {          // (meanwhile)
-            const int t = threadIdx.x - 64;
-            const float p = powf(a.decay[head], (float)t);
-            pw[t] = p;
-            if (t < C) fall_s[C - 1 - t] = p;
-        }
-        __syncthreads();
-        seg = __builtin_amdgcn_readfirstlane(walk_s[0]), from = __builtin_amdgcn_readfirstlane(walk_s[1]), to = __builtin_amdgcn_readfirstlane(walk_s[2]);
-        if (seg < 0) return;
-    } else {
-        seg = longest_first(a, a.heads * (a.dv / VW));
-    }
-    const int32_t* ch = a.chunks + 4 * seg;
-    const int row0 = ch[0], n_rows = ch[1] < to ? ch[1] : to, seq = ch[2];
-    const bool last = ch[1] <= to && (seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0);
+    // portion, tokens that are only followed, the portion behind it (PIECES: known behind the first barrier; none is begun with where workgroups are more than portions)
+    int seg = PIECES && (int)blockIdx.y >= a.n_chunks ? -1 : longest_first(a, a.heads * slices), from = 0, next_seg = -1;
+    int row0 = 0, n_rows = 0;
+    int64_t slot = -1;
+    bool last = true, known = !PIECES;
+    auto open = [&]() __attribute__((always_inline)) {                         // the portion `seg`, whole
+        const int32_t* ch = a.chunks + 4 * seg;
+        row0 = ch[0], n_rows = ch[1], slot = a.state_slots[ch[2]];
+        last = seg + 1 == a.n_chunks || a.chunks[4 * (seg + 1) + 3] == 0;
+    };
+    if (seg >= 0) open();
     if (SUMMARY && last) return;                     // (nothing follows it)
-    const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lq = lane & 15, lg = lane >> 4;
+    int lane = threadIdx.x & 63, lq = lane & 15, lg = lane >> 4;
+    const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool prepares = wave_id >= CW;
     const int wave = prepares ? wave_id - CW : wave_id;
-    const int64_t slot = a.state_slots[seq];
     const int64_t head_state = (int64_t)a.dk * a.dv;
-    if (n_rows <= 0) {
-        if (SUMMARY || (last && slot >= 0 && ch[3] > 0))
-            pass_segment<SUMMARY>(a.seg_state + ((int64_t)seg * a.heads + head) * head_state + v0, a.state + (slot * a.heads + head) * head_state + v0, DK, VW, a.dv);
-        return;
-    }
     if constexpr (!PIECES) {
+        if (n_rows <= 0) {
+            if (SUMMARY || (last && slot >= 0 && a.chunks[4 * seg + 3] > 0))
+                pass_segment<SUMMARY>(a.seg_state + ((int64_t)seg * a.heads + head) * head_state + v0, a.state + (slot * a.heads + head) * head_state + v0, DK, VW, a.dv);
+            return;
+        }
         if (threadIdx.x <= C) {
             const float p = powf(a.decay[head], (float)threadIdx.x);
             pw[threadIdx.x] = p;
@@ -395,9 +402,28 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
         }
         __syncthreads();
     }
+    // PIECES: what was chosen (behind the first barrier): whether that is another portion than the one begun with
+    auto look = [&]() __attribute__((always_inline)) {
+        const int at = __builtin_amdgcn_readfirstlane(walk_s[0]), to = __builtin_amdgcn_readfirstlane(walk_s[2]);
+        from = __builtin_amdgcn_readfirstlane(walk_s[1]), next_seg = __builtin_amdgcn_readfirstlane(walk_s[3]);
+        const bool other = at != seg;
+        seg = at;
+        if (to < n_rows) n_rows = to, last = false;
+        if (other) {                                 // (none, or a second piece)
+            row0 = __builtin_amdgcn_readfirstlane(walk_s[4]), n_rows = __builtin_amdgcn_readfirstlane(walk_s[5]), last = true;
+            if (seg >= 0) slot = a.state_slots[a.chunks[4 * seg + 2]];
+        }
+        return other;
+    };
+    auto take_next = [&]() __attribute__((always_inline)) {
+        if (!PIECES || next_seg < 0) return false;
+        seg = next_seg, next_seg = -1, from = 0;
+        open();
+        return true;
+    };
 
     if (prepares) {
-        const int tid = threadIdx.x - 64 * CW;
+        int tid = threadIdx.x - 64 * CW;
         const uint16_t* qkv = reinterpret_cast<const uint16_t*>(a.qkv);
         const int64_t k_off = (int64_t)a.heads * a.dk + head * DK, v_off = 2 * (int64_t)a.heads * a.dk + (int64_t)head * a.dv + v0, q_off = (int64_t)head * DK;
         u32x4 qr[NQ], kr[NQ], vr[NV];
@@ -421,7 +447,7 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
         auto base_of = [&](int t0) __attribute__((always_inline)) { return reinterpret_cast<const unsigned char*>(qkv + (int64_t)(row0 + t0) * a.qkv_stride); };
         // (every chunk asks for as many rows as any other, in straight line, the last one's again behind the end: behind a branch around loads the compiler waits
         // for all that are in flight instead of the ones it needs)
-        const int t_last = (n_rows - 1) / C * C;
+        int t_last = 0;
         constexpr std::bool_constant<!SUMMARY> with_q{};
         constexpr std::bool_constant<false> no_q{};
         auto fetch_qk = [&](int t, auto q) __attribute__((always_inline)) {
@@ -470,10 +496,11 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
             }
         };
         // weights D[key 16 jt + 4 lg + r][query 16 tile + lq]: PT waves share a tile of queries, every PT-th tile of keys each; keys behind all queries stay zero
-        const int tile = wave / PT, Rq = 16 * tile + lq;
+        const int tile = wave / PT;
+        int Rq = 16 * tile + lq;
         constexpr int KT = 4 / PT;                   // key tiles a wave may have
         float fall[KT][4];
-        if constexpr (!SUMMARY) {
+        auto falls = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < KT; ++i) {
                 const int jt = PT * i + wave % PT;
@@ -485,7 +512,8 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
                 const int to = Rq * PLD + 32 * (jt >> 1) + 8 * lg + 4 * (jt & 1);
                 if (jt > tile) *reinterpret_cast<u32x2*>(p_lds + to) = *reinterpret_cast<u32x2*>(p_lds + C * PLD + to) = u32x2{0u, 0u};
             }
-        }
+        };
+        if constexpr (!SUMMARY && !PIECES) falls();
         auto weights_of = [&](auto nc, int buf) __attribute__((always_inline)) {       // nc key tiles; only the last can be the queries' own
             constexpr int N = decltype(nc)::value;
             const unsigned char *kimg = kimg0 + buf * KIMG, *qimg = qimg0 + buf * KIMG;
@@ -529,74 +557,66 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
                 }
             }
         };
-        place(C);
-        int t0 = 0, buf = 0;
-        if (PIECES && from) {                        // (at least three chunks)
-            fetch_qk(0, no_q);
-            fetch_v(0);
-            stage_qk(0, 0, no_q);
-            fetch_qk(C, no_q);
-            stage_v(0, 0);
-            fetch_v(C);
-            lds_only_barrier();
-            lds_only_barrier();
-            auto follow = [&](auto q) __attribute__((always_inline)) {
-                stage_qk(t0 + C, buf ^ 1, no_q);
-                fetch_qk(t0 + 2 * C, q);
-                lds_only_barrier();
-                stage_v(t0 + C, buf ^ 1);
-                fetch_v(t0 + 2 * C);
-                lds_only_barrier();
-                t0 += C;
-                buf ^= 1;
-            };
-            while (t0 < from - 2 * C) follow(no_q);
-            follow(with_q);                          // (asks for the first chunk that has outputs)
-        } else {
-            fetch_qk(0, with_q);
-            fetch_v(0);
-            stage_qk(0, 0, with_q);
-            fetch_qk(C, with_q);
-            stage_v(0, 0);
-            fetch_v(C);
-            lds_only_barrier();
-            weights(0);
-            lds_only_barrier();
-        }
-        for (; t0 < n_rows; t0 += C, buf ^= 1) {
-            const bool next = t0 + C < n_rows;
-            if (next) stage_qk(t0 + C, buf ^ 1, with_q);
-            fetch_qk(t0 + 2 * C, with_q);
-            lds_only_barrier();
-            if (next) {
-                weights(buf ^ 1);
-                stage_v(t0 + C, buf ^ 1);
+        for (;;) {
+            if constexpr (PIECES) lane = lane_now() & 63, tid = (64 * wave + lane) & (T - 1), lq = lane & 15, lg = lane >> 4, Rq = 16 * tile + lq;
+            if (!PIECES || n_rows > 0) {
+                t_last = (n_rows - 1) / C * C;
+                place(C);
+                fetch_qk(0, with_q);
+                fetch_v(0);
+                stage_qk(0, 0, with_q);
+                fetch_qk(C, with_q);
+                stage_v(0, 0);
+                fetch_v(C);
             }
-            fetch_v(t0 + 2 * C);
-            lds_only_barrier();
+            if (!known || n_rows > 0) lds_only_barrier();
+            if (!known) {
+                known = true;
+                if (look()) continue;
+                t_last = (n_rows - 1) / C * C;
+            }
+            if (!PIECES || n_rows > 0) {
+                int t0 = 0, buf = 0;
+                if constexpr (PIECES) falls();
+                if (PIECES && from) {                // (at least three chunks)
+                    lds_only_barrier();
+                    auto follow = [&](auto q) __attribute__((always_inline)) {
+                        stage_qk(t0 + C, buf ^ 1, no_q);
+                        fetch_qk(t0 + 2 * C, q);
+                        lds_only_barrier();
+                        stage_v(t0 + C, buf ^ 1);
+                        fetch_v(t0 + 2 * C);
+                        lds_only_barrier();
+                        t0 += C;
+                        buf ^= 1;
+                    };
+                    while (t0 < from - 2 * C) follow(no_q);
+                    follow(with_q);                  // (asks for the first chunk that has outputs)
+                } else {
+                    weights(0);
+                    lds_only_barrier();
+                }
+                for (; t0 < n_rows; t0 += C, buf ^= 1) {
+                    const bool next = t0 + C < n_rows;
+                    if (next) stage_qk(t0 + C, buf ^ 1, with_q);
+                    fetch_qk(t0 + 2 * C, with_q);
+                    lds_only_barrier();
+                    if (next) {
+                        weights(buf ^ 1);
+                        stage_v(t0 + C, buf ^ 1);
+                    }
+                    fetch_v(t0 + 2 * C);
+                    lds_only_barrier();
+                }
+            }
+            if (!take_next()) return;
         }
-        return;
     }
 
     // state: value column v0 + 16 wave + lq, key rows 16 t + 4 lg + r
     f32x4 S[DT];
-    const int sv = v0 + 16 * wave + lq;
-#pragma unroll
-    for (int t = 0; t < DT; ++t) S[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (!SUMMARY) {
-        const float* src = nullptr;
-        if (a.summaries) src = a.seg_state + ((int64_t)seg * a.heads + head) * head_state;
-        else if (slot >= 0 && a.positions[row0] > 0) src = a.state + (slot * a.heads + head) * head_state;
-        if (src) {
-#pragma unroll
-            for (int t = 0; t < DT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) S[t][r] = src[(int64_t)(16 * t + 4 * lg + r) * a.dv + sv];
-        }
-    }
-    const int tr = 4 * lg + (lq >> 2), tp = lq & 3;  // transposed reads: row and column quarter this lane addresses
-    lds_only_barrier();
-    lds_only_barrier();
+    int sv = v0 + 16 * wave + lq;
+    int tr = 4 * lg + (lq >> 2), tp = lq & 3;        // transposed reads: row and column quarter this lane addresses
     // what a followed chunk does to the state: the second half of the loop below.  (Shared with it as a function, that loop loses 1 % of its speed)
     auto values = [&](bf16x8 (&vf)[2], const unsigned char* vimg) __attribute__((always_inline)) {
 #pragma unroll
@@ -643,111 +663,149 @@ __global__ __launch_bounds__(64 * (CW + PW)) void lightning_pair_kernel(const Li
             }
         }
     };
-    int t0 = 0, buf = 0;
-    if constexpr (PIECES) {
-        for (; t0 < from; t0 += C, buf ^= 1) {
-            bf16x8 vf[2];
-            values(vf, vimg0 + buf * VIMG);
-            lds_only_barrier();
-            advance(vf, C, kimg0 + buf * KIMG);
-            lds_only_barrier();
+    for (;;) {
+        // (what hangs on the lane is computed for each portion: held over them it would not fit the registers; the mask tells the compiler that lanes are 64)
+        if constexpr (PIECES) lane = lane_now() & 63, lq = lane & 15, lg = lane >> 4, sv = v0 + 16 * wave + lq, tr = 4 * lg + (lq >> 2), tp = lq & 3;
+        if (!known && wave_id == 0) {                // (before the state is asked for: loads are waited for in their order)
+            const LightningWalk w = lightning_walk_of(a, a.heads * slices, blockIdx.y, seg);
+            if (lane == 0) walk_s[0] = w.seg, walk_s[1] = w.from, walk_s[2] = w.to, walk_s[3] = w.next, walk_s[4] = w.row0, walk_s[5] = w.rows;
         }
-    }
-    for (; t0 < n_rows; t0 += C, buf ^= 1) {
-        const int n = n_rows - t0 < C ? n_rows - t0 : C;
-        const unsigned char *kimg = kimg0 + buf * KIMG, *qimg = qimg0 + buf * KIMG, *vimg = vimg0 + buf * VIMG;
-        // value fragments: lane = column 16 wave + lq, slots = keys 32 hh + 4 lg + 0..3 and the same + 16
-        bf16x8 vf[2];
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * wave + (tp >> 1);
-            const u32x2 lo = lds_tr16(vimg + ra * VROW + (pc ^ swzv(ra)) * 16 + (tp & 1) * 8), hi = lds_tr16(vimg + rb * VROW + (pc ^ swzv(rb)) * 16 + (tp & 1) * 8);
-            const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
-            vf[hh] = *reinterpret_cast<const bf16x8*>(&raw);
-        }
+        for (int t = 0; t < DT; ++t) S[t] = f32x4{0.f, 0.f, 0.f, 0.f};
         if constexpr (!SUMMARY) {
-            uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + (int64_t)(row0 + t0) * a.out_stride + (int64_t)head * a.dv + v0 + 16 * wave + 4 * lg;
-            // what the state gives: slots of a 32-wide step are key rows 16 (2 st) + 4 lg + 0..3 and 16 (2 st + 1) + 4 lg + 0..3
-            f32x4 o[4];                              // o^T: value 16 wave + 4 lg + r, token 16 it + lq
+            const float* src = nullptr;
+            if (a.summaries) src = a.seg_state + ((int64_t)seg * a.heads + head) * head_state;
+            else if (slot >= 0 && (!PIECES || (known ? false : n_rows > 0)) && a.positions[row0] > 0) src = a.state + (slot * a.heads + head) * head_state;
+            if (src) {
 #pragma unroll
-            for (int it = 0; it < 4; ++it) o[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int t = 0; t < DT; ++t)
 #pragma unroll
-            for (int st = 0; st < DK / 32; ++st) {
-                const f32x4 s0 = S[2 * st], s1 = S[2 * st + 1];
-                const float v[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
-                bf16x8 hi, lo;
-                split_hi_lo(v, hi, lo);
-#pragma unroll
-                for (int it = 0; it < 4; ++it) {
-                    const int R = 16 * it + lq;
-                    const unsigned char* qrow = qimg + R * KROW + (lg & 1) * 8;
-                    const u32x2 qa = *reinterpret_cast<const u32x2*>(qrow + ((4 * st + (lg >> 1)) ^ swz(R)) * 16);
-                    const u32x2 qb = *reinterpret_cast<const u32x2*>(qrow + ((4 * st + 2 + (lg >> 1)) ^ swz(R)) * 16);
-                    const u32x4 raw = {qa[0], qa[1], qb[0], qb[1]};
-                    const bf16x8 qf = *reinterpret_cast<const bf16x8*>(&raw);
-                    o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, qf, o[it], 0, 0, 0);
-                    o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, qf, o[it], 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int it = 0; it < 4; ++it) o[it] *= pw[16 * it + lq + 1];
-#pragma unroll
-            for (int it = 0; it < 4; ++it)
-#pragma unroll
-                for (int hh = 0; hh <= it / 2; ++hh) {
-                    const uint16_t* pr = p_lds + (16 * it + lq) * PLD + 32 * hh + 8 * lg;
-                    o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(pr), o[it], 0, 0, 0);
-                    o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(pr + C * PLD), o[it], 0, 0, 0);
-                }
-#pragma unroll
-            for (int it = 0; it < 4; ++it)
-                if (16 * it + lq < n) act_st4(out + (16 * it + lq) * a.out_stride, o[it]);
-        }
-        lds_only_barrier();                          // the weights may be replaced
-        // ---- the state behind these tokens
-        const float decayed = pw[n];
-#pragma unroll
-        for (int t = 0; t < DT; ++t) S[t] *= decayed;
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            const u32x4 raw = *reinterpret_cast<const u32x4*>(&vf[hh]);
-            f32x4 fall[2];                           // what a value decays by until the chunk's end
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const int key = 32 * hh + 16 * q + 4 * lg;
-                if (n == C) {
-                    fall[q] = *reinterpret_cast<const f32x4*>(fall_s + key);
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) fall[q][r] = pw[key + r < n ? n - 1 - key - r : 0];
-                }
-            }
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = (j & 1 ? bf16_hi(raw[j >> 1]) : bf16_lo(raw[j >> 1])) * fall[j >> 2][j & 3];
-            bf16x8 hi, lo;
-            split_hi_lo(v, hi, lo);
-            const int ra = 32 * hh + tr, rb = ra + 16;
-#pragma unroll
-            for (int t = 0; t < DT; ++t) {
-                const int pc = 2 * t + (tp >> 1);
-                const u32x2 klo = lds_tr16(kimg + ra * KROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8), khi = lds_tr16(kimg + rb * KROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8);
-                const u32x4 kraw = {klo[0], klo[1], khi[0], khi[1]};
-                const bf16x8 kf = *reinterpret_cast<const bf16x8*>(&kraw);
-                S[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, hi, S[t], 0, 0, 0);
-                S[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, lo, S[t], 0, 0, 0);
+                    for (int r = 0; r < 4; ++r) S[t][r] = src[(int64_t)(16 * t + 4 * lg + r) * a.dv + sv];
             }
         }
-        lds_only_barrier();                          // this chunk's images may be replaced
-    }
-    float* dst = nullptr;
-    if constexpr (SUMMARY) dst = a.seg_state + ((int64_t)seg * a.heads + head) * head_state;
-    else if (last && slot >= 0) dst = a.state + (slot * a.heads + head) * head_state;
-    if (dst) {
+        if (!known && wave_id != 0) {
+            const int t = 64 * wave_id - 64 + lane;
+            if (t <= C) {
+                const float p = powf(a.decay[head], (float)t);
+                pw[t] = p;
+                if (t < C) fall_s[C - 1 - t] = p;
+            }
+        }
+        if (!known || n_rows > 0) lds_only_barrier();
+        if (!known) {
+            known = true;
+            if (look()) continue;
+        }
+        if (!PIECES || n_rows > 0) {
+            lds_only_barrier();
+            int t0 = 0, buf = 0;
+            if constexpr (PIECES) {
+                for (; t0 < from; t0 += C, buf ^= 1) {
+                    bf16x8 vf[2];
+                    values(vf, vimg0 + buf * VIMG);
+                    lds_only_barrier();
+                    advance(vf, C, kimg0 + buf * KIMG);
+                    lds_only_barrier();
+                }
+            }
+            for (; t0 < n_rows; t0 += C, buf ^= 1) {
+                const int n = n_rows - t0 < C ? n_rows - t0 : C;
+                const unsigned char *kimg = kimg0 + buf * KIMG, *qimg = qimg0 + buf * KIMG, *vimg = vimg0 + buf * VIMG;
+                // value fragments: lane = column 16 wave + lq, slots = keys 32 hh + 4 lg + 0..3 and the same + 16
+                bf16x8 vf[2];
 #pragma unroll
-        for (int t = 0; t < DT; ++t)
+                for (int hh = 0; hh < 2; ++hh) {
+                    const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * wave + (tp >> 1);
+                    const u32x2 lo = lds_tr16(vimg + ra * VROW + (pc ^ swzv(ra)) * 16 + (tp & 1) * 8), hi = lds_tr16(vimg + rb * VROW + (pc ^ swzv(rb)) * 16 + (tp & 1) * 8);
+                    const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
+                    vf[hh] = *reinterpret_cast<const bf16x8*>(&raw);
+                }
+                if constexpr (!SUMMARY) {
+                    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + (int64_t)(row0 + t0) * a.out_stride + (int64_t)head * a.dv + v0 + 16 * wave + 4 * lg;
+                    // what the state gives: slots of a 32-wide step are key rows 16 (2 st) + 4 lg + 0..3 and 16 (2 st + 1) + 4 lg + 0..3
+                    f32x4 o[4];                              // o^T: value 16 wave + 4 lg + r, token 16 it + lq
 #pragma unroll
-            for (int r = 0; r < 4; ++r) dst[(int64_t)(16 * t + 4 * lg + r) * a.dv + sv] = S[t][r];
+                    for (int it = 0; it < 4; ++it) o[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int st = 0; st < DK / 32; ++st) {
+                        const f32x4 s0 = S[2 * st], s1 = S[2 * st + 1];
+                        const float v[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+                        bf16x8 hi, lo;
+                        split_hi_lo(v, hi, lo);
+#pragma unroll
+                        for (int it = 0; it < 4; ++it) {
+                            const int R = 16 * it + lq;
+                            const unsigned char* qrow = qimg + R * KROW + (lg & 1) * 8;
+                            const u32x2 qa = *reinterpret_cast<const u32x2*>(qrow + ((4 * st + (lg >> 1)) ^ swz(R)) * 16);
+                            const u32x2 qb = *reinterpret_cast<const u32x2*>(qrow + ((4 * st + 2 + (lg >> 1)) ^ swz(R)) * 16);
+                            const u32x4 raw = {qa[0], qa[1], qb[0], qb[1]};
+                            const bf16x8 qf = *reinterpret_cast<const bf16x8*>(&raw);
+                            o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, qf, o[it], 0, 0, 0);
+                            o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, qf, o[it], 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+                    for (int it = 0; it < 4; ++it) o[it] *= pw[16 * it + lq + 1];
+#pragma unroll
+                    for (int it = 0; it < 4; ++it)
+#pragma unroll
+                        for (int hh = 0; hh <= it / 2; ++hh) {
+                            const uint16_t* pr = p_lds + (16 * it + lq) * PLD + 32 * hh + 8 * lg;
+                            o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(pr), o[it], 0, 0, 0);
+                            o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(pr + C * PLD), o[it], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int it = 0; it < 4; ++it)
+                        if (16 * it + lq < n) act_st4(out + (16 * it + lq) * a.out_stride, o[it]);
+                }
+                lds_only_barrier();                          // the weights may be replaced
+                // ---- the state behind these tokens
+                const float decayed = pw[n];
+#pragma unroll
+                for (int t = 0; t < DT; ++t) S[t] *= decayed;
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    const u32x4 raw = *reinterpret_cast<const u32x4*>(&vf[hh]);
+                    f32x4 fall[2];                           // what a value decays by until the chunk's end
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const int key = 32 * hh + 16 * q + 4 * lg;
+                        if (n == C) {
+                            fall[q] = *reinterpret_cast<const f32x4*>(fall_s + key);
+                        } else {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) fall[q][r] = pw[key + r < n ? n - 1 - key - r : 0];
+                        }
+                    }
+                    float v[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) v[j] = (j & 1 ? bf16_hi(raw[j >> 1]) : bf16_lo(raw[j >> 1])) * fall[j >> 2][j & 3];
+                    bf16x8 hi, lo;
+                    split_hi_lo(v, hi, lo);
+                    const int ra = 32 * hh + tr, rb = ra + 16;
+#pragma unroll
+                    for (int t = 0; t < DT; ++t) {
+                        const int pc = 2 * t + (tp >> 1);
+                        const u32x2 klo = lds_tr16(kimg + ra * KROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8), khi = lds_tr16(kimg + rb * KROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8);
+                        const u32x4 kraw = {klo[0], klo[1], khi[0], khi[1]};
+                        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(&kraw);
+                        S[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, hi, S[t], 0, 0, 0);
+                        S[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, lo, S[t], 0, 0, 0);
+                    }
+                }
+                lds_only_barrier();                          // this chunk's images may be replaced
+            }
+            float* dst = nullptr;
+            if constexpr (SUMMARY) dst = a.seg_state + ((int64_t)seg * a.heads + head) * head_state;
+            else if (last && slot >= 0) dst = a.state + (slot * a.heads + head) * head_state;
+            if (dst) {
+#pragma unroll
+                for (int t = 0; t < DT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) dst[(int64_t)(16 * t + 4 * lg + r) * a.dv + sv] = S[t][r];
+            }
+        }
+        if (!take_next()) return;
     }
 }
 
@@ -942,11 +1000,11 @@ int pair_dk(const LightningArgs& a, hipStream_t stream) {
         rc = check_launch("lightning starts");
         if (rc) return rc;
     }
-    // The longest portions as two pieces, where whole ones come to 193 to 320 workgroups: fewer are better cut into segments, more fill the CUs more than once and even out.  Choosing takes
-    // 2 us, for nothing where a portion continues (9000 tokens of 16, 16 heads of 128: 74.4 us against 73.5); so other launches have a kernel without it, as have those of less than four
-    // chunks a portion (3000 of 20: 29 against 32).
-    if (!a.summaries && a.n_chunks > 1 && a.n_chunks <= kSplitPortions && walks * a.n_chunks > 192 && walks * a.n_chunks <= 320 && a.rows >= 4 * C * a.n_chunks) {
-        grid.y = 2 * a.n_chunks;
+    // The longest portions as two pieces, where whole ones come to 193 to 320 workgroups: fewer are better cut into segments, more fill the CUs more than once and even out.  Other launches
+    // have a kernel without that, as have those of less than four chunks a portion.
+    const int places = 256 / walks, most = lightning_most_cut(places);
+    if (!a.summaries && most && a.n_chunks <= kSplitPortions && walks * a.n_chunks > 192 && walks * a.n_chunks <= 320 && a.rows >= 4 * C * a.n_chunks) {
+        if (a.n_chunks < places) grid.y = a.n_chunks + most < places ? a.n_chunks + most : places;
         if (lds > 64 * 1024)
             (void)hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_pair_kernel<DK, CW, PW, false, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         lightning_pair_kernel<DK, CW, PW, false, true><<<grid, 64 * (CW + PW), lds, stream>>>(a);

@@ -622,12 +622,6 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
 // and, before, 4.5 of lookups and first images and 6 to 8 of results.  3000 tokens, 32 experts of 1536: 371 us in two launches, 313 with the parts one after the other, 308 overlapped;
 // 12000 966, 935, 930; 1024 wide, of 768, 6000 176, 164, 160.  (Announced from the next part's loop without a wait of its own: 1 % slower, rows came later to those who waited)
 // Few operations on shared words: 256 workgroups that look at eight lists when theirs is at an end took 25 us for it.
-// this lane, not held in a register
-__device__ __forceinline__ int lane_now() {
-    int l;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n v_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-    return l;
-}
 constexpr int kListWords = 32, kRanOut = 16;         // tickets a line each; in the first line, whether a wait ran out
 constexpr uint32_t kWaitLimit = 1 << 22;             // polls of about a microsecond
 struct MoeBothArgs {

@@ -335,6 +335,16 @@ def test_lightning_long_portions_as_two_pieces(heads, dk, dv, lengths, behind):
     assert torch.equal(state[n - 1 - none], start[n - 1 - none])
 
 
+# as many portions as CUs for a head, and more: second pieces in place of the shortest, those behind others, empty ones among them, holders that are empty; a workgroup that has neither
+SHORT = [1500, 1400, 100, 0, 300, 900, 1300, 64, 20, 400, 500, 0, 200, 193, 1, 130]
+@pytest.mark.parametrize("heads,dk,dv,lengths", [
+    (16, 128, 128, SHORT), (16, 64, 64, SHORT), (16, 128, 128, SHORT + [700, 90, 63]), (8, 64, 128, [1500, 1300, 1100, 900] + [150 + 7 * i for i in range(20)] + [0, 0, 0, 1, 33, 64, 65, 70]),
+    (32, 128, 64, [1500, 900, 0, 0, 64, 40, 300, 1, 128]), (16, 128, 128, [2000, 1900, 1800, 1700, 900] + [0] * 11), (16, 64, 64, [3000, 2500, 800, 700, 300, 200, 190, 180, 100, 100, 90, 80,
+                                                                                                                        64, 20, 0, 0, 1])])
+def test_lightning_pieces_in_place_of_portions(heads, dk, dv, lengths):
+    test_lightning_long_portions_as_two_pieces(heads, dk, dv, lengths, False)
+
+
 @pytest.mark.parametrize("stride", [(1 << 25) - 8, 34_100_000])
 @pytest.mark.parametrize("heads,dk,dv", [(2, 64, 64), (1, 64, 128), (1, 128, 64), (2, 128, 128)])
 def test_lightning_rows_far_apart(heads, dk, dv, stride):

@@ -21,8 +21,9 @@ __device__ __forceinline__ bool prompt_tile(const PagedAttendArgs& a, int* words
 }
 
 // WIDE: 128 rows a workgroup on 32 x 32 tiles (attend_walk32); otherwise 64 rows on 16 x 16 tiles.  The same sums to the bit.
+// (heads of 128 / 64: three workgroups a CU, as their images allow; without the bound 169 registers for 168, and 195 -> 212 us for 4 prompts of 12000 tokens, 16 heads)
 template <int DK, int DV, bool WIDE>
-__global__ __launch_bounds__(256, WIDE || DK + DV <= 320 ? 2 : 1) void paged_prompt_kernel(const PagedAttendArgs a) {
+__global__ __launch_bounds__(256, WIDE && DK == 128 && DV == 64 ? 3 : WIDE || DK + DV <= 320 ? 2 : 1) void paged_prompt_kernel(const PagedAttendArgs a) {
     using Images = TileImages<DK, DV>;
     constexpr int WR = WIDE ? 32 : 16, BM = 4 * WR, BN = Images::BN, KP = Images::KP, VP = Images::VP, NK = Images::NK, NV = Images::NV;
     extern __shared__ __attribute__((aligned(512))) unsigned char lds[];

@@ -422,12 +422,14 @@ struct PromptTile {
 };
 
 constexpr int kFewPrompts = 3;
+__host__ __device__ __forceinline__ bool few_prompts(int batch) { return batch > 1 && batch <= kFewPrompts; }
 
-// Up to three sequences (grid: heads x sequences x query tiles of the longest prompt): the tiles that see the most keys start first, whichever sequence they are of and however many
+// Two or three sequences (grid: heads x sequences x query tiles of the longest prompt): the tiles that see the most keys start first, whichever sequence they are of and however many
 // keys it has cached, and a workgroup number that no tile is left for comes after all others.  Workgroups are dealt round-robin over the 8 XCDs, each with an L2 of its own: from 16
 // pairs (sequence, key head) on, a multiple of 8, the tiles of a pair go to one XCD, the pairs with the most work dealt first, back and forth; fewer make one list for all XCDs.
 // Against the order of the grid: 2 prompts of 2834 tokens, 512 of them cached, 16 / 8 heads of 128, 88.6 -> 72.9 us; 2 of 2703, 1280 cached, 14 / 2 of 64, 57.9 -> 53.9; over pages, 3 of
 // 4792, 16 heads, 74.2 -> 70.9.  With more sequences finding the tile takes longer (1.5 us for 24) than the order gives: 9 of 11522, 28 / 4 heads of 128, 200 -> 208; 30 of 2294 27.0 -> 30.2.
+// One alone has its heaviest tiles first in the order of the grid, and finding them is 0.7 us: over pages, 61 of 300 to 5000 tokens, 0.92 to 0.99 of the speed.
 // Lane i of the first wave holds sequence i.  span > 0: keys a query sees at most.  words: 8 of the workgroup's LDS, free again behind it.
 template <int BM>
 __device__ __forceinline__ bool few_prompts_tile(const int32_t* cu_q, const int32_t* cu_k, int batch, int heads, int kv_heads, int span, int* words, PromptTile& t) {

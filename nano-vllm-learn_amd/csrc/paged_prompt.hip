@@ -9,9 +9,9 @@ namespace nvh {
 
 namespace {
 
-template <int BM>
+template <int BM, bool ORDERED>
 __device__ __forceinline__ bool prompt_tile(const PagedAttendArgs& a, int* words, PromptTile& t) {
-    if (a.batch <= kFewPrompts) {
+    if constexpr (ORDERED) {
         if (!few_prompts_tile<BM>(a.cu_q, a.cu_k, a.batch, a.heads, a.kv_heads, a.chunk > 0 ? a.chunk : a.window, words, t)) return false;
     } else {
         attend_unit(a.heads, t.qt, t.head, t.b);
@@ -20,15 +20,16 @@ __device__ __forceinline__ bool prompt_tile(const PagedAttendArgs& a, int* words
     return t.qt * BM < t.sq && t.sk >= t.sq;
 }
 
-// WIDE: 128 rows a workgroup on 32 x 32 tiles (attend_walk32); otherwise 64 rows on 16 x 16 tiles.  The same sums to the bit.
+// WIDE: 128 rows a workgroup on 32 x 32 tiles (attend_walk32); otherwise 64 rows on 16 x 16 tiles.  The same sums to the bit.  ORDERED: few_prompts_tile (of its own: the code in front
+// of other launches was 0.2 us).
 // (heads of 128 / 64: three workgroups a CU, as their images allow; without the bound 169 registers for 168, and 195 -> 212 us for 4 prompts of 12000 tokens, 16 heads)
-template <int DK, int DV, bool WIDE>
+template <int DK, int DV, bool WIDE, bool ORDERED>
 __global__ __launch_bounds__(256, WIDE && DK == 128 && DV == 64 ? 3 : WIDE || DK + DV <= 320 ? 2 : 1) void paged_prompt_kernel(const PagedAttendArgs a) {
     using Images = TileImages<DK, DV>;
     constexpr int WR = WIDE ? 32 : 16, BM = 4 * WR, BN = Images::BN, KP = Images::KP, VP = Images::VP, NK = Images::NK, NV = Images::NV;
     extern __shared__ __attribute__((aligned(512))) unsigned char lds[];
     PromptTile tile;
-    if (!prompt_tile<BM>(a, reinterpret_cast<int*>(lds), tile)) return;
+    if (!prompt_tile<BM, ORDERED>(a, reinterpret_cast<int*>(lds), tile)) return;
     const int head = tile.head, b = tile.b, q_beg = tile.q_beg, sq = tile.sq, sk = tile.sk, q0 = tile.qt * BM;
     const int shift = sk - sq;                       // query row r has position r + shift
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane & (WR - 1), lg = lane / WR;
@@ -130,13 +131,21 @@ __global__ __launch_bounds__(256, WIDE && DK == 128 && DV == 64 ? 3 : WIDE || DK
     }
 }
 
-template <int DK, int DV, bool WIDE>
-int launch_one(const PagedAttendArgs& a, hipStream_t stream) {
+template <int DK, int DV, bool WIDE, bool ORDERED>
+int launch_form(const PagedAttendArgs& a, hipStream_t stream) {
     constexpr size_t lds = TileImages<DK, DV>::BYTES;
     constexpr int BM = WIDE ? 128 : 64;
-    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paged_prompt_kernel<DK, DV, WIDE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    paged_prompt_kernel<DK, DV, WIDE><<<dim3(a.heads, a.batch, (a.max_q + BM - 1) / BM), 256, lds, stream>>>(a);
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paged_prompt_kernel<DK, DV, WIDE, ORDERED>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    paged_prompt_kernel<DK, DV, WIDE, ORDERED><<<dim3(a.heads, a.batch, (a.max_q + BM - 1) / BM), 256, lds, stream>>>(a);
     return check_launch("paged_attend_prompt");
+}
+// Two or three portions in the order of their work, unless all workgroups run at once where the images leave room for two and more on a CU (64 rows): finding the tile is 0.7 us of 15 to 30,
+// and nothing waits for a CU (32 sets of 2 and 3 portions: 0.93 to 1.0 of the speed with the order, six of them 1.06 to 1.18).
+template <int DK, int DV, bool WIDE>
+int launch_one(const PagedAttendArgs& a, hipStream_t stream) {
+    constexpr int64_t room = 163840 / TileImages<DK, DV>::BYTES;
+    const bool at_once = !WIDE && room > 1 && ((int64_t)a.rows + 63 * (int64_t)a.batch) * a.heads <= 64 * 256 * room;
+    return few_prompts(a.batch) && !at_once ? launch_form<DK, DV, WIDE, true>(a, stream) : launch_form<DK, DV, WIDE, false>(a, stream);
 }
 template <int DK, int DV>
 int launch_dims(const PagedAttendArgs& a, hipStream_t stream) {

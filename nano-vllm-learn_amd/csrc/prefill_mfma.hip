@@ -168,7 +168,7 @@ __device__ __forceinline__ void prefill_tile_of_block(const PrefillArgs& a, int&
 }
 
 __device__ __forceinline__ bool prefill_tile(const PrefillArgs& a, int* words, PromptTile& t) {
-    if (a.batch <= kFewPrompts) return few_prompts_tile<128>(a.cu_q, a.cu_k, a.batch, a.h, a.kvh, 0, words, t);
+    if (few_prompts(a.batch)) return few_prompts_tile<128>(a.cu_q, a.cu_k, a.batch, a.h, a.kvh, 0, words, t);
     prefill_tile_of_block(a, t.qt, t.head, t.b);
     prompt_rows(a.cu_q, a.cu_k, t);
     return t.qt * 128 < t.sq;

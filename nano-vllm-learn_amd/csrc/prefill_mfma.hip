@@ -1008,9 +1008,13 @@ int launch_one(const PrefillArgs& a, hipStream_t stream, const char* what) {
     return check_launch(what);
 }
 
+// Heads of 64 with exact P: registers and images let four workgroups on a CU.  That is 1.03 to 1.1 times as fast from two rounds of them on; in fewer the CUs that got the longest
+// walks keep them beside three others, and three are better: 32 heads, 4 prompts of 6943 tokens (1.75 rounds) 151 -> 124 us, 16 heads, 8 of 10487 (1.3) 90 -> 78, one of 8890 (1.1)
+// 279 -> 264; 14 heads, 2 of 11840 (1.3) 251 -> 220.  (As many rows as launch_d takes uneven sequences to have.)
 template <int D, bool PAGED, int PV>
 int launch_one32(const PrefillArgs& a, hipStream_t stream, const char* what) {
-    constexpr int lds = (int)TileImages<D, D>::BYTES;
+    const bool three = D == 64 && PV == 0 && 0.5 * ((double)a.max_seqlen_q * a.batch + a.max_seqlen_q) * a.h < 2.0 * 128 * 1024;
+    const int lds = three ? 44 * 1024 : (int)TileImages<D, D>::BYTES;
     prefill32_kernel<D, PAGED, PV><<<dim3(a.h, a.batch, (a.max_seqlen_q + 127) / 128), 256, lds, stream>>>(a);
     return check_launch(what);
 }

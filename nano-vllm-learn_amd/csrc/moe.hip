@@ -353,40 +353,53 @@ struct ExpertTile {
 // The tiles of an expert share its pairs evenly, in units of what the waves multiply at a time, instead of all but the last being full: workgroups of one length fill the rounds that the
 // CUs take them in better.  (1024 wide, 3000 tokens 132 -> 129 us.  In units of a row of every wave's tiles a tile of 240 would multiply 256, eight times an expert: 16384 tokens at
 // 2048 wide 1155 -> 1160)
+// rows 0: eight row tiles at a time, whosever they are.  For launches of up to a workgroup a CU: an expert's tiles together would leave the experts with the most pairs to one XCD.  (8 experts
+// of 1536, 2048 wide, 99 tokens of an uneven route, gate | up 24.8 -> 22.0 us; 16 of 512, 4096 wide, 322 tokens 40.8 -> 37.3)
+constexpr int kAlone = 256;
+// a / b of up to 2^20 (by 32 bits: half of the instructions in front of a workgroup's first load)
+__device__ __forceinline__ int few_over(int a, int b) { return (int)(((float)a + 0.5f) * fast_rcp((float)b)); }
 template <int TM, int UNIT>
 __device__ __forceinline__ ExpertTile find_tile(const int32_t* table, int tiles, int nx, int idx, int lo, int hi, int rows, int lane) {
     ExpertTile to;
-    const int m = lo + idx / nx;
-    {   // the only tile of its expert: nothing to order or share (100 tokens, 32 experts, a call 39.8 -> 39.4 us)
-        const int4 own = reinterpret_cast<const int4*>(table)[m];
-        const int before = table[4 * (m ? m - 1 : 0)], behind = table[4 * (m + 1 < tiles ? m + 1 : m)];
-        if ((!m || before != own.x) && (m + 1 == tiles || behind != own.x)) return ExpertTile{idx - (m - lo) * nx, m, own.x, own.y, own.z};
+    int m, nt;
+    if (rows) {
+        m = lo + idx / nx;
+        nt = idx - (m - lo) * nx;
+    } else {
+        const int g = few_over(idx, 8 * nx), in = idx - g * 8 * nx, gm = tiles - 8 * g < 8 ? tiles - 8 * g : 8;
+        nt = few_over(in, gm);
+        m = 8 * g + in - nt * gm;
     }
     const int at = m - 32 + lane;                    // a tile of the expert, and 63 around it
     const int4 t = reinterpret_cast<const int4*>(table)[at < 0 ? 0 : at < tiles ? at : tiles - 1];
     to.expert = __builtin_amdgcn_readlane(t.x, 32);
     const uint64_t same = __builtin_amdgcn_ballot_w64(at >= 0 && at < tiles && t.x == to.expert);
+    // the only tile of its expert: nothing to order or share (100 tokens, 32 experts, a call 39.8 -> 39.4 us)
+    if ((same >> 31 & 7) == 2) return ExpertTile{nt, m, to.expert, __builtin_amdgcn_readlane(t.y, 32), __builtin_amdgcn_readlane(t.z, 32)};
     const int back = __builtin_clz(~(uint32_t)same | 1), ahead = __builtin_ctz(~(uint32_t)(same >> 33));
     const bool all_seen = back + 1 + ahead < 32;     // (lane 0's and lane 63's are not of it then); otherwise the eight around this one that are
     int from = m - back, to_end = m + ahead + 1;
     const int n = to_end - from, t0 = from;
-    if (!all_seen) {
-        from = from > (m & ~7) ? from : m & ~7;
-        to_end = to_end < (m | 7) + 1 ? to_end : (m | 7) + 1;
+    to.nt = nt, to.mt = m;
+    if (rows) {
+        if (!all_seen) {
+            from = from > (m & ~7) ? from : m & ~7;
+            to_end = to_end < (m | 7) + 1 ? to_end : (m | 7) + 1;
+        }
+        from = from > lo ? from : lo;
+        to_end = to_end < hi ? to_end : hi;
+        int in = idx - (from - lo) * nx;
+        const int span = to_end - from, groups = (span + rows - 1) / rows;
+        rows = few_over(span + groups - 1, groups);    // nine tiles: five and four
+        const int g = few_over(in, rows * nx), left = span - rows * g, gm = left < rows ? left : rows;
+        in -= g * rows * nx;
+        to.nt = few_over(in, gm);
+        to.mt = from + rows * g + in - to.nt * gm;
     }
-    from = from > lo ? from : lo;
-    to_end = to_end < hi ? to_end : hi;
-    int in = idx - (from - lo) * nx;
-    const int span = to_end - from, groups = (span + rows - 1) / rows;
-    rows = (span + groups - 1) / groups;    // nine tiles: five and four
-    const int g = in / (rows * nx), left = span - rows * g, gm = left < rows ? left : rows;
-    in -= g * rows * nx;
-    to.nt = in / gm;
-    to.mt = from + rows * g + in - to.nt * gm;
     to.first = __builtin_amdgcn_readlane(t.y, to.mt - m + 32);
     to.live = __builtin_amdgcn_readlane(t.z, to.mt - m + 32);
     if (all_seen && n > 1) {
-        const int all = (n - 1) * TM + __builtin_amdgcn_readlane(t.z, t0 + n - 1 - m + 32), each = (all + n * UNIT - 1) / (n * UNIT) * UNIT, nth = to.mt - t0;
+        const int all = (n - 1) * TM + __builtin_amdgcn_readlane(t.z, t0 + n - 1 - m + 32), each = few_over(all + n * UNIT - 1, n * UNIT) * UNIT, nth = to.mt - t0;
         to.first += nth * (each - TM);
         to.live = all - nth * each < each ? all - nth * each : each;
     }
@@ -599,7 +612,7 @@ __global__ __launch_bounds__(64 * MW * NW) void moe_gemm_kernel(const MoeGemmArg
     const int nx = gridDim.x, tiles = a.tiles[3], total = nx * tiles, lin = (int)(blockIdx.x + gridDim.x * blockIdx.y), per = total >> 3;
     if (lin >= total) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const ExpertTile to = find_tile<G::TM, G::UNIT>(a.tiles, tiles, nx, lin < per * 8 ? (lin & 7) * per + (lin >> 3) : lin, 0, tiles, 8, lane);
+    const ExpertTile to = find_tile<G::TM, G::UNIT>(a.tiles, tiles, nx, lin < per * 8 ? (lin & 7) * per + (lin >> 3) : lin, 0, tiles, total <= kAlone ? 0 : 8, lane);
     const int iters = a.k / TK;                      // (k is a multiple of 64: even)
     ExpertFeed<G> feed;
     feed.aim(GLU, a, to, wave, lane);

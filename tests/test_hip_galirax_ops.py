@@ -96,7 +96,7 @@ PORTIONS = [(2, 2), (64, 64), (2, 65), (65, 129), (130, 300), (300, 300), (3, 40
 @pytest.mark.parametrize("window,keep", MASKS + [(200, 1)])
 @pytest.mark.parametrize("heads,kvh,dim,vdim", [s for s in SHAPES if max(s[2:]) <= 256])
 def test_prompt(heads, kvh, dim, vdim, window, keep):
-    """Portions of several sequences (rows, keys) in one launch; long portions take the two-tile form."""
+    """Portions of several sequences (rows, keys) in one launch, 64 rows a workgroup."""
     from nanovllm_hip import ops
     sink = randn(heads, seed=6, dtype=F32)
     for portions in (PORTIONS[:5], PORTIONS[3:]) if dim <= 128 else (PORTIONS[2:6],):

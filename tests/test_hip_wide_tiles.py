@@ -62,3 +62,52 @@ def test_few_portions_over_pages(portions, window, keep, chunk):
             if r:
                 assert torch.equal(got[at:at + r], run(slice(at, at + r), slice(i, i + 1), r)), (heads, i)
             at += r
+
+
+def attend_portions(pg, q, portions, some, most, heads, kvh, chunk=0, turn=None, window=0, keep=0):
+    """Rows of the portions `some`, one after the other."""
+    from nanovllm_hip import ops
+    first = sum(r for r, _ in portions[:some.start or 0])
+    rows = slice(first, first + sum(r for r, _ in portions[some]))
+
+    def cu(lengths):
+        return torch.tensor([0, *lengths]).cumsum(0).int().cuda()
+    return pg.unpad(ops.paged_attend_prompt(pg.pad_q(q[rows]), pg.cache(), pg.tables[some].contiguous().cuda(), cu(r for r, _ in portions[some]), cu(k for _, k in portions[some]), most, heads,
+                                            kvh, pg.dk, pg.dv, 0.2, window, keep, None, chunk=chunk, turn=turn), heads)
+
+
+# 128 rows a workgroup with pairs split over the XCDs and as one list; 64 rows in launches of more workgroups than run at once (no portion of more than 256 rows), and where a CU holds one
+@pytest.mark.parametrize("heads,kvh,dim,portions", [
+    (96, 16, 128, ((130, 900), (257, 257))), (96, 16, 64, ((1, 1), (300, 364), (364, 400))), (112, 2, 128, ((0, 5), (513, 600))), (112, 16, 128, ((250, 250), (130, 900), (256, 300))),
+    (112, 2, 64, ((256, 700), (250, 250), (255, 255))), (8, 8, 256, ((200, 200), (257, 600))), (6, 2, 256, ((1, 300), (140, 140), (65, 700)))])
+@pytest.mark.parametrize("window,keep,chunk", [(0, 0, 0), (70, 40, 0), (0, 0, 96)])
+def test_portions_in_the_order_of_their_work(heads, kvh, dim, portions, window, keep, chunk):
+    from paged_cases import Pages
+    pg = Pages([k for _, k in portions], kvh, dim, dim, torch.bfloat16, seed=4)
+    q = torch.randn(sum(r for r, _ in portions), heads, dim, generator=torch.Generator().manual_seed(heads)).bfloat16()
+    got, at = attend_portions(pg, q, portions, slice(0, len(portions)), max(r for r, _ in portions), heads, kvh, chunk, None, window, keep), 0
+    for i, (r, _) in enumerate(portions):
+        if r:
+            assert torch.equal(got[at:at + r], attend_portions(pg, q, portions, slice(i, i + 1), r, heads, kvh, chunk, None, window, keep)), i
+        at += r
+
+
+@pytest.mark.parametrize("dim,vdim,turned,shift", [(64, 64, 64, 0), (128, 128, 128, 0), (128, 128, 62, 0), (128, 64, 64, 1), (192, 128, 100, 1), (64, 128, 6, 0)])
+def test_turned_outputs_of_many_rows(dim, vdim, turned, shift):
+    """Outputs turned back by 128 rows a workgroup: all columns and some, pairs that do not come in twos, a table `shift` floats behind a border of 8 bytes; the bits of each portion alone
+    (64 rows a workgroup), and rows near the reference."""
+    from paged_cases import Pages, close
+    from test_hip_zaposun_ops import attend_ref, table_of, turned_back
+    heads, kvh, chunk, portions = 48, 2, 100, ((300, 300), (3, 400), (130, 190), (327, 470))
+    whole = table_of(turned)
+    table = torch.cat([whole.new_zeros(shift), whole.flatten()])[shift:].view_as(whole)
+    pg = Pages([k for _, k in portions], kvh, dim, vdim, torch.bfloat16, seed=3)
+    q = torch.randn(sum(r for r, _ in portions), heads, dim, generator=torch.Generator().manual_seed(8)).bfloat16()
+    got, at = attend_portions(pg, q, portions, slice(0, 4), 327, heads, kvh, chunk, table), 0
+    for i, (r, k) in enumerate(portions):
+        assert torch.equal(got[at:at + r], attend_portions(pg, q, portions, slice(i, i + 1), r, heads, kvh, chunk, table)), i
+        for t in {0, 31, 32, 63, 64, 127, 128, r // 2, r - 1}:
+            if t < r:
+                want = turned_back(attend_ref(q[at + t], pg.k[i], pg.v[i], k - r + t, 0.2, chunk, 0), k - r + t, table)
+                close(got[at + t], want, torch.bfloat16, f"portion {i} row {t}")
+        at += r

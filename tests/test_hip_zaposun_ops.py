@@ -539,7 +539,7 @@ PORTIONS = [(2, 2), (64, 64), (2, 65), (65, 129), (130, 300), (300, 300), (3, 40
 @pytest.mark.parametrize("chunk,keep", [(1, 0), (64, 0), (65, 3), (37, 0), (130, 70), (1000, 0)])
 @pytest.mark.parametrize("heads,kvh,dim,vdim", [s for s in SHAPES if max(s[2:]) <= 256])
 def test_prompt_in_chunks(heads, kvh, dim, vdim, chunk, keep):
-    """Portions of several sequences (rows, keys) in one launch; long portions take the two-tile form."""
+    """Portions of several sequences (rows, keys) in one launch, 64 rows a workgroup."""
     table = table_of(vdim)
     for portions in (PORTIONS[:5], PORTIONS[3:]) if dim <= 128 else (PORTIONS[2:6],):
         pg = Pages([k for _, k in portions], kvh, dim, vdim, BF16, seed=3)

@@ -43,7 +43,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 // Diagnostic build only (-DNVH_STAMPS, tools/probes/stamp_prefill.py): wave 0 of every workgroup records the clock at
-// fixed points (slot k of 32 per workgroup).  Never compiled into the shipped library.
+// fixed points (slot k of 32 per workgroup) in the kernels of 64 rows a workgroup; prefill32_kernel (128 rows) records none.  Never compiled into the shipped library.
 #ifdef NVH_STAMPS
 #define PF_STAMP(k)                                                                                      \
     do {                                                                                                 \

@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 209          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch, _status, _variant */
+#define NVH_VERSION 210          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch, _status, _variant; 210: nvh_decode_layers */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -266,6 +266,39 @@ int nvh_greedy_advance(const void* logits, int n_rows, int n, int64_t logits_row
                        int64_t* input_ids, int64_t* positions, int32_t* context_lens, int32_t* slot_mapping,
                        const int32_t* block_tables, int64_t bt_row_stride, int block_size,
                        int64_t* tokens_log, int64_t log_row_stride, int64_t* row_steps, int dtype, void* stream);
+
+/*
+ * The layers of a decode step in ONE launch, for one or two sequences of a model whose layers fit the LDS of the chip (Qwen2-0.5B, Qwen3-0.6B): per layer the five
+ * launches of nvh_linear_small_m_ex / nvh_paged_decode (nanovllm/models/qwen3.py:179-193), same arithmetic and rounding points, same cache.
+ *   layers          host array (read during the call): weights as those calls take them (qkv and gate_up with the norm folded in; q_norm_w / k_norm_w both or neither,
+ *                   the same for all layers; qkv_bias may be NULL), caches [blocks, block_size, kvh, hd]
+ *   x, out          the residual stream [m, hidden] in front of the first and behind the last layer; two buffers.  out_packed: also in fragment order, or NULL
+ *   slot_mapping    < 0: the row is not stored.  A row's earlier tokens may be other rows of this call.  context_lens 0: attends to nothing
+ *   workspace       nvh_decode_layers_workspace bytes (0: these sizes are not served), ZERO-FILLED once, then for calls of the same sizes only; ONE launch at a time per
+ *                   workspace.  Launches with workspaces of their own may run side by side.
+ */
+typedef struct {
+    const void *qkv_w, *qkv_bias, *q_norm_w, *k_norm_w, *o_w, *gate_up_w, *down_w;
+    void *k_cache, *v_cache;
+} nvh_decode_layer;
+typedef struct {
+    const void* x; int64_t x_row_stride;
+    void* out; int64_t out_row_stride;
+    void* out_packed;
+    int32_t m, hidden, h, kvh, hd, inter, n_layers;
+    float norm_eps, post_eps, qk_eps, scale;
+    const nvh_decode_layer* layers;
+    const int64_t* positions; const float* cos_sin;
+    const int32_t *slot_mapping, *context_lens, *block_tables;
+    int64_t bt_row_stride; int32_t block_size, max_blocks;
+    void* workspace; size_t workspace_bytes;
+} nvh_decode_layers_desc;
+size_t nvh_decode_layers_workspace(int m, int hidden, int h, int kvh, int hd, int inter, int n_layers);
+/* longest context for which this is faster than a launch for each part (longer ones are served all the same) */
+int nvh_decode_layers_tokens(int m, int hidden, int h, int kvh, int hd, int inter, int n_layers);
+int nvh_decode_layers(const nvh_decode_layers_desc* desc, int dtype, void* stream);
+/* tests: spin_limit = polls before a workgroup does the shares it waits for (0 = default); workgroups from late_from on start late_for sleeps late */
+int nvh_decode_layers_variant(uint32_t spin_limit, int late_from, int late_for, const nvh_decode_layers_desc* desc, int dtype, void* stream);
 
 /*
  * Engine widening: weight-streaming linear layer for decode-sized batches, out = x . W^T (+ bias), m <= 64 rows.

@@ -26,9 +26,9 @@ MODEL_SOURCES = {
     "Zaposun": ["api_paged.hip", "attn_prep.hip", "paged_attend.hip", "paged_prompt.hip", "streams.hip", "mamba.hip", "wkv.hip"],
     "Kekapel": ["api_talk.hip", "attn_prep.hip", "talk_rows.hip", "talk_prompt.hip", "api_moe.hip", "moe.hip"],
 }
-SOURCES = ["api.hip", "store_kvcache.hip", "paged_decode.hip", "prefill_mfma.hip", "rope_store.hip", "allreduce_oneshot.hip", "qkv_attend.hip", *LINEAR_SOURCES,
+SOURCES = ["api.hip", "store_kvcache.hip", "paged_decode.hip", "prefill_mfma.hip", "rope_store.hip", "allreduce_oneshot.hip", "qkv_attend.hip", "api_decode_layers.hip", "decode_layers.hip", *LINEAR_SOURCES,
            *dict.fromkeys(s for sources in MODEL_SOURCES.values() for s in sources)]
-HEADERS = ["common.h", "kernels.h", "hybrid.h", "mixers.h", "attend_tile.h", "paged_rows.h", "talk.h", "api_common.h", "decode_chunked.h", os.path.join("..", "..", "include", "nvh_attn.h")]
+HEADERS = ["common.h", "kernels.h", "hybrid.h", "mixers.h", "attend_tile.h", "paged_rows.h", "talk.h", "api_common.h", "decode_chunked.h", "decode_layers.h", os.path.join("..", "..", "include", "nvh_attn.h")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -amdgpu-mfma-vgpr-form: MFMA results stay in the architectural VGPRs.  By default hipcc parks accumulators in the AGPR file
 # and pays a v_accvgpr_read/write per element wherever VALU code touches them (softmax on S, rescale of O): 159 such moves in
@@ -43,7 +43,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=f
          "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument"]
 # rope_store.hip must round RoPE's products and sums separately (bit parity with the reference's elementwise fp32 ops);
 # HIP's default backend contraction ignores the source pragma, so that file is built with contraction off.
-FILE_FLAGS = {"rope_store.hip": ["-ffp-contract=off"], "skinny_gemm.hip": ["-ffp-contract=off"], "linear_stream.hip": ["-ffp-contract=off"]}   # its RoPE epilogue too
+FILE_FLAGS = {"rope_store.hip": ["-ffp-contract=off"], "skinny_gemm.hip": ["-ffp-contract=off"], "linear_stream.hip": ["-ffp-contract=off"], "decode_layers.hip": ["-ffp-contract=off"]}   # its RoPE epilogue too
 
 
 def _digest(sources=SOURCES):

@@ -33,6 +33,21 @@ class LinearDesc(ctypes.Structure):
                 ("x_groups", ctypes.c_int32), ("x_group_rows", ctypes.c_int32), ("x_group_stride", ctypes.c_int32)]
 
 
+class DecodeLayer(ctypes.Structure):
+    """nvh_decode_layer (include/nvh_attn.h)."""
+    _fields_ = [(name, ctypes.c_void_p) for name in ("qkv_w", "qkv_bias", "q_norm_w", "k_norm_w", "o_w", "gate_up_w", "down_w", "k_cache", "v_cache")]
+
+
+class DecodeLayersDesc(ctypes.Structure):
+    """nvh_decode_layers_desc (include/nvh_attn.h)."""
+    _fields_ = [("x", ctypes.c_void_p), ("x_row_stride", ctypes.c_int64), ("out", ctypes.c_void_p), ("out_row_stride", ctypes.c_int64), ("out_packed", ctypes.c_void_p),
+                ("m", ctypes.c_int32), ("hidden", ctypes.c_int32), ("h", ctypes.c_int32), ("kvh", ctypes.c_int32), ("hd", ctypes.c_int32), ("inter", ctypes.c_int32),
+                ("n_layers", ctypes.c_int32), ("norm_eps", ctypes.c_float), ("post_eps", ctypes.c_float), ("qk_eps", ctypes.c_float), ("scale", ctypes.c_float),
+                ("layers", ctypes.POINTER(DecodeLayer)), ("positions", ctypes.c_void_p), ("cos_sin", ctypes.c_void_p), ("slot_mapping", ctypes.c_void_p),
+                ("context_lens", ctypes.c_void_p), ("block_tables", ctypes.c_void_p), ("bt_row_stride", ctypes.c_int64), ("block_size", ctypes.c_int32),
+                ("max_blocks", ctypes.c_int32), ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t)]
+
+
 class NormResidualDesc(ctypes.Structure):
     """nvh_norm_residual_desc (include/nvh_attn.h)."""
     _fields_ = [("x", ctypes.c_void_p), ("xb", ctypes.c_void_p), ("packed", ctypes.c_void_p), ("y", ctypes.c_void_p),
@@ -254,6 +269,10 @@ _SIGS = {
                            [ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]),
     "nvh_linear_small_m_ex": (ctypes.c_int, [ctypes.POINTER(LinearDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_linear_small_m_workspace": (ctypes.c_size_t, [ctypes.c_int] * 4),
+    "nvh_decode_layers_workspace": (ctypes.c_size_t, [ctypes.c_int] * 7),
+    "nvh_decode_layers_tokens": (ctypes.c_int, [ctypes.c_int] * 7),
+    "nvh_decode_layers": (ctypes.c_int, [ctypes.POINTER(DecodeLayersDesc), ctypes.c_int, ctypes.c_void_p]),
+    "nvh_decode_layers_variant": (ctypes.c_int, [ctypes.c_uint32, ctypes.c_int, ctypes.c_int, ctypes.POINTER(DecodeLayersDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_qkv_rope_attend": (ctypes.c_int, [ctypes.POINTER(LinearDesc), ctypes.c_void_p, ctypes.c_void_p, _c_i32p, _c_i32p, ctypes.c_int, ctypes.c_int,
                                            ctypes.c_int64, ctypes.c_float, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "nvh_qkv_rope_attend_variant": (ctypes.c_int, [ctypes.c_int, ctypes.c_uint32, ctypes.c_int, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(LinearDesc),

@@ -381,6 +381,11 @@ class QwenForCausalLM(nn.Module):
                              attn_p=torch.zeros(rows * self.layers[0].self_attn.o_proj.weight.shape[1], dtype=torch.bfloat16, device=device),
                              y=torch.zeros((m, cfg.hidden_size), dtype=torch.bfloat16, device=device),     # TP: partial sums to all-reduce
                              ws=torch.zeros(need, dtype=torch.uint8, device=device))
+            a = self.layers[0].self_attn
+            sizes = (m, cfg.hidden_size, a.num_heads, a.num_kv_heads, a.head_dim, inter, len(self.layers))
+            need = 0 if _tp()[1] > 1 else ops.decode_layers_workspace_bytes(*sizes)
+            bufs[key]["layers_ws"] = torch.zeros(need, dtype=torch.uint8, device=device) if need else None
+            bufs[key]["layers_tokens"] = ops.decode_layers_tokens(*sizes) if need else 0
         return bufs[key]
 
     def _forward_decode_fused(self, residual, positions, packed0=None):
@@ -395,6 +400,9 @@ class QwenForCausalLM(nn.Module):
         fw = self._folded_weights()
         m = residual.shape[0]
         b = self._decode_buffers(m, residual.device)
+        cache = self.layers[0].self_attn.attn.k_cache
+        if cache.dim() == 4 and ctx.block_tables.shape[1] * cache.shape[1] <= b["layers_tokens"]:      # (the table is as wide as the longest context may get)
+            return self._forward_decode_layers(residual, positions, ctx, b)
         resid_p, act_p, attn_p, ws, ybuf = b["resid_p"], b["act_p"], b["attn_p"], b["ws"], b["y"]
         tp = _tp()[1]
         # weight prefetch (nvh_linear_desc.prefetch): the qkv launch runs 36 workgroups and the o_proj launch 56 on 256 CUs, each
@@ -457,6 +465,19 @@ class QwenForCausalLM(nn.Module):
                 ops.fused_linear(act_p, mlp.down_proj.weight, x_packed_rows=m, epilogue="none", out=ybuf, workspace=ws)
                 tp_all_reduce_residual_add_pack(ybuf, residual, resid_p)
         return PackedResidual(residual, resid_p)
+
+    def _forward_decode_layers(self, x, positions, ctx, b):
+        """The same step for a few sequences of a model whose layers fit the chip's LDS: all layers in one launch (csrc/decode_layers.hip)."""
+        from .. import ops
+        fw, cfg, a = self._folded_weights(), self.cfg, self.layers[0].self_attn
+        layers = [dict(qkv_w=fw["qkv"][i], qkv_bias=l.self_attn.qkv_proj.bias, q_norm_w=l.self_attn.q_norm.weight if a.qk_norm else None,
+                       k_norm_w=l.self_attn.k_norm.weight if a.qk_norm else None, o_w=l.self_attn.o_proj.weight, gate_up_w=fw["gate_up"][i],
+                       down_w=l.mlp.down_proj.weight, k_cache=l.self_attn.attn.k_cache, v_cache=l.self_attn.attn.v_cache) for i, l in enumerate(self.layers)]
+        out = ops.decode_layers(x, layers, num_heads=a.num_heads, num_kv_heads=a.num_kv_heads, head_dim=a.head_dim, inter=self.layers[0].mlp.down_proj.weight.shape[1],
+                                norm_eps=cfg.rms_norm_eps, post_eps=cfg.rms_norm_eps, qk_eps=cfg.rms_norm_eps, positions=positions,
+                                cos_sin=a.rotary_emb.table(x.device), slot_mapping=ctx.slot_mapping, context_lens=ctx.context_lens, block_tables=ctx.block_tables,
+                                softmax_scale=a.attn.scale, out_packed=b["resid_p"], workspace=b["layers_ws"])
+        return PackedResidual(out, b["resid_p"])
 
     def compute_logits(self, hidden_states):
         w = self.embed_tokens.weight if self.cfg.tie_word_embeddings else self.lm_head.weight

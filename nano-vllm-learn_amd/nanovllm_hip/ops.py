@@ -555,6 +555,56 @@ def qkv_rope_attend_status(workspace=None, device=None) -> int:
     return int(v.value)
 
 
+def decode_layers_workspace_bytes(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers) -> int:
+    """Scratch of decode_layers for these sizes, zero-filled once by the caller; 0: they are not served in one launch."""
+    return int(_lib.load().nvh_decode_layers_workspace(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers))
+
+
+def decode_layers_tokens(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers) -> int:
+    """Longest context for which decode_layers is faster than a launch for each part of a layer."""
+    return int(_lib.load().nvh_decode_layers_tokens(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers))
+
+
+def decode_layers(x, layers, *, num_heads, num_kv_heads, head_dim, inter, norm_eps, post_eps, positions, cos_sin, slot_mapping, context_lens, block_tables, workspace,
+                  qk_eps=1e-6, softmax_scale=None, out=None, out_packed=None, spin_limit=0, late_from=0, late_for=0):
+    """nvh_decode_layers: all layers of a decode step of one or two sequences in one launch (nanovllm/models/qwen3.py:179-193).
+
+    x [m, hidden]: the stream in front of the first layer; returns it behind the last one (`out`, never x), also in fragment order if out_packed is given.
+    layers: a dict per layer of qkv_w (norm folded in), qkv_bias (or None), q_norm_w, k_norm_w (both or None), o_w, gate_up_w (norm folded in), down_w, k_cache, v_cache.
+    spin_limit, late_from, late_for: tests only (nvh_decode_layers_variant)."""
+    m, hidden = x.shape
+    _require_gpu_bf16(x=x)
+    _require_i32(slot_mapping=slot_mapping, context_lens=context_lens, block_tables=block_tables)
+    assert x.stride(1) == 1 and positions.dtype == torch.int64 and positions.numel() == m and positions.is_contiguous() and positions.is_cuda
+    assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.shape[-1] == head_dim
+    assert slot_mapping.numel() == m and slot_mapping.is_contiguous() and context_lens.numel() == m and context_lens.is_contiguous()
+    assert block_tables.dim() == 2 and block_tables.shape[0] == m and block_tables.stride(1) == 1
+    nqkv, qsize, page = (num_heads + 2 * num_kv_heads) * head_dim, num_heads * head_dim, layers[0]["k_cache"].shape[1]
+    shapes = dict(qkv_w=(nqkv, hidden), o_w=(hidden, qsize), gate_up_w=(2 * inter, hidden), down_w=(hidden, inter), qkv_bias=(nqkv,), q_norm_w=(head_dim,), k_norm_w=(head_dim,))
+    descs = (_lib.DecodeLayer * len(layers))()
+    for desc, layer in zip(descs, layers):
+        for name, _ in desc._fields_:
+            t = layer.get(name)
+            if t is not None:
+                assert t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous() and (tuple(t.shape) == shapes[name] if name in shapes else
+                                                                                         tuple(t.shape[1:]) == (page, num_kv_heads, head_dim)), name
+                setattr(desc, name, t.data_ptr())
+    if out is None:
+        out = torch.empty((m, hidden), dtype=torch.bfloat16, device=x.device)
+    _require_gpu_bf16(out=out)
+    assert out.shape == x.shape and out.stride(1) == 1 and workspace.is_cuda and workspace.is_contiguous()
+    assert out_packed is None or (out_packed.dtype == torch.bfloat16 and out_packed.is_contiguous() and out_packed.numel() >= (m + 15) // 16 * 16 * hidden)
+    d = _lib.DecodeLayersDesc(
+        x=x.data_ptr(), x_row_stride=x.stride(0), out=out.data_ptr(), out_row_stride=out.stride(0), out_packed=None if out_packed is None else out_packed.data_ptr(),
+        m=m, hidden=hidden, h=num_heads, kvh=num_kv_heads, hd=head_dim, inter=inter, n_layers=len(layers), norm_eps=norm_eps, post_eps=post_eps, qk_eps=qk_eps,
+        scale=head_dim ** -0.5 if softmax_scale is None else softmax_scale, layers=descs, positions=positions.data_ptr(), cos_sin=cos_sin.data_ptr(),
+        slot_mapping=slot_mapping.data_ptr(), context_lens=context_lens.data_ptr(), block_tables=block_tables.data_ptr(), bt_row_stride=block_tables.stride(0),
+        block_size=page, max_blocks=block_tables.shape[1], workspace=workspace.data_ptr(), workspace_bytes=workspace.numel() * workspace.element_size())
+    rc = _lib.load().nvh_decode_layers_variant(spin_limit, late_from, late_for, ctypes.byref(d), NVH_BF16, _stream())
+    _lib.check(rc, "nvh_decode_layers")
+    return out
+
+
 def linear_candidate_groups(n, k) -> int:
     return int(_lib.load().nvh_linear_small_m_candidate_groups(n, k))
 

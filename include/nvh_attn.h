@@ -268,7 +268,7 @@ int nvh_greedy_advance(const void* logits, int n_rows, int n, int64_t logits_row
                        int64_t* tokens_log, int64_t log_row_stride, int64_t* row_steps, int dtype, void* stream);
 
 /*
- * The layers of a decode step in ONE launch, for one or two sequences of a model whose layers fit the LDS of the chip (Qwen2-0.5B, Qwen3-0.6B): per layer the five
+ * The layers of a decode step in ONE launch, for up to three sequences of a model whose layers fit the registers of the chip (Qwen2-0.5B, Qwen3-0.6B): per layer the five
  * launches of nvh_linear_small_m_ex / nvh_paged_decode (nanovllm/models/qwen3.py:179-193), same arithmetic and rounding points, same cache.
  *   layers          host array (read during the call): weights as those calls take them (qkv and gate_up with the norm folded in; q_norm_w / k_norm_w both or neither,
  *                   the same for all layers; qkv_bias may be NULL), caches [blocks, block_size, kvh, hd]

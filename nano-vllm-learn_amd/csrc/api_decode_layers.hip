@@ -7,25 +7,25 @@
 
 namespace nvh {
 
-static int up(int x, int to) { return (x + to - 1) / to * to; }
 static uint32_t magic_of(uint32_t d) { return (uint32_t)((1ull << 32) / d + 1); }
 
 int plan_decode_layers(DecodeLayersArgs& a, int cus, int m, int hidden, int h, int kvh, int hd, int inter, int layers) {
     if (m < 1 || m > kDecodeLayersRows || (hd != 64 && hd != 128) || kvh <= 0 || h % kvh || h / kvh > 16 || layers < 1 || layers > kDecodeLayersMost) return 0;
-    if (hidden % 8 || inter % 8 || hidden <= 0 || inter <= 0 || hidden > 8192 || inter > 16384 || cus < 64) return 0;
     const int qsize = h * hd, nqkv = (h + 2 * kvh) * hd;
-    const int kv = kDecodeLayersWalkers(hd) * kDecodeLayersBuffers(hd) * 64 * hd;
+    // what a wave holds of the weights: rows of up to 2, 4 and 10 times 64 pieces of 16 bytes
+    if (hidden % 8 || inter % 8 || hidden <= 0 || inter <= 0 || hidden > 1024 || qsize > 2048 || inter > 5120 || cus < 64) return 0;
+    const int kv = kDecodeLayersWalkers * kDecodeLayersBuffers * 64 * hd;
+    const int front_lds = kLdsCommon + kv + 2 * m * (hidden + qsize) + 16 * (2 * hd + 16) + 2 * m * 2 * hd + kDecodeLayersWalkers * 2 * 16 * 4, rest_lds = kLdsCommon + 2 * m * (hidden + inter);
+    const int lds = front_lds > rest_lds ? front_lds : rest_lds;
+    if (lds > kDecodeLayersLds) return 0;
     auto per = [](int n, int parts) { return (n + parts - 1) / parts; };
-    int best = 0, best_rounds = 0, best_load = 0, best_lds = 0;
+    int best = 0, best_rounds = 0, best_load = 0;
     for (int nf = 16; nf <= cus - 16; nf += 4) {
         const int nm = cus - nf;
         const int rq = per(nqkv, nf), ro = per(hidden, nf), rg = per(inter, nm), rd = per(hidden, nm);
-        if (nf < m * kvh || rq > kDecodeLayersColumns || ro > kDecodeLayersColumns || rg > kDecodeLayersColumns || rd > kDecodeLayersColumns) continue;
-        const int f = up(rq * hidden * 2, 1024) + up(ro * qsize * 2, 1024) + kv + 2 * m * (hidden + qsize) + 16 * (2 * hd + 16) + 2 * m * 2 * hd + kDecodeLayersWalkers(hd) * 2 * 16 * 4;
-        const int g = 2 * up(rg * hidden * 2, 1024) + up(rd * inter * 2, 1024) + 2 * m * (hidden + inter);
-        if (kLdsCommon + f > kDecodeLayersLds || kLdsCommon + g > kDecodeLayersLds) continue;
-        const int rounds = per(rq, 24) + per(ro, 24) + 2 * per(rg, 24) + per(rd, 24), load = f > g ? f : g;
-        if (!best || rounds < best_rounds || (rounds == best_rounds && load < best_load)) { best = nf; best_rounds = rounds; best_load = load; best_lds = kLdsCommon + load; }
+        if (nf < m * kvh || rq > 48 || ro > 24 || rg > 24 || rd > 8) continue;             // eight waves with three columns each, one of down; two rounds of qkv
+        const int f = rq * hidden + ro * qsize, g = 2 * rg * hidden + rd * inter, load = f > g ? f : g, rounds = per(rq, 24);
+        if (!best || rounds < best_rounds || (rounds == best_rounds && load < best_load)) { best = nf; best_rounds = rounds; best_load = load; }
     }
     if (!best) return 0;
     const int nf = best, nm = cus - nf;
@@ -33,31 +33,27 @@ int plan_decode_layers(DecodeLayersArgs& a, int cus, int m, int hidden, int h, i
     a.grid = cus; a.nf = nf; a.nm = nm;
     a.chunks = nf / (m * kvh) < 16 ? nf / (m * kvh) : 16;
     a.shares = m * kvh * a.chunks;
-    // Attention is the front's alone, its tiles of 16 tokens come a round of the waves at a time (1.3 us), where a launch of its own has the whole chip: five rounds of one
-    // sequence are worth what the rest gains, three of two.  Whole steps, one launch against five a layer: Qwen3-0.6B one sequence of 2000 / 4096 tokens (3 / 5 rounds) 652 / 755 us
-    // against 768 / 817; two of 768 / 1500 / 2500 (2 / 4 / 6 rounds) 666 / 765 / 867 against 737 / 771 / 834; Qwen2-0.5B two of 4096 (3 rounds) 572 against 639
-    a.most_tokens = a.chunks * kDecodeLayersWalkers(hd) * 16 * (m == 1 ? 5 : 3);
+    // Attention is the front's alone, its tokens come a round (two tiles of 16 of each of eight waves) behind the other, where a launch of its own has the whole chip: up to six times
+    // 128 tokens a share of one sequence, three and a half of two, two and a half of three are worth what the rest gains.  Whole steps, this against five launches a layer: Qwen3-0.6B one sequence of 4096 tokens (2.8 times 128 a share)
+    // 655 us against 822; two of 1500 / 2500 / 3500 (2.1 / 3.6 / 5 times) 678 / 807 / 888 against 777 / 832 / 847; three of 1500 (3.2) 807 against 837; Qwen2-0.5B two of 4096 (2.7)
+    // 566 against 628, three of 2048 / 4096 (2 / 4) 579 / 671 against 623 / 640
+    a.most_tokens = a.chunks * kDecodeLayersWalkers * 16 * (m == 1 ? 12 : m == 2 ? 7 : 5) / 2;
     a.nf_magic = magic_of(nf); a.nm_magic = magic_of(nm); a.chunks_magic = magic_of(a.chunks); a.kvh_magic = magic_of(kvh); a.group_magic = magic_of(a.group); a.h_magic = magic_of(h);
     a.o_qkv = 0; a.o_o = m * nqkv; a.o_act = a.o_o + m * hidden; a.o_down = a.o_act + m * inter; a.o_rec = a.o_down + m * hidden;
     a.layer_words = a.o_rec + (int64_t)a.shares * a.group * 2 * (hd + 2);
     int at = kLdsCommon;
     auto take = [&](int bytes) { const int x = at; at += bytes; return x; };
-    a.l_region[0] = take(up(per(nqkv, nf) * hidden * 2, 1024));
-    a.l_region[2] = take(up(per(hidden, nf) * qsize * 2, 1024));
     a.l_kv = take(kv);
     a.l_x[0] = take(2 * m * hidden);
     a.l_x[2] = take(2 * m * qsize);
     a.l_q = take(16 * (2 * hd + 16));
     a.l_news = take(2 * m * 2 * hd);
-    a.l_ml = take(kDecodeLayersWalkers(hd) * 2 * 16 * 4);
-    a.l_region[1] = a.l_x[1] = 0;
+    a.l_ml = take(kDecodeLayersWalkers * 2 * 16 * 4);
+    a.l_x[1] = 0;
     at = kLdsCommon;
-    a.l_up = up(per(inter, nm) * hidden * 2, 1024);
-    a.l_region[3] = take(2 * a.l_up);
-    a.l_region[4] = take(up(per(hidden, nm) * inter * 2, 1024));
     a.l_x[3] = take(2 * m * hidden);
     a.l_x[4] = take(2 * m * inter);
-    return best_lds;
+    return lds;
 }
 
 static int device_cus() {

@@ -8,13 +8,12 @@
 namespace nvh {
 
 constexpr int kDecodeLayersMost = 32;            // layers of a launch: their pointers are kernel arguments (4 KB)
-constexpr int kDecodeLayersRows = 2;             // sequences of a step
+constexpr int kDecodeLayersRows = 3;             // sequences of a step
 constexpr int kDecodeLayersLds = 160 * 1024;
 constexpr int kDecodeLayersSync = 1024;          // bytes in front of the words: [0] launches so far, [32] workgroups of this one, [64] a workgroup gave up
-constexpr int kDecodeLayersColumns = 48;         // of a workgroup's share of a projection (of gate and of up each)
+constexpr int kDecodeLayersColumns = 48;            // of a workgroup's share of a projection (of gate and of up each)
 constexpr int kLdsSay = 0, kLdsResults = 128, kLdsRope = kLdsResults + kDecodeLayersRows * kDecodeLayersColumns * 4, kLdsCommon = kLdsRope + kDecodeLayersRows * 128 * 4;     // bytes of LDS both kinds of workgroup lay out alike
-constexpr int kDecodeLayersWalkers(int hd) { return hd == 64 ? 8 : 4; }      // attention: waves that take tiles of 16 tokens, and tiles of a wave in LDS
-constexpr int kDecodeLayersBuffers(int hd) { return hd == 64 ? 2 : 1; }
+constexpr int kDecodeLayersWalkers = 8, kDecodeLayersBuffers = 2;      // attention: waves that take tiles of 16 tokens, and tiles of a wave in LDS
 
 struct DecodeLayersArgs {
     const uint16_t* x;                           // [m, hidden], the stream in front of the first layer
@@ -40,7 +39,7 @@ struct DecodeLayersArgs {
     uint32_t nf_magic, nm_magic, chunks_magic, kvh_magic, group_magic, h_magic;
     int o_qkv, o_o, o_act, o_down, o_rec;        // words of a layer
     int l_kv, l_q, l_news, l_ml;      // bytes of LDS
-    int l_region[5], l_up, l_x[5];               // weights (up's behind gate's) and inputs of the phases
+    int l_x[5];                                  // inputs of the phases
     nvh_decode_layer layer[kDecodeLayersMost];
 };
 

@@ -1,25 +1,28 @@
-// A decode step's layers in one launch, for one or two sequences: (folded RMSNorm ->) qkv projection -> (q/k norm ->) RoPE, K/V store and attention over pages ->
-// output projection + residual -> (folded RMSNorm ->) gate_up, SiLU -> down projection + residual, for every layer of a decoder whose layers fit the LDS of the
-// chip (Qwen2-0.5B: 30 MB a layer, 40 MB of LDS).  Replaces five launches a layer (nanovllm/models/qwen3.py:179-193).
+// A decode step's layers in one launch, for up to three sequences: (folded RMSNorm ->) qkv projection -> (q/k norm ->) RoPE, K/V store and attention over pages ->
+// output projection + residual -> (folded RMSNorm ->) gate_up, SiLU -> down projection + residual, for every layer of a decoder whose layers fit the registers of
+// the chip (Qwen2-0.5B: 30 MB a layer, 128 MB of registers).  Replaces five launches a layer (nanovllm/models/qwen3.py:179-193).
 //
 // What bounds such a step is latency.  A launch that depends on the one before costs 1.5 us of boundary, 0.5 of dispatch and 1.9 until its first weights arrive,
 // five times a layer (Qwen2-0.5B, one sequence: 22 us a layer, whose weights stream in 6).  Here:
 //   * The workgroups, one a CU, stay.  `nf` of them (the front) hold rows of the qkv and output projections and attend, the others hold rows of gate_up and
-//     down.  A workgroup keeps its rows of the weights in LDS and asks for the next layer's as soon as it is done with this layer's: the front's weights and
-//     keys travel while the others work, theirs while the front works.  (Weights asked for while a workgroup itself waits would cost it their time: a wave's
-//     loads, and those of a CU, return in order, and a poll waits behind them.)
+//     down.  A wave keeps its rows of the weights in registers and asks for the next layer's as soon as the workgroup is done with this layer's: the front's
+//     weights and keys travel while the others work, theirs while the front works.  (Weights asked for while a workgroup itself waits would cost it their time: a
+//     wave's loads, and those of a CU, return in order, and a poll waits behind them.  The others ask for two pieces at a time: 200 CUs with all of theirs under way
+//     keep the front's polls waiting; four at a time 362 -> 366 us a step.)
 //   * Results go from workgroup to workgroup through memory, marked: an activation is a 4-byte word (bf16 value, low half of the launch's number), a share of
 //     an attention output an 8-byte word (fp32 value, number of the launch).  Both are written and read whole, so a reader that finds the mark has the value:
-//     no flag, no fence, no second trip.  A hop between all workgroups takes 1.5 to 1.8 us, with a flag for each workgroup 2.4 to 3.2.  Stores are written
+//     no flag, no fence, no second trip.  A hop between all workgroups takes 1.2 to 1.6 us, with a flag for each workgroup 2.4 to 3.2.  Stores are written
 //     through, loads pass the caches (sc1).  Every layer has words of its own, so no word is written twice by a launch, and every launch writes all that it
 //     reads: what such a word holds before is the mark of an earlier launch (or 0, as it was allocated).
 //   * A wait that lasts too long (`spin_limit` polls, 3 ms: workgroups that have not been placed yet, because another stream's kernels hold their CUs) is ended
 //     by work: the workgroup goes through the phases since its last one and does every share of which no results have come, whose ever it is.  A share's inputs
 //     are complete when it is done; done twice it writes the same bits; and nothing is overwritten that a share reads.  So the step ends however few workgroups
 //     run at a time.
-// A column of a product is a wave's: its lanes take 16-byte pieces of the weight row and of the activations and add up (reads of 1 KB from LDS without conflicts;
-// 16 x 16 matrix tiles would read 64 lanes' worth for the few columns a workgroup has: 2.1 us for the down projection where this takes 0.7).
-// One sequence of 513 to 1024 tokens, Qwen2-0.5B, whole step with the LM head: 603 -> 387 us; two sequences 604 -> 459; Qwen3-0.6B 733 -> 556 and 737 -> 666.
+// A column of a product is a wave's: its lanes hold 16-byte pieces of the weight row, 64 apart, and add up products with the same pieces of the activations
+// (16 x 16 matrix tiles would read 64 lanes' worth of LDS for the few columns a workgroup has: 2.1 us for the down projection where this takes 0.5).  Eight waves of
+// three columns rather than twelve of two: sums and epilogues are issued by fewer waves.  Up to three rows; four would take as long as launches of their own.
+// Whole step with the LM head, contexts of 513 to 1024 tokens, launches -> this: Qwen2-0.5B one sequence 604 -> 362 us (layers with LDS for the weights and twelve
+// waves 387), two 605 -> 446, three 611 -> 525; Qwen3-0.6B 734 -> 507, 741 -> 602, 768 -> 728.
 // Arithmetic and rounding points are those of linear_stream.hip, rope_store.hip and decode_chunked.h (P as hi + lo); sums have another order.
 #include "decode_layers.h"
 
@@ -32,11 +35,13 @@ namespace nvh {
 
 namespace {
 
-constexpr int kWavesWg = 12, kThreads = kWavesWg * 64;
+constexpr int kWavesWg = 8, kThreads = kWavesWg * 64;
+constexpr int kColumns = 3;                      // of a projection that a wave takes at a time (down: one)
 constexpr int kPhases = 5;
 constexpr int kMostColumns = kDecodeLayersColumns;
+constexpr int kHeld = 24;                        // 16-byte registers of weights
 constexpr int kRounds = 2;                       // rounds of the waves over the columns of a share, at most (plan_decode_layers)
-constexpr int kFlightFront = 4, kFlightRest = 2;               // loads of weights a wave has under way
+constexpr int kFlightFront = 8, kFlightRest = 2;               // loads of weights a wave has under way
 enum { PH_QKV, PH_ATTEND, PH_O, PH_GATE_UP, PH_DOWN };
 
 __device__ __forceinline__ void barrier_lds() {  // orders LDS traffic only: loads into LDS stay in flight
@@ -56,7 +61,7 @@ __device__ __forceinline__ Word* uniform(const Word* p) {
 // N 16-byte loads past the caches, waited for: base + off[i]
 template <int N>
 __device__ __forceinline__ void load_through(u32x4 (&v)[N], const Word* base, const uint32_t (&off)[N]) {
-    static_assert(N == 1 || N == 2 || N == 4 || N == 8 || N == 16, "");
+    static_assert(N == 1 || N == 2 || N == 4 || N == 8, "");
     if constexpr (N == 1) {
         asm volatile("global_load_dwordx4 %0, %1, %2 sc1\n s_waitcnt vmcnt(0)" : "=&v"(v[0]) : "v"(off[0]), "s"(base) : "memory");
     } else if constexpr (N == 2) {
@@ -66,25 +71,6 @@ __device__ __forceinline__ void load_through(u32x4 (&v)[N], const Word* base, co
         asm volatile("global_load_dwordx4 %0, %4, %8 sc1\n global_load_dwordx4 %1, %5, %8 sc1\n global_load_dwordx4 %2, %6, %8 sc1\n"
                      "global_load_dwordx4 %3, %7, %8 sc1\n s_waitcnt vmcnt(0)"
                      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]) : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base) : "memory");
-    } else if constexpr (N == 16) {
-        asm volatile("global_load_dwordx4 %0, %16, %32 sc1\n"
-                     "global_load_dwordx4 %1, %17, %32 sc1\n"
-                     "global_load_dwordx4 %2, %18, %32 sc1\n"
-                     "global_load_dwordx4 %3, %19, %32 sc1\n"
-                     "global_load_dwordx4 %4, %20, %32 sc1\n"
-                     "global_load_dwordx4 %5, %21, %32 sc1\n"
-                     "global_load_dwordx4 %6, %22, %32 sc1\n"
-                     "global_load_dwordx4 %7, %23, %32 sc1\n"
-                     "global_load_dwordx4 %8, %24, %32 sc1\n"
-                     "global_load_dwordx4 %9, %25, %32 sc1\n"
-                     "global_load_dwordx4 %10, %26, %32 sc1\n"
-                     "global_load_dwordx4 %11, %27, %32 sc1\n"
-                     "global_load_dwordx4 %12, %28, %32 sc1\n"
-                     "global_load_dwordx4 %13, %29, %32 sc1\n"
-                     "global_load_dwordx4 %14, %30, %32 sc1\n"
-                     "global_load_dwordx4 %15, %31, %32 sc1\n s_waitcnt vmcnt(0)"
-                     : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]), "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11]), "=&v"(v[12]), "=&v"(v[13]), "=&v"(v[14]), "=&v"(v[15])
-                     : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]), "v"(off[5]), "v"(off[6]), "v"(off[7]), "v"(off[8]), "v"(off[9]), "v"(off[10]), "v"(off[11]), "v"(off[12]), "v"(off[13]), "v"(off[14]), "v"(off[15]), "s"(base) : "memory");
     } else {
         asm volatile("global_load_dwordx4 %0, %8, %16 sc1\n global_load_dwordx4 %1, %9, %16 sc1\n global_load_dwordx4 %2, %10, %16 sc1\n"
                      "global_load_dwordx4 %3, %11, %16 sc1\n global_load_dwordx4 %4, %12, %16 sc1\n global_load_dwordx4 %5, %13, %16 sc1\n"
@@ -118,16 +104,18 @@ __device__ __forceinline__ Args& fresh_args() {
 template <int N>
 __device__ __forceinline__ void loads_left() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// sums over the wave of two values: of the first in the lower 32 lanes, of the second in the upper ones
-__device__ __forceinline__ float sum_two(float x, float y) {
-    float t = fold32(x, y);
-    t = sum_xor16(t);
-    return group_sum<16>(t);
+// Sums over the wave of four values: a row of 16 lanes each, in the order 0, 2, 1, 3 (column_of)
+__device__ __forceinline__ float sum_four(float v0, float v1, float v2, float v3) { return group_sum<16>(fold16(fold32(v0, v1), fold32(v2, v3))); }
+__device__ __forceinline__ int column_of(int lane) { return (lane >> 5) | ((lane >> 3) & 2); }
+__device__ __forceinline__ float sum_wave(float v) {
+    v = sum_xor16(v);
+    v = sum_xor32(v);
+    return group_sum<16>(v);
 }
 
 template <int D>
 struct Walk {                                    // attention: waves that take 16-token tiles, and tiles of a wave in LDS
-    static constexpr int kWaves = kDecodeLayersWalkers(D), kBufs = kDecodeLayersBuffers(D);
+    static constexpr int kWaves = kDecodeLayersWalkers, kBufs = kDecodeLayersBuffers;
     static constexpr int kRow = D * 2, kImage = 16 * kRow, kBuf = 2 * kImage, kWave = kBufs * kBuf;
 };
 
@@ -151,7 +139,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
             for (int i = 0; i < a.late_for; ++i) __builtin_amdgcn_s_sleep(8);    // (tests: workgroups that start late)
     }
     // what every layer needs of the step's rows: context, slot, cos and sin of the position
-    LdsWord* const row_ctx = say + 8, * const row_slot = say + 8 + M;
+    LdsWord* const row_ctx = say + 8, * const row_slot = say + 16;
     float* const rope = reinterpret_cast<float*>(lds + kLdsRope);
     {
         Args& a = fresh_args();
@@ -168,7 +156,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
     auto layer_words = [&](Args& a, int l) { return uniform((const Word*)a.ws + (int64_t)l * a.layer_words); };
 
     // ---- a share of a projection: n columns from c0 on (gate_up: n of gate and the same n of up), contraction k
-    struct Share { int c0, n, k, region, x; };
+    struct Share { int c0, n, k, x; };
     auto share = [&](Args& a, int ph, int role) {
         Share s;
         const int N = ph == PH_QKV ? a.nqkv : ph == PH_GATE_UP ? a.inter : a.hidden;
@@ -177,26 +165,33 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
         s.c0 = div_by(N * role, R, magic);
         s.n = div_by(N * (role + 1), R, magic) - s.c0;
         s.k = ph == PH_O ? a.qsize : ph == PH_DOWN ? a.inter : a.hidden;
-        s.region = a.l_region[ph];
         s.x = a.l_x[ph];
         return s;
     };
-    // ---- this wave's part of a share's weights into LDS, as they lie in memory
-    auto ask_rows = [&](const uint16_t* w, int bytes, int to) {
-        const int lane = lane_now();
-        const char* const src = reinterpret_cast<const char*>(w);
-        for (int i = wave * 1024; i < bytes; i += kWavesWg * 1024) {
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + min(i + 16 * lane, bytes - 16)),
-                                             (__attribute__((address_space(3))) void*)(lds + to + i), 16, 0, NVH_DMA_AUX);
+    // ---- the weights of this wave's columns, in registers: a row's 16-byte pieces lie 64 apart in a lane (zeros past its end: the buffer says where that is).
+    // Front: qkv, two rounds of three columns of two pieces, then the output projection, three of four; the others: gate, up, three columns of two each, then down, one of ten
+    u32x4 held[kHeld];
+    auto row_buffer = [&](const uint16_t* w, int row, int rows, int k, int skip) {         // (no such row, or none left behind `skip` bytes: zeros, and no traffic)
+        const int bytes = row < rows && 2 * k > skip ? 2 * k - skip : 0;
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(w + (int64_t)(row < rows ? row : 0) * k + skip / 2), 0, bytes, 0x00020000);
+    };
+    auto ask_weights = [&](Args& a, int l, int role) {
+        const Share s = share(a, front ? PH_QKV : PH_GATE_UP, role), t = share(a, front ? PH_O : PH_DOWN, role);
+        const uint16_t* const w = reinterpret_cast<const uint16_t*>(front ? a.layer[l].qkv_w : a.layer[l].gate_up_w) + (int64_t)s.c0 * s.k;
+        const uint16_t* const v = reinterpret_cast<const uint16_t*>(front ? a.layer[l].o_w : a.layer[l].down_w) + (int64_t)t.c0 * t.k;
+        const int c = kColumns * wave, d = front ? c + kColumns * kWavesWg : c;
+        const uint16_t* const w2 = front ? w : w + (int64_t)a.inter * s.k;
+        const __amdgpu_buffer_rsrc_t row[9] = {
+            row_buffer(w, c, s.n, s.k, 0), row_buffer(w, c + 1, s.n, s.k, 0), row_buffer(w, c + 2, s.n, s.k, 0),
+            row_buffer(w2, d, s.n, s.k, 0), row_buffer(w2, d + 1, s.n, s.k, 0), row_buffer(w2, d + 2, s.n, s.k, 0),
+            row_buffer(v, front ? c : wave, t.n, t.k, 0), row_buffer(v, front ? c + 1 : wave, t.n, t.k, front ? 0 : 4096), row_buffer(v, front ? c + 2 : wave, t.n, t.k, front ? 0 : 8192)};
+        const int at = 16 * lane_now();
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i) {
+            held[i] = __builtin_amdgcn_raw_buffer_load_b128(row[i < 12 ? i >> 1 : i / 4 + 3], at, 1024 * (i < 12 ? i & 1 : i & 3), NVH_DMA_AUX);
             if (front) loads_left<kFlightFront - 1>();
             else loads_left<kFlightRest - 1>();
         }
-    };
-    auto ask_weights = [&](Args& a, int l, int ph, int role) {
-        const Share s = share(a, ph, role);
-        const uint16_t* const w = reinterpret_cast<const uint16_t*>(ph == PH_QKV ? a.layer[l].qkv_w : ph == PH_O ? a.layer[l].o_w : ph == PH_GATE_UP ? a.layer[l].gate_up_w : a.layer[l].down_w);
-        ask_rows(w + (int64_t)s.c0 * s.k, s.n * s.k * 2, s.region);
-        if (ph == PH_GATE_UP) ask_rows(w + (int64_t)(a.inter + s.c0) * s.k, s.n * s.k * 2, s.region + a.l_up);
     };
 
     // ---- attention: what a share is
@@ -278,14 +273,8 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
     auto ask_layer = [&](int l) {                                                // everything of the next layer that waits for nothing
         l = __builtin_amdgcn_readfirstlane(l);
         Args& a = fresh_args();
-        if (front) {
-            ask_weights(a, l, PH_QKV, own);
-            ask_tiles(a, l, own);
-            ask_weights(a, l, PH_O, own);
-        } else {
-            ask_weights(a, l, PH_GATE_UP, own);
-            ask_weights(a, l, PH_DOWN, own);
-        }
+        ask_weights(a, l, own);
+        if (front) ask_tiles(a, l, own);
     };
 
     // ---- gathering.  quads: 16-byte pieces, thread t takes t, t + kThreads, ...; use(piece, words) for each.  Marks are checked piece by piece
@@ -333,56 +322,46 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
             for (int c = tid; c < per; c += kThreads) *reinterpret_cast<u32x4*>(lds + x + m * 2 * a.hidden + 16 * c) = *reinterpret_cast<const u32x4*>(a.x + m * a.x_stride + 8 * c);
     };
 
-    // ---- products of R rows of weights with the M rows of activations: this lane's share of each sum.  A lane takes every 64th piece of 16 bytes; U pieces of
-    // each row are asked for at once
-    auto dots = [&](const unsigned char* x, int k, const unsigned char* const (&w)[4], auto rows_tag, auto unroll_tag, auto norm_tag, float (&acc)[4][M], float (&ss)[M]) {
-        constexpr int R = decltype(rows_tag)::value, U = decltype(unroll_tag)::value;
-        constexpr bool norm = decltype(norm_tag)::value;
-        const int lane = lane_now(), pieces = k >> 3;
-        for (int p0 = 0; p0 < pieces; p0 += 64 * U) {
-            u32x4 xv[U][M], wv[U][R];
+    // ---- products of R rows of P pieces with the M rows of activations: this lane's share of each sum.  piece(row, i): a piece of the row's weights
+    auto dots = [&](const unsigned char* x, int k, auto rows_tag, auto pieces_tag, auto norm_tag, float (&acc)[6][M], float (&ss)[M], auto piece) {
+        constexpr int R = decltype(rows_tag)::value, P = decltype(pieces_tag)::value;
+        const int lane = lane_now(), last = (k >> 3) - 1;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int p = p0 + 64 * u + lane;
+        for (int m = 0; m < M; ++m) {
+            if (m > 0) asm volatile("" ::: "memory");                            // (a row's pieces at a time: registers)
+            u32x4 xv[P];
 #pragma unroll
-                for (int m = 0; m < M; ++m) xv[u][m] = u32x4{0, 0, 0, 0};
+            for (int i = 0; i < P; ++i) xv[i] = *reinterpret_cast<const u32x4*>(x + m * 2 * k + 16 * min(64 * i + lane, last));
 #pragma unroll
-                for (int r = 0; r < R; ++r) wv[u][r] = u32x4{0, 0, 0, 0};
-                if (p < pieces) {
+            for (int i = 0; i < P; ++i) {
+                if (64 * i + lane > last) xv[i] = u32x4{0, 0, 0, 0};
+                u32x4 wv[R];
 #pragma unroll
-                    for (int m = 0; m < M; ++m) xv[u][m] = *reinterpret_cast<const u32x4*>(x + m * 2 * k + 16 * p);
+                for (int r = 0; r < R; ++r) wv[r] = piece(r, i);
 #pragma unroll
-                    for (int r = 0; r < R; ++r) wv[u][r] = *reinterpret_cast<const u32x4*>(w[r] + 16 * p);
+                for (int j = 0; j < 4; ++j) {
+                    if constexpr (decltype(norm_tag)::value) ss[m] = dot2_bf16(xv[i][j], xv[i][j], ss[m]);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) acc[r][m] = dot2_bf16(xv[i][j], wv[r][j], acc[r][m]);
                 }
             }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int m = 0; m < M; ++m)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        if (norm) ss[m] = dot2_bf16(xv[u][m][i], xv[u][m][i], ss[m]);
-#pragma unroll
-                        for (int r = 0; r < R; ++r) acc[r][m] = dot2_bf16(xv[u][m][i], wv[u][r][i], acc[r][m]);
-                    }
         }
     };
 
     bool have_x = false;                                                         // the stream that the residual sums need is in LDS
     // ---- one share of a projection: a wave takes two columns (gate_up: two of gate and the two of up that belong to them) of every 24
-    // ready: its weights have been asked for.  Returns whether a wait ran out
-    auto project = [&](auto phase, int l, int role, bool ready) -> bool {
+    // help: another workgroup's, whose weights are not held but read.  Returns whether a wait ran out
+    auto project = [&](auto phase, auto help, int l, int role) -> bool {
         constexpr int ph = decltype(phase)::value;
         constexpr bool norm = ph == PH_QKV || ph == PH_GATE_UP;
-        constexpr int C = ph == PH_DOWN ? 1 : 2;                                 // columns a wave takes at a time
+        constexpr int C = ph == PH_DOWN ? 1 : kColumns;
         Args& a = fresh_args();
         const int G = a.group, lane = lane_now(), tid = wave * 64 + lane;
         Word* const words = layer_words(a, l);
         const Share s = share(a, ph, role);
-        const int half = C == 2 ? lane >> 5 : 0, row = C * wave + half;
+        const int column = C > 1 ? column_of(lane) : 0, row = C * wave + column;
         const unsigned char* const xs = lds + s.x;
-        const unsigned char* const ws = lds + s.region;
-        const int up = a.l_up, hidden = a.hidden;
+        const int hidden = a.hidden;
         const float eps = ph == PH_QKV ? a.norm_eps : a.post_eps;
         const bool at_end = ph == PH_DOWN && l == a.layers - 1;
         const float inv_k = 1.f / (float)s.k;
@@ -394,10 +373,9 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
         for (int i = 0; i < kRounds; ++i) bias[i] = 0.f;
         if (ph == PH_QKV && a.layer[l].qkv_bias) {
 #pragma unroll
-            for (int i = 0; i < kRounds; ++i) bias[i] = (float)reinterpret_cast<const __bf16*>(a.layer[l].qkv_bias)[s.c0 + min(row + 2 * kWavesWg * i, s.n - 1)];
+            for (int i = 0; i < kRounds; ++i) bias[i] = (float)reinterpret_cast<const __bf16*>(a.layer[l].qkv_bias)[s.c0 + min(row + C * kWavesWg * i, s.n - 1)];
         }
-        asm volatile("" ::"s"(s.c0), "s"(s.n), "s"(s.k), "s"(up), "s"(hidden), "s"(eps), "s"(to), "s"(width), "s"((int)at_end), "s"(inv_k));      // read in front of the wait
-        if (!ready) ask_weights(a, l, ph, role);
+        asm volatile("" ::"s"(s.c0), "s"(s.n), "s"(s.k), "s"(hidden), "s"(eps), "s"(to), "s"(width), "s"((int)at_end), "s"(inv_k));      // read in front of the wait
         if (ph == PH_QKV || (ph == PH_O && !have_x)) gather_input(a, tid, l, a.l_x[PH_QKV]);
         if (ph == PH_GATE_UP || (ph == PH_DOWN && !have_x)) gather_rows(tid, words + a.o_o, hidden, a.l_x[PH_GATE_UP]);
         if (ph == PH_DOWN) gather_rows(tid, words + a.o_act, s.k, s.x);
@@ -445,30 +423,58 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
                 };
                 if (used == 1) merge(0, std::integral_constant<int, 1>{});
                 else if (used == 2) merge(0, std::integral_constant<int, 2>{});
-                else if (used <= 4) merge(0, std::integral_constant<int, 4>{});
                 else
-                    for (int c0 = 0; c0 < used; c0 += 8) merge(c0, std::integral_constant<int, 8>{});
+                    for (int c0 = 0; c0 < used; c0 += 4) merge(c0, std::integral_constant<int, 4>{});
                 const float inv = mx == -INFINITY ? 0.f : fast_rcp(sum);         // (no tokens: zeros)
                 *reinterpret_cast<uint32_t*>(lds + s.x + 2 * (bh * D + 2 * d2)) = pack_bf16x2(o0 * inv, o1 * inv);
             }
         }
-        drain_loads();                                                           // this wave's part of the weights
         barrier_lds();
-        const bool late = __builtin_amdgcn_readfirstlane(say[flag]) != 0;
-        for (int i = 0; C * (wave + kWavesWg * i) < s.n; ++i) {
-            const int r0 = C * (wave + kWavesWg * i), r1 = min(r0 + 1, s.n - 1), r = r0 + half;
-            float acc[4][M], ss[M];
 #pragma unroll
-            for (int m = 0; m < M; ++m) acc[0][m] = acc[1][m] = acc[2][m] = acc[3][m] = ss[m] = 0.f;
-            const unsigned char* const rows[4] = {ws + r0 * 2 * s.k, ws + r1 * 2 * s.k, ws + up + r0 * 2 * s.k, ws + up + r1 * 2 * s.k};
-            dots(xs, s.k, rows, std::integral_constant<int, ph == PH_GATE_UP ? 4 : C>{}, std::integral_constant<int, ph == PH_DOWN ? (M == 1 ? 10 : 5) : 2>{}, std::bool_constant<norm>{}, acc, ss);
+        for (int i = 0; i < (ph == PH_QKV ? kRounds : 1); ++i) {
+            if (C * (wave + kWavesWg * i) >= s.n) continue;
+            const int r = C * (wave + kWavesWg * i) + column;
+            float acc[6][M], ss[M];
+#pragma unroll
+            for (int m = 0; m < M; ++m) acc[0][m] = acc[1][m] = acc[2][m] = acc[3][m] = acc[4][m] = acc[5][m] = ss[m] = 0.f;
+            constexpr int R = ph == PH_GATE_UP ? 6 : C, P = ph == PH_DOWN ? 10 : ph == PH_O ? 4 : 2, from = ph == PH_O || ph == PH_DOWN ? 12 : 0;
+            using std::integral_constant;
+            if constexpr (decltype(help)::value) {
+                const uint16_t* const w = reinterpret_cast<const uint16_t*>(ph == PH_QKV ? a.layer[l].qkv_w : ph == PH_O ? a.layer[l].o_w : ph == PH_GATE_UP ? a.layer[l].gate_up_w
+                                                                                                                                                          : a.layer[l].down_w) + (int64_t)s.c0 * s.k;
+                const int c = C * (wave + kWavesWg * i);
+                __amdgpu_buffer_rsrc_t rows[R];
+#pragma unroll
+                for (int q = 0; q < R; ++q) rows[q] = row_buffer(w + (q >= 3 ? (int64_t)a.inter * s.k : 0), c + q % 3, s.n, s.k, 0);
+#pragma unroll 1
+                for (int p = lane; p < (s.k >> 3) + lane; p += 64) {             // (the same sums in the same order, few registers)
+                    u32x4 wv[R];
+#pragma unroll
+                    for (int q = 0; q < R; ++q) wv[q] = __builtin_amdgcn_raw_buffer_load_b128(rows[q], 16 * p, 0, 0);
+#pragma unroll
+                    for (int m = 0; m < M; ++m) {
+                        u32x4 xv = *reinterpret_cast<const u32x4*>(xs + m * 2 * s.k + 16 * min(p, (s.k >> 3) - 1));
+                        if (p >= s.k >> 3) xv = u32x4{0, 0, 0, 0};
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            if constexpr (norm) ss[m] = dot2_bf16(xv[j], xv[j], ss[m]);
+#pragma unroll
+                            for (int q = 0; q < R; ++q) acc[q][m] = dot2_bf16(xv[j], wv[q][j], acc[q][m]);
+                        }
+                    }
+                }
+            } else if (i == 0) {
+                dots(xs, s.k, integral_constant<int, R>{}, integral_constant<int, P>{}, std::bool_constant<norm>{}, acc, ss, [&](int r, int p) { return held[from + r * P + p]; });
+            } else {
+                dots(xs, s.k, integral_constant<int, R>{}, integral_constant<int, P>{}, std::bool_constant<norm>{}, acc, ss, [&](int r, int p) { return held[6 + r * 2 + p]; });
+            }
 #pragma unroll
             for (int m = 0; m < M; ++m) {
-                float y = sum_two(acc[0][m], acc[C - 1][m]), u = 0.f;
-                if (ph == PH_GATE_UP) u = sum_two(acc[2][m], acc[3][m]);
-                float scale = 1.f;
-                if (norm) scale = rsqrtf(sum_two(ss[m], ss[m]) * inv_k + eps);
-                if ((C == 2 ? lane & 31 : lane) || r >= s.n) continue;
+                const float y = C > 1 ? sum_four(acc[0][m], acc[1][m], acc[2][m], 0.f) : sum_wave(acc[0][m]);
+                float u = 0.f, scale = 1.f;
+                if (ph == PH_GATE_UP) u = sum_four(acc[3][m], acc[4][m], acc[5][m], 0.f);
+                if (norm) scale = rsqrtf(sum_wave(ss[m]) * inv_k + eps);
+                if ((C > 1 ? lane & 15 : lane) || column >= C || r >= s.n) continue;
                 uint32_t v;
                 if (ph == PH_QKV) {
                     v = bf16_bits(y * scale + (i == 0 ? bias[0] : bias[1]));
@@ -482,6 +488,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
             }
         }
         barrier_lds();
+        const bool late = __builtin_amdgcn_readfirstlane(say[flag]) != 0;
         // one wave stores a row's results: words of a line that come from several waves are so many writes one behind the other at the memory side, with polls
         // between them (hop 2.8 us instead of 1.3)
         if (wave < M && lane < s.n && !late) {
@@ -497,7 +504,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
     };
 
     // ---- one share of the attention
-    auto attend = [&](int l, int role, bool ready) -> bool {
+    auto attend = [&](auto help, int l, int role) -> bool {
         Args& a = fresh_args();
         const int G = a.group, lane = lane_now(), tid = wave * 64 + lane, lq = lane & 15, lg = lane >> 4;
         Word* const words = layer_words(a, l);
@@ -513,10 +520,31 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
         unsigned char* const kv_wave = kv0 + wave * W::kWave;
         Word* const rec = uniform(words + a.o_rec + (int64_t)(ck.pair * a.chunks + ck.c) * G * (2 * (D + 2)));
         const float scale_log2 = a.scale_log2;
-        if (!ready) {                                                            // (another workgroup's share: the own tiles are found again behind it)
+        if constexpr (decltype(help)::value) {                                   // (another workgroup's share: the own tiles are found again behind it)
             find_tiles(a, role);
             ask_tiles(a, l, role);
         }
+        // addresses of the operands, found in front of the wait
+        constexpr int B = W::kBufs;
+        typedef const __attribute__((address_space(3))) bf16x8 LdsFrag;
+        const int dp = lane % LPT, dr = lane / LPT;
+        const int vq = lq >> 2, vp = lq & 3, vR = 4 * lg + vq;                   // lane 4q + p of its group addresses key row q, dims 4p..
+        uint32_t q_at = lds_offset(qs + min(lq, G - 1) * (2 * D + 16) + lg * 16), k_at[STEPS], v_at[DT], fin_at = lds_offset(kv_wave) + lq * 4 * D + 16 * lg;
+#pragma unroll
+        for (int st = 0; st < STEPS; ++st) {
+            k_at[st] = lds_offset(kv_wave) + lq * W::kRow + (((4 * st + lg) ^ chunk_swizzle<LPT>(lq)) * 16);
+            asm volatile("" : "+v"(k_at[st]));
+        }
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+            v_at[t] = lds_offset(kv_wave) + W::kImage + vR * W::kRow + (vp & 1) * 8 + ((2 * t + (vp >> 1)) ^ chunk_swizzle_v<LPT>(vR)) * 16;
+            asm volatile("" : "+v"(v_at[t]));
+        }
+        asm volatile("" : "+v"(q_at), "+v"(fin_at));
+        int mg = tid / (D / 2), md = tid % (D / 2);                              // what this thread merges first: head, pair of dims
+        uint32_t ml_at = lds_offset(ml) + 4 * mg, ow_at = lds_offset(kv0) + 8 * tid;
+        asm volatile("" : "+v"(ml_at), "+v"(ow_at), "+v"(mg), "+v"(md));
+        asm volatile("" ::"s"(rec), "s"(scale_log2), "s"(live_waves));
         drain_loads();                                                           // the first tiles (in front of the rows this share stores, whose acknowledgement nobody needs)
         // q heads of the group; k and v of every row (a row's earlier tokens may be rows of this batch): four dims of each half of a head to a thread
         const int items = (G + 2 * M) * LPT;
@@ -548,9 +576,11 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
             u32x4 v[2];
             const uint32_t o = 4u * (uint32_t)(m * a.nqkv + head * D + 4 * c8);
             const uint32_t off[2] = {o, o + 2 * D};
-            for (uint32_t spins = 0;;) {
+            bool there = false;
+            for (uint32_t spins = 0; !there;) {
                 load_through(v, src, off);
-                if ((marked(v[0], mark16) && marked(v[1], mark16)) || ran_out(spins)) break;
+                there = marked(v[0], mark16) && marked(v[1], mark16);
+                if (!there && ran_out(spins)) break;
             }
             float x1[4], x2[4];
 #pragma unroll
@@ -580,100 +610,114 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
             unsigned char* const dst = (is_q ? qs + hh * (2 * D + 16) : news + (2 * m + (is_v ? 1 : 0)) * 2 * D) + 8 * c8;
             *reinterpret_cast<u32x2*>(dst) = p1;
             *reinterpret_cast<u32x2*>(dst + D) = p2;
-            if (row) {
+            if (row && there) {
                 *reinterpret_cast<u32x2*>(row) = p1;
                 *reinterpret_cast<u32x2*>(row + D / 2) = p2;
             }
         }
         barrier_lds();
-        const bool late = __builtin_amdgcn_readfirstlane(say[flag]) != 0;
-        if (late) return true;
         if (wave < live_waves) {
             bf16x8 qf[STEPS];
 #pragma unroll
-            for (int st = 0; st < STEPS; ++st) qf[st] = *reinterpret_cast<const bf16x8*>(qs + min(lq, G - 1) * (2 * D + 16) + (4 * st + lg) * 16);
-            const int dp = lane % LPT, dr = lane / LPT;
+            for (int st = 0; st < STEPS; ++st) qf[st] = *(LdsFrag*)(q_at + 64 * st);
             float m_run = -INFINITY, l_run = 0.f;
             f32x4 o[DT];
 #pragma unroll
             for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            int buf = 0;
-            for (int tile = tile0; tile < ck.tiles; tile += tile_step) {
-                if (tile >= tile0 + W::kBufs * tile_step) drain_loads();
-                const int t0 = 16 * tile, n_live = ck.ctx - t0;
-                unsigned char* const lds_k = kv_wave + buf * W::kBuf;
-                unsigned char* const lds_v = lds_k + W::kImage;
-                int from = tile_from[0];
-                if (W::kBufs > 1 && tile == tile0 + tile_step) from = tile_from[W::kBufs - 1];
-                else if (tile != tile0) from = new_row(ck, tile, slot_of(a, ck, t0));
-                for (uint64_t hits = __builtin_amdgcn_ballot_w64(from >= 0 && lg == 0); hits; hits &= hits - 1) {
-                    const int T = __builtin_ctzll(hits), m = __builtin_amdgcn_readlane(from, T);
-                    const int which = lane / LPT, p = lane % LPT;
-                    if (which < 2) {
-                        const u32x4 v = *reinterpret_cast<const u32x4*>(news + (2 * m + which) * 2 * D + 16 * p);
-                        *reinterpret_cast<u32x4*>(which ? lds_v + T * W::kRow + (p ^ chunk_swizzle_v<LPT>(T)) * 16 : lds_k + T * W::kRow + (p ^ chunk_swizzle<LPT>(T)) * 16) = v;
+            auto tiles = [&](int tile, auto first_tag) {                         // the tiles of both buffers together
+                constexpr bool first = decltype(first_tag)::value;
+                f32x4 sT[B];
+                u32x2 vt[B][DT];
+#pragma unroll
+                for (int b = 0; b < B; ++b) {
+                    const int at = tile + b * tile_step, n_live = ck.ctx - 16 * at;
+                    sT[b] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+                    if (n_live <= 0) continue;                                   // (the same for the wave)
+                    unsigned char* const lds_k = kv_wave + b * W::kBuf;
+                    unsigned char* const lds_v = lds_k + W::kImage;
+                    const int from = first ? tile_from[b] : new_row(ck, at, slot_of(a, ck, 16 * at));
+                    for (uint64_t hits = __builtin_amdgcn_ballot_w64(from >= 0 && lg == 0); hits; hits &= hits - 1) {
+                        const int T = __builtin_ctzll(hits), m = __builtin_amdgcn_readlane(from, T);
+                        const int which = lane / LPT, p = lane % LPT;
+                        if (which < 2) {
+                            const u32x4 v = *reinterpret_cast<const u32x4*>(news + (2 * m + which) * 2 * D + 16 * p);
+                            *reinterpret_cast<u32x4*>(which ? lds_v + T * W::kRow + (p ^ chunk_swizzle_v<LPT>(T)) * 16 : lds_k + T * W::kRow + (p ^ chunk_swizzle<LPT>(T)) * 16) = v;
+                        }
+                    }
+                    if (n_live < 16) {                                           // rows past the context: P = 0 must not meet a value that is not finite
+#pragma unroll
+                        for (int i = 0; i < NI; ++i) {
+                            const int T = i * TPI + dr;
+                            if (T >= n_live) *reinterpret_cast<u32x4*>(lds_v + T * W::kRow + dp * 16) = u32x4{0, 0, 0, 0};
+                        }
+                    }
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    sT[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int st = 0; st < STEPS; ++st) {
+                        const bf16x8 kf = *(LdsFrag*)(k_at[st] + b * W::kBuf);
+                        sT[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[st], sT[b], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int t = 0; t < DT; ++t) vt[b][t] = ds_read_tr16_b64_asm(v_at[t] + b * W::kBuf);
+                    if (n_live < 16) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (4 * lg + r >= n_live) sT[b][r] = -INFINITY;
                     }
                 }
-                if (n_live < 16) {                                           // rows past the context: P = 0 must not meet a value that is not finite
-#pragma unroll
-                    for (int i = 0; i < NI; ++i) {
-                        const int T = i * TPI + dr;
-                        if (T >= n_live) *reinterpret_cast<u32x4*>(lds_v + T * W::kRow + dp * 16) = u32x4{0, 0, 0, 0};
-                    }
-                }
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                f32x4 sT = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int st = 0; st < STEPS; ++st) {
-                    const bf16x8 kf = *reinterpret_cast<const bf16x8*>(lds_k + lq * W::kRow + (((4 * st + lg) ^ chunk_swizzle<LPT>(lq)) * 16));
-                    sT = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[st], sT, 0, 0, 0);
-                }
-                const int vq = lq >> 2, vp = lq & 3, R = 4 * lg + vq;        // lane 4q + p of its group addresses key row q, dims 4p..
-                const uint32_t vrow = lds_offset(lds_v + R * W::kRow + (vp & 1) * 8);
-                const int swz = chunk_swizzle_v<LPT>(R);
-                u32x2 vt[DT];
-#pragma unroll
-                for (int t = 0; t < DT; ++t) vt[t] = ds_read_tr16_b64_asm(vrow + ((2 * t + (vp >> 1)) ^ swz) * 16);
-                if (n_live < 16) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (4 * lg + r >= n_live) sT[r] = -INFINITY;
-                }
-                asm volatile("s_nop 7\n\ts_nop 7" : "+v"(sT));               // the maxima below are asm statements: the compiler does not pad them behind the products
-                float mx = max2(max2(sT[0], sT[1]), max2(sT[2], sT[3]));
+                static_assert(B == 2, "");
+                asm volatile("s_nop 7\n\ts_nop 7" : "+v"(sT[0]), "+v"(sT[1]));   // the maxima below are asm statements: the compiler does not pad them behind the products
+                float mx = max2(max2(max2(sT[0][0], sT[0][1]), max2(sT[0][2], sT[0][3])), max2(max2(sT[1][0], sT[1][1]), max2(sT[1][2], sT[1][3])));
                 mx = max_xor16(mx);
                 mx = max_xor32(mx);
                 const float m_new = max2(m_run, mx * scale_log2), alpha = fast_exp2(m_run - m_new);
-                bf16x4 p_hi, p_lo;
+                bf16x4 p_hi[B], p_lo[B];
                 float lsum = 0.f;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float pv = fast_exp2(fmaf(sT[r], scale_log2, -m_new));
-                    lsum += pv;
-                    p_hi[r] = (__bf16)pv;
-                    p_lo[r] = (__bf16)(pv - (float)p_hi[r]);
-                }
+                for (int b = 0; b < B; ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float pv = fast_exp2(fmaf(sT[b][r], scale_log2, -m_new));
+                        lsum += pv;
+                        p_hi[b][r] = (__bf16)pv;
+                        p_lo[b][r] = (__bf16)(pv - (float)p_hi[b][r]);
+                    }
                 l_run = l_run * alpha + lsum;
                 m_run = m_new;
+                if (!first) {
 #pragma unroll
-                for (int t = 0; t < DT; ++t) o[t] = o[t] * alpha;
+                    for (int t = 0; t < DT; ++t) o[t] = o[t] * alpha;
+                }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 __builtin_amdgcn_sched_barrier(0);
                 typedef short s16x4 __attribute__((ext_vector_type(4)));
-                const s16x4 hi = __builtin_bit_cast(s16x4, p_hi), lo = __builtin_bit_cast(s16x4, p_lo);
 #pragma unroll
-                for (int t = 0; t < DT; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, vt[t]), hi, o[t], 0, 0, 0);
+                for (int b = 0; b < B; ++b) {
+                    if (ck.ctx <= 16 * (tile + b * tile_step)) continue;
 #pragma unroll
-                for (int t = 0; t < DT; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, vt[t]), lo, o[t], 0, 0, 0);
-                if (tile + W::kBufs * tile_step < ck.tiles) ask_tile(a, l, ck, tile + W::kBufs * tile_step, slot_of(a, ck, 16 * (tile + W::kBufs * tile_step)), buf);
-                buf = buf + 1 == W::kBufs ? 0 : buf + 1;
+                    for (int t = 0; t < DT; ++t)
+                        o[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, vt[b][t]), __builtin_bit_cast(s16x4, p_hi[b]), o[t], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < DT; ++t)
+                        o[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, vt[b][t]), __builtin_bit_cast(s16x4, p_lo[b]), o[t], 0, 0, 0);
+                }
+#pragma unroll
+                for (int b = 0; b < B; ++b) {
+                    const int next = tile + (B + b) * tile_step;
+                    if (next < ck.tiles) ask_tile(a, l, ck, next, slot_of(a, ck, 16 * next), b);
+                }
+            };
+            tiles(tile0, std::true_type{});
+            for (int tile = tile0 + B * tile_step; tile < ck.tiles; tile += B * tile_step) {
+                drain_loads();
+                tiles(tile, std::false_type{});
             }
             l_run = sum_xor16(l_run);
             l_run = sum_xor32(l_run);
             if (lq < G) {                                                    // over this wave's own images, all read by now
-                float* const fin = reinterpret_cast<float*>(kv_wave) + lq * D + 4 * lg;
 #pragma unroll
-                for (int t = 0; t < DT; ++t) *reinterpret_cast<f32x4*>(fin + 16 * t) = o[t];
+                for (int t = 0; t < DT; ++t) *(__attribute__((address_space(3))) f32x4*)(fin_at + 64 * t) = o[t];
                 if (lg == 0) {
                     ml[(wave * 2 + 0) * 16 + lq] = m_run;
                     ml[(wave * 2 + 1) * 16 + lq] = l_run;
@@ -681,16 +725,17 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
             }
         }
         barrier_lds();
-        for (int it = tid; it < G * D / 2; it += kThreads) {                 // two dims of a head to a thread
-            const int g = it / (D / 2), d2 = it % (D / 2);
+        const bool late = __builtin_amdgcn_readfirstlane(say[flag]) != 0;
+        for (int it = tid; it < G * D / 2; it += kThreads) {                     // two dims of a head to a thread
+            typedef const __attribute__((address_space(3))) float LdsFloat;
+            typedef const __attribute__((address_space(3))) f32x2 LdsPair;
             float mw[W::kWaves], lw[W::kWaves];
             f32x2 ow[W::kWaves];
 #pragma unroll
-            for (int w = 0; w < W::kWaves; ++w) {                            // (waves without tiles repeat the last one that has some, and do not count)
-                const int wc = min(w, max(live_waves - 1, 0));
-                mw[w] = ml[(wc * 2 + 0) * 16 + g];
-                lw[w] = ml[(wc * 2 + 1) * 16 + g];
-                ow[w] = reinterpret_cast<const f32x2*>(kv0 + wc * W::kWave)[it];
+            for (int w = 0; w < W::kWaves; ++w) {                                // (waves without tiles hold what they held: not counted)
+                mw[w] = w < live_waves ? *(LdsFloat*)(ml_at + 128 * w) : -INFINITY;
+                lw[w] = *(LdsFloat*)(ml_at + 128 * w + 64);
+                ow[w] = *(LdsPair*)(ow_at + w * W::kWave);
             }
             float mx = -INFINITY, sum = 0.f;
             f32x2 ov = {0.f, 0.f};
@@ -700,28 +745,35 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
                 for (int w = 1; w < W::kWaves; ++w) mx = fmaxf(mx, mw[w]);
 #pragma unroll
                 for (int w = 0; w < W::kWaves; ++w) {
-                    const float f = w < live_waves ? fast_exp2(mw[w] - mx) : 0.f;
-                    ov[0] = fmaf(ow[w][0], f, ov[0]);
-                    ov[1] = fmaf(ow[w][1], f, ov[1]);
-                    sum = fmaf(lw[w], f, sum);
+                    if (w < live_waves) {
+                        const float f = fast_exp2(mw[w] - mx);
+                        ov[0] = fmaf(ow[w][0], f, ov[0]);
+                        ov[1] = fmaf(ow[w][1], f, ov[1]);
+                        sum = fmaf(lw[w], f, sum);
+                    }
                 }
             }
-            Word* const p = rec + g * (2 * (D + 2));
-            st16_global_sc1((void*)(p + 4 * d2), u32x4{__float_as_uint(ov[0]), mark32, __float_as_uint(ov[1]), mark32});
-            if (d2 == 0) st16_global_sc1((void*)(p + 2 * D), u32x4{__float_as_uint(mx), mark32, __float_as_uint(sum), mark32});
+            if (!late) {
+                Word* const p = rec + mg * (2 * (D + 2));
+                st16_global_sc1((void*)(p + 4 * md), u32x4{__float_as_uint(ov[0]), mark32, __float_as_uint(ov[1]), mark32});
+                if (md == 0) st16_global_sc1((void*)(p + 2 * D), u32x4{__float_as_uint(mx), mark32, __float_as_uint(sum), mark32});
+            }
+            ml_at += 4 * (kThreads / (D / 2));
+            ow_at += 8 * kThreads;
+            mg += kThreads / (D / 2);
         }
-        return false;
+        return late;
     };
-    auto run = [&](int l, int ph, int role, bool ready) -> bool {
+    auto run = [&](auto help, int l, int ph, int role) -> bool {
         flag ^= 1;
         l = __builtin_amdgcn_readfirstlane(l);                                   // (what the compiler does not see: else it reads the layer's pointers by vector loads)
         role = __builtin_amdgcn_readfirstlane(role);
         switch (__builtin_amdgcn_readfirstlane(ph)) {
-            case PH_QKV: return project(std::integral_constant<int, PH_QKV>{}, l, role, ready);
-            case PH_ATTEND: return attend(l, role, ready);
-            case PH_O: return project(std::integral_constant<int, PH_O>{}, l, role, ready);
-            case PH_GATE_UP: return project(std::integral_constant<int, PH_GATE_UP>{}, l, role, ready);
-            default: return project(std::integral_constant<int, PH_DOWN>{}, l, role, ready);
+            case PH_QKV: return project(std::integral_constant<int, PH_QKV>{}, help, l, role);
+            case PH_ATTEND: return attend(help, l, role);
+            case PH_O: return project(std::integral_constant<int, PH_O>{}, help, l, role);
+            case PH_GATE_UP: return project(std::integral_constant<int, PH_GATE_UP>{}, help, l, role);
+            default: return project(std::integral_constant<int, PH_DOWN>{}, help, l, role);
         }
     };
 
@@ -760,31 +812,31 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
     int l = 0, ph = front ? PH_QKV : PH_GATE_UP, last = 0, rescues = 0;
     int help_t = -1, help_role = 0;                                              // phase (of all layers) and share to look at next, while helping
     bool lost = false;
-    if (front) find_tiles(fresh_args(), own);
-    ask_layer(0);
+    bool find = true, ask = true;                                                // the first tiles, and what the layer reads, are to be asked for (again)
     while (l < layers && !lost) {
-        int rl = l, rp = ph, rr = own;
         if (help_t >= 0) {
-            rl = help_t / kPhases;
-            rp = help_t - rl * kPhases;
+            const int rl = help_t / kPhases, rp = help_t - rl * kPhases;
             if (help_role >= (rp <= PH_O ? fresh_args().nf : fresh_args().nm)) {
                 help_role = 0;
                 if (++help_t < l * kPhases + ph) continue;
                 help_t = -1;                                                     // what this workgroup waited for is there
                 limit = min(fresh_args().spin_limit, 64u);
                 lost = ++rescues > 2 * kPhases * layers;
-                if (front) find_tiles(fresh_args(), own);
-                ask_layer(l);
+                find = ask = true;
                 continue;
             }
-            rr = help_role++;
-            if (complete(rl, rp, rr)) continue;
-        }
-        const bool out = run(rl, rp, rr, help_t < 0);
-        if (help_t >= 0) {
-            lost = out;                                                          // (the inputs of a share that is done here are complete)
+            const int role = help_role++;
+            if (complete(rl, rp, role)) continue;
+            lost = run(std::true_type{}, rl, rp, role);                          // (the inputs of a share that is done here are complete)
             __syncthreads();
-        } else if (out) {
+            continue;
+        }
+        if (ask) {
+            if (front && find) find_tiles(fresh_args(), own);
+            ask_layer(l);
+            find = ask = false;
+        }
+        if (run(std::false_type{}, l, ph, own)) {
             __syncthreads();                                                     // (waits for this wave's loads into LDS, too)
             if (threadIdx.x == 0) say[2] = say[3] = 0;
             __syncthreads();
@@ -792,15 +844,17 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
             limit = 1u << 20;
             help_t = last;
             help_role = 0;
+            continue;
+        }
+        last = l * kPhases + ph;
+        have_x = ph == PH_QKV || ph == PH_GATE_UP || (ph == PH_ATTEND && have_x);
+        if (ph == (front ? PH_O : PH_DOWN)) {
+            ph = front ? PH_QKV : PH_GATE_UP;
+            ++l;
+            barrier_lds();                                                       // the images of this layer have been read
+            ask = l < layers;
         } else {
-            last = l * kPhases + ph;
-            have_x = ph == PH_QKV || ph == PH_GATE_UP || (ph == PH_ATTEND && have_x);
-            const bool layer_done = ph == (front ? PH_O : PH_DOWN);
-            ph = layer_done ? (front ? PH_QKV : PH_GATE_UP) : ph + 1;
-            if (layer_done && ++l < layers) {
-                barrier_lds();                                                   // the weights of this layer have been read
-                ask_layer(l);
-            }
+            ++ph;
         }
     }
     drain_loads();
@@ -833,7 +887,7 @@ int launch_decode_layers(const DecodeLayersArgs& a, int hd, bool qk_norm, int ld
     auto rows = [&](auto d, auto norm) {
         constexpr int D = decltype(d)::value;
         constexpr bool N = decltype(norm)::value;
-        return a.m == 1 ? go(decode_layers_kernel<D, N, 1>) : go(decode_layers_kernel<D, N, 2>);
+        return a.m == 1 ? go(decode_layers_kernel<D, N, 1>) : a.m == 2 ? go(decode_layers_kernel<D, N, 2>) : go(decode_layers_kernel<D, N, 3>);
     };
     auto heads = [&](auto d) { return qk_norm ? rows(d, std::true_type{}) : rows(d, std::false_type{}); };
     return hd == 64 ? heads(std::integral_constant<int, 64>{}) : heads(std::integral_constant<int, 128>{});

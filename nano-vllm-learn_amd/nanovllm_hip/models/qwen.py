@@ -467,7 +467,7 @@ class QwenForCausalLM(nn.Module):
         return PackedResidual(residual, resid_p)
 
     def _forward_decode_layers(self, x, positions, ctx, b):
-        """The same step for a few sequences of a model whose layers fit the chip's LDS: all layers in one launch (csrc/decode_layers.hip)."""
+        """The same step for a few sequences of a model whose layers fit the chip's registers: all layers in one launch (csrc/decode_layers.hip)."""
         from .. import ops
         fw, cfg, a = self._folded_weights(), self.cfg, self.layers[0].self_attn
         layers = [dict(qkv_w=fw["qkv"][i], qkv_bias=l.self_attn.qkv_proj.bias, q_norm_w=l.self_attn.q_norm.weight if a.qk_norm else None,

@@ -567,7 +567,7 @@ def decode_layers_tokens(m, hidden, num_heads, num_kv_heads, head_dim, inter, la
 
 def decode_layers(x, layers, *, num_heads, num_kv_heads, head_dim, inter, norm_eps, post_eps, positions, cos_sin, slot_mapping, context_lens, block_tables, workspace,
                   qk_eps=1e-6, softmax_scale=None, out=None, out_packed=None, spin_limit=0, late_from=0, late_for=0):
-    """nvh_decode_layers: all layers of a decode step of one or two sequences in one launch (nanovllm/models/qwen3.py:179-193).
+    """nvh_decode_layers: all layers of a decode step of up to three sequences in one launch (nanovllm/models/qwen3.py:179-193).
 
     x [m, hidden]: the stream in front of the first layer; returns it behind the last one (`out`, never x), also in fragment order if out_packed is given.
     layers: a dict per layer of qkv_w (norm folded in), qkv_bias (or None), q_norm_w, k_norm_w (both or None), o_w, gate_up_w (norm folded in), down_w, k_cache, v_cache.

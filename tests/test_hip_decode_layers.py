@@ -90,7 +90,7 @@ SMALL, WIDE = (256, 4, 2, 64, 512), (384, 4, 4, 128, 640)
 
 
 @pytest.mark.parametrize("shape,norm", [(SMALL, False), (WIDE, True), ((264, 7, 1, 64, 1000), True), ((896, 14, 2, 64, 4864), False), ((1024, 16, 8, 128, 3072), True), ((512, 16, 1, 128, 256), False)])
-@pytest.mark.parametrize("contexts", [[1], [17], [256], [257], [700], [4500], [0], [300, 1], [1030, 2111], [0, 33]])
+@pytest.mark.parametrize("contexts", [[1], [17], [256], [257], [700], [4500], [0], [300, 1], [1030, 2111], [0, 33], [40, 300, 1], [600, 0, 1500]])
 def test_layers_against_64_bits(shape, norm, contexts):
     s = build(*shape, 3, norm, contexts)
     ws = scratch(s)
@@ -183,7 +183,7 @@ def test_replays():
 
 def test_refusals():
     from nanovllm_hip import ops
-    assert ops.decode_layers_workspace_bytes(3, 896, 14, 2, 64, 4864, 24) == 0
+    assert ops.decode_layers_workspace_bytes(4, 896, 14, 2, 64, 4864, 24) == 0
     assert ops.decode_layers_workspace_bytes(1, 3584, 28, 4, 128, 18944, 28) == 0           # 466 MB a layer
     assert ops.decode_layers_workspace_bytes(1, 896, 14, 2, 64, 4864, 33) == 0
     s = build(*SMALL, 1, False, [5])

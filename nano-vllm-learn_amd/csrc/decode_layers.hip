@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
         const int at = 16 * lane_now();
 #pragma unroll
         for (int i = 0; i < kHeld; ++i) {
-            held[i] = __builtin_amdgcn_raw_buffer_load_b128(row[i < 12 ? i >> 1 : i / 4 + 3], at, 1024 * (i < 12 ? i & 1 : i & 3), NVH_DMA_AUX);
+            held[i] = __builtin_amdgcn_raw_buffer_load_b128(row[i < 12 ? i >> 1 : i / 4 + 3], at + 1024 * (i < 12 ? i & 1 : i & 3), 0, NVH_DMA_AUX);       // (what the check of the end sees: not the scalar offset)
             if (front) loads_left<kFlightFront - 1>();
             else loads_left<kFlightRest - 1>();
         }

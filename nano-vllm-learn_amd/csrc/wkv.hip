@@ -31,11 +31,18 @@ constexpr float kMaxDecay = 100.f;                   // log2 units a channel may
 
 __device__ __forceinline__ float log2_decay(float z) { return -kLog2e * __expf(z); }
 
+// two numbers as bf16, the compiler not knowing what from: it would round the first one once more where its half is taken out again
+__device__ __forceinline__ uint32_t packed(float x, float y) {
+    uint32_t v = pack_bf16x2(x, y);
+    asm("" : "+v"(v));
+    return v;
+}
+
 __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
     u32x4 h, l;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        h[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
+        h[j] = packed(v[2 * j], v[2 * j + 1]);
         l[j] = pack_bf16x2(v[2 * j] - bf16_lo(h[j]), v[2 * j + 1] - bf16_hi(h[j]));
     }
     hi = *reinterpret_cast<const bf16x8*>(&h);
@@ -48,6 +55,67 @@ __device__ __forceinline__ int fresh(int v) {
     return v;
 }
 
+// The rows of a chunk, `n` of them from `base` on, of which a thread takes the bytes at `col` of row `row`.  Where offsets fit 32 bits the rows are a raw buffer whose end is the last row's:
+// the thread's first row's offset and an addition per load, where the row's clamp and product took 20 cycles; what lies behind reads as zero and is not stored.
+template <typename Off>
+struct ChunkRows {
+    __amdgpu_buffer_rsrc_t buf;
+    uint32_t row_bytes;
+    __device__ __forceinline__ ChunkRows(const void* base, int64_t bytes, int n, int width)
+        : buf(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)((n - 1) * (uint32_t)bytes + width), 0x00020000)), row_bytes((uint32_t)bytes) {}
+    __device__ __forceinline__ uint32_t first(int row, int col) const { return row * row_bytes + col; }
+    __device__ __forceinline__ uint32_t word(uint32_t at, int i, int, int) const { return __builtin_amdgcn_raw_buffer_load_b32(buf, (int)(at + i * row_bytes), 0, 0); }
+    __device__ __forceinline__ u32x4 four(uint32_t at, int i, int, int) const { return __builtin_amdgcn_raw_buffer_load_b128(buf, (int)(at + i * row_bytes), 0, 0); }
+    __device__ __forceinline__ void put(uint32_t at, int i, int, int, u32x4 v) const { __builtin_amdgcn_raw_buffer_store_b128(v, buf, (int)(at + i * row_bytes), 0, 0); }
+};
+// (rows further apart; behind the last row that row again)
+template <>
+struct ChunkRows<int64_t> {
+    unsigned char* base;
+    int64_t row_bytes;
+    int n;
+    __device__ __forceinline__ ChunkRows(const void* base, int64_t bytes, int n, int) : base(static_cast<unsigned char*>(const_cast<void*>(base))), row_bytes(bytes), n(n) {}
+    __device__ __forceinline__ uint32_t first(int, int) const { return 0; }
+    __device__ __forceinline__ unsigned char* in(int row, int col) const { return base + (int64_t)(row < n ? row : n - 1) * row_bytes + col; }
+    __device__ __forceinline__ uint32_t word(uint32_t, int i, int row, int col) const { return *reinterpret_cast<const uint32_t*>(in(fresh(row) + i, col)); }
+    __device__ __forceinline__ u32x4 four(uint32_t, int i, int row, int col) const { return *reinterpret_cast<const u32x4*>(in(fresh(row) + i, col)); }
+    __device__ __forceinline__ void put(uint32_t, int i, int row, int col, u32x4 v) const {
+        if (row + i < n) *reinterpret_cast<u32x4*>(in(row + i, col)) = v;
+    }
+};
+
+// d[i] summed over the 32 or 64 lanes of a token's channels, for eight tokens at once: every step adds half of one token's lanes to half of another's, so that each lane ends with one token
+template <int LANES>
+__device__ __forceinline__ float sums_of_eight(float (&d)[8]) {
+    float e[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) e[i] = LANES == 64 ? fold32(d[i], d[i + 4]) : fold16(d[i], d[i + 4]);
+    if constexpr (LANES == 64) {
+        float f[2] = {fold16(e[0], e[2]), fold16(e[1], e[3])};
+        asm("s_nop 1\n"
+            "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %0, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+            "s_nop 1"
+            : "+&v"(f[0]) : "v"(f[1]));
+        f[0] += dpp_f32<0x141>(f[0]);                // row_half_mirror
+        e[0] = f[0];
+    } else {
+        asm("s_nop 1\n"
+            "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+            "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n v_add_f32_dpp %1, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xc\n"
+            "s_nop 1\n"
+            "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0x5\n v_add_f32_dpp %0, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xa\n"
+            "s_nop 1"
+            : "+&v"(e[0]), "+&v"(e[1]) : "v"(e[2]), "v"(e[3]));
+    }
+    e[0] += dpp_f32<0xB1>(e[0]);                     // quad_perm [1,0,3,2]
+    return e[0] + dpp_f32<0x4E>(e[0]);               // quad_perm [2,3,0,1]
+}
+
+template <int LANES>
+__device__ __forceinline__ int which_of_eight(int lane) {    // the token whose sum this lane has
+    return LANES == 64 ? (lane >> 5) * 4 + (lane >> 4 & 1) * 2 + (lane >> 3 & 1) : (lane >> 4 & 1) * 4 + (lane >> 2 & 3);
+}
+
 template <int DIM>
 struct WkvLds {
     static constexpr int WAVES = DIM / 16, ROW = DIM * 2, IMG = C * ROW;
@@ -55,24 +123,28 @@ struct WkvLds {
     uint16_t p[2][C][PLD];                                                     // weights, hi | lo (token by token: outputs, [wave][16][16] fp32)
     float tot[8][DIM];                                                         // log decays by groups of 8 tokens
     float to_mid[DIM], to_end[DIM], mid_to_end[DIM];                           // what a channel decays by up to m, over the chunk, from m on
+    float w0[DIM], u[DIM];                                                     // (of the preparing waves' channels, whose registers are full)
     float bonus[C];
-    float red[WAVES][C];
+    float o[C][DIM + 4];                                                       // outputs on their way from a column of 16 tokens to rows
     int strong;
 };
 
 // DIM / 16 waves consume: wave w holds value columns 16 w .., state and outputs of this chunk.  As many prepare the next one: log decays and their sums, r~ and k~,
 // weights.  Three parts a chunk, one barrier behind each; the images are written when this chunk's consumers are done with them:
-//   consume: outputs, state, sums of squares | norm, gate, store          |
-//   prepare: log decays of chunk i + 1       | images, tables of i + 1    | weights of i + 1
-// What bounds it is issue and latency, not memory: a wave alone issues a vector instruction every 5.5 cycles, four together every 2.3 to 3.3, so two workgroups per CU
-// (heads of 64: 62 KB and 128 registers each) keep four waves on every SIMD; no register of theirs may be spilled inside the loop, a reload waits for every row in
-// flight.  (Heads of 128: 16 waves and 108 KB, one workgroup per CU; at 128 registers some are spilled.)
-// A chunk of a head of 64 takes 4.0 us alone and 7.8 beside a second one (6.8 and 13.9 with one kind of wave, 275 registers and one workgroup per CU); 11 portions of
-// 1090 tokens on average, 32 heads: 274 -> 153 us, 40 prompts of 410: 384 -> 166; heads of 128 about half the time.
-// Off: bytes from a chunk's first row.  32 bits where 64 rows fit them: a sequence of 1536 tokens takes 102.5 us against 106.1 in 64 bits, eight of them 122.5 against 128.
+//   consume: outputs, state               | norm, gate, store  | half of the weights of i + 1
+//   prepare: values of chunk i + 1        | images, tables     | log decays of chunk i + 2, the other half
+// (heads of 128, and rows far apart: | decays of i + 1 | values, images | weights |; the values' registers have no room there).
+// What bounds it is issue and latency, not memory: 780 vector instructions a chunk and SIMD, where there were 1240 (rows by a buffer descriptor instead of a clamp and a 64-bit product each,
+// masks only in a last chunk, eight tokens' sums at once, halves that are not rounded twice).  Two workgroups per CU (heads of 64: 79 KB and 128 registers each) keep four waves on every
+// SIMD; no register of theirs may be spilled inside the loop: a reload waits for every row in flight (four of them: 129 us where none takes 103).
+// Gates and results go by whole rows, through LDS: taken where the products leave them, 32 bytes of 16 rows a wave, they were 20 of 103 us.
+// Measured, 32 heads of 64, 11 portions of 1090 tokens in the mean, three sets of lengths: 126, 114, 132 -> 97, 83, 110 us; 19 of 500: 74 -> 57; three of 2950, in segments: 100 -> 82.
+// 16 heads of 128, 11 of 1090: 445 -> 398, 30 of 550: 405 -> 361 (some registers of 128 are spilled there).
+// Two sets of images, one workgroup a CU and two parts a chunk instead: 106, 109, 139.
 template <int DIM, bool SUMMARY, typename Off>
 __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(const WkvArgs a) {
     using Lds = WkvLds<DIM>;
+    constexpr bool AHEAD = DIM == 64 && sizeof(Off) == 4;                // (at 128 more than 128 registers)
     constexpr int ROW = DIM * 2, DT = DIM / 16, CP = DIM / 2, WAVES = Lds::WAVES, T = DIM * 4;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     Lds& lds = *reinterpret_cast<Lds*>(smem);
@@ -92,135 +164,203 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
         return;
     }
 
+    // weights D[key 16 jt + 4 lg + r][query 16 qg + lq]: the twelve 16 x 16 tiles the outputs read, dealt to all waves, first those that consume: four on
+    // the diagonal, then six below it, then the two above it, which are zero
+    auto weights = [&](auto prepares) __attribute__((always_inline)) {
+        if (SUMMARY) return;
+        constexpr bool P = decltype(prepares)::value;
+        const int lane_ = fresh(lane), lq = lane_ & 15, lg = lane_ >> 4;
+#pragma unroll
+        for (int x0 = P && AHEAD ? WAVES : 0; x0 < 12; x0 += AHEAD ? 2 * WAVES : WAVES) {
+            const int x = x0 + (P ? wave_id - WAVES : wave_id), y = x - 4;
+            if (x >= 12) break;
+            const int qg = x < 4 ? x : y < 6 ? (y > 2) + (y > 0) + 1 : 2 * (y - 6), jt = x < 4 ? x : y < 6 ? y - qg * (qg - 1) / 2 : qg + 1;
+            const int q0 = 16 * ROW * qg, k0 = 16 * ROW * jt;
+            f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int st = 0; st < DIM / 32; ++st) {
+                const int at = lq * ROW + ((4 * st + lg) ^ swz(lq)) * 16;  // (of 16 rows further on the same)
+                const bf16x8 qh = *reinterpret_cast<const bf16x8*>(lds.r_hi + q0 + at), ql = *reinterpret_cast<const bf16x8*>(lds.r_lo + q0 + at);
+                const bf16x8 kh = *reinterpret_cast<const bf16x8*>(lds.k_hi + k0 + at), kl = *reinterpret_cast<const bf16x8*>(lds.k_lo + k0 + at);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh, s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, ql, s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qh, s, 0, 0, 0);
+            }
+            float p[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) p[r] = s[r];
+            if (x0 == 0 && (WAVES == 4 || x < 4)) {
+                const float bonus = lds.bonus[16 * qg + lq];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p[r] = lq > 4 * lg + r ? s[r] : lq == 4 * lg + r ? bonus : 0.f;
+            } else if (x0 + WAVES > 10) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p[r] = x < 10 ? s[r] : 0.f;
+            }
+            const u32x2 hi = {packed(p[0], p[1]), packed(p[2], p[3])};
+            const u32x2 lo = {pack_bf16x2(p[0] - bf16_lo(hi[0]), p[1] - bf16_hi(hi[0])), pack_bf16x2(p[2] - bf16_lo(hi[1]), p[3] - bf16_hi(hi[1]))};
+            uint16_t* const to = &lds.p[0][lq][8 * lg] + (16 * PLD * qg + 32 * (jt >> 1) + 4 * (jt & 1));
+            *reinterpret_cast<u32x2*>(to) = hi;
+            *reinterpret_cast<u32x2*>(to + C * PLD) = lo;
+        }
+    };
     if (wave_id >= WAVES) {
         // ---- this thread's rows of a chunk: channels 2 cp, 2 cp + 1 of tokens 8 tg ..; two 16-byte pieces of values
         const int tid = threadIdx.x - T, wave = wave_id - WAVES, cp = tid % CP, tg = tid / CP;
         const int hc = head * DIM + 2 * cp;
-        const float w0a = a.w0[hc], w0b = a.w0[hc + 1];
-        float ua = 0.f, ub = 0.f;
-        if constexpr (!SUMMARY) {
-            ua = a.u[hc];
-            ub = a.u[hc + 1];
-        }
+        *reinterpret_cast<f32x2*>(&lds.w0[2 * cp]) = *reinterpret_cast<const f32x2*>(a.w0 + hc);
+        if constexpr (!SUMMARY) *reinterpret_cast<f32x2*>(&lds.u[2 * cp]) = *reinterpret_cast<const f32x2*>(a.u + hc);
         uint32_t rr[8], kk[8], zz[8];
         u32x4 vv[2];
-        // a chunk's rows, past the segment's end its last one.  Every chunk asks for as many rows as any other, in straight line: behind a branch around loads the
-        // compiler waits for all that are in flight instead of the ones it needs
-        const Off row_bytes = (Off)a.stride * 2, z_bytes = (Off)a.z_stride * 2;
+        // a chunk's rows.  Every chunk asks for as many rows as any other, in straight line: behind a branch around loads the compiler waits for all that are in flight
+        // instead of the ones it needs
         const int t_last = (n_rows - 1) / C * C;
         auto rows_of = [&](const void* p, int64_t stride, int t0) __attribute__((always_inline)) {
-            return reinterpret_cast<const unsigned char*>(p) + 2 * ((int64_t)(row0 + t0) * stride + head * DIM);
+            return ChunkRows<Off>(reinterpret_cast<const unsigned char*>(p) + 2 * ((int64_t)(row0 + t0) * stride + head * DIM), stride * 2, n_rows - t0 < C ? n_rows - t0 : C, ROW);
         };
+        const int v_row = tid / (DIM / 8), v_col = tid % (DIM / 8) * 16;
         auto fetch_z = [&](int t) __attribute__((always_inline)) {
-            const int t0 = t < t_last ? t : t_last, top = n_rows - t0 - 1, tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
-            const unsigned char* zb = rows_of(a.z, a.z_stride, t0);
+            const auto z = rows_of(a.z, a.z_stride, t < t_last ? t : t_last);
+            const uint32_t at = z.first(fresh(8 * tg), 4 * cp);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) zz[i] = *reinterpret_cast<const uint32_t*>(zb + ((Off)(8 * tg + i < top ? 8 * tg + i : top) * z_bytes + 4 * cp));
+            for (int i = 0; i < 8; ++i) zz[i] = z.word(at, i, 8 * tg, 4 * cp);
         };
         auto fetch = [&](int t) __attribute__((always_inline)) {
-            const int t0 = t < t_last ? t : t_last, top = n_rows - t0 - 1, tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
-            const unsigned char *kb = rows_of(a.k, a.stride, t0), *rb = rows_of(a.r, a.stride, t0), *vb = rows_of(a.v, a.stride, t0);
+            const int t0 = t < t_last ? t : t_last;
+            const auto k = rows_of(a.k, a.stride, t0), r = rows_of(a.r, a.stride, t0);
+            const uint32_t at = k.first(fresh(8 * tg), 4 * cp);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const Off at = (Off)(8 * tg + i < top ? 8 * tg + i : top) * row_bytes + 4 * cp;
-                kk[i] = *reinterpret_cast<const uint32_t*>(kb + at);
-                if constexpr (!SUMMARY) rr[i] = *reinterpret_cast<const uint32_t*>(rb + at);
+                kk[i] = k.word(at, i, 8 * tg, 4 * cp);
+                if constexpr (!SUMMARY) rr[i] = r.word(at, i, 8 * tg, 4 * cp);
             }
+        };
+        auto fetch_v = [&](int t) __attribute__((always_inline)) {
+            const auto v = rows_of(a.v, a.stride, t < t_last ? t : t_last);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int e = j * T + tid, r = e / (DIM / 8);
-                vv[j] = *reinterpret_cast<const u32x4*>(vb + ((Off)(r < top ? r : top) * row_bytes + e % (DIM / 8) * 16));
-            }
+            for (int j = 0; j < 2; ++j) vv[j] = v.four(v.first(fresh(v_row), v_col), j * (T * 8 / DIM), v_row, v_col);
         };
         float la[8], lb[8];                          // sums of log decays up to and with token i of the group
         auto decays = [&](int n) __attribute__((always_inline)) {
+            const f32x2 w0 = *reinterpret_cast<const f32x2*>(&lds.w0[2 * cp]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                la[i] = log2_decay(bf16_lo(zz[i]) + w0[0]);
+                lb[i] = log2_decay(bf16_hi(zz[i]) + w0[1]);
+            }
+            if (n < C) {
+                const int left = fresh(n - 8 * tg);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    la[i] = i < left ? la[i] : 0.f;
+                    lb[i] = i < left ? lb[i] : 0.f;
+                }
+            }
             float sa = 0.f, sb = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float da = log2_decay(bf16_lo(zz[i]) + w0a), db = log2_decay(bf16_hi(zz[i]) + w0b);
-                const bool ok = 8 * tg + i < n;
-                sa += ok ? da : 0.f;
-                sb += ok ? db : 0.f;
-                la[i] = sa;
-                lb[i] = sb;
+                la[i] = sa += la[i];
+                lb[i] = sb += lb[i];
             }
             *reinterpret_cast<f32x2*>(&lds.tot[tg][2 * cp]) = f32x2{sa, sb};
         };
-        float dec_a = 0.f, dec_b = 0.f;
+        float dec_a = 0.f, dec_b = 0.f, bonus = 0.f;
+        f32x2 mid, end;                              // sums of log decays up to m and over the chunk
         bool strong = false;
-        auto images = [&](int t0, int n) __attribute__((always_inline)) {
-            const int tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
-            if (n < C) {                             // keys and values past the end count nothing
+        uint32_t kh[8], kl[8], rh[8], rl[8];         // k~ and r~ as hi and lo halves; of a strong chunk k and r over kh and kl
+        auto values = [&](int n) __attribute__((always_inline)) {
+            if (n < C) {                             // keys past the end count nothing
+                const int left = fresh(n - 8 * tg);
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (8 * tg + i >= n) kk[i] = 0u;
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    if ((j * T + tid) / (DIM / 8) >= n) vv[j] = u32x4{0u, 0u, 0u, 0u};
+                for (int i = 0; i < 8; ++i) kk[i] = i < left ? kk[i] : 0u;
             }
             float oa = 0.f, ob = 0.f, ma = 0.f, mb = 0.f, fa = 0.f, fb = 0.f;
 #pragma unroll
             for (int g = 0; g < 8; ++g) {
                 const f32x2 s = *reinterpret_cast<const f32x2*>(&lds.tot[g][2 * cp]);
-                oa += g < tg ? s[0] : 0.f;
-                ob += g < tg ? s[1] : 0.f;
-                if (g < 4) {
-                    ma += s[0];
-                    mb += s[1];
-                }
+                oa = g == tg ? fa : oa;
+                ob = g == tg ? fb : ob;
                 fa += s[0];
                 fb += s[1];
+                if (g == 3) {
+                    ma = fa;
+                    mb = fb;
+                }
             }
             dec_a += fa;
             dec_b += fb;
             // (every wave holds all channels: they agree)
             strong = __builtin_amdgcn_ballot_w64(!(fminf(fminf(ma, fa - ma), fminf(mb, fb - mb)) >= -kMaxDecay)) != 0;
-            const int pofs = (cp & 3) * 4;
+            mid = f32x2{ma, mb};
+            end = f32x2{fa, fb};
+            if constexpr (!SUMMARY) {                // r . u k of the 8 tokens: over the lanes that hold a token's channels
+                const f32x2 u = *reinterpret_cast<const f32x2*>(&lds.u[2 * cp]);
+                const float ua = u[0], ub = u[1];
+                float d[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d[i] = bf16_lo(rr[i]) * ua * bf16_lo(kk[i]) + bf16_hi(rr[i]) * ub * bf16_hi(kk[i]);
+                bonus = sums_of_eight<CP>(d);
+            }
             if (!strong) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    const int t = 8 * tg + i, at = t * ROW + (((cp >> 2) ^ swz(t)) * 16) + pofs;
                     const float ia = oa + la[i], ib = ob + lb[i];
                     const float ka = bf16_lo(kk[i]) * fast_exp2(ma - ia), kb = bf16_hi(kk[i]) * fast_exp2(mb - ib);
-                    const uint32_t kh = pack_bf16x2(ka, kb);
-                    *reinterpret_cast<uint32_t*>(lds.k_hi + at) = kh;
-                    *reinterpret_cast<uint32_t*>(lds.k_lo + at) = pack_bf16x2(ka - bf16_lo(kh), kb - bf16_hi(kh));
+                    kh[i] = packed(ka, kb);
+                    kl[i] = pack_bf16x2(ka - bf16_lo(kh[i]), kb - bf16_hi(kh[i]));
                     if constexpr (!SUMMARY) {
                         const float ea = oa + (i ? la[i ? i - 1 : 0] : 0.f), eb = ob + (i ? lb[i ? i - 1 : 0] : 0.f);
                         const float ra = bf16_lo(rr[i]) * fast_exp2(ea - ma), rb = bf16_hi(rr[i]) * fast_exp2(eb - mb);
-                        const uint32_t rh = pack_bf16x2(ra, rb);
-                        *reinterpret_cast<uint32_t*>(lds.r_hi + at) = rh;
-                        *reinterpret_cast<uint32_t*>(lds.r_lo + at) = pack_bf16x2(ra - bf16_lo(rh), rb - bf16_hi(rh));
+                        rh[i] = packed(ra, rb);
+                        rl[i] = pack_bf16x2(ra - bf16_lo(rh[i]), rb - bf16_hi(rh[i]));
+                    }
+                    if (AHEAD && (i & 1)) __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    kh[i] = kk[i];
+                    if constexpr (!SUMMARY) kl[i] = rr[i];
+                }
+            }
+        };
+        auto images = [&](int t0, int n) __attribute__((always_inline)) {
+            const int tid = fresh(threadIdx.x - T), cp = tid % CP, tg = tid / CP;
+            if (n < C) {                             // values past the end count nothing
+                const int v_left = fresh(n - tid / (DIM / 8));
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) vv[j][q] = j * (T * 8 / DIM) < v_left ? vv[j][q] : 0u;
+            }
+            if (!strong) {
+                const int pofs = (cp & 3) * 4;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int t = 8 * tg + i, at = t * ROW + (((cp >> 2) ^ swz(t)) * 16) + pofs;
+                    *reinterpret_cast<uint32_t*>(lds.k_hi + at) = kh[i];
+                    *reinterpret_cast<uint32_t*>(lds.k_lo + at) = kl[i];
+                    if constexpr (!SUMMARY) {
+                        *reinterpret_cast<uint32_t*>(lds.r_hi + at) = rh[i];
+                        *reinterpret_cast<uint32_t*>(lds.r_lo + at) = rl[i];
                     }
                 }
             } else {
                 // (rare: z is read again, its registers hold the next chunk's)
                 float* w_f = reinterpret_cast<float*>(lds.r_hi);
-                const unsigned char* zb = rows_of(a.z, a.z_stride, t0);
+                const auto zs = rows_of(a.z, a.z_stride, t0);
 #pragma unroll 1
                 for (int i = 0; i < 8; ++i) {
                     const int t = 8 * tg + i;
-                    const uint32_t z = *reinterpret_cast<const uint32_t*>(zb + ((Off)(t < n ? t : n - 1) * z_bytes + 4 * cp));
+                    const uint32_t z = zs.word(zs.first(8 * tg, 4 * cp), i, 8 * tg, 4 * cp);
+                    const float w0a = lds.w0[2 * cp], w0b = lds.w0[2 * cp + 1];
                     *reinterpret_cast<f32x2*>(w_f + t * DIM + 2 * cp) = f32x2{fast_exp2(log2_decay(bf16_lo(z) + w0a)), fast_exp2(log2_decay(bf16_hi(z) + w0b))};
                 }
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const int t = 8 * tg + i;
-                    *reinterpret_cast<uint32_t*>(lds.k_hi + t * ROW + 4 * cp) = kk[i];
-                    if constexpr (!SUMMARY) *reinterpret_cast<uint32_t*>(lds.k_lo + t * ROW + 4 * cp) = rr[i];
-                }
-            }
-            if constexpr (!SUMMARY) {                // r . u k of the 8 tokens: over the lanes that hold a token's channels
-                float d[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    d[i] = bf16_lo(rr[i]) * ua * bf16_lo(kk[i]) + bf16_hi(rr[i]) * ub * bf16_hi(kk[i]);
-                    d[i] = sum_xor16(group_sum<16>(d[i]));
-                    if constexpr (CP == 64) d[i] = sum_xor32(d[i]);
-                }
-                if (cp == 0) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) lds.bonus[8 * tg + i] = d[i];
+                    *reinterpret_cast<uint32_t*>(lds.k_hi + t * ROW + 4 * cp) = kh[i];
+                    if constexpr (!SUMMARY) *reinterpret_cast<uint32_t*>(lds.k_lo + t * ROW + 4 * cp) = kl[i];
                 }
             }
 #pragma unroll
@@ -228,58 +368,45 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
                 const int e = j * T + tid, t = e / (DIM / 8), pc = e % (DIM / 8);
                 *reinterpret_cast<u32x4*>(lds.v + t * ROW + (pc ^ swz(t)) * 16) = vv[j];
             }
+            if constexpr (!SUMMARY) lds.bonus[8 * tg + which_of_eight<CP>(tid & 63)] = bonus;      // (all lanes of a token hold it)
             if (tg == 0) {
-                *reinterpret_cast<f32x2*>(&lds.to_mid[2 * cp]) = f32x2{fast_exp2(ma), fast_exp2(mb)};
-                *reinterpret_cast<f32x2*>(&lds.to_end[2 * cp]) = f32x2{fast_exp2(fa), fast_exp2(fb)};
-                *reinterpret_cast<f32x2*>(&lds.mid_to_end[2 * cp]) = f32x2{fast_exp2(fa - ma), fast_exp2(fb - mb)};
+                *reinterpret_cast<f32x2*>(&lds.to_mid[2 * cp]) = f32x2{fast_exp2(mid[0]), fast_exp2(mid[1])};
+                *reinterpret_cast<f32x2*>(&lds.to_end[2 * cp]) = f32x2{fast_exp2(end[0]), fast_exp2(end[1])};
+                *reinterpret_cast<f32x2*>(&lds.mid_to_end[2 * cp]) = f32x2{fast_exp2(end[0] - mid[0]), fast_exp2(end[1] - mid[1])};
                 if (cp == 0) lds.strong = strong;
             }
         };
-        // weights D[key 16 jt + 4 lg + r][query 16 qg + lq]: the twelve 16 x 16 tiles the outputs read, dealt to the waves
-        auto weights = [&]() __attribute__((always_inline)) {
-            if (SUMMARY || strong) return;
-            const int lane_ = fresh(lane), lq = lane_ & 15, lg = lane_ >> 4;
-#pragma unroll
-            for (int x0 = 0; x0 < 12; x0 += WAVES) {
-                const int x = x0 + wave;
-                if (x >= 12) break;
-                const int qg = x < 4 ? x >> 1 : 2 + ((x - 4) >> 2), jt = x < 4 ? x & 1 : (x - 4) & 3, Rq = 16 * qg + lq, Rk = 16 * jt + lq;
-                f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int st = 0; st < DIM / 32; ++st) {
-                    const int qat = Rq * ROW + ((4 * st + lg) ^ swz(Rq)) * 16, kat = Rk * ROW + ((4 * st + lg) ^ swz(Rk)) * 16;
-                    const bf16x8 qh = *reinterpret_cast<const bf16x8*>(lds.r_hi + qat), ql = *reinterpret_cast<const bf16x8*>(lds.r_lo + qat);
-                    const bf16x8 kh = *reinterpret_cast<const bf16x8*>(lds.k_hi + kat), kl = *reinterpret_cast<const bf16x8*>(lds.k_lo + kat);
-                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh, s, 0, 0, 0);
-                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, ql, s, 0, 0, 0);
-                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qh, s, 0, 0, 0);
-                }
-                const float bonus = lds.bonus[Rq];
-                float p[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int back = Rq - (16 * jt + 4 * lg + r);
-                    p[r] = back > 0 ? s[r] : back == 0 ? bonus : 0.f;
-                }
-                const u32x2 hi = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
-                const u32x2 lo = {pack_bf16x2(p[0] - bf16_lo(hi[0]), p[1] - bf16_hi(hi[0])), pack_bf16x2(p[2] - bf16_lo(hi[1]), p[3] - bf16_hi(hi[1]))};
-                const int at = 32 * (jt >> 1) + 8 * lg + 4 * (jt & 1);
-                *reinterpret_cast<u32x2*>(&lds.p[0][Rq][at]) = hi;
-                *reinterpret_cast<u32x2*>(&lds.p[1][Rq][at]) = lo;
-            }
-        };
+        auto rows = [&](int t0) { return n_rows - t0 < C ? n_rows - t0 : C; };
         fetch_z(0);
         fetch(0);
-        auto rows = [&](int t0) { return n_rows - t0 < C ? n_rows - t0 : C; };
+        fetch_v(0);
+        if constexpr (AHEAD) {
+            decays(rows(0));
+            fetch_z(C);
+        }
+        lds_only_barrier();
         for (int t0 = 0; t0 < n_rows + C; t0 += C) {         // prepares the chunk at t0 while the one in front of it is consumed
             const bool there = t0 < n_rows;
-            if (there) decays(rows(t0));
-            fetch_z(t0 + C);
+            if constexpr (AHEAD) {
+                if (there) values(rows(t0));
+                fetch(t0 + C);
+            } else {
+                if (there) decays(rows(t0));
+                fetch_z(t0 + C);
+            }
             lds_only_barrier();
+            if constexpr (!AHEAD) {
+                if (there) values(rows(t0));
+            }
             if (there) images(t0, rows(t0));
-            fetch(t0 + C);
+            if constexpr (!AHEAD) fetch(t0 + C);
+            fetch_v(t0 + C);
             lds_only_barrier();
-            if (there) weights();
+            if constexpr (AHEAD) {
+                if (t0 + C < n_rows) decays(rows(t0 + C));
+                fetch_z(t0 + 2 * C);
+            }
+            if (there && !strong) weights(std::true_type{});
             lds_only_barrier();
         }
         if constexpr (SUMMARY) {
@@ -303,25 +430,36 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
             for (int t = 0; t < DT; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) S[t][r] = src[(16 * t + 4 * lg + r) * DIM + sv];
+#pragma unroll
+            for (int t = 0; t < DT; ++t) asm volatile("" : "+v"(S[t]));        // (waited for here, not in the loop)
         }
     }
-    f32x4 nw = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (!SUMMARY) nw = *reinterpret_cast<const f32x4*>(a.norm + head * DIM + 16 * wave + 4 * lg);
+    // this thread's pieces of a chunk's gates and results, 8 columns each: token row + 32 j
+    const int row = threadIdx.x / (DIM / 8), col = threadIdx.x % (DIM / 8) * 8;
+    f32x8 nw = {};
+    if constexpr (!SUMMARY) nw = act_ld8(a.norm + head * DIM + col);
     const float inv_n = 1.f / a.n;
-    u32x2 gate[4];                                   // gates of four tokens, 4 columns
-    const Off g_bytes = (Off)a.stride * 2, out_bytes = (Off)a.out_stride * 2;
+    u32x4 gate[2];
+    auto rows_of = [&](const void* p, int64_t stride, int t0) __attribute__((always_inline)) {
+        return ChunkRows<Off>(reinterpret_cast<const unsigned char*>(p) + 2 * ((int64_t)(row0 + t0) * stride + head * DIM), stride * 2, n_rows - t0 < C ? n_rows - t0 : C, ROW);
+    };
     auto fetch_gate = [&](int t0) __attribute__((always_inline)) {
         if constexpr (!SUMMARY) {
-            const unsigned char* gb = reinterpret_cast<const unsigned char*>(a.g) + 2 * ((int64_t)(row0 + t0) * a.stride + head * DIM);
-            const int top = n_rows - t0 - 1, lane_ = fresh(lane), lq = lane_ & 15, col_bytes = 2 * (16 * wave + 4 * (lane_ >> 4));
+            const auto g = rows_of(a.g, a.stride, t0);
 #pragma unroll
-            for (int it = 0; it < 4; ++it) gate[it] = *reinterpret_cast<const u32x2*>(gb + ((Off)(16 * it + lq < top ? 16 * it + lq : top) * g_bytes + col_bytes));
+            for (int j = 0; j < 2; ++j) gate[j] = g.four(g.first(row, 2 * col), 32 * j, row, 2 * col);
         }
     };
-    const int tr = 4 * lg + (lq >> 2), tp = lq & 3;  // transposed reads: row and column quarter this lane addresses
+    // transposed reads of columns 16 t ..: row and column quarter this lane addresses (of 16 rows further on the same)
+    auto tr_at = [&](int t) __attribute__((always_inline)) {
+        const int lane_ = DIM == 64 ? lane : fresh(lane), tr = lane_ >> 2, tp = lane_ & 3;
+        return tr * ROW + ((2 * t + (tp >> 1)) ^ swz(tr)) * 16 + (tp & 1) * 8;
+    };
     fetch_gate(0);
-    lds_only_barrier();
-    lds_only_barrier();
+    lds_only_barrier();                              // the first chunk's decays,
+    lds_only_barrier();                              // values,
+    lds_only_barrier();                              // images
+    if (AHEAD && !__builtin_amdgcn_readfirstlane(lds.strong)) weights(std::false_type{});
     lds_only_barrier();
     for (int t0 = 0; t0 < n_rows; t0 += C) {
         const int n = n_rows - t0 < C ? n_rows - t0 : C;
@@ -331,8 +469,8 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
             bf16x8 vf[2];
 #pragma unroll
             for (int hh = 0; hh < 2; ++hh) {
-                const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * wave + (tp >> 1);
-                const u32x2 lo = lds_tr16(lds.v + ra * ROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8), hi = lds_tr16(lds.v + rb * ROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8);
+                const unsigned char* const at = lds.v + tr_at(wave) + 32 * ROW * hh;
+                const u32x2 lo = lds_tr16(at), hi = lds_tr16(at + 16 * ROW);
                 const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
                 vf[hh] = *reinterpret_cast<const bf16x8*>(&raw);
             }
@@ -351,11 +489,16 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
                     }
                     bf16x8 hi, lo;
                     split8(sc, hi, lo);
+                    const int lane_ = AHEAD ? lane : fresh(lane), lq = lane_ & 15, lg = lane_ >> 4;
+                    const int pa = lq * ROW + ((4 * st + (lg >> 1)) ^ swz(lq)) * 16 + (lg & 1) * 8, pb = lq * ROW + ((4 * st + 2 + (lg >> 1)) ^ swz(lq)) * 16 + (lg & 1) * 8;
 #pragma unroll
                     for (int it = 0; it < 4; ++it) {
-                        const int R = 16 * it + lq, pa = ((4 * st + (lg >> 1)) ^ swz(R)) * 16 + (lg & 1) * 8, pb = ((4 * st + 2 + (lg >> 1)) ^ swz(R)) * 16 + (lg & 1) * 8;
-                        const u32x2 ha = *reinterpret_cast<const u32x2*>(lds.r_hi + R * ROW + pa), hb = *reinterpret_cast<const u32x2*>(lds.r_hi + R * ROW + pb);
-                        const u32x2 xa = *reinterpret_cast<const u32x2*>(lds.r_lo + R * ROW + pa), xb = *reinterpret_cast<const u32x2*>(lds.r_lo + R * ROW + pb);
+                        const int R = 16 * ROW * it;
+                        // (kept apart, or two rows' or both images' reads become one, whose halves have to be moved)
+                        const u32x2 ha = *reinterpret_cast<const u32x2*>(lds.r_hi + R + pa), hb = *reinterpret_cast<const u32x2*>(lds.r_hi + R + pb);
+                        if constexpr (AHEAD) asm volatile("" ::: "memory");
+                        const u32x2 xa = *reinterpret_cast<const u32x2*>(lds.r_lo + R + pa), xb = *reinterpret_cast<const u32x2*>(lds.r_lo + R + pb);
+                        if constexpr (AHEAD) asm volatile("" ::: "memory");
                         const u32x4 hraw = {ha[0], ha[1], hb[0], hb[1]}, lraw = {xa[0], xa[1], xb[0], xb[1]};
                         const bf16x8 qh = *reinterpret_cast<const bf16x8*>(&hraw), ql = *reinterpret_cast<const bf16x8*>(&lraw);
                         o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, qh, o[it], 0, 0, 0);
@@ -374,15 +517,14 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
             // ---- the state behind these tokens
 #pragma unroll
             for (int t = 0; t < DT; ++t) {
+                const int k_at = tr_at(t);
                 f32x4 M = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int hh = 0; hh < 2; ++hh) {
-                    const int ra = 32 * hh + tr, rb = ra + 16, pc = 2 * t + (tp >> 1);
-                    const int pa = ra * ROW + (pc ^ swz(ra)) * 16 + (tp & 1) * 8, pb = rb * ROW + (pc ^ swz(rb)) * 16 + (tp & 1) * 8;
 #pragma unroll
                     for (int q = 0; q < 2; ++q) {
-                        const unsigned char* img = q ? lds.k_lo : lds.k_hi;
-                        const u32x2 ka = lds_tr16(img + pa), kb = lds_tr16(img + pb);
+                        const unsigned char* const at = (q ? lds.k_lo : lds.k_hi) + k_at + 32 * ROW * hh;
+                        const u32x2 ka = lds_tr16(at), kb = lds_tr16(at + 16 * ROW);
                         const u32x4 kraw = {ka[0], ka[1], kb[0], kb[1]};
                         M = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&kraw), vf[hh], M, 0, 0, 0);
                     }
@@ -425,33 +567,29 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
         }
         if constexpr (!SUMMARY) {
 #pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                float ss = sum4(o[it] * o[it]);
-                ss = sum_xor16(ss);
-                ss = sum_xor32(ss);
-                if (lg == 0) lds.red[wave][16 * it + lq] = ss;
-            }
+            for (int it = 0; it < 4; ++it) *reinterpret_cast<f32x4*>(&lds.o[16 * it + lq][16 * wave + 4 * lg]) = o[it];
         }
-        lds_only_barrier();                          // this chunk's images may be replaced; sums of squares are there
+        lds_only_barrier();                          // this chunk's images may be replaced; outputs are there
         if constexpr (!SUMMARY) {
             // ---- norm over the head's columns, gate
-            const int lane_ = fresh(lane), lq = lane_ & 15, lg = lane_ >> 4, col_bytes = 2 * (16 * wave + 4 * lg);
-            unsigned char* out = reinterpret_cast<unsigned char*>(a.out) + 2 * ((int64_t)(row0 + t0) * a.out_stride + head * DIM) + col_bytes;
+            const auto out = rows_of(a.out, a.out_stride, t0);
 #pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                float ss = 0.f;
+            for (int j = 0; j < 2; ++j) {
+                const f32x8 y = act_ld8(&lds.o[row + 32 * j][col]), g = unpack8(gate[j]);
+                const float inv = __builtin_amdgcn_rsqf(group_sum<DIM / 8>(sum4(y.a * y.a) + sum4(y.b * y.b)) * inv_n + a.eps);
+                f32x8 r;
 #pragma unroll
-                for (int w = 0; w < WAVES; ++w) ss += lds.red[w][16 * it + lq];
-                const float inv = __builtin_amdgcn_rsqf(ss * inv_n + a.eps);
-                const float g[4] = {bf16_lo(gate[it][0]), bf16_hi(gate[it][0]), bf16_lo(gate[it][1]), bf16_hi(gate[it][1])};
-                f32x4 r;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) r[k] = o[it][k] * inv * nw[k] * (g[k] * fast_rcp(1.f + fast_exp2(-kLog2e * g[k])));
-                if (16 * it + lq < n) act_st4(reinterpret_cast<uint16_t*>(out + (Off)(16 * it + lq) * out_bytes), r);
+                for (int k = 0; k < 4; ++k) {
+                    r.a[k] = y.a[k] * inv * nw.a[k] * (g.a[k] * fast_rcp(1.f + fast_exp2(-kLog2e * g.a[k])));
+                    r.b[k] = y.b[k] * inv * nw.b[k] * (g.b[k] * fast_rcp(1.f + fast_exp2(-kLog2e * g.b[k])));
+                }
+                out.put(out.first(row, 2 * col), 32 * j, row, 2 * col,
+                        u32x4{pack_bf16x2(r.a[0], r.a[1]), pack_bf16x2(r.a[2], r.a[3]), pack_bf16x2(r.b[0], r.b[1]), pack_bf16x2(r.b[2], r.b[3])});
             }
             fetch_gate(t0 + C < n_rows ? t0 + C : t0);
         }
-        lds_only_barrier();
+        lds_only_barrier();                          // the next chunk's images
+        if (AHEAD && t0 + C < n_rows && !__builtin_amdgcn_readfirstlane(lds.strong)) weights(std::false_type{});
         lds_only_barrier();
     }
     float* dst = nullptr;

@@ -431,6 +431,27 @@ def test_wkv_rows_far_apart(heads, dim, decay, stride):
         assert (far[:, 6 * cols:] == 7).all() and all(torch.equal(far[:, i * cols:(i + 1) * cols], t) for i, t in enumerate(near))
 
 
+@pytest.mark.parametrize("rows", [1, 31, 32, 33, 63, 64, 65, 129])
+@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 128)])
+def test_wkv_rows_of_others(heads, dim, rows):
+    """A portion among rows that are not its own: what lies behind its last one is neither read (NaN) nor written, with result rows 8 bytes off a multiple of 16."""
+    cols, first = heads * dim, 3
+    layer = Wkv([rows], heads, dim, dim, BF16)
+    mine = [layer.rows(w, [(0, 0, rows, 0)]) for w in ("r", "k", "v", "g", "z")]
+    wide = torch.full((rows + 70, 5 * cols), float("nan"), dtype=BF16, device="cuda")
+    wide[first:first + rows] = torch.cat(mine, dim=1)
+    out = torch.full((rows + 70, cols + 4), 7.0, dtype=BF16, device="cuda")
+    state = torch.full((1, heads, dim, dim), 30.0).cuda()
+    pos, slots = torch.arange(rows + 70).cuda() - first, torch.zeros(1, dtype=torch.int32, device="cuda")
+    ops().wkv_chunks(*(wide[:, i * cols:(i + 1) * cols] for i in range(5)), layer.params, layer.eps, dim, pos, slots,
+                     torch.tensor([(first, rows, 0, 0)], dtype=torch.int32).cuda(), False, state, out=out[:, :cols])
+    o, s = layer.want[0]
+    close(out[first:first + rows, :cols].view(rows, heads, dim), o, BF16, slack=2)
+    close(state[0], s, F32, slack=64)
+    out[first:first + rows, :cols] = 7.0
+    assert (out == 7).all()
+
+
 @pytest.mark.parametrize("heads,dim,dtype,generic", [(3, 64, BF16, False), (2, 128, BF16, False), (2, 64, BF16, True), (2, 24, F32, True)])
 @pytest.mark.parametrize("decay", ["usual", "strong"])
 def test_wkv_segments_without_rows(heads, dim, dtype, generic, decay):

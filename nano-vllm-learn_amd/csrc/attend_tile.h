@@ -181,7 +181,7 @@ __device__ __forceinline__ void attend_walk(unsigned char* lds, int n_tiles, flo
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const float p0 = sT[qs][2 * hh + (j >> 1)][2 * (j & 1)], p1 = sT[qs][2 * hh + (j >> 1)][2 * (j & 1) + 1];
-                        hraw[j] = pack_bf16x2(p0, p1);
+                        hraw[j] = pack_bf16x2_once(p0, p1);
                         lraw[j] = pack_bf16x2(p0 - bf16_lo(hraw[j]), p1 - bf16_hi(hraw[j]));
                     }
                     p_hi[qs] = *reinterpret_cast<const bf16x8*>(&hraw);
@@ -370,7 +370,7 @@ __device__ __forceinline__ void attend_walk32(unsigned char* lds, int n_tiles, f
                     if constexpr (F16) {
                         hi[i][j] = pack_f16x2(p0, p1);
                     } else {
-                        hi[i][j] = pack_bf16x2(p0, p1);
+                        hi[i][j] = pack_bf16x2_once(p0, p1);
                         lo[i][j] = pack_bf16x2(p0 - bf16_lo(hi[i][j]), p1 - bf16_hi(hi[i][j]));
                     }
                 }

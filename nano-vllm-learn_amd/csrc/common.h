@@ -29,6 +29,13 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     return *reinterpret_cast<uint32_t*>(&r);
 }
 
+// the same, the compiler not knowing what from: where the halves are taken out again (hi and lo parts) it would round the first number once more instead of shifting the word
+__device__ __forceinline__ uint32_t pack_bf16x2_once(float lo, float hi) {
+    uint32_t v = pack_bf16x2(lo, hi);
+    asm("" : "+v"(v));
+    return v;
+}
+
 // acc + a.lo*b.lo + a.hi*b.hi with bf16 operands packed two per dword (v_dot2c_f32_bf16)
 __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float acc) {
     return __builtin_amdgcn_fdot2_f32_bf16(*reinterpret_cast<bf16x2_t*>(&a), *reinterpret_cast<bf16x2_t*>(&b), acc, false);

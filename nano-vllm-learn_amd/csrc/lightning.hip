@@ -23,7 +23,7 @@ __device__ __forceinline__ void split_hi_lo(const float (&v)[8], bf16x8& hi, bf1
     u32x4 h, l;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        h[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
+        h[j] = pack_bf16x2_once(v[2 * j], v[2 * j + 1]);
         l[j] = pack_bf16x2(v[2 * j] - bf16_lo(h[j]), v[2 * j + 1] - bf16_hi(h[j]));
     }
     hi = *reinterpret_cast<const bf16x8*>(&h);
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
                     const int back = Rq - (16 * jt + 4 * lg + r);
                     p[r] = back >= 0 ? s[jt][r] * pw[back >= 0 ? back : 0] : 0.f;
                 }
-                const u32x2 hi = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+                const u32x2 hi = {pack_bf16x2_once(p[0], p[1]), pack_bf16x2_once(p[2], p[3])};
                 const u32x2 lo = {pack_bf16x2(p[0] - bf16_lo(hi[0]), p[1] - bf16_hi(hi[0])), pack_bf16x2(p[2] - bf16_lo(hi[1]), p[3] - bf16_hi(hi[1]))};
                 const int at = Rq * PLD + 32 * (jt >> 1) + 8 * lg + 4 * (jt & 1);
                 *reinterpret_cast<u32x2*>(p_lds + at) = hi;
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
 // ahead by hand (121).
 template <int DK, int CW>
 constexpr size_t pair_lds_bytes(bool summary) {
-    return (size_t)2 * C * (DK * (summary ? 1 : 2) + 16 * CW) * 2 + (summary ? 0 : (size_t)2 * C * PLD * 2);
+    return (size_t)2 * C * (DK * (summary ? 1 : 2) + 16 * CW) * 2 + (summary ? 0 : (size_t)2 * C * PLD * 2 + (size_t)C * (16 * CW + 8) * 2);
 }
 
 // Whole portions that nothing comes in front of: the longest of them as two pieces of the same length in time.  The second one follows the state over the first one's tokens (keys and
@@ -367,6 +367,8 @@ __global__ __launch_bounds__(64 * (CW + PW), DK == 64 && CW == 4 ? 4 : 1) void l
     unsigned char* vimg0 = kimg0 + 2 * KIMG;                                   // [2][C][VW] values
     unsigned char* qimg0 = vimg0 + 2 * VIMG;                                   // [2][C][DK] queries
     uint16_t* p_lds = reinterpret_cast<uint16_t*>(qimg0 + 2 * KIMG);           // [hi | lo][C][PLD] weights
+    constexpr int OLD = VW + 8;
+    uint16_t* o_lds = p_lds + 2 * C * PLD;                                     // [C][OLD] outputs, on their way from columns of 16 tokens to rows
     __shared__ __attribute__((aligned(16))) float pw[C + 1], fall_s[C];        // decay^0 .. decay^C; decay^(C - 1 - key)
     auto swz = [](int r) { return KROW == 128 ? (r >> 1) & 7 : r & 15; };      // rows of 256 bytes span all banks: 16 of them apart, not 8
     auto swzv = [](int r) { return VROW == 128 ? (r >> 1) & 7 : (2 * r) & 14; };
@@ -539,7 +541,7 @@ __global__ __launch_bounds__(64 * (CW + PW), DK == 64 && CW == 4 ? 4 : 1) void l
                     p[r] = s[i][r] * fall[i][r];
                     if (i == N - 1 && 16 * jt + 4 * lg + r > Rq) p[r] = 0.f;
                 }
-                const u32x2 hi = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+                const u32x2 hi = {pack_bf16x2_once(p[0], p[1]), pack_bf16x2_once(p[2], p[3])};
                 const u32x2 lo = {pack_bf16x2(p[0] - bf16_lo(hi[0]), p[1] - bf16_hi(hi[0])), pack_bf16x2(p[2] - bf16_lo(hi[1]), p[3] - bf16_hi(hi[1]))};
                 const int to = Rq * PLD + 32 * (jt >> 1) + 8 * lg + 4 * (jt & 1);
                 *reinterpret_cast<u32x2*>(p_lds + to) = hi;
@@ -721,7 +723,6 @@ __global__ __launch_bounds__(64 * (CW + PW), DK == 64 && CW == 4 ? 4 : 1) void l
                     vf[hh] = *reinterpret_cast<const bf16x8*>(&raw);
                 }
                 if constexpr (!SUMMARY) {
-                    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + (int64_t)(row0 + t0) * a.out_stride + (int64_t)head * a.dv + v0 + 16 * wave + 4 * lg;
                     // what the state gives: slots of a 32-wide step are key rows 16 (2 st) + 4 lg + 0..3 and 16 (2 st + 1) + 4 lg + 0..3
                     f32x4 o[4];                              // o^T: value 16 wave + 4 lg + r, token 16 it + lq
 #pragma unroll
@@ -738,6 +739,7 @@ __global__ __launch_bounds__(64 * (CW + PW), DK == 64 && CW == 4 ? 4 : 1) void l
                             const unsigned char* qrow = qimg + R * KROW + (lg & 1) * 8;
                             const u32x2 qa = *reinterpret_cast<const u32x2*>(qrow + ((4 * st + (lg >> 1)) ^ swz(R)) * 16);
                             const u32x2 qb = *reinterpret_cast<const u32x2*>(qrow + ((4 * st + 2 + (lg >> 1)) ^ swz(R)) * 16);
+                            asm volatile("" ::: "memory");   // (kept apart, or two rows' reads become one, whose halves have to be moved)
                             const u32x4 raw = {qa[0], qa[1], qb[0], qb[1]};
                             const bf16x8 qf = *reinterpret_cast<const bf16x8*>(&raw);
                             o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, qf, o[it], 0, 0, 0);
@@ -755,10 +757,19 @@ __global__ __launch_bounds__(64 * (CW + PW), DK == 64 && CW == 4 ? 4 : 1) void l
                             o[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[hh], *reinterpret_cast<const bf16x8*>(pr + C * PLD), o[it], 0, 0, 0);
                         }
 #pragma unroll
-                    for (int it = 0; it < 4; ++it)
-                        if (16 * it + lq < n) act_st4(out + (16 * it + lq) * a.out_stride, o[it]);
+                    for (int it = 0; it < 4; ++it) act_st4(o_lds + (16 * it + lq) * OLD + 16 * wave + 4 * lg, o[it]);
                 }
-                lds_only_barrier();                          // the weights may be replaced
+                lds_only_barrier();                          // the weights may be replaced; outputs are there
+                if constexpr (!SUMMARY) {
+                    typedef u32x4 __attribute__((aligned(8))) u32x4_half;      // (rows of results may be 8 bytes off a multiple of 16)
+                    const int row = (64 * wave + lane) / VP, col = (64 * wave + lane) % VP * 8;
+                    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + (int64_t)(row0 + t0) * a.out_stride + (int64_t)head * a.dv + v0;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const u32x4 v = *reinterpret_cast<const u32x4*>(o_lds + (row + 32 * j) * OLD + col);
+                        if (row + 32 * j < n) *reinterpret_cast<u32x4_half*>(out + (row + 32 * j) * a.out_stride + col) = v;
+                    }
+                }
                 // ---- the state behind these tokens
                 const float decayed = pw[n];
 #pragma unroll

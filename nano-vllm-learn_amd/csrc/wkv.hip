@@ -31,18 +31,11 @@ constexpr float kMaxDecay = 100.f;                   // log2 units a channel may
 
 __device__ __forceinline__ float log2_decay(float z) { return -kLog2e * __expf(z); }
 
-// two numbers as bf16, the compiler not knowing what from: it would round the first one once more where its half is taken out again
-__device__ __forceinline__ uint32_t packed(float x, float y) {
-    uint32_t v = pack_bf16x2(x, y);
-    asm("" : "+v"(v));
-    return v;
-}
-
 __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
     u32x4 h, l;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        h[j] = packed(v[2 * j], v[2 * j + 1]);
+        h[j] = pack_bf16x2_once(v[2 * j], v[2 * j + 1]);
         l[j] = pack_bf16x2(v[2 * j] - bf16_lo(h[j]), v[2 * j + 1] - bf16_hi(h[j]));
     }
     hi = *reinterpret_cast<const bf16x8*>(&h);
@@ -197,7 +190,7 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
 #pragma unroll
                 for (int r = 0; r < 4; ++r) p[r] = x < 10 ? s[r] : 0.f;
             }
-            const u32x2 hi = {packed(p[0], p[1]), packed(p[2], p[3])};
+            const u32x2 hi = {pack_bf16x2_once(p[0], p[1]), pack_bf16x2_once(p[2], p[3])};
             const u32x2 lo = {pack_bf16x2(p[0] - bf16_lo(hi[0]), p[1] - bf16_hi(hi[0])), pack_bf16x2(p[2] - bf16_lo(hi[1]), p[3] - bf16_hi(hi[1]))};
             uint16_t* const to = &lds.p[0][lq][8 * lg] + (16 * PLD * qg + 32 * (jt >> 1) + 4 * (jt & 1));
             *reinterpret_cast<u32x2*>(to) = hi;
@@ -306,12 +299,12 @@ __global__ __launch_bounds__(DIM * 8, DIM == 64 ? 4 : 1) void wkv_walk_kernel(co
                 for (int i = 0; i < 8; ++i) {
                     const float ia = oa + la[i], ib = ob + lb[i];
                     const float ka = bf16_lo(kk[i]) * fast_exp2(ma - ia), kb = bf16_hi(kk[i]) * fast_exp2(mb - ib);
-                    kh[i] = packed(ka, kb);
+                    kh[i] = pack_bf16x2_once(ka, kb);
                     kl[i] = pack_bf16x2(ka - bf16_lo(kh[i]), kb - bf16_hi(kh[i]));
                     if constexpr (!SUMMARY) {
                         const float ea = oa + (i ? la[i ? i - 1 : 0] : 0.f), eb = ob + (i ? lb[i ? i - 1 : 0] : 0.f);
                         const float ra = bf16_lo(rr[i]) * fast_exp2(ea - ma), rb = bf16_hi(rr[i]) * fast_exp2(eb - mb);
-                        rh[i] = packed(ra, rb);
+                        rh[i] = pack_bf16x2_once(ra, rb);
                         rl[i] = pack_bf16x2(ra - bf16_lo(rh[i]), rb - bf16_hi(rh[i]));
                     }
                     if (AHEAD && (i & 1)) __builtin_amdgcn_sched_barrier(0);

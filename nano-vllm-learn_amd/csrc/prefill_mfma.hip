@@ -538,20 +538,19 @@ __device__ __forceinline__ bool prefill_varlen_body(const PrefillArgs& a, unsign
     // ---- finalise: total row sum over the 4 lane groups, normalise, store 4 contiguous dims per tile
     float l = sum_xor16(l_run);
     l = sum_xor32(l);
-    if (!q_ok) return true;
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    const int64_t orow = ((int64_t)(q_beg + my_q) * a.h + head) * D;
+    if (a.out_f32) {
+        if (!q_ok) return true;
+        const int64_t orow = ((int64_t)(q_beg + my_q) * a.h + head) * D;
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
-        const int d0 = 16 * t + 4 * lg;
-        const f32x4 r = o[t] * inv;
-        if (a.out_f32) {
-            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + orow + d0) = r;
-        } else {
-            u32x2 pk = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
-            *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.out) + orow + d0) = pk;
-        }
+        for (int t = 0; t < DT; ++t) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + orow + 16 * t + 4 * lg) = o[t] * inv;
+        return true;
     }
+    uint16_t* const o_lds = reinterpret_cast<uint16_t*>(lds_all + (KS == 2 ? (4 * DT + 2) * 1024 : 0)) + wave * WR * kRowOut<D>;         // (behind the second group's sums)
+#pragma unroll
+    for (int t = 0; t < DT; ++t) act_st4(o_lds + lq * kRowOut<D> + 16 * t + 4 * lg, o[t] * inv);
+    const int r0 = q0 + wave * WR;
+    rows_out<D, WR>(o_lds, lane, [&](int r) { return r0 + r < sq ? reinterpret_cast<uint16_t*>(a.out) + ((int64_t)(q_beg + r0 + r) * a.h + head) * D : nullptr; });
     return true;
 }
 
@@ -658,13 +657,18 @@ __device__ __forceinline__ bool prefill32_body(const PrefillArgs& a, unsigned ch
             if (key + N - 1 > wave_first_key || key + N > sk) hide_scores(s, [&](int at) { return at <= limit; });
         },
         [&](f32x4 (&v)[D / 8]) {
-            if (my_q >= sq) return;
-            const int64_t at = ((int64_t)(q_beg + my_q) * a.h + head) * D + 4 * lh;
+            if (a.out_f32) {
+                if (my_q >= sq) return;
+                const int64_t at = ((int64_t)(q_beg + my_q) * a.h + head) * D + 4 * lh;
 #pragma unroll
-            for (int u = 0; u < D / 8; ++u) {
-                if (a.out_f32) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + at + 8 * u) = v[u];
-                else act_st4(reinterpret_cast<uint16_t*>(a.out) + at + 8 * u, v[u]);
+                for (int u = 0; u < D / 8; ++u) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + at + 8 * u) = v[u];
+                return;
             }
+            uint16_t* const o_lds = reinterpret_cast<uint16_t*>(lds) + wave * WR * kRowOut<D>;
+#pragma unroll
+            for (int u = 0; u < D / 8; ++u) act_st4(o_lds + lq * kRowOut<D> + 8 * u + 4 * lh, v[u]);
+            const int r0 = q0 + wave * WR;
+            rows_out<D, WR>(o_lds, lane, [&](int r) { return r0 + r < sq ? reinterpret_cast<uint16_t*>(a.out) + ((int64_t)(q_beg + r0 + r) * a.h + head) * D : nullptr; });
         });
     return true;
 }
@@ -683,7 +687,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 && 
             __builtin_amdgcn_s_barrier();
             int qt = at.qt, head = at.head, b = at.b;
             asm volatile("" : "+s"(qt), "+s"(head), "+s"(b));        // (the exact body shares no value with the abandoned one)
-            for (int sub = 0; sub < 2; ++sub) prefill_varlen_body<D, false, false, false, 1>(a, lds, qt * 2 + sub, head, b);
+            for (int sub = 0; sub < 2; ++sub) {
+                if (sub) lds_only_barrier();         // (results leave through the images' memory)
+                prefill_varlen_body<D, false, false, false, 1>(a, lds, qt * 2 + sub, head, b);
+            }
         }
     } else {
         prefill32_body<D, PAGED, PV == 1, false>(a, lds, at);

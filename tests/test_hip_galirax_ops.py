@@ -308,6 +308,33 @@ def test_lightning_chunk_borders_behind_a_state(heads, dk, dv):
         close(state[i], s, BF16, f"state {i}", slack=0.05)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (3, 64, 128), (2, 128, 64), (1, 128, 128), (1, 256, 256), (48, 64, 64), (48, 128, 128)])
+def test_results_leave_by_rows(heads, dim, vdim):
+    """Results that change places in LDS on their way out: rows 8 bytes off a multiple of 16 get the bits of rows side by side, and nothing is written beside or behind
+    them; portions of one row, a tile, one to either side, for workgroups of 64 rows and (48 heads) of 128."""
+    from nanovllm_hip import ops
+    portions = [(1, 70), (15, 15), (16, 200), (17, 17), (31, 90), (63, 63), (64, 300), (65, 65), (127, 400), (129, 129)]
+    rows, kvh = sum(r for r, _ in portions), 1
+    pg = Pages([k for _, k in portions], kvh, dim, vdim, BF16, seed=3)
+    q, cu = pg.pad_q(randn(rows, heads, dim, seed=8)), lambda lengths: torch.tensor([0] + list(lengths)).cumsum(0).int().cuda()
+    how = pg.cache(), pg.tables.cuda(), cu(r for r, _ in portions), cu(k for _, k in portions), 129, heads, kvh, pg.dk, pg.dv, 0.2
+    cols = heads * pg.dv
+    want, out = ops.paged_attend_prompt(q, *how), torch.full((rows + 130, cols + 4), 7.0, dtype=BF16, device="cuda")
+    ops.paged_attend_prompt(q, *how, out=out[:rows, :cols])
+    assert torch.equal(out[:rows, :cols], want) and (out[:, cols:] == 7).all() and (out[rows:] == 7).all()
+
+
+@pytest.mark.parametrize("heads,dk,dv,rows", [(2, 64, 64, 63), (2, 64, 128, 65), (1, 128, 128, 31), (1, 128, 256, 161), (16, 128, 128, 33)])
+def test_lightning_results_leave_by_rows(heads, dk, dv, rows):
+    from nanovllm_hip import ops
+    x, decay, cols = randn(rows, heads * (2 * dk + dv), seed=3).cuda(), torch.tensor((DECAYS * heads)[:heads], dtype=F32).cuda(), heads * dv
+    how = torch.arange(rows).cuda(), torch.zeros(1, dtype=torch.int32, device="cuda"), torch.tensor([(0, rows, 0, 0)], dtype=torch.int32).cuda(), False
+    out, states = torch.full((rows + 70, cols + 4), 7.0, dtype=BF16, device="cuda"), [torch.zeros(1, heads, dk, dv, device="cuda") for _ in range(2)]
+    want = ops.lightning_chunks(x, decay, *how, states[0])
+    ops.lightning_chunks(x, decay, *how, states[1], out=out[:rows, :cols])
+    assert torch.equal(out[:rows, :cols], want) and torch.equal(*states) and (out[:, cols:] == 7).all() and (out[rows:] == 7).all()
+
+
 # a few long portions among short ones, portions of 192, 193, 256 and 257 tokens (the shortest that are cut), without rows, one behind a state, as many as are looked at and one more
 UNEVEN = [1500, 700, 90, 300, 64, 0, 1, 400, 193, 1000, 20, 192, 257, 256]
 @pytest.mark.parametrize("heads,dk,dv,lengths,behind", [

@@ -326,7 +326,7 @@ __global__ __launch_bounds__(HPW == 1 ? 1024 : 512) void talk_prompt_kernel(cons
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float p0 = s[i >> 1][2 * (i & 1)], p1 = s[i >> 1][2 * (i & 1) + 1];
-                hraw[i] = pack_bf16x2_once(p0, p1);
+                hraw[i] = pack_bf16x2(p0, p1);
                 asm volatile("" : "+v"(hraw[i]));    // (its halves are taken from here, not converted once more)
                 lraw[i] = pack_bf16x2(p0 - bf16_lo(hraw[i]), p1 - bf16_hi(hraw[i]));
             }

@@ -265,7 +265,8 @@ __global__ __launch_bounds__(256) void lightning_walk_kernel(const LightningArgs
 // What bounds it is issue (a wave alone issues a vector instruction every 5.5 cycles, three together every 2.7) and, with all CUs busy, the rows that all ask for at
 // once; so a workgroup has three waves per SIMD and takes 16 CW columns, 128 where they come in such numbers: queries and keys are prepared once for all of them,
 // not for every 64.  A chunk takes 3.8 us alone and 5.0 on all CUs, 9.1 for two workgroups of the 64-column walk; 16 prompts of 1024 tokens on average, 16 heads of
-// 128: 251 -> 108 us; 40 prompts of 410: 302 -> 157.  Measured and not better: eight waves with 32 columns each (121), sixteen waves (114), fragments read a step
+// 128: 251 -> 108 us; 40 prompts of 410: 302 -> 157.  Results leave by whole rows, through LDS, and the queries' reads are kept apart: 104.4 -> 99.6
+// there.  Measured and not better: eight waves with 32 columns each (121), sixteen waves (114), fragments read a step
 // ahead by hand (121).
 template <int DK, int CW>
 constexpr size_t pair_lds_bytes(bool summary) {

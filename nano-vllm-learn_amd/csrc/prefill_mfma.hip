@@ -979,15 +979,19 @@ void prefill_short_kernel(const PrefillArgs a) {
         if (my_q < sq) {
             const float inv = l > 0.f ? 1.f / l : 0.f;
             const int64_t orow = ((int64_t)(q_beg + my_q) * a.h + head) * D;
+            if (a.out_f32) {
 #pragma unroll
-            for (int tt = 0; tt < DT; ++tt) {
-                const int d0 = 16 * tt + 4 * lg;
-                const f32x4 r = o[tt] * inv;
-                if (a.out_f32) {
-                    *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + orow + d0) = r;
-                } else {
-                    u32x2 pk = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
-                    *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.out) + orow + d0) = pk;
+                for (int tt = 0; tt < DT; ++tt) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + orow + 16 * tt + 4 * lg) = o[tt] * inv;
+            } else {
+                // two tiles at a time, their halves changed between neighbouring lane groups of a row: 64 bytes of each row a store instead of 32, and half as many.  (The images stay
+                // in use; whole rows through LDS of their own were no faster.)  256 sequences of 128, 14 / 2 heads of 64, 32.8 -> 31.1 us; 64 of up to 120, 16 / 8 of 128, 21.5 -> 20.3
+                uint16_t* const to = reinterpret_cast<uint16_t*>(a.out) + orow + 16 * (lg & 1) + 8 * (lg >> 1);
+#pragma unroll
+                for (int tt = 0; tt < DT; tt += 2) {
+                    const f32x4 r = o[tt] * inv, n = o[tt + 1] * inv;
+                    const auto x = __builtin_amdgcn_permlane16_swap(pack_bf16x2(r[0], r[1]), pack_bf16x2(n[0], n[1]), false, false);
+                    const auto y = __builtin_amdgcn_permlane16_swap(pack_bf16x2(r[2], r[3]), pack_bf16x2(n[2], n[3]), false, false);
+                    *reinterpret_cast<u32x4*>(to + 16 * tt) = u32x4{x[0], y[0], x[1], y[1]};
                 }
             }
         }

@@ -279,7 +279,8 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
 
     // ---- gathering.  quads: 16-byte pieces, thread t takes t, t + kThreads, ...; use(piece, words) for each.  Marks are checked piece by piece
     uint32_t limit = fresh_args().spin_limit;
-    int flag = 2;                                                                // a word for every other share: a wave may wait for the next while another still looks at this one's
+    int flag = 2;                                                                // a word for every other share that passes barriers: a wave may wait for the next one while another still
+                                                                                 // looks at this one's (attention that a workgroup has no share of passes none, and leaves the word as it is)
     auto ran_out = [&](uint32_t& spins) {
         if (++spins < limit) return false;
         say[flag] = 1;
@@ -511,6 +512,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
         if (role >= a.shares) return false;
         const Chunk ck = chunk_of(a, role);
         if (ck.c >= max(ck.used, 1)) return false;                           // (without tokens the first share says so)
+        flag ^= 1;
         unsigned char* const qs = lds + a.l_q;                               // [head][D + 8]
         unsigned char* const news = lds + a.l_news;                          // [row of the batch][k, v][D]
         float* const ml = reinterpret_cast<float*>(lds + a.l_ml);            // [wave][max, sum][16]
@@ -765,7 +767,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
         return late;
     };
     auto run = [&](auto help, int l, int ph, int role) -> bool {
-        flag ^= 1;
+        if (ph != PH_ATTEND) flag ^= 1;                                          // (there behind the early ends)
         l = __builtin_amdgcn_readfirstlane(l);                                   // (what the compiler does not see: else it reads the layer's pointers by vector loads)
         role = __builtin_amdgcn_readfirstlane(role);
         switch (__builtin_amdgcn_readfirstlane(ph)) {

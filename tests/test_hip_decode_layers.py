@@ -148,6 +148,21 @@ def test_workgroups_that_start_late(late_from):
     assert ws.view(torch.int32)[[0, 32, 64]].tolist() == [4, 0, 0]           # launches; workgroups started; gave up
 
 
+@pytest.mark.parametrize("shape,norm", [((896, 14, 2, 64, 4864), False), ((1024, 16, 8, 128, 3072), True), ((512, 16, 1, 128, 256), False)])
+@pytest.mark.parametrize("contexts", [[1], [700], [4500], [0, 33], [1030, 2111], [40, 300, 1], [600, 0, 1500]])
+@pytest.mark.parametrize("late_from", [1, 20, 250])
+def test_help_in_every_form(shape, norm, contexts, late_from):
+    """Shares of both widths of heads, with and without q/k norm, of one to three rows, several rounds of tiles and none, done by workgroups that wait, most of which have no share of
+    the attention: a wait's end concerns the whole workgroup or nobody."""
+    s = build(*shape, 3, norm, contexts)
+    ws = scratch(s)
+    want = call(s, ws)
+    for _ in range(2):
+        assert torch.equal(call(s, ws, spin_limit=8, late_from=late_from, late_for=2000), want)
+    assert torch.equal(call(s, ws), want)
+    assert ws.view(torch.int32)[[0, 32, 64]].tolist() == [4, 0, 0]
+
+
 def test_two_launches_side_by_side():
     a, b = build(896, 14, 2, 64, 4864, 3, False, [500], seed=1), build(896, 14, 2, 64, 4864, 3, False, [900, 20], seed=2)
     wa, wb = scratch(a), scratch(b)

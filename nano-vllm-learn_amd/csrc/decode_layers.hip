@@ -132,9 +132,14 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
     LdsWord* const say = (LdsWord*)(lds + kLdsSay);                              // [0] launch number, [1] results are missing, [2], [3] a wait of this share ran out
     if (threadIdx.x == 0) {
         Args& a = fresh_args();
-        say[0] = load_word((const Word*)a.sync);
+        // Launches so far and, in the high half, workgroups of this one that have started: the last of them puts the next launch's number there, when all others hold
+        // this one's.  (A load, a counter and a wait of one workgroup for all to have started would need an end for that wait, and a number for whoever starts behind it.)
+        typedef __attribute__((address_space(1))) uint64_t Start;
+        Start* const start = (Start*)a.sync;
+        const uint64_t was = __hip_atomic_fetch_add(start, 1ull << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)(was >> 32) == (uint32_t)a.grid - 1) __hip_atomic_store(start, (uint64_t)((uint32_t)was + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        say[0] = (uint32_t)was;
         say[1] = say[2] = say[3] = 0;
-        __hip_atomic_fetch_add(a.sync + 32, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if ((int)blockIdx.x >= a.late_from)
             for (int i = 0; i < a.late_for; ++i) __builtin_amdgcn_s_sleep(8);    // (tests: workgroups that start late)
     }
@@ -860,19 +865,12 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
         }
     }
     drain_loads();
-    if (threadIdx.x == 0) {
+    if (lost && threadIdx.x == 0) {                                              // (never seen.  A workgroup that gave up leaves no plausible results, and says so)
         Args& a = fresh_args();
-        if (lost) {                                                              // (never seen.  A workgroup that gave up leaves no plausible results, and says so)
-            store_word((Word*)a.sync + 64, 1u);
-            for (int i = 0; i < M * a.hidden; ++i) {
-                a.out[i / a.hidden * a.out_stride + i % a.hidden] = 0x7fff;
-                if (a.out_packed) a.out_packed[pack_index(i / a.hidden, i % a.hidden, a.hidden)] = 0x7fff;
-            }
-        }
-        if (blockIdx.x == 0) {                                                   // the number of the next launch, once every workgroup of this one has read its own
-            for (int i = 0; i < 1 << 24 && load_word((const Word*)a.sync + 32) != (uint32_t)a.grid; ++i) __builtin_amdgcn_s_sleep(8);
-            store_word((Word*)a.sync + 32, 0u);
-            store_word((Word*)a.sync, launch + 1);
+        store_word((Word*)a.sync + 64, 1u);
+        for (int i = 0; i < M * a.hidden; ++i) {
+            a.out[i / a.hidden * a.out_stride + i % a.hidden] = 0x7fff;
+            if (a.out_packed) a.out_packed[pack_index(i / a.hidden, i % a.hidden, a.hidden)] = 0x7fff;
         }
     }
 }

@@ -206,3 +206,19 @@ def test_refusals():
         call(s, torch.zeros(256, dtype=torch.uint8, device="cuda"))
     with pytest.raises(Exception, match="out may not be x"):
         call(s, scratch(s), out=s["x"])
+
+
+@pytest.mark.parametrize("first", [0xfffd, 0xfffffffd])
+def test_launch_numbers_come_round(first):
+    """Marks are 16 bits of the launch's number beside an activation and 32 beside a share of the attention: past their ends nothing of the launch before is taken for this one's."""
+    s = build(*SMALL, 3, False, [700, 90])
+    ws = scratch(s)
+    head = ws.view(torch.int64)
+    head[0] = first
+    want = {}
+    for n in range(1, 7):
+        s["x"].mul_(-1)                                      # (every launch has other results than the one before)
+        got = call(s, ws)
+        assert torch.equal(got, want.setdefault(n % 2, got.clone()))
+        assert head[0].item() == (first + n) % 2 ** 32       # the next launch's number, and no workgroup started
+    assert not torch.equal(want[0], want[1]) and error(want[0], exact(s)[0]) < BOUND

@@ -113,6 +113,13 @@ int nvh_decode_layers_variant(uint32_t spin_limit, int late_from, int late_for, 
     return launch_decode_layers(a, d->hd, qk_norm, lds, (hipStream_t)stream);
 }
 
+int nvh_decode_layers_status(const void* workspace, uint32_t* gave_up) {
+    REQUIRE(workspace && gave_up, NVH_E_NULL, "decode_layers_status: null pointer");
+    const hipError_t e = hipMemcpy(gave_up, (const uint32_t*)workspace + kDecodeLayersGaveUp, sizeof(uint32_t), hipMemcpyDeviceToHost);
+    REQUIRE(e == hipSuccess, (int)e, "decode_layers_status: %s", hipGetErrorString(e));
+    return 0;
+}
+
 int nvh_decode_layers(const nvh_decode_layers_desc* d, int dtype, void* stream) { return nvh_decode_layers_variant(0, 0, 0, d, dtype, stream); }
 
 }  // extern "C"

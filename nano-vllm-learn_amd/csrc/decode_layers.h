@@ -10,7 +10,8 @@ namespace nvh {
 constexpr int kDecodeLayersMost = 32;            // layers of a launch: their pointers are kernel arguments (4 KB)
 constexpr int kDecodeLayersRows = 3;             // sequences of a step
 constexpr int kDecodeLayersLds = 160 * 1024;
-constexpr int kDecodeLayersSync = 1024;          // bytes in front of the words: [0] launches so far, [1] workgroups of this one that have started, [64] a workgroup gave up
+constexpr int kDecodeLayersSync = 1024;          // bytes in front of the words: [0] launches so far, [1] workgroups of this one that have started,
+constexpr int kDecodeLayersGaveUp = 64;          // [64] a workgroup gave up
 constexpr int kDecodeLayersColumns = 48;            // of a workgroup's share of a projection (of gate and of up each)
 constexpr int kLdsSay = 0, kLdsResults = 128, kLdsRope = kLdsResults + kDecodeLayersRows * kDecodeLayersColumns * 4, kLdsCommon = kLdsRope + kDecodeLayersRows * 128 * 4;     // bytes of LDS both kinds of workgroup lay out alike
 constexpr int kDecodeLayersWalkers = 8, kDecodeLayersBuffers = 2;      // attention: waves that take tiles of 16 tokens, and tiles of a wave in LDS

@@ -867,7 +867,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
     drain_loads();
     if (lost && threadIdx.x == 0) {                                              // (never seen.  A workgroup that gave up leaves no plausible results, and says so)
         Args& a = fresh_args();
-        store_word((Word*)a.sync + 64, 1u);
+        store_word((Word*)a.sync + kDecodeLayersGaveUp, 1u);
         for (int i = 0; i < M * a.hidden; ++i) {
             a.out[i / a.hidden * a.out_stride + i % a.hidden] = 0x7fff;
             if (a.out_packed) a.out_packed[pack_index(i / a.hidden, i % a.hidden, a.hidden)] = 0x7fff;

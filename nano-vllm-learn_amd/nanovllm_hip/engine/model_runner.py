@@ -253,13 +253,15 @@ class ModelRunner:
 
     def raise_if_device_failed(self):
         """At a point where the host has synchronised: a time-out marked by one of the bounded device-side waits (the one-shot all-reduce of
-        any rank; the one-launch qkv + attention form) must surface as an error on every rank, not as garbage tokens."""
+        any rank; the one-launch qkv + attention form; a decode step's layers in one launch) must surface as an error on every rank, not as garbage tokens."""
         if self.comm is not None:
             from ..distributed import raise_if_failed
             raise_if_failed()
         from ..models import qwen
         if qwen.QKV_ATTEND_MODE in ("one_launch", "auto") and self.device.type == "cuda" and ops.qkv_rope_attend_status(device=self.device):
             raise RuntimeError("nvh_qkv_rope_attend (one launch): a consumer's wait for the projection's producers ran out; the step's rows are NaN")
+        if self.device.type == "cuda" and getattr(self.model, "decode_gave_up", bool)():
+            raise RuntimeError("nvh_decode_layers: a workgroup gave up waiting for others' results; the steps since then are not to be used")
 
     def close(self):
         """Release the tensor-parallel communicator's IPC mappings (every rank, after the last step)."""

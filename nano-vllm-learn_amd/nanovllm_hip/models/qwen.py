@@ -479,6 +479,12 @@ class QwenForCausalLM(nn.Module):
                                 softmax_scale=a.attn.scale, out_packed=b["resid_p"], workspace=b["layers_ws"])
         return PackedResidual(out, b["resid_p"])
 
+    def decode_gave_up(self):
+        """Host-synchronous: has a step of all layers in one launch given up since its scratch was made?  (Every step since then is suspect.)"""
+        from .. import ops
+        held = [b["layers_ws"] for b in self.__dict__.get("_decode_bufs", {}).values() if b["layers_ws"] is not None]
+        return any(ops.decode_layers_status(ws) for ws in held)
+
     def compute_logits(self, hidden_states):
         w = self.embed_tokens.weight if self.cfg.tie_word_embeddings else self.lm_head.weight
         if isinstance(hidden_states, PackedResidual):                 # fused decode path: final RMSNorm in the LM-head launch

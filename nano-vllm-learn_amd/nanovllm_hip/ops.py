@@ -605,6 +605,13 @@ def decode_layers(x, layers, *, num_heads, num_kv_heads, head_dim, inter, norm_e
     return out
 
 
+def decode_layers_status(workspace) -> int:
+    """Host-synchronous: non-zero behind a decode_layers launch (that has finished) on this workspace of which a workgroup gave up (its outputs are not to be used); until it is zero-filled again."""
+    v = ctypes.c_uint32(0)
+    _lib.check(_lib.load().nvh_decode_layers_status(workspace.data_ptr(), ctypes.byref(v)), "nvh_decode_layers_status")
+    return int(v.value)
+
+
 def linear_candidate_groups(n, k) -> int:
     return int(_lib.load().nvh_linear_small_m_candidate_groups(n, k))
 

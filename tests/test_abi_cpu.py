@@ -98,6 +98,12 @@ def test_argument_validation_without_gpu(lib):
     assert lib.nvh_prefill_varlen_pv16(p, p, p, p, p, p, 0, 0, 0, 0, 14, 2, 64, 896, 128, 128, 0.125, 0, 0, None, 0, None) == 0   # empty batch
 
 
+def test_decode_layers_status_refuses_null_pointers(lib):
+    v = ctypes.c_uint32(5)
+    assert lib.nvh_decode_layers_status(None, ctypes.byref(v)) == -5 and b"decode_layers_status" in lib.nvh_last_error()
+    assert lib.nvh_decode_layers_status(ctypes.c_void_p(4096), None) == -5
+
+
 def test_experts_in_one_call_refuse_scratch_that_is_too_small(lib):
     """Scratch is a pure function of the sizes (no tiles up to 64 rows in bf16, always some in fp32); nothing is launched without all of it."""
     from nanovllm_hip import _lib

@@ -1,0 +1,40 @@
+"""Decode steps of one to three sequences, whose layers are one launch (nvh_decode_layers), as the engine runs them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FAMILIES = {"qwen2": {}, "qwen3": dict(num_attention_heads=4, num_key_value_heads=2, head_dim=128, hidden_size=512, intermediate_size=1024, qkv_bias=False, qk_norm=True)}
+
+
+def engine(family, **kw):
+    from nanovllm_hip.engine.llm_engine import LLMEngine
+    from nanovllm_hip.models import qwen
+    cfg = qwen.model_config("Qwen2-0.5B", num_hidden_layers=3, vocab_size=2048, **FAMILIES[family])
+    return LLMEngine(cfg, num_kvcache_blocks=12, seed=4, **kw)
+
+
+def prefilled(eng, lengths, new):
+    from nanovllm_hip.engine.sequence import Sequence
+    gen = torch.Generator().manual_seed(11)
+    seqs = [Sequence(torch.randint(0, 2048, (n,), generator=gen).tolist(), max_tokens=new) for n in lengths]
+    eng.prefill(seqs, reserve_tokens=new)
+    return seqs
+
+
+def test_a_step_that_gave_up_is_an_error():
+    eng = engine("qwen2")
+    seqs = prefilled(eng, (40, 7), 8)
+    session = eng.runner.decode_session(seqs, 8, use_graph=False)
+    session.step(2)
+    eng.runner.raise_if_device_failed()
+    held = [b["layers_ws"] for b in eng.runner.model._decode_bufs.values() if b["layers_ws"] is not None]
+    assert len(held) == 1 and held[0].view(torch.int32)[0] == 2            # (two launches)
+    held[0].view(torch.int32)[64] = 1                                      # what a workgroup leaves that gives up
+    with pytest.raises(RuntimeError, match="gave up"):
+        eng.runner.raise_if_device_failed()
+    with pytest.raises(RuntimeError, match="gave up"):
+        session.finish()
+    with torch.inference_mode():
+        held[0].zero_()
+    eng.runner.raise_if_device_failed()

@@ -10,7 +10,7 @@ namespace nvh {
 static uint32_t magic_of(uint32_t d) { return (uint32_t)((1ull << 32) / d + 1); }
 
 int plan_decode_layers(DecodeLayersArgs& a, int cus, int m, int hidden, int h, int kvh, int hd, int inter, int layers) {
-    if (m < 1 || m > kDecodeLayersRows || (hd != 64 && hd != 128) || kvh <= 0 || h % kvh || h / kvh > 16 || layers < 1 || layers > kDecodeLayersMost) return 0;
+    if (m < 1 || m > kDecodeLayersRows || (hd != 64 && hd != 128) || h <= 0 || kvh <= 0 || h % kvh || h / kvh > 16 || layers < 1 || layers > kDecodeLayersMost) return 0;
     const int qsize = h * hd, nqkv = (h + 2 * kvh) * hd;
     // what a wave holds of the weights: rows of up to 2, 4 and 10 times 64 pieces of 16 bytes
     if (hidden % 8 || inter % 8 || hidden <= 0 || inter <= 0 || hidden > 1024 || qsize > 2048 || inter > 5120 || cus < 64) return 0;

@@ -246,3 +246,25 @@ def test_pack_index_matches_the_torch_packer():
     assert torch.equal(ops.unpack_rows(xp, m, c), x)
     assert lib.nvh_linear_small_m_workspace(32, 896, 896, 2) == 0           # K <= 1024: one workgroup per tile, no hand-off
     assert lib.nvh_linear_small_m_workspace(32, 896, 4864, 2) >= 56 * 4 + 56 * 5 * (2 * 256 + 32) * 4
+
+
+# what the split of a decode step's layers over a chip of 256 CUs says of these sizes (0: not served): in a process of its own, a division by zero would end it
+_PLAN = """
+import ctypes
+from nanovllm_hip import _lib
+plan = ctypes.CDLL(_lib.LIB_PATH)["_ZN3nvh18plan_decode_layersERNS_16DecodeLayersArgsEiiiiiiii"]
+args = (ctypes.c_char * 8192)()
+for m, hidden, h, kvh, hd, inter, layers in {sizes}:
+    print(plan(args, 256, m, hidden, h, kvh, hd, inter, layers))
+"""
+
+
+def test_decode_layers_plan_refuses_sizes_without_heads():
+    import subprocess
+    import sys
+    good = (1, 896, 14, 2, 64, 4864, 24)
+    bad = [(1, 896, h, kvh, 64, 4864, 24) for h, kvh in ((0, 2), (-2, 2), (-14, 2), (14, 0), (14, -2), (-14, -2))] + [(0, *good[1:]), (1, 0, *good[2:]), (*good[:5], 0, 24), (*good[:6], 0)]
+    done = subprocess.run([sys.executable, "-c", _PLAN.format(sizes=[good, *bad])], capture_output=True, text=True, timeout=300, cwd=os.path.join(ROOT, "nano-vllm-learn_amd"))
+    assert done.returncode == 0, done.stderr[-500:]
+    first, *rest = [int(x) for x in done.stdout.split()]
+    assert first > 0 and rest == [0] * len(bad)

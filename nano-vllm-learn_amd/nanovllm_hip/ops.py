@@ -575,9 +575,10 @@ def decode_layers(x, layers, *, num_heads, num_kv_heads, head_dim, inter, norm_e
     m, hidden = x.shape
     _require_gpu_bf16(x=x)
     _require_i32(slot_mapping=slot_mapping, context_lens=context_lens, block_tables=block_tables)
-    assert x.stride(1) == 1 and positions.dtype == torch.int64 and positions.numel() == m and positions.is_contiguous() and positions.is_cuda
+    # (positions and slots of more rows than x has: the first ones count, as for fused_linear's "rope_store")
+    assert x.stride(1) == 1 and positions.dtype == torch.int64 and positions.numel() >= m and positions.is_contiguous() and positions.is_cuda
     assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.shape[-1] == head_dim
-    assert slot_mapping.numel() == m and slot_mapping.is_contiguous() and context_lens.numel() == m and context_lens.is_contiguous()
+    assert slot_mapping.numel() >= m and slot_mapping.is_contiguous() and context_lens.numel() == m and context_lens.is_contiguous()
     assert block_tables.dim() == 2 and block_tables.shape[0] == m and block_tables.stride(1) == 1
     nqkv, qsize, page = (num_heads + 2 * num_kv_heads) * head_dim, num_heads * head_dim, layers[0]["k_cache"].shape[1]
     shapes = dict(qkv_w=(nqkv, hidden), o_w=(hidden, qsize), gate_up_w=(2 * inter, hidden), down_w=(hidden, inter), qkv_bias=(nqkv,), q_norm_w=(head_dim,), k_norm_w=(head_dim,))

@@ -38,3 +38,25 @@ def test_a_step_that_gave_up_is_an_error():
     with torch.inference_mode():
         held[0].zero_()
     eng.runner.raise_if_device_failed()
+
+
+@torch.inference_mode()
+def logits(eng, seqs, more=0):
+    """One decode step, not kept; positions and slots of `more` rows than there are sequences."""
+    from nanovllm_hip import reset_context, set_context
+    from nanovllm_hip.engine.model_runner import build_decode_meta
+    m, model = {k: v.cuda() for k, v in build_decode_meta(seqs).items()}, eng.runner.model
+    slots, positions = (torch.cat([m[k], m[k].new_zeros(more)]) for k in ("slot_mapping", "positions"))
+    set_context(False, slot_mapping=slots, context_lens=m["context_lens"], block_tables=m["block_tables"])
+    try:
+        return model.compute_logits(model(m["input_ids"], positions)).float()
+    finally:
+        reset_context()
+
+
+def test_positions_and_slots_of_more_rows():
+    """Buffers made for the largest batch, as the projection's launch takes them: the first rows count."""
+    eng = engine("qwen2")
+    seqs = prefilled(eng, (40, 7), 4)
+    want = logits(eng, seqs)
+    assert torch.equal(logits(eng, seqs, more=6), want)

@@ -401,7 +401,9 @@ class QwenForCausalLM(nn.Module):
         m = residual.shape[0]
         b = self._decode_buffers(m, residual.device)
         cache = self.layers[0].self_attn.attn.k_cache
-        if cache.dim() == 4 and ctx.block_tables.shape[1] * cache.shape[1] <= b["layers_tokens"]:      # (the table is as wide as the longest context may get)
+        # (the switches say how the launches of a layer run: set, they ask for launches.  The table is as wide as the longest context may get)
+        plain = QKV_ATTEND_MODE == "two_launches" and PREFETCH_WEIGHTS and not KV_AHEAD
+        if plain and cache.dim() == 4 and ctx.block_tables.shape[1] * cache.shape[1] <= b["layers_tokens"]:
             return self._forward_decode_layers(residual, positions, ctx, b)
         resid_p, act_p, attn_p, ws, ybuf = b["resid_p"], b["act_p"], b["attn_p"], b["ws"], b["y"]
         tp = _tp()[1]

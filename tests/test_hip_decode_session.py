@@ -60,3 +60,19 @@ def test_positions_and_slots_of_more_rows():
     seqs = prefilled(eng, (40, 7), 4)
     want = logits(eng, seqs)
     assert torch.equal(logits(eng, seqs, more=6), want)
+
+
+@pytest.mark.parametrize("switch,value", [("QKV_ATTEND_MODE", "auto"), ("QKV_ATTEND_MODE", "two_launches_kv_prefetch"), ("PREFETCH_WEIGHTS", False), ("KV_AHEAD", "o_k")])
+def test_switches_of_the_launches_are_followed(switch, value, monkeypatch):
+    from nanovllm_hip import ops
+    from nanovllm_hip.models import qwen
+    eng = engine("qwen2")
+    seqs = prefilled(eng, (40, 7), 4)
+    calls = []
+    real = ops.decode_layers
+    monkeypatch.setattr(ops, "decode_layers", lambda *a, **kw: calls.append(1) or real(*a, **kw))
+    want = logits(eng, seqs)
+    assert len(calls) == 1
+    monkeypatch.setattr(qwen, switch, value)
+    got = logits(eng, seqs)
+    assert len(calls) == 1 and (got - want).abs().max() <= 3e-2 * want.abs().max()

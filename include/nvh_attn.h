@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 211          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch, _status, _variant; 210: nvh_decode_layers; 211: nvh_decode_layers_status */
+#define NVH_VERSION 211          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch, _status, _variant; 210: nvh_decode_layers; 211: nvh_decode_layers_status, nvh_decode_layers_stream */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -297,7 +297,10 @@ size_t nvh_decode_layers_workspace(int m, int hidden, int h, int kvh, int hd, in
 /* longest context for which this is faster than a launch for each part (longer ones are served all the same) */
 int nvh_decode_layers_tokens(int m, int hidden, int h, int kvh, int hd, int inter, int n_layers);
 int nvh_decode_layers(const nvh_decode_layers_desc* desc, int dtype, void* stream);
-/* Workgroups wait for each other; a wait that lasts too long (3 ms) is ended by doing what is missing.  One that still finds its inputs incomplete gives up: its launch's outputs are not
+/* 1: launches on this stream may use every CU of the device.  Workgroups wait for each other; with fewer CUs some start only behind others' ends, which costs a wait that runs out for
+ * nearly every part (Qwen2-0.5B, 248 CUs: 16 ms a step; launches 0.63) */
+int nvh_decode_layers_stream(void* stream);
+/* A wait that lasts too long (3 ms) is ended by doing what is missing.  One that still finds its inputs incomplete gives up: its launch's outputs are not
  * to be used (NaN where no other workgroup has written), and the status, read from the workspace behind that launch, is 1 until that is zero-filled again (host-synchronous, not capturable). */
 int nvh_decode_layers_status(const void* workspace, uint32_t* gave_up);
 /* tests: spin_limit = polls before a workgroup does the shares it waits for (0 = default); workgroups from late_from on start late_for sleeps late */

@@ -113,6 +113,19 @@ int nvh_decode_layers_variant(uint32_t spin_limit, int late_from, int late_for, 
     return launch_decode_layers(a, d->hd, qk_norm, lds, (hipStream_t)stream);
 }
 
+int nvh_decode_layers_stream(void* stream) {
+    constexpr int kWords = 32;
+    uint32_t mask[kWords] = {};
+    const int cus = device_cus(), words = (cus + 31) / 32;
+    if (cus <= 0 || words > kWords || hipExtStreamGetCUMask((hipStream_t)stream, words, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return cus > 0;                                                          // (no answer: a stream like others)
+    }
+    int n = 0;
+    for (int i = 0; i < words; ++i) n += __builtin_popcount(mask[i]);
+    return n >= cus;
+}
+
 int nvh_decode_layers_status(const void* workspace, uint32_t* gave_up) {
     REQUIRE(workspace && gave_up, NVH_E_NULL, "decode_layers_status: null pointer");
     const hipError_t e = hipMemcpy(gave_up, (const uint32_t*)workspace + kDecodeLayersGaveUp, sizeof(uint32_t), hipMemcpyDeviceToHost);

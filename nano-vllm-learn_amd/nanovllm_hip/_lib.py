@@ -272,6 +272,7 @@ _SIGS = {
     "nvh_decode_layers_workspace": (ctypes.c_size_t, [ctypes.c_int] * 7),
     "nvh_decode_layers_tokens": (ctypes.c_int, [ctypes.c_int] * 7),
     "nvh_decode_layers": (ctypes.c_int, [ctypes.POINTER(DecodeLayersDesc), ctypes.c_int, ctypes.c_void_p]),
+    "nvh_decode_layers_stream": (ctypes.c_int, [ctypes.c_void_p]),
     "nvh_decode_layers_status": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint32)]),
     "nvh_decode_layers_variant": (ctypes.c_int, [ctypes.c_uint32, ctypes.c_int, ctypes.c_int, ctypes.POINTER(DecodeLayersDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_qkv_rope_attend": (ctypes.c_int, [ctypes.POINTER(LinearDesc), ctypes.c_void_p, ctypes.c_void_p, _c_i32p, _c_i32p, ctypes.c_int, ctypes.c_int,

@@ -416,6 +416,18 @@ class DecodeSession:
 
     @torch.inference_mode()
     def _capture(self):
+        # recorded on streams made here, replayed on the current one: which of them may use every CU is asked of the current one
+        model = self.runner.model
+        chosen = getattr(model, "decode_in_one_launch", None)
+        if chosen:
+            model.decode_in_one_launch = ops.decode_layers_stream_ok()
+        try:
+            self._capture_graphs()
+        finally:
+            if chosen:
+                model.decode_in_one_launch = chosen
+
+    def _capture_graphs(self):
         # capture must not disturb the live state: snapshot, warm up + capture, restore
         self._capture_saved = saved = [t.clone() for t in self._live()]
         stream = torch.cuda.Stream(device=self.runner.device)

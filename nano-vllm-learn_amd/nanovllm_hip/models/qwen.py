@@ -315,6 +315,8 @@ def _fused_decode_ok(cfg, x):
 
 
 class QwenForCausalLM(nn.Module):
+    decode_in_one_launch = True      # all layers of a step of few sequences in one launch, where that is faster; False: a launch for each part of a layer
+
     def __init__(self, cfg: ModelConfig):
         super().__init__()
         self.cfg = cfg
@@ -402,8 +404,8 @@ class QwenForCausalLM(nn.Module):
         b = self._decode_buffers(m, residual.device)
         cache = self.layers[0].self_attn.attn.k_cache
         # (the switches say how the launches of a layer run: set, they ask for launches.  The table is as wide as the longest context may get)
-        plain = QKV_ATTEND_MODE == "two_launches" and PREFETCH_WEIGHTS and not KV_AHEAD
-        if plain and cache.dim() == 4 and ctx.block_tables.shape[1] * cache.shape[1] <= b["layers_tokens"]:
+        plain = self.decode_in_one_launch and QKV_ATTEND_MODE == "two_launches" and PREFETCH_WEIGHTS and not KV_AHEAD
+        if plain and cache.dim() == 4 and ctx.block_tables.shape[1] * cache.shape[1] <= b["layers_tokens"] and ops.decode_layers_stream_ok():
             return self._forward_decode_layers(residual, positions, ctx, b)
         resid_p, act_p, attn_p, ws, ybuf = b["resid_p"], b["act_p"], b["attn_p"], b["ws"], b["y"]
         tp = _tp()[1]

@@ -606,6 +606,11 @@ def decode_layers(x, layers, *, num_heads, num_kv_heads, head_dim, inter, norm_e
     return out
 
 
+def decode_layers_stream_ok() -> bool:
+    """May launches on the current stream use every CU of the device?  (decode_layers is slow where they may not: its workgroups wait for each other.)"""
+    return bool(_lib.load().nvh_decode_layers_stream(_stream()))
+
+
 def decode_layers_status(workspace) -> int:
     """Host-synchronous: non-zero behind a decode_layers launch (that has finished) on this workspace of which a workgroup gave up (its outputs are not to be used); until it is zero-filled again."""
     v = ctypes.c_uint32(0)

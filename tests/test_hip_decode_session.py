@@ -76,3 +76,28 @@ def test_switches_of_the_launches_are_followed(switch, value, monkeypatch):
     monkeypatch.setattr(qwen, switch, value)
     got = logits(eng, seqs)
     assert len(calls) == 1 and (got - want).abs().max() <= 3e-2 * want.abs().max()
+
+
+@pytest.mark.parametrize("cus", [256, 192])
+def test_streams_that_may_not_use_every_cu_get_launches(cus, monkeypatch):
+    """Workgroups that wait for each other all want a CU: eager steps and a session that is replayed on such a stream take launches."""
+    import ctypes
+    from nanovllm_hip import ops
+    words = (torch.cuda.get_device_properties(0).multi_processor_count + 31) // 32
+    mask = (ctypes.c_uint32 * words)(*[(1 << min(max(cus - 32 * i, 0), 32)) - 1 for i in range(words)])
+    hip, handle = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p()
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(handle), words, mask) == 0
+    calls, real = [], ops.decode_layers
+    monkeypatch.setattr(ops, "decode_layers", lambda *a, **kw: calls.append(1) or real(*a, **kw))
+    eng = engine("qwen2")
+    seqs = prefilled(eng, (40, 7), 8)
+    want = logits(eng, seqs)
+    assert len(calls) == 1
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.ExternalStream(handle.value)):
+        got = logits(eng, seqs)
+        session = eng.runner.decode_session(seqs, 8)
+        session.step(8)
+        torch.cuda.synchronize()
+    assert (len(calls) > 1) == (cus >= 256) and eng.runner.model.decode_in_one_launch
+    assert (got - want).abs().max() <= 3e-2 * want.abs().max()

@@ -22,6 +22,63 @@ def prefilled(eng, lengths, new):
     return seqs
 
 
+@pytest.fixture
+def one_launch(monkeypatch):
+    """Steps whose layers went in one launch (recorded ones count once)."""
+    from nanovllm_hip import ops
+    calls, real = [], ops.decode_layers
+    monkeypatch.setattr(ops, "decode_layers", lambda *a, **kw: calls.append(1) or real(*a, **kw))
+    return calls
+
+
+@pytest.mark.parametrize("family", ["qwen2", "qwen3"])
+@pytest.mark.parametrize("lengths", [(250,), (1,), (511, 40), (250, 300, 7), (250, 300, 7, 40)])
+def test_sessions_against_steps_of_the_host(family, lengths, one_launch):
+    """Generation over a page's end: a session that replays recorded steps (one and four at a time; embedded rows come from the arg-max launch, positions and slots advance on the
+    device), one that runs them, and steps whose metadata the host makes give the same tokens."""
+    eng, new = engine(family), 23
+    few = len(lengths) <= 3
+    tokens = []
+    for graph in (True, False):
+        seqs = prefilled(eng, lengths, new)
+        session = eng.runner.decode_session(seqs, new, use_graph=graph)
+        assert session.fuse_embed and (session.graph_multi is not None) == graph
+        before = len(one_launch)
+        assert not graph or before == (6 if few else 0)      # (a step to warm up, one recorded, four recorded)
+        session.step(new)
+        assert len(one_launch) - before == (new if few and not graph else 0)
+        tokens.append(session.finish())
+        for s in seqs:
+            eng.block_manager.deallocate(s)
+    seqs, host = prefilled(eng, lengths, new), []
+    for _ in range(new):
+        host.append(eng.runner.run(seqs, False))
+        for s, t in zip(seqs, host[-1]):
+            s.append_token(t)
+    assert tokens[0] == tokens[1] == host
+
+
+def test_the_one_launch_up_to_its_width_of_tables(one_launch):
+    """The choice is by the longest context that the block table holds; launches give the same logits beyond it."""
+    from nanovllm_hip import reset_context, set_context
+    from nanovllm_hip.engine.model_runner import build_decode_meta
+    eng = engine("qwen2")
+    seqs, model = prefilled(eng, (40, 300, 7), 4), eng.runner.model
+    want = logits(eng, seqs)
+    pages = model._decode_bufs[(3, "cuda:0")]["layers_tokens"] // 256
+    m = {k: v.cuda() for k, v in build_decode_meta(seqs).items()}
+    assert len(one_launch) == 1 and 0 < pages
+    for width, count in ((pages, 2), (pages + 1, 2), (pages, 3)):
+        table = m["block_tables"].new_zeros(3, width)
+        table[:, :m["block_tables"].shape[1]] = m["block_tables"]
+        with torch.inference_mode():
+            set_context(False, slot_mapping=m["slot_mapping"], context_lens=m["context_lens"], block_tables=table)
+            got = model.compute_logits(model(m["input_ids"], m["positions"])).float()
+            reset_context()
+        assert len(one_launch) == count
+        assert torch.equal(got, want) if width == pages else (got - want).abs().max() <= 3e-2 * want.abs().max()
+
+
 def test_a_step_that_gave_up_is_an_error():
     eng = engine("qwen2")
     seqs = prefilled(eng, (40, 7), 8)

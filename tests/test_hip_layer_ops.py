@@ -185,9 +185,10 @@ def test_fused_linear_rope_store_equals_linear_then_rope_store(H, KVH, D):
     assert torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
 
 
-def test_fused_decode_layer_path_close_to_unfused():
-    """The 6-launch decode path (norm prologues, residual/SiLU/RoPE epilogues) against the 10-launch path on the same
-    weights and cache state: logits agree to bf16 accumulation noise."""
+@pytest.mark.parametrize("one_launch", [True, False])
+def test_fused_decode_layer_path_close_to_unfused(one_launch):
+    """The fused decode path, all layers in one launch and five launches a layer (norms in the projections, residual/SiLU/RoPE
+    epilogues), against the 10-launch path on the same weights and cache state: logits agree to bf16 accumulation noise."""
     from nanovllm_hip.engine.llm_engine import LLMEngine
     from nanovllm_hip.engine.model_runner import build_decode_meta
     from nanovllm_hip.engine.sequence import Sequence
@@ -199,6 +200,7 @@ def test_fused_decode_layer_path_close_to_unfused():
     logits = []
     for fused in (True, False):
         eng = LLMEngine(cfg, num_kvcache_blocks=12, seed=2)
+        eng.runner.model.decode_in_one_launch = one_launch
         seqs = [Sequence(p, max_tokens=4) for p in prompts]
         eng.prefill(seqs, reserve_tokens=4)
         m = build_decode_meta(seqs)
@@ -214,6 +216,8 @@ def test_fused_decode_layer_path_close_to_unfused():
                 reset_context()
         finally:
             qwen._fused_decode_ok = orig
+        held = [b["layers_ws"] for b in eng.runner.model.__dict__.get("_decode_bufs", {}).values()]
+        assert sum(int(ws.view(torch.int32)[0]) for ws in held if ws is not None) == (fused and one_launch)      # launches that did all layers
     scale = logits[1].abs().max()
     assert (logits[0] - logits[1]).abs().max() <= 3e-2 * scale
     assert (logits[0].argmax(-1) == logits[1].argmax(-1)).all()

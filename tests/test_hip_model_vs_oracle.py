@@ -59,13 +59,11 @@ class OracleAttention(torch.nn.Module):
 def _runner(backend, cfg_kwargs, monkeypatch):
     from nanovllm_hip.engine.model_runner import ModelRunner
     from nanovllm_hip.models import qwen
-    if backend == "oracle":
-        monkeypatch.setattr(qwen, "resolve_attention", lambda name, block_size=256: (OracleAttention, {}))
-    cfg = qwen.model_config("Qwen2-0.5B", attn_backend=backend, **cfg_kwargs)
-    r = ModelRunner(cfg, num_kvcache_blocks=12, seed=4)
-    if backend == "oracle":
-        monkeypatch.undo()
-    return r
+    with monkeypatch.context() as patch:
+        if backend == "oracle":
+            patch.setattr(qwen, "resolve_attention", lambda name, block_size=256: (OracleAttention, {}))
+        cfg = qwen.model_config("Qwen2-0.5B", attn_backend=backend, **cfg_kwargs)
+        return ModelRunner(cfg, num_kvcache_blocks=12, seed=4)
 
 
 @torch.inference_mode()
@@ -97,9 +95,13 @@ def _logits_inner(runner, seqs, is_prefill, dev, set_context, reset_context, bui
 
 
 @pytest.mark.parametrize("fused", [False, True], ids=["plain_layer", "fused_decode_layer"])
+@pytest.mark.parametrize("count", [4, 3, 2, 1])               # sequences; the fused decode steps of up to three are all layers in one launch
 @pytest.mark.parametrize("family", ["qwen2", "qwen3"])
-def test_decoder_stack_hip_vs_oracle_attention(family, fused, monkeypatch):
+def test_decoder_stack_hip_vs_oracle_attention(family, count, fused, monkeypatch):
+    from nanovllm_hip import ops
     from nanovllm_hip.engine.sequence import Sequence
+    one_launch, real = [], ops.decode_layers
+    monkeypatch.setattr(ops, "decode_layers", lambda *a, **kw: one_launch.append(1) or real(*a, **kw))
     kw = dict(num_hidden_layers=2, vocab_size=2048)
     if family == "qwen3":                                       # per-head q/k RMSNorm before RoPE, no bias, D = 128, G = 2
         kw.update(num_attention_heads=4, num_key_value_heads=2, head_dim=128, hidden_size=512, intermediate_size=1024, qkv_bias=False, qk_norm=True)
@@ -111,8 +113,8 @@ def test_decoder_stack_hip_vs_oracle_attention(family, fused, monkeypatch):
     assert type(hip.model.layers[0].self_attn.attn).__module__.endswith("attention_hip")
 
     g = torch.Generator().manual_seed(11)
-    lens = (300, 17, 256, 1)                                    # crosses a block, ends on a block boundary, single token
-    tables = ([3, 7], [1], [5, 2], [9])                         # 256 -> 257 tokens needs a second block: booked up front
+    lens = (300, 17, 256, 1)[-count:]                           # crosses a block, ends on a block boundary, single token
+    tables = ([3, 7], [1], [5, 2], [9])[-count:]                # 256 -> 257 tokens needs a second block: booked up front
     steps = 3
 
     def mk():
@@ -145,6 +147,7 @@ def test_decoder_stack_hip_vs_oracle_attention(family, fused, monkeypatch):
         for s_a, s_b, t in zip(sa, sb, tok_b.tolist()):         # both sides continue with the oracle side's token
             s_a.append_token(t)
             s_b.append_token(t)
+    assert len(one_launch) == (steps if fused and count <= 3 else 0)
     # the K/V rows the hip side stored (RoPE + store fused into one launch / the qkv GEMM epilogue) against the oracle module's caches
     for la_, lb_ in zip(hip.model.layers, ora.model.layers):
         kc = la_.self_attn.attn.k_cache.float().cpu().numpy()

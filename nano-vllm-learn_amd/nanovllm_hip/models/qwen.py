@@ -374,7 +374,7 @@ class QwenForCausalLM(nn.Module):
             inter = self.layers[0].mlp.down_proj.weight.shape[1]
             head = self.embed_tokens.weight if cfg.tie_word_embeddings else self.lm_head.weight
             need = max(ops.linear_workspace_bytes(m, head.shape[0], cfg.hidden_size, "none"),
-                       ops.linear_workspace_bytes(m, cfg.hidden_size, cfg.hidden_size, "residual_add"),
+                       ops.linear_workspace_bytes(m, cfg.hidden_size, self.layers[0].self_attn.o_proj.weight.shape[1], "residual_add"),
                        ops.linear_workspace_bytes(m, cfg.hidden_size, inter, "residual_add"),
                        ops.linear_workspace_bytes(m, self.layers[0].self_attn.qkv_proj.weight.shape[0], cfg.hidden_size, "rope_store"),
                        ops.linear_workspace_bytes(m, 2 * inter, cfg.hidden_size, "silu_mul"), 16)

@@ -158,3 +158,16 @@ def test_streams_that_may_not_use_every_cu_get_launches(cus, monkeypatch):
         torch.cuda.synchronize()
     assert (len(calls) > 1) == (cus >= 256) and eng.runner.model.decode_in_one_launch
     assert (got - want).abs().max() <= 3e-2 * want.abs().max()
+
+
+@pytest.mark.parametrize("hidden,heads", [(256, 16), (512, 32)])
+def test_attention_outputs_wider_than_the_stream(hidden, heads, monkeypatch):
+    """The output projection's launch splits a long contraction: its scratch is sized by the heads, not by the stream."""
+    from nanovllm_hip.models import qwen
+    monkeypatch.setitem(FAMILIES, "wide", dict(num_attention_heads=heads, num_key_value_heads=4, head_dim=128, hidden_size=hidden, intermediate_size=512, qkv_bias=False, qk_norm=True))
+    eng = engine("wide")
+    seqs = prefilled(eng, (40, 300, 7, 5), 4)
+    got = logits(eng, seqs)
+    monkeypatch.setattr(qwen, "FUSED_DECODE", False)
+    want = logits(eng, seqs)
+    assert (got - want).abs().max() <= 3e-2 * want.abs().max()

@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NVH_VERSION 211          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch, _status, _variant; 210: nvh_decode_layers; 211: nvh_decode_layers_status, nvh_decode_layers_stream */
+#define NVH_VERSION 211          /* major*100 + minor; 201: nvh_allreduce_status; 202: nvh_linear_desc.prefetch; 203: NVH_DECODE_CHUNKED_P256; 204: nvh_qkv_rope_attend; 205: nvh_prefill_varlen_pv16; 206: nvh_linear_desc.glu_*, nvh_rglru_*, nvh_latent_*; 207: nvh_rglru_desc.links, nvh_prefill_step, nvh_moe_experts; 208: nvh_rglru_desc.rows, links_bytes, nvh_scan_whole_channels; 209: nvh_moe_experts_one_launch, _status, _variant; 210: nvh_decode_layers; 211: nvh_decode_layers_status, _stream, _tokens_for */
 
 /* dtype codes */
 #define NVH_BF16 0
@@ -294,8 +294,9 @@ typedef struct {
     void* workspace; size_t workspace_bytes;
 } nvh_decode_layers_desc;
 size_t nvh_decode_layers_workspace(int m, int hidden, int h, int kvh, int hd, int inter, int n_layers);
-/* longest context for which this is faster than a launch for each part (longer ones are served all the same) */
+/* contexts up to which this is faster than a launch for each part (longer ones are served all the same; 0: for none), by an estimate; _tokens: of layers without q/k norm */
 int nvh_decode_layers_tokens(int m, int hidden, int h, int kvh, int hd, int inter, int n_layers);
+int nvh_decode_layers_tokens_for(int m, int hidden, int h, int kvh, int hd, int inter, int n_layers, int qk_norm);
 int nvh_decode_layers(const nvh_decode_layers_desc* desc, int dtype, void* stream);
 /* 1: launches on this stream may use every CU of the device.  Workgroups wait for each other; with fewer CUs some start only behind others' ends, which costs a wait that runs out for
  * nearly every part (Qwen2-0.5B, 248 CUs: 16 ms a step; launches 0.63) */

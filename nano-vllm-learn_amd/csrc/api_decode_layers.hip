@@ -33,11 +33,6 @@ int plan_decode_layers(DecodeLayersArgs& a, int cus, int m, int hidden, int h, i
     a.grid = cus; a.nf = nf; a.nm = nm;
     a.chunks = nf / (m * kvh) < 16 ? nf / (m * kvh) : 16;
     a.shares = m * kvh * a.chunks;
-    // Attention is the front's alone, its tokens come a round (two tiles of 16 of each of eight waves) behind the other, where a launch of its own has the whole chip: up to six times
-    // 128 tokens a share of one sequence, three and a half of two, two and a half of three are worth what the rest gains.  Whole steps, this against five launches a layer: Qwen3-0.6B one sequence of 4096 tokens (2.8 times 128 a share)
-    // 655 us against 822; two of 1500 / 2500 / 3500 (2.1 / 3.6 / 5 times) 678 / 807 / 888 against 777 / 832 / 847; three of 1500 (3.2) 807 against 837; Qwen2-0.5B two of 4096 (2.7)
-    // 566 against 628, three of 2048 / 4096 (2 / 4) 579 / 671 against 623 / 640
-    a.most_tokens = a.chunks * kDecodeLayersWalkers * 16 * (m == 1 ? 12 : m == 2 ? 7 : 5) / 2;
     a.nf_magic = magic_of(nf); a.nm_magic = magic_of(nm); a.chunks_magic = magic_of(a.chunks); a.kvh_magic = magic_of(kvh); a.group_magic = magic_of(a.group); a.h_magic = magic_of(h);
     a.o_qkv = 0; a.o_o = m * nqkv; a.o_act = a.o_o + m * hidden; a.o_down = a.o_act + m * inter; a.o_rec = a.o_down + m * hidden;
     a.layer_words = a.o_rec + (int64_t)a.shares * a.group * 2 * (hd + 2);
@@ -54,6 +49,33 @@ int plan_decode_layers(DecodeLayersArgs& a, int cus, int m, int hidden, int h, i
     a.l_x[3] = take(2 * m * hidden);
     a.l_x[4] = take(2 * m * inter);
     return lds;
+}
+
+// Contexts up to which this beats launches of their own, a multiple of 128, 0 for none.  Us a layer, from 3800 timed steps of 730 random shapes (1 to 32 layers; contexts of 1 to 12288): a
+// launch saves 5.9 where one row is served and 1.2 less for each further one, 0.21 - 0.03 m a MB of weights, 1.5 with a q/k norm (a launch of its own there), and the split attention of a
+// launch costs 0.5 up to 1024 tokens and 0.3 for every 1024.  It costs here, one behind the other: reading the shares of the attention (the output projection's workgroups read all of
+// them, 1024 values and four shares a trip; 0.35 a trip alone, 0.6 in traffic of several rows), and 2.5 for every further round of tiles.  Starting all CUs is 8.  What is left has to be 0.85
+// a layer, for all contexts up to that one.  Of 2480 of those steps that it then takes the slowest has 0.95 of the launches' speed and three others less than 0.99; by tokens a share
+// alone, the second bound here, 349 of 3100 were slower, up to 0.63: three rows of 768 / 16 / 2 heads of 128, 5120 tokens, 476 us by launches and 629; one layer 31 and 41.
+int decode_layers_tokens(int cus, int m, int hidden, int h, int kvh, int hd, int inter, int layers, bool qk_norm) {
+    DecodeLayersArgs a{};
+    if (!plan_decode_layers(a, cus, m, hidden, h, kvh, hd, inter, layers)) return 0;
+    const float mb = 2e-6f * ((float)hidden * (a.nqkv + a.qsize) + 3.f * (float)hidden * inter);
+    // Attention is the front's alone, its tokens come a round (two tiles of 16 of each of eight waves) behind the other, where a launch of its own has the whole chip: up to six times
+    // 128 tokens a share of one sequence, three and a half of two, two and a half of three.  Whole steps, this against launches: Qwen3-0.6B one sequence of 4096 tokens (2.8 times 128 a
+    // share) 654 us against 823; two of 1500 / 2500 / 3500 (2.1 / 3.6 / 5 times) 682 / 806 / 888 against 776 / 828 / 845; three of 1500 (3.2) 807 against 837; Qwen2-0.5B two of 4096
+    // (2.7) 564 against 628, three of 2048 / 4096 (2 / 4) 579 / 671 against 619 / 639
+    const int most = a.chunks * kDecodeLayersWalkers * 16 * (m == 1 ? 12 : m == 2 ? 7 : 5) / 2;
+    int tokens = 0;
+    for (int ctx = 128; ctx <= most; ctx += 128) {
+        const int used = (ctx + 255) / 256 < a.chunks ? (ctx + 255) / 256 : a.chunks, rounds = (ctx + 256 * used - 1) / (256 * used);
+        const int trips = (m * a.qsize + 1023) / 1024 * (used <= 2 ? 1 : (used + 3) / 4);
+        const float gain = 5.9f - 1.2f * m + (0.21f - 0.03f * m) * mb + (qk_norm ? 1.5f : 0.f) - (a.qsize > 1024 ? 0.5f : 0.f) + 0.5f * (ctx < 1024 ? ctx : 1024) / 1024 + 0.3f * ctx / 1024 -
+                           (m == 1 ? 0.35f : 0.6f) * trips - 2.5f * (rounds - 1);
+        if (layers * (gain - 0.85f) < 8.f) break;
+        tokens = ctx;
+    }
+    return tokens;
 }
 
 static int device_cus() {
@@ -75,8 +97,11 @@ size_t nvh_decode_layers_workspace(int m, int hidden, int h, int kvh, int hd, in
 }
 
 int nvh_decode_layers_tokens(int m, int hidden, int h, int kvh, int hd, int inter, int n_layers) {
-    DecodeLayersArgs a{};
-    return plan_decode_layers(a, device_cus(), m, hidden, h, kvh, hd, inter, n_layers) ? a.most_tokens : 0;
+    return decode_layers_tokens(device_cus(), m, hidden, h, kvh, hd, inter, n_layers, false);
+}
+
+int nvh_decode_layers_tokens_for(int m, int hidden, int h, int kvh, int hd, int inter, int n_layers, int qk_norm) {
+    return decode_layers_tokens(device_cus(), m, hidden, h, kvh, hd, inter, n_layers, qk_norm != 0);
 }
 
 int nvh_decode_layers_variant(uint32_t spin_limit, int late_from, int late_for, const nvh_decode_layers_desc* d, int dtype, void* stream) {

@@ -33,7 +33,7 @@ struct DecodeLayersArgs {
     int64_t layer_words;
     int m, hidden, h, kvh, group, inter, nqkv, qsize, layers, block_size, max_blocks;
     int grid, nf, nm;                            // workgroups; of the front; of the feed-forward
-    int chunks, shares, most_tokens;             // attention: shares of a (sequence, key head); of all; contexts up to which this beats launches of their own
+    int chunks, shares;                          // attention: shares of a (sequence, key head); of all
     float norm_eps, post_eps, qk_eps, scale_log2;
     uint32_t spin_limit;
     int late_from, late_for;
@@ -48,6 +48,8 @@ static_assert(sizeof(DecodeLayersArgs) <= 4096, "kernel arguments");
 
 // Fills everything but pointers; returns the bytes of LDS, 0 if these sizes are not served.
 int plan_decode_layers(DecodeLayersArgs& a, int cus, int m, int hidden, int h, int kvh, int hd, int inter, int layers);
+// Longest context up to which it pays (0: never): of any step whose table is no wider.
+int decode_layers_tokens(int cus, int m, int hidden, int h, int kvh, int hd, int inter, int layers, bool qk_norm);
 int launch_decode_layers(const DecodeLayersArgs& a, int hd, bool qk_norm, int lds, hipStream_t stream);
 
 }  // namespace nvh

@@ -271,6 +271,7 @@ _SIGS = {
     "nvh_linear_small_m_workspace": (ctypes.c_size_t, [ctypes.c_int] * 4),
     "nvh_decode_layers_workspace": (ctypes.c_size_t, [ctypes.c_int] * 7),
     "nvh_decode_layers_tokens": (ctypes.c_int, [ctypes.c_int] * 7),
+    "nvh_decode_layers_tokens_for": (ctypes.c_int, [ctypes.c_int] * 8),
     "nvh_decode_layers": (ctypes.c_int, [ctypes.POINTER(DecodeLayersDesc), ctypes.c_int, ctypes.c_void_p]),
     "nvh_decode_layers_stream": (ctypes.c_int, [ctypes.c_void_p]),
     "nvh_decode_layers_status": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint32)]),

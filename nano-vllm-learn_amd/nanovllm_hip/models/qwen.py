@@ -385,9 +385,9 @@ class QwenForCausalLM(nn.Module):
                              ws=torch.zeros(need, dtype=torch.uint8, device=device))
             a = self.layers[0].self_attn
             sizes = (m, cfg.hidden_size, a.num_heads, a.num_kv_heads, a.head_dim, inter, len(self.layers))
-            need = 0 if _tp()[1] > 1 else ops.decode_layers_workspace_bytes(*sizes)
-            bufs[key]["layers_ws"] = torch.zeros(need, dtype=torch.uint8, device=device) if need else None
-            bufs[key]["layers_tokens"] = ops.decode_layers_tokens(*sizes) if need else 0
+            tokens = 0 if _tp()[1] > 1 else ops.decode_layers_tokens(*sizes, qk_norm=a.qk_norm)
+            bufs[key]["layers_ws"] = torch.zeros(ops.decode_layers_workspace_bytes(*sizes), dtype=torch.uint8, device=device) if tokens else None
+            bufs[key]["layers_tokens"] = tokens
         return bufs[key]
 
     def _forward_decode_fused(self, residual, positions, packed0=None):

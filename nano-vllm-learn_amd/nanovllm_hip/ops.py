@@ -560,9 +560,9 @@ def decode_layers_workspace_bytes(m, hidden, num_heads, num_kv_heads, head_dim, 
     return int(_lib.load().nvh_decode_layers_workspace(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers))
 
 
-def decode_layers_tokens(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers) -> int:
-    """Longest context for which decode_layers is faster than a launch for each part of a layer."""
-    return int(_lib.load().nvh_decode_layers_tokens(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers))
+def decode_layers_tokens(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers, qk_norm=False) -> int:
+    """Contexts up to which decode_layers is faster than a launch for each part of a layer; 0: none."""
+    return int(_lib.load().nvh_decode_layers_tokens_for(m, hidden, num_heads, num_kv_heads, head_dim, inter, layers, int(qk_norm)))
 
 
 def decode_layers(x, layers, *, num_heads, num_kv_heads, head_dim, inter, norm_eps, post_eps, positions, cos_sin, slot_mapping, context_lens, block_tables, workspace,

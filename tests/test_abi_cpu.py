@@ -268,3 +268,18 @@ def test_decode_layers_plan_refuses_sizes_without_heads():
     assert done.returncode == 0, done.stderr[-500:]
     first, *rest = [int(x) for x in done.stdout.split()]
     assert first > 0 and rest == [0] * len(bad)
+
+
+def test_a_decode_step_is_one_launch_where_that_is_faster():
+    """Contexts up to which it is chosen on 256 CUs, beside steps timed both ways: (m, hidden, heads, key heads, width, inter, layers, q/k norm), a context, launches / one launch."""
+    from nanovllm_hip import _lib
+    tokens = ctypes.CDLL(_lib.LIB_PATH)["_ZN3nvh20decode_layers_tokensEiiiiiiiib"]
+    qwen2, qwen3 = (896, 14, 2, 64, 4864, 24, False), (1024, 16, 8, 128, 3072, 28, True)
+    timed = [((1, *qwen2), 4096, 1.54), ((1, *qwen2), 12288, 1.23), ((2, *qwen2), 1024, 1.37), ((2, *qwen2), 4096, 1.11), ((3, *qwen2), 2048, 1.07), ((3, *qwen2), 4096, 0.95),
+             ((1, *qwen3), 9216, 1.09), ((2, *qwen3), 2560, 1.03), ((2, *qwen3), 3500, 0.96), ((3, *qwen3), 1024, 1.07),
+             ((3, 768, 16, 2, 128, 2368, 16, True), 1115, 0.94), ((3, 768, 16, 2, 128, 2368, 16, True), 5120, 0.76), ((3, 256, 7, 1, 128, 960, 32, False), 59, 0.92),
+             ((3, 896, 16, 1, 128, 2944, 32, False), 5120, 0.80), ((2, 256, 16, 2, 128, 4800, 2, False), 1090, 0.85), ((1, 512, 4, 1, 64, 448, 1, False), 3, 0.95),
+             ((3, 256, 16, 2, 64, 3776, 1, True), 125, 0.83), ((2, 640, 16, 1, 64, 960, 24, False), 7168, 0.95), ((1, 384, 8, 1, 128, 5056, 16, False), 12288, 1.20)]
+    for sizes, context, speed in timed:
+        assert (tokens(256, *sizes) >= context) == (speed > 1), (sizes, context, tokens(256, *sizes))
+    assert tokens(256, 4, *qwen2) == tokens(32, 1, *qwen2) == tokens(256, 1, 896, 0, 2, 64, 4864, 24, False) == 0

@@ -7,6 +7,13 @@ pytestmark = pytest.mark.gpu
 FAMILIES = {"qwen2": {}, "qwen3": dict(num_attention_heads=4, num_key_value_heads=2, head_dim=128, hidden_size=512, intermediate_size=1024, qkv_bias=False, qk_norm=True)}
 
 
+@pytest.fixture(autouse=True)
+def one_launch_pays(monkeypatch):
+    """Models of three layers are run the way that larger ones are."""
+    from nanovllm_hip import ops
+    monkeypatch.setattr(ops, "decode_layers_tokens", lambda m, *a, **kw: 2560 if m <= 3 else 0)
+
+
 def engine(family, **kw):
     from nanovllm_hip.engine.llm_engine import LLMEngine
     from nanovllm_hip.models import qwen

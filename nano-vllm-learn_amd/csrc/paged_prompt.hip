@@ -111,10 +111,12 @@ __global__ __launch_bounds__(256, WIDE && DK == 128 && DV == 64 ? 3 : WIDE || DK
             [&](f32x4 (&v)[DV / 8]) {
                 if (a.o_cos_sin && q_ok) turn_back_tiles<8>(v, a.o_cos_sin, my_q + shift, a.max_position, a.o_rot, lg);
                 uint16_t* const o_lds = reinterpret_cast<uint16_t*>(lds) + wave * WR * kRowOut<DV>;
+                int out_lane = lane;                 // (not seen by the compiler yet: no address is held over the walk)
+                asm volatile("" : "+v"(out_lane));
 #pragma unroll
-                for (int u = 0; u < DV / 8; ++u) act_st4(o_lds + lq * kRowOut<DV> + 8 * u + 4 * lg, v[u]);
+                for (int u = 0; u < DV / 8; ++u) act_st4(o_lds + (out_lane & (WR - 1)) * kRowOut<DV> + 8 * u + 4 * (out_lane / WR), v[u]);
                 const int r0 = q0 + wave * WR;
-                rows_out<DV, WR>(o_lds, lane, [&](int r) { return r0 + r < sq ? reinterpret_cast<uint16_t*>(a.out) + (int64_t)(q_beg + r0 + r) * a.out_stride + head * DV : nullptr; });
+                rows_out<DV, WR>(o_lds, out_lane, [&](int r) { return r0 + r < sq ? reinterpret_cast<uint16_t*>(a.out) + (int64_t)(q_beg + r0 + r) * a.out_stride + head * DV : nullptr; });
             });
     } else {
         attend_walk<DK, DV, 1>(

@@ -665,10 +665,12 @@ __device__ __forceinline__ bool prefill32_body(const PrefillArgs& a, unsigned ch
                 return;
             }
             uint16_t* const o_lds = reinterpret_cast<uint16_t*>(lds) + wave * WR * kRowOut<D>;
+            int out_lane = lane;                     // (not seen by the compiler yet: addresses held over the walk would cost heads of 64 with exact P the fourth workgroup a CU)
+            asm volatile("" : "+v"(out_lane));
 #pragma unroll
-            for (int u = 0; u < D / 8; ++u) act_st4(o_lds + lq * kRowOut<D> + 8 * u + 4 * lh, v[u]);
+            for (int u = 0; u < D / 8; ++u) act_st4(o_lds + (out_lane & (WR - 1)) * kRowOut<D> + 8 * u + 4 * (out_lane / WR), v[u]);
             const int r0 = q0 + wave * WR;
-            rows_out<D, WR>(o_lds, lane, [&](int r) { return r0 + r < sq ? reinterpret_cast<uint16_t*>(a.out) + ((int64_t)(q_beg + r0 + r) * a.h + head) * D : nullptr; });
+            rows_out<D, WR>(o_lds, out_lane, [&](int r) { return r0 + r < sq ? reinterpret_cast<uint16_t*>(a.out) + ((int64_t)(q_beg + r0 + r) * a.h + head) * D : nullptr; });
         });
     return true;
 }

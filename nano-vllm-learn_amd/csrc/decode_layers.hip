@@ -21,8 +21,11 @@
 // A column of a product is a wave's: its lanes hold 16-byte pieces of the weight row, 64 apart, and add up products with the same pieces of the activations
 // (16 x 16 matrix tiles would read 64 lanes' worth of LDS for the few columns a workgroup has: 2.1 us for the down projection where this takes 0.5).  Eight waves of
 // three columns rather than twelve of two: sums and epilogues are issued by fewer waves.  Up to three rows; four would take as long as launches of their own.
-// Whole step with the LM head, contexts of 513 to 1024 tokens, launches -> this: Qwen2-0.5B one sequence 604 -> 362 us (layers with LDS for the weights and twelve
-// waves 387), two 605 -> 446, three 611 -> 525; Qwen3-0.6B 734 -> 507, 741 -> 602, 768 -> 728.
+// Whole step with the LM head, contexts of 513 to 1024 tokens, launches -> this: Qwen2-0.5B one sequence 598 -> 354 us (layers with LDS for the weights and twelve
+// waves 387), two 606 -> 443, three 606 -> 527; Qwen3-0.6B 730 -> 502, 733 -> 598, 761 -> 720.  For which sizes and contexts: decode_layers_tokens.
+// Beside another stream (Qwen2-0.5B, one sequence; launches in brackets): copies of 256 MB 600 us (1130), small kernels 360 (603), attention over prompts 385 (602, at times 2770),
+// products of 2048 400 (602), two such sessions 673 each (728): other streams' kernels get no CU while the step runs.  On a stream that may not use every CU workgroups start behind
+// others' ends, and each part waits for that: 16 ms with 248 CUs, 53 with 128 (launches 0.63, 0.73).
 // Arithmetic and rounding points are those of linear_stream.hip, rope_store.hip and decode_chunked.h (P as hi + lo); sums have another order.
 #include "decode_layers.h"
 
@@ -355,7 +358,7 @@ __global__ __launch_bounds__(kThreads) void decode_layers_kernel(const DecodeLay
     };
 
     bool have_x = false;                                                         // the stream that the residual sums need is in LDS
-    // ---- one share of a projection: a wave takes two columns (gate_up: two of gate and the two of up that belong to them) of every 24
+    // ---- one share of a projection: a wave takes three columns (gate_up: three of gate and the three of up that belong to them; down: one) of every 24
     // help: another workgroup's, whose weights are not held but read.  Returns whether a wait ran out
     auto project = [&](auto phase, auto help, int l, int role) -> bool {
         constexpr int ph = decltype(phase)::value;

@@ -307,7 +307,7 @@ class PackedResidual:
 
 
 def _fused_decode_ok(cfg, x):
-    """The 5-launch decoder layer (6 with Qwen3's q/k-norm) applies to single-GPU decode batches of at most 64 rows."""
+    """The fused decode step (_forward_decode_fused) applies to decode batches of at most 64 rows."""
     from ..utils.context import get_context
     ctx = get_context()
     return (FUSED_DECODE and x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= 64 and not ctx.is_prefill
@@ -328,8 +328,8 @@ class QwenForCausalLM(nn.Module):
 
     def forward(self, input_ids, positions, embedded=None):
         """embedded = (hidden [m, hidden], packed) — fused decode path only: the token embeddings already looked up by the
-        previous step's nvh_greedy_advance_candidates_embed, row-major (it becomes the residual stream, updated in place) and in
-        fragment order (what layer 0's projection reads); input_ids is then not touched."""
+        previous step's nvh_greedy_advance_candidates_embed, row-major (the residual stream in front of the first layer; a step by launches
+        updates it in place) and in fragment order (what layer 0's projection reads); input_ids is then not touched."""
         if embedded is not None:
             assert _fused_decode_ok(self.cfg, embedded[0]) and self._fused_shapes_ok()
             return self._forward_decode_fused(embedded[0], positions, packed0=embedded[1])
@@ -391,9 +391,11 @@ class QwenForCausalLM(nn.Module):
         return bufs[key]
 
     def _forward_decode_fused(self, residual, positions, packed0=None):
-        """Decode step with 6 launches per layer (qkv, attention split + combine, o_proj, gate_up, down): the norms ride in the
-        projections (folded weights + epilogue row scale), residual adds / SiLU*mul / RoPE+store are GEMM epilogues.
-        `residual` is the running residual stream (the embedding output, updated in place); every GEMM that updates it also
+        """Decode step: all layers in one launch for few sequences (_forward_decode_layers), else five launches per layer (qkv,
+        attention, o_proj, gate_up, down; with q/k norm one more): the norms ride in the projections (folded weights + epilogue row
+        scale), residual adds / SiLU*mul / RoPE+store are GEMM epilogues.
+        `residual` is the residual stream (the embedding output); the launches update it in place, the one launch leaves it and
+        returns a new one.  By launches, every GEMM that updates it also
         writes it in fragment order for the next GEMM (csrc/linear_stream.hip), and the MLP activation exists only in that
         order.  The final norm belongs to the LM head's launch, so this returns the un-normalised stream as a PackedResidual."""
         from .. import ops
@@ -471,7 +473,7 @@ class QwenForCausalLM(nn.Module):
         return PackedResidual(residual, resid_p)
 
     def _forward_decode_layers(self, x, positions, ctx, b):
-        """The same step for a few sequences of a model whose layers fit the chip's registers: all layers in one launch (csrc/decode_layers.hip)."""
+        """The same step for a few sequences of a model whose layers fit the chip's registers: all layers in one launch (csrc/decode_layers.hip).  x stays as it is."""
         from .. import ops
         fw, cfg, a = self._folded_weights(), self.cfg, self.layers[0].self_attn
         layers = [dict(qkv_w=fw["qkv"][i], qkv_bias=l.self_attn.qkv_proj.bias, q_norm_w=l.self_attn.q_norm.weight if a.qk_norm else None,
